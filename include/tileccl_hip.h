@@ -303,6 +303,19 @@ int tccl_allreduce_staged(void* tensor, int32_t dtype, int64_t numel, void* stag
                           uint32_t ranks, const tccl_heap_view* heap, int64_t* fault, int64_t spin_limit_ns,
                           void* stream);
 
+/* tccl_collective_direct: the same five collectives (TCCL_STAGED_*, the same buffers, results and bits) for a
+ * caller that carries every rank's role in one launch and whose inputs are complete on `stream`, as on
+ * one GPU: no staging, no signal words, no waits.  The all-reduce of one unit reads it from every slice, adds
+ * (ranks ascending, fp32) and stores the sum to every slice, so it moves 2 x world tensor sizes where the
+ * staged protocol moves (4 + world) x world. */
+int tccl_collective_direct(int32_t op, const void* src, void* dst, int32_t dtype, int64_t block_elems, int32_t root,
+                           const tccl_heap_view* heap, void* stream);
+/* tccl_allreduce_chunk: one rank's part of an in-place all-reduce (tile_allreduce): chunk heap->rank of
+ * `tensor` (numel / world_size elements) summed over the ranks' tensors (the own value first, then ranks
+ * ascending, fp32, one rounding) and stored into every rank's tensor.  A rank reads and writes only its own
+ * chunk index, so the ranks' calls may run in any order. */
+int tccl_allreduce_chunk(void* tensor, int32_t dtype, int64_t numel, const tccl_heap_view* heap, void* stream);
+
 /* ---- fused operations --------------------------------------------------------------------
  * variant S0: GEMM kernel, then the communication kernel, stream-ordered.
  * variant S1: one launch; GEMM workgroups signal locks[tile]; communication workgroups

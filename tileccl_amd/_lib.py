@@ -151,6 +151,8 @@ SIGNATURES = {
         C.c_int,
         [_i32, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _i32, _i32, _i32, C.c_uint32, _i32, _P(HeapView), _vp, _i64, _vp],
     ),
+    "tccl_collective_direct": (C.c_int, [_i32, _vp, _vp, _i32, _i64, _i32, _P(HeapView), _vp]),
+    "tccl_allreduce_chunk": (C.c_int, [_vp, _i32, _i64, _P(HeapView), _vp]),
     "tccl_allreduce_staged": (
         C.c_int,
         [_vp, _i32, _i64, _vp, _vp, _vp, _i32, _i32, _i32, C.c_uint32, _P(HeapView), _vp, _i64, _vp],

@@ -12,6 +12,7 @@
 #pragma GCC visibility push(default)
 #include "../../include/tileccl_hip.h"
 #pragma GCC visibility pop
+#include "tccl_bulk.h"
 #include "tccl_comm.h"
 #include "tccl_gemm.h"
 #include "tccl_gemm256.h"
@@ -126,17 +127,13 @@ __global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g) {
 #endif
 }
 
-// The stand-alone bulk kernels (S0's second kernel, the scatter / gather / block copies, the stand-alone
-// reduction): the communication role with everything else compiled out.  The full role (per-tile and
-// per-group waits, every reduction type) is a large kernel, and a launch of it took 1.2 us longer to move
-// the same bytes (the 128 MiB exchange of the 4096 x 4096 x 1024 all-gather: 21.5 against 20.3 us).
-__global__ __launch_bounds__(256) void copy_kernel(tccl::CommArgs c) {
-  __shared__ int word[4];
-  tccl::comm_role<tccl::kThreadsComm, tccl::kBulkCopy>(c, (int)blockIdx.x, (int)gridDim.x, word);
+// The transfers that wait for nothing (tccl_bulk.h): blockIdx.y is the rectangle.
+__global__ __launch_bounds__(256) void copy_kernel(tccl::BulkCopyArgs a) {
+  tccl::bulk_copy<tccl::kThreadsComm>(a, (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x);
 }
-__global__ __launch_bounds__(256) void reduce_kernel(tccl::CommArgs c) {
-  __shared__ int word[4];
-  tccl::comm_role<tccl::kThreadsComm, tccl::kBulkReduce>(c, (int)blockIdx.x, (int)gridDim.x, word);
+template <typename PT, typename OT, int kRanks>
+__global__ __launch_bounds__(256) void reduce_kernel(tccl::BulkReduceArgs a) {
+  tccl::bulk_reduce<PT, OT, kRanks, tccl::kThreadsComm>(a, a.first_owner + (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Staged collectives: workgroup w carries slot w % slots of the (w / slots)-th rank named in a.ranks.
@@ -329,12 +326,22 @@ int check_heap(const tccl_heap_view* h) {
   return 0;
 }
 
-int set_task_units(tccl::CommArgs* c, const tccl_transport_desc* tr, bool reduce) {
-  const int unit_elems = reduce ? 8 : 16 / c->esize;
-  int elems = tr ? (reduce && tr->reduce_elems > 0 ? tr->reduce_elems : tr->copy_elems) : 0;
-  if (elems <= 0) elems = 16384;
+// Elements per task of a transport descriptor, checked: whole 16-byte units (reductions: 8 elements).
+int task_elems(const tccl_transport_desc* tr, bool reduce) {
+  const int elems = tr ? (reduce && tr->reduce_elems > 0 ? tr->reduce_elems : tr->copy_elems) : 0;
+  return elems > 0 ? elems : 16384;
+}
+
+int check_task_elems(const tccl_transport_desc* tr, bool reduce, int esize) {
+  const int elems = task_elems(tr, reduce), unit_elems = reduce ? 8 : 16 / esize;
   if (elems % unit_elems) return fail(TCCL_ERR_UNSUPPORTED, "task size %d elements is not a multiple of %d", elems, unit_elems);
-  c->copy_units = c->reduce_units = elems / unit_elems;
+  return 0;
+}
+
+int set_task_units(tccl::CommArgs* c, const tccl_transport_desc* tr, bool reduce) {
+  const int rc = check_task_elems(tr, reduce, c->esize);
+  if (rc) return rc;
+  c->copy_units = c->reduce_units = task_elems(tr, reduce) / (reduce ? 8 : 16 / c->esize);
   return 0;
 }
 
@@ -464,7 +471,7 @@ void set_row_divider(tccl::PullArgs* p, uint32_t upr, uint32_t pitch, uint32_t s
 // after the last tile then does it).
 bool build_background(const tccl::CommArgs& c, tccl::PullArgs* p) {
   memset(p, 0, sizeof *p);
-  if (c.op != tccl::kOpAllGather || c.granularity == tccl::kBulk || !(c.directions & tccl::kDirPull) || c.world <= 1) return false;
+  if (c.op != tccl::kOpAllGather || !(c.directions & tccl::kDirPull) || c.world <= 1) return false;
   const bool by_tile = c.granularity == tccl::kPerTile;
   int band_shift = 0;
   if (by_tile) {
@@ -575,38 +582,116 @@ int check_comm_span(const tccl::CommArgs& c) {
   return check_rows_span(c.M, pitch);
 }
 
-int launch_comm(const tccl::CommArgs& c, int wgs, hipStream_t stream) {
-  const int span = check_comm_span(c);
-  if (span) return span;
-  if (wgs < 1) wgs = 1;
-  if (c.granularity != tccl::kBulk) return fail(TCCL_ERR_INVALID, "a stand-alone communication launch is a bulk one");
-  if (c.op == tccl::kOpReduceScatter)
-    hipLaunchKernelGGL(reduce_kernel, dim3(wgs), dim3(tccl::kThreadsComm), 0, stream, c);
-  else
-    hipLaunchKernelGGL(copy_kernel, dim3(wgs), dim3(tccl::kThreadsComm), 0, stream, c);
+// ---- stand-alone transfers -------------------------------------------------------------------
+// Workgroups of a stand-alone kernel, per CU.  Copies: swept on the 128 MiB exchange of the 4096 x 4096 x 1024
+// all-gather (2 / 4 / 8 per CU: 20.7 / 20.3 / 19.7 us).
+#ifndef TCCL_BULK_COPY_WGS
+#define TCCL_BULK_COPY_WGS 8
+#endif
+#ifndef TCCL_BULK_REDUCE_WGS
+#define TCCL_BULK_REDUCE_WGS 8
+#endif
+// Units a copying workgroup takes at a time: one 16-byte access per thread while that does not fill the
+// device, then more, up to 32 KiB (tasks of 128 KiB took 21.7 us instead of 19.7 on that exchange).
+constexpr int kBulkTaskUnits = 2048;
+
+uint32_t all_but(int world, int rank) { return ((1u << world) - 1u) & ~(1u << rank); }
+
+int launch_bulk_copy(tccl::BulkCopyArgs& a, int transfers, int64_t rows, const tccl_device_info& dev, hipStream_t stream) {
+  a.units = (int)(rows * a.upr);
+  if (a.units <= 0 || transfers <= 0) return 0;
+  const int64_t wgs = (int64_t)dev.compute_units * TCCL_BULK_COPY_WGS;
+  int64_t task = ((int64_t)a.units * transfers + wgs - 1) / wgs;
+  task = (task + tccl::kThreadsComm - 1) / tccl::kThreadsComm * tccl::kThreadsComm;
+  if (task > kBulkTaskUnits) task = kBulkTaskUnits;
+  a.task_units = (int)task;
+  int64_t x = (a.units + task - 1) / task;
+  if (x > wgs / transfers) x = wgs / transfers;
+  hipLaunchKernelGGL(copy_kernel, dim3((unsigned)x, (unsigned)transfers), dim3(tccl::kThreadsComm), 0, stream, a);
   TCCL_HIP(hipGetLastError());
   return 0;
 }
 
-// Workgroups of a stand-alone bulk kernel, per CU: 8 for copies, 4 for reductions.  Swept on the 128 MiB
-// exchange of the 4096 x 4096 x 1024 all-gather (2 / 4 / 8 per CU: 20.7 / 20.3 / 19.7 us; tasks of 128 KiB
-// instead of 32 KiB: 21.7 us) and on the reductions of the reduce-scatter configurations (4 per CU ahead
-// of 8 by 3-4 %).
-#ifndef TCCL_BULK_COPY_WGS
-#define TCCL_BULK_COPY_WGS 8
-#endif
-int bulk_comm_wgs(const tccl_device_info& dev, const tccl::CommArgs& c) {
-  return dev.compute_units * (c.op == tccl::kOpReduceScatter ? 4 : TCCL_BULK_COPY_WGS);
+template <typename PT, typename OT>
+void launch_reduce_t(const tccl::BulkReduceArgs& a, dim3 grid, int ranks, hipStream_t stream) {
+  const dim3 block(tccl::kThreadsComm);
+  if (ranks == 2)
+    hipLaunchKernelGGL((reduce_kernel<PT, OT, 2>), grid, block, 0, stream, a);
+  else if (ranks == 4)
+    hipLaunchKernelGGL((reduce_kernel<PT, OT, 4>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((reduce_kernel<PT, OT, 8>), grid, block, 0, stream, a);
 }
 
-// The second kernel of S0 waits for nothing, so a plan's TileGroups mean nothing to it: it
-// sweeps the whole block (a reduce-scatter: each owner's shard) as one run of tasks.  Cut
-// along the plan's groups, its tasks came out ragged at every group border (8192 x 4096
-// all-gather: 123 us with eight groups against 117 us with one).
-void make_bulk(tccl::CommArgs* c) {
-  c->granularity = tccl::kBulk;
-  c->row_starts = c->row_ends = c->tile_counts = nullptr;
-  c->n_groups = c->op == tccl::kOpReduceScatter ? c->world : 1;
+int launch_bulk_reduce(tccl::BulkReduceArgs& a, int owners, int64_t rows, int partial_dtype, int out_dtype, const tccl_device_info& dev,
+                       hipStream_t stream) {
+  a.units = (int)(rows * a.upr);
+  if (a.units <= 0 || owners <= 0) return 0;
+  const int ranks = a.world <= 2 ? 2 : (a.world <= 4 ? 4 : 8);
+  const int64_t per_wg = (int64_t)tccl::kThreadsComm * (8 / ranks);
+  int64_t x = (a.units + per_wg - 1) / per_wg;
+  const int64_t most = (int64_t)dev.compute_units * TCCL_BULK_REDUCE_WGS / owners;
+  if (x > most) x = most;
+  const dim3 grid((unsigned)x, (unsigned)owners);
+  const int key = partial_dtype * 4 + out_dtype;
+  switch (key) {
+    case TCCL_F32 * 4 + TCCL_F32: launch_reduce_t<float, float>(a, grid, ranks, stream); break;
+    case TCCL_F32 * 4 + TCCL_F16: launch_reduce_t<float, _Float16>(a, grid, ranks, stream); break;
+    case TCCL_F32 * 4 + TCCL_BF16: launch_reduce_t<float, __bf16>(a, grid, ranks, stream); break;
+    case TCCL_F16 * 4 + TCCL_F16: launch_reduce_t<_Float16, _Float16>(a, grid, ranks, stream); break;
+    case TCCL_F16 * 4 + TCCL_BF16: launch_reduce_t<_Float16, __bf16>(a, grid, ranks, stream); break;
+    case TCCL_BF16 * 4 + TCCL_BF16: launch_reduce_t<__bf16, __bf16>(a, grid, ranks, stream); break;
+    case TCCL_BF16 * 4 + TCCL_F16: launch_reduce_t<__bf16, _Float16>(a, grid, ranks, stream); break;
+    default: return fail(TCCL_ERR_UNSUPPORTED, "reduce: no kernel for partial dtype %d, output dtype %d", partial_dtype, out_dtype);
+  }
+  TCCL_HIP(hipGetLastError());
+  return 0;
+}
+
+// The transfer of a GEMM + collective operation as a launch of its own (the second kernel of S0).
+int launch_bulk(const tccl::CommArgs& c, const tccl_device_info& dev, hipStream_t stream) {
+  const int span = check_comm_span(c);
+  if (span) return span;
+  if (c.op == tccl::kOpReduceScatter) {
+    const int shard = c.M / c.world;
+    tccl::BulkReduceArgs a;
+    memset(&a, 0, sizeof a);
+    a.heap_bases = c.heap_bases;
+    a.rank = c.rank;
+    a.world = c.world;
+    a.src = (int64_t)(uintptr_t)c.C;
+    a.dst = (int64_t)(uintptr_t)c.rs_out;
+    a.src_shift = shard * c.ldc_bytes;
+    a.src_pitch = (uint32_t)c.ldc_bytes;
+    a.dst_pitch = (uint32_t)c.ld_rs_out_bytes;
+    a.upr = c.N / 8;
+    a.first_owner = c.emulate_peer ? 0 : c.rank;
+    return launch_bulk_reduce(a, c.emulate_peer ? c.world : 1, shard, c.partial_dtype, c.out_dtype, dev, stream);
+  }
+  tccl::BulkCopyArgs a;
+  memset(&a, 0, sizeof a);
+  a.heap_bases = c.heap_bases;
+  a.rank = c.rank;
+  a.world = c.world;
+  int n = 0;
+  if (c.op == tccl::kOpAllScatter) {
+    a.src = (int64_t)(uintptr_t)c.C + (int64_t)c.src_col_off * c.esize;
+    a.dst = (int64_t)(uintptr_t)c.C + (int64_t)c.dst_col_off * c.esize;
+    a.src_pitch = (uint32_t)c.ldc_bytes;
+    a.dst_pitch = (uint32_t)((int64_t)c.dst_ld * c.esize);
+    a.upr = c.cols * c.esize / 16;
+    a.t[n++] = {0, 0, c.rank, all_but(c.world, c.rank)};
+  } else {
+    a.src = a.dst = (int64_t)(uintptr_t)c.out;
+    a.src_pitch = a.dst_pitch = (uint32_t)c.ld_out_bytes;
+    a.upr = c.N * c.esize / 16;
+    const int64_t block = c.M * c.ld_out_bytes;
+    if (c.directions & tccl::kDirPull)
+      for (int p = 0; p < c.world; ++p)
+        if (p != c.rank) a.t[n++] = {p * block, p * block, p, 1u << c.rank};
+    if (c.directions & tccl::kDirPush) a.t[n++] = {c.rank * block, c.rank * block, c.rank, all_but(c.world, c.rank)};
+  }
+  return launch_bulk_copy(a, n, c.M, dev, stream);
 }
 
 // The shards that make up the GEMM's A operand, when the chained operation reads them in place.
@@ -673,9 +758,8 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     if (variant == TCCL_S0_BULK) {
       int rc = launch_gemm256(d->in_dtype, d->out_dtype, g, m, wgs, stream);
       if (rc) return rc;
-      make_bulk(&c);
       if (c.world <= 1 && c.op != tccl::kOpReduceScatter) return 0;
-      return launch_comm(c, bulk_comm_wgs(dev, c), stream);
+      return launch_bulk(c, dev, stream);
     }
     Fused256Args f;
     f.g = g;
@@ -717,9 +801,8 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     memset(&none, 0, sizeof none);
     int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, none, compute, 0, trace_start, stream);
     if (rc) return rc;
-    make_bulk(&c);
     if (c.world <= 1 && c.op != tccl::kOpReduceScatter) return 0;
-    return launch_comm(c, bulk_comm_wgs(dev, c), stream);
+    return launch_bulk(c, dev, stream);
   }
   int comm = tr && tr->num_comm_wgs > 0 ? tr->num_comm_wgs : dev.compute_units;
   s.epoch = sync->epoch > 0 ? sync->epoch : 1;
@@ -1020,28 +1103,18 @@ int tccl_scatter_cols(const void* C, int32_t M, int64_t ldc, int32_t elem_bytes,
   if ((rc = check_rows_span(M, (ldc > sc->dst_ld ? ldc : (int64_t)sc->dst_ld) * elem_bytes))) return rc;
   tccl_device_info dev;
   if ((rc = query_device(-1, &dev))) return rc;
-  tccl::GemmArgs g;
-  memset(&g, 0, sizeof g);
-  g.C = (void*)C;
-  g.M = M;
-  g.N = N;
-  g.ldc = ldc;
-  g.block_m = g.block_n = 128;
-  g.group_m = 8;
-  g.tile_rows = (M + 127) / 128;
-  g.tile_cols = (N + 127) / 128;
-  g.xcds = 1;
-  g.span = 1;
-  tccl::CommArgs c;
-  fill_comm_common(&c, g, elem_bytes, heap, nullptr, nullptr);
-  c.op = tccl::kOpAllScatter;
-  c.granularity = tccl::kBulk;
-  c.src_col_off = sc->src_col_offset;
-  c.cols = sc->cols;
-  c.dst_ld = sc->dst_ld;
-  c.dst_col_off = sc->dst_col_offset;
-  if ((rc = set_task_units(&c, nullptr, false))) return rc;
-  return launch_comm(c, bulk_comm_wgs(dev, c), (hipStream_t)stream);
+  tccl::BulkCopyArgs a;
+  memset(&a, 0, sizeof a);
+  a.heap_bases = heap->heap_bases;
+  a.rank = heap->rank;
+  a.world = heap->world_size;
+  a.src = (int64_t)(uintptr_t)C + (int64_t)sc->src_col_offset * elem_bytes;
+  a.dst = (int64_t)(uintptr_t)C + (int64_t)sc->dst_col_offset * elem_bytes;
+  a.src_pitch = (uint32_t)(ldc * elem_bytes);
+  a.dst_pitch = (uint32_t)((int64_t)sc->dst_ld * elem_bytes);
+  a.upr = sc->cols * elem_bytes / 16;
+  a.t[0] = {0, 0, heap->rank, all_but(heap->world_size, heap->rank)};
+  return launch_bulk_copy(a, 1, M, dev, (hipStream_t)stream);
 }
 
 int tccl_exchange_rows(void* out, int32_t rows_per_rank, int32_t N, int64_t ld, int32_t elem_bytes,
@@ -1056,26 +1129,23 @@ int tccl_exchange_rows(void* out, int32_t rows_per_rank, int32_t N, int64_t ld, 
   if ((rc = check_rows_span(rows_per_rank, ld * elem_bytes))) return rc;
   tccl_device_info dev;
   if ((rc = query_device(-1, &dev))) return rc;
-  tccl::GemmArgs g;
-  memset(&g, 0, sizeof g);
-  g.C = (char*)out + (int64_t)heap->rank * rows_per_rank * ld * elem_bytes;
-  g.M = rows_per_rank;
-  g.N = N;
-  g.ldc = ld;
-  g.block_m = g.block_n = 128;
-  g.group_m = 8;
-  g.tile_rows = (rows_per_rank + 127) / 128;
-  g.tile_cols = (N + 127) / 128;
-  g.xcds = 1;
-  g.span = 1;
-  tccl::CommArgs c;
-  fill_comm_common(&c, g, elem_bytes, heap, nullptr, tr);
-  c.op = tccl::kOpAllGather;
-  c.granularity = tccl::kBulk;
-  c.out = (char*)out;
-  c.ld_out_bytes = ld * elem_bytes;
-  if ((rc = set_task_units(&c, tr, false))) return rc;
-  return launch_comm(c, bulk_comm_wgs(dev, c), (hipStream_t)stream);
+  if ((rc = check_task_elems(tr, false, elem_bytes))) return rc;
+  const int64_t pitch = ld * elem_bytes, block = rows_per_rank * pitch;
+  const int directions = tr ? tr->directions : TCCL_DIR_PUSH;
+  tccl::BulkCopyArgs a;
+  memset(&a, 0, sizeof a);
+  a.heap_bases = heap->heap_bases;
+  a.rank = heap->rank;
+  a.world = heap->world_size;
+  a.src = a.dst = (int64_t)(uintptr_t)out;
+  a.src_pitch = a.dst_pitch = (uint32_t)pitch;
+  a.upr = N * elem_bytes / 16;
+  int n = 0;
+  if (directions & TCCL_DIR_PULL)
+    for (int p = 0; p < a.world; ++p)
+      if (p != a.rank) a.t[n++] = {p * block, p * block, p, 1u << a.rank};
+  if (directions & TCCL_DIR_PUSH) a.t[n++] = {a.rank * block, a.rank * block, a.rank, all_but(a.world, a.rank)};
+  return launch_bulk_copy(a, n, rows_per_rank, dev, (hipStream_t)stream);
 }
 
 int tccl_copy_block(void* dst, uint32_t dst_ranks, const void* src, int32_t src_rank, int32_t rows, int64_t row_bytes,
@@ -1095,29 +1165,18 @@ int tccl_copy_block(void* dst, uint32_t dst_ranks, const void* src, int32_t src_
   if (dst_ranks == 0) return 0;
   tccl_device_info dev;
   if ((rc = query_device(-1, &dev))) return rc;
-  tccl::GemmArgs g;
-  memset(&g, 0, sizeof g);
-  g.C = (void*)src;
-  g.M = rows;
-  g.N = (int)row_bytes;
-  g.ldc = src_pitch_bytes;
-  g.block_m = g.block_n = 128;
-  g.group_m = 8;
-  g.tile_rows = (rows + 127) / 128;
-  g.tile_cols = (int)((row_bytes + 127) / 128);
-  g.xcds = 1;
-  g.span = 1;
-  tccl::CommArgs c;
-  fill_comm_common(&c, g, 1, heap, nullptr, nullptr);
-  c.op = tccl::kOpCopyBlock;
-  c.granularity = tccl::kBulk;
-  c.out = (char*)dst;
-  c.ld_out_bytes = dst_pitch_bytes;
-  c.copy_src_rank = src_rank;
-  c.copy_dst_ranks = dst_ranks;
-  // 32 KiB per task, whatever the element type of the caller's data
-  c.copy_units = c.reduce_units = 2048;
-  return launch_comm(c, bulk_comm_wgs(dev, c), (hipStream_t)stream);
+  tccl::BulkCopyArgs a;
+  memset(&a, 0, sizeof a);
+  a.heap_bases = heap->heap_bases;
+  a.rank = heap->rank;
+  a.world = heap->world_size;
+  a.src = (int64_t)(uintptr_t)src;
+  a.dst = (int64_t)(uintptr_t)dst;
+  a.src_pitch = (uint32_t)src_pitch_bytes;
+  a.dst_pitch = (uint32_t)dst_pitch_bytes;
+  a.upr = (int)(row_bytes / 16);
+  a.t[0] = {0, 0, src_rank, dst_ranks};
+  return launch_bulk_copy(a, 1, rows, dev, (hipStream_t)stream);
 }
 
 int tccl_gather_cols(void* gathered, int64_t ld_gathered, const void* shard, int64_t ld_shard, int32_t M,
@@ -1136,27 +1195,19 @@ int tccl_gather_cols(void* gathered, int64_t ld_gathered, const void* shard, int
   if ((rc = check_rows_span(M, (ld_gathered > ld_shard ? ld_gathered : ld_shard) * elem_bytes))) return rc;
   tccl_device_info dev;
   if ((rc = query_device(-1, &dev))) return rc;
-  tccl::GemmArgs g;
-  memset(&g, 0, sizeof g);
-  g.C = (void*)shard;
-  g.M = M;
-  g.N = cols;
-  g.ldc = ld_shard;
-  g.block_m = g.block_n = 128;
-  g.group_m = 8;
-  g.tile_rows = (M + 127) / 128;
-  g.tile_cols = (cols + 127) / 128;
-  g.xcds = 1;
-  g.span = 1;
-  tccl::CommArgs c;
-  fill_comm_common(&c, g, elem_bytes, heap, nullptr, tr);
-  c.op = tccl::kOpGatherCols;
-  c.granularity = tccl::kBulk;
-  c.directions = TCCL_DIR_PUSH | TCCL_DIR_PULL;  // the own shard is copied, the peers' are pulled
-  c.out = (char*)gathered;
-  c.ld_out_bytes = ld_gathered * elem_bytes;
-  if ((rc = set_task_units(&c, tr, false))) return rc;
-  return launch_comm(c, bulk_comm_wgs(dev, c), (hipStream_t)stream);
+  if ((rc = check_task_elems(tr, false, elem_bytes))) return rc;
+  tccl::BulkCopyArgs a;
+  memset(&a, 0, sizeof a);
+  a.heap_bases = heap->heap_bases;
+  a.rank = heap->rank;
+  a.world = heap->world_size;
+  a.src = (int64_t)(uintptr_t)shard;
+  a.dst = (int64_t)(uintptr_t)gathered;
+  a.src_pitch = (uint32_t)(ld_shard * elem_bytes);
+  a.dst_pitch = (uint32_t)(ld_gathered * elem_bytes);
+  a.upr = cols * elem_bytes / 16;
+  for (int p = 0; p < a.world; ++p) a.t[p] = {0, (int64_t)p * cols * elem_bytes, p, 1u << a.rank};
+  return launch_bulk_copy(a, a.world, M, dev, (hipStream_t)stream);
 }
 
 static int fill_reduce(tccl::CommArgs* c, const void* partial, int partial_dtype, void* out, int out_dtype, int64_t ld_out,
@@ -1194,24 +1245,18 @@ int tccl_reduce_rows(const void* partial, int32_t partial_dtype, int64_t ld_part
   if ((rc = check_rows_span(M, ld_partial * esize)) || (rc = check_rows_span(M, ld_out * 4))) return rc;
   tccl_device_info dev;
   if ((rc = query_device(-1, &dev))) return rc;
-  tccl::GemmArgs g;
-  memset(&g, 0, sizeof g);
-  g.C = (void*)partial;
-  g.M = M;
-  g.N = N;
-  g.ldc = ld_partial;
-  g.block_m = g.block_n = 128;
-  g.group_m = 8;
-  g.tile_rows = (M + 127) / 128;
-  g.tile_cols = (N + 127) / 128;
-  g.xcds = 1;
-  g.span = 1;
   tccl::CommArgs c;
-  fill_comm_common(&c, g, esize, heap, nullptr, tr);
+  memset(&c, 0, sizeof c);
+  c.heap_bases = heap->heap_bases;
+  c.rank = heap->rank;
+  c.world = heap->world_size;
+  c.C = (char*)partial;
+  c.ldc_bytes = ld_partial * esize;
+  c.M = M;
+  c.N = N;
   if ((rc = fill_reduce(&c, partial, partial_dtype, out, out_dtype, ld_out, M, N, heap->world_size, emulate_peer, true))) return rc;
-  c.granularity = tccl::kBulk;
-  if ((rc = set_task_units(&c, tr, true))) return rc;
-  return launch_comm(c, bulk_comm_wgs(dev, c), (hipStream_t)stream);
+  if ((rc = check_task_elems(tr, true, esize))) return rc;
+  return launch_bulk(c, dev, (hipStream_t)stream);
 }
 
 static int allscatter_impl(const tccl_gemm_desc* d, const tccl_scatter_desc* sc, const tccl_heap_view* heap,
@@ -1297,6 +1342,97 @@ int tccl_collective_staged(int32_t op, const void* src, void* dst, int32_t dtype
   a.spin_ticks = (spin_limit_ns > 0 ? spin_limit_ns : kDefaultSpinNs) / 10 + 1;
   hipLaunchKernelGGL(staged_kernel, dim3(roles * slots), dim3(256), 0, (hipStream_t)stream, a);
   TCCL_HIP(hipGetLastError());
+  return 0;
+}
+
+// A collective whose inputs are complete and whose roles are all carried by one launch needs no staging and
+// no waits: each byte of a result is read from where it lies and written where it is wanted.
+int tccl_collective_direct(int32_t op, const void* src, void* dst, int32_t dtype, int64_t block_elems, int32_t root,
+                           const tccl_heap_view* heap, void* stream) {
+  static const char* const names[] = {"allreduce", "allgather", "reduce_scatter", "broadcast", "scatter"};
+  int rc = check_heap(heap);
+  if (rc) return rc;
+  if (op < TCCL_STAGED_ALLREDUCE || op > TCCL_STAGED_SCATTER) return fail(TCCL_ERR_INVALID, "collective_direct: unknown op %d", op);
+  const char* name = names[op];
+  const bool reduces = op == TCCL_STAGED_ALLREDUCE || op == TCCL_STAGED_REDUCE_SCATTER;
+  const bool in_place = op == TCCL_STAGED_ALLREDUCE || op == TCCL_STAGED_BROADCAST;
+  const int esize = (int)dtype_size(dtype), world = heap->world_size;
+  if (!esize || (reduces && dtype != TCCL_F16 && dtype != TCCL_BF16 && dtype != TCCL_F32))
+    return fail(TCCL_ERR_UNSUPPORTED, "%s_direct: dtype %d", name, dtype);
+  if (!dst || (!in_place && !src) || block_elems <= 0) return fail(TCCL_ERR_INVALID, "%s_direct: bad arguments", name);
+  if (root < 0 || root >= world) return fail(TCCL_ERR_INVALID, "%s_direct: root=%d out of range [0, %d)", name, root, world);
+  const int per_unit = 16 / esize;
+  if (block_elems % per_unit || !aligned16(dst) || (!in_place && !aligned16(src)))
+    return fail(TCCL_ERR_UNSUPPORTED, "%s_direct: blocks must be whole 16-byte units (%d elements)", name, per_unit);
+  if (reduces && block_elems % 8) return fail(TCCL_ERR_UNSUPPORTED, "%s_direct: blocks must be multiples of 8 elements", name);
+  tccl_device_info dev;
+  if ((rc = query_device(-1, &dev))) return rc;
+  const int64_t block = block_elems * esize, piece = 1ll << 30;  // a launch addresses its rectangle with 32-bit offsets
+  for (int64_t at = 0; at < block; at += piece) {
+    const int64_t bytes = block - at < piece ? block - at : piece;
+    if (reduces) {
+      tccl::BulkReduceArgs a;
+      memset(&a, 0, sizeof a);
+      a.heap_bases = heap->heap_bases;
+      a.rank = heap->rank;
+      a.world = world;
+      a.src = (int64_t)(uintptr_t)(in_place ? dst : src) + at;
+      a.dst = (int64_t)(uintptr_t)dst + at;
+      a.src_shift = in_place ? 0 : block;
+      a.src_pitch = a.dst_pitch = (uint32_t)bytes;
+      a.upr = (int)(bytes / esize / 8);
+      a.ascending = a.to_all = in_place ? 1 : 0;
+      rc = launch_bulk_reduce(a, in_place ? 1 : world, 1, dtype, dtype, dev, (hipStream_t)stream);
+    } else {
+      tccl::BulkCopyArgs a;
+      memset(&a, 0, sizeof a);
+      a.heap_bases = heap->heap_bases;
+      a.rank = heap->rank;
+      a.world = world;
+      a.src = (int64_t)(uintptr_t)(in_place ? dst : src) + at;
+      a.dst = (int64_t)(uintptr_t)dst + at;
+      a.src_pitch = a.dst_pitch = (uint32_t)bytes;
+      a.upr = (int)(bytes / 16);
+      int n = 0;
+      if (op == TCCL_STAGED_ALLGATHER)
+        for (int r = 0; r < world; ++r) a.t[n++] = {0, r * block, r, (1u << world) - 1u};
+      else if (op == TCCL_STAGED_BROADCAST)
+        a.t[n++] = {0, 0, root, all_but(world, root)};
+      else
+        for (int q = 0; q < world; ++q) a.t[n++] = {q * block, 0, root, 1u << q};
+      rc = launch_bulk_copy(a, n, 1, dev, (hipStream_t)stream);
+    }
+    if (rc) return rc;
+  }
+  return 0;
+}
+
+int tccl_allreduce_chunk(void* tensor, int32_t dtype, int64_t numel, const tccl_heap_view* heap, void* stream) {
+  int rc = check_heap(heap);
+  if (rc) return rc;
+  const int esize = (int)dtype_size(dtype), world = heap->world_size;
+  if (dtype != TCCL_F16 && dtype != TCCL_BF16 && dtype != TCCL_F32) return fail(TCCL_ERR_UNSUPPORTED, "allreduce_chunk: dtype %d", dtype);
+  if (!tensor || numel <= 0 || numel % world) return fail(TCCL_ERR_INVALID, "allreduce_chunk: bad arguments");
+  if ((numel / world) % 8 || !aligned16(tensor))
+    return fail(TCCL_ERR_UNSUPPORTED, "allreduce_chunk: a rank's chunk must be a multiple of 8 elements and 16-byte aligned");
+  tccl_device_info dev;
+  if ((rc = query_device(-1, &dev))) return rc;
+  const int64_t chunk = numel / world * esize, piece = 1ll << 30;
+  for (int64_t at = 0; at < chunk; at += piece) {
+    const int64_t bytes = chunk - at < piece ? chunk - at : piece;
+    tccl::BulkReduceArgs a;
+    memset(&a, 0, sizeof a);
+    a.heap_bases = heap->heap_bases;
+    a.rank = heap->rank;
+    a.world = world;
+    a.src = a.dst = (int64_t)(uintptr_t)tensor + at;
+    a.src_shift = a.dst_shift = chunk;
+    a.src_pitch = a.dst_pitch = (uint32_t)bytes;
+    a.upr = (int)(bytes / esize / 8);
+    a.first_owner = heap->rank;
+    a.to_all = 1;
+    if ((rc = launch_bulk_reduce(a, 1, 1, dtype, dtype, dev, (hipStream_t)stream))) return rc;
+  }
   return 0;
 }
 

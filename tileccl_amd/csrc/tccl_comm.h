@@ -9,14 +9,13 @@
 // access (global_load_dwordx4 / global_store_dwordx4), a wavefront covers 1 KiB of a row
 // per instruction, and every thread keeps several loads in flight before its stores.
 //
-// Four operations share the machinery (reference call sites in brackets):
+// Three operations share the machinery (reference call sites in brackets):
 //   all-scatter     column block of C -> every peer's C   [patterns/_helpers.py:86-199]
 //   all-gather      row block of `out` <-> peers' `out`   [primitives/collectives.py:613-663]
 //   reduce-scatter  out = cast(sum over ranks of partial) [primitives/collectives.py:730-783]
-//   gather-columns  rank p's input shard -> column block p of this rank's gathered input
-//                   [gather worker of patterns/chained_ag_gemm_rs.py:262-340]
-// and three granularities: bulk (no waiting; the second kernel of S0), per plan tile
-// (S1: locks[tile] >= epoch) and per TileGroup (S2: tile_wait_ge on counter[group]).
+// and two granularities: per plan tile (S1: locks[tile] >= epoch) and per TileGroup
+// (S2: tile_wait_ge on counter[group]).  Transfers that wait for nothing (S0's second kernel, the
+// stand-alone collectives) are the kernels of tccl_bulk.h.
 #pragma once
 
 #include "tccl_device.h"
@@ -28,8 +27,8 @@ typedef _Float16 f16x8v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-enum OpKind { kOpNone = 0, kOpAllScatter = 1, kOpAllGather = 2, kOpReduceScatter = 3, kOpGatherCols = 4, kOpCopyBlock = 5 };
-enum Granularity { kBulk = 0, kPerTile = 1, kPerGroup = 2 };
+enum OpKind { kOpNone = 0, kOpAllScatter = 1, kOpAllGather = 2, kOpReduceScatter = 3 };
+enum Granularity { kPerTile = 1, kPerGroup = 2 };
 enum { kDirPush = 1, kDirPull = 2 };
 enum { kF16 = 0, kBF16 = 1, kF32 = 2 };  // the codes of include/tileccl_hip.h
 
@@ -45,14 +44,8 @@ struct CommArgs {
   // all-scatter placement (elements)
   int src_col_off, cols, dst_ld, dst_col_off;
   // all-gather: gathered output of this rank; rank r's block starts at row r*M.
-  // gather-columns: C is this rank's input shard (M x N), out the gathered input whose
-  // column block r (N columns wide) comes from rank r's shard.
-  // copy-block: the rectangle at C (M rows of N bytes, esize 1) is read in slice `copy_src_rank`
-  // and written at out in every slice of the mask `copy_dst_ranks`.
   char* out;
   int64_t ld_out_bytes;
-  int copy_src_rank;
-  uint32_t copy_dst_ranks;
   // reduce-scatter: C is the partial; rs_out the owner's shard
   char* rs_out;
   int64_t ld_rs_out_bytes;
@@ -116,17 +109,19 @@ constexpr int kBulkReducePolicy = kStreaming;
 
 // ---- copy: units [u_lo, u_hi) of the rectangle, one source slice, any number of targets ----
 // kPolicy is the cache policy of both sides: kCoherent inside fused launches (the source
-// was just written by other workgroups, the target will be read by a peer), kStreaming
-// for the stand-alone bulk kernel.
+// was just written by other workgroups, the target will be read by a peer), kBulkCopyPolicy
+// in the stand-alone kernels.
 constexpr int kCopyHalf = 4;  // 16-byte accesses per thread in one of the two register sets
 
 template <int kPolicy, int kThreads>
 struct CopyBatch {
-  const CommArgs& a;
-  const Xfer& x;
+  const int64_t* heap_bases;
+  int world;
+  uint32_t dst_ranks;
+  int64_t dst_off;  // relative to a slice base
   __amdgpu_buffer_rsrc_t src;
   bool flat;
-  uint32_t sp, dp;
+  uint32_t upr, sp, dp;
   int tid, u_hi;
 
   TCCL_D void load(int u0, u32x4 (&v)[kCopyHalf], uint32_t (&doff)[kCopyHalf]) const {
@@ -138,7 +133,7 @@ struct CopyBatch {
         soff = (uint32_t)u * 16u;
         doff[k] = soff;
       } else {
-        const uint32_t r = (uint32_t)u / (uint32_t)x.upr, c = (uint32_t)u - r * (uint32_t)x.upr;
+        const uint32_t r = (uint32_t)u / upr, c = (uint32_t)u - r * upr;
         soff = r * sp + c * 16u;
         doff[k] = r * dp + c * 16u;
       }
@@ -147,9 +142,9 @@ struct CopyBatch {
     }
   }
   TCCL_D void store(int u0, const u32x4 (&v)[kCopyHalf], const uint32_t (&doff)[kCopyHalf]) const {
-    for (int q = 0; q < a.world; ++q) {
-      if (!((x.dst_ranks >> q) & 1u)) continue;
-      const __amdgpu_buffer_rsrc_t dst = window(a.heap_bases[q] + x.dst_off);
+    for (int q = 0; q < world; ++q) {
+      if (!((dst_ranks >> q) & 1u)) continue;
+      const __amdgpu_buffer_rsrc_t dst = window(heap_bases[q] + dst_off);
 #pragma unroll
       for (int k = 0; k < kCopyHalf; ++k)
         if (u0 + tid + k * kThreads < u_hi) st16<kPolicy>(dst, doff[k], v[k]);
@@ -162,11 +157,8 @@ struct CopyBatch {
 // mixed instead of a read phase and a write phase (all workgroups of a launch start together and would
 // otherwise alternate in step).
 template <int kPolicy, int kThreads>
-TCCL_D void run_copy(const CommArgs& a, const Xfer& x, int u_lo, int u_hi) {
-  const int src_rank = __builtin_ctz(x.src_ranks);
-  const CopyBatch<kPolicy, kThreads> b{a, x, window(a.heap_bases[src_rank] + x.src_off),
-                                       (x.src_pitch == (int64_t)x.upr * 16) && (x.dst_pitch == x.src_pitch),
-                                       (uint32_t)x.src_pitch, (uint32_t)x.dst_pitch, (int)threadIdx.x, u_hi};
+TCCL_D void run_copy(CopyBatch<kPolicy, kThreads> b, int u_lo, int u_hi) {
+  b.u_hi = u_hi;
   constexpr int kBatch = kThreads * kCopyHalf;
   u32x4 v0[kCopyHalf], v1[kCopyHalf];
   uint32_t d0[kCopyHalf], d1[kCopyHalf];
@@ -307,38 +299,21 @@ TCCL_D void run_reduce(const CommArgs& a, const Xfer& x, int u_lo, int u_hi) {
     case kBF16 * 4 + kBF16: run_reduce_t<__bf16, __bf16, kPolicy, kThreads>(a, x, u_lo, u_hi); break;
     case kBF16 * 4 + kF16: run_reduce_t<__bf16, _Float16, kPolicy, kThreads>(a, x, u_lo, u_hi); break;
     case kF16 * 4 + kBF16: run_reduce_t<_Float16, __bf16, kPolicy, kThreads>(a, x, u_lo, u_hi); break;
-    case kF32 * 4 + kF32:  // the stand-alone reduction only: the fused launches write 16-bit shards
-      if constexpr (kPolicy != kCoherent) run_reduce_t<float, float, kPolicy, kThreads>(a, x, u_lo, u_hi);
-      break;
     default: break;
   }
 }
 
-// kOnly names what a stand-alone bulk kernel is compiled for (kAllRoles: everything, fused launches included).
-enum BulkOnly { kAllRoles = 0, kBulkCopy = 1, kBulkReduce = 2 };
-
-template <int kThreads, int kOnly = kAllRoles>
+template <int kThreads>
 TCCL_D void run_xfer(const CommArgs& a, const Xfer& x, int u_lo, int u_hi) {
-  if constexpr (kOnly == kBulkCopy) {
-    run_copy<kBulkCopyPolicy, kThreads>(a, x, u_lo, u_hi);
-    return;
-  }
-  if constexpr (kOnly == kBulkReduce) {
-    if (x.reduce) run_reduce<kBulkReducePolicy, kThreads>(a, x, u_lo, u_hi);
-    return;
-  }
-  const bool fused = a.granularity != kBulk;
   if (x.reduce) {
-    if (fused)
-      run_reduce<kCoherent, kThreads>(a, x, u_lo, u_hi);
-    else
-      run_reduce<kBulkReducePolicy, kThreads>(a, x, u_lo, u_hi);
-  } else {
-    if (fused)
-      run_copy<kCoherent, kThreads>(a, x, u_lo, u_hi);
-    else
-      run_copy<kBulkCopyPolicy, kThreads>(a, x, u_lo, u_hi);
+    run_reduce<kCoherent, kThreads>(a, x, u_lo, u_hi);
+    return;
   }
+  run_copy(CopyBatch<kCoherent, kThreads>{a.heap_bases, a.world, x.dst_ranks, x.dst_off,
+                                          window(a.heap_bases[__builtin_ctz(x.src_ranks)] + x.src_off),
+                                          (x.src_pitch == (int64_t)x.upr * 16) && (x.dst_pitch == x.src_pitch), (uint32_t)x.upr,
+                                          (uint32_t)x.src_pitch, (uint32_t)x.dst_pitch, (int)threadIdx.x, u_hi},
+           u_lo, u_hi);
 }
 
 // ---- rectangles of the three operations ----------------------------------------------------------
@@ -383,38 +358,10 @@ TCCL_D bool make_xfer(const CommArgs& a, bool pull, int peer, int r0, int r1, in
     x.upr = (c1 - c0) * a.esize / 16;
     return x.dst_ranks != 0;
   }
-  if (a.op == kOpCopyBlock) {
-    // tile_put / tile_get (primitives/communication.py:133-225) on a whole rectangle: both
-    // addresses are the calling rank's own, translated into the slices named.
-    x.src_ranks = 1u << a.copy_src_rank;
-    x.dst_ranks = a.copy_dst_ranks;
-    x.src_pitch = a.ldc_bytes;
-    x.dst_pitch = a.ld_out_bytes;
-    x.src_off = slice_offset(a, a.C) + r0 * x.src_pitch + (int64_t)c0 * a.esize;
-    x.dst_off = slice_offset(a, a.out) + r0 * x.dst_pitch + (int64_t)c0 * a.esize;
-    x.rows = r1 - r0;
-    x.upr = (c1 - c0) * a.esize / 16;
-    return x.dst_ranks != 0;
-  }
-  if (a.op == kOpGatherCols) {
-    // Column block `owner` of this rank's gathered input is rank `owner`'s shard
-    // (chained_ag_gemm_rs.py:270-337); the "push" direction is the copy of the own shard.
-    const int owner = pull ? peer : a.rank;
-    x.src_ranks = 1u << owner;
-    x.dst_ranks = 1u << a.rank;
-    x.src_pitch = a.ldc_bytes;
-    x.dst_pitch = a.ld_out_bytes;
-    x.src_off = slice_offset(a, a.C) + r0 * x.src_pitch + (int64_t)c0 * a.esize;
-    x.dst_off = slice_offset(a, a.out) + r0 * x.dst_pitch + ((int64_t)owner * a.N + c0) * a.esize;
-    x.rows = r1 - r0;
-    x.upr = (c1 - c0) * a.esize / 16;
-    return true;
-  }
   // Reduce-scatter: rows belong to owner = row / (M / world); the owner's shard is rs_out.
   const int shard = a.M / a.world;
   const int owner = r0 / shard;
   if (owner != a.rank && !a.emulate_peer) return false;
-  const int out_esize = a.out_dtype == kF32 ? 4 : 2;
   x.reduce = 1;
   x.first_rank = owner;
   x.src_ranks = all_ranks(a.world);
@@ -422,7 +369,7 @@ TCCL_D bool make_xfer(const CommArgs& a, bool pull, int peer, int r0, int r1, in
   x.src_pitch = a.ldc_bytes;
   x.dst_pitch = a.ld_rs_out_bytes;
   x.src_off = slice_offset(a, a.C) + r0 * x.src_pitch + (int64_t)c0 * a.esize;
-  x.dst_off = slice_offset(a, a.rs_out) + (int64_t)(r0 - owner * shard) * x.dst_pitch + (int64_t)c0 * out_esize;
+  x.dst_off = slice_offset(a, a.rs_out) + (int64_t)(r0 - owner * shard) * x.dst_pitch + (int64_t)c0 * 2;
   x.rows = r1 - r0;
   x.upr = (c1 - c0) / 8;
   return true;
@@ -511,18 +458,18 @@ TCCL_D bool rs_not_mine(const CommArgs& a, int row) {
 // sources are ready or soon will be, independent of this rank's GEMM), then pushes /
 // reductions in production order.  Workgroup w takes tasks w, w + n, w + 2n, ...; no
 // GEMM workgroup ever waits on a communication workgroup, so the order is deadlock-free.
-template <int kThreads = kThreadsComm, int kOnly = kAllRoles>
+template <int kThreads = kThreadsComm>
 TCCL_D void comm_role(const CommArgs& a, int wg, int num_wgs, int* lds_word) {
   if (a.op == kOpNone || num_wgs <= 0) return;
   Waiter wait{a, lds_word, now_ticks() + a.spin_ticks};
   const int peers = a.world - 1;
   const bool is_rs = a.op == kOpReduceScatter;
-  const bool do_pull = (a.op == kOpAllGather || a.op == kOpGatherCols) && (a.directions & kDirPull) && peers > 0;
+  const bool do_pull = a.op == kOpAllGather && (a.directions & kDirPull) && peers > 0;
   const bool do_push = is_rs || (a.directions & kDirPush);
   const int unit_elems = is_rs ? 8 : 16 / a.esize;
   const int units_per_task = is_rs ? a.reduce_units : a.copy_units;
 
-  if (kOnly == kAllRoles && a.granularity == kPerTile) {
+  if (a.granularity == kPerTile) {
     const int total = a.tile_rows * a.tile_cols;
     const int n_pull = do_pull ? peers * total : 0;
     const int n_all = n_pull + (do_push ? total : 0);
@@ -552,8 +499,7 @@ TCCL_D void comm_role(const CommArgs& a, int wg, int num_wgs, int* lds_word) {
     return;
   }
 
-  // Bulk and per-group: tasks are ranges of units_per_task units of a group's rectangle
-  // (bulk treats the plan's groups as plain work partitions and never waits).
+  // Per group: tasks are ranges of units_per_task units of a group's rectangle.
   const int row_units = is_rs ? a.N / 8 : (a.op == kOpAllScatter ? a.cols : a.N) / unit_elems;
   int total = 0;
   for (int g = 0; g < a.n_groups; ++g) total += cdiv((group_hi(a, g) - group_lo(a, g)) * row_units, units_per_task);
@@ -576,19 +522,15 @@ TCCL_D void comm_role(const CommArgs& a, int wg, int num_wgs, int* lds_word) {
     }
     if (g >= a.n_groups) break;
     if (rs_not_mine(a, group_lo(a, g))) continue;
-    bool ok = true;
-    if (kOnly == kAllRoles && a.granularity == kPerGroup) {
-      uint32_t ranks = pull ? (1u << peer) : (is_rs ? all_ranks(a.world) : (1u << a.rank));
-      ok = wait.group(g, ranks);
-    }
+    const bool ok = wait.group(g, pull ? (1u << peer) : (is_rs ? all_ranks(a.world) : (1u << a.rank)));
     Xfer x;
     if (ok && make_xfer(a, pull, peer, group_lo(a, g), group_hi(a, g), 0, a.N, x)) {
       const int units = x.rows * x.upr;
       const int lo = local * units_per_task;
       const int hi = lo + units_per_task < units ? lo + units_per_task : units;
-      if (lo < hi) run_xfer<kThreads, kOnly>(a, x, lo, hi);
+      if (lo < hi) run_xfer<kThreads>(a, x, lo, hi);
     }
-    if (kOnly == kAllRoles && a.granularity == kPerGroup) task_done(a, g, tasks_g * tasks_factor);
+    task_done(a, g, tasks_g * tasks_factor);
   }
 }
 
