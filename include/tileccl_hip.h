@@ -93,7 +93,8 @@ typedef struct tccl_gemm_desc {
   /* Column shards stacked as row blocks (the rank_major_column_shards layout of
    * tileccl.ops.gemm_reducescatter, ops.py:315,646).  0 or 1: plain GEMM.  w > 1: A has M/w
    * rows and B has w*N columns; row block q of C (rows [q*M/w, (q+1)*M/w)) is
-   * A @ B[:, q*N:(q+1)*N].  M/w must be a multiple of the plan tile's rows. */
+   * A @ B[:, q*N:(q+1)*N].  M/w must be a multiple of the plan tile's rows, except in a
+   * tccl_gemm_reducescatter with w == world_size and TCCL_RS_PEERS_RESIDENT. */
   int32_t column_shards;
 } tccl_gemm_desc;
 
@@ -109,6 +110,9 @@ typedef struct tccl_gemm_desc {
  * be >= K.  The reference's GEMM takes arbitrary strides (kernels/gemm.py:139-151); this and the
  * row-major form are the two it meets in practice.  With column_shards = w, B has w * N columns. */
 #define TCCL_GEMM_B_KMAJOR 2
+
+/* The launch's sync descriptor is the head of a tccl_sync_desc_arrivals. */
+#define TCCL_GEMM_ARRIVALS 4
 
 #define TCCL_RS_EMULATE_PEERS 1
 #define TCCL_RS_PEERS_RESIDENT 2
@@ -147,6 +151,16 @@ typedef struct tccl_sync_desc {
   int64_t* fault;               /* int64[1] or NULL: set non-zero if a bounded wait expired */
   int64_t spin_limit_ns;        /* bound of every device-side wait; 0 = library default (2 s) */
 } tccl_sync_desc;
+
+/* What `sync` points at in a launch whose gemm->flags has TCCL_GEMM_ARRIVALS (pass &x.sync).
+ *   arrivals   uint32[total_tiles], device memory (in the heap or not), zeroed once by the host and zero
+ *              again after every launch.
+ * With them small problems are computed in tiles smaller than a plan tile (up to 5 times as fast at
+ * 16 x 2048 x 4096): the last of a plan tile's tiles, found by counting here, publishes it. */
+typedef struct tccl_sync_desc_arrivals {
+  tccl_sync_desc sync;
+  int32_t* arrivals;
+} tccl_sync_desc_arrivals;
 
 /* ---- symmetric heap view -------------------------------------------------------------
  * heap_bases is the int64[world_size] device array of slice base addresses

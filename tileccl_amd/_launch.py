@@ -256,10 +256,12 @@ class SyncWords:
     lock_epoch: int = 0
     spin_limit_ns: int = DEFAULT_SPIN_LIMIT_NS
     max_tasks_per_tile: int = 1 << 16
+    arrivals: torch.Tensor | None = None  # one counter per plan tile, zero between launches (tccl_sync_desc_arrivals)
+    arrivals_from_capture: bool = False  # zeroed by a recorded fill only: every launch has to clear them itself
     clear_every_launch: bool = False  # set by the first launch recorded into a graph
 
     def reset(self) -> None:
-        for t in (self.locks, self.counter, self.barrier, self.trace_comm_counter, self.trace_start_clock,
+        for t in (self.locks, self.counter, self.barrier, self.arrivals, self.trace_comm_counter, self.trace_start_clock,
                   self.trace_ready_clock, self.trace_done_clock, self.fault):
             if t is not None:
                 t.zero_()
@@ -271,7 +273,7 @@ class SyncWords:
         tile_by_tile = variant == "s1"
         if self.clear_every_launch or torch.cuda.is_current_stream_capturing():
             self.clear_every_launch = True
-            for t in (self.locks, self.counter, self.barrier):
+            for t in (self.locks, self.counter, self.barrier, self.arrivals if self.arrivals_from_capture else None):
                 if t is not None:
                     t.zero_()
             self.epoch = self.lock_epoch = 0
@@ -284,8 +286,17 @@ class SyncWords:
         self.epoch += 1
         return self.epoch
 
-    def desc(self, variant: str = "s2") -> _lib.SyncDesc:
-        s = _lib.SyncDesc()
+    def tile_arrivals(self) -> torch.Tensor:
+        """The arrival counters, made on first use for every plan tile these words have signals for."""
+        if self.arrivals is None:
+            tiles = max(int(t.numel()) for t in (self.locks, self.plan.group_table if self.plan is not None else None) if t is not None)
+            self.arrivals_from_capture = torch.cuda.is_current_stream_capturing()
+            self.arrivals = torch.zeros(tiles, dtype=torch.int32, device="cuda:0")
+        return self.arrivals
+
+    def desc(self, variant: str = "s2") -> _lib.SyncDescArrivals:
+        s = _lib.SyncDescArrivals()
+        s.arrivals = ptr(self.tile_arrivals())
         s.locks = ptr(self.locks)
         s.counter = ptr(self.counter)
         s.barrier = ptr(self.barrier)

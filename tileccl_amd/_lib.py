@@ -63,6 +63,7 @@ class GemmDesc(C.Structure):
 
 GEMM_OWN_ROWS_IN_REGISTERS = 1  # TCCL_GEMM_OWN_ROWS_IN_REGISTERS
 GEMM_B_KMAJOR = 2  # TCCL_GEMM_B_KMAJOR
+GEMM_ARRIVALS = 4  # TCCL_GEMM_ARRIVALS
 STAGED_ALLREDUCE, STAGED_ALLGATHER, STAGED_REDUCE_SCATTER, STAGED_BROADCAST, STAGED_SCATTER = range(5)  # TCCL_STAGED_*
 
 
@@ -84,6 +85,12 @@ class SyncDesc(C.Structure):
         ("fault", C.c_void_p),
         ("spin_limit_ns", C.c_int64),
     ]
+
+
+class SyncDescArrivals(SyncDesc):
+    """``tccl_sync_desc_arrivals``: what GEMM_ARRIVALS announces."""
+
+    _fields_ = [("arrivals", C.c_void_p)]
 
 
 class HeapView(C.Structure):

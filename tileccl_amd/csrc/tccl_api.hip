@@ -19,6 +19,7 @@
 #include "tccl_kernels256.h"
 #include "tccl_probe.h"
 #include "tccl_staged.h"
+#include "tccl_stream.h"
 
 namespace {
 
@@ -195,7 +196,8 @@ bool plan_tile_fits_macro(const tccl_gemm_desc* d) {
   return (d->block_m == 128 || d->block_m == 256) && (d->block_n == 128 || d->block_n == 256);
 }
 
-int check_gemm(const tccl_gemm_desc* d) {
+// ragged_shards: row blocks of column_shards need not be whole plan tiles.
+int check_gemm(const tccl_gemm_desc* d, bool ragged_shards = false) {
   if (!d) return fail(TCCL_ERR_INVALID, "gemm descriptor is NULL");
   if (!d->A || !d->B || !d->C) return fail(TCCL_ERR_INVALID, "gemm: A, B and C must be non-NULL");
   if (d->M <= 0 || d->N <= 0 || d->K <= 0) return fail(TCCL_ERR_INVALID, "gemm: M, N, K must be positive (got %d, %d, %d)", d->M, d->N, d->K);
@@ -211,7 +213,7 @@ int check_gemm(const tccl_gemm_desc* d) {
     return fail(TCCL_ERR_UNSUPPORTED, "gemm: fp8 inputs need the 256x256 kernel (macro_tile 0 or 256, plan tile edges 128 or 256)");
   if (d->out_dtype == TCCL_F8E4M3) return fail(TCCL_ERR_UNSUPPORTED, "gemm: fp8 output is not supported");
   const int shards = d->column_shards > 1 ? d->column_shards : 1;
-  if (d->column_shards < 0 || d->M % shards || (shards > 1 && (d->M / shards) % d->block_m))
+  if (d->column_shards < 0 || d->M % shards || (shards > 1 && !ragged_shards && (d->M / shards) % d->block_m))
     return fail(TCCL_ERR_INVALID, "gemm: column_shards=%d must split M=%d into blocks of whole %d-row plan tiles", d->column_shards, d->M, d->block_m);
   if (d->in_dtype == TCCL_F8E4M3 && shards > 1 && (d->M / shards) % 256)
     return fail(TCCL_ERR_UNSUPPORTED, "gemm: fp8 inputs with column_shards need row blocks of whole 256-row tiles");
@@ -741,12 +743,175 @@ bool gather_in_place(const tccl_gemm_desc* d, const tccl_device_info& dev, int k
   return k_shard % 64 == 0 && d->column_shards <= 1 && !(d->flags & TCCL_GEMM_B_KMAJOR);
 }
 
+// ---- streaming path (tccl_stream.h) -------------------------------------------------------------
+// Estimated time of a launch, in us.  A tile's operands pass its CU's vector memory path once, at the rate measured
+// for its shape (KB/us, between that of a k-major and that of a row-major B: 73 and 33, 85 and 45, 85 and 58, 87 and
+// 72, 57 and 50); a tile's sums take the last term.  Measured on 16 .. 256 x
+// 2048 x 4096, 1024 x 1024 x 2048, 1000 x 2064 x 1000, 300 x 768 x 1024 and 512 x 512 x 256, bf16.  Neither the layout
+// of B nor the variant enters, so that all of them add the products up in the same order: the same bits.
+struct StreamCost {
+  double rate, sums;
+};
+constexpr StreamCost kStreamCost[tccl::kStreamShapeCount] = {{46, 0.0}, {60, 0.1}, {70, 0.3}, {80, 0.5}, {54, 1.2}};
+constexpr double kLaunchUs = 3.7;
+
+int64_t stream_tiles(int shape, int64_t seg_rows, int64_t segs, int64_t N) {
+  const int64_t bm = 16 * tccl::kStreamShapes[shape].mb, bn = 16 * tccl::kStreamShapes[shape].nb;
+  return (seg_rows + bm - 1) / bm * segs * ((N + bn - 1) / bn);
+}
+
+double stream_cost(int shape, int64_t K) {
+  const tccl::StreamShape& s = tccl::kStreamShapes[shape];
+  return kLaunchUs + (double)(16 * (s.mb + s.nb) * 2 * K) / 1024.0 / kStreamCost[shape].rate + kStreamCost[shape].sums;
+}
+
+// The 128 x 128-tile kernel: K steps of 32, 0.19 us each with a few tiles and 0.3 us once every CU has one; its fused
+// form (three stages instead of five) takes half as long again.  In between, for both.
+double tile128_cost(int64_t M, int64_t N, int64_t K, int cus) {
+  const int64_t tiles = (M + 127) / 128 * ((N + 127) / 128);
+  const double load = tiles >= cus / 2 ? 1.0 : (double)tiles / (cus / 2);
+  const double rounds = (double)((tiles + 2 * cus - 1) / (2 * cus));
+  return kLaunchUs + rounds * ((double)((K + 31) / 32) * (0.19 + 0.11 * load) * 1.25 + 1.0);
+}
+
+// The caller's arrival words, if it has brought any.
+uint32_t* arrival_words(const tccl_gemm_desc* d, const tccl_sync_desc* sync) {
+  if (!sync || !(d->flags & TCCL_GEMM_ARRIVALS)) return nullptr;
+  return (uint32_t*)((const tccl_sync_desc_arrivals*)sync)->arrivals;
+}
+
+// The streaming shape to use for this problem, or -1: another kernel is quicker, or the call names things the
+// streaming kernel does not have (a tile, workgroup counts, clock stamps).  Signals need the caller's arrival words.
+// At most one tile per CU: beyond that the larger tiles are about as quick (1000 x 2064 x 1000 in 528 tiles: 17.5 against
+// 13 .. 18 us), and the workgroups of a reduce-scatter that wait for a peer's partials are all resident beside the peer's.
+int stream_shape(const tccl_gemm_desc* d, const tccl_sync_desc* sync, const tccl_transport_desc* tr, int variant, int64_t seg_rows,
+                 const tccl_device_info& dev) {
+  if (d->in_dtype != TCCL_F16 && d->in_dtype != TCCL_BF16) return -1;
+  if (d->out_dtype != TCCL_F32 && d->out_dtype != d->in_dtype) return -1;
+  if (d->macro_tile != 0 || d->num_wgs > 0 || (tr && tr->num_comm_wgs > 0)) return -1;
+  const bool fused = variant != TCCL_S0_BULK;
+  if (fused) {
+    if (!arrival_words(d, sync)) return -1;
+    if (sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock || sync->trace_comm_counter) return -1;
+  }
+  if (use_macro(d, dev, fused)) return -1;
+  int best = -1;
+  double least = tile128_cost(d->M, d->N, d->K, dev.compute_units);
+  for (int i = 0; i < tccl::kStreamShapeCount; ++i) {
+    if (stream_tiles(i, seg_rows, d->M / seg_rows, d->N) > dev.compute_units) continue;
+    const double us = stream_cost(i, d->K);
+    if (us < least) {
+      least = us;
+      best = i;
+    }
+  }
+  return best;
+}
+
+void build_stream(const tccl_gemm_desc* d, const tccl::GemmArgs& g, int64_t seg_rows, const tccl_device_info& dev, tccl::StreamArgs* a) {
+  memset(a, 0, sizeof *a);
+  a->A = d->A;
+  a->B = d->B;
+  a->C = (char*)d->C;
+  a->lda = d->lda;
+  a->ldb = d->ldb;
+  a->ldc = d->ldc;
+  a->M = d->M;
+  a->N = d->N;
+  a->K = d->K;
+  a->alpha = d->alpha;
+  a->out_dtype = d->out_dtype;
+  a->seg_rows = (int)seg_rows;
+  a->wrapped = g.wrap_rows > 0;
+  a->xcds = dev.xcds;
+  a->block_m = g.block_m;
+  a->block_n = g.block_n;
+  a->group_m = g.group_m;
+  a->plan_rows = g.tile_rows;
+  a->plan_cols = g.tile_cols;
+  a->world = 1;
+}
+
+int stream_status(int rc) { return rc == 0 ? 0 : hip_fail((hipError_t)rc, "streaming GEMM launch"); }
+
+// A reduce-scatter launch's own part of the arguments.
+void add_stream_reduce(const tccl::CommArgs& c, const tccl_gemm_desc* d, tccl::StreamArgs* a) {
+  a->heap_bases = c.heap_bases;
+  a->rank = c.rank;
+  a->world = c.world;
+  a->first_seg = (c.rank + 1) % c.world;  // this rank's own rows come last: what its peers wait for comes first
+  tccl::StreamReduce& r = a->reduce;
+  r.active = 1;
+  r.emulate_peer = c.emulate_peer;
+  r.peers_resident = c.peers_resident;
+  r.own_in_registers = (d->flags & TCCL_GEMM_OWN_ROWS_IN_REGISTERS) != 0;
+  r.out_dtype = c.out_dtype;
+  r.out = c.rs_out;
+  r.ld_out_bytes = c.ld_rs_out_bytes;
+  r.locks = c.locks;
+  r.counter = c.counter;
+  r.tile_counts = c.tile_counts;
+  r.fault = c.fault;
+  r.spin_ticks = c.spin_ticks;
+}
+
+int run_stream(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc* sync, int variant, int shape, int64_t seg_rows,
+               const tccl_device_info& dev, const tccl::GemmArgs& g, hipStream_t stream) {
+  tccl::StreamArgs a;
+  build_stream(d, g, seg_rows, dev, &a);
+  const bool kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) != 0;
+  if (variant == TCCL_S0_BULK) {
+    const int rc = stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, nullptr, 0, stream));
+    if (rc || (c.world <= 1 && c.op != tccl::kOpReduceScatter)) return rc;
+    return launch_bulk(c, dev, stream);
+  }
+  a.heap_bases = c.heap_bases;
+  a.rank = c.rank;
+  a.world = c.world;
+  a.arrivals = arrival_words(d, sync);
+  a.s.epoch = sync->epoch > 0 ? sync->epoch : 1;
+  if (variant == TCCL_S1_TILE) {
+    a.s.mode = tccl::kSignalTile;
+    a.s.locks = sync->locks;
+    c.granularity = tccl::kPerTile;
+  } else {
+    a.s.mode = tccl::kSignalGroup;
+    a.s.counter = sync->counter;
+    a.s.group_table = sync->group_table;
+    c.granularity = tccl::kPerGroup;
+  }
+  if (c.op == tccl::kOpReduceScatter) {
+    add_stream_reduce(c, d, &a);
+    return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, nullptr, 0, stream));
+  }
+  if (build_push(c, g, &a.push)) c.directions &= ~tccl::kDirPush;
+  if (c.op != tccl::kOpAllGather || !(c.directions & tccl::kDirPull) || c.world <= 1)
+    return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, nullptr, 0, stream));
+  // The pulls, in tasks small enough that every communication workgroup has one.
+  int tasks = (c.world - 1) * g.tile_rows * g.tile_cols;
+  if (c.granularity == tccl::kPerGroup) {
+    const int64_t units = (int64_t)c.M * c.N * c.esize / 16 * (c.world - 1);
+    int64_t per = (units + dev.compute_units - 1) / dev.compute_units;
+    per = (per + 255) / 256 * 256;
+    if (per < c.copy_units) c.copy_units = (int)per;
+    tasks = (int)((units + c.copy_units - 1) / c.copy_units);
+  }
+  const int wgs = tasks < dev.compute_units ? tasks : dev.compute_units;
+  return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, &c, wgs, stream));
+}
+
 // GEMM (+ optional communication role) for one of the three operations.
 int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc* sync, const tccl_transport_desc* tr,
                 int variant, const tccl_device_info& dev, const tccl::GemmArgs& g, hipStream_t stream,
                 const GatherSpec* gather = nullptr, const tccl_heap_view* heap = nullptr) {
   const int span = c.op != tccl::kOpNone ? check_comm_span(c) : 0;
   if (span) return span;
+  if (!gather) {
+    // Tiles of a reduce-scatter must not straddle two owners' rows.
+    const int64_t seg = g.wrap_rows > 0 ? g.wrap_rows : (c.op == tccl::kOpReduceScatter ? d->M / c.world : d->M);
+    const int shape = stream_shape(d, sync, tr, variant, seg, dev);
+    if (shape >= 0) return run_stream(d, c, sync, variant, shape, seg, dev, g, stream);
+  }
   const int total_tiles = g.tile_rows * g.tile_cols;
   const int compute = default_gemm_wgs(d, dev, total_tiles);
   tccl::SignalArgs s;
@@ -1066,6 +1231,13 @@ int tccl_gemm(const tccl_gemm_desc* d, void* stream) {
   if ((rc = query_device(-1, &dev))) return rc;
   tccl::GemmArgs g;
   build_gemm_args(d, dev, &g);
+  const int64_t seg = g.wrap_rows > 0 ? g.wrap_rows : d->M;
+  const int shape = stream_shape(d, nullptr, nullptr, TCCL_S0_BULK, seg, dev);
+  if (shape >= 0) {
+    tccl::StreamArgs a;
+    build_stream(d, g, seg, dev, &a);
+    return stream_status(tccl::launch_stream(d->in_dtype, g.b_kmajor != 0, shape, a, nullptr, 0, (hipStream_t)stream));
+  }
   tccl::SignalArgs s;
   memset(&s, 0, sizeof s);
   if (use_macro(d, dev, false)) {
@@ -1539,7 +1711,9 @@ int tccl_gemm_allgather_static(const tccl_gemm_desc* d, void* out, int64_t ld_ou
   sync.epoch = epoch;
   sync.fault = fault;
   sync.spin_limit_ns = spin_limit_ns;
-  return allgather_impl(d, out, ld_out, heap, &sync, tr, variant, (int64_t)sizeof(StaticWords), (hipStream_t)stream);
+  tccl_gemm_desc own = *d;
+  own.flags &= ~TCCL_GEMM_ARRIVALS;  // `sync` is this function's
+  return allgather_impl(&own, out, ld_out, heap, &sync, tr, variant, (int64_t)sizeof(StaticWords), (hipStream_t)stream);
 }
 
 int tccl_static_call_words(uint32_t call, int32_t tile_count, int32_t* epoch, int32_t* counter_start, int32_t* counter_ready) {
@@ -1588,17 +1762,55 @@ int tccl_static_reset(void* stream) {
   return tccl_fill_i32((int32_t*)sc->words, (int64_t)(sizeof(sc->words) / sizeof(int32_t)), 0, stream);
 }
 
+// Column shards of M rows that are no whole plan tiles: no signals, so the peers' partials have to be there.
+static int reduce_ragged_shards(const tccl_gemm_desc* d, void* out, int32_t out_dtype, int64_t ld_out, const tccl_heap_view* heap,
+                                const tccl_sync_desc* sync, const tccl_transport_desc* tr, int32_t mode, hipStream_t stream) {
+  if (!(mode & TCCL_RS_PEERS_RESIDENT))
+    return fail(TCCL_ERR_INVALID, "reducescatter: column shards of %d rows carry no signals (plan tiles have %d rows): the peers must be resident",
+                d->M / d->column_shards, d->block_m);
+  tccl_device_info dev;
+  int rc = query_device(-1, &dev);
+  if (rc) return rc;
+  tccl::GemmArgs g;
+  build_gemm_args(d, dev, &g);
+  tccl::CommArgs c;
+  fill_comm_common(&c, g, (int)dtype_size(d->out_dtype), heap, sync, tr);
+  if ((rc = fill_reduce(&c, d->C, d->out_dtype, out, out_dtype, ld_out, d->M, d->N, heap->world_size, mode))) return rc;
+  if ((rc = check_task_elems(tr, true, c.esize)) || (rc = check_comm_span(c))) return rc;
+  const int shape = stream_shape(d, nullptr, tr, TCCL_S0_BULK, g.wrap_rows, dev);
+  if (shape >= 0) {
+    tccl::StreamArgs a;
+    build_stream(d, g, g.wrap_rows, dev, &a);
+    add_stream_reduce(c, d, &a);
+    return stream_status(tccl::launch_stream(d->in_dtype, g.b_kmajor != 0, shape, a, nullptr, 0, stream));
+  }
+  // One GEMM per column block, then the reduction.
+  const size_t isz = dtype_size(d->in_dtype);
+  for (int q = 0; q < d->column_shards; ++q) {
+    tccl_gemm_desc one = *d;
+    one.M = g.wrap_rows;
+    one.column_shards = 0;
+    one.B = (const char*)d->B + (int64_t)q * d->N * (g.b_kmajor ? d->ldb : 1) * (int64_t)isz;
+    one.C = (char*)d->C + (int64_t)q * g.wrap_rows * d->ldc * c.esize;
+    if ((rc = tccl_gemm(&one, stream))) return rc;
+  }
+  return launch_bulk(c, dev, stream);
+}
+
 int tccl_gemm_reducescatter(const tccl_gemm_desc* d, void* out, int32_t out_dtype, int64_t ld_out,
                             const tccl_heap_view* heap, const tccl_sync_desc* sync, const tccl_transport_desc* tr,
                             int32_t emulate_peer, int32_t variant, void* stream) {
-  int rc = check_gemm(d);
+  int rc = check_gemm(d, true);
   if (rc) return rc;
   if ((rc = check_heap(heap))) return rc;
   if (variant < TCCL_S0_BULK || variant > TCCL_S2_TILEGROUP) return fail(TCCL_ERR_INVALID, "unknown variant %d", variant);
-  if ((rc = check_sync(sync, variant))) return rc;
   if (!out || ld_out < d->N) return fail(TCCL_ERR_INVALID, "reducescatter: bad output");
   const int esize = (int)dtype_size(d->out_dtype);
   const int shard = d->M / heap->world_size;
+  const bool ragged = d->column_shards == heap->world_size && d->M % heap->world_size == 0 && shard % d->block_m;
+  if (!ragged && (rc = check_sync(sync, variant))) return rc;
+  if (ragged)
+    return reduce_ragged_shards(d, out, out_dtype, ld_out, heap, sync, tr, emulate_peer, (hipStream_t)stream);
   if (d->M % heap->world_size || shard % d->block_m)
     return fail(TCCL_ERR_INVALID, "reducescatter: M=%d must split into world_size=%d shards of whole %d-row plan tiles", d->M, heap->world_size, d->block_m);
   tccl_device_info dev;

@@ -1,0 +1,444 @@
+// Streaming MFMA GEMM for gfx950 (CDNA4), 16-bit inputs: small outputs, where the large-tile kernels leave
+// most of the device idle (decoding rows, short prompts, ragged and narrow problems).
+//
+// One workgroup produces one output tile of (16 kMB) x (16 kNB); its kWaves wavefronts each take every
+// kWaves-th K block of 64 for the WHOLE tile, straight from memory into the operand registers of
+// v_mfma_f32_16x16x32 (no LDS and no barrier in the K loop), and add their accumulators up through LDS at the
+// end.  So a tile of 16 rows of a 4096-deep product is sixteen chains of four K blocks, all requested at once,
+// instead of one chain of 128 K steps.  Measured, bf16, 16 x 2048 x 4096: 7.3 us with a k-major B and 11.5 us row-major
+// against 29 us on the 128 x 128-tile kernel, whose 16 tiles keep 16 CUs busy (40 us in its fused form);
+// 1024 x 1024 x 2048: 12.4 against 20.8 us; an empty launch takes 3.7 us of that.
+//
+// What bounds it: the vector memory path of a CU delivers about 85 KB/us of operands here, and each operand
+// byte of a tile passes it once, (kMB + kNB) * 2 KiB per 64 k; tiles are as large as the output allows while
+// every CU still gets one (stream_shape() in tccl_api.hip).  A row-major B is slower because a narrow tile reads
+// 32 to 128 bytes of each k row.
+#pragma once
+
+#include "tccl_comm.h"
+#include "tccl_gemm.h"
+
+namespace tccl {
+
+// Epilogue of a reduce-scatter: see ReduceArgs of tccl_gemm256.h for the meaning of the members.
+struct StreamReduce {
+  int active, emulate_peer, peers_resident, own_in_registers;
+  int out_dtype;
+  char* out;
+  int64_t ld_out_bytes;
+  const int32_t* locks;
+  const int32_t* counter;
+  const int32_t* tile_counts;
+  int64_t* fault;
+  int64_t spin_ticks;
+};
+
+struct StreamArgs {
+  const void* A;
+  const void* B;
+  char* C;
+  int64_t lda, ldb, ldc;  // elements
+  int M, N, K;            // C is M x N
+  float alpha;
+  int out_dtype;
+  // Rows come in segments (the owners' shards of a reduce-scatter, stacked column shards); tiles do not straddle
+  // them.  `wrapped`: segment q is A (seg_rows x K) times columns [q N, (q + 1) N) of B.
+  int seg_rows, wrapped;
+  int first_seg;                   // segments are visited from this one on, wrapping around
+  int tiles_m, tiles_n, total;     // tiles per segment, along the columns, in all
+  int xcds, per_xcd;               // XCD x works on tiles [x per_xcd, (x + 1) per_xcd): neighbours share a slab of B in its L2
+  // Signals: a plan tile is published when the last of its tiles has been stored.
+  SignalArgs s;
+  uint32_t* arrivals;              // one per plan tile, zero between launches
+  int block_m, block_n, group_m, plan_rows, plan_cols;
+  const int64_t* heap_bases;
+  int rank, world;
+  PushArgs push;
+  StreamReduce reduce;
+};
+
+#if defined(__HIP_DEVICE_COMPILE__)
+template <typename InT, int kMB, int kNB, int kWaves, bool kBKMajor>
+struct StreamGemm {
+  typedef typename Mfma<InT>::Vec Vec;
+  static_assert(sizeof(InT) == 2, "16-bit inputs");
+  static constexpr int kBM = 16 * kMB, kBN = 16 * kNB;
+  // K blocks of 64 in flight per wavefront, within the registers that kWaves wavefronts leave each.
+  static constexpr int kBudget = (kWaves >= 16 ? 64 : 128) / ((kMB + kNB) * 8);
+  static constexpr int kDepth = kBudget < 1 ? 1 : (kBudget > 4 ? 4 : kBudget);
+  static constexpr int kSlots = kMB * kNB;            // accumulator quads per lane
+  // LDS of a wavefront: one K block on its way from load order to operand order, then its sums.
+  static constexpr int kStagedBlocks = kMB + kNB;
+  static constexpr int kWaveBytes = kStagedBlocks * 2048 > kSlots * 1024 ? kStagedBlocks * 2048 : kSlots * 1024;
+  static constexpr int kPitch = kBN * 4 + 16;         // bytes of a row of sums
+  static constexpr int kRowsBytes = kBM * kPitch;
+  static constexpr int kLdsBytes = kWaves * kWaveBytes > kRowsBytes ? kWaves * kWaveBytes : kRowsBytes;
+
+  const StreamArgs& a;
+  char* lds;
+  const int lane, wave;
+
+  TCCL_D StreamGemm(const StreamArgs& args, char* l)
+      : a(args), lds(l), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) {}
+
+  static TCCL_D uint32_t clamp_u32(int64_t v) { return v > 0xfffffff0ll ? 0xfffffff0u : (v < 0 ? 0u : (uint32_t)v); }
+
+  // One K block of 64 as it is loaded, 16 bytes per lane with neighbouring lanes on neighbouring addresses (a
+  // load whose lanes 0..3 lie in four rows takes in a third of the bytes per clock: 34 against 104 KB/us per CU).
+  //   A, k-major B: rows of 128 bytes; instruction h of a 16-row block covers its rows 8 h + l / 8, chunk l % 8.
+  //   Row-major B: 64 k rows of 32 kNB bytes; instruction h covers rows h * kRowsPerLoad + l / (2 kNB).
+  struct Block {
+    u32x4 a[2 * kMB], b[2 * kNB];
+  };
+  static constexpr int kRowsPerLoad = 32 / kNB;
+  static constexpr uint32_t kOutside = 0xffffff00u;  // beyond every buffer: reads as zero
+
+  __amdgpu_buffer_rsrc_t ra, rb;
+  uint32_t off_a, off_b, pitch_a, pitch_b;  // this lane's offset in K block 0; bytes per row
+  int kg, i16;
+
+  // kTail: the block may reach past K; a chunk, or a row of B, at k >= K reads as zero.
+  template <bool kTail>
+  TCCL_D void load(Block& v, int kb) const {
+    const bool past = kTail && kb * 64 + 8 * (lane & 7) >= a.K;
+#pragma unroll
+    for (int h = 0; h < 2 * kMB; ++h) {
+      const uint32_t o = off_a + (uint32_t)(8 * h) * pitch_a + (uint32_t)kb * 128u;
+      v.a[h] = __builtin_amdgcn_raw_buffer_load_b128(ra, past ? kOutside : o, 0, 0);
+    }
+#pragma unroll
+    for (int h = 0; h < 2 * kNB; ++h) {
+      if constexpr (kBKMajor) {
+        const uint32_t o = off_b + (uint32_t)(8 * h) * pitch_b + (uint32_t)kb * 128u;
+        v.b[h] = __builtin_amdgcn_raw_buffer_load_b128(rb, past ? kOutside : o, 0, 0);
+      } else {
+        const int k = kb * 64 + h * kRowsPerLoad;  // and the lane's row
+        const bool none = off_b == kOutside || (kTail && k + lane / (2 * kNB) >= a.K);
+        v.b[h] = __builtin_amdgcn_raw_buffer_load_b128(rb, none ? kOutside : off_b + (uint32_t)k * pitch_b, 0, 0);
+      }
+    }
+  }
+
+  // Load order -> operand order through this wavefront's own LDS (a wavefront's LDS operations execute in the
+  // order issued: no barrier).
+  //   Rows of 128 bytes: chunk c of row r in slot c ^ ((r >> 1) & 7), read with ds_read_b128.
+  //   Row-major B: the 32-byte units of k row k permuted by swizzle(k), so that the eight rows that 32 lanes of a
+  //   transposing read (ds_read_b64_tr_b16) touch at a time lie in different banks.
+  static TCCL_D int swizzle(int k) {
+    if constexpr (kNB >= 8) return (2 * (k & 3)) ^ ((k >> 3) & 1);
+    if constexpr (kNB == 4) return (k & 2) ^ ((k >> 3) & 1);
+    return kNB == 2 ? (k >> 3) & 1 : 0;
+  }
+  static TCCL_D int row_at(int k) { return kNB == 1 ? k ^ (4 * ((k >> 3) & 1)) : k; }
+  TCCL_D void stage(const Block& v) const {
+    char* at = lds + wave * kWaveBytes;
+#pragma unroll
+    for (int h = 0; h < 2 * kMB; ++h) {
+      const int r = 8 * h + (lane >> 3);
+      *(u32x4*)(at + r * 128 + (((lane & 7) ^ ((r >> 1) & 7)) << 4)) = v.a[h];
+    }
+    at += kMB * 2048;
+#pragma unroll
+    for (int h = 0; h < 2 * kNB; ++h) {
+      if constexpr (kBKMajor) {
+        const int r = 8 * h + (lane >> 3);
+        *(u32x4*)(at + r * 128 + (((lane & 7) ^ ((r >> 1) & 7)) << 4)) = v.b[h];
+      } else {
+        const int k = h * kRowsPerLoad + lane / (2 * kNB), c = lane % (2 * kNB);
+        *(u32x4*)(at + row_at(k) * (32 * kNB) + ((c ^ (2 * swizzle(k))) << 4)) = v.b[h];
+      }
+    }
+  }
+  // Operand of 16-row block `block` (A, k-major B), 32-k half h: lane l holds k 8 (l / 16) .. + 7 of row l % 16.
+  TCCL_D Vec staged(int block, int h) const {
+    return *(const Vec*)(lds + wave * kWaveBytes + block * 2048 + i16 * 128 + (((4 * h + kg) ^ ((i16 >> 1) & 7)) << 4));
+  }
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(3))) s16x4 LdsQuad;
+  // Column block j of row-major B: two transposing reads (k rows 8 kg + 0 .. 3 and + 4 .. 7).
+  TCCL_D Vec turned(int j, int h) const {
+    const int t = i16 >> 2, cq = i16 & 3;
+    const char* at = lds + wave * kWaveBytes + kMB * 2048;
+    s16x4 half[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int k = 32 * h + 8 * kg + 4 * q + t;
+      const char* p = at + row_at(k) * (32 * kNB) + (((2 * j + (cq >> 1)) ^ (2 * swizzle(k))) << 4) + (cq & 1) * 8;
+      half[q] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)p);
+    }
+    const s16x8 both = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(Vec, both);
+  }
+
+  TCCL_D void multiply(f32x4 (&acc)[kMB][kNB]) const {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      Vec fa[kMB], fb[kNB];
+#pragma unroll
+      for (int j = 0; j < kNB; ++j) {
+        if constexpr (kBKMajor)
+          fb[j] = staged(kMB + j, h);
+        else
+          fb[j] = turned(j, h);
+      }
+#pragma unroll
+      for (int i = 0; i < kMB; ++i) fa[i] = staged(i, h);
+#pragma unroll
+      for (int i = 0; i < kMB; ++i)
+#pragma unroll
+        for (int j = 0; j < kNB; ++j) acc[i][j] = Mfma<InT>::run16(fb[j], fa[i], acc[i][j]);
+    }
+  }
+
+  TCCL_D void refill(Block& v, int kb, int whole, int blocks) const {
+    if (kb < whole)
+      load<false>(v, kb);
+    else if (kb < blocks)
+      load<true>(v, kb);
+  }
+
+  TCCL_D void k_loop(f32x4 (&acc)[kMB][kNB]) const {
+    const int blocks = (a.K + 63) / 64, whole = a.K / 64;
+    Block v[kDepth];
+    // This wavefront's blocks are wave, wave + kWaves, ...; the last one of all may be a partial one.
+    int next = wave;
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d, next += kWaves) refill(v[d], next, whole, blocks);
+    for (int kb = wave; kb < blocks;) {
+#pragma unroll
+      for (int d = 0; d < kDepth; ++d) {
+        if (kb < blocks) {
+          stage(v[d]);
+          refill(v[d], next, whole, blocks);  // the block is in LDS: its registers are free
+          multiply(acc);
+          kb += kWaves;
+          next += kWaves;
+        }
+      }
+    }
+  }
+
+  TCCL_D void run(int slot) {
+    int tile = slot;
+    if (a.xcds > 1) tile = (slot % a.xcds) * a.per_xcd + slot / a.xcds;
+    if (tile >= a.total) return;
+    // Row tiles of one segment run fastest: the tiles that share a column slab of B sit on one XCD.
+    const int per_seg = a.tiles_m * a.tiles_n;
+    int seg = tile / per_seg;
+    const int in = tile - seg * per_seg;
+    const int tn = in / a.tiles_m, tm = in - tn * a.tiles_m;
+    const int segs = a.total / per_seg;
+    seg += a.first_seg;
+    if (seg >= segs) seg -= segs;
+    const int row_in = tm * kBM, col0 = tn * kBN;  // relative to the segment
+    const int row0 = seg * a.seg_rows + row_in;    // row of C
+
+    i16 = lane & 15;
+    kg = lane >> 4;
+    const int a_row = a.wrapped ? row_in : row0, a_rows = a.wrapped ? a.seg_rows : a.M;
+    const int64_t b_col = (a.wrapped ? (int64_t)seg * a.N : 0) + col0;
+    pitch_a = (uint32_t)(a.lda * 2);
+    pitch_b = (uint32_t)(a.ldb * 2);
+    const InT* A = (const InT*)a.A + (int64_t)a_row * a.lda;
+    ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(((int64_t)(a_rows - 1 - a_row) * a.lda + a.K) * 2), 0x00020000);
+    off_a = (uint32_t)(lane >> 3) * pitch_a + (uint32_t)(lane & 7) * 16u;
+    const int cols_left = a.N - col0;  // columns of this segment from col0 on
+    if constexpr (kBKMajor) {
+      const InT* B = (const InT*)a.B + b_col * a.ldb;
+      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(cols_left - 1) * a.ldb + a.K) * 2), 0x00020000);
+      off_b = (uint32_t)(lane >> 3) * pitch_b + (uint32_t)(lane & 7) * 16u;
+    } else {
+      const InT* B = (const InT*)a.B + b_col;
+      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(a.K - 1) * a.ldb + cols_left) * 2), 0x00020000);
+      const int c = lane % (2 * kNB);
+      off_b = 8 * c < cols_left ? (uint32_t)(lane / (2 * kNB)) * pitch_b + (uint32_t)c * 16u : kOutside;
+    }
+
+    f32x4 acc[kMB][kNB];
+#pragma unroll
+    for (int i = 0; i < kMB; ++i)
+#pragma unroll
+      for (int j = 0; j < kNB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    k_loop(acc);
+
+    // The wavefronts' accumulators are added up through LDS ([slot][lane] of each, conflict-free) and the sums
+    // staged as rows, from which every thread takes chunks of 8 columns.
+#pragma unroll
+    for (int i = 0; i < kMB; ++i)
+#pragma unroll
+      for (int j = 0; j < kNB; ++j) *(f32x4*)(lds + wave * kWaveBytes + ((i * kNB + j) * 64 + lane) * 16) = acc[i][j];
+    __syncthreads();
+    constexpr int kMine = (kSlots + kWaves - 1) / kWaves;
+    f32x4 sum[kMine];
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) {
+      const int slot_no = wave + m * kWaves;
+      if (slot_no < kSlots) {
+        sum[m] = *(const f32x4*)(lds + (slot_no * 64 + lane) * 16);
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) {
+          const f32x4 x = *(const f32x4*)(lds + w * kWaveBytes + (slot_no * 64 + lane) * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[m][e] += x[e];
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) {
+      const int slot_no = wave + m * kWaves;
+      if (slot_no < kSlots) {
+        const int i = slot_no / kNB, j = slot_no % kNB;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[m][e] *= a.alpha;
+        *(f32x4*)(lds + (16 * i + i16) * kPitch + (16 * j + 4 * kg) * 4) = sum[m];
+      }
+    }
+    __syncthreads();
+    const bool coherent = a.s.mode != kSignalNone;
+    const int owner = seg;
+    bool ok = true;
+    if (a.reduce.active && (owner == a.rank || a.reduce.emulate_peer) && !a.reduce.peers_resident) ok = wait_for_peers(row0, col0);
+    constexpr int kChunksPerRow = kBN / 8, kChunks = kBM * kChunksPerRow;
+    for (int c = (int)threadIdx.x; c < kChunks; c += kWaves * 64) {
+      const int row = c / kChunksPerRow, col = c % kChunksPerRow * 8;
+      if (row_in + row >= a.seg_rows || col0 + col >= a.N) continue;
+      float f[8];
+      const f32x4 lo = *(const f32x4*)(lds + row * kPitch + col * 4), hi = *(const f32x4*)(lds + row * kPitch + col * 4 + 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[e] = lo[e];
+        f[4 + e] = hi[e];
+      }
+      finish(f, owner, row_in, row0, col0, row, col, coherent, ok);
+    }
+    publish(row0, col0);
+  }
+
+  TCCL_D static void put(__amdgpu_buffer_rsrc_t w, uint32_t off, const float (&f)[8], int dtype, bool coherent) {
+    if (coherent) {
+      if (dtype == kF16)
+        store8<_Float16, kCoherent>(w, off, f);
+      else if (dtype == kBF16)
+        store8<__bf16, kCoherent>(w, off, f);
+      else
+        store8<float, kCoherent>(w, off, f);
+    } else {
+      if (dtype == kF16)
+        store8<_Float16, 0>(w, off, f);
+      else if (dtype == kBF16)
+        store8<__bf16, 0>(w, off, f);
+      else
+        store8<float, 0>(w, off, f);
+    }
+  }
+  TCCL_D static void get(__amdgpu_buffer_rsrc_t w, uint32_t off, float (&f)[8], int dtype) {
+    if (dtype == kF16)
+      Load8<_Float16, kCoherent>::run(w, off, f);
+    else if (dtype == kBF16)
+      Load8<__bf16, kCoherent>::run(w, off, f);
+    else
+      Load8<float, kCoherent>::run(w, off, f);
+  }
+
+  // One chunk of 8 columns: to C, to the peers, or into the reduction.
+  TCCL_D void finish(float (&f)[8], int owner, int row_in, int row0, int col0, int row, int col, bool coherent, bool ok) const {
+    const int esz = a.out_dtype == kF32 ? 4 : 2;
+    const int64_t c_at = (int64_t)(uintptr_t)a.C + ((int64_t)row0 * a.ldc + col0) * esz;
+    const uint32_t off = (uint32_t)((row * a.ldc + col) * esz);
+    const bool reduces = a.reduce.active && (owner == a.rank || a.reduce.emulate_peer) && ok;
+    const bool store = !(a.reduce.active && owner == a.rank && a.reduce.own_in_registers && ok);
+    if (store) put(window(c_at), off, f, a.out_dtype, coherent);
+    for (int t = 0; t < a.push.world; ++t) {
+      const int c = col0 + col;
+      if (t == a.push.rank || c < a.push.col_lo || c >= a.push.col_hi) continue;
+      const int64_t to = (int64_t)(uintptr_t)a.C + (a.heap_bases[t] - a.heap_bases[a.push.rank]) +
+                         ((int64_t)row0 * a.push.ld + col0 + a.push.col_shift) * esz;
+      put(window(to), (uint32_t)((row * a.push.ld + col) * esz), f, a.out_dtype, true);
+    }
+    if (!reduces) return;
+    // The owner's partial first, then the other ranks ascending; this rank's is the value as stored.
+    float mine[8], sum[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mine[e] = a.out_dtype == kF32 ? f[e] : (a.out_dtype == kF16 ? (float)(_Float16)f[e] : (float)(__bf16)f[e]);
+    const int64_t my_base = a.heap_bases[a.rank];
+    for (int i = 0; i < a.world; ++i) {
+      const int p = i == 0 ? owner : (i <= owner ? i - 1 : i);
+      float v[8];
+      if (p == a.rank) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = mine[e];
+      } else {
+        get(window(c_at + (a.heap_bases[p] - my_base)), off, v, a.out_dtype);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum[e] = i == 0 ? v[e] : sum[e] + v[e];
+    }
+    const int64_t out = (int64_t)(uintptr_t)a.reduce.out + (a.heap_bases[owner] - my_base) + (int64_t)row_in * a.reduce.ld_out_bytes + (int64_t)col0 * 2;
+    put(window(out), (uint32_t)(row * a.reduce.ld_out_bytes + col * 2), sum, a.reduce.out_dtype, false);
+  }
+
+  TCCL_D int plan_tile(int row0, int col0) const {
+    return tile_id_of(row0 / a.block_m, col0 / a.block_n, a.plan_rows, a.plan_cols, a.group_m);
+  }
+
+  // The peers' partials of the plan tile under (row0, col0) are published (bounded wait).
+  TCCL_D bool wait_for_peers(int row0, int col0) const {
+    __shared__ int verdict;
+    if (threadIdx.x == 0) {
+      const int tile = plan_tile(row0, col0);
+      const int64_t deadline = now_ticks() + a.reduce.spin_ticks;
+      bool ok = true;
+      for (int p = 0; p < a.world && ok; ++p) {
+        if (p == a.rank) continue;
+        if (a.s.mode == kSignalTile) {
+          ok = tile_wait_ge<true>(translate_ptr(a.reduce.locks, a.rank, p, a.heap_bases), tile, a.s.epoch, deadline);
+        } else {
+          const int g = a.s.group_table[tile];
+          const int32_t need = (int32_t)((uint32_t)a.s.epoch * (uint32_t)a.reduce.tile_counts[g]);
+          ok = tile_wait_ge<true>(translate_ptr(a.reduce.counter, a.rank, p, a.heap_bases), g, need, deadline);
+        }
+      }
+      if (!ok && a.reduce.fault) *a.reduce.fault = 1;
+      verdict = ok ? 1 : 0;
+    }
+    __syncthreads();
+    return verdict != 0;
+  }
+
+  TCCL_D void publish(int row0, int col0) const {
+    if (a.s.mode == kSignalNone) return;
+    wait_vmem();  // this wavefront's write-through stores have landed
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const int tile = plan_tile(row0, col0);
+    // Tiles of this plan tile: those of its rows and columns that lie inside the segment and N.
+    const int pr = row0 / a.block_m * a.block_m, pc = col0 / a.block_n * a.block_n;
+    const int seg0 = row0 / a.seg_rows * a.seg_rows;
+    const int rows = (pr + a.block_m < seg0 + a.seg_rows ? pr + a.block_m : seg0 + a.seg_rows) - pr;
+    const int cols = (pc + a.block_n < a.N ? pc + a.block_n : a.N) - pc;
+    const uint32_t n = (uint32_t)(((rows + kBM - 1) / kBM) * ((cols + kBN - 1) / kBN));
+    // Counts to n - 1 and starts over by itself, so the word is zero again when the launch has ended.
+    const uint32_t before = n > 1 ? atomicInc(&a.arrivals[tile], n - 1) : 0u;
+    if (before != n - 1) return;
+    if (a.s.mode == kSignalTile)
+      tile_publish(a.s.locks, tile, a.s.epoch);
+    else
+      tile_signal_add<true>(a.s.counter, a.s.group_table[tile], 1);
+  }
+};
+#endif  // __HIP_DEVICE_COMPILE__
+
+// Tile shapes that exist (16 mb x 16 nb, wavefronts), smallest first.
+struct StreamShape {
+  int mb, nb, waves;
+};
+constexpr StreamShape kStreamShapes[] = {{1, 1, 16}, {1, 2, 16}, {2, 2, 16}, {2, 4, 8}, {4, 4, 4}};
+constexpr int kStreamShapeCount = (int)(sizeof(kStreamShapes) / sizeof(kStreamShapes[0]));
+
+// Defined in tccl_stream.hip.  Fills in the tile counts and launches; `comm` non-NULL: `comm_wgs` workgroups
+// after the tiles' run the communication role with it (the pulls of an all-gather).  0 or a hipError_t.
+int launch_stream(int in_dtype, bool b_kmajor, int shape, StreamArgs& a, const CommArgs* comm, int comm_wgs, hipStream_t stream);
+
+}  // namespace tccl

@@ -220,8 +220,9 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     fault word if a producer is missing: the mode for ranks that really run side by side and
     have made the same number of calls.
     ``implementation`` is accepted for signature parity; there is one implementation here.
-    When ``M`` is not a multiple of the 128-row plan tile, one GEMM per column block and the
-    bulk reduction run instead.
+    When ``M`` is not a multiple of the 128-row plan tile there are no signals: the peers' partials
+    are taken to be there, in one launch where the streaming kernel is the quicker one and
+    otherwise with one GEMM per column block and the bulk reduction.
     """
     if implementation not in ("auto", "device", "hip"):
         raise ValueError(f"unsupported gemm_reducescatter implementation {implementation!r}")
@@ -238,27 +239,23 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     tall = partial.view(k.world_size * k.M, k.output_cols)  # row block q = the shard rank q owns
     view = _launch.heap_view(ctx.heap_bases, k.rank, k.world_size)
     transport = _launch.transport_desc(_lib.DIR_PULL, 16384, 16384, 0)
+    mode = (_lib.RS_PEERS_RESIDENT if peers_resident else 0) | (_lib.RS_EMULATE_PEERS if emulate_peer else 0)
+    flags = _lib.GEMM_OWN_ROWS_IN_REGISTERS if own_rows_in_registers else 0
+    words, sync = None, None
     if k.M % 128 == 0:
         words = _reduce_scatter_words(ctx, k.world_size, k.M, k.output_cols)
-        gemm = _launch.gemm_desc(A, B, tall, column_shards=k.world_size,
-                                 flags=_lib.GEMM_OWN_ROWS_IN_REGISTERS if own_rows_in_registers else 0)
+        flags |= _lib.GEMM_ARRIVALS
         if variant != "s0":
             words.next_epoch(variant)
         sync = words.desc(variant)
-        mode = (_lib.RS_PEERS_RESIDENT if peers_resident else 0) | (_lib.RS_EMULATE_PEERS if emulate_peer else 0)
-        rc = lib.tccl_gemm_reducescatter(
-            C.byref(gemm), _launch.ptr(Cx), _launch.dtype_code(Cx.dtype), int(Cx.stride(0)), C.byref(view), C.byref(sync),
-            C.byref(transport), mode, _launch.VARIANTS[variant], stream,
-        )
-        _lib.check(rc, f"tccl_gemm_reducescatter[{variant}]")
-        ctx.__dict__["_reduce_scatter_last_words"] = words
-        return Cx
-    for q in range(k.world_size):
-        cols = B[:, q * k.output_cols:(q + 1) * k.output_cols]
-        _lib.check(lib.tccl_gemm(C.byref(_launch.gemm_desc(A, cols, partial[q])), stream), "tccl_gemm")
-    rc = lib.tccl_reduce_rows(
-        _launch.ptr(tall), _launch.dtype_code(tall.dtype), int(tall.stride(0)), _launch.ptr(Cx), _launch.dtype_code(Cx.dtype),
-        int(Cx.stride(0)), int(tall.shape[0]), int(tall.shape[1]), C.byref(view), C.byref(transport), int(emulate_peer), stream,
+    else:  # no whole plan tiles: one launch (or a GEMM per column block and a reduction) without signals
+        mode |= _lib.RS_PEERS_RESIDENT
+    gemm = _launch.gemm_desc(A, B, tall, column_shards=k.world_size, flags=flags)
+    rc = lib.tccl_gemm_reducescatter(
+        C.byref(gemm), _launch.ptr(Cx), _launch.dtype_code(Cx.dtype), int(Cx.stride(0)), C.byref(view), _launch.byref(sync),
+        C.byref(transport), mode, _launch.VARIANTS[variant], stream,
     )
-    _lib.check(rc, "tccl_reduce_rows")
+    _lib.check(rc, f"tccl_gemm_reducescatter[{variant}]")
+    if words is not None:
+        ctx.__dict__["_reduce_scatter_last_words"] = words
     return Cx

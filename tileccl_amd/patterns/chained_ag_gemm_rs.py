@@ -96,7 +96,8 @@ class ChainedAGGemmRSPattern:
             raise ValueError(f"gathered_workspace must be ({M}, {K}) of {input_shard.dtype}")
 
         gemm = _launch.gemm_desc(
-            gathered_workspace, W, output, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self._stage.GROUP_M
+            gathered_workspace, W, output, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self._stage.GROUP_M,
+            flags=_lib.GEMM_ARRIVALS,
         )
         view = _launch.heap_view(self.ctx.heap_bases, self.ctx.rank, world_size)
         compute_wgs, comm_wgs = self._stage._wg_split()

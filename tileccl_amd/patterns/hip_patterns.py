@@ -76,7 +76,8 @@ class _HipAllScatterPattern(Pattern):
             )
         compute_wgs, comm_wgs = self._wg_split()
         gemm = _launch.gemm_desc(
-            A, B, C_out, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self.GROUP_M, num_wgs=compute_wgs
+            A, B, C_out, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self.GROUP_M, num_wgs=compute_wgs,
+            flags=_lib.GEMM_ARRIVALS,
         )
         scatter = _lib.ScatterDesc(
             spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset

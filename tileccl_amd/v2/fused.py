@@ -181,7 +181,7 @@ class FusedGemmAllGather(_FusedBase):
         alpha = float(alpha) * float(scale_a) * float(scale_b)  # per-tensor dequantisation scales of fp8 inputs
         gemm = _launch.gemm_desc(
             A, B, self.local_block, block_m=self.block_m, block_n=self.block_n, group_m=self.group_m,
-            alpha=alpha, num_wgs=self.num_gemm_wgs, macro_tile=self.macro_tile,
+            alpha=alpha, num_wgs=self.num_gemm_wgs, macro_tile=self.macro_tile, flags=_lib.GEMM_ARRIVALS,
         )
         view, transport, sync = self._descs(self.directions, variant)
         rc = _lib.load().tccl_gemm_allgather(
@@ -235,7 +235,7 @@ class FusedGemmReduceScatter(_FusedBase):
         gemm = _launch.gemm_desc(
             A, B, self.partial, block_m=self.block_m, block_n=self.block_n, group_m=self.group_m,
             alpha=alpha, num_wgs=self.num_gemm_wgs, macro_tile=self.macro_tile,
-            flags=_lib.GEMM_OWN_ROWS_IN_REGISTERS if self.own_rows_in_registers else 0,
+            flags=_lib.GEMM_ARRIVALS | (_lib.GEMM_OWN_ROWS_IN_REGISTERS if self.own_rows_in_registers else 0),
         )
         view, transport, sync = self._descs(_lib.DIR_PULL, variant)
         rc = _lib.load().tccl_gemm_reducescatter(
