@@ -113,10 +113,21 @@ def pack_operand(t: torch.Tensor, rows: int, cols: int, role: str) -> torch.Tens
     return out
 
 
-def gemm_operands(A: torch.Tensor, B: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, int, int, int, int]:
-    """(A, B, K, lda, ldb, flag bits) as the kernels read them.  An operand they can address in place
-    (16-byte row vectors: A with contiguous rows, B with contiguous rows or columns, K a whole number
-    of vectors) is passed through; any other layout the reference's pointer arithmetic accepts
+@dataclass(frozen=True, slots=True)
+class OperandPlan:
+    """How the kernels read A and B of one layout: in place, or from packed copies."""
+
+    pack_a: bool
+    pack_b: bool
+    K: int  # zero-filled up to whole 16-byte vectors where an operand is packed
+    lda: int
+    ldb: int
+    b_flags: int
+
+
+def operand_plan(A: torch.Tensor, B: torch.Tensor) -> OperandPlan:
+    """An operand the kernels can address in place (16-byte row vectors: A with contiguous rows, B with contiguous rows
+    or columns, K a whole number of vectors) is passed through; any other layout the reference's pointer arithmetic accepts
     (``/root/reference/tileccl/kernels/gemm.py:63-66,139-151``: a transposed A, strided slices, odd K)
     is packed into a dense buffer first, K zero-filled up to the next whole vector, which adds exact zeros
     to every dot product."""
@@ -129,16 +140,29 @@ def gemm_operands(A: torch.Tensor, B: torch.Tensor) -> tuple[torch.Tensor, torch
     vec = _vector_elems(A)
     k_pad = (K + vec - 1) // vec * vec
     lda = int(A.stride(0)) if M > 1 else int(K)
-    if k_pad != K or (K > 1 and A.stride(1) != 1) or lda < K or not _rows_vectorised(A, lda):
-        A, lda = pack_operand(A, M, k_pad, "A"), k_pad
+    pack_a = k_pad != K or (K > 1 and A.stride(1) != 1) or lda < K or not _rows_vectorised(A, lda)
     layout = _b_layout(B) if k_pad == K else None
-    if layout is None:
-        N = B.shape[1]
-        B, layout = pack_operand(B, k_pad, N, "B"), (N, 0)
-    return A, B, k_pad, lda, layout[0], layout[1]
+    ldb, flags = layout or (int(B.shape[1]), 0)
+    return OperandPlan(pack_a, layout is None, int(k_pad), k_pad if pack_a else lda, ldb, flags)
 
 
-def gemm_desc(
+def planned_operands(plan: OperandPlan, A: torch.Tensor, B: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """(A, B) with the operands that ``plan`` says so packed on the current stream."""
+    if plan.pack_a:
+        A = pack_operand(A, A.shape[0], plan.K, "A")
+    if plan.pack_b:
+        B = pack_operand(B, plan.K, B.shape[1], "B")
+    return A, B
+
+
+def gemm_operands(A: torch.Tensor, B: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, int, int, int, int]:
+    """(A, B, K, lda, ldb, flag bits) as the kernels read them (``operand_plan``), packed where need be."""
+    plan = operand_plan(A, B)
+    A, B = planned_operands(plan, A, B)
+    return A, B, plan.K, plan.lda, plan.ldb, plan.b_flags
+
+
+def _gemm_desc(
     A: torch.Tensor,
     B: torch.Tensor,
     C_out: torch.Tensor,
@@ -151,7 +175,8 @@ def gemm_desc(
     macro_tile: int = 0,
     flags: int = 0,
     column_shards: int = 0,
-) -> _lib.GemmDesc:
+) -> tuple[_lib.GemmDesc, OperandPlan]:
+    """The descriptor without its operands' addresses, and how those are to be read."""
     if not (A.is_cuda and B.is_cuda and C_out.is_cuda):
         raise ValueError("GEMM operands must be device tensors")
     if A.dtype != B.dtype:
@@ -166,20 +191,96 @@ def gemm_desc(
         M, N = M * column_shards, N // column_shards
     if tuple(C_out.shape) != (M, N):
         raise ValueError(f"C shape mismatch: expected ({M}, {N}), got {tuple(C_out.shape)}")
-    A, B, K, lda, ldb, b_flags = gemm_operands(A, B)
+    plan = operand_plan(A, B)
     d = _lib.GemmDesc()
-    d.operands = (A, B)  # a packed operand lives as long as the descriptor
-    d.A, d.B, d.C = ptr(A), ptr(B), ptr(C_out)
-    d.M, d.N, d.K = int(M), int(N), int(K)
-    d.lda, d.ldb, d.ldc = lda, ldb, _row_major(C_out, "C")
+    d.C = ptr(C_out)
+    d.M, d.N, d.K = int(M), int(N), plan.K
+    d.lda, d.ldb, d.ldc = plan.lda, plan.ldb, _row_major(C_out, "C")
     d.in_dtype, d.out_dtype = dtype_code(A.dtype), dtype_code(C_out.dtype)
     d.alpha = float(alpha)
     d.block_m, d.block_n, d.group_m = int(block_m), int(block_n), int(group_m)
     d.num_wgs = int(num_wgs)
     d.macro_tile = int(macro_tile)
-    d.flags = int(flags) | b_flags
+    d.flags = int(flags) | plan.b_flags
     d.column_shards = int(column_shards)
+    return d, plan
+
+
+def gemm_desc(A: torch.Tensor, B: torch.Tensor, C_out: torch.Tensor, **how) -> _lib.GemmDesc:
+    """The descriptor of ``C_out = A @ B`` (keywords: ``_gemm_desc``), operands packed where need be."""
+    d, plan = _gemm_desc(A, B, C_out, **how)
+    A, B = planned_operands(plan, A, B)
+    d.operands = (A, B)  # a packed operand lives as long as the descriptor
+    d.A, d.B = ptr(A), ptr(B)
     return d
+
+
+def layout_key(t: torch.Tensor) -> tuple:
+    """Everything about a tensor that a descriptor depends on, except where it lies."""
+    return t.shape, t.stride(), t.dtype, t.device, t.data_ptr() & 15
+
+
+class BoundCall:
+    """One fused operation on tensors of one layout: the descriptors are built and checked once, a call fills in the
+    addresses, the launch number and the stream.  Not shared between threads while it runs (``CallCache``)."""
+
+    __slots__ = ("gemm", "plan", "words", "sync", "variant", "fn", "args", "what", "keep")
+
+    def __init__(self, gemm: _lib.GemmDesc, plan: OperandPlan, words: "SyncWords | None", variant: str, fn, args, what: str, keep=()) -> None:
+        self.gemm, self.words, self.variant, self.fn, self.what, self.keep = gemm, words, variant, fn, what, keep
+        self.plan = plan if plan.pack_a or plan.pack_b else None
+        self.sync = None if words is None else words.desc(variant)
+        self.args = tuple(byref(self.sync) if a is SYNC else a for a in args)
+
+    def __call__(self, A: torch.Tensor, B: torch.Tensor) -> None:
+        gemm = self.gemm
+        if self.plan is not None:
+            A, B = planned_operands(self.plan, A, B)
+        gemm.A, gemm.B = A.data_ptr(), B.data_ptr()
+        words = self.words
+        if words is not None:
+            if self.variant != "s0":  # S1 launches number the locks they write, S2 launches the counters
+                self.sync.epoch = words.next_epoch(self.variant)
+            self.sync.spin_limit_ns = words.spin_limit_ns
+        rc = self.fn(*self.args, stream_ptr())
+        if rc:
+            _lib.check(rc, self.what)
+
+
+SYNC = object()  # stands for the sync descriptor in a BoundCall's arguments
+
+
+class CallCache:
+    """Bounded cache of things one thread at a time may use: ``take`` removes what it returns, ``put`` gives it back (a
+    second thread that comes in between builds its own)."""
+
+    __slots__ = ("entries", "limit")
+
+    def __init__(self, limit: int = 64) -> None:
+        self.entries: dict = {}
+        self.limit = limit
+
+    def take(self, key):
+        return self.entries.pop(key, None)
+
+    def put(self, key, value) -> None:
+        entries = self.entries
+        while len(entries) >= self.limit:
+            try:
+                del entries[next(iter(entries))]
+            except (KeyError, StopIteration, RuntimeError):  # another thread was quicker
+                break
+        entries[key] = value
+
+
+def view_of(heap) -> _lib.HeapView:
+    """The heap's view descriptor, built once per heap (kernels only read it)."""
+    view = heap.__dict__.get("_view_desc")
+    bases = heap.get_heap_bases()  # raises once the heap has been cleaned up
+    if view is None:
+        view = heap.__dict__["_view_desc"] = heap_view(bases, heap.rank, heap.world_size)
+        view.bases = bases  # lives as long as a descriptor that names it
+    return view
 
 
 def heap_view(heap_bases: torch.Tensor, rank: int, world_size: int) -> _lib.HeapView:

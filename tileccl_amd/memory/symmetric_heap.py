@@ -167,9 +167,7 @@ class SymmetricHeap:
     def owns_tensor(self, tensor: torch.Tensor) -> bool:
         if self._buffer is None or tensor.device != self._device:
             return False
-        if tensor.numel() == 0:
-            return True
-        return self._local_ptr <= int(tensor.data_ptr()) < self._local_ptr + self._size
+        return 0 <= tensor.data_ptr() - self._local_ptr < self._size or tensor.numel() == 0
 
     is_symmetric = owns_tensor
 

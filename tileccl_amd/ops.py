@@ -393,6 +393,23 @@ def build_gemm_allscatter_plan(
     return direct(C, contract.rhs_layout, contract.output_layout)
 
 
+def _plan_for_call(A: Any, B: Any, C: Any, *, ctx, pattern: PatternLike, hw_info, **how) -> GemmAllScatterPlan | GemmAllScatterMixedLayoutPlan:
+    """The plan of a call that brings none, kept with the context's workspaces (bounded, and dropped with them when another
+    heap is attached): nothing in it depends on more than the shapes, the device and the keywords."""
+    ctx = ctx if ctx is not None else tileccl_amd.current_context()
+    if hw_info is not None or not (pattern is None or isinstance(pattern, str)):
+        return build_gemm_allscatter_plan(A, B, C, ctx=ctx, pattern=pattern, hw_info=hw_info, **how)
+    plans = ctx._workspace_cache.setdefault("tileccl_amd.allscatter_plans", {})
+    key = (A.shape, B.shape, C.shape, A.device, B.device, C.device, C.dtype, pattern, *how.values())
+    plan = plans.get(key) if ctx.heap is not None else None
+    if plan is None:
+        plan = build_gemm_allscatter_plan(A, B, C, ctx=ctx, pattern=pattern, **how)
+        if len(plans) >= 64:
+            plans.pop(next(iter(plans)), None)
+        plans[key] = plan
+    return plan
+
+
 def gemm_allscatter(
     A: Any,
     B: Any,
@@ -407,7 +424,7 @@ def gemm_allscatter(
     storage_kind: str = "symmetric",
 ) -> Any:
     """``C = A @ B`` on this rank, then this rank's column block lands in every peer's ``C``."""
-    plan = build_gemm_allscatter_plan(
+    plan = _plan_for_call(
         A,
         B,
         C,
@@ -434,7 +451,7 @@ def gemm_allscatter_sharded(
     storage_kind: str = "symmetric",
 ) -> Any:
     """shard/shard contract: ``B_shard (K, N/ws)``, ``C_shard (M, N/ws)``; ``full_N`` is mandatory."""
-    plan = build_gemm_allscatter_plan(
+    plan = _plan_for_call(
         A,
         B_shard,
         C_shard,

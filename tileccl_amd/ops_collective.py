@@ -156,20 +156,61 @@ def gemm_allgather(A: Any, B_shard: Any, Cx: Any, *, ctx=None, storage_kind: str
     tile by tile, ``"s2"`` TileGroup (default), or a ``Pattern`` instance.
     """
     ctx = ctx if ctx is not None else tileccl_amd.current_context()
-    k = resolve_gemm_allgather_contract(A, B_shard, Cx, ctx=ctx, storage_kind=storage_kind)
+    if not isinstance(variant, str):
+        _gather_bind(ctx, resolve_gemm_allgather_contract(A, B_shard, Cx, ctx=ctx, storage_kind=storage_kind), A, B_shard, Cx, variant)
+        return Cx
+    return run_gather(ctx, A, B_shard, Cx, storage_kind, variant)
+
+
+def _calls_of(ctx, what: str) -> _launch.CallCache:
+    """Bound calls of an operation, kept with the context's workspaces."""
+    return ctx._workspace_cache.setdefault(f"tileccl_amd.{what}_calls", _launch.CallCache())
+
+
+def run_gather(ctx, A: Any, B_shard: Any, Cx: Any, storage_kind: str, variant: str, expected: "GemmAllGatherContract | None" = None) -> Any:
+    """``gemm_allgather``; ``expected``: a plan's contract, which the tensors' must equal (``ValueError`` otherwise)."""
+    heap = ctx.require_heap()
+    calls = _calls_of(ctx, "gather")
+    key = (_launch.layout_key(A), _launch.layout_key(B_shard), _launch.layout_key(Cx), variant, storage_kind)
+    entry = calls.take(key)
+    if entry is None or entry[1] is not heap or not heap.owns_tensor(Cx):
+        k = resolve_gemm_allgather_contract(A, B_shard, Cx, ctx=ctx, storage_kind=storage_kind)
+        if expected is not None and k != expected:
+            raise ContractChanged  # before anything is allocated for the call: the ranks' heaps stay in step
+        entry = (k, heap, *_gather_bind(ctx, k, A, B_shard, Cx, variant, launch=False))
+    k, _, pattern, call, offset = entry
+    if expected is not None and k is not expected and k != expected:
+        calls.put(key, entry)
+        raise ContractChanged
+    call.gemm.C = Cx.data_ptr() + offset
+    call(A, B_shard)
+    calls.put(key, entry)
+    pattern._last_sync = call.words
+    return Cx
+
+
+class ContractChanged(ValueError):
+    """The tensors of a plan's call are not those that the plan was made for."""
+
+
+def _gather_bind(ctx, k: GemmAllGatherContract, A: Any, B_shard: Any, Cx: Any, variant: str | Pattern, launch: bool = True):
+    """The all-scatter launch on this rank's column block of ``C``: run through the pattern, or its bound call with the
+    block's byte offset."""
     lo = k.rank * k.shard_cols if k.world_size > 1 else 0
     block = Cx[:, lo:lo + k.shard_cols]  # the GEMM's output: this rank's columns of the full C
     shape = (k.M, k.full_N)
     spec = PatternExecutionSpec(
         M=k.M, K=k.K, full_N=k.full_N, local_N=k.shard_cols, rank=k.rank, world_size=k.world_size,
-        rhs=PatternTensorSpec((k.K, k.full_N), (k.K, k.shard_cols), k.rank, k.world_size, "shard", storage_kind),
-        output=PatternTensorSpec(shape, shape, k.rank, k.world_size, "full", storage_kind),
+        rhs=PatternTensorSpec((k.K, k.full_N), (k.K, k.shard_cols), k.rank, k.world_size, "shard", k.storage_kind),
+        output=PatternTensorSpec(shape, shape, k.rank, k.world_size, "full", k.storage_kind),
         # relative to the block: all of its columns go to the same columns of the peer's C
         scatter_src_col_offset=0, scatter_cols=k.shard_cols, scatter_dst_leading_dim=k.full_N, scatter_dst_col_offset=0,
     )
     pattern = _pattern_for(ctx, variant)
-    pattern.execute(A, B_shard, block, spec=spec)
-    return Cx
+    if launch:
+        pattern.execute(A, B_shard, block, spec=spec)
+        return None
+    return pattern, pattern._bind(A, B_shard, block, spec, ctx.require_heap()), int(block.data_ptr() - Cx.data_ptr())
 
 
 def _reduce_scatter_words(ctx, world: int, M: int, cols: int):
@@ -229,33 +270,59 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     if variant not in _launch.VARIANTS:
         raise ValueError(f"unknown variant {variant!r}; expected one of {sorted(_launch.VARIANTS)}")
     ctx = ctx if ctx is not None else tileccl_amd.current_context()
-    k = resolve_gemm_reducescatter_contract(A, B, Cx, ctx=ctx, storage_kind=storage_kind)
-    lib = _lib.load()
-    stream = _launch.stream_ptr()
+    return run_reduce(ctx, A, B, Cx, storage_kind, variant, emulate_peer, own_rows_in_registers, peers_resident)
+
+
+def run_reduce(ctx, A: Any, B: Any, Cx: Any, storage_kind: str, variant: str, emulate_peer: bool = False,
+               own_rows_in_registers: bool = True, peers_resident: bool = True,
+               expected: "GemmReduceScatterContract | None" = None) -> Any:
+    """``gemm_reducescatter``; ``expected``: a plan's contract, which the tensors' must equal (``ValueError`` otherwise)."""
+    heap = ctx.require_heap()
+    calls = _calls_of(ctx, "reduce")
+    key = (_launch.layout_key(A), _launch.layout_key(B), _launch.layout_key(Cx), variant, storage_kind, emulate_peer,
+           own_rows_in_registers, peers_resident)
+    entry = calls.take(key)
+    if entry is None or entry[1] is not heap or not heap.owns_tensor(Cx):
+        k = resolve_gemm_reducescatter_contract(A, B, Cx, ctx=ctx, storage_kind=storage_kind)
+        if expected is not None and k != expected:
+            raise ContractChanged  # before anything is allocated for the call: the ranks' heaps stay in step
+        entry = (k, heap, _reduce_bind(ctx, k, A, B, Cx, variant, emulate_peer, own_rows_in_registers, peers_resident))
+    k, _, call = entry
+    if expected is not None and k is not expected and k != expected:
+        calls.put(key, entry)
+        raise ContractChanged
     if k.world_size == 1:
-        _lib.check(lib.tccl_gemm(C.byref(_launch.gemm_desc(A, B, Cx)), stream), "tccl_gemm")
-        return Cx
+        call.gemm.C = Cx.data_ptr()
+    else:
+        call.args[1].value = Cx.data_ptr()
+    call(A, B)
+    calls.put(key, entry)
+    if call.words is not None:
+        ctx.__dict__["_reduce_scatter_last_words"] = call.words
+    return Cx
+
+
+def _reduce_bind(ctx, k: GemmReduceScatterContract, A: Any, B: Any, Cx: Any, variant: str, emulate_peer: bool,
+                 own_rows_in_registers: bool, peers_resident: bool) -> _launch.BoundCall:
+    lib = _lib.load()
+    if k.world_size == 1:
+        gemm, plan = _launch._gemm_desc(A, B, Cx)
+        return _launch.BoundCall(gemm, plan, None, "s0", lib.tccl_gemm, (C.byref(gemm),), "tccl_gemm")
     partial = ctx.workspace("gemm_reducescatter.partial", k.world_size, k.M, k.output_cols, dtype=torch.float32)
     tall = partial.view(k.world_size * k.M, k.output_cols)  # row block q = the shard rank q owns
-    view = _launch.heap_view(ctx.heap_bases, k.rank, k.world_size)
     transport = _launch.transport_desc(_lib.DIR_PULL, 16384, 16384, 0)
     mode = (_lib.RS_PEERS_RESIDENT if peers_resident else 0) | (_lib.RS_EMULATE_PEERS if emulate_peer else 0)
     flags = _lib.GEMM_OWN_ROWS_IN_REGISTERS if own_rows_in_registers else 0
-    words, sync = None, None
+    words = None
     if k.M % 128 == 0:
         words = _reduce_scatter_words(ctx, k.world_size, k.M, k.output_cols)
         flags |= _lib.GEMM_ARRIVALS
-        if variant != "s0":
-            words.next_epoch(variant)
-        sync = words.desc(variant)
     else:  # no whole plan tiles: one launch (or a GEMM per column block and a reduction) without signals
         mode |= _lib.RS_PEERS_RESIDENT
-    gemm = _launch.gemm_desc(A, B, tall, column_shards=k.world_size, flags=flags)
-    rc = lib.tccl_gemm_reducescatter(
-        C.byref(gemm), _launch.ptr(Cx), _launch.dtype_code(Cx.dtype), int(Cx.stride(0)), C.byref(view), _launch.byref(sync),
-        C.byref(transport), mode, _launch.VARIANTS[variant], stream,
+    gemm, plan = _launch._gemm_desc(A, B, tall, column_shards=k.world_size, flags=flags)
+    return _launch.BoundCall(
+        gemm, plan, words, variant, lib.tccl_gemm_reducescatter,
+        (C.byref(gemm), C.c_void_p(Cx.data_ptr()), _launch.dtype_code(Cx.dtype), int(Cx.stride(0)), C.byref(_launch.view_of(ctx.require_heap())),
+         _launch.SYNC if words is not None else None, C.byref(transport), mode, _launch.VARIANTS[variant]),
+        f"tccl_gemm_reducescatter[{variant}]",
     )
-    _lib.check(rc, f"tccl_gemm_reducescatter[{variant}]")
-    if words is not None:
-        ctx.__dict__["_reduce_scatter_last_words"] = words
-    return Cx

@@ -17,8 +17,10 @@ from dataclasses import asdict, dataclass, fields
 from typing import Any
 
 import tileccl_amd
+from tileccl_amd import _launch
 from tileccl_amd import ops_collective as _fused
 from tileccl_amd import primitives as _prim
+from tileccl_amd.primitives import collectives as _collectives
 
 
 def _shape(t: Any) -> "tuple[int, ...]":
@@ -87,9 +89,12 @@ class AllGatherPlan(_PlanMixin):
                                                               "src.numel": self.block_size})
 
     def execute(self, src: Any, output: Any, *, validate: bool = True) -> Any:
+        heap = self.ctx.require_heap()
+        if src.shape == self.input_shape and output.shape == self.output_shape and _collectives.run_known_allgather(src, output, heap):
+            return output
         if validate:
             self.validate_tensors(src, output)
-        _prim.allgather(src, output, self.ctx.require_heap())
+        _prim.allgather(src, output, heap)
         return output
 
 
@@ -100,6 +105,9 @@ def build_allgather_plan(src: Any, output: Any, *, ctx=None, storage_kind: str =
 
 def allgather(src: Any, output: Any, *, ctx=None, storage_kind: str = "symmetric") -> Any:
     """Every rank contributes ``src`` and ends with all ranks' blocks, in rank order, in ``output``."""
+    ctx = _context(ctx)
+    if ctx.heap is not None and _collectives.run_known_allgather(src, output, ctx.heap):
+        return output
     return build_allgather_plan(src, output, ctx=ctx, storage_kind=storage_kind).execute(src, output, validate=False)
 
 
@@ -126,9 +134,12 @@ class AllReducePlan(_PlanMixin):
         _allreduce_block(tensor, ctx=self.ctx, op=self.op, expected={"tensor shape": self.tensor_shape, "tensor.numel": self.block_size})
 
     def execute(self, tensor: Any, *, validate: bool = True) -> Any:
+        heap = self.ctx.require_heap()
+        if self.op == "sum" and tensor.shape == self.tensor_shape and _collectives.run_known_allreduce(tensor, heap):
+            return tensor
         if validate:
             self.validate_tensors(tensor)
-        _prim.allreduce(tensor, self.ctx.require_heap(), self.op)
+        _prim.allreduce(tensor, heap, self.op)
         return tensor
 
 
@@ -139,6 +150,9 @@ def build_allreduce_plan(tensor: Any, *, ctx=None, op: str = "sum", storage_kind
 
 def allreduce(tensor: Any, *, ctx=None, op: str = "sum", storage_kind: str = "symmetric") -> Any:
     """In place: once every rank has called, ``tensor`` holds the sum over the ranks."""
+    ctx = _context(ctx)
+    if op == "sum" and ctx.heap is not None and _collectives.run_known_allreduce(tensor, ctx.heap):
+        return tensor
     return build_allreduce_plan(tensor, ctx=ctx, op=op, storage_kind=storage_kind).execute(tensor, validate=False)
 
 
@@ -168,9 +182,12 @@ class ReduceScatterPlan(_PlanMixin):
                                                                    "output.numel": self.block_size})
 
     def execute(self, src: Any, output: Any, *, validate: bool = True) -> Any:
+        heap = self.ctx.require_heap()
+        if src.shape == self.input_shape and output.shape == self.output_shape and _collectives.run_known_reduce_scatter(src, output, heap):
+            return output
         if validate:
             self.validate_tensors(src, output)
-        _prim.reduce_scatter(src, output, self.ctx.require_heap(), "sum", self.implementation)
+        _prim.reduce_scatter(src, output, heap, "sum", self.implementation)
         return output
 
 
@@ -186,6 +203,9 @@ def build_reduce_scatter_plan(src: Any, output: Any, *, ctx=None, implementation
 
 def reduce_scatter(src: Any, output: Any, *, ctx=None, implementation: str = "auto", storage_kind: str = "symmetric") -> Any:
     """``output`` = the sum over ranks of block ``rank`` of their ``src``."""
+    ctx = _context(ctx)
+    if implementation in ("auto", "reference", "device") and ctx.heap is not None and _collectives.run_known_reduce_scatter(src, output, ctx.heap):
+        return output
     plan = build_reduce_scatter_plan(src, output, ctx=ctx, implementation=implementation, storage_kind=storage_kind)
     return plan.execute(src, output, validate=False)
 
@@ -208,9 +228,14 @@ class GemmAllGatherPlan(_PlanMixin):
             raise ValueError(_STALE.format(name="GemmAllGatherPlan"))
 
     def execute(self, A: Any, B_shard: Any, C: Any, *, validate: bool = True) -> Any:
-        if validate:
-            self.validate_tensors(A, B_shard, C)
-        return _fused.gemm_allgather(A, B_shard, C, ctx=self.ctx, storage_kind=self.storage_kind, variant=self.variant)
+        if not isinstance(self.variant, str):
+            if validate:
+                self.validate_tensors(A, B_shard, C)
+            return _fused.gemm_allgather(A, B_shard, C, ctx=self.ctx, storage_kind=self.storage_kind, variant=self.variant)
+        try:
+            return _fused.run_gather(self.ctx, A, B_shard, C, self.storage_kind, self.variant, self.contract if validate else None)
+        except _fused.ContractChanged:
+            raise ValueError(_STALE.format(name="GemmAllGatherPlan")) from None
 
 
 def build_gemm_allgather_plan(A: Any, B_shard: Any, C: Any, *, ctx=None, storage_kind: str = "symmetric",
@@ -235,10 +260,12 @@ class GemmReduceScatterPlan(_PlanMixin):
             raise ValueError(_STALE.format(name="GemmReduceScatterPlan"))
 
     def execute(self, A: Any, B: Any, C: Any, *, validate: bool = True) -> Any:
-        if validate:
-            self.validate_tensors(A, B, C)
-        return _fused.gemm_reducescatter(A, B, C, ctx=self.ctx, implementation=self.implementation,
-                                         storage_kind=self.storage_kind, variant=self.variant)
+        if self.variant not in _launch.VARIANTS:
+            raise ValueError(f"unknown variant {self.variant!r}; expected one of {sorted(_launch.VARIANTS)}")
+        try:
+            return _fused.run_reduce(self.ctx, A, B, C, self.storage_kind, self.variant, expected=self.contract if validate else None)
+        except _fused.ContractChanged:
+            raise ValueError(_STALE.format(name="GemmReduceScatterPlan")) from None
 
 
 def build_gemm_reducescatter_plan(A: Any, B: Any, C: Any, *, ctx=None, implementation: str = "auto",
@@ -293,7 +320,8 @@ class AllGatherGemmReduceScatterPlan(_PlanMixin):
             raise ValueError(_STALE.format(name="AllGatherGemmReduceScatterPlan"))
 
     def execute(self, input_shard: Any, W: Any, output: Any, *, validate: bool = True) -> Any:
-        if validate:
+        k = self.contract
+        if validate and not (input_shard.shape == (k.M, k.K_shard) and W.shape == (k.K, k.N) and output.shape == (k.M, k.N)):
             self.validate_tensors(input_shard, W, output)
         from tileccl_amd.patterns.chained_ag_gemm_rs import ChainedAGGemmRSPattern
 

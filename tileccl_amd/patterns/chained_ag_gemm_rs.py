@@ -63,6 +63,7 @@ class ChainedAGGemmRSPattern:
         # The GEMM + scatter stages reuse the all-scatter pattern's plan and signal words.
         self._stage = _SCHEDULES[schedule](ctx, BLOCK_M=BLOCK_M, BLOCK_N=BLOCK_N, BLOCK_K=BLOCK_K)
         self._last_sync: _launch.SyncWords | None = None
+        self._calls = _launch.CallCache()
 
     def execute(
         self,
@@ -71,6 +72,31 @@ class ChainedAGGemmRSPattern:
         output: torch.Tensor,
         gathered_workspace: torch.Tensor | None = None,
     ) -> torch.Tensor:
+        heap = self.ctx.require_heap()
+        if gathered_workspace is None:
+            gathered_workspace = self.ctx.workspace(
+                "chained_ag_gemm_rs.gathered_input", input_shard.shape[0], W.shape[0], dtype=input_shard.dtype
+            )
+        key = tuple(_launch.layout_key(t) for t in (input_shard, W, output, gathered_workspace))
+        call = self._calls.take(key)
+        if call is None or call.keep is not heap:
+            call = self._bind(input_shard, W, output, gathered_workspace, heap)
+        if self.ctx.world_size > 1:
+            for name, t in (("input_shard", input_shard), ("output", output)):
+                if not heap.owns_tensor(t):
+                    raise ValueError(
+                        f"{name} must live in the symmetric heap when world_size > 1: peers address it "
+                        "at the same offset in their slices"
+                    )
+        call.gemm.C = output.data_ptr()
+        call.args[1].value = input_shard.data_ptr()
+        call(gathered_workspace, W)
+        self._calls.put(key, call)
+        self._last_sync = call.words
+        return output
+
+    def _bind(self, input_shard, W, output, gathered_workspace, heap) -> _launch.BoundCall:
+        """Check the shapes and build the descriptors of a call on tensors of these layouts."""
         M, K_shard = input_shard.shape
         K, N = W.shape
         world_size = self.ctx.world_size
@@ -80,49 +106,22 @@ class ChainedAGGemmRSPattern:
             )
         if tuple(output.shape) != (M, N):
             raise ValueError(f"output shape {tuple(output.shape)} must be (M, N) = ({M}, {N})")
-        heap = self.ctx.require_heap()
-        if world_size > 1:
-            for name, t in (("input_shard", input_shard), ("output", output)):
-                if not heap.owns_tensor(t):
-                    raise ValueError(
-                        f"{name} must live in the symmetric heap when world_size > 1: peers address it "
-                        "at the same offset in their slices"
-                    )
-        if gathered_workspace is None:
-            gathered_workspace = self.ctx.workspace(
-                "chained_ag_gemm_rs.gathered_input", M, K, dtype=input_shard.dtype
-            )
-        elif tuple(gathered_workspace.shape) != (M, K) or gathered_workspace.dtype != input_shard.dtype:
+        if tuple(gathered_workspace.shape) != (M, K) or gathered_workspace.dtype != input_shard.dtype:
             raise ValueError(f"gathered_workspace must be ({M}, {K}) of {input_shard.dtype}")
-
-        gemm = _launch.gemm_desc(
-            gathered_workspace, W, output, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self._stage.GROUP_M,
-            flags=_lib.GEMM_ARRIVALS,
-        )
-        view = _launch.heap_view(self.ctx.heap_bases, self.ctx.rank, world_size)
         compute_wgs, comm_wgs = self._stage._wg_split()
-        gemm.num_wgs = compute_wgs
+        gemm, plan = _launch._gemm_desc(
+            gathered_workspace, W, output, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self._stage.GROUP_M,
+            num_wgs=compute_wgs, flags=_lib.GEMM_ARRIVALS,
+        )
         transport = _launch.transport_desc(_lib.DIR_PUSH, self._stage._copy_elems(), None, comm_wgs)
         words = self._stage._sync_words(M, N, output)
-        sync = None
-        if words is not None:
-            variant = "s1" if self._stage.variant == _lib.S1_TILE else "s2"
-            words.next_epoch(variant)
-            sync = words.desc(variant)
-        rc = _lib.load().tccl_chained_ag_gemm_rs(
-            C.byref(gemm),
-            _launch.ptr(input_shard),
-            _launch._row_major(input_shard, "input_shard"),
-            K_shard,
-            C.byref(view),
-            C.byref(sync) if sync is not None else None,
-            C.byref(transport),
-            self._stage.variant,
-            _launch.stream_ptr(),
+        variant = {_lib.S0_BULK: "s0", _lib.S1_TILE: "s1", _lib.S2_TILEGROUP: "s2"}[self._stage.variant]
+        return _launch.BoundCall(
+            gemm, plan, words, variant, _lib.load().tccl_chained_ag_gemm_rs,
+            (C.byref(gemm), C.c_void_p(), _launch._row_major(input_shard, "input_shard"), K_shard, C.byref(_launch.view_of(heap)),
+             _launch.SYNC if words is not None else None, C.byref(transport), self._stage.variant),
+            f"tccl_chained_ag_gemm_rs[{self.schedule}]", heap,
         )
-        _lib.check(rc, f"tccl_chained_ag_gemm_rs[{self.schedule}]")
-        self._last_sync = words
-        return output
 
     def check_faults(self) -> None:
         """Synchronise and raise if a bounded device-side wait of the last launch expired."""

@@ -47,6 +47,7 @@ class _HipAllScatterPattern(Pattern):
         # workspaces, and shared by every pattern instance of the same kind and tiling.
         cache = getattr(ctx, "_workspace_cache", None)
         self._sync: dict[tuple, _launch.SyncWords] = cache if isinstance(cache, dict) else {}
+        self._calls = _launch.CallCache()
 
     # -- hooks -------------------------------------------------------------------------
     def _sync_words(self, M: int, N: int, C_out: torch.Tensor) -> _launch.SyncWords | None:
@@ -74,33 +75,35 @@ class _HipAllScatterPattern(Pattern):
                 "C must live in the symmetric heap when world_size > 1: the scatter writes it at the "
                 "same offset in every peer's slice"
             )
+        key = (_launch.layout_key(A), _launch.layout_key(B), _launch.layout_key(C_out), spec.scatter_src_col_offset, spec.scatter_cols,
+               spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
+        call = self._calls.take(key)
+        if call is None or call.keep is not heap:
+            call = self._bind(A, B, C_out, spec, heap)
+        call.gemm.C = C_out.data_ptr()
+        call(A, B)
+        self._calls.put(key, call)
+        self._last_sync = call.words
+        if call.words is not None and call.words.host_plan is not None:
+            self.last_plan = call.words.host_plan
+
+    def _bind(self, A, B, C_out, spec, heap) -> _launch.BoundCall:
         compute_wgs, comm_wgs = self._wg_split()
-        gemm = _launch.gemm_desc(
+        gemm, plan = _launch._gemm_desc(
             A, B, C_out, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self.GROUP_M, num_wgs=compute_wgs,
             flags=_lib.GEMM_ARRIVALS,
         )
         scatter = _lib.ScatterDesc(
             spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset
         )
-        view = _launch.heap_view(self.ctx.heap_bases, spec.rank, spec.world_size)
         transport = _launch.transport_desc(_lib.DIR_PUSH, self._copy_elems(), None, comm_wgs)
         words = self._sync_words(spec.M, spec.local_N, C_out)
-        sync = None
-        if words is not None:
-            variant = "s1" if self.variant == _lib.S1_TILE else "s2"
-            words.next_epoch(variant)
-            sync = words.desc(variant)
-        rc = _lib.load().tccl_gemm_allscatter(
-            C.byref(gemm),
-            C.byref(scatter),
-            C.byref(view),
-            C.byref(sync) if sync is not None else None,
-            C.byref(transport),
-            self.variant,
-            _launch.stream_ptr(),
+        variant = {_lib.S0_BULK: "s0", _lib.S1_TILE: "s1", _lib.S2_TILEGROUP: "s2"}[self.variant]
+        return _launch.BoundCall(
+            gemm, plan, words, variant, _lib.load().tccl_gemm_allscatter,
+            (C.byref(gemm), C.byref(scatter), C.byref(_launch.view_of(heap)), _launch.SYNC if words is not None else None,
+             C.byref(transport), self.variant), f"tccl_gemm_allscatter[{self.name}]", heap,
         )
-        _lib.check(rc, f"tccl_gemm_allscatter[{self.name}]")
-        self._last_sync = words
 
     def _copy_elems(self) -> int:
         return 16384

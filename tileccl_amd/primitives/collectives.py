@@ -87,12 +87,52 @@ def _whole_units(collective: str, block: int, element_size: int, *, reduce: bool
         raise ValueError(f"{collective}: a rank's block of {block} elements is not a multiple of {need}")
 
 
+_KNOWN_LIMIT = 64
+
+
+# Each collective has a quick way for tensors like those of an earlier call: ``heap.__dict__["_known_calls"]`` holds what that call,
+# checked in full, was found to need, by the tensors' shapes, strides, types and devices.  Where a tensor lies is
+# looked at on every call.  ``run_known_*`` launches and returns True, or returns False: the caller then goes the whole way.
+
+
+def _remember(heap, key, what) -> None:
+    calls = heap.__dict__.setdefault("_known_calls", {})
+    if len(calls) >= _KNOWN_LIMIT:
+        calls.clear()
+    calls[key] = what
+
+
 def allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> None:
     """Every rank ends with ``[tensor_rank0 | tensor_rank1 | ...]`` in ``output``.
 
     Direct write (reference :628-630): the caller's block goes into block ``rank`` of every
     rank's ``output``, its own included, in one launch.
     """
+    if not run_known_allgather(tensor, output, heap):
+        _remember(heap, _pair_key("allgather", tensor, output), _check_allgather(tensor, output, heap))
+        run_known_allgather(tensor, output, heap)
+
+
+def _pair_key(op: str, tensor: torch.Tensor, output: torch.Tensor) -> tuple:
+    return op, tensor.shape, tensor.stride(), tensor.dtype, tensor.device, output.shape, output.stride(), output.dtype, output.device
+
+
+def run_known_allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> bool:
+    calls = heap.__dict__.get("_known_calls")
+    nbytes = calls.get(_pair_key("allgather", tensor, output)) if calls is not None else None
+    if nbytes is None or not (heap.owns_tensor(tensor) and heap.owns_tensor(output)):
+        return False
+    if nbytes:
+        rc = _lib.load().tccl_copy_block(
+            output.data_ptr() + heap.rank * nbytes, (1 << heap.world_size) - 1, tensor.data_ptr(), heap.rank, 1, nbytes, nbytes, nbytes,
+            _launch.byref(_launch.view_of(heap)), _launch.stream_ptr(),
+        )
+        _lib.check(rc, "tccl_copy_block")
+    return True
+
+
+def _check_allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> int:
+    """The contract of ``allgather``; returns the bytes of a rank's block."""
     world = heap.world_size
     _validate_world_size(world)
     block = _pair_block("allgather", tensor=tensor, output=output, world_size=world)
@@ -103,11 +143,9 @@ def allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> None:
     _on_heap(output, heap, "output")
     if tensor.dtype != output.dtype:
         raise ValueError(f"allgather expects one dtype, got tensor={tensor.dtype}, output={output.dtype}")
-    if block == 0:
-        return
-    _whole_units("allgather", block, tensor.element_size())
-    mine = output.reshape(-1)[heap.rank * block : (heap.rank + 1) * block]
-    copy_block(mine, tensor.reshape(-1), heap, src_rank=heap.rank, dst_ranks=range(world))
+    if block:
+        _whole_units("allgather", block, tensor.element_size())
+    return block * tensor.element_size()
 
 
 def broadcast(tensor: torch.Tensor, heap, root: int = 0) -> None:
@@ -145,21 +183,6 @@ def scatter(tensor: torch.Tensor, output: torch.Tensor, heap, *, root: int = 0) 
         copy_block(out, flat[r * block : (r + 1) * block], heap, src_rank=root, dst_ranks=(r,))
 
 
-def _reduce_chunk(collective: str, tensor: torch.Tensor, out: torch.Tensor, heap, block: int) -> None:
-    """out = sum over ranks of chunk ``heap.rank`` of their ``tensor`` (peer reads, fp32 accumulate)."""
-    if tensor.dtype not in _REDUCE_IN:
-        raise ValueError(f"{collective} supports fp16, bf16 and fp32 tensors, got {tensor.dtype}")
-    if out.dtype not in _REDUCE_OUT and not (out.dtype == torch.float32 and tensor.dtype == torch.float32):
-        raise ValueError(f"{collective} writes fp16 or bf16 (fp32 for fp32 tensors), got {out.dtype} from {tensor.dtype}")
-    _whole_units(collective, block, tensor.element_size(), reduce=True)
-    view = _launch.heap_view(heap.get_heap_bases(), heap.rank, heap.world_size)
-    rc = _lib.load().tccl_reduce_rows(
-        _launch.ptr(tensor), _launch.dtype_code(tensor.dtype), block, _launch.ptr(out), _launch.dtype_code(out.dtype), block,
-        heap.world_size, block, _launch.byref(view), None, 0, _launch.stream_ptr(),
-    )
-    _lib.check(rc, f"tccl_reduce_rows[{collective}]")
-
-
 def reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap, op: str = "sum", implementation: str = "auto") -> None:
     """``output`` = sum over ranks of chunk ``rank`` of their ``tensor`` (peer reads).
 
@@ -170,6 +193,28 @@ def reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap, op: str = "
         raise ValueError(f"Only op='sum' is currently supported, got {op!r}")
     if implementation not in {"auto", "reference", "device"}:
         raise ValueError(f"implementation must be one of {{'auto', 'reference', 'device'}}, got {implementation!r}")
+    if not run_known_reduce_scatter(tensor, output, heap):
+        _remember(heap, _pair_key("reduce_scatter", tensor, output), _check_reduce_scatter(tensor, output, heap))
+        run_known_reduce_scatter(tensor, output, heap)
+
+
+def run_known_reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap) -> bool:
+    calls = heap.__dict__.get("_known_calls")
+    known = calls.get(_pair_key("reduce_scatter", tensor, output)) if calls is not None else None
+    if known is None or not (heap.owns_tensor(tensor) and heap.owns_tensor(output)):
+        return False
+    block, in_code, out_code = known
+    if block:
+        rc = _lib.load().tccl_reduce_rows(
+            tensor.data_ptr(), in_code, block, output.data_ptr(), out_code, block, heap.world_size, block,
+            _launch.byref(_launch.view_of(heap)), None, 0, _launch.stream_ptr(),
+        )
+        _lib.check(rc, "tccl_reduce_rows[reduce_scatter]")
+    return True
+
+
+def _check_reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap) -> tuple[int, int, int]:
+    """The contract of ``reduce_scatter``; returns a block's elements and the two type codes."""
     world = heap.world_size
     _validate_world_size(world)
     block = _pair_block("reduce_scatter", tensor=tensor, output=output, world_size=world)
@@ -179,32 +224,53 @@ def reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap, op: str = "
     _on_heap(tensor, heap, "tensor")
     _on_heap(output, heap, "output")
     if block == 0:
-        return
-    _reduce_chunk("reduce_scatter", tensor, output, heap, block)
+        return 0, 0, 0
+    if tensor.dtype not in _REDUCE_IN:
+        raise ValueError(f"reduce_scatter supports fp16, bf16 and fp32 tensors, got {tensor.dtype}")
+    if output.dtype not in _REDUCE_OUT and not (output.dtype == torch.float32 and tensor.dtype == torch.float32):
+        raise ValueError(f"reduce_scatter writes fp16 or bf16 (fp32 for fp32 tensors), got {output.dtype} from {tensor.dtype}")
+    _whole_units("reduce_scatter", block, tensor.element_size(), reduce=True)
+    return block, _launch.dtype_code(tensor.dtype), _launch.dtype_code(output.dtype)
 
 
 def allreduce(tensor: torch.Tensor, heap, op: str = "sum") -> None:
     """In place: once every rank has called, every rank's ``tensor`` holds the sum over ranks."""
     if op != "sum":
         raise ValueError(f"Only op='sum' is currently supported, got {op!r}")
+    if not run_known_allreduce(tensor, heap):
+        _remember(heap, ("allreduce", tensor.shape, tensor.stride(), tensor.dtype, tensor.device), _check_allreduce(tensor, heap))
+        run_known_allreduce(tensor, heap)
+
+
+def run_known_allreduce(tensor: torch.Tensor, heap) -> bool:
+    calls = heap.__dict__.get("_known_calls")
+    known = calls.get(("allreduce", tensor.shape, tensor.stride(), tensor.dtype, tensor.device)) if calls is not None else None
+    if known is None or not heap.owns_tensor(tensor):
+        return False
+    numel, code = known
+    if numel:
+        rc = _lib.load().tccl_allreduce_chunk(
+            tensor.data_ptr(), code, numel, _launch.byref(_launch.view_of(heap)), _launch.stream_ptr()
+        )
+        _lib.check(rc, "tccl_allreduce_chunk")
+    return True
+
+
+def _check_allreduce(tensor: torch.Tensor, heap) -> tuple[int, int]:
+    """The contract of ``allreduce``; returns the elements to sum (none: nothing to do) and the type code."""
     world = heap.world_size
     _validate_world_size(world)
     _contiguous("allreduce", tensor, "tensor")
     _on_heap(tensor, heap, "tensor")
     numel = int(tensor.numel())
     if world == 1 or numel == 0:
-        return  # local identity (reference :2563-2583)
+        return 0, 0  # local identity (reference :2563-2583)
     if tensor.dtype not in _REDUCE_IN:
         raise ValueError(f"allreduce supports fp16, bf16 and fp32 tensors, got {tensor.dtype}")
     if numel % world:
         raise ValueError(f"allreduce tensor.numel={numel} must be divisible by world_size={world}")
-    block = numel // world
-    _whole_units("allreduce", block, tensor.element_size(), reduce=True)
-    view = _launch.heap_view(heap.get_heap_bases(), heap.rank, world)
-    rc = _lib.load().tccl_allreduce_chunk(
-        _launch.ptr(tensor), _launch.dtype_code(tensor.dtype), numel, _launch.byref(view), _launch.stream_ptr()
-    )
-    _lib.check(rc, "tccl_allreduce_chunk")
+    _whole_units("allreduce", numel // world, tensor.element_size(), reduce=True)
+    return numel, _launch.dtype_code(tensor.dtype)
 
 
 # ---------------------------------------------------------------------------------------------
@@ -312,7 +378,7 @@ def _staged(name: str, op: int, srcs, dsts, heaps, block: int, *, root: int = 0,
     _whole_units(name, block, esz)
     code = _launch.dtype_code(first.dtype if reduces else _BYTES_AS.get(esz, first.dtype))  # copies move bytes
     if chunk_elems is None and pipeline_slots is None and len(set(carried)) == world and not (reduces and block % 8):
-        view = _launch.heap_view(heaps[0].get_heap_bases(), 0, world)
+        view = _launch.view_of(heaps[0])
         rc = _lib.load().tccl_collective_direct(
             op, _launch.ptr(srcs[0]) if srcs is not None else None, _launch.ptr(dsts[0]), code, block, int(root),
             _launch.byref(view), _launch.stream_ptr(),
@@ -330,7 +396,7 @@ def _staged(name: str, op: int, srcs, dsts, heaps, block: int, *, root: int = 0,
     ws = cache[key]
     base_epoch = ws.reserve_epoch_range(chunks)
     ws.fault.zero_()
-    view = _launch.heap_view(heaps[0].get_heap_bases(), 0, world)
+    view = _launch.view_of(heaps[0])
     mask = 0
     for r in carried:
         mask |= 1 << r

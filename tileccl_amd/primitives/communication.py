@@ -43,7 +43,7 @@ def copy_block(dst: torch.Tensor, src: torch.Tensor, heap, *, src_rank: int, dst
                 mask |= 1 << int(r)
     if nbytes == 0 or mask == 0:
         return
-    view = _launch.heap_view(heap.get_heap_bases(), heap.rank, heap.world_size)
+    view = _launch.view_of(heap)
     rc = _lib.load().tccl_copy_block(
         _launch.ptr(dst), mask, _launch.ptr(src), int(src_rank), 1, nbytes, nbytes, nbytes, _launch.byref(view),
         _launch.stream_ptr(),

@@ -79,6 +79,8 @@ class _FusedBase:
         self.signals: TileGroupSignalState | None = None
         self.words: _launch.SyncWords | None = None
         self.locks: torch.Tensor | None = None
+        self.directions = 0
+        self._calls = _launch.CallCache()
 
     # -- planning -----------------------------------------------------------------------
     def _build_plan(self, M: int, N: int, elem_bytes: int, spec: CollectiveSpec) -> None:
@@ -137,17 +139,28 @@ class _FusedBase:
             self.heap.peer_view(self.signals.counter, peer).fill_(PEER_READY)
             self.heap.peer_view(self.locks, peer).fill_(PEER_READY)
 
-    def _descs(self, directions: int, variant: str):
-        assert self.words is not None
+    def _call_key(self, A: torch.Tensor, B: torch.Tensor, variant: str) -> tuple:
+        """What a bound call depends on: the operands' layouts and this operation's settings."""
+        return (A.shape, A.stride(), B.shape, B.stride(), A.dtype, B.dtype, A.device, B.device, A.data_ptr() & 15, B.data_ptr() & 15,
+                variant, self.directions, self.macro_tile, self.num_gemm_wgs, self.num_comm_wgs)
+
+    def _cached(self, key: tuple) -> "_launch.BoundCall | None":
+        self.heap.get_heap_bases()  # raises once the heap has been cleaned up
+        call = self._calls.take(key)
+        return call if call is not None and call.words is self.words and call.keep is self.transport else None
+
+    def _bound(self, A: torch.Tensor, B: torch.Tensor, out: torch.Tensor, variant: str, flags: int):
+        """(gemm descriptor, operand plan, view, transport) of a new bound call."""
         if variant not in _launch.VARIANTS:
             raise ValueError(f"unknown variant {variant!r}; expected one of {sorted(_launch.VARIANTS)}")
-        view = _launch.heap_view(self.heap.get_heap_bases(), self.rank, self.world_size)
-        transport = _launch.transport_desc(
-            directions, self.transport.copy_elems, self.transport.reduce_elems, self.num_comm_wgs
+        gemm, plan = _launch._gemm_desc(
+            A, B, out, block_m=self.block_m, block_n=self.block_n, group_m=self.group_m,
+            num_wgs=self.num_gemm_wgs, macro_tile=self.macro_tile, flags=flags | _lib.GEMM_ARRIVALS,
         )
-        if variant != "s0":  # S1 launches number the locks they write, S2 launches the counters
-            self.words.next_epoch(variant)
-        return view, transport, self.words.desc(variant)
+        transport = _launch.transport_desc(
+            self.directions, self.transport.copy_elems, self.transport.reduce_elems, self.num_comm_wgs
+        )
+        return gemm, plan, _launch.view_of(self.heap), transport
 
     def check_faults(self) -> None:
         if self.words is not None:
@@ -178,17 +191,18 @@ class FusedGemmAllGather(_FusedBase):
 
     def __call__(self, A: torch.Tensor, B: torch.Tensor, variant: str = "s2", alpha: float = 1.0,
                  scale_a: float = 1.0, scale_b: float = 1.0) -> torch.Tensor:
-        alpha = float(alpha) * float(scale_a) * float(scale_b)  # per-tensor dequantisation scales of fp8 inputs
-        gemm = _launch.gemm_desc(
-            A, B, self.local_block, block_m=self.block_m, block_n=self.block_n, group_m=self.group_m,
-            alpha=alpha, num_wgs=self.num_gemm_wgs, macro_tile=self.macro_tile, flags=_lib.GEMM_ARRIVALS,
-        )
-        view, transport, sync = self._descs(self.directions, variant)
-        rc = _lib.load().tccl_gemm_allgather(
-            C.byref(gemm), _launch.ptr(self.out), int(self.out.stride(0)), C.byref(view), C.byref(sync),
-            C.byref(transport), _launch.VARIANTS[variant], _launch.stream_ptr(),
-        )
-        _lib.check(rc, f"tccl_gemm_allgather[{variant}]")
+        key = self._call_key(A, B, variant)
+        call = self._cached(key)
+        if call is None:
+            gemm, plan, view, transport = self._bound(A, B, self.local_block, variant, 0)
+            call = _launch.BoundCall(
+                gemm, plan, self.words, variant, _lib.load().tccl_gemm_allgather,
+                (C.byref(gemm), _launch.ptr(self.out), int(self.out.stride(0)), C.byref(view), _launch.SYNC, C.byref(transport),
+                 _launch.VARIANTS[variant]), f"tccl_gemm_allgather[{variant}]", self.transport,
+            )
+        call.gemm.alpha = float(alpha) * float(scale_a) * float(scale_b)  # per-tensor dequantisation scales of fp8 inputs
+        call(A, B)
+        self._calls.put(key, call)
         return self.out
 
 
@@ -217,6 +231,7 @@ class FusedGemmReduceScatter(_FusedBase):
         self.M, self.N = M, N
         self.emulate_peer = emulate_peer
         self.own_rows_in_registers = own_rows_in_registers
+        self.directions = _lib.DIR_PULL
         spec = reduce_scatter_spec(world_size=self.world_size)
         self.shard_rows = spec.shard_rows(M)
         self.partial = heap.allocate_tensor((M, N), partial_dtype)
@@ -231,17 +246,19 @@ class FusedGemmReduceScatter(_FusedBase):
 
     def __call__(self, A: torch.Tensor, B: torch.Tensor, variant: str = "s2", alpha: float = 1.0,
                  scale_a: float = 1.0, scale_b: float = 1.0) -> torch.Tensor:
-        alpha = float(alpha) * float(scale_a) * float(scale_b)  # per-tensor dequantisation scales of fp8 inputs
-        gemm = _launch.gemm_desc(
-            A, B, self.partial, block_m=self.block_m, block_n=self.block_n, group_m=self.group_m,
-            alpha=alpha, num_wgs=self.num_gemm_wgs, macro_tile=self.macro_tile,
-            flags=_lib.GEMM_ARRIVALS | (_lib.GEMM_OWN_ROWS_IN_REGISTERS if self.own_rows_in_registers else 0),
-        )
-        view, transport, sync = self._descs(_lib.DIR_PULL, variant)
-        rc = _lib.load().tccl_gemm_reducescatter(
-            C.byref(gemm), _launch.ptr(self.out), _launch.dtype_code(self.out.dtype), int(self.out.stride(0)),
-            C.byref(view), C.byref(sync), C.byref(transport), int(self.emulate_peer),
-            _launch.VARIANTS[variant], _launch.stream_ptr(),
-        )
-        _lib.check(rc, f"tccl_gemm_reducescatter[{variant}]")
+        key = (*self._call_key(A, B, variant), self.emulate_peer, self.own_rows_in_registers)
+        call = self._cached(key)
+        if call is None:
+            gemm, plan, view, transport = self._bound(
+                A, B, self.partial, variant, _lib.GEMM_OWN_ROWS_IN_REGISTERS if self.own_rows_in_registers else 0
+            )
+            call = _launch.BoundCall(
+                gemm, plan, self.words, variant, _lib.load().tccl_gemm_reducescatter,
+                (C.byref(gemm), _launch.ptr(self.out), _launch.dtype_code(self.out.dtype), int(self.out.stride(0)), C.byref(view),
+                 _launch.SYNC, C.byref(transport), int(self.emulate_peer), _launch.VARIANTS[variant]),
+                f"tccl_gemm_reducescatter[{variant}]", self.transport,
+            )
+        call.gemm.alpha = float(alpha) * float(scale_a) * float(scale_b)  # per-tensor dequantisation scales of fp8 inputs
+        call(A, B)
+        self._calls.put(key, call)
         return self.out
