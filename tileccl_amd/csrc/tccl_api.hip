@@ -102,29 +102,28 @@ __global__ __launch_bounds__(256, 3) void fused_kernel(tccl::GemmArgs g, tccl::S
   __shared__ __attribute__((aligned(1024))) char stage2[tccl::kStage128];
   if ((int)blockIdx.x < num_compute) {
     if (trace_start && blockIdx.x == 0 && threadIdx.x == 0) *trace_start = tccl::now_ticks();
-    tccl::GemmRole<InT, OutT>(g, push, stage0, stage1, stage2).run(s, (int)blockIdx.x, num_compute);
+    tccl::EpilogueReduce none;
+    none.active = 0;
+    tccl::GemmRole<InT, OutT>(g, push, none, stage0, stage1, stage2).run(s, (int)blockIdx.x, num_compute);
   } else {
     tccl::comm_role(c, (int)blockIdx.x - num_compute, (int)gridDim.x - num_compute, (int*)stage0);
   }
 #endif
 }
 
-// The GEMM alone on 128 x 128 tiles: no communication workgroup has to fit beside it, so it takes five
-// stages (80 KiB, two workgroups per CU): a load then has three steps and a half to arrive instead of
-// one and a half.
-template <typename InT, typename OutT>
-__global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g) {
+// Launches without communication workgroups: the GEMM alone, pushes from the epilogue, reductions in it
+// (kReduce).  Nothing has to fit beside two of them on a CU, so they take five stages (80 KiB): a load then has three
+// steps and a half to arrive instead of one and a half.  1000 x 2064 x 1008 with its push: 18.3 us with three stages,
+// MEASURED128 with five.
+template <typename InT, typename OutT, bool kReduce>
+__global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::PushArgs push, tccl::EpilogueReduce reduce) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) char stage0[tccl::kStage128];
   __shared__ __attribute__((aligned(1024))) char stage1[tccl::kStage128];
   __shared__ __attribute__((aligned(1024))) char stage2[tccl::kStage128];
   __shared__ __attribute__((aligned(1024))) char stage3[tccl::kStage128];
   __shared__ __attribute__((aligned(1024))) char stage4[tccl::kStage128];
-  tccl::SignalArgs s;
-  s.mode = tccl::kSignalNone;
-  tccl::PushArgs push;
-  push.world = 0;
-  tccl::GemmRole<InT, OutT, 5>(g, push, stage0, stage1, stage2, stage3, stage4).run(s, (int)blockIdx.x, (int)gridDim.x);
+  tccl::GemmRole<InT, OutT, 5>(g, push, reduce, stage0, stage1, stage2, stage3, stage4).template run<kReduce>(s, (int)blockIdx.x, (int)gridDim.x);
 #endif
 }
 
@@ -364,25 +363,31 @@ int check_sync(const tccl_sync_desc* s, int variant) {
 // ------------------------------------------------------------------------------------------
 template <typename InT, typename OutT>
 int launch_fused_t(const tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::CommArgs& c, const tccl::PushArgs& push,
-                   int compute, int comm, int64_t* trace_start, hipStream_t stream) {
-  if (comm == 0 && s.mode == tccl::kSignalNone && !trace_start)
-    hipLaunchKernelGGL((gemm128_kernel<InT, OutT>), dim3(compute), dim3(tccl::kThreads), 0, stream, g);
+                   const tccl::EpilogueReduce& reduce, int compute, int comm, int64_t* trace_start, hipStream_t stream) {
+  const dim3 block(tccl::kThreads);
+  if (reduce.active)
+    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, true>), dim3(compute), block, 0, stream, g, s, push, reduce);
+  else if (comm == 0 && !trace_start)
+    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, false>), dim3(compute), block, 0, stream, g, s, push, reduce);
   else
-    hipLaunchKernelGGL((fused_kernel<InT, OutT>), dim3(compute + comm), dim3(tccl::kThreads), 0, stream, g, s, c, push, compute,
-                       trace_start);
+    hipLaunchKernelGGL((fused_kernel<InT, OutT>), dim3(compute + comm), block, 0, stream, g, s, c, push, compute, trace_start);
   TCCL_HIP(hipGetLastError());
   return 0;
 }
 
 int launch_fused(int in_dtype, int out_dtype, const tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::CommArgs& c,
-                 int compute, int comm, int64_t* trace_start, hipStream_t stream, const tccl::PushArgs* push_args = nullptr) {
+                 int compute, int comm, int64_t* trace_start, hipStream_t stream, const tccl::PushArgs* push_args = nullptr,
+                 const tccl::EpilogueReduce* reduce_args = nullptr) {
   tccl::PushArgs push;
   memset(&push, 0, sizeof push);
   if (push_args) push = *push_args;
-  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F16) return launch_fused_t<_Float16, _Float16>(g, s, c, push, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F32) return launch_fused_t<_Float16, float>(g, s, c, push, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_BF16) return launch_fused_t<__bf16, __bf16>(g, s, c, push, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_F32) return launch_fused_t<__bf16, float>(g, s, c, push, compute, comm, trace_start, stream);
+  tccl::EpilogueReduce reduce;
+  memset(&reduce, 0, sizeof reduce);
+  if (reduce_args) reduce = *reduce_args;
+  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F16) return launch_fused_t<_Float16, _Float16>(g, s, c, push, reduce, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F32) return launch_fused_t<_Float16, float>(g, s, c, push, reduce, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_BF16) return launch_fused_t<__bf16, __bf16>(g, s, c, push, reduce, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_F32) return launch_fused_t<__bf16, float>(g, s, c, push, reduce, compute, comm, trace_start, stream);
   return fail(TCCL_ERR_UNSUPPORTED, "gemm: no kernel for in_dtype=%d, out_dtype=%d", in_dtype, out_dtype);
 }
 
@@ -834,18 +839,19 @@ void build_stream(const tccl_gemm_desc* d, const tccl::GemmArgs& g, int64_t seg_
 
 int stream_status(int rc) { return rc == 0 ? 0 : hip_fail((hipError_t)rc, "streaming GEMM launch"); }
 
-// A reduce-scatter launch's own part of the arguments.
-void add_stream_reduce(const tccl::CommArgs& c, const tccl_gemm_desc* d, tccl::StreamArgs* a) {
-  a->heap_bases = c.heap_bases;
-  a->rank = c.rank;
-  a->world = c.world;
-  a->first_seg = (c.rank + 1) % c.world;  // this rank's own rows come last: what its peers wait for comes first
-  tccl::StreamReduce& r = a->reduce;
+// A reduce-scatter carried out in the epilogue.
+tccl::EpilogueReduce build_epilogue_reduce(const tccl::CommArgs& c, const tccl_gemm_desc* d) {
+  tccl::EpilogueReduce r;
+  memset(&r, 0, sizeof r);
   r.active = 1;
   r.emulate_peer = c.emulate_peer;
   r.peers_resident = c.peers_resident;
   r.own_in_registers = (d->flags & TCCL_GEMM_OWN_ROWS_IN_REGISTERS) != 0;
   r.out_dtype = c.out_dtype;
+  r.rank = c.rank;
+  r.world = c.world;
+  r.shard_rows = c.M / c.world;
+  r.heap_bases = c.heap_bases;
   r.out = c.rs_out;
   r.ld_out_bytes = c.ld_rs_out_bytes;
   r.locks = c.locks;
@@ -853,6 +859,15 @@ void add_stream_reduce(const tccl::CommArgs& c, const tccl_gemm_desc* d, tccl::S
   r.tile_counts = c.tile_counts;
   r.fault = c.fault;
   r.spin_ticks = c.spin_ticks;
+  return r;
+}
+
+void add_stream_reduce(const tccl::CommArgs& c, const tccl_gemm_desc* d, tccl::StreamArgs* a) {
+  a->heap_bases = c.heap_bases;
+  a->rank = c.rank;
+  a->world = c.world;
+  a->first_seg = (c.rank + 1) % c.world;  // this rank's own rows come last: what its peers wait for comes first
+  a->reduce = build_epilogue_reduce(c, d);
 }
 
 int run_stream(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc* sync, int variant, int shape, int64_t seg_rows,
@@ -986,7 +1001,22 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // launch keeps the pushes in the communication role, whose tasks carry the per-group clock stamps.
   tccl::PushArgs push;
   memset(&push, 0, sizeof push);
-  const bool traced = sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock;
+  const bool traced = sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock || sync->trace_comm_counter;
+  if (c.op == tccl::kOpReduceScatter && !traced && c.world > 1 && !(tr && tr->num_comm_wgs > 0)) {
+    // With the peers' partials there the sums follow as a kernel of their own: one in `world` tiles would do all the
+    // reading otherwise, on as many CUs (1024 x 4096 x 2048, four ranks: 37 us; GEMM and reduction one after the other
+    // 30 us; communication workgroups beside a three-stage GEMM 48 us).
+    if (c.peers_resident && !c.emulate_peer) {
+      const int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, compute, 0, nullptr, stream);
+      return rc ? rc : launch_bulk(c, dev, stream);
+    }
+    // Otherwise they happen in the epilogue.  Workgroups that wait for a peer's partials must leave room for the peer's own
+    // launch: at most one per CU (two fit).
+    if (c.peers_resident || compute <= dev.compute_units) {
+      const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
+      return launch_fused(d->in_dtype, d->out_dtype, g, s, c, compute, 0, nullptr, stream, nullptr, &r);
+    }
+  }
   if (!traced && build_push(c, g, &push)) {
     c.directions &= ~tccl::kDirPush;
     if (c.op != tccl::kOpReduceScatter && !(c.directions & tccl::kDirPull)) comm = 0;

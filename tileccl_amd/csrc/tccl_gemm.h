@@ -44,6 +44,7 @@
 // written (gemm.py:163-167); the K tail is zero-filled (gemm.py:153-160).
 #pragma once
 
+#include "tccl_comm.h"
 #include "tccl_device.h"
 
 namespace tccl {
@@ -52,7 +53,6 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTile = 128;                        // sub-tile edge
 constexpr int kBK = 32;                           // K per step
@@ -134,6 +134,24 @@ struct PushArgs {
   const int64_t* heap_bases;  // C's address inside target q is C + heap_bases[q] - heap_bases[rank]
 };
 
+// Reduce-scatter carried out in the epilogue of the GEMM: the tiles of rows this rank owns take the peers' partials
+// and leave as output; under single-GPU emulation the other owners' rows are reduced as well.
+struct EpilogueReduce {
+  int active, emulate_peer;
+  int peers_resident;    // the peers' partials are complete in memory: their words are not looked at
+  int own_in_registers;  // own rows: no partial is stored
+  int out_dtype;
+  int rank, world, shard_rows;
+  const int64_t* heap_bases;
+  char* out;             // this rank's output shard (the partial is the GEMM's C)
+  int64_t ld_out_bytes;
+  const int32_t* locks;  // this rank's words; a peer's sit at the same slice offset
+  const int32_t* counter;
+  const int32_t* tile_counts;
+  int64_t* fault;
+  int64_t spin_ticks;
+};
+
 template <typename T>
 struct Mfma;
 template <>
@@ -175,6 +193,7 @@ struct GemmRole {
 
   const GemmArgs& g;
   const PushArgs& push;  // world == 0: nothing leaves from the epilogue
+  const EpilogueReduce& reduce;
   char* st0;
   char* st1;
   char* st2;
@@ -183,9 +202,9 @@ struct GemmRole {
   const int tid, lane, wave, wm, wn;
 
   // The wavefront's number lives in a scalar register: the LDS addresses its loads land at derive from it.
-  TCCL_D GemmRole(const GemmArgs& args, const PushArgs& push_args, char* s0, char* s1, char* s2, char* s3 = nullptr,
-                  char* s4 = nullptr)
-      : g(args), push(push_args), st0(s0), st1(s1), st2(s2), st3(s3), st4(s4), tid(threadIdx.x), lane(threadIdx.x & 63),
+  TCCL_D GemmRole(const GemmArgs& args, const PushArgs& push_args, const EpilogueReduce& reduce_args, char* s0, char* s1, char* s2,
+                  char* s3 = nullptr, char* s4 = nullptr)
+      : g(args), push(push_args), reduce(reduce_args), st0(s0), st1(s1), st2(s2), st3(s3), st4(s4), tid(threadIdx.x), lane(threadIdx.x & 63),
         wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wm(wave >> 1), wn(wave & 1) {}
 
   static TCCL_D int fresh(int v) {
@@ -337,8 +356,10 @@ struct GemmRole {
   // Each wavefront stages a 32-row slab (two row blocks) in its own 8 KiB window and writes it out
   // with 16-byte stores that are contiguous along the row; a wavefront's LDS operations execute in
   // the order issued, so nothing inside the loop waits for another wavefront.
-  template <int kPolicy>
-  TCCL_D void epilogue(int row0, int col0, const f32x4 (&acc)[4][4]) const {
+  // kReduce: the launch is a reduce-scatter that reduces here; `sums`: this sub-tile's rows are summed (its owner is this
+  // rank, or emulated, and the peers' partials are there).
+  template <int kPolicy, bool kReduce>
+  TCCL_D void epilogue(int row0, int col0, const f32x4 (&acc)[4][4], bool sums) const {
     constexpr int kEsz = sizeof(OutT);
     constexpr int kRowBytes = 64 * kEsz;       // one wave row: 64 columns
     constexpr int kChunks = kRowBytes / 16;    // 16-byte chunks per row (8 or 16)
@@ -353,6 +374,8 @@ struct GemmRole {
     // write-through when a communication workgroup will read it right after the signal.
     OutT* C = (OutT*)g.C + (int64_t)row0 * g.ldc + col0;
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void*)C, 0, 0xffffffffu, 0x00020000);
+    const int owner = kReduce ? row0 / reduce.shard_rows : 0;
+    const bool store = !(kReduce && sums && owner == reduce.rank && reduce.own_in_registers);
     __syncthreads();  // every wavefront has left the K loop's stages
 #pragma unroll
     for (int bi = 0; bi < 2; ++bi) {
@@ -390,7 +413,64 @@ struct GemmRole {
         lrow[r] = wm * 64 + bi * 32 + row;
         lcol[r] = wn * 64 + chunk * kPerChunk;
         live[r] = row0 + lrow[r] < g.M && col0 + lcol[r] < g.N;
+        if (kReduce && !store) continue;
         if (live[r]) __builtin_amdgcn_raw_buffer_store_b128(v[r], rc, (uint32_t)((lrow[r] * g.ldc + lcol[r]) * kEsz), 0, kPolicy);
+      }
+      if (kReduce && sums) {
+        // The owner's partial first, then the other ranks ascending; this rank's is the value as it would be stored.
+        const int64_t my_base = reduce.heap_bases[reduce.rank];
+        const __amdgpu_buffer_rsrc_t to = window((int64_t)(uintptr_t)reduce.out + (reduce.heap_bases[owner] - my_base) +
+                                                 (int64_t)(row0 - owner * reduce.shard_rows) * reduce.ld_out_bytes + (int64_t)col0 * 2);
+        // The addends of kBatch chunks from kPeers ranks are requested together.
+        constexpr int kBatch = 4, kPeers = 4;
+#pragma unroll
+        for (int b = 0; b < kRounds; b += kBatch) {
+          float sum[kBatch][kPerChunk];
+          for (int i0 = 0; i0 < reduce.world; i0 += kPeers) {
+            u32x4 w[kPeers][kBatch];
+#pragma unroll
+            for (int i = 0; i < kPeers; ++i) {
+              const int n = i0 + i, p = n == 0 ? owner : (n <= owner ? n - 1 : n);
+              if (n >= reduce.world) break;
+              const __amdgpu_buffer_rsrc_t from = window((int64_t)(uintptr_t)C + (reduce.heap_bases[p] - my_base));
+#pragma unroll
+              for (int r = 0; r < kBatch; ++r)
+                w[i][r] = p == reduce.rank ? v[b + r]
+                                           : ld16<kCoherent>(from, live[b + r] ? (uint32_t)((lrow[b + r] * g.ldc + lcol[b + r]) * kEsz) : 0u);
+            }
+#pragma unroll
+            for (int i = 0; i < kPeers; ++i) {
+              if (i0 + i >= reduce.world) break;
+#pragma unroll
+              for (int r = 0; r < kBatch; ++r) {
+                OutT e[kPerChunk];
+                __builtin_memcpy(e, &w[i][r], 16);
+#pragma unroll
+                for (int j = 0; j < kPerChunk; ++j) sum[r][j] = i0 + i == 0 ? (float)e[j] : sum[r][j] + (float)e[j];
+              }
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < kBatch; ++r) {
+            if (!live[b + r]) continue;
+            const uint32_t off = (uint32_t)(lrow[b + r] * reduce.ld_out_bytes + lcol[b + r] * 2);
+            uint16_t h[kPerChunk];
+#pragma unroll
+            for (int j = 0; j < kPerChunk; ++j)
+              h[j] = reduce.out_dtype == kBF16 ? __builtin_bit_cast(uint16_t, (__bf16)sum[r][j])
+                                               : __builtin_bit_cast(uint16_t, (_Float16)sum[r][j]);
+            if constexpr (kPerChunk == 4) {
+              typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+              u32x2 o;
+              __builtin_memcpy(&o, h, 8);
+              __builtin_amdgcn_raw_buffer_store_b64(o, to, off, 0, kStreaming);
+            } else {
+              u32x4 o;
+              __builtin_memcpy(&o, h, 16);
+              st16<kStreaming>(to, off, o);
+            }
+          }
+        }
       }
       // Fused push: the same chunks go to every peer's slice from the registers they sit in; the tile is
       // never read back.  The signal that follows the tile's last store covers these stores as well.
@@ -414,8 +494,8 @@ struct GemmRole {
   }
 
   // ---- one 128 x 128 sub-tile -------------------------------------------------------------------
-  template <int kPolicy, bool kBKMajor>
-  TCCL_D void subtile(int row0, int col0) const {
+  template <int kPolicy, bool kBKMajor, bool kReduce>
+  TCCL_D void subtile(int row0, int col0, int tile_id, const SignalArgs& s) const {
     f32x4 acc[4][4];  // cleared two registers per instruction
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -483,29 +563,65 @@ struct GemmRole {
       }
     }
     wait_vmem();  // the look-ahead loads must not land on the epilogue's staging
-    epilogue<kPolicy>(row0, col0, acc);
+    bool sums = false;
+    if constexpr (kReduce) {
+      const int owner = row0 / reduce.shard_rows;
+      sums = (owner == reduce.rank || reduce.emulate_peer) && peers_there(tile_id, s);
+    }
+    epilogue<kPolicy, kReduce>(row0, col0, acc, sums);
+  }
+
+  // The peers' partials of plan tile `tile_id` are published (one lane waits, bounded).
+  TCCL_D bool peers_there(int tile_id, const SignalArgs& s) const {
+    if (reduce.peers_resident) return true;
+    volatile int* verdict = (volatile int*)st2;  // the epilogue stages in st0 and st1
+    __syncthreads();  // every wavefront has left the K loop's stages
+    if (tid == 0) {
+      const int64_t deadline = now_ticks() + reduce.spin_ticks;
+      bool ok = true;
+      for (int p = 0; p < reduce.world && ok; ++p) {
+        if (p == reduce.rank) continue;
+        if (s.mode == kSignalTile) {
+          ok = tile_wait_ge<true>(translate_ptr(reduce.locks, reduce.rank, p, reduce.heap_bases), tile_id, s.epoch, deadline);
+        } else {
+          const int gid = s.group_table[tile_id];
+          const int32_t need = (int32_t)((uint32_t)s.epoch * (uint32_t)reduce.tile_counts[gid]);
+          ok = tile_wait_ge<true>(translate_ptr(reduce.counter, reduce.rank, p, reduce.heap_bases), gid, need, deadline);
+        }
+      }
+      if (!ok && reduce.fault) *reduce.fault = 1;
+      *verdict = ok ? 1 : 0;
+    }
+    __syncthreads();
+    return *verdict != 0;
   }
 
   // ---- persistent loop over plan tiles ----------------------------------------------------------
+  template <bool kReduce = false>
   TCCL_D void run(const SignalArgs& s, int wg, int num_wgs) const {
     const int total = g.tile_rows * g.tile_cols;
     for (int slot = wg; slot < total; slot += num_wgs) {
-      const int tile_id = tile_for_slot(slot, total, g.xcds, g.span);
-      const TileCoord tc = tile_coords(tile_id, g.tile_rows, g.tile_cols, g.group_m);
+      int tile_id = tile_for_slot(slot, total, g.xcds, g.span);
+      TileCoord tc = tile_coords(tile_id, g.tile_rows, g.tile_cols, g.group_m);
+      if constexpr (kReduce) {  // this rank's own rows come last: what its peers wait for comes first
+        tc.m += (reduce.rank + 1) % reduce.world * (g.tile_rows / reduce.world);
+        if (tc.m >= g.tile_rows) tc.m -= g.tile_rows;
+        tile_id = tile_id_of(tc.m, tc.n, g.tile_rows, g.tile_cols, g.group_m);
+      }
       for (int sm = 0; sm < g.block_m; sm += kTile)
         for (int sn = 0; sn < g.block_n; sn += kTile) {
           const int row0 = tc.m * g.block_m + sm, col0 = tc.n * g.block_n + sn;
           if (row0 >= g.M || col0 >= g.N) continue;
           if (s.mode == kSignalNone) {
             if (g.b_kmajor)
-              subtile<0, true>(row0, col0);
+              subtile<0, true, kReduce>(row0, col0, tile_id, s);
             else
-              subtile<0, false>(row0, col0);
+              subtile<0, false, kReduce>(row0, col0, tile_id, s);
           } else {
             if (g.b_kmajor)
-              subtile<kCoherent, true>(row0, col0);
+              subtile<kCoherent, true, kReduce>(row0, col0, tile_id, s);
             else
-              subtile<kCoherent, false>(row0, col0);
+              subtile<kCoherent, false, kReduce>(row0, col0, tile_id, s);
           }
         }
       if (s.mode != kSignalNone) {

@@ -20,19 +20,6 @@
 
 namespace tccl {
 
-// Epilogue of a reduce-scatter: see ReduceArgs of tccl_gemm256.h for the meaning of the members.
-struct StreamReduce {
-  int active, emulate_peer, peers_resident, own_in_registers;
-  int out_dtype;
-  char* out;
-  int64_t ld_out_bytes;
-  const int32_t* locks;
-  const int32_t* counter;
-  const int32_t* tile_counts;
-  int64_t* fault;
-  int64_t spin_ticks;
-};
-
 struct StreamArgs {
   const void* A;
   const void* B;
@@ -45,8 +32,8 @@ struct StreamArgs {
   // them.  `wrapped`: segment q is A (seg_rows x K) times columns [q N, (q + 1) N) of B.
   int seg_rows, wrapped;
   int first_seg;                   // segments are visited from this one on, wrapping around
-  int tiles_m, tiles_n, total;     // tiles per segment, along the columns, in all
-  int xcds, per_xcd;               // XCD x works on tiles [x per_xcd, (x + 1) per_xcd): neighbours share a slab of B in its L2
+  int tiles_m, tiles_n, segs;      // tiles down and across a segment; segments
+  int xcds, per_xcd;               // XCD x works on tiles [x per_xcd, (x + 1) per_xcd) of a segment: neighbours share a slab of B in its L2
   // Signals: a plan tile is published when the last of its tiles has been stored.
   SignalArgs s;
   uint32_t* arrivals;              // one per plan tile, zero between launches
@@ -54,7 +41,7 @@ struct StreamArgs {
   const int64_t* heap_bases;
   int rank, world;
   PushArgs push;
-  StreamReduce reduce;
+  EpilogueReduce reduce;
 };
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -220,17 +207,16 @@ struct StreamGemm {
   }
 
   TCCL_D void run(int slot) {
-    int tile = slot;
-    if (a.xcds > 1) tile = (slot % a.xcds) * a.per_xcd + slot / a.xcds;
-    if (tile >= a.total) return;
-    // Row tiles of one segment run fastest: the tiles that share a column slab of B sit on one XCD.
-    const int per_seg = a.tiles_m * a.tiles_n;
-    int seg = tile / per_seg;
-    const int in = tile - seg * per_seg;
+    // Every segment is spread over all XCDs (an XCD's link to memory would otherwise carry one owner's reductions alone).
+    // Within an XCD's part row tiles run fastest: those that share a column slab of B.
+    const int per_seg = a.tiles_m * a.tiles_n, slots_per_seg = a.xcds * a.per_xcd;
+    int seg = slot / slots_per_seg;
+    const int at = slot - seg * slots_per_seg;
+    const int in = at % a.xcds * a.per_xcd + at / a.xcds;
+    if (in >= per_seg) return;
     const int tn = in / a.tiles_m, tm = in - tn * a.tiles_m;
-    const int segs = a.total / per_seg;
     seg += a.first_seg;
-    if (seg >= segs) seg -= segs;
+    if (seg >= a.segs) seg -= a.segs;
     const int row_in = tm * kBM, col0 = tn * kBN;  // relative to the segment
     const int row0 = seg * a.seg_rows + row_in;    // row of C
 
@@ -363,17 +349,26 @@ struct StreamGemm {
 #pragma unroll
     for (int e = 0; e < 8; ++e) mine[e] = a.out_dtype == kF32 ? f[e] : (a.out_dtype == kF16 ? (float)(_Float16)f[e] : (float)(__bf16)f[e]);
     const int64_t my_base = a.heap_bases[a.rank];
-    for (int i = 0; i < a.world; ++i) {
-      const int p = i == 0 ? owner : (i <= owner ? i - 1 : i);
-      float v[8];
-      if (p == a.rank) {
+    constexpr int kPeers = 4;  // ranks whose addends are requested together
+    for (int i0 = 0; i0 < a.world; i0 += kPeers) {
+      float v[kPeers][8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = mine[e];
-      } else {
-        get(window(c_at + (a.heap_bases[p] - my_base)), off, v, a.out_dtype);
+      for (int i = 0; i < kPeers; ++i) {
+        const int n = i0 + i, p = n == 0 ? owner : (n <= owner ? n - 1 : n);
+        if (n >= a.world) break;
+        if (p == a.rank) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[i][e] = mine[e];
+        } else {
+          get(window(c_at + (a.heap_bases[p] - my_base)), off, v[i], a.out_dtype);
+        }
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sum[e] = i == 0 ? v[e] : sum[e] + v[e];
+      for (int i = 0; i < kPeers; ++i) {
+        if (i0 + i >= a.world) break;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] = i0 + i == 0 ? v[i][e] : sum[e] + v[i][e];
+      }
     }
     const int64_t out = (int64_t)(uintptr_t)a.reduce.out + (a.heap_bases[owner] - my_base) + (int64_t)row_in * a.reduce.ld_out_bytes + (int64_t)col0 * 2;
     put(window(out), (uint32_t)(row * a.reduce.ld_out_bytes + col * 2), sum, a.reduce.out_dtype, false);

@@ -35,9 +35,9 @@ int launch_t(StreamArgs& a, const CommArgs* comm, int comm_wgs, hipStream_t stre
   constexpr StreamShape s = kStreamShapes[kShape];
   a.tiles_m = (a.seg_rows + 16 * s.mb - 1) / (16 * s.mb);
   a.tiles_n = (a.N + 16 * s.nb - 1) / (16 * s.nb);
-  a.total = a.tiles_m * a.tiles_n * (a.M / a.seg_rows);
-  a.per_xcd = (a.total + a.xcds - 1) / a.xcds;
-  const int tile_wgs = a.per_xcd * a.xcds;
+  a.segs = a.M / a.seg_rows;
+  a.per_xcd = (a.tiles_m * a.tiles_n + a.xcds - 1) / a.xcds;
+  const int tile_wgs = a.segs * a.xcds * a.per_xcd;
   const dim3 block(s.waves * 64);
   if (comm)
     hipLaunchKernelGGL((stream_pull_kernel<InT, s.mb, s.nb, s.waves, kBKMajor>), dim3(tile_wgs + comm_wgs), block, 0, stream, a, *comm, tile_wgs);
