@@ -111,6 +111,9 @@ typedef struct tccl_gemm_desc {
  * row-major form are the two it meets in practice.  With column_shards = w, B has w * N columns. */
 #define TCCL_GEMM_B_KMAJOR 2
 
+/* Row-major B has n (0 .. 15, less than a 16-byte vector) rows fewer than K: they are taken as zero.  For a K that is
+ * no whole number of vectors: A is then a zero-filled copy, B may stay where it is.  flags |= n << this. */
+#define TCCL_GEMM_B_SHORT_SHIFT 8
 /* The launch's sync descriptor is the head of a tccl_sync_desc_arrivals. */
 #define TCCL_GEMM_ARRIVALS 4
 
@@ -223,6 +226,14 @@ int tccl_fill_i32(int32_t* words, int64_t n, int32_t value, void* stream);
 int tccl_pack_matrix(const void* src, int64_t stride_row, int64_t stride_col, int32_t rows, int32_t cols,
                      void* dst, int64_t ld_dst, int32_t dst_rows, int32_t dst_cols, int32_t elem_bytes,
                      void* stream);
+/* One or two such matrices (both operands of a GEMM) in one launch. */
+typedef struct tccl_pack_desc {
+  const void* src;
+  void* dst;
+  int64_t stride_row, stride_col, ld_dst;
+  int32_t rows, cols, dst_rows, dst_cols;
+} tccl_pack_desc;
+int tccl_pack_matrices(const tccl_pack_desc* matrices, int32_t n, int32_t elem_bytes, void* stream);
 /* Single-word primitives, one launch each, for tests of the device semantics
  * (sync/primitives.py:357-500, tileccl_v2/ipc.py:137-254).  result: device int32[1]. */
 int tccl_prim_signal(int32_t* locks, int32_t index, void* stream);

@@ -91,12 +91,10 @@ _PACKED: dict[tuple, torch.Tensor] = {}
 _PACKED_LIMIT = 8
 
 
-def pack_operand(t: torch.Tensor, rows: int, cols: int, role: str) -> torch.Tensor:
-    """``t`` as a dense ``rows x cols`` matrix (zero beyond ``t``'s own shape), written by one
-    ``tccl_pack_matrix`` launch on the current stream.  The buffer is kept per (role, shape, dtype,
-    stream) and reused by the next call with that key, which the stream orders behind this one's GEMM,
-    unless a descriptor that has not been dropped yet still points at it."""
-    key = (role, rows, cols, t.dtype, t.device, stream_ptr())
+def _pack_buffer(t: torch.Tensor, rows: int, cols: int, role: str, stream: int) -> torch.Tensor:
+    """A dense ``rows x cols`` buffer, kept per (role, shape, dtype, stream) and reused by the next call with that key, which
+    the stream orders behind this one's GEMM, unless a descriptor that has not been dropped yet still points at it."""
+    key = (role, rows, cols, t.dtype, t.device, stream)
     out = _PACKED.pop(key, None)
     if out is not None and sys.getrefcount(out) > 2:  # this name and the call's argument
         out = None
@@ -105,12 +103,27 @@ def pack_operand(t: torch.Tensor, rows: int, cols: int, role: str) -> torch.Tens
             _PACKED.pop(next(iter(_PACKED)))
         out = torch.empty((rows, cols), dtype=t.dtype, device=t.device)
     _PACKED[key] = out  # most recently used last
-    rc = _lib.load().tccl_pack_matrix(
-        ptr(t), int(t.stride(0)), int(t.stride(1)), int(t.shape[0]), int(t.shape[1]),
-        ptr(out), cols, rows, cols, t.element_size(), stream_ptr(),
-    )
-    _lib.check(rc, f"tccl_pack_matrix[{role}]")
     return out
+
+
+def _pack(jobs: "list[tuple[torch.Tensor, int, int, str]]") -> "list[torch.Tensor]":
+    """Each (tensor, rows, cols, role) as a dense ``rows x cols`` matrix, zero beyond the tensor's own shape: one
+    launch on the current stream."""
+    stream = stream_ptr()
+    descs = (_lib.PackDesc * len(jobs))()
+    outs = []
+    for d, (t, rows, cols, role) in zip(descs, jobs):
+        out = _pack_buffer(t, rows, cols, role, stream)
+        d.src, d.dst = t.data_ptr(), out.data_ptr()
+        d.stride_row, d.stride_col = t.stride()
+        d.ld_dst = cols
+        d.rows, d.cols = t.shape
+        d.dst_rows, d.dst_cols = rows, cols
+        outs.append(out)
+    rc = _lib.load().tccl_pack_matrices(descs, len(jobs), outs[0].element_size(), stream)
+    if rc:
+        _lib.check(rc, "tccl_pack_matrices")
+    return outs
 
 
 @dataclass(frozen=True, slots=True)
@@ -141,17 +154,21 @@ def operand_plan(A: torch.Tensor, B: torch.Tensor) -> OperandPlan:
     k_pad = (K + vec - 1) // vec * vec
     lda = int(A.stride(0)) if M > 1 else int(K)
     pack_a = k_pad != K or (K > 1 and A.stride(1) != 1) or lda < K or not _rows_vectorised(A, lda)
-    layout = _b_layout(B) if k_pad == K else None
+    layout = _b_layout(B)
+    if layout is not None and k_pad != K:  # a row-major B need not have the rows that A is filled up with
+        layout = (layout[0], (k_pad - K) << _lib.GEMM_B_SHORT_SHIFT) if not layout[1] else None
     ldb, flags = layout or (int(B.shape[1]), 0)
     return OperandPlan(pack_a, layout is None, int(k_pad), k_pad if pack_a else lda, ldb, flags)
 
 
 def planned_operands(plan: OperandPlan, A: torch.Tensor, B: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """(A, B) with the operands that ``plan`` says so packed on the current stream."""
+    if plan.pack_a and plan.pack_b:
+        return tuple(_pack([(A, A.shape[0], plan.K, "A"), (B, plan.K, B.shape[1], "B")]))
     if plan.pack_a:
-        A = pack_operand(A, A.shape[0], plan.K, "A")
+        (A,) = _pack([(A, A.shape[0], plan.K, "A")])
     if plan.pack_b:
-        B = pack_operand(B, plan.K, B.shape[1], "B")
+        (B,) = _pack([(B, plan.K, B.shape[1], "B")])
     return A, B
 
 

@@ -64,6 +64,7 @@ class GemmDesc(C.Structure):
 GEMM_OWN_ROWS_IN_REGISTERS = 1  # TCCL_GEMM_OWN_ROWS_IN_REGISTERS
 GEMM_B_KMAJOR = 2  # TCCL_GEMM_B_KMAJOR
 GEMM_ARRIVALS = 4  # TCCL_GEMM_ARRIVALS
+GEMM_B_SHORT_SHIFT = 8  # TCCL_GEMM_B_SHORT_SHIFT
 STAGED_ALLREDUCE, STAGED_ALLGATHER, STAGED_REDUCE_SCATTER, STAGED_BROADCAST, STAGED_SCATTER = range(5)  # TCCL_STAGED_*
 
 
@@ -115,6 +116,20 @@ class TransportDesc(C.Structure):
     ]
 
 
+class PackDesc(C.Structure):
+    _fields_ = [
+        ("src", C.c_void_p),
+        ("dst", C.c_void_p),
+        ("stride_row", C.c_int64),
+        ("stride_col", C.c_int64),
+        ("ld_dst", C.c_int64),
+        ("rows", C.c_int32),
+        ("cols", C.c_int32),
+        ("dst_rows", C.c_int32),
+        ("dst_cols", C.c_int32),
+    ]
+
+
 STATIC_MAX_TILES, STATIC_MAX_GROUPS = 16384, 64
 
 
@@ -143,6 +158,7 @@ SIGNATURES = {
     "tccl_heap_destroy": (C.c_int, [_vp]),
     "tccl_fill_i32": (C.c_int, [_vp, _i64, _i32, _vp]),
     "tccl_pack_matrix": (C.c_int, [_vp, _i64, _i64, _i32, _i32, _vp, _i64, _i32, _i32, _i32, _vp]),
+    "tccl_pack_matrices": (C.c_int, [_P(PackDesc), _i32, _i32, _vp]),
     "tccl_prim_signal": (C.c_int, [_vp, _i32, _vp]),
     "tccl_prim_signal_add": (C.c_int, [_vp, _i32, _i32, _vp, _vp]),
     "tccl_prim_try_wait": (C.c_int, [_vp, _i32, _i32, _i32, _vp, _vp]),

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256, 3) void fused_kernel(tccl::GemmArgs g, tccl::S
 // Launches without communication workgroups: the GEMM alone, pushes from the epilogue, reductions in it
 // (kReduce).  Nothing has to fit beside two of them on a CU, so they take five stages (80 KiB): a load then has three
 // steps and a half to arrive instead of one and a half.  1000 x 2064 x 1008 with its push: 18.3 us with three stages,
-// MEASURED128 with five.
+// 16.4 with five (traced).
 template <typename InT, typename OutT, bool kReduce>
 __global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::PushArgs push, tccl::EpilogueReduce reduce) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -156,25 +156,52 @@ __global__ void fill_kernel(int32_t* w, int64_t n, int32_t v) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) w[i] = v;
 }
 
-// Strided matrix -> dense rows, one 64 x 64 patch per workgroup through LDS: the patch is read along
-// whichever source index is closer in memory and written along the destination's rows, so both sides
-// move whole lines whatever the source's strides are.  Elements outside the source are written as zero.
+// Strided matrices -> dense rows, one 64 x 64 patch per workgroup through LDS: the patch is read along
+// whichever source index is closer in memory and written along the destination's rows in 16-byte vectors, so
+// both sides move whole lines whatever the source's strides are.  Elements outside the source are written as
+// zero.  Both operands of a GEMM are one launch, and a thread's sixteen reads are all requested before the first is
+// used: 1000 x 1003 transposed and 1003 x 2064 took 9.8 and 10.4 us one after the other, 5.8 us together.
+struct PackJobs {
+  tccl_pack_desc job[2];
+  int first[2];  // first workgroup of each job
+};
 template <typename T>
-__global__ __launch_bounds__(256) void pack_kernel(const T* src, int64_t stride_row, int64_t stride_col, int rows, int cols,
-                                                   T* dst, int64_t ld_dst, int dst_rows, int dst_cols) {
-  __shared__ T patch[64][65];
-  const int r0 = (int)blockIdx.y * 64, c0 = (int)blockIdx.x * 64;
+__global__ __launch_bounds__(256) void pack_kernel(PackJobs jobs, int n) {
+  constexpr int kVec = 16 / (int)sizeof(T), kPitch = 64 + kVec;
+  __shared__ __attribute__((aligned(16))) T patch[64 * kPitch];
+  const int which = n > 1 && (int)blockIdx.x >= jobs.first[1] ? 1 : 0;
+  const tccl_pack_desc& p = jobs.job[which];
+  const int wg = (int)blockIdx.x - jobs.first[which];
+  const int across = (p.dst_cols + 63) / 64;
+  const int r0 = wg / across * 64, c0 = wg % across * 64;
   const int fast = (int)threadIdx.x & 63, slow = (int)threadIdx.x >> 6;
-  const bool along_cols = stride_col <= stride_row;
-  for (int i = slow; i < 64; i += 4) {
-    const int r = along_cols ? i : fast, c = along_cols ? fast : i;
-    T v = 0;
-    if (r0 + r < rows && c0 + c < cols) v = src[(int64_t)(r0 + r) * stride_row + (int64_t)(c0 + c) * stride_col];
-    patch[r][c] = v;
+  const bool along_cols = p.stride_col <= p.stride_row;
+  const T* src = (const T*)p.src;
+  T v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int r = along_cols ? slow + 4 * i : fast, c = along_cols ? fast : slow + 4 * i;
+    const bool live = r0 + r < p.rows && c0 + c < p.cols;
+    v[i] = live ? src[(int64_t)(r0 + r) * p.stride_row + (int64_t)(c0 + c) * p.stride_col] : (T)0;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int r = along_cols ? slow + 4 * i : fast, c = along_cols ? fast : slow + 4 * i;
+    patch[r * kPitch + c] = v[i];
   }
   __syncthreads();
-  for (int i = slow; i < 64; i += 4)
-    if (r0 + i < dst_rows && c0 + fast < dst_cols) dst[(int64_t)(r0 + i) * ld_dst + c0 + fast] = patch[i][fast];
+  T* dst = (T*)p.dst;
+  const bool vectors = (((uintptr_t)p.dst | (uint64_t)(p.ld_dst * (int64_t)sizeof(T))) & 15) == 0;
+  for (int u = (int)threadIdx.x; u < 64 * (64 / kVec); u += 256) {
+    const int r = u / (64 / kVec), c = u % (64 / kVec) * kVec;
+    if (r0 + r >= p.dst_rows || c0 + c >= p.dst_cols) continue;
+    T* to = dst + (int64_t)(r0 + r) * p.ld_dst + c0 + c;
+    if (vectors && c0 + c + kVec <= p.dst_cols) {
+      *(tccl::u32x4*)to = *(const tccl::u32x4*)&patch[r * kPitch + c];
+    } else {
+      for (int e = 0; e < kVec && c0 + c + e < p.dst_cols; ++e) to[e] = patch[r * kPitch + c + e];
+    }
+  }
 }
 
 __global__ void prim_signal_kernel(int32_t* locks, int i) { tccl::tile_signal(locks, i); }
@@ -220,6 +247,9 @@ int check_gemm(const tccl_gemm_desc* d, bool ragged_shards = false) {
   if (d->K % in_vec) return fail(TCCL_ERR_UNSUPPORTED, "gemm: K=%d must be a multiple of %d", d->K, in_vec);
   if (d->N % 8) return fail(TCCL_ERR_UNSUPPORTED, "gemm: N=%d must be a multiple of 8", d->N);
   const bool b_kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) != 0;
+  const int b_short = (d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15;
+  if (b_short >= in_vec || b_short >= d->K || (b_short && b_kmajor))
+    return fail(TCCL_ERR_INVALID, "gemm: B can lack fewer than %d rows of K, and only row-major (%d)", in_vec, b_short);
   if (d->lda < d->K || d->ldb < (b_kmajor ? (int64_t)d->K : (int64_t)d->N * shards) || d->ldc < d->N)
     return fail(TCCL_ERR_INVALID, "gemm: leading dimension smaller than the row length");
   if (d->lda % in_vec || d->ldb % in_vec || d->ldc % out_vec || !aligned16(d->A) || !aligned16(d->B) || !aligned16(d->C))
@@ -272,6 +302,7 @@ int build_gemm_args(const tccl_gemm_desc* d, const tccl_device_info& dev, tccl::
   }
   g->wrap_rows = d->column_shards > 1 ? d->M / d->column_shards : 0;
   g->b_kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) ? 1 : 0;
+  g->b_short = (d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15;
   return 0;
 }
 
@@ -824,6 +855,7 @@ void build_stream(const tccl_gemm_desc* d, const tccl::GemmArgs& g, int64_t seg_
   a->M = d->M;
   a->N = d->N;
   a->K = d->K;
+  a->b_short = g.b_short;
   a->alpha = d->alpha;
   a->out_dtype = d->out_dtype;
   a->seg_rows = (int)seg_rows;
@@ -1200,29 +1232,45 @@ int tccl_fill_i32(int32_t* words, int64_t n, int32_t value, void* stream) {
   return 0;
 }
 
-int tccl_pack_matrix(const void* src, int64_t stride_row, int64_t stride_col, int32_t rows, int32_t cols, void* dst,
-                     int64_t ld_dst, int32_t dst_rows, int32_t dst_cols, int32_t elem_bytes, void* stream) {
-  if (dst_rows <= 0 || dst_cols <= 0) return 0;
-  if (!src || !dst) return fail(TCCL_ERR_INVALID, "pack_matrix: NULL pointer");
-  if (rows < 0 || cols < 0 || rows > dst_rows || cols > dst_cols || stride_row < 0 || stride_col < 0 || ld_dst < dst_cols)
-    return fail(TCCL_ERR_INVALID, "pack_matrix: source %dx%d (strides %lld, %lld) does not fit a %dx%d destination of pitch %lld",
-                rows, cols, (long long)stride_row, (long long)stride_col, dst_rows, dst_cols, (long long)ld_dst);
-  const dim3 grid((unsigned)((dst_cols + 63) / 64), (unsigned)((dst_rows + 63) / 64));
-  if (grid.y > 65535u) return fail(TCCL_ERR_UNSUPPORTED, "pack_matrix: more than 65535 x 64 rows");
+int tccl_pack_matrices(const tccl_pack_desc* descs, int32_t n, int32_t elem_bytes, void* stream) {
+  if (n <= 0) return 0;
+  if (!descs || n > 2) return fail(TCCL_ERR_INVALID, "pack_matrices: one or two matrices, got %d", n);
+  PackJobs jobs;
+  memset(&jobs, 0, sizeof jobs);
+  int kept = 0;
+  int64_t wgs = 0;
+  for (int i = 0; i < n; ++i) {
+    const tccl_pack_desc& p = descs[i];
+    if (p.dst_rows <= 0 || p.dst_cols <= 0) continue;
+    if (!p.src || !p.dst) return fail(TCCL_ERR_INVALID, "pack_matrix: NULL pointer");
+    if (p.rows < 0 || p.cols < 0 || p.rows > p.dst_rows || p.cols > p.dst_cols || p.stride_row < 0 || p.stride_col < 0 || p.ld_dst < p.dst_cols)
+      return fail(TCCL_ERR_INVALID, "pack_matrix: source %dx%d (strides %lld, %lld) does not fit a %dx%d destination of pitch %lld",
+                  p.rows, p.cols, (long long)p.stride_row, (long long)p.stride_col, p.dst_rows, p.dst_cols, (long long)p.ld_dst);
+    jobs.job[kept] = p;
+    jobs.first[kept] = (int)wgs;
+    ++kept;
+    wgs += ((int64_t)p.dst_rows + 63) / 64 * (((int64_t)p.dst_cols + 63) / 64);
+    if (wgs > 0x7fffffffll) return fail(TCCL_ERR_UNSUPPORTED, "pack_matrix: more than 2^31 patches of 64 x 64");
+  }
+  if (kept == 0) return 0;
   const hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((unsigned)wgs), block(256);
   if (elem_bytes == 1)
-    hipLaunchKernelGGL(pack_kernel<uint8_t>, grid, dim3(256), 0, st, (const uint8_t*)src, stride_row, stride_col, rows, cols,
-                       (uint8_t*)dst, ld_dst, dst_rows, dst_cols);
+    hipLaunchKernelGGL(pack_kernel<uint8_t>, grid, block, 0, st, jobs, kept);
   else if (elem_bytes == 2)
-    hipLaunchKernelGGL(pack_kernel<uint16_t>, grid, dim3(256), 0, st, (const uint16_t*)src, stride_row, stride_col, rows, cols,
-                       (uint16_t*)dst, ld_dst, dst_rows, dst_cols);
+    hipLaunchKernelGGL(pack_kernel<uint16_t>, grid, block, 0, st, jobs, kept);
   else if (elem_bytes == 4)
-    hipLaunchKernelGGL(pack_kernel<uint32_t>, grid, dim3(256), 0, st, (const uint32_t*)src, stride_row, stride_col, rows, cols,
-                       (uint32_t*)dst, ld_dst, dst_rows, dst_cols);
+    hipLaunchKernelGGL(pack_kernel<uint32_t>, grid, block, 0, st, jobs, kept);
   else
     return fail(TCCL_ERR_INVALID, "pack_matrix: elem_bytes=%d must be 1, 2 or 4", elem_bytes);
   TCCL_HIP(hipGetLastError());
   return 0;
+}
+
+int tccl_pack_matrix(const void* src, int64_t stride_row, int64_t stride_col, int32_t rows, int32_t cols, void* dst,
+                     int64_t ld_dst, int32_t dst_rows, int32_t dst_cols, int32_t elem_bytes, void* stream) {
+  const tccl_pack_desc p{src, dst, stride_row, stride_col, ld_dst, rows, cols, dst_rows, dst_cols};
+  return tccl_pack_matrices(&p, 1, elem_bytes, stream);
 }
 
 int tccl_prim_signal(int32_t* locks, int32_t index, void* stream) {

@@ -80,6 +80,8 @@ struct GemmArgs {
   int wrap_rows;
   // B is k-major: element (k, n) at B[n * ldb + k] (the `.t()` view of an (N, K) tensor).
   int b_kmajor;
+  // Row-major B lacks its last b_short of the K rows: they read as zero (A is zero there as well).
+  int b_short;
 };
 
 // Where a tile whose first output row is row0 and first output column col0 reads its operands.
@@ -233,7 +235,7 @@ struct GemmRole {
     const InT* A = (const InT*)g.A + (int64_t)o.a_row * g.lda;
     const InT* B = (const InT*)g.B + (kBKMajor ? (int64_t)o.b_col * g.ldb : (int64_t)o.b_col);
     s.a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(((int64_t)(o.a_rows - 1 - o.a_row) * g.lda + g.K) * 2), 0x00020000);
-    const int64_t b_elems = kBKMajor ? (int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K : (int64_t)(g.K - 1) * g.ldb + (o.b_cols - o.b_col);
+    const int64_t b_elems = kBKMajor ? (int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K : (int64_t)(g.K - 1 - g.b_short) * g.ldb + (o.b_cols - o.b_col);
     s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(b_elems * 2), 0x00020000);
     // Bits 1 and 2 of a row's number come from the lane alone (a piece starts on a multiple of 16).
     const int kc = (ln & 3) ^ ((ln >> 3) & 3);

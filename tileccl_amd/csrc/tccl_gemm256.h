@@ -351,7 +351,7 @@ struct Gemm256 {
     if constexpr (kBKMajor)
       s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K) * kEsz), 0x00020000);
     else
-      s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(g.K - 1) * g.ldb + (o.b_cols - o.b_col)) * kEsz), 0x00020000);
+      s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(g.K - 1 - g.b_short) * g.ldb + (o.b_cols - o.b_col)) * kEsz), 0x00020000);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int row = 8 * (4 * wave + i) + (lane >> 3);

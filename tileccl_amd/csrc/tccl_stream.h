@@ -26,6 +26,7 @@ struct StreamArgs {
   char* C;
   int64_t lda, ldb, ldc;  // elements
   int M, N, K;            // C is M x N
+  int b_short;            // rows that a row-major B lacks at the end of K: they read as zero
   float alpha;
   int out_dtype;
   // Rows come in segments (the owners' shards of a reduce-scatter, stacked column shards); tiles do not straddle
@@ -236,7 +237,7 @@ struct StreamGemm {
       off_b = (uint32_t)(lane >> 3) * pitch_b + (uint32_t)(lane & 7) * 16u;
     } else {
       const InT* B = (const InT*)a.B + b_col;
-      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(a.K - 1) * a.ldb + cols_left) * 2), 0x00020000);
+      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(a.K - 1 - a.b_short) * a.ldb + cols_left) * 2), 0x00020000);
       const int c = lane % (2 * kNB);
       off_b = 8 * c < cols_left ? (uint32_t)(lane / (2 * kNB)) * pitch_b + (uint32_t)c * 16u : kOutside;
     }
