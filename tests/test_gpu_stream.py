@@ -38,6 +38,24 @@ def test_gemm_alone(lib, M, N, K, dtype, out, layout):
         assert bool((got[M] == 7.0).all())
 
 
+@pytest.mark.parametrize("layout", ["kn", "nk"])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (17, 1008, 528), (100, 1040, 2000), (190, 1008, 1008), (250, 2000, 464), (1000, 1040, 208),
+                                   (1500, 2000, 400)])
+def test_gemm_alone_e4m3(lib, M, N, K, layout):
+    """The same shapes with e4m3 inputs (128 k per block), the last one in two 64 x 64 tiles per CU."""
+    from tileccl_amd import _launch, _lib
+    from tileccl_amd.v2 import SymmetricHeap
+
+    with SymmetricHeap.create_all(64 << 20, 1)[0] as heap:
+        A, B = (seeded(s, k, torch.float32, scale=64.0).clamp(-448, 448).to(torch.float8_e4m3fn) for s, k in (((M, K), 1), ((K, N), 2)))
+        got = torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda")
+        d = _launch.gemm_desc(into_heap(heap, A), weight(heap, B, layout), got[:M], alpha=K**-0.5 / 4096)
+        _lib.check(lib.tccl_gemm(C.byref(d), _launch.stream_ptr()), "tccl_gemm")
+        torch.cuda.synchronize()
+        assert_gemm_close(got[:M], (A.float() @ B.float()) * (K**-0.5 / 4096), tight=1e-3)
+        assert bool((got[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("variant", ["s1", "s2"])
 @pytest.mark.parametrize("world,layout", [(2, "kn"), (3, "nk")])
 @pytest.mark.parametrize("M,N,K", SHAPES)

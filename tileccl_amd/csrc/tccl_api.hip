@@ -796,9 +796,17 @@ int64_t stream_tiles(int shape, int64_t seg_rows, int64_t segs, int64_t N) {
   return (seg_rows + bm - 1) / bm * segs * ((N + bn - 1) / bn);
 }
 
-double stream_cost(int shape, int64_t K) {
+double stream_cost(int shape, int64_t k_bytes, int64_t rounds) {
   const tccl::StreamShape& s = tccl::kStreamShapes[shape];
-  return kLaunchUs + (double)(16 * (s.mb + s.nb) * 2 * K) / 1024.0 / kStreamCost[shape].rate + kStreamCost[shape].sums;
+  return kLaunchUs + (double)rounds * ((double)(16 * (s.mb + s.nb) * k_bytes) / 1024.0 / kStreamCost[shape].rate + kStreamCost[shape].sums);
+}
+
+// The 256 x 256-tile kernel with e4m3 inputs: K steps of 128, 1.05 us each, and 1 us (half the CUs storing: 4.5 us) of
+// epilogue per tile.  16 .. 2048 x 2048 x 4096 .. 512: within 10 %.
+double tile256_f8_cost(int64_t M, int64_t N, int64_t K, int cus) {
+  const int64_t tiles = (M + 255) / 256 * ((N + 255) / 256);
+  const double load = tiles >= cus / 2 ? 1.0 : (double)tiles / (cus / 2);
+  return kLaunchUs + (double)((tiles + cus - 1) / cus) * ((double)((K + 127) / 128) * 1.05 + 1.0 + 3.5 * load);
 }
 
 // The 128 x 128-tile kernel: K steps of 32, 0.19 us each with a few tiles and 0.3 us once every CU has one; its fused
@@ -820,22 +828,25 @@ uint32_t* arrival_words(const tccl_gemm_desc* d, const tccl_sync_desc* sync) {
 // streaming kernel does not have (a tile, workgroup counts, clock stamps).  Signals need the caller's arrival words.
 // At most one tile per CU: beyond that the larger tiles are about as quick (1000 x 2064 x 1000 in 528 tiles: 17.5 against
 // 13 .. 18 us), and the workgroups of a reduce-scatter that wait for a peer's partials are all resident beside the peer's.
+// e4m3 inputs have no 128 x 128-tile kernel to turn to: up to four 64 x 64 tiles per CU (two are resident).
 int stream_shape(const tccl_gemm_desc* d, const tccl_sync_desc* sync, const tccl_transport_desc* tr, int variant, int64_t seg_rows,
                  const tccl_device_info& dev) {
-  if (d->in_dtype != TCCL_F16 && d->in_dtype != TCCL_BF16) return -1;
-  if (d->out_dtype != TCCL_F32 && d->out_dtype != d->in_dtype) return -1;
+  const bool f8 = d->in_dtype == TCCL_F8E4M3;
+  if (!f8 && d->out_dtype != TCCL_F32 && d->out_dtype != d->in_dtype) return -1;
   if (d->macro_tile != 0 || d->num_wgs > 0 || (tr && tr->num_comm_wgs > 0)) return -1;
   const bool fused = variant != TCCL_S0_BULK;
   if (fused) {
     if (!arrival_words(d, sync)) return -1;
     if (sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock || sync->trace_comm_counter) return -1;
   }
-  if (use_macro(d, dev, fused)) return -1;
+  if (!f8 && use_macro(d, dev, fused)) return -1;
+  const int cus = dev.compute_units;
   int best = -1;
-  double least = tile128_cost(d->M, d->N, d->K, dev.compute_units);
+  double least = f8 ? tile256_f8_cost(d->M, d->N, d->K, cus) : tile128_cost(d->M, d->N, d->K, cus);
   for (int i = 0; i < tccl::kStreamShapeCount; ++i) {
-    if (stream_tiles(i, seg_rows, d->M / seg_rows, d->N) > dev.compute_units) continue;
-    const double us = stream_cost(i, d->K);
+    const int64_t tiles = stream_tiles(i, seg_rows, d->M / seg_rows, d->N);
+    if (tiles > (f8 && i == tccl::kStreamShapeCount - 1 ? 4 * cus : cus)) continue;
+    const double us = stream_cost(i, d->K * (f8 ? 1 : 2), (tiles + cus - 1) / cus);
     if (us < least) {
       least = us;
       best = i;
@@ -957,7 +968,10 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     // Tiles of a reduce-scatter must not straddle two owners' rows.
     const int64_t seg = g.wrap_rows > 0 ? g.wrap_rows : (c.op == tccl::kOpReduceScatter ? d->M / c.world : d->M);
     const int shape = stream_shape(d, sync, tr, variant, seg, dev);
-    if (shape >= 0) return run_stream(d, c, sync, variant, shape, seg, dev, g, stream);
+    // Tiles that wait for a peer (the own rows', the last ones) leave every CU room for the peer's launch.
+    const bool waits = c.op == tccl::kOpReduceScatter && variant != TCCL_S0_BULK && !c.peers_resident && c.world > 1;
+    if (shape >= 0 && !(waits && stream_tiles(shape, seg, 1, d->N) > dev.compute_units))
+      return run_stream(d, c, sync, variant, shape, seg, dev, g, stream);
   }
   const int total_tiles = g.tile_rows * g.tile_cols;
   const int compute = default_gemm_wgs(d, dev, total_tiles);

@@ -30,7 +30,7 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 enum OpKind { kOpNone = 0, kOpAllScatter = 1, kOpAllGather = 2, kOpReduceScatter = 3 };
 enum Granularity { kPerTile = 1, kPerGroup = 2 };
 enum { kDirPush = 1, kDirPull = 2 };
-enum { kF16 = 0, kBF16 = 1, kF32 = 2 };  // the codes of include/tileccl_hip.h
+enum { kF16 = 0, kBF16 = 1, kF32 = 2, kF8E4M3 = 3 };  // the codes of include/tileccl_hip.h
 
 struct CommArgs {
   int op, granularity, directions;

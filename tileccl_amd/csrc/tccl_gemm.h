@@ -171,6 +171,23 @@ struct Mfma<__bf16> {
   static TCCL_D f32x4 run16(Vec a, Vec b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 };
 
+// OCP fp8 e4m3 ("e4m3fn"), the 8-bit input type of gfx950's v_mfma_f32_32x32x64_f8f6f4.
+struct fp8e4m3 {
+  uint8_t bits;
+};
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+#if defined(__HIP_DEVICE_COMPILE__)
+template <>
+struct Mfma<fp8e4m3> {
+  typedef i32x8 Vec;  // 32 consecutive k of one row / column
+  // cbsz = blgp = 0 selects e4m3 for both operands; zero scale operands select the unscaled form.
+  static TCCL_D f32x16 run(Vec a, Vec b, f32x16 c) { return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0); }
+  // 16 x 16 x 128: lane l holds 32 consecutive k (group l / 16) of row / column l % 16 and gets
+  // D[4 * (l / 16) + e][l % 16], e = 0..3.
+  static TCCL_D f32x4 run16(Vec a, Vec b, f32x4 c) { return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0); }
+};
+#endif
+
 // fp32 -> output element, round to nearest even (what a cast of the accumulator does in
 // the reference, gemm.py:167 / bulk_sync.py:238).
 template <typename OutT>

@@ -1,4 +1,4 @@
-// Streaming MFMA GEMM for gfx950 (CDNA4), 16-bit inputs: small outputs, where the large-tile kernels leave
+// Streaming MFMA GEMM for gfx950 (CDNA4), 16-bit and e4m3 inputs: small outputs, where the large-tile kernels leave
 // most of the device idle (decoding rows, short prompts, ragged and narrow problems).
 //
 // One workgroup produces one output tile of (16 kMB) x (16 kNB); its kWaves wavefronts each take every
@@ -49,7 +49,8 @@ struct StreamArgs {
 template <typename InT, int kMB, int kNB, int kWaves, bool kBKMajor>
 struct StreamGemm {
   typedef typename Mfma<InT>::Vec Vec;
-  static_assert(sizeof(InT) == 2, "16-bit inputs");
+  static constexpr int kEsz = sizeof(InT), kVec = 16 / kEsz;  // elements per 16-byte chunk
+  static constexpr int kKB = 128 / kEsz;                      // K per block: 64, or 128 for e4m3
   static constexpr int kBM = 16 * kMB, kBN = 16 * kNB;
   // K blocks of 64 in flight per wavefront, within the registers that kWaves wavefronts leave each.
   static constexpr int kBudget = (kWaves >= 16 ? 64 : 128) / ((kMB + kNB) * 8);
@@ -71,14 +72,15 @@ struct StreamGemm {
 
   static TCCL_D uint32_t clamp_u32(int64_t v) { return v > 0xfffffff0ll ? 0xfffffff0u : (v < 0 ? 0u : (uint32_t)v); }
 
-  // One K block of 64 as it is loaded, 16 bytes per lane with neighbouring lanes on neighbouring addresses (a
+  // One K block as it is loaded, 16 bytes per lane with neighbouring lanes on neighbouring addresses (a
   // load whose lanes 0..3 lie in four rows takes in a third of the bytes per clock: 34 against 104 KB/us per CU).
   //   A, k-major B: rows of 128 bytes; instruction h of a 16-row block covers its rows 8 h + l / 8, chunk l % 8.
-  //   Row-major B: 64 k rows of 32 kNB bytes; instruction h covers rows h * kRowsPerLoad + l / (2 kNB).
+  //   Row-major B: 64 k rows of 32 kNB bytes (e4m3: 128 of 16 kNB); instruction h covers kRowsPerLoad of them.
   struct Block {
     u32x4 a[2 * kMB], b[2 * kNB];
   };
-  static constexpr int kRowsPerLoad = 32 / kNB;
+  static constexpr int kRowBytes = 16 * kNB * kEsz, kRowLanes = kRowBytes / 16;  // of a k row of row-major B in a tile
+  static constexpr int kRowsPerLoad = 64 / kRowLanes;
   static constexpr uint32_t kOutside = 0xffffff00u;  // beyond every buffer: reads as zero
 
   __amdgpu_buffer_rsrc_t ra, rb;
@@ -88,7 +90,7 @@ struct StreamGemm {
   // kTail: the block may reach past K; a chunk, or a row of B, at k >= K reads as zero.
   template <bool kTail>
   TCCL_D void load(Block& v, int kb) const {
-    const bool past = kTail && kb * 64 + 8 * (lane & 7) >= a.K;
+    const bool past = kTail && kb * kKB + kVec * (lane & 7) >= a.K;
 #pragma unroll
     for (int h = 0; h < 2 * kMB; ++h) {
       const uint32_t o = off_a + (uint32_t)(8 * h) * pitch_a + (uint32_t)kb * 128u;
@@ -100,8 +102,8 @@ struct StreamGemm {
         const uint32_t o = off_b + (uint32_t)(8 * h) * pitch_b + (uint32_t)kb * 128u;
         v.b[h] = __builtin_amdgcn_raw_buffer_load_b128(rb, past ? kOutside : o, 0, 0);
       } else {
-        const int k = kb * 64 + h * kRowsPerLoad;  // and the lane's row
-        const bool none = off_b == kOutside || (kTail && k + lane / (2 * kNB) >= a.K);
+        const int k = kb * kKB + h * kRowsPerLoad;  // and the lane's row
+        const bool none = off_b == kOutside || (kTail && k + lane / kRowLanes >= a.K);
         v.b[h] = __builtin_amdgcn_raw_buffer_load_b128(rb, none ? kOutside : off_b + (uint32_t)k * pitch_b, 0, 0);
       }
     }
@@ -110,14 +112,15 @@ struct StreamGemm {
   // Load order -> operand order through this wavefront's own LDS (a wavefront's LDS operations execute in the
   // order issued: no barrier).
   //   Rows of 128 bytes: chunk c of row r in slot c ^ ((r >> 1) & 7), read with ds_read_b128.
-  //   Row-major B: the 32-byte units of k row k permuted by swizzle(k), so that the eight rows that 32 lanes of a
-  //   transposing read (ds_read_b64_tr_b16) touch at a time lie in different banks.
+  //   Row-major B: the 32-byte units (e4m3: 16-byte chunks) of k row k permuted by swizzle(k), so that the rows that
+  //   32 lanes of a transposing read (ds_read_b64_tr_b16, _tr_b8) touch at a time lie in different banks.
   static TCCL_D int swizzle(int k) {
+    if constexpr (kEsz == 1) return kNB == 4 ? ((k >> 2) & 1) | (((k >> 4) & 1) << 1) : (kNB == 2 ? (k >> 4) & 1 : 0);
     if constexpr (kNB >= 8) return (2 * (k & 3)) ^ ((k >> 3) & 1);
     if constexpr (kNB == 4) return (k & 2) ^ ((k >> 3) & 1);
     return kNB == 2 ? (k >> 3) & 1 : 0;
   }
-  static TCCL_D int row_at(int k) { return kNB == 1 ? k ^ (4 * ((k >> 3) & 1)) : k; }
+  static TCCL_D int row_at(int k) { return kNB == 1 && kEsz == 2 ? k ^ (4 * ((k >> 3) & 1)) : k; }
   TCCL_D void stage(const Block& v) const {
     char* at = lds + wave * kWaveBytes;
 #pragma unroll
@@ -132,36 +135,62 @@ struct StreamGemm {
         const int r = 8 * h + (lane >> 3);
         *(u32x4*)(at + r * 128 + (((lane & 7) ^ ((r >> 1) & 7)) << 4)) = v.b[h];
       } else {
-        const int k = h * kRowsPerLoad + lane / (2 * kNB), c = lane % (2 * kNB);
-        *(u32x4*)(at + row_at(k) * (32 * kNB) + ((c ^ (2 * swizzle(k))) << 4)) = v.b[h];
+        const int k = h * kRowsPerLoad + lane / kRowLanes, c = lane % kRowLanes;
+        *(u32x4*)(at + row_at(k) * kRowBytes + ((c ^ (kEsz * swizzle(k))) << 4)) = v.b[h];
       }
     }
   }
-  // Operand of 16-row block `block` (A, k-major B), 32-k half h: lane l holds k 8 (l / 16) .. + 7 of row l % 16.
-  TCCL_D Vec staged(int block, int h) const {
-    return *(const Vec*)(lds + wave * kWaveBytes + block * 2048 + i16 * 128 + (((4 * h + kg) ^ ((i16 >> 1) & 7)) << 4));
+  // 16-byte chunk 4 h + l / 16 of row l % 16 of 16-row block `block` (A, k-major B): the 16-bit operand of 32-k half h (k
+  // 8 (l / 16) .. + 7 of it); the e4m3 operand of a whole block is both (k 16 (l / 16) .. + 15 and 64 + that).
+  TCCL_D u32x4 chunk(int block, int h) const {
+    return *(const u32x4*)(lds + wave * kWaveBytes + block * 2048 + i16 * 128 + (((4 * h + kg) ^ ((i16 >> 1) & 7)) << 4));
   }
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef short s16x8 __attribute__((ext_vector_type(8)));
   typedef __attribute__((address_space(3))) s16x4 LdsQuad;
-  // Column block j of row-major B: two transposing reads (k rows 8 kg + 0 .. 3 and + 4 .. 7).
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) i32x2 LdsPair;
+  // Column block j of row-major B, transposed on the way out: 16-bit, 32-k half h, two reads (k rows 8 kg + 0 .. 3 and
+  // + 4 .. 7); e4m3, the whole block, four reads (k rows 16 kg + 0, 8, 64, 72 and the seven after each).
   TCCL_D Vec turned(int j, int h) const {
-    const int t = i16 >> 2, cq = i16 & 3;
     const char* at = lds + wave * kWaveBytes + kMB * 2048;
-    s16x4 half[2];
+    if constexpr (kEsz == 2) {
+      const int t = i16 >> 2, cq = i16 & 3;
+      s16x4 half[2];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int k = 32 * h + 8 * kg + 4 * q + t;
-      const char* p = at + row_at(k) * (32 * kNB) + (((2 * j + (cq >> 1)) ^ (2 * swizzle(k))) << 4) + (cq & 1) * 8;
-      half[q] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)p);
+      for (int q = 0; q < 2; ++q) {
+        const int k = 32 * h + 8 * kg + 4 * q + t;
+        const char* p = at + row_at(k) * kRowBytes + (((2 * j + (cq >> 1)) ^ (2 * swizzle(k))) << 4) + (cq & 1) * 8;
+        half[q] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)p);
+      }
+      const s16x8 both = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+      return __builtin_bit_cast(Vec, both);
+    } else {
+      i32x8 v;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = 16 * kg + 8 * (q & 1) + 64 * (q >> 1) + (i16 >> 1);
+        const char* p = at + k * kRowBytes + ((j ^ swizzle(k)) << 4) + (i16 & 1) * 8;
+        const i32x2 x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsPair*)p);
+        v[2 * q] = x[0];
+        v[2 * q + 1] = x[1];
+      }
+      return __builtin_bit_cast(Vec, v);
     }
-    const s16x8 both = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(Vec, both);
+  }
+  TCCL_D Vec staged(int block, int h) const {
+    if constexpr (kEsz == 2) {
+      return __builtin_bit_cast(Vec, chunk(block, h));
+    } else {
+      typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+      const u32x8 both = __builtin_shufflevector(chunk(block, 0), chunk(block, 1), 0, 1, 2, 3, 4, 5, 6, 7);
+      return __builtin_bit_cast(Vec, both);
+    }
   }
 
   TCCL_D void multiply(f32x4 (&acc)[kMB][kNB]) const {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kEsz; ++h) {  // one MFMA deep for e4m3, two for the 16-bit types
       Vec fa[kMB], fb[kNB];
 #pragma unroll
       for (int j = 0; j < kNB; ++j) {
@@ -187,7 +216,7 @@ struct StreamGemm {
   }
 
   TCCL_D void k_loop(f32x4 (&acc)[kMB][kNB]) const {
-    const int blocks = (a.K + 63) / 64, whole = a.K / 64;
+    const int blocks = (a.K + kKB - 1) / kKB, whole = a.K / kKB;
     Block v[kDepth];
     // This wavefront's blocks are wave, wave + kWaves, ...; the last one of all may be a partial one.
     int next = wave;
@@ -225,21 +254,21 @@ struct StreamGemm {
     kg = lane >> 4;
     const int a_row = a.wrapped ? row_in : row0, a_rows = a.wrapped ? a.seg_rows : a.M;
     const int64_t b_col = (a.wrapped ? (int64_t)seg * a.N : 0) + col0;
-    pitch_a = (uint32_t)(a.lda * 2);
-    pitch_b = (uint32_t)(a.ldb * 2);
+    pitch_a = (uint32_t)(a.lda * kEsz);
+    pitch_b = (uint32_t)(a.ldb * kEsz);
     const InT* A = (const InT*)a.A + (int64_t)a_row * a.lda;
-    ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(((int64_t)(a_rows - 1 - a_row) * a.lda + a.K) * 2), 0x00020000);
+    ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(((int64_t)(a_rows - 1 - a_row) * a.lda + a.K) * kEsz), 0x00020000);
     off_a = (uint32_t)(lane >> 3) * pitch_a + (uint32_t)(lane & 7) * 16u;
     const int cols_left = a.N - col0;  // columns of this segment from col0 on
     if constexpr (kBKMajor) {
       const InT* B = (const InT*)a.B + b_col * a.ldb;
-      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(cols_left - 1) * a.ldb + a.K) * 2), 0x00020000);
+      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(cols_left - 1) * a.ldb + a.K) * kEsz), 0x00020000);
       off_b = (uint32_t)(lane >> 3) * pitch_b + (uint32_t)(lane & 7) * 16u;
     } else {
       const InT* B = (const InT*)a.B + b_col;
-      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(a.K - 1 - a.b_short) * a.ldb + cols_left) * 2), 0x00020000);
-      const int c = lane % (2 * kNB);
-      off_b = 8 * c < cols_left ? (uint32_t)(lane / (2 * kNB)) * pitch_b + (uint32_t)c * 16u : kOutside;
+      rb = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(a.K - 1 - a.b_short) * a.ldb + cols_left) * kEsz), 0x00020000);
+      const int c = lane % kRowLanes;
+      off_b = kVec * c < cols_left ? (uint32_t)(lane / kRowLanes) * pitch_b + (uint32_t)c * 16u : kOutside;
     }
 
     f32x4 acc[kMB][kNB];

@@ -61,6 +61,8 @@ int launch_shape(int shape, StreamArgs& a, const CommArgs* comm, int comm_wgs, h
 }  // namespace
 
 int launch_stream(int in_dtype, bool b_kmajor, int shape, StreamArgs& a, const CommArgs* comm, int comm_wgs, hipStream_t stream) {
+  if (in_dtype == kF8E4M3)
+    return b_kmajor ? launch_shape<fp8e4m3, true>(shape, a, comm, comm_wgs, stream) : launch_shape<fp8e4m3, false>(shape, a, comm, comm_wgs, stream);
   if (in_dtype == kF16)
     return b_kmajor ? launch_shape<_Float16, true>(shape, a, comm, comm_wgs, stream) : launch_shape<_Float16, false>(shape, a, comm, comm_wgs, stream);
   return b_kmajor ? launch_shape<__bf16, true>(shape, a, comm, comm_wgs, stream) : launch_shape<__bf16, false>(shape, a, comm, comm_wgs, stream);
