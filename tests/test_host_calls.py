@@ -1,0 +1,132 @@
+"""Bound calls (``_launch.bind`` / ``_host.Table``): which tensors find a call, and what the entry point is given."""
+
+import ctypes as C
+
+import pytest
+import torch
+
+from tileccl_amd import _launch, _lib
+
+ENTRY = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p)
+
+
+@pytest.fixture
+def table(lib):
+    host = _lib.host()
+    capturing = []
+    host.setup(lambda device: 0x5000 + device, lambda: bool(capturing), _lib.check)
+    yield host.Table(), capturing
+    _lib._host = None
+    _lib.host()  # torch's stream again
+
+
+class Heap:
+    def __init__(self, t, size):
+        self.local_base, self.size = t.data_ptr(), size
+
+
+def bound(table, key, tensors, returns=0, **how):
+    seen = []
+
+    @ENTRY
+    def entry(a, b, c, stream):
+        seen.append((a, b, c, stream))
+        return returns
+
+    _launch.bind(table, key, tensors, entry, ((0, 64), -3, (1, 0)), "entry", **how)
+    return seen, entry
+
+
+@pytest.mark.parametrize("change", ["none", "moved", "shape", "strides", "dtype", "alignment", "outside", "key", "count"])
+def test_which_tensors_find_a_call(table, change):
+    table, _ = table
+    buf = torch.zeros(4096, dtype=torch.float32)
+    a, b = buf[:64].view(8, 8), buf[64:128].view(8, 8)
+    seen, keep = bound(table, ("op", 1, a), (a, b), heap=Heap(buf, 1024), tag="tag")
+    key, found = ("op", 1, a), (a, b)
+    if change == "moved":
+        found = (b, a)
+    elif change == "shape":
+        found = (a, b[:7])
+    elif change == "strides":
+        found = (a.t(), b)
+    elif change == "dtype":
+        found = (a, b.view(torch.int32))
+    elif change == "alignment":
+        found = (a, buf[65:129].view(8, 8))
+    elif change == "outside":
+        found = (a, buf[256:320].view(8, 8))  # starts at byte 1024: just past the heap
+    elif change == "key":
+        key = ("op", 1, a.clone())  # anything but plain values counts by identity
+    elif change == "count":
+        found = (a,)
+    hit = change in ("none", "moved")
+    assert table.launch(key, None, *found) == ("tag" if hit else None)
+    assert seen == ([(found[0].data_ptr() + 64, -3, found[1].data_ptr(), 0x5000)] if hit else [])
+    assert table.launch(("op", 1, a), None, a, "no tensor") is None
+
+
+def test_one_offset_on_every_rank_and_reported_errors(table):
+    table, _ = table
+    buf = torch.zeros(256, dtype=torch.float32)
+    a, b, off = buf[:64], buf[128:192], buf[132:196]
+    seen, keep = bound(table, ("op",), (a, b), bases=[a.data_ptr(), b.data_ptr()])
+    assert table.launch(("op",), None, a, off) is None and table.launch(("op",), None, a, b) is True and len(seen) == 1
+    _, keep2 = bound(table, ("bad",), (a, b), returns=_lib.ERR_INVALID)
+    with pytest.raises(ValueError, match="entry"):
+        table.launch(("bad",), None, a, b)
+
+
+def test_the_table_is_bounded(table):
+    table, _ = table
+    a = torch.zeros(8)
+    keep = [bound(table, ("op", i), (a, a)) for i in range(70)]
+    assert len(table) == 64
+    assert table.launch(("op", 5), None, a, a) is None and table.launch(("op", 6), None, a, a) is True
+
+
+@pytest.mark.parametrize("variant,attr", [("s2", "epoch"), ("s1", "lock_epoch"), ("s0", None)])
+def test_descriptors_and_launch_numbers(table, variant, attr):
+    """The GEMM descriptor gets the operands' addresses and alpha, the sync descriptor the number ``next_epoch`` would give."""
+    table, capturing = table
+
+    class Words:
+        epoch = lock_epoch = 0
+        clear_every_launch = False
+        max_tasks_per_tile = 1 << 16
+        spin_limit_ns = 77
+        asked = 0
+
+        def desc(self, _variant):
+            return _lib.SyncDescArrivals(locks=0x1230)
+
+        def next_epoch(self, which):
+            assert which == variant
+            self.asked += 1
+            return 40
+
+    words, seen = Words(), []
+
+    @C.CFUNCTYPE(C.c_int, C.POINTER(_lib.GemmDesc), C.POINTER(_lib.SyncDescArrivals), C.c_void_p)
+    def entry(gemm, sync, stream):
+        seen.append((gemm[0].A, gemm[0].B, gemm[0].C, gemm[0].M, gemm[0].alpha, sync[0].locks, sync[0].epoch, sync[0].spin_limit_ns))
+        return 0
+
+    a, b, c = (torch.zeros(16) for _ in range(3))
+    gemm = _lib.GemmDesc(M=5, alpha=1.0)
+    _launch.bind(table, ("g",), (a, b, c), entry, (gemm, _launch.SYNC), "g", gemm=gemm, words=words, variant=variant, c=(2, 32))
+
+    def numbers():
+        assert table.launch(("g",), 0.5, a, b, c) is True
+        assert seen[-1][:6] == (a.data_ptr(), b.data_ptr(), c.data_ptr() + 32, 5, 0.5, 0x1230) and seen[-1][7] == 77
+        return seen[-1][6]
+
+    if attr is None:
+        assert numbers() == 0 and words.epoch == words.lock_epoch == words.asked == 0
+        return
+    assert [numbers(), numbers()] == [1, 2] and getattr(words, attr) == 2 and words.asked == 0
+    setattr(words, attr, (1 << 14))  # max_tasks_per_tile leaves room for 2**14 launches
+    assert numbers() == 40 and words.asked == 1
+    setattr(words, attr, 3)
+    capturing.append(1)
+    assert numbers() == 40 and words.asked == 2

@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes as C
 import sys
 from dataclasses import dataclass, field
+from functools import partial
 
 import torch
 
@@ -232,62 +233,57 @@ def gemm_desc(A: torch.Tensor, B: torch.Tensor, C_out: torch.Tensor, **how) -> _
     return d
 
 
-def layout_key(t: torch.Tensor) -> tuple:
-    """Everything about a tensor that a descriptor depends on, except where it lies."""
-    return t.shape, t.stride(), t.dtype, t.device, t.data_ptr() & 15
+SYNC = object()  # stands for the sync descriptor in the arguments of a bound call
 
 
-class BoundCall:
-    """One fused operation on tensors of one layout: the descriptors are built and checked once, a call fills in the
-    addresses, the launch number and the stream.  Not shared between threads while it runs (``CallCache``)."""
-
-    __slots__ = ("gemm", "plan", "words", "sync", "variant", "fn", "args", "what", "keep")
-
-    def __init__(self, gemm: _lib.GemmDesc, plan: OperandPlan, words: "SyncWords | None", variant: str, fn, args, what: str, keep=()) -> None:
-        self.gemm, self.words, self.variant, self.fn, self.what, self.keep = gemm, words, variant, fn, what, keep
-        self.plan = plan if plan.pack_a or plan.pack_b else None
-        self.sync = None if words is None else words.desc(variant)
-        self.args = tuple(byref(self.sync) if a is SYNC else a for a in args)
-
-    def __call__(self, A: torch.Tensor, B: torch.Tensor) -> None:
-        gemm = self.gemm
-        if self.plan is not None:
-            A, B = planned_operands(self.plan, A, B)
-        gemm.A, gemm.B = A.data_ptr(), B.data_ptr()
-        words = self.words
-        if words is not None:
-            if self.variant != "s0":  # S1 launches number the locks they write, S2 launches the counters
-                self.sync.epoch = words.next_epoch(self.variant)
-            self.sync.spin_limit_ns = words.spin_limit_ns
-        rc = self.fn(*self.args, stream_ptr())
-        if rc:
-            _lib.check(rc, self.what)
+def call_table(owner: dict):
+    """The bound calls kept with ``owner`` (a heap's or an operation's ``__dict__``, a context's workspaces): at most 64."""
+    table = owner.get("tileccl_amd.calls")
+    if table is None:
+        table = owner["tileccl_amd.calls"] = _lib.host().Table()
+    return table
 
 
-SYNC = object()  # stands for the sync descriptor in a BoundCall's arguments
+def bind(table, key: tuple, tensors: tuple, fn, args: tuple, what: str, *, gemm: _lib.GemmDesc | None = None,
+         plan: "OperandPlan | None" = None, words: "SyncWords | None" = None, variant: str = "s0", tag=None, c=None, heap=None,
+         on_heap: int | None = None, bases=None) -> None:
+    """Keep a checked call for tensors laid out like ``tensors``: ``table.launch(key, alpha, *tensors)`` issues ``fn(*args, stream)``
+    and returns ``tag`` (``True`` by default); it returns ``None`` where no call of the table fits.
+
+    In ``args``, ``gemm`` stands for a copy of that descriptor with the addresses of the first two tensors as A and B (packed
+    first where ``plan`` says so) and, with ``c=(i, offset)``, tensor ``i``'s as C; ``SYNC`` for ``words``' descriptor with
+    the launch's number; ``(i, offset)`` for the address of tensor ``i``; other descriptors are passed as they are.
+    The tensors of the bit mask ``on_heap`` (default: all) must start inside ``heap``; with ``bases`` all tensors must lie at
+    one distance from their base.  Tensors for which that does not hold find no call."""
+    host = _lib.host()
+    keep = [words]  # what the descriptors point at lives as long as the call
+
+    def value(a):
+        if a is gemm and a is not None:
+            return host.GEMM
+        if a is SYNC:
+            return None if words is None else host.SYNC
+        if isinstance(a, C.Structure):
+            keep.append(a)
+            return C.addressof(a)
+        return a
+
+    sync = None if words is None else words.desc(variant)
+    packs = plan is not None and (plan.pack_a or plan.pack_b)
+    table.add(host.Call(
+        C.cast(fn, C.c_void_p).value, what, tuple(value(a) for a in args), tensors, key, tag=tag,
+        gemm=C.addressof(gemm) if gemm is not None else 0, c=c, sync=C.addressof(sync) if sync is not None else 0, words=words,
+        variant=variant, on_heap=on_heap, heap=(heap.local_base, heap.size) if heap is not None else None, bases=bases,
+        prepare=partial(planned_operands, plan) if packs else None, keep=keep,
+    ))
 
 
-class CallCache:
-    """Bounded cache of things one thread at a time may use: ``take`` removes what it returns, ``put`` gives it back (a
-    second thread that comes in between builds its own)."""
-
-    __slots__ = ("entries", "limit")
-
-    def __init__(self, limit: int = 64) -> None:
-        self.entries: dict = {}
-        self.limit = limit
-
-    def take(self, key):
-        return self.entries.pop(key, None)
-
-    def put(self, key, value) -> None:
-        entries = self.entries
-        while len(entries) >= self.limit:
-            try:
-                del entries[next(iter(entries))]
-            except (KeyError, StopIteration, RuntimeError):  # another thread was quicker
-                break
-        entries[key] = value
+def issue(table, key: tuple, alpha, *tensors):
+    """Launch a call that has just been bound."""
+    tag = table.launch(key, alpha, *tensors)
+    if tag is None:
+        raise RuntimeError(f"the call bound as {key} does not fit the tensors it was made for")
+    return tag
 
 
 def view_of(heap) -> _lib.HeapView:

@@ -252,3 +252,28 @@ def check(code: int, what: str) -> None:
     if code > 0:
         raise RuntimeError(f"HIP error in {what}: error code {code} ({detail})")
     raise RuntimeError(f"{what}: {detail} (code {code})")
+
+
+_host = None
+
+
+def host():
+    """The CPython extension that issues repeated calls (``csrc/tccl_host.cpp``), set up on first use."""
+    global _host
+    if _host is None:
+        import torch
+
+        load()
+        try:
+            from tileccl_amd import _host as module
+        except ImportError as e:
+            raise RuntimeError(
+                f"tileccl_amd._host cannot be imported ({e}). Run `python -m tileccl_amd.csrc.build` (or "
+                "__graft_entry__.build()) first; there is no fallback."
+            ) from e
+        from tileccl_amd import _launch
+
+        capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)
+        module.setup(_launch._raw_stream or (lambda _device: _launch.stream_ptr()), capturing, check)
+        _host = module
+    return _host

@@ -15,6 +15,7 @@ from dataclasses import dataclass, field
 from typing import Any, Literal
 
 import tileccl_amd
+from tileccl_amd import _launch
 from tileccl_amd.patterns import (
     BulkSyncPattern,
     FusedSequentialPattern,
@@ -24,6 +25,7 @@ from tileccl_amd.patterns import (
     WGSpecializedPattern,
 )
 from tileccl_amd.patterns.contracts import PatternExecutionSpec, resolve_pattern_execution
+from tileccl_amd.patterns.hip_patterns import _HipAllScatterPattern
 
 __all__ = [
     "gemm_allgather",
@@ -410,6 +412,25 @@ def _plan_for_call(A: Any, B: Any, C: Any, *, ctx, pattern: PatternLike, hw_info
     return plan
 
 
+def _scatter(A: Any, B: Any, C: Any, ctx, pattern: PatternLike, hw_info, **how) -> Any:
+    """A call that brings no plan.  The launch that it comes to is kept with the context's workspaces as well, and the next call
+    on tensors of these layouts goes straight to it."""
+    ctx = ctx if ctx is not None else tileccl_amd.current_context()
+    named = hw_info is None and (pattern is None or isinstance(pattern, str)) and ctx.heap is not None
+    if named:
+        calls = _launch.call_table(ctx._workspace_cache)
+        key = ("allscatter", ctx.heap.local_base, pattern, *how.values())
+        if calls.launch(key, None, A, B, C) is not None:
+            return C
+    plan = _plan_for_call(A, B, C, ctx=ctx, pattern=pattern, hw_info=hw_info, **how)
+    impl = getattr(plan, "pattern_impl", None)
+    if named and isinstance(impl, _HipAllScatterPattern) and (ctx.world_size == 1 or ctx.heap.owns_tensor(C)):
+        impl._bind(calls, key, (A, B, C), (2, 0), plan.execution, ctx.heap)
+        _launch.issue(calls, key, None, A, B, C)
+        return C
+    return plan.execute(A, B, C, validate=False)
+
+
 def gemm_allscatter(
     A: Any,
     B: Any,
@@ -424,19 +445,7 @@ def gemm_allscatter(
     storage_kind: str = "symmetric",
 ) -> Any:
     """``C = A @ B`` on this rank, then this rank's column block lands in every peer's ``C``."""
-    plan = _plan_for_call(
-        A,
-        B,
-        C,
-        ctx=ctx,
-        full_N=full_N,
-        b_layout=b_layout,
-        c_layout=c_layout,
-        pattern=pattern,
-        hw_info=hw_info,
-        storage_kind=storage_kind,
-    )
-    return plan.execute(A, B, C, validate=False)
+    return _scatter(A, B, C, ctx, pattern, hw_info, full_N=full_N, b_layout=b_layout, c_layout=c_layout, storage_kind=storage_kind)
 
 
 def gemm_allscatter_sharded(
@@ -451,16 +460,4 @@ def gemm_allscatter_sharded(
     storage_kind: str = "symmetric",
 ) -> Any:
     """shard/shard contract: ``B_shard (K, N/ws)``, ``C_shard (M, N/ws)``; ``full_N`` is mandatory."""
-    plan = _plan_for_call(
-        A,
-        B_shard,
-        C_shard,
-        ctx=ctx,
-        full_N=full_N,
-        b_layout="shard",
-        c_layout="shard",
-        pattern=pattern,
-        hw_info=hw_info,
-        storage_kind=storage_kind,
-    )
-    return plan.execute(A, B_shard, C_shard, validate=False)
+    return _scatter(A, B_shard, C_shard, ctx, pattern, hw_info, full_N=full_N, b_layout="shard", c_layout="shard", storage_kind=storage_kind)

@@ -16,7 +16,6 @@ contracts ``:1406-1549``).  Here the same contracts run on this package's kernel
 
 from __future__ import annotations
 
-import ctypes as C
 from dataclasses import dataclass
 from typing import Any
 
@@ -162,30 +161,19 @@ def gemm_allgather(A: Any, B_shard: Any, Cx: Any, *, ctx=None, storage_kind: str
     return run_gather(ctx, A, B_shard, Cx, storage_kind, variant)
 
 
-def _calls_of(ctx, what: str) -> _launch.CallCache:
-    """Bound calls of an operation, kept with the context's workspaces."""
-    return ctx._workspace_cache.setdefault(f"tileccl_amd.{what}_calls", _launch.CallCache())
-
-
 def run_gather(ctx, A: Any, B_shard: Any, Cx: Any, storage_kind: str, variant: str, expected: "GemmAllGatherContract | None" = None) -> Any:
     """``gemm_allgather``; ``expected``: a plan's contract, which the tensors' must equal (``ValueError`` otherwise)."""
     heap = ctx.require_heap()
-    calls = _calls_of(ctx, "gather")
-    key = (_launch.layout_key(A), _launch.layout_key(B_shard), _launch.layout_key(Cx), variant, storage_kind)
-    entry = calls.take(key)
-    if entry is None or entry[1] is not heap or not heap.owns_tensor(Cx):
+    calls = _launch.call_table(ctx._workspace_cache)
+    key = ("gather", heap.local_base, variant, storage_kind, expected)
+    ran = calls.launch(key, None, A, B_shard, Cx)
+    if ran is None:
         k = resolve_gemm_allgather_contract(A, B_shard, Cx, ctx=ctx, storage_kind=storage_kind)
         if expected is not None and k != expected:
             raise ContractChanged  # before anything is allocated for the call: the ranks' heaps stay in step
-        entry = (k, heap, *_gather_bind(ctx, k, A, B_shard, Cx, variant, launch=False))
-    k, _, pattern, call, offset = entry
-    if expected is not None and k is not expected and k != expected:
-        calls.put(key, entry)
-        raise ContractChanged
-    call.gemm.C = Cx.data_ptr() + offset
-    call(A, B_shard)
-    calls.put(key, entry)
-    pattern._last_sync = call.words
+        _gather_bind(ctx, k, A, B_shard, Cx, variant, calls, key)
+        ran = _launch.issue(calls, key, None, A, B_shard, Cx)
+    pattern, pattern._last_sync = ran
     return Cx
 
 
@@ -193,9 +181,8 @@ class ContractChanged(ValueError):
     """The tensors of a plan's call are not those that the plan was made for."""
 
 
-def _gather_bind(ctx, k: GemmAllGatherContract, A: Any, B_shard: Any, Cx: Any, variant: str | Pattern, launch: bool = True):
-    """The all-scatter launch on this rank's column block of ``C``: run through the pattern, or its bound call with the
-    block's byte offset."""
+def _gather_bind(ctx, k: GemmAllGatherContract, A: Any, B_shard: Any, Cx: Any, variant: str | Pattern, calls=None, key=None) -> None:
+    """The all-scatter launch on this rank's column block of ``C``: run through the pattern, or kept as a call in ``calls``."""
     lo = k.rank * k.shard_cols if k.world_size > 1 else 0
     block = Cx[:, lo:lo + k.shard_cols]  # the GEMM's output: this rank's columns of the full C
     shape = (k.M, k.full_N)
@@ -207,10 +194,11 @@ def _gather_bind(ctx, k: GemmAllGatherContract, A: Any, B_shard: Any, Cx: Any, v
         scatter_src_col_offset=0, scatter_cols=k.shard_cols, scatter_dst_leading_dim=k.full_N, scatter_dst_col_offset=0,
     )
     pattern = _pattern_for(ctx, variant)
-    if launch:
+    if calls is None:
         pattern.execute(A, B_shard, block, spec=spec)
-        return None
-    return pattern, pattern._bind(A, B_shard, block, spec, ctx.require_heap()), int(block.data_ptr() - Cx.data_ptr())
+        return
+    words = pattern._sync_words(k.M, k.shard_cols, block)
+    pattern._bind(calls, key, (A, B_shard, Cx), (2, int(block.data_ptr() - Cx.data_ptr())), spec, ctx.require_heap(), block, (pattern, words))
 
 
 def _reduce_scatter_words(ctx, world: int, M: int, cols: int):
@@ -278,36 +266,28 @@ def run_reduce(ctx, A: Any, B: Any, Cx: Any, storage_kind: str, variant: str, em
                expected: "GemmReduceScatterContract | None" = None) -> Any:
     """``gemm_reducescatter``; ``expected``: a plan's contract, which the tensors' must equal (``ValueError`` otherwise)."""
     heap = ctx.require_heap()
-    calls = _calls_of(ctx, "reduce")
-    key = (_launch.layout_key(A), _launch.layout_key(B), _launch.layout_key(Cx), variant, storage_kind, emulate_peer,
-           own_rows_in_registers, peers_resident)
-    entry = calls.take(key)
-    if entry is None or entry[1] is not heap or not heap.owns_tensor(Cx):
+    calls = _launch.call_table(ctx._workspace_cache)
+    key = ("reduce", heap.local_base, variant, storage_kind, emulate_peer, own_rows_in_registers, peers_resident, expected)
+    ran = calls.launch(key, None, A, B, Cx)
+    if ran is None:
         k = resolve_gemm_reducescatter_contract(A, B, Cx, ctx=ctx, storage_kind=storage_kind)
         if expected is not None and k != expected:
             raise ContractChanged  # before anything is allocated for the call: the ranks' heaps stay in step
-        entry = (k, heap, _reduce_bind(ctx, k, A, B, Cx, variant, emulate_peer, own_rows_in_registers, peers_resident))
-    k, _, call = entry
-    if expected is not None and k is not expected and k != expected:
-        calls.put(key, entry)
-        raise ContractChanged
-    if k.world_size == 1:
-        call.gemm.C = Cx.data_ptr()
-    else:
-        call.args[1].value = Cx.data_ptr()
-    call(A, B)
-    calls.put(key, entry)
-    if call.words is not None:
-        ctx.__dict__["_reduce_scatter_last_words"] = call.words
+        _reduce_bind(calls, key, ctx, k, A, B, Cx, variant, emulate_peer, own_rows_in_registers, peers_resident)
+        ran = _launch.issue(calls, key, None, A, B, Cx)
+    if ran is not True:
+        ctx.__dict__["_reduce_scatter_last_words"] = ran
     return Cx
 
 
-def _reduce_bind(ctx, k: GemmReduceScatterContract, A: Any, B: Any, Cx: Any, variant: str, emulate_peer: bool,
-                 own_rows_in_registers: bool, peers_resident: bool) -> _launch.BoundCall:
+def _reduce_bind(calls, key: tuple, ctx, k: GemmReduceScatterContract, A: Any, B: Any, Cx: Any, variant: str, emulate_peer: bool,
+                 own_rows_in_registers: bool, peers_resident: bool) -> None:
     lib = _lib.load()
     if k.world_size == 1:
         gemm, plan = _launch._gemm_desc(A, B, Cx)
-        return _launch.BoundCall(gemm, plan, None, "s0", lib.tccl_gemm, (C.byref(gemm),), "tccl_gemm")
+        _launch.bind(calls, key, (A, B, Cx), lib.tccl_gemm, (gemm,), "tccl_gemm", gemm=gemm, plan=plan, c=(2, 0), heap=ctx.require_heap(),
+                     on_heap=0b100)
+        return
     partial = ctx.workspace("gemm_reducescatter.partial", k.world_size, k.M, k.output_cols, dtype=torch.float32)
     tall = partial.view(k.world_size * k.M, k.output_cols)  # row block q = the shard rank q owns
     transport = _launch.transport_desc(_lib.DIR_PULL, 16384, 16384, 0)
@@ -320,9 +300,10 @@ def _reduce_bind(ctx, k: GemmReduceScatterContract, A: Any, B: Any, Cx: Any, var
     else:  # no whole plan tiles: one launch (or a GEMM per column block and a reduction) without signals
         mode |= _lib.RS_PEERS_RESIDENT
     gemm, plan = _launch._gemm_desc(A, B, tall, column_shards=k.world_size, flags=flags)
-    return _launch.BoundCall(
-        gemm, plan, words, variant, lib.tccl_gemm_reducescatter,
-        (C.byref(gemm), C.c_void_p(Cx.data_ptr()), _launch.dtype_code(Cx.dtype), int(Cx.stride(0)), C.byref(_launch.view_of(ctx.require_heap())),
-         _launch.SYNC if words is not None else None, C.byref(transport), mode, _launch.VARIANTS[variant]),
-        f"tccl_gemm_reducescatter[{variant}]",
+    _launch.bind(
+        calls, key, (A, B, Cx), lib.tccl_gemm_reducescatter,
+        (gemm, (2, 0), _launch.dtype_code(Cx.dtype), int(Cx.stride(0)), _launch.view_of(ctx.require_heap()), _launch.SYNC, transport, mode,
+         _launch.VARIANTS[variant]),
+        f"tccl_gemm_reducescatter[{variant}]", gemm=gemm, plan=plan, words=words, variant=variant, tag=words, heap=ctx.require_heap(),
+        on_heap=0b100,
     )

@@ -22,7 +22,6 @@ meant by its docstring, ``concat_k(shards) @ W``, is what is computed here.
 
 from __future__ import annotations
 
-import ctypes as C
 from typing import Any
 
 import torch
@@ -63,7 +62,7 @@ class ChainedAGGemmRSPattern:
         # The GEMM + scatter stages reuse the all-scatter pattern's plan and signal words.
         self._stage = _SCHEDULES[schedule](ctx, BLOCK_M=BLOCK_M, BLOCK_N=BLOCK_N, BLOCK_K=BLOCK_K)
         self._last_sync: _launch.SyncWords | None = None
-        self._calls = _launch.CallCache()
+        self._calls = _launch.call_table({})
 
     def execute(
         self,
@@ -77,25 +76,22 @@ class ChainedAGGemmRSPattern:
             gathered_workspace = self.ctx.workspace(
                 "chained_ag_gemm_rs.gathered_input", input_shard.shape[0], W.shape[0], dtype=input_shard.dtype
             )
-        key = tuple(_launch.layout_key(t) for t in (input_shard, W, output, gathered_workspace))
-        call = self._calls.take(key)
-        if call is None or call.keep is not heap:
-            call = self._bind(input_shard, W, output, gathered_workspace, heap)
-        if self.ctx.world_size > 1:
-            for name, t in (("input_shard", input_shard), ("output", output)):
-                if not heap.owns_tensor(t):
-                    raise ValueError(
-                        f"{name} must live in the symmetric heap when world_size > 1: peers address it "
-                        "at the same offset in their slices"
-                    )
-        call.gemm.C = output.data_ptr()
-        call.args[1].value = input_shard.data_ptr()
-        call(gathered_workspace, W)
-        self._calls.put(key, call)
-        self._last_sync = call.words
+        key = (heap.local_base,)
+        ran = self._calls.launch(key, None, gathered_workspace, W, output, input_shard)
+        if ran is None:
+            if self.ctx.world_size > 1:
+                for name, t in (("input_shard", input_shard), ("output", output)):
+                    if not heap.owns_tensor(t):
+                        raise ValueError(
+                            f"{name} must live in the symmetric heap when world_size > 1: peers address it "
+                            "at the same offset in their slices"
+                        )
+            self._bind(key, input_shard, W, output, gathered_workspace, heap)
+            ran = _launch.issue(self._calls, key, None, gathered_workspace, W, output, input_shard)
+        self._last_sync = None if ran is True else ran
         return output
 
-    def _bind(self, input_shard, W, output, gathered_workspace, heap) -> _launch.BoundCall:
+    def _bind(self, key, input_shard, W, output, gathered_workspace, heap) -> None:
         """Check the shapes and build the descriptors of a call on tensors of these layouts."""
         M, K_shard = input_shard.shape
         K, N = W.shape
@@ -116,11 +112,12 @@ class ChainedAGGemmRSPattern:
         transport = _launch.transport_desc(_lib.DIR_PUSH, self._stage._copy_elems(), None, comm_wgs)
         words = self._stage._sync_words(M, N, output)
         variant = {_lib.S0_BULK: "s0", _lib.S1_TILE: "s1", _lib.S2_TILEGROUP: "s2"}[self._stage.variant]
-        return _launch.BoundCall(
-            gemm, plan, words, variant, _lib.load().tccl_chained_ag_gemm_rs,
-            (C.byref(gemm), C.c_void_p(), _launch._row_major(input_shard, "input_shard"), K_shard, C.byref(_launch.view_of(heap)),
-             _launch.SYNC if words is not None else None, C.byref(transport), self._stage.variant),
-            f"tccl_chained_ag_gemm_rs[{self.schedule}]", heap,
+        _launch.bind(
+            self._calls, key, (gathered_workspace, W, output, input_shard), _lib.load().tccl_chained_ag_gemm_rs,
+            (gemm, (3, 0), _launch._row_major(input_shard, "input_shard"), K_shard, _launch.view_of(heap), _launch.SYNC, transport,
+             self._stage.variant),
+            f"tccl_chained_ag_gemm_rs[{self.schedule}]", gemm=gemm, plan=plan, words=words, variant=variant, tag=words, c=(2, 0),
+            heap=heap, on_heap=0b1100 if world_size > 1 else 0,
         )
 
     def check_faults(self) -> None:

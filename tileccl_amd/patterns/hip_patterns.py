@@ -7,7 +7,6 @@ has no in-tree reference kernel; it follows the planning contract of ``tileccl_v
 
 from __future__ import annotations
 
-import ctypes as C
 from typing import Any
 
 import torch
@@ -47,7 +46,7 @@ class _HipAllScatterPattern(Pattern):
         # workspaces, and shared by every pattern instance of the same kind and tiling.
         cache = getattr(ctx, "_workspace_cache", None)
         self._sync: dict[tuple, _launch.SyncWords] = cache if isinstance(cache, dict) else {}
-        self._calls = _launch.CallCache()
+        self._calls = _launch.call_table({})
 
     # -- hooks -------------------------------------------------------------------------
     def _sync_words(self, M: int, N: int, C_out: torch.Tensor) -> _launch.SyncWords | None:
@@ -75,22 +74,25 @@ class _HipAllScatterPattern(Pattern):
                 "C must live in the symmetric heap when world_size > 1: the scatter writes it at the "
                 "same offset in every peer's slice"
             )
-        key = (_launch.layout_key(A), _launch.layout_key(B), _launch.layout_key(C_out), spec.scatter_src_col_offset, spec.scatter_cols,
-               spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
-        call = self._calls.take(key)
-        if call is None or call.keep is not heap:
-            call = self._bind(A, B, C_out, spec, heap)
-        call.gemm.C = C_out.data_ptr()
-        call(A, B)
-        self._calls.put(key, call)
-        self._last_sync = call.words
-        if call.words is not None and call.words.host_plan is not None:
-            self.last_plan = call.words.host_plan
+        key = (heap.local_base, spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
+        ran = self._calls.launch(key, None, A, B, C_out)
+        if ran is None:
+            self._bind(self._calls, key, (A, B, C_out), (2, 0), spec, heap)
+            ran = _launch.issue(self._calls, key, None, A, B, C_out)
+        self._ran(ran)
 
-    def _bind(self, A, B, C_out, spec, heap) -> _launch.BoundCall:
+    def _ran(self, words: "_launch.SyncWords | bool") -> None:
+        """A bound call of this pattern has been issued (its tag: the words it signals through, if any)."""
+        self._last_sync = None if words is True else words
+        if words is not True and words.host_plan is not None:
+            self.last_plan = words.host_plan
+
+    def _bind(self, table, key: tuple, tensors: tuple, c: tuple, spec, heap, C_out: "torch.Tensor | None" = None, tag=None) -> None:
+        """Keep the call on ``tensors`` (A, B and the one that holds C, at byte ``c[1]``; ``C_out``: C itself, by default all of it)."""
         compute_wgs, comm_wgs = self._wg_split()
+        C_out = C_out if C_out is not None else tensors[2]
         gemm, plan = _launch._gemm_desc(
-            A, B, C_out, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self.GROUP_M, num_wgs=compute_wgs,
+            tensors[0], tensors[1], C_out, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self.GROUP_M, num_wgs=compute_wgs,
             flags=_lib.GEMM_ARRIVALS,
         )
         scatter = _lib.ScatterDesc(
@@ -99,10 +101,11 @@ class _HipAllScatterPattern(Pattern):
         transport = _launch.transport_desc(_lib.DIR_PUSH, self._copy_elems(), None, comm_wgs)
         words = self._sync_words(spec.M, spec.local_N, C_out)
         variant = {_lib.S0_BULK: "s0", _lib.S1_TILE: "s1", _lib.S2_TILEGROUP: "s2"}[self.variant]
-        return _launch.BoundCall(
-            gemm, plan, words, variant, _lib.load().tccl_gemm_allscatter,
-            (C.byref(gemm), C.byref(scatter), C.byref(_launch.view_of(heap)), _launch.SYNC if words is not None else None,
-             C.byref(transport), self.variant), f"tccl_gemm_allscatter[{self.name}]", heap,
+        _launch.bind(
+            table, key, tensors, _lib.load().tccl_gemm_allscatter,
+            (gemm, scatter, _launch.view_of(heap), _launch.SYNC, transport, self.variant), f"tccl_gemm_allscatter[{self.name}]",
+            gemm=gemm, plan=plan, words=words, variant=variant, tag=words if tag is None else tag, c=c, heap=heap,
+            on_heap=0b100 if spec.world_size > 1 else 0,
         )
 
     def _copy_elems(self) -> int:

@@ -87,19 +87,8 @@ def _whole_units(collective: str, block: int, element_size: int, *, reduce: bool
         raise ValueError(f"{collective}: a rank's block of {block} elements is not a multiple of {need}")
 
 
-_KNOWN_LIMIT = 64
-
-
-# Each collective has a quick way for tensors like those of an earlier call: ``heap.__dict__["_known_calls"]`` holds what that call,
-# checked in full, was found to need, by the tensors' shapes, strides, types and devices.  Where a tensor lies is
-# looked at on every call.  ``run_known_*`` launches and returns True, or returns False: the caller then goes the whole way.
-
-
-def _remember(heap, key, what) -> None:
-    calls = heap.__dict__.setdefault("_known_calls", {})
-    if len(calls) >= _KNOWN_LIMIT:
-        calls.clear()
-    calls[key] = what
+# Each collective has a quick way for tensors like those of an earlier call, which was checked in full and is kept with the heap
+# (``_launch.bind``).  ``run_known_*`` issues it and returns True, or returns False: the caller then goes the whole way.
 
 
 def allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> None:
@@ -108,27 +97,21 @@ def allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> None:
     Direct write (reference :628-630): the caller's block goes into block ``rank`` of every
     rank's ``output``, its own included, in one launch.
     """
-    if not run_known_allgather(tensor, output, heap):
-        _remember(heap, _pair_key("allgather", tensor, output), _check_allgather(tensor, output, heap))
-        run_known_allgather(tensor, output, heap)
-
-
-def _pair_key(op: str, tensor: torch.Tensor, output: torch.Tensor) -> tuple:
-    return op, tensor.shape, tensor.stride(), tensor.dtype, tensor.device, output.shape, output.stride(), output.dtype, output.device
+    if run_known_allgather(tensor, output, heap):
+        return
+    nbytes = _check_allgather(tensor, output, heap)
+    if nbytes:
+        table, key = _launch.call_table(heap.__dict__), ("allgather", heap.local_base)
+        _launch.bind(
+            table, key, (tensor, output), _lib.load().tccl_copy_block,
+            ((1, heap.rank * nbytes), (1 << heap.world_size) - 1, (0, 0), heap.rank, 1, nbytes, nbytes, nbytes, _launch.view_of(heap)),
+            "tccl_copy_block", heap=heap,
+        )
+        _launch.issue(table, key, None, tensor, output)
 
 
 def run_known_allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> bool:
-    calls = heap.__dict__.get("_known_calls")
-    nbytes = calls.get(_pair_key("allgather", tensor, output)) if calls is not None else None
-    if nbytes is None or not (heap.owns_tensor(tensor) and heap.owns_tensor(output)):
-        return False
-    if nbytes:
-        rc = _lib.load().tccl_copy_block(
-            output.data_ptr() + heap.rank * nbytes, (1 << heap.world_size) - 1, tensor.data_ptr(), heap.rank, 1, nbytes, nbytes, nbytes,
-            _launch.byref(_launch.view_of(heap)), _launch.stream_ptr(),
-        )
-        _lib.check(rc, "tccl_copy_block")
-    return True
+    return _launch.call_table(heap.__dict__).launch(("allgather", heap.local_base), None, tensor, output) is not None
 
 
 def _check_allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> int:
@@ -193,24 +176,21 @@ def reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap, op: str = "
         raise ValueError(f"Only op='sum' is currently supported, got {op!r}")
     if implementation not in {"auto", "reference", "device"}:
         raise ValueError(f"implementation must be one of {{'auto', 'reference', 'device'}}, got {implementation!r}")
-    if not run_known_reduce_scatter(tensor, output, heap):
-        _remember(heap, _pair_key("reduce_scatter", tensor, output), _check_reduce_scatter(tensor, output, heap))
-        run_known_reduce_scatter(tensor, output, heap)
+    if run_known_reduce_scatter(tensor, output, heap):
+        return
+    block, in_code, out_code = _check_reduce_scatter(tensor, output, heap)
+    if block:
+        table, key = _launch.call_table(heap.__dict__), ("reduce_scatter", heap.local_base)
+        _launch.bind(
+            table, key, (tensor, output), _lib.load().tccl_reduce_rows,
+            ((0, 0), in_code, block, (1, 0), out_code, block, heap.world_size, block, _launch.view_of(heap), None, 0),
+            "tccl_reduce_rows[reduce_scatter]", heap=heap,
+        )
+        _launch.issue(table, key, None, tensor, output)
 
 
 def run_known_reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap) -> bool:
-    calls = heap.__dict__.get("_known_calls")
-    known = calls.get(_pair_key("reduce_scatter", tensor, output)) if calls is not None else None
-    if known is None or not (heap.owns_tensor(tensor) and heap.owns_tensor(output)):
-        return False
-    block, in_code, out_code = known
-    if block:
-        rc = _lib.load().tccl_reduce_rows(
-            tensor.data_ptr(), in_code, block, output.data_ptr(), out_code, block, heap.world_size, block,
-            _launch.byref(_launch.view_of(heap)), None, 0, _launch.stream_ptr(),
-        )
-        _lib.check(rc, "tccl_reduce_rows[reduce_scatter]")
-    return True
+    return _launch.call_table(heap.__dict__).launch(("reduce_scatter", heap.local_base), None, tensor, output) is not None
 
 
 def _check_reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap) -> tuple[int, int, int]:
@@ -237,23 +217,20 @@ def allreduce(tensor: torch.Tensor, heap, op: str = "sum") -> None:
     """In place: once every rank has called, every rank's ``tensor`` holds the sum over ranks."""
     if op != "sum":
         raise ValueError(f"Only op='sum' is currently supported, got {op!r}")
-    if not run_known_allreduce(tensor, heap):
-        _remember(heap, ("allreduce", tensor.shape, tensor.stride(), tensor.dtype, tensor.device), _check_allreduce(tensor, heap))
-        run_known_allreduce(tensor, heap)
+    if run_known_allreduce(tensor, heap):
+        return
+    numel, code = _check_allreduce(tensor, heap)
+    if numel:
+        table, key = _launch.call_table(heap.__dict__), ("allreduce", heap.local_base)
+        _launch.bind(
+            table, key, (tensor,), _lib.load().tccl_allreduce_chunk,
+            ((0, 0), code, numel, _launch.view_of(heap)), "tccl_allreduce_chunk", heap=heap,
+        )
+        _launch.issue(table, key, None, tensor)
 
 
 def run_known_allreduce(tensor: torch.Tensor, heap) -> bool:
-    calls = heap.__dict__.get("_known_calls")
-    known = calls.get(("allreduce", tensor.shape, tensor.stride(), tensor.dtype, tensor.device)) if calls is not None else None
-    if known is None or not heap.owns_tensor(tensor):
-        return False
-    numel, code = known
-    if numel:
-        rc = _lib.load().tccl_allreduce_chunk(
-            tensor.data_ptr(), code, numel, _launch.byref(_launch.view_of(heap)), _launch.stream_ptr()
-        )
-        _lib.check(rc, "tccl_allreduce_chunk")
-    return True
+    return _launch.call_table(heap.__dict__).launch(("allreduce", heap.local_base), None, tensor) is not None
 
 
 def _check_allreduce(tensor: torch.Tensor, heap) -> tuple[int, int]:
@@ -361,6 +338,12 @@ def _one_per_rank(name: str, what: str, tensors, heaps) -> None:
         raise ValueError(f"{name} expects the {what} at the same heap offset on every rank")
 
 
+def _no_fault(heap) -> torch.Tensor:
+    if heap not in _NO_FAULT:
+        _NO_FAULT[heap] = torch.zeros(1, dtype=torch.int64, device="cuda:0")
+    return _NO_FAULT[heap]
+
+
 def _staged(name: str, op: int, srcs, dsts, heaps, block: int, *, root: int = 0, chunk_elems=None, pipeline_slots=None,
             ranks=None, spin_limit_ns: int = _DEFAULT_SPIN_NS) -> torch.Tensor:
     """One launch of ``tccl_collective_staged`` with the roles of ``ranks`` (default: every rank).
@@ -384,9 +367,7 @@ def _staged(name: str, op: int, srcs, dsts, heaps, block: int, *, root: int = 0,
             _launch.byref(view), _launch.stream_ptr(),
         )
         _lib.check(rc, f"tccl_collective_direct[{name}]")
-        if heaps[0] not in _NO_FAULT:
-            _NO_FAULT[heaps[0]] = torch.zeros(1, dtype=torch.int64, device=first.device)
-        return _NO_FAULT[heaps[0]]
+        return _no_fault(heaps[0])
     chunk_elems, chunks, slots = resolve_staged_execution(block, esz, world, chunk_elems=chunk_elems, pipeline_slots=pipeline_slots)
     segments = world if op in (_lib.STAGED_REDUCE_SCATTER, _lib.STAGED_SCATTER) else 1
     cache = _STAGED.setdefault(heaps[0], {})
@@ -416,10 +397,25 @@ def allreduce_staged(tensors, heaps, op: str = "sum", **how) -> torch.Tensor:
     ``chunk_elems``, ``pipeline_slots``, ``ranks``, ``spin_limit_ns``: see ``_staged``."""
     if op != "sum":
         raise ValueError(f"Only op='sum' is currently supported, got {op!r}")
+    plain = not how and 1 < len(heaps) == len(tensors) <= 8  # (a table's calls have few tensors)
+    if plain:
+        bases = [h.local_base for h in heaps]
+        table, key = _launch.call_table(heaps[0].__dict__), ("allreduce_staged", *bases)
+        fault = table.launch(key, None, *tensors)
+        if fault is not None:
+            return fault
     _validate_world_size(len(heaps))
     _one_per_rank("allreduce_staged", "tensor", tensors, heaps)
     if tensors[0].dtype not in _REDUCE_IN:
         raise ValueError(f"allreduce_staged supports fp16, bf16 and fp32 tensors, got {tensors[0].dtype}")
+    numel = int(tensors[0].numel())
+    if plain and numel and numel % 8 == 0:  # what `_staged` would do, kept for the next call
+        _launch.bind(
+            table, key, tuple(tensors), _lib.load().tccl_collective_direct,
+            (_lib.STAGED_ALLREDUCE, None, (0, 0), _launch.dtype_code(tensors[0].dtype), numel, 0, _launch.view_of(heaps[0])),
+            "tccl_collective_direct[allreduce_staged]", tag=_no_fault(heaps[0]), heap=heaps[0], on_heap=1, bases=bases,
+        )
+        return _launch.issue(table, key, None, *tensors)
     return _staged("allreduce_staged", _lib.STAGED_ALLREDUCE, None, tensors, heaps, int(tensors[0].numel()), **how)
 
 

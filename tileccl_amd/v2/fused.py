@@ -19,7 +19,6 @@ which is the full two-rank exchange running through one HBM.
 
 from __future__ import annotations
 
-import ctypes as C
 
 import torch
 
@@ -80,7 +79,7 @@ class _FusedBase:
         self.words: _launch.SyncWords | None = None
         self.locks: torch.Tensor | None = None
         self.directions = 0
-        self._calls = _launch.CallCache()
+        self._calls = _launch.call_table({})
 
     # -- planning -----------------------------------------------------------------------
     def _build_plan(self, M: int, N: int, elem_bytes: int, spec: CollectiveSpec) -> None:
@@ -139,18 +138,17 @@ class _FusedBase:
             self.heap.peer_view(self.signals.counter, peer).fill_(PEER_READY)
             self.heap.peer_view(self.locks, peer).fill_(PEER_READY)
 
-    def _call_key(self, A: torch.Tensor, B: torch.Tensor, variant: str) -> tuple:
-        """What a bound call depends on: the operands' layouts and this operation's settings."""
-        return (A.shape, A.stride(), B.shape, B.stride(), A.dtype, B.dtype, A.device, B.device, A.data_ptr() & 15, B.data_ptr() & 15,
-                variant, self.directions, self.macro_tile, self.num_gemm_wgs, self.num_comm_wgs)
+    def _launch_known(self, A: torch.Tensor, B: torch.Tensor, variant: str, alpha: float, *settings: object) -> None:
+        """Issue the bound call for operands of these layouts and this operation's present settings, made if need be."""
+        key = (variant, self.directions, self.macro_tile, self.num_gemm_wgs, self.num_comm_wgs, self.words, self.transport,
+               self.heap.local_base, *settings)
+        if self._calls.launch(key, alpha, A, B) is None:
+            self.heap.get_heap_bases()  # raises once the heap has been cleaned up
+            self._bind(key, A, B, variant)
+            _launch.issue(self._calls, key, alpha, A, B)
 
-    def _cached(self, key: tuple) -> "_launch.BoundCall | None":
-        self.heap.get_heap_bases()  # raises once the heap has been cleaned up
-        call = self._calls.take(key)
-        return call if call is not None and call.words is self.words and call.keep is self.transport else None
-
-    def _bound(self, A: torch.Tensor, B: torch.Tensor, out: torch.Tensor, variant: str, flags: int):
-        """(gemm descriptor, operand plan, view, transport) of a new bound call."""
+    def _bound(self, key: tuple, A: torch.Tensor, B: torch.Tensor, out: torch.Tensor, variant: str, flags: int, fn, what: str, args) -> None:
+        """Keep the call ``fn(gemm, *args(view, transport), variant)`` for operands of these layouts."""
         if variant not in _launch.VARIANTS:
             raise ValueError(f"unknown variant {variant!r}; expected one of {sorted(_launch.VARIANTS)}")
         gemm, plan = _launch._gemm_desc(
@@ -160,7 +158,8 @@ class _FusedBase:
         transport = _launch.transport_desc(
             self.directions, self.transport.copy_elems, self.transport.reduce_elems, self.num_comm_wgs
         )
-        return gemm, plan, _launch.view_of(self.heap), transport
+        _launch.bind(self._calls, key, (A, B), fn, (gemm, *args(_launch.view_of(self.heap), transport), _launch.VARIANTS[variant]),
+                     f"{what}[{variant}]", gemm=gemm, plan=plan, words=self.words, variant=variant)
 
     def check_faults(self) -> None:
         if self.words is not None:
@@ -191,19 +190,13 @@ class FusedGemmAllGather(_FusedBase):
 
     def __call__(self, A: torch.Tensor, B: torch.Tensor, variant: str = "s2", alpha: float = 1.0,
                  scale_a: float = 1.0, scale_b: float = 1.0) -> torch.Tensor:
-        key = self._call_key(A, B, variant)
-        call = self._cached(key)
-        if call is None:
-            gemm, plan, view, transport = self._bound(A, B, self.local_block, variant, 0)
-            call = _launch.BoundCall(
-                gemm, plan, self.words, variant, _lib.load().tccl_gemm_allgather,
-                (C.byref(gemm), _launch.ptr(self.out), int(self.out.stride(0)), C.byref(view), _launch.SYNC, C.byref(transport),
-                 _launch.VARIANTS[variant]), f"tccl_gemm_allgather[{variant}]", self.transport,
-            )
-        call.gemm.alpha = float(alpha) * float(scale_a) * float(scale_b)  # per-tensor dequantisation scales of fp8 inputs
-        call(A, B)
-        self._calls.put(key, call)
+        # per-tensor dequantisation scales of fp8 inputs
+        self._launch_known(A, B, variant, float(alpha) * float(scale_a) * float(scale_b))
         return self.out
+
+    def _bind(self, key: tuple, A: torch.Tensor, B: torch.Tensor, variant: str) -> None:
+        self._bound(key, A, B, self.local_block, variant, 0, _lib.load().tccl_gemm_allgather, "tccl_gemm_allgather",
+                    lambda view, transport: (_launch.ptr(self.out), int(self.out.stride(0)), view, _launch.SYNC, transport))
 
 
 class FusedGemmReduceScatter(_FusedBase):
@@ -246,19 +239,12 @@ class FusedGemmReduceScatter(_FusedBase):
 
     def __call__(self, A: torch.Tensor, B: torch.Tensor, variant: str = "s2", alpha: float = 1.0,
                  scale_a: float = 1.0, scale_b: float = 1.0) -> torch.Tensor:
-        key = (*self._call_key(A, B, variant), self.emulate_peer, self.own_rows_in_registers)
-        call = self._cached(key)
-        if call is None:
-            gemm, plan, view, transport = self._bound(
-                A, B, self.partial, variant, _lib.GEMM_OWN_ROWS_IN_REGISTERS if self.own_rows_in_registers else 0
-            )
-            call = _launch.BoundCall(
-                gemm, plan, self.words, variant, _lib.load().tccl_gemm_reducescatter,
-                (C.byref(gemm), _launch.ptr(self.out), _launch.dtype_code(self.out.dtype), int(self.out.stride(0)), C.byref(view),
-                 _launch.SYNC, C.byref(transport), int(self.emulate_peer), _launch.VARIANTS[variant]),
-                f"tccl_gemm_reducescatter[{variant}]", self.transport,
-            )
-        call.gemm.alpha = float(alpha) * float(scale_a) * float(scale_b)  # per-tensor dequantisation scales of fp8 inputs
-        call(A, B)
-        self._calls.put(key, call)
+        # per-tensor dequantisation scales of fp8 inputs
+        self._launch_known(A, B, variant, float(alpha) * float(scale_a) * float(scale_b), self.emulate_peer, self.own_rows_in_registers)
         return self.out
+
+    def _bind(self, key: tuple, A: torch.Tensor, B: torch.Tensor, variant: str) -> None:
+        self._bound(key, A, B, self.partial, variant, _lib.GEMM_OWN_ROWS_IN_REGISTERS if self.own_rows_in_registers else 0,
+                    _lib.load().tccl_gemm_reducescatter, "tccl_gemm_reducescatter",
+                    lambda view, transport: (_launch.ptr(self.out), _launch.dtype_code(self.out.dtype), int(self.out.stride(0)), view,
+                                             _launch.SYNC, transport, int(self.emulate_peer)))
