@@ -127,6 +127,39 @@ __global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g, tccl:
 #endif
 }
 
+// At most one tile per CU and a K of some length: K steps of 64, four stages of 32 KiB.  Twice the bytes in flight,
+// half the barriers, and 128-byte pieces of the rows of A (of a k-major B), which cost less where rows start off a
+// 64-byte boundary.  bf16, row-major / k-major B: 2573 x 968 x 3520 41.7 / 42.0 -> 34.3 / 31.8 us, 370 x 5280 x 1656
+// 23.0 / 27.6 -> 21.1 / 22.7, 512 x 7168 x 2944 33.7 / 34.2 -> 29.0 / 28.2.
+template <typename InT, typename OutT>
+__global__ __launch_bounds__(256, 1) void gemm128_deep_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::PushArgs push) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(1024))) char stage0[tccl::kStageDeep];
+  __shared__ __attribute__((aligned(1024))) char stage1[tccl::kStageDeep];
+  __shared__ __attribute__((aligned(1024))) char stage2[tccl::kStageDeep];
+  __shared__ __attribute__((aligned(1024))) char stage3[tccl::kStageDeep];
+  tccl::EpilogueReduce none;
+  none.active = 0;
+  tccl::GemmRole<InT, OutT, 4, 4, 2>(g, push, none, stage0, stage1, stage2, stage3).run(s, (int)blockIdx.x, (int)gridDim.x);
+#endif
+}
+
+// 128 x 256 tiles, eight wavefronts, K steps of 64 in three stages of 48 KiB: a quarter less operand traffic per FLOP
+// than two 128 x 128 workgroups on a CU, and half as many tiles to share out.  bf16, row-major / k-major B, against
+// those two: 6854 x 520 x 2248 51.2 / 61.0 -> 32.1 / 37.7 us, 534 x 7088 x 2960 60.0 / 72.8 -> 38.8 / 45.7, 1956 x
+// 2784 x 2096 43.2 / 51.9 -> 31.2 / 35.7, 1061 x 4432 x 1088 24.5 / 24.0 -> 19.1 / 18.1.
+template <typename InT, typename OutT>
+__global__ __launch_bounds__(512, 2) void gemm_wide_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::PushArgs push) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(1024))) char stage0[tccl::kStageWide];
+  __shared__ __attribute__((aligned(1024))) char stage1[tccl::kStageWide];
+  __shared__ __attribute__((aligned(1024))) char stage2[tccl::kStageWide];
+  tccl::EpilogueReduce none;
+  none.active = 0;
+  tccl::GemmRole<InT, OutT, 3, 8, 2>(g, push, none, stage0, stage1, stage2).run(s, (int)blockIdx.x, (int)gridDim.x);
+#endif
+}
+
 // The transfers that wait for nothing (tccl_bulk.h): blockIdx.y is the rectangle.
 __global__ __launch_bounds__(256) void copy_kernel(tccl::BulkCopyArgs a) {
   tccl::bulk_copy<tccl::kThreadsComm>(a, (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x);
@@ -301,6 +334,7 @@ int build_gemm_args(const tccl_gemm_desc* d, const tccl_device_info& dev, tccl::
     g->span = gemm_span(wgs < total ? wgs : total, d->group_m, dev.xcds);
   }
   g->wrap_rows = d->column_shards > 1 ? d->M / d->column_shards : 0;
+  g->ragged = 0;
   g->b_kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) ? 1 : 0;
   g->b_short = (d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15;
   return 0;
@@ -392,22 +426,31 @@ int check_sync(const tccl_sync_desc* s, int variant) {
 // ------------------------------------------------------------------------------------------
 // Launchers
 // ------------------------------------------------------------------------------------------
+// Kernels for 16-bit inputs, beside the streaming one (tccl_stream.h).  They add products up in the same order: the
+// same bits.
+enum TileKernel { kTiles128, kTiles128Deep, kTilesWide, kTiles256 };
+
 template <typename InT, typename OutT>
-int launch_fused_t(const tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::CommArgs& c, const tccl::PushArgs& push,
-                   const tccl::EpilogueReduce& reduce, int compute, int comm, int64_t* trace_start, hipStream_t stream) {
+int launch_fused_t(tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::CommArgs& c, const tccl::PushArgs& push,
+                   const tccl::EpilogueReduce& reduce, TileKernel kernel, int compute, int comm, int64_t* trace_start, hipStream_t stream) {
   const dim3 block(tccl::kThreads);
   if (reduce.active)
     hipLaunchKernelGGL((gemm128_kernel<InT, OutT, true>), dim3(compute), block, 0, stream, g, s, push, reduce);
-  else if (comm == 0 && !trace_start)
-    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, false>), dim3(compute), block, 0, stream, g, s, push, reduce);
-  else
+  else if (comm > 0 || trace_start)
     hipLaunchKernelGGL((fused_kernel<InT, OutT>), dim3(compute + comm), block, 0, stream, g, s, c, push, compute, trace_start);
+  else if (kernel == kTilesWide)
+    hipLaunchKernelGGL((gemm_wide_kernel<InT, OutT>), dim3(compute), dim3(tccl::kThreadsWide), 0, stream, g, s, push);
+  else if (kernel == kTiles128Deep)
+    hipLaunchKernelGGL((gemm128_deep_kernel<InT, OutT>), dim3(compute), block, 0, stream, g, s, push);
+  else
+    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, false>), dim3(compute), block, 0, stream, g, s, push, reduce);
   TCCL_HIP(hipGetLastError());
   return 0;
 }
 
-int launch_fused(int in_dtype, int out_dtype, const tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::CommArgs& c,
-                 int compute, int comm, int64_t* trace_start, hipStream_t stream, const tccl::PushArgs* push_args = nullptr,
+// `compute` workgroups for the tiles of 128 x 128; the other kernels take what is left of them.
+int launch_fused(int in_dtype, int out_dtype, const tccl::GemmArgs& gemm, const tccl::SignalArgs& s, const tccl::CommArgs& c,
+                 TileKernel kernel, int compute, int comm, int64_t* trace_start, hipStream_t stream, const tccl::PushArgs* push_args = nullptr,
                  const tccl::EpilogueReduce* reduce_args = nullptr) {
   tccl::PushArgs push;
   memset(&push, 0, sizeof push);
@@ -415,10 +458,16 @@ int launch_fused(int in_dtype, int out_dtype, const tccl::GemmArgs& g, const tcc
   tccl::EpilogueReduce reduce;
   memset(&reduce, 0, sizeof reduce);
   if (reduce_args) reduce = *reduce_args;
-  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F16) return launch_fused_t<_Float16, _Float16>(g, s, c, push, reduce, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F32) return launch_fused_t<_Float16, float>(g, s, c, push, reduce, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_BF16) return launch_fused_t<__bf16, __bf16>(g, s, c, push, reduce, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_F32) return launch_fused_t<__bf16, float>(g, s, c, push, reduce, compute, comm, trace_start, stream);
+  tccl::GemmArgs g = gemm;
+  if (kernel == kTilesWide) {
+    const int per = 256 / g.block_n, total = g.tile_rows * ((g.tile_cols + per - 1) / per);
+    if (compute > total) compute = total;
+    g.span = gemm_span(compute, g.group_m, g.xcds);
+  }
+  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F16) return launch_fused_t<_Float16, _Float16>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F32) return launch_fused_t<_Float16, float>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_BF16) return launch_fused_t<__bf16, __bf16>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_F32) return launch_fused_t<__bf16, float>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
   return fail(TCCL_ERR_UNSUPPORTED, "gemm: no kernel for in_dtype=%d, out_dtype=%d", in_dtype, out_dtype);
 }
 
@@ -464,6 +513,60 @@ int default_macro_wgs(const tccl_gemm_desc* d, const tccl_device_info& dev) {
   if (n > dev.compute_units) n = dev.compute_units;
   if (n > total) n = total;
   return n < 1 ? 1 : n;
+}
+
+// ---- the choice among the tiled kernels ------------------------------------------------------------
+// Estimated time of a launch, in us beside the launch itself: workgroups take tiles in rounds, a round takes a K
+// step's time per 64 k (more of it the more CUs are busy: they share the XCDs' L2s and the part's power) and the
+// stores at its end, and rows off a 64-byte boundary cost each step something.
+struct TileCost {
+  double idle, busy;          // K step with few and with all workgroups at work: idle, idle + busy
+  double misaligned;          // added to a step where rows of A or of a k-major B start off 64-byte boundaries
+  double stores, stores_busy; // end of a tile
+  double pushes;              // and for each tile that goes to peers as well
+};
+constexpr TileCost kCost256 = {1.05, 0.28, 0.08, 3.0, 4.0, 3.5};
+constexpr TileCost kCostWide = {0.60, 0.25, 0.12, 2.5, 1.5, 3.0};
+constexpr TileCost kCostDeep = {0.42, 0.13, 0.12, 2.0, 0.0, 1.5};
+constexpr TileCost kCost128 = {0.50, 0.15, 0.12, 0.5, 0.0, 1.5};   // one workgroup per CU
+constexpr TileCost kCost128Two = {1.25, 0.0, 0.10, 1.5, 0.0, 1.5}; // two: as soon as some CU has two
+
+double rounds_us(const TileCost& c, int64_t tiles, int slots, int K, bool pushes) {
+  const double steps = (K + 63) / 64, step = c.idle + (K % 32 ? c.misaligned : 0.0), end = c.stores + (pushes ? c.pushes : 0.0);
+  const double rest = (double)(tiles % slots) / slots;
+  double us = (double)(tiles / slots) * (steps * (step + c.busy) + end + c.stores_busy);
+  if (rest > 0) us += steps * (step + c.busy * rest) + end + c.stores_busy * rest;
+  return us;
+}
+
+struct TileChoice {
+  TileKernel kernel;
+  double us;
+};
+
+// The quickest kernel for `segs` row blocks of `seg_rows` rows in a launch that carries nothing but pushes.  Measured, bf16,
+// on 40 shapes of 100 .. 2200 tiles of 128 x 128: the choice is the quickest kernel or within 12 % of it.
+// What keeps to the old rule: tiles named by the caller, plan tiles other than 128 x 128, workgroup counts.
+TileChoice choose_tiles(const tccl_gemm_desc* d, int64_t seg_rows, int64_t segs, bool allow256, bool pushes, const tccl_device_info& dev) {
+  if (d->in_dtype == TCCL_F8E4M3) return {kTiles256, 0};
+  if (d->macro_tile != 0 || d->num_wgs > 0 || d->block_m != 128 || d->block_n != 128)
+    return {allow256 && use_macro(d, dev, false) ? kTiles256 : kTiles128, 0};
+  const int cus = dev.compute_units;
+  const int64_t rows = (seg_rows + 127) / 128 * segs, small = rows * ((d->N + 127) / 128), wide = rows * ((d->N + 255) / 256);
+  TileChoice best = {kTiles128, small <= cus ? rounds_us(kCost128, small, cus, d->K, pushes) : rounds_us(kCost128Two, small, 2 * cus, d->K, pushes)};
+  const auto offer = [&](TileKernel kernel, double us) {
+    if (us < best.us) best = {kernel, us};
+  };
+  if (small <= cus) offer(kTiles128Deep, rounds_us(kCostDeep, small, cus, d->K, pushes));
+  if (small > cus) offer(kTilesWide, rounds_us(kCostWide, wide, cus, d->K, pushes));
+  if (allow256 && (segs == 1 || seg_rows % 256 == 0))
+    offer(kTiles256, rounds_us(kCost256, (seg_rows + 255) / 256 * segs * ((d->N + 255) / 256), cus, d->K, pushes));
+  return best;
+}
+
+int tile_wgs(TileKernel kernel, const tccl_gemm_desc* d, const tccl_device_info& dev, int total_tiles) {
+  const int n = default_gemm_wgs(d, dev, total_tiles);
+  return kernel != kTiles128 && n > dev.compute_units ? dev.compute_units : n;
 }
 
 // Large-tile kernels: B row-major ones are instantiated here, the k-major ones in tccl_kmajor.hip.
@@ -973,12 +1076,27 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     if (shape >= 0 && !(waits && stream_tiles(shape, seg, 1, d->N) > dev.compute_units))
       return run_stream(d, c, sync, variant, shape, seg, dev, g, stream);
   }
+  const bool traced = sync && (sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock || sync->trace_comm_counter);
+  // Does the launch carry nothing but pushes (reductions over resident partials follow as a kernel of their own)?
+  const bool resident_sums = c.op == tccl::kOpReduceScatter && c.peers_resident && !c.emulate_peer;
+  const bool lone = !gather && (variant == TCCL_S0_BULK ||
+                                (!traced && !(tr && tr->num_comm_wgs > 0) &&
+                                 (c.op == tccl::kOpReduceScatter ? resident_sums && c.world > 1
+                                                                 : c.world <= 1 || c.op != tccl::kOpAllGather || !(c.directions & tccl::kDirPull))));
+  // A reduce-scatter on large tiles sums in their epilogue: the rule for launches that carry more decides there.
+  const bool sums_inside = variant != TCCL_S0_BULK && c.op == tccl::kOpReduceScatter && use_macro(d, dev, true);
+  TileKernel kernel = use_macro(d, dev, variant != TCCL_S0_BULK) ? kTiles256 : kTiles128;
+  if (lone && !sums_inside) {
+    const int segs = d->column_shards > 1 ? d->column_shards : 1;
+    const bool allow256 = plan_tile_fits_macro(d) && !(variant != TCCL_S0_BULK && c.op == tccl::kOpReduceScatter);
+    kernel = choose_tiles(d, d->M / segs, segs, allow256, variant != TCCL_S0_BULK && c.op != tccl::kOpReduceScatter && c.world > 1, dev).kernel;
+  }
   const int total_tiles = g.tile_rows * g.tile_cols;
-  const int compute = default_gemm_wgs(d, dev, total_tiles);
+  const int compute = tile_wgs(kernel, d, dev, total_tiles);
   tccl::SignalArgs s;
   memset(&s, 0, sizeof s);
   int64_t* trace_start = sync ? sync->trace_start_clock : nullptr;
-  if (use_macro(d, dev, variant != TCCL_S0_BULK)) {
+  if (kernel == kTiles256) {
     const int wgs = default_macro_wgs(d, dev);
     const tccl::Macro m = build_macro(d, dev, wgs);
     if (variant == TCCL_S0_BULK) {
@@ -1025,7 +1143,7 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   if (variant == TCCL_S0_BULK) {
     tccl::CommArgs none;
     memset(&none, 0, sizeof none);
-    int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, none, compute, 0, trace_start, stream);
+    int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, none, kernel, compute, 0, trace_start, stream);
     if (rc) return rc;
     if (c.world <= 1 && c.op != tccl::kOpReduceScatter) return 0;
     return launch_bulk(c, dev, stream);
@@ -1047,27 +1165,26 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // launch keeps the pushes in the communication role, whose tasks carry the per-group clock stamps.
   tccl::PushArgs push;
   memset(&push, 0, sizeof push);
-  const bool traced = sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock || sync->trace_comm_counter;
   if (c.op == tccl::kOpReduceScatter && !traced && c.world > 1 && !(tr && tr->num_comm_wgs > 0)) {
     // With the peers' partials there the sums follow as a kernel of their own: one in `world` tiles would do all the
     // reading otherwise, on as many CUs (1024 x 4096 x 2048, four ranks: 37 us; GEMM and reduction one after the other
     // 30 us; communication workgroups beside a three-stage GEMM 48 us).
-    if (c.peers_resident && !c.emulate_peer) {
-      const int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, compute, 0, nullptr, stream);
+    if (resident_sums) {
+      const int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, kernel, compute, 0, nullptr, stream);
       return rc ? rc : launch_bulk(c, dev, stream);
     }
     // Otherwise they happen in the epilogue.  Workgroups that wait for a peer's partials must leave room for the peer's own
     // launch: at most one per CU (two fit).
     if (c.peers_resident || compute <= dev.compute_units) {
       const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
-      return launch_fused(d->in_dtype, d->out_dtype, g, s, c, compute, 0, nullptr, stream, nullptr, &r);
+      return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);
     }
   }
   if (!traced && build_push(c, g, &push)) {
     c.directions &= ~tccl::kDirPush;
     if (c.op != tccl::kOpReduceScatter && !(c.directions & tccl::kDirPull)) comm = 0;
   }
-  return launch_fused(d->in_dtype, d->out_dtype, g, s, c, compute, comm, trace_start, stream, &push);
+  return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kernel, compute, comm, trace_start, stream, &push);
 }
 
 
@@ -1332,13 +1449,15 @@ int tccl_gemm(const tccl_gemm_desc* d, void* stream) {
   }
   tccl::SignalArgs s;
   memset(&s, 0, sizeof s);
-  if (use_macro(d, dev, false)) {
+  const int segs = d->column_shards > 1 ? d->column_shards : 1;
+  const TileKernel kernel = choose_tiles(d, d->M / segs, segs, plan_tile_fits_macro(d), false, dev).kernel;
+  if (kernel == kTiles256) {
     const int wgs = default_macro_wgs(d, dev);
     return launch_gemm256(d->in_dtype, d->out_dtype, g, build_macro(d, dev, wgs), wgs, (hipStream_t)stream);
   }
   tccl::CommArgs none;
   memset(&none, 0, sizeof none);
-  return launch_fused(d->in_dtype, d->out_dtype, g, s, none, default_gemm_wgs(d, dev, g.tile_rows * g.tile_cols), 0, nullptr,
+  return launch_fused(d->in_dtype, d->out_dtype, g, s, none, kernel, tile_wgs(kernel, d, dev, g.tile_rows * g.tile_cols), 0, nullptr,
                       (hipStream_t)stream);
 }
 
@@ -1876,12 +1995,25 @@ static int reduce_ragged_shards(const tccl_gemm_desc* d, void* out, int32_t out_
     add_stream_reduce(c, d, &a);
     return stream_status(tccl::launch_stream(d->in_dtype, g.b_kmajor != 0, shape, a, nullptr, 0, stream));
   }
-  // One GEMM per column block, then the reduction.
+  // All column blocks in one launch, each with tile rows of its own, or, where they are large enough to fill the device,
+  // one GEMM per block (four blocks of 1956 x 696 x 2096: 42 us with the sums, 119 us one after the other); then the
+  // reduction.
+  tccl_gemm_desc one = *d;
+  one.M = g.wrap_rows;
+  one.column_shards = 0;
+  const TileChoice together = choose_tiles(d, g.wrap_rows, d->column_shards, false, false, dev);
+  const double apart = d->column_shards * (kLaunchUs + choose_tiles(&one, one.M, 1, plan_tile_fits_macro(&one), false, dev).us);
+  if (d->in_dtype != TCCL_F8E4M3 && d->block_m == 128 && d->block_n == 128 && d->macro_tile != 256 && together.us < apart) {
+    g.ragged = 1;
+    g.tile_rows = (g.wrap_rows + 127) / 128 * d->column_shards;
+    tccl::SignalArgs s;
+    memset(&s, 0, sizeof s);
+    rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, together.kernel, tile_wgs(together.kernel, d, dev, g.tile_rows * g.tile_cols), 0,
+                      nullptr, stream);
+    return rc ? rc : launch_bulk(c, dev, stream);
+  }
   const size_t isz = dtype_size(d->in_dtype);
   for (int q = 0; q < d->column_shards; ++q) {
-    tccl_gemm_desc one = *d;
-    one.M = g.wrap_rows;
-    one.column_shards = 0;
     one.B = (const char*)d->B + (int64_t)q * d->N * (g.b_kmajor ? d->ldb : 1) * (int64_t)isz;
     one.C = (char*)d->C + (int64_t)q * g.wrap_rows * d->ldc * c.esize;
     if ((rc = tccl_gemm(&one, stream))) return rc;

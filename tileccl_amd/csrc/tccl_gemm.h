@@ -55,13 +55,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTile = 128;                        // sub-tile edge
-constexpr int kBK = 32;                           // K per step
 constexpr int kThreads = 256;                     // threads per workgroup
-constexpr int kARow128 = kBK * 2;                 // bytes of an A row in a stage
-constexpr int kAStage128 = kTile * kARow128;      // 8 192
-constexpr int kBPitch128 = kTile * 2;             // bytes of a k row of B in a stage
-constexpr int kBStage128 = kBK * kBPitch128;      // 8 192 (k-major B: 128 rows of 64 B, the same)
-constexpr int kStage128 = kAStage128 + kBStage128;  // A then B: 16 384; three such stages per workgroup
+constexpr int kStage128 = 16384;                  // a K step of 32: A 128 x 64 B, B 32 x 256 B
+constexpr int kStageDeep = 32768;                 // a K step of 64: A 128 x 128 B, B 64 x 256 B
+constexpr int kThreadsWide = 512;                 // wide form
+constexpr int kStageWide = 49152;                 // a K step of 64: A 128 x 128 B, B 64 x 512 B
 
 enum SignalMode { kSignalNone = 0, kSignalTile = 1, kSignalGroup = 2 };
 
@@ -78,6 +76,8 @@ struct GemmArgs {
   // Column shards stacked as row blocks (0: plain GEMM): C row block q of wrap_rows rows is
   // A (wrap_rows x K) times columns [q * N, (q + 1) * N) of B; tiles never straddle two blocks.
   int wrap_rows;
+  // The row blocks are no whole tiles: each starts a tile row of its own (tile_rows counts them all).
+  int ragged;
   // B is k-major: element (k, n) at B[n * ldb + k] (the `.t()` view of an (N, K) tensor).
   int b_kmajor;
   // Row-major B lacks its last b_short of the K rows: they read as zero (A is zero there as well).
@@ -200,9 +200,19 @@ template <>
 TCCL_D float to_out<float>(float v) { return v; }
 
 #if defined(__HIP_DEVICE_COMPILE__)
-template <typename InT, typename OutT, int kStages = 3>
+template <typename InT, typename OutT, int kStages = 3, int kWaves = 4, int kHalves = 1>
 struct GemmRole {
-  static_assert(kStages == 3 || kStages == 5, "three stages (48 KiB: three workgroups per CU) or five (80 KiB: two)");
+  static constexpr int kWn = kWaves / 2, kCols = 64 * kWn;      // wavefronts across, columns of a sub-tile
+  static constexpr int kStepK = 32 * kHalves;
+  static constexpr int kRowB = 2 * kStepK;                      // bytes of an A row in a stage
+  static constexpr int kRowLanes = kRowB / 16;                  // lanes that fetch one
+  static constexpr int kAStage = kTile * kRowB;
+  static constexpr int kBPitch = kCols * 2;                     // bytes of a k row of B in a stage
+  static constexpr int kStage = kAStage + kStepK * kBPitch;
+  static constexpr int kBLanes = kBPitch / 16;                  // lanes that fetch a k row of B
+  static constexpr int kALoads = kAStage / 1024 / kWaves;           // 1 KiB pieces per wavefront and step
+  static constexpr int kBLoads = kStepK * kBPitch / 1024 / kWaves;
+  static constexpr int kLoads = kALoads + kBLoads;
   typedef typename Mfma<InT>::Vec Vec;
   static_assert(sizeof(InT) == 2, "16-bit inputs");
   typedef __attribute__((address_space(3))) void LdsVoid;
@@ -224,7 +234,7 @@ struct GemmRole {
   TCCL_D GemmRole(const GemmArgs& args, const PushArgs& push_args, const EpilogueReduce& reduce_args, char* s0, char* s1, char* s2,
                   char* s3 = nullptr, char* s4 = nullptr)
       : g(args), push(push_args), reduce(reduce_args), st0(s0), st1(s1), st2(s2), st3(s3), st4(s4), tid(threadIdx.x), lane(threadIdx.x & 63),
-        wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wm(wave >> 1), wn(wave & 1) {}
+        wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wm(wave / kWn), wn(wave % kWn) {}
 
   static TCCL_D int fresh(int v) {
     asm volatile("" : "+v"(v));
@@ -233,16 +243,19 @@ struct GemmRole {
   static TCCL_D uint32_t clamp_u32(int64_t v) { return v > 0xffffffffll ? 0xffffffffu : (v < 0 ? 0u : (uint32_t)v); }
 
   // ---- global -> LDS ------------------------------------------------------------------------
-  // Per K step a wavefront fetches two 1 KiB pieces of each operand:
-  //   A piece i: rows 16 (2 wave + i) .. + 15      (lane l: row + l / 4, slot l % 4)
-  //   B piece j: k rows 4 (2 wave + j) .. + 3      (lane l: k row + l / 16, slot l % 16)
-  //   k-major B piece j: columns 16 (2 wave + j) .. + 15, as A.
+  // Per K step a wavefront fetches two 1 KiB pieces of A and kBLoads of B (wide form in brackets):
+  //   A piece i: rows 16 [8] (2 wave + i) .. + 15 [7]    (lane l: row + l / 4 [8], slot l % 4 [8])
+  //   B piece j: k rows 4 (2 wave + j) .. + 3            (lane l: k row + l / 16, slot l % 16)
+  //              [2 (4 wave + j), + 1                    (lane l: k row + l / 32, slot l % 32)]
+  //   k-major B piece j: columns as A's rows.
   struct Source {
     __amdgpu_buffer_rsrc_t a, b;
-    uint32_t off_a[2], off_b[2];  // byte offsets of this lane's 16-byte loads, K step 0
-    uint32_t step_a, step_b;      // byte advance per K step
-    int k_lane;                   // first k of this lane's chunk of an A row (of a k-major B row) within a step
+    uint32_t off_a[kALoads], off_b[kBLoads];  // byte offsets of this lane's 16-byte loads, K step 0
+    uint32_t step_a, step_b;            // byte advance per K step
+    int k_lane[2];                      // first k of this lane's chunk of a row of piece 0 / 1 (even / odd pieces) within a step
   };
+  // Swizzle of an A row (of a k-major B row) in a stage: 16-byte chunk c in slot c ^ swizzle(row).
+  static TCCL_D int swizzle(int row) { return (row >> 1) & (kRowLanes - 1); }
 
   template <bool kBKMajor>
   TCCL_D Source make_source(int row0, int col0) const {
@@ -254,46 +267,56 @@ struct GemmRole {
     s.a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(((int64_t)(o.a_rows - 1 - o.a_row) * g.lda + g.K) * 2), 0x00020000);
     const int64_t b_elems = kBKMajor ? (int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K : (int64_t)(g.K - 1 - g.b_short) * g.ldb + (o.b_cols - o.b_col);
     s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(b_elems * 2), 0x00020000);
-    // Bits 1 and 2 of a row's number come from the lane alone (a piece starts on a multiple of 16).
-    const int kc = (ln & 3) ^ ((ln >> 3) & 3);
-    s.k_lane = kc * 8;
+    constexpr int kRows = 64 / kRowLanes;  // rows of a piece
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = 16 * (2 * wave + i) + (ln >> 2);
-      s.off_a[i] = (uint32_t)(row * g.lda * 2 + kc * 16);
+    for (int i = 0; i < 2; ++i) s.k_lane[i] = ((ln % kRowLanes) ^ swizzle(kRows * i + ln / kRowLanes)) * 8;
+#pragma unroll
+    for (int i = 0; i < kALoads; ++i) s.off_a[i] = (uint32_t)((kRows * (kALoads * wave + i) + ln / kRowLanes) * g.lda * 2 + s.k_lane[i & 1] * 2);
+#pragma unroll
+    for (int j = 0; j < kBLoads; ++j) {
       if constexpr (kBKMajor) {
-        s.off_b[i] = (uint32_t)(row * g.ldb * 2 + kc * 16);
+        const int row = kRows * (kBLoads * wave + j) + ln / kRowLanes;
+        s.off_b[j] = (uint32_t)(row * g.ldb * 2 + s.k_lane[j & 1] * 2);
       } else {
-        const int k = 4 * (2 * wave + i) + (ln >> 4);
-        const int c = (ln & 15) ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1));
-        s.off_b[i] = (uint32_t)(k * g.ldb * 2 + c * 16);
+        const int k = 64 / kBLanes * (kBLoads * wave + j) + ln / kBLanes;
+        const int c = (ln % kBLanes) ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1));
+        s.off_b[j] = (uint32_t)(k * g.ldb * 2 + c * 16);
       }
     }
-    s.step_a = kBK * 2;
-    s.step_b = kBKMajor ? (uint32_t)(kBK * 2) : (uint32_t)(kBK * g.ldb * 2);
+    s.step_a = kStepK * 2;
+    s.step_b = kBKMajor ? (uint32_t)(kStepK * 2) : (uint32_t)(kStepK * g.ldb * 2);
     return s;
   }
 
   // Piece i of K step kt, straight into `stage`.
   TCCL_D void issue_a(char* stage, const Source& s, int kt, int i) const {
-    const bool dead = kt * kBK + s.k_lane >= g.K;
+    const bool dead = kt * kStepK + s.k_lane[i & 1] >= g.K;
     const uint32_t oa = dead ? 0xfffffff0u : s.off_a[i] + kt * s.step_a;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.a, (LdsVoid*)(stage + (2 * wave + i) * 1024), 16, oa, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.a, (LdsVoid*)(stage + (kALoads * wave + i) * 1024), 16, oa, 0, 0, 0);
   }
   template <bool kBKMajor>
   TCCL_D void issue_b(char* stage, const Source& s, int kt, int i) const {
     uint32_t ob = s.off_b[i] + kt * s.step_b;  // row-major B: rows >= K lie past the end of the buffer
-    if constexpr (kBKMajor) ob = (kt * kBK + s.k_lane >= g.K) ? 0xfffffff0u : ob;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.b, (LdsVoid*)(stage + kAStage128 + (2 * wave + i) * 1024), 16, ob, 0, 0, 0);
+    if constexpr (kBKMajor) ob = (kt * kStepK + s.k_lane[i & 1] >= g.K) ? 0xfffffff0u : ob;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.b, (LdsVoid*)(stage + kAStage + (kBLoads * wave + i) * 1024), 16, ob, 0, 0, 0);
+  }
+  // Load number n of a K step: A 0, B 0, A 1, B 1, then the rest of B.
+  template <bool kBKMajor>
+  TCCL_D void issue(char* stage, const Source& s, int kt, int n) const {
+    if (n < 2 * kALoads && !(n & 1))
+      issue_a(stage, s, kt, n >> 1);
+    else
+      issue_b<kBKMajor>(stage, s, kt, n < 2 * kALoads ? n >> 1 : n - kALoads);
   }
   template <bool kBKMajor>
-  TCCL_D void issue_piece(char* stage, const Source& s, int kt, int i) const {
-    issue_a(stage, s, kt, i);
-    issue_b<kBKMajor>(stage, s, kt, i);
+  TCCL_D void issue_step(char* stage, const Source& s, int kt) const {
+#pragma unroll
+    for (int n = 0; n < kLoads; ++n) issue<kBKMajor>(stage, s, kt, n);
   }
 
   // ---- LDS -> MFMA operands -------------------------------------------------------------------
   // 16 x 16 x 32 operands: lane l holds the 8 consecutive k of group l / 16 for row (column) l % 16.
+  // (the wide form's second 32-k half: A chunks 4 + group, i.e. bit 2 of the slot flipped; B k rows 32 further on)
   struct Reader {
     uint32_t a_base;   // this lane's row of A row block 0, slot applied
     uint32_t b_base0;  // this lane's address for column block 0
@@ -302,25 +325,27 @@ struct GemmRole {
   TCCL_D Reader make_reader() const {
     const int i16 = lane & 15, kg = lane >> 4;
     Reader r;
-    r.a_base = (uint32_t)((wm * 64 + i16) * kARow128 + ((kg ^ ((i16 >> 1) & 3)) << 4));
+    r.a_base = (uint32_t)((wm * 64 + i16) * kRowB + ((kg ^ swizzle(i16)) << 4));
     if constexpr (kBKMajor) {
-      r.b_base0 = (uint32_t)(kAStage128 + (wn * 64 + i16) * kARow128 + ((kg ^ ((i16 >> 1) & 3)) << 4));
+      r.b_base0 = (uint32_t)(kAStage + (wn * 64 + i16) * kRowB + ((kg ^ swizzle(i16)) << 4));
     } else {
       // Lane group kg covers k rows 8 kg .. + 7 in two transposing reads (k + 0, k + 4).
       const int t = i16 >> 2, cq = i16 & 3;
       const int chunk = (wn * 8 + (cq >> 1)) ^ (4 * t) ^ (2 * (kg & 1));
-      r.b_base0 = (uint32_t)(kAStage128 + (8 * kg + t) * kBPitch128 + chunk * 16 + (cq & 1) * 8);
+      r.b_base0 = (uint32_t)(kAStage + (8 * kg + t) * kBPitch + chunk * 16 + (cq & 1) * 8);
     }
     return r;
   }
-  TCCL_D Vec load_a(const char* stage, const Reader& r, int rb) const { return *(const Vec*)(stage + r.a_base + rb * 16 * kARow128); }
+  TCCL_D Vec load_a(const char* stage, const Reader& r, int h, int rb) const {
+    return *(const Vec*)(stage + (r.a_base ^ (uint32_t)(64 * h)) + rb * 16 * kRowB);
+  }
   template <bool kBKMajor>
-  TCCL_D Vec load_b(const char* stage, const Reader& r, int cb) const {
-    if constexpr (kBKMajor) return *(const Vec*)(stage + r.b_base0 + cb * 16 * kARow128);
+  TCCL_D Vec load_b(const char* stage, const Reader& r, int h, int cb) const {
+    if constexpr (kBKMajor) return *(const Vec*)(stage + (r.b_base0 ^ (uint32_t)(64 * h)) + cb * 16 * kRowB);
     // column block cb: two chunks further on (the XOR commutes with the swizzle terms)
-    const char* pb = stage + (r.b_base0 ^ (uint32_t)(32 * cb));
+    const char* pb = stage + (r.b_base0 ^ (uint32_t)(32 * cb)) + 32 * h * kBPitch;
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)pb);
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)(pb + 4 * kBPitch128));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)(pb + 4 * kBPitch));
     const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(Vec, both);
   }
@@ -329,41 +354,45 @@ struct GemmRole {
     Vec fa[4], fb[4];
   };
 
-  // One K step: four items (A row block rb against the four B column blocks).  On entry fa[0], fa[1] and
-  // fb[0..3] hold this step's operands; items 0 and 1 fetch fa[2] and fa[3]; the last item, behind the
-  // barrier, fetches the next step's fa[0], fa[1] from `nxt` and reloads each fb in place.  The four loads of
-  // K step kt_load into `far` (the stage read during the step before) go out one per item: a wavefront issues
-  // nothing else while the address unit accepts its load, and the four wavefronts reach an item together.
-  // The fourth goes out behind the barrier, so at the barrier the loads that may still be in flight are
-  // those of the kStages - 2 steps before, less that one.
-  static constexpr int kInFlight = 4 * (kStages - 2) - 1;
+  // One K step: four items per 32-k half (A row block rb against the four B column blocks).  On entry fa[0], fa[1]
+  // and fb[0..3] hold this step's operands; items 0 and 1 of a half fetch fa[2] and fa[3]; its last item
+  // fetches the next half's fa[0], fa[1] and reloads each fb in place, the step's last item, behind the
+  // barrier, from `nxt`.  The loads of K step kt_load into `far` (the stage read during the step before) go out one per
+  // item: a wavefront issues nothing else while the address unit accepts its load, and the wavefronts reach an item
+  // together.  At the barrier the loads that may still be in flight are those of the kStages - 2 steps before
+  // (four-wavefront form: less the fourth one, which goes out behind the barrier).
+  static constexpr int kItems = 4 * kHalves;
+  static constexpr int kInFlight = kLoads * (kStages - 2) - (kLoads >= kItems ? kLoads - kItems + 1 : 0);
   template <bool kBKMajor>
   TCCL_D void k_step(const char* cur, const char* nxt, char* far, const Source& src, const Reader& rd, int kt_load,
                      f32x4 (&acc)[4][4], Frags& f) const {
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-      if (rb == 3) {
+    for (int it = 0; it < kItems; ++it) {
+      const int rb = it & 3, h = it >> 2;
+      const bool last = it == kItems - 1;
+      const char* from = last ? nxt : cur;  // of the next half's operands
+      const int hn = last ? 0 : h + 1;
+      if (last) {
         // The loads of K step t + 1 (into `nxt`) have landed; this wavefront's reads of `cur` are done.
         // The barrier is the bare instruction (__syncthreads() carries a release fence); the empty asm
         // keeps LDS accesses from moving across it.
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kInFlight) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        f.fa[0] = load_a(nxt, rd, 0);
-        f.fa[1] = load_a(nxt, rd, 1);
-      } else if (rb < 2) {
-        f.fa[rb + 2] = load_a(cur, rd, rb + 2);
       }
-      if (rb & 1)
-        issue_b<kBKMajor>(far, src, kt_load, rb >> 1);
-      else
-        issue_a(far, src, kt_load, rb >> 1);
+      if (rb == 3) {
+        f.fa[0] = load_a(from, rd, hn, 0);
+        f.fa[1] = load_a(from, rd, hn, 1);
+      } else if (rb < 2) {
+        f.fa[rb + 2] = load_a(cur, rd, h, rb + 2);
+      }
+      if (it < kLoads) issue<kBKMajor>(far, src, kt_load, it);
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
         acc[rb][cb] = Mfma<InT>::run16(f.fb[cb], f.fa[rb], acc[rb][cb]);
         if (rb == 3) {
           __builtin_amdgcn_sched_barrier(0);
-          f.fb[cb] = load_b<kBKMajor>(nxt, rd, cb);
+          f.fb[cb] = load_b<kBKMajor>(from, rd, hn, cb);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -378,12 +407,13 @@ struct GemmRole {
   // kReduce: the launch is a reduce-scatter that reduces here; `sums`: this sub-tile's rows are summed (its owner is this
   // rank, or emulated, and the peers' partials are there).
   template <int kPolicy, bool kReduce>
-  TCCL_D void epilogue(int row0, int col0, const f32x4 (&acc)[4][4], bool sums) const {
+  TCCL_D void epilogue(int row0, int row_end, int col0, const f32x4 (&acc)[4][4], bool sums) const {
     constexpr int kEsz = sizeof(OutT);
     constexpr int kRowBytes = 64 * kEsz;       // one wave row: 64 columns
     constexpr int kChunks = kRowBytes / 16;    // 16-byte chunks per row (8 or 16)
     constexpr int kPerChunk = 16 / kEsz;       // elements per chunk
-    char* win = (wave < 2 ? st0 : st1) + (wave & 1) * 8192;  // 8 KiB per wavefront (fp32 worst case)
+    constexpr int kWindows = kStage / 8192;  // 8 KiB per wavefront (fp32 worst case), in stages 0 and 1
+    char* win = (wave < kWindows ? st0 : st1) + (wave % kWindows) * 8192;
     // The lane id is taken afresh: what the epilogue derives from it is invariant across tiles
     // and would otherwise be hoisted out of the tile loop and held in registers through the K loop.
     const int ln = fresh(lane);
@@ -431,7 +461,7 @@ struct GemmRole {
         v[r] = *(const u32x4*)(win + row * kRowBytes + ((chunk ^ (row & 7)) * 16));
         lrow[r] = wm * 64 + bi * 32 + row;
         lcol[r] = wn * 64 + chunk * kPerChunk;
-        live[r] = row0 + lrow[r] < g.M && col0 + lcol[r] < g.N;
+        live[r] = row0 + lrow[r] < row_end && col0 + lcol[r] < g.N;
         if (kReduce && !store) continue;
         if (live[r]) __builtin_amdgcn_raw_buffer_store_b128(v[r], rc, (uint32_t)((lrow[r] * g.ldc + lcol[r]) * kEsz), 0, kPolicy);
       }
@@ -512,9 +542,9 @@ struct GemmRole {
     }
   }
 
-  // ---- one 128 x 128 sub-tile -------------------------------------------------------------------
+  // ---- one 128 x kCols sub-tile -------------------------------------------------------------------
   template <int kPolicy, bool kBKMajor, bool kReduce>
-  TCCL_D void subtile(int row0, int col0, int tile_id, const SignalArgs& s) const {
+  TCCL_D void subtile(int row0, int row_end, int col0, int tile_id, const SignalArgs& s) const {
     f32x4 acc[4][4];  // cleared two registers per instruction
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -533,28 +563,21 @@ struct GemmRole {
 
     const Source src = make_source<kBKMajor>(row0, col0);
     const Reader rd = make_reader<kBKMajor>();
-    const int ksteps = (g.K + kBK - 1) / kBK;
+    const int ksteps = (g.K + kStepK - 1) / kStepK;
     __syncthreads();  // the previous sub-tile's epilogue has left LDS
-    // K steps 0 .. kStages - 2 go out up front (past K: zeros, never consumed); the order within a step is
-    // the one k_step() issues in (A 0, B 0, A 1, B 1).
-    issue_piece<kBKMajor>(st0, src, 0, 0);
-    issue_piece<kBKMajor>(st0, src, 0, 1);
-    issue_piece<kBKMajor>(st1, src, 1, 0);
-    issue_piece<kBKMajor>(st1, src, 1, 1);
-    if constexpr (kStages == 5) {
-      issue_piece<kBKMajor>(st2, src, 2, 0);
-      issue_piece<kBKMajor>(st2, src, 2, 1);
-      issue_piece<kBKMajor>(st3, src, 3, 0);
-      issue_piece<kBKMajor>(st3, src, 3, 1);
-    }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (kStages - 2)) : "memory");  // stage 0 has landed
+    // K steps 0 .. kStages - 2 go out up front (past K: zeros, never consumed).
+    issue_step<kBKMajor>(st0, src, 0);
+    issue_step<kBKMajor>(st1, src, 1);
+    if constexpr (kStages >= 4) issue_step<kBKMajor>(st2, src, 2);
+    if constexpr (kStages == 5) issue_step<kBKMajor>(st3, src, 3);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads * (kStages - 2)) : "memory");  // stage 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     Frags f;
-    f.fa[0] = load_a(st0, rd, 0);
-    f.fa[1] = load_a(st0, rd, 1);
+    f.fa[0] = load_a(st0, rd, 0, 0);
+    f.fa[1] = load_a(st0, rd, 0, 1);
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b<kBKMajor>(st0, rd, cb);
+    for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b<kBKMajor>(st0, rd, 0, cb);
     // Step t computes from stage t % kStages, fetches its last operands from the next one and loads K step
     // t + kStages - 1 into the one before.  Stages are named statically (the compiler tracks loads into LDS
     // per array), so the loop comes in rounds of kStages steps with an exit after every step.
@@ -566,6 +589,17 @@ struct GemmRole {
         if (kt + 2 >= ksteps) break;
         k_step<kBKMajor>(st2, st0, st1, src, rd, kt + 4, acc, f);
         if (kt + 3 >= ksteps) break;
+      }
+    } else if constexpr (kStages == 4) {
+      for (int kt = 0;; kt += 4) {
+        k_step<kBKMajor>(st0, st1, st3, src, rd, kt + 3, acc, f);
+        if (kt + 1 >= ksteps) break;
+        k_step<kBKMajor>(st1, st2, st0, src, rd, kt + 4, acc, f);
+        if (kt + 2 >= ksteps) break;
+        k_step<kBKMajor>(st2, st3, st1, src, rd, kt + 5, acc, f);
+        if (kt + 3 >= ksteps) break;
+        k_step<kBKMajor>(st3, st0, st2, src, rd, kt + 6, acc, f);
+        if (kt + 4 >= ksteps) break;
       }
     } else {
       for (int kt = 0;; kt += 5) {
@@ -587,7 +621,7 @@ struct GemmRole {
       const int owner = row0 / reduce.shard_rows;
       sums = (owner == reduce.rank || reduce.emulate_peer) && peers_there(tile_id, s);
     }
-    epilogue<kPolicy, kReduce>(row0, col0, acc, sums);
+    epilogue<kPolicy, kReduce>(row0, row_end, col0, acc, sums);
   }
 
   // The peers' partials of plan tile `tile_id` are published (one lane waits, bounded).
@@ -616,43 +650,54 @@ struct GemmRole {
   }
 
   // ---- persistent loop over plan tiles ----------------------------------------------------------
+  // A workgroup takes a plan tile at a time, as sub-tiles; in the wide form, where one is narrower than a sub-tile, the
+  // one on its right with it.
   template <bool kReduce = false>
   TCCL_D void run(const SignalArgs& s, int wg, int num_wgs) const {
-    const int total = g.tile_rows * g.tile_cols;
+    const int per = kWn == 4 ? kCols / g.block_n : 1;  // plan tiles across
+    const int cols = kWn == 4 ? (g.tile_cols + per - 1) / per : g.tile_cols;
+    const int total = g.tile_rows * cols;
     for (int slot = wg; slot < total; slot += num_wgs) {
-      int tile_id = tile_for_slot(slot, total, g.xcds, g.span);
-      TileCoord tc = tile_coords(tile_id, g.tile_rows, g.tile_cols, g.group_m);
+      TileCoord tc = tile_coords(tile_for_slot(slot, total, g.xcds, g.span), g.tile_rows, cols, g.group_m);
       if constexpr (kReduce) {  // this rank's own rows come last: what its peers wait for comes first
         tc.m += (reduce.rank + 1) % reduce.world * (g.tile_rows / reduce.world);
         if (tc.m >= g.tile_rows) tc.m -= g.tile_rows;
-        tile_id = tile_id_of(tc.m, tc.n, g.tile_rows, g.tile_cols, g.group_m);
       }
+      tc.n *= per;
+      int first_row = tc.m * g.block_m, row_end = g.M;
+      if (g.ragged) {
+        const int tiles = (g.wrap_rows + g.block_m - 1) / g.block_m, q = tc.m / tiles;
+        first_row = q * g.wrap_rows + (tc.m - q * tiles) * g.block_m;
+        row_end = (q + 1) * g.wrap_rows;
+      }
+      const int tile_id = kReduce ? tile_id_of(tc.m, tc.n, g.tile_rows, g.tile_cols, g.group_m) : 0;
       for (int sm = 0; sm < g.block_m; sm += kTile)
-        for (int sn = 0; sn < g.block_n; sn += kTile) {
-          const int row0 = tc.m * g.block_m + sm, col0 = tc.n * g.block_n + sn;
-          if (row0 >= g.M || col0 >= g.N) continue;
+        for (int sn = 0; sn < per * g.block_n; sn += kCols) {
+          const int row0 = first_row + sm, col0 = tc.n * g.block_n + sn;
+          if (row0 >= row_end || col0 >= g.N) continue;
           if (s.mode == kSignalNone) {
             if (g.b_kmajor)
-              subtile<0, true, kReduce>(row0, col0, tile_id, s);
+              subtile<0, true, kReduce>(row0, row_end, col0, tile_id, s);
             else
-              subtile<0, false, kReduce>(row0, col0, tile_id, s);
+              subtile<0, false, kReduce>(row0, row_end, col0, tile_id, s);
           } else {
             if (g.b_kmajor)
-              subtile<kCoherent, true, kReduce>(row0, col0, tile_id, s);
+              subtile<kCoherent, true, kReduce>(row0, row_end, col0, tile_id, s);
             else
-              subtile<kCoherent, false, kReduce>(row0, col0, tile_id, s);
+              subtile<kCoherent, false, kReduce>(row0, row_end, col0, tile_id, s);
           }
         }
       if (s.mode != kSignalNone) {
         // The tile was stored write-through; once every wave's stores have completed the
-        // data is visible device-wide and one lane may publish the signal.
+        // data is visible device-wide and one lane (per plan tile) may publish the signal.
         wait_vmem();
         __syncthreads();
-        if (tid == 0) {
+        if (tid < per && tc.n + tid < g.tile_cols) {
+          const int done = tile_id_of(tc.m, tc.n + tid, g.tile_rows, g.tile_cols, g.group_m);
           if (s.mode == kSignalTile)
-            tile_publish(s.locks, tile_id, s.epoch);
+            tile_publish(s.locks, done, s.epoch);
           else
-            tile_signal_add<true>(s.counter, s.group_table[tile_id], 1);
+            tile_signal_add<true>(s.counter, s.group_table[done], 1);
         }
       }
     }
