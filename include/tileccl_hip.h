@@ -156,10 +156,12 @@ typedef struct tccl_sync_desc {
 } tccl_sync_desc;
 
 /* What `sync` points at in a launch whose gemm->flags has TCCL_GEMM_ARRIVALS (pass &x.sync).
- *   arrivals   uint32[total_tiles], device memory (in the heap or not), zeroed once by the host and zero
+ *   arrivals   uint32[TCCL_ARRIVAL_STRIDE * total_tiles] (a counter at the start of each tile's words, which
+ *              no other tile's counting then holds up), device memory (in the heap or not), zeroed once by the host and zero
  *              again after every launch.
  * With them small problems are computed in tiles smaller than a plan tile (up to 5 times as fast at
  * 16 x 2048 x 4096): the last of a plan tile's tiles, found by counting here, publishes it. */
+#define TCCL_ARRIVAL_STRIDE 32
 typedef struct tccl_sync_desc_arrivals {
   tccl_sync_desc sync;
   int32_t* arrivals;

@@ -233,6 +233,7 @@ def gemm_desc(A: torch.Tensor, B: torch.Tensor, C_out: torch.Tensor, **how) -> _
     return d
 
 
+_ENTRIES: dict[str, tuple] = {}  # an operation's entry point and its address
 SYNC = object()  # stands for the sync descriptor in the arguments of a bound call
 
 
@@ -256,24 +257,26 @@ def bind(table, key: tuple, tensors: tuple, fn, args: tuple, what: str, *, gemm:
     The tensors of the bit mask ``on_heap`` (default: all) must start inside ``heap``; with ``bases`` all tensors must lie at
     one distance from their base.  Tensors for which that does not hold find no call."""
     host = _lib.host()
+    entry = _ENTRIES.get(what)
+    if entry is None or entry[0] is not fn:
+        entry = _ENTRIES[what] = fn, C.cast(fn, C.c_void_p).value
     keep = [words]  # what the descriptors point at lives as long as the call
-
-    def value(a):
+    passed = []
+    for a in args:
         if a is gemm and a is not None:
-            return host.GEMM
-        if a is SYNC:
-            return None if words is None else host.SYNC
-        if isinstance(a, C.Structure):
+            a = host.GEMM
+        elif a is SYNC:
+            a = None if words is None else host.SYNC
+        elif isinstance(a, C.Structure):
             keep.append(a)
-            return C.addressof(a)
-        return a
-
+            a = C.addressof(a)
+        passed.append(a)
     sync = None if words is None else words.desc(variant)
     packs = plan is not None and (plan.pack_a or plan.pack_b)
     table.add(host.Call(
-        C.cast(fn, C.c_void_p).value, what, tuple(value(a) for a in args), tensors, key, tag=tag,
-        gemm=C.addressof(gemm) if gemm is not None else 0, c=c, sync=C.addressof(sync) if sync is not None else 0, words=words,
-        variant=variant, on_heap=on_heap, heap=(heap.local_base, heap.size) if heap is not None else None, bases=bases,
+        entry[1], what, tuple(passed), tensors, key, tag=tag, gemm=0 if gemm is None else C.addressof(gemm), c=c,
+        sync=0 if sync is None else C.addressof(sync), words=words, variant=variant, on_heap=on_heap,
+        heap=None if heap is None else (heap.local_base, heap.size), bases=bases,
         prepare=partial(planned_operands, plan) if packs else None, keep=keep,
     ))
 
@@ -370,7 +373,7 @@ class SyncWords:
     lock_epoch: int = 0
     spin_limit_ns: int = DEFAULT_SPIN_LIMIT_NS
     max_tasks_per_tile: int = 1 << 16
-    arrivals: torch.Tensor | None = None  # one counter per plan tile, zero between launches (tccl_sync_desc_arrivals)
+    arrivals: torch.Tensor | None = None  # a counter per plan tile, zero between launches (tccl_sync_desc_arrivals)
     arrivals_from_capture: bool = False  # zeroed by a recorded fill only: every launch has to clear them itself
     clear_every_launch: bool = False  # set by the first launch recorded into a graph
 
@@ -405,7 +408,7 @@ class SyncWords:
         if self.arrivals is None:
             tiles = max(int(t.numel()) for t in (self.locks, self.plan.group_table if self.plan is not None else None) if t is not None)
             self.arrivals_from_capture = torch.cuda.is_current_stream_capturing()
-            self.arrivals = torch.zeros(tiles, dtype=torch.int32, device="cuda:0")
+            self.arrivals = torch.zeros(tiles * _lib.ARRIVAL_STRIDE, dtype=torch.int32, device="cuda:0")
         return self.arrivals
 
     def desc(self, variant: str = "s2") -> _lib.SyncDescArrivals:

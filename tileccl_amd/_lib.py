@@ -64,6 +64,7 @@ class GemmDesc(C.Structure):
 GEMM_OWN_ROWS_IN_REGISTERS = 1  # TCCL_GEMM_OWN_ROWS_IN_REGISTERS
 GEMM_B_KMAJOR = 2  # TCCL_GEMM_B_KMAJOR
 GEMM_ARRIVALS = 4  # TCCL_GEMM_ARRIVALS
+ARRIVAL_STRIDE = 32  # words per plan tile of tccl_sync_desc_arrivals.arrivals
 GEMM_B_SHORT_SHIFT = 8  # TCCL_GEMM_B_SHORT_SHIFT
 STAGED_ALLREDUCE, STAGED_ALLGATHER, STAGED_REDUCE_SCATTER, STAGED_BROADCAST, STAGED_SCATTER = range(5)  # TCCL_STAGED_*
 

@@ -39,6 +39,7 @@ int hip_fail(hipError_t e, const char* what) {
   return fail((int)e, "HIP error in %s: %s (%d)", what, hipGetErrorString(e), (int)e);
 }
 
+static_assert(tccl::kArrivalStride == TCCL_ARRIVAL_STRIDE, "the kernel and the interface agree");
 #define TCCL_HIP(call)                                  \
   do {                                                  \
     hipError_t e_ = (call);                             \
@@ -974,7 +975,7 @@ void build_stream(const tccl_gemm_desc* d, const tccl::GemmArgs& g, int64_t seg_
   a->out_dtype = d->out_dtype;
   a->seg_rows = (int)seg_rows;
   a->wrapped = g.wrap_rows > 0;
-  a->xcds = dev.xcds;
+  a->xcd_shift = dev.xcds == 8 ? 3 : 0;  // query_device() knows no others
   a->block_m = g.block_m;
   a->block_n = g.block_n;
   a->group_m = g.group_m;
@@ -1022,7 +1023,7 @@ int run_stream(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc*
   build_stream(d, g, seg_rows, dev, &a);
   const bool kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) != 0;
   if (variant == TCCL_S0_BULK) {
-    const int rc = stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, nullptr, 0, stream));
+    const int rc = stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, stream));
     if (rc || (c.world <= 1 && c.op != tccl::kOpReduceScatter)) return rc;
     return launch_bulk(c, dev, stream);
   }
@@ -1043,22 +1044,27 @@ int run_stream(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc*
   }
   if (c.op == tccl::kOpReduceScatter) {
     add_stream_reduce(c, d, &a);
-    return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, nullptr, 0, stream));
+    return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, stream));
   }
   if (build_push(c, g, &a.push)) c.directions &= ~tccl::kDirPush;
   if (c.op != tccl::kOpAllGather || !(c.directions & tccl::kDirPull) || c.world <= 1)
-    return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, nullptr, 0, stream));
-  // The pulls, in tasks small enough that every communication workgroup has one.
-  int tasks = (c.world - 1) * g.tile_rows * g.tile_cols;
-  if (c.granularity == tccl::kPerGroup) {
-    const int64_t units = (int64_t)c.M * c.N * c.esize / 16 * (c.world - 1);
-    int64_t per = (units + dev.compute_units - 1) / dev.compute_units;
-    per = (per + 255) / 256 * 256;
-    if (per < c.copy_units) c.copy_units = (int)per;
-    tasks = (int)((units + c.copy_units - 1) / c.copy_units);
-  }
-  const int wgs = tasks < dev.compute_units ? tasks : dev.compute_units;
-  return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, &c, wgs, stream));
+    return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, stream));
+  a.pull.active = 1;
+  a.pull.cus = dev.compute_units;
+  a.pull.rows = c.M;
+  a.pull.pitch = (uint32_t)c.ld_out_bytes;
+  a.pull.upr = (uint32_t)((int64_t)c.N * c.esize / 16);
+  a.pull.block_bytes = c.M * c.ld_out_bytes;
+  a.pull.out = c.out;
+  a.pull.words = variant == TCCL_S1_TILE ? c.locks : c.counter;
+  a.pull.row_starts = c.row_starts;
+  a.pull.row_ends = c.row_ends;
+  a.pull.tile_counts = c.tile_counts;
+  a.pull.n_groups = c.n_groups;
+  a.pull.word_stride = c.word_stride;
+  a.pull.fault = c.fault;
+  a.pull.spin_ticks = c.spin_ticks;
+  return stream_status(tccl::launch_stream(d->in_dtype, kmajor, shape, a, stream));
 }
 
 // GEMM (+ optional communication role) for one of the three operations.
@@ -1445,7 +1451,7 @@ int tccl_gemm(const tccl_gemm_desc* d, void* stream) {
   if (shape >= 0) {
     tccl::StreamArgs a;
     build_stream(d, g, seg, dev, &a);
-    return stream_status(tccl::launch_stream(d->in_dtype, g.b_kmajor != 0, shape, a, nullptr, 0, (hipStream_t)stream));
+    return stream_status(tccl::launch_stream(d->in_dtype, g.b_kmajor != 0, shape, a, (hipStream_t)stream));
   }
   tccl::SignalArgs s;
   memset(&s, 0, sizeof s);
@@ -1993,7 +1999,7 @@ static int reduce_ragged_shards(const tccl_gemm_desc* d, void* out, int32_t out_
     tccl::StreamArgs a;
     build_stream(d, g, g.wrap_rows, dev, &a);
     add_stream_reduce(c, d, &a);
-    return stream_status(tccl::launch_stream(d->in_dtype, g.b_kmajor != 0, shape, a, nullptr, 0, stream));
+    return stream_status(tccl::launch_stream(d->in_dtype, g.b_kmajor != 0, shape, a, stream));
   }
   // All column blocks in one launch, each with tile rows of its own, or, where they are large enough to fill the device,
   // one GEMM per block (four blocks of 1956 x 696 x 2096: 42 us with the sums, 119 us one after the other); then the

@@ -200,6 +200,20 @@ template <>
 TCCL_D float to_out<float>(float v) { return v; }
 
 #if defined(__HIP_DEVICE_COMPILE__)
+// Request every 64-byte line of the kernel arguments at once.  The compiler reads arguments
+// where it first needs them, each group of reads followed by its own wait, so a kernel's
+// start used to be a chain of a dozen dependent trips to memory before the first operand load
+// could go out; after this the later reads hit in the scalar cache.
+template <int kBytes>
+TCCL_D void warm_kernargs() {
+  typedef const __attribute__((address_space(4))) uint32_t* Words;
+  Words p = (Words)__builtin_amdgcn_kernarg_segment_ptr();
+  uint32_t any = 0;
+#pragma unroll
+  for (int o = 0; o < kBytes; o += 64) any |= p[o / 4];
+  asm volatile("" ::"s"(any));
+}
+
 template <typename InT, typename OutT, int kStages = 3, int kWaves = 4, int kHalves = 1>
 struct GemmRole {
   static constexpr int kWn = kWaves / 2, kCols = 64 * kWn;      // wavefronts across, columns of a sub-tile

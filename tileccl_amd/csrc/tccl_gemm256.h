@@ -205,20 +205,6 @@ TCCL_D T late_kernarg(int offset) {
   return v;
 }
 
-// Request every 64-byte line of the kernel arguments at once.  The compiler reads arguments
-// where it first needs them, each group of reads followed by its own wait, so a kernel's
-// start used to be a chain of a dozen dependent trips to memory before the first operand load
-// could go out; after this the later reads hit in the scalar cache.
-template <int kBytes>
-TCCL_D void warm_kernargs() {
-  typedef const __attribute__((address_space(4))) uint32_t* Words;
-  Words p = (Words)__builtin_amdgcn_kernarg_segment_ptr();
-  uint32_t any = 0;
-#pragma unroll
-  for (int o = 0; o < kBytes; o += 64) any |= p[o / 4];
-  asm volatile("" ::"s"(any));
-}
-
 // kBKMajor: B is given with k contiguous (element (k, n) at B[n * ldb + k], what a `.t()` view of
 // an (N, K) weight is: the reference's kernels take any strides, kernels/gemm.py:139-151).  The B
 // stage then has the A stage's layout (256 n rows of 128 bytes, same swizzle) and is read with

@@ -20,6 +20,33 @@
 
 namespace tccl {
 
+// Counters of neighbouring plan tiles in one cache line take each other's time: 256 tiles of one launch counting into 16
+// words of a line or two cost it 2.2 us (512 x 512 x 256, two ranks: 8.3 -> 6.0 us; 16 x 2048 x 4096 9.2 -> 8.5).
+constexpr int kArrivalStride = 32;
+
+// The pull half of an all-gather: this rank's copy of every peer's row block.  Where the tiles leave CUs idle, workgroups
+// behind theirs (`first` on) share it out and run beside them.  Otherwise (a tile's LDS fills most of a CU: such
+// workgroups would start when the tiles end) every workgroup takes a share: it looks at the words that the share depends
+// on when it starts; if the peers are ready the share is requested with its tile's stores, ahead of the wait that
+// those need anyway, and if not it waits (bounded) behind its own signal.
+struct StreamPull {
+  int active;
+  int cus;              // of the device
+  int first;            // the first workgroup that pulls
+  int rows;             // of a block
+  uint32_t upr, pitch;  // 16-byte units and bytes per row
+  int64_t block_bytes;  // from one block to the next
+  char* out;            // block 0 of the gathered output in this rank's slice
+  const int32_t* words;  // this rank's TileGroup counters or locks; a peer's: word_stride apart, or (0) at the same slice offset
+  const int32_t* row_starts;
+  const int32_t* row_ends;
+  const int32_t* tile_counts;
+  int n_groups;
+  int64_t word_stride;
+  int64_t* fault;
+  int64_t spin_ticks;
+};
+
 struct StreamArgs {
   const void* A;
   const void* B;
@@ -34,15 +61,17 @@ struct StreamArgs {
   int seg_rows, wrapped;
   int first_seg;                   // segments are visited from this one on, wrapping around
   int tiles_m, tiles_n, segs;      // tiles down and across a segment; segments
-  int xcds, per_xcd;               // XCD x works on tiles [x per_xcd, (x + 1) per_xcd) of a segment: neighbours share a slab of B in its L2
+  uint32_t tiles_m_magic;          // 2^32 / tiles_m, rounded up: n / tiles_m is mulhi(n, magic) for the tile numbers there are
+  int xcd_shift, per_xcd;          // of 2^xcd_shift XCDs, XCD x works on tiles [x per_xcd, (x + 1) per_xcd) of a segment: neighbours share a slab of B in its L2
   // Signals: a plan tile is published when the last of its tiles has been stored.
   SignalArgs s;
-  uint32_t* arrivals;              // one per plan tile, zero between launches
+  uint32_t* arrivals;              // one per plan tile, kArrivalStride words apart, zero between launches
   int block_m, block_n, group_m, plan_rows, plan_cols;
   const int64_t* heap_bases;
   int rank, world;
   PushArgs push;
   EpilogueReduce reduce;
+  StreamPull pull;
 };
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -62,6 +91,17 @@ struct StreamGemm {
   static constexpr int kPitch = kBN * 4 + 16;         // bytes of a row of sums
   static constexpr int kRowsBytes = kBM * kPitch;
   static constexpr int kLdsBytes = kWaves * kWaveBytes > kRowsBytes ? kWaves * kWaveBytes : kRowsBytes;
+
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  // What a tile's end needs from memory and the divisions that its signal takes: done while the first operands are on
+  // their way.  Behind the tile's stores, where they are used, they were a chain of trips to memory and of scalar
+  // instructions with nothing to overlap them (176 x 1440 x 336, pushed to three peers: 8.5 -> 7.6 us).
+  struct Signal {
+    int tile;        // the plan tile under this tile
+    uint32_t tiles;  // tiles of it
+    int32_t group;   // its TileGroup (group mode)
+    u32x2 base;      // lane p: rank p's heap base
+  };
 
   const StreamArgs& a;
   char* lds;
@@ -215,13 +255,16 @@ struct StreamGemm {
       load<true>(v, kb);
   }
 
-  TCCL_D void k_loop(f32x4 (&acc)[kMB][kNB]) const {
+  // `meanwhile` runs once the first blocks have been requested.
+  template <typename Meanwhile>
+  TCCL_D void k_loop(f32x4 (&acc)[kMB][kNB], Meanwhile meanwhile) const {
     const int blocks = (a.K + kKB - 1) / kKB, whole = a.K / kKB;
     Block v[kDepth];
     // This wavefront's blocks are wave, wave + kWaves, ...; the last one of all may be a partial one.
     int next = wave;
 #pragma unroll
     for (int d = 0; d < kDepth; ++d, next += kWaves) refill(v[d], next, whole, blocks);
+    meanwhile();
     for (int kb = wave; kb < blocks;) {
 #pragma unroll
       for (int d = 0; d < kDepth; ++d) {
@@ -237,14 +280,103 @@ struct StreamGemm {
   }
 
   TCCL_D void run(int slot) {
+    if (!a.pull.active) {
+      tile(slot, nullptr);
+      return;
+    }
+    const bool pulls = slot >= a.pull.first, at_start = a.pull.first == 0 && pull_ready(slot, false);
+    if (tile(slot, a.pull.first == 0 ? &at_start : nullptr)) return;  // its share has gone out with the tile
+    if (pulls && pull_ready(slot, true)) pull_share(slot);
+  }
+
+  // The units of a block that workgroup `slot` pulls.
+  TCCL_D void share(int slot, uint32_t& lo, uint32_t& hi) const {
+    const uint32_t units = (uint32_t)a.pull.rows * a.pull.upr, wgs = gridDim.x - a.pull.first, per = (units + wgs - 1) / wgs;
+    lo = (uint32_t)(slot - a.pull.first) * per;
+    lo = lo < units ? lo : units;
+    hi = units - lo < per ? units : lo + per;
+  }
+  // What the share depends on, for every peer: the TileGroups, or plan tiles, that cover its rows.  `wait`: spin until they
+  // are complete (false: a deadline passed); otherwise this thread's words alone, looked at once.
+  TCCL_D bool pull_ready(int slot, bool wait) const {
+    uint32_t lo, hi;
+    share(slot, lo, hi);
+    if (lo >= hi) return true;
+    const int r0 = (int)(lo / a.pull.upr), r1 = (int)((hi - 1) / a.pull.upr);
+    const int t0 = r0 / a.block_m, tiles = (r1 / a.block_m - t0 + 1) * a.plan_cols;
+    const int per_peer = a.s.mode == kSignalTile ? tiles : a.pull.n_groups;
+    bool ok = true;
+    const int64_t deadline = wait ? now_ticks() + a.pull.spin_ticks : 0;
+    for (int i = (int)threadIdx.x; i < per_peer * (a.world - 1); i += kWaves * 64) {
+      const int q = i / per_peer, k = i - q * per_peer, p = q < a.rank ? q : q + 1;
+      const int32_t* words = a.pull.word_stride ? (const int32_t*)((const char*)a.pull.words + (int64_t)(p - a.rank) * a.pull.word_stride)
+                                                : translate_ptr(a.pull.words, a.rank, p, a.heap_bases);
+      int index = k;
+      int32_t need = a.s.epoch;
+      if (a.s.mode == kSignalTile) {
+        index = tile_id_of(t0 + k / a.plan_cols, k % a.plan_cols, a.plan_rows, a.plan_cols, a.group_m);
+      } else {
+        if (a.pull.row_starts[k] > r1 || a.pull.row_ends[k] <= r0) continue;
+        need = (int32_t)((uint32_t)a.s.epoch * (uint32_t)a.pull.tile_counts[k]);
+      }
+      if (wait) {
+        ok = ok && tile_wait_ge<true>(words, index, need, deadline);
+      } else {
+        ok = ok && word_reached(__hip_atomic_load(&words[index], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), need);
+      }
+    }
+    if (!wait) return ok;
+    if (!ok && a.pull.fault) *a.pull.fault = 1;
+    return __syncthreads_and(ok);
+  }
+  TCCL_D void pull_share(int slot) const {
+    uint32_t lo, hi;
+    share(slot, lo, hi);
+    const int64_t mine = a.heap_bases[a.rank];
+    // Several peers' units are requested before any is stored: a wait for a load is also one for every store before it.
+    constexpr int kPeers = 4, kBatch = 2;
+    for (int q0 = 0; q0 < a.world - 1; q0 += kPeers) {
+      for (uint32_t u0 = lo + threadIdx.x; u0 < hi; u0 += kBatch * kWaves * 64) {
+        u32x4 v[kPeers][kBatch];
+        uint32_t off[kBatch];
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+          const uint32_t u = u0 + (uint32_t)(b * kWaves * 64), row = u / a.pull.upr;
+          off[b] = row * a.pull.pitch + (u - row * a.pull.upr) * 16u;
+        }
+#pragma unroll
+        for (int i = 0; i < kPeers; ++i) {
+          const int q = q0 + i, p = q < a.rank ? q : q + 1;
+          if (q >= a.world - 1) break;
+          const __amdgpu_buffer_rsrc_t from = window((int64_t)(uintptr_t)a.pull.out + p * a.pull.block_bytes + (a.heap_bases[p] - mine));
+#pragma unroll
+          for (int b = 0; b < kBatch; ++b)
+            if (u0 + (uint32_t)(b * kWaves * 64) < hi) v[i][b] = ld16<kCoherent>(from, off[b]);
+        }
+#pragma unroll
+        for (int i = 0; i < kPeers; ++i) {
+          const int q = q0 + i, p = q < a.rank ? q : q + 1;
+          if (q >= a.world - 1) break;
+          const __amdgpu_buffer_rsrc_t to = window((int64_t)(uintptr_t)a.pull.out + p * a.pull.block_bytes);
+#pragma unroll
+          for (int b = 0; b < kBatch; ++b)
+            if (u0 + (uint32_t)(b * kWaves * 64) < hi) st16<kStreaming>(to, off[b], v[i][b]);
+        }
+      }
+    }
+  }
+
+  // One tile.  `ready`: the launch pulls, and this thread's words were complete at the start; true if the share
+  // has been pulled here.
+  TCCL_D bool tile(int slot, const bool* ready) {
     // Every segment is spread over all XCDs (an XCD's link to memory would otherwise carry one owner's reductions alone).
     // Within an XCD's part row tiles run fastest: those that share a column slab of B.
-    const int per_seg = a.tiles_m * a.tiles_n, slots_per_seg = a.xcds * a.per_xcd;
-    int seg = slot / slots_per_seg;
+    const int per_seg = a.tiles_m * a.tiles_n, slots_per_seg = a.per_xcd << a.xcd_shift;
+    int seg = a.segs > 1 ? slot / slots_per_seg : 0;
     const int at = slot - seg * slots_per_seg;
-    const int in = at % a.xcds * a.per_xcd + at / a.xcds;
-    if (in >= per_seg) return;
-    const int tn = in / a.tiles_m, tm = in - tn * a.tiles_m;
+    const int in = (at & ((1 << a.xcd_shift) - 1)) * a.per_xcd + (at >> a.xcd_shift);
+    if (in >= per_seg || at >= slots_per_seg) return false;
+    const int tn = a.tiles_m > 1 ? (int)__umulhi((uint32_t)in, a.tiles_m_magic) : in, tm = in - tn * a.tiles_m;
     seg += a.first_seg;
     if (seg >= a.segs) seg -= a.segs;
     const int row_in = tm * kBM, col0 = tn * kBN;  // relative to the segment
@@ -276,7 +408,8 @@ struct StreamGemm {
     for (int i = 0; i < kMB; ++i)
 #pragma unroll
       for (int j = 0; j < kNB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    k_loop(acc);
+    Signal signal;
+    k_loop(acc, [&] { signal = look_up(row0, col0); });
 
     // The wavefronts' accumulators are added up through LDS ([slot][lane] of each, conflict-free) and the sums
     // staged as rows, from which every thread takes chunks of 8 columns.
@@ -327,9 +460,12 @@ struct StreamGemm {
         f[e] = lo[e];
         f[4 + e] = hi[e];
       }
-      finish(f, owner, row_in, row0, col0, row, col, coherent, ok);
+      finish(f, signal, owner, row_in, row0, col0, row, col, coherent, ok);
     }
-    publish(row0, col0);
+    const bool pulled = ready && __syncthreads_and(*ready);
+    if (pulled) pull_share(slot);
+    publish(signal);
+    return pulled;
   }
 
   TCCL_D static void put(__amdgpu_buffer_rsrc_t w, uint32_t off, const float (&f)[8], int dtype, bool coherent) {
@@ -359,7 +495,7 @@ struct StreamGemm {
   }
 
   // One chunk of 8 columns: to C, to the peers, or into the reduction.
-  TCCL_D void finish(float (&f)[8], int owner, int row_in, int row0, int col0, int row, int col, bool coherent, bool ok) const {
+  TCCL_D void finish(float (&f)[8], const Signal& signal, int owner, int row_in, int row0, int col0, int row, int col, bool coherent, bool ok) const {
     const int esz = a.out_dtype == kF32 ? 4 : 2;
     const int64_t c_at = (int64_t)(uintptr_t)a.C + ((int64_t)row0 * a.ldc + col0) * esz;
     const uint32_t off = (uint32_t)((row * a.ldc + col) * esz);
@@ -369,7 +505,7 @@ struct StreamGemm {
     for (int t = 0; t < a.push.world; ++t) {
       const int c = col0 + col;
       if (t == a.push.rank || c < a.push.col_lo || c >= a.push.col_hi) continue;
-      const int64_t to = (int64_t)(uintptr_t)a.C + (a.heap_bases[t] - a.heap_bases[a.push.rank]) +
+      const int64_t to = (int64_t)(uintptr_t)a.C + (base_of(signal, t) - base_of(signal, a.push.rank)) +
                          ((int64_t)row0 * a.push.ld + col0 + a.push.col_shift) * esz;
       put(window(to), (uint32_t)((row * a.push.ld + col) * esz), f, a.out_dtype, true);
     }
@@ -432,25 +568,42 @@ struct StreamGemm {
     return verdict != 0;
   }
 
-  TCCL_D void publish(int row0, int col0) const {
+  TCCL_D Signal look_up(int row0, int col0) const {
+    Signal s;
+    s.tile = 0;
+    s.tiles = 1;
+    s.group = 0;
+    s.base = u32x2{0, 0};
+    if (a.push.world > 0) s.base = __builtin_amdgcn_raw_buffer_load_b64(window((int64_t)(uintptr_t)a.heap_bases), 8u * (uint32_t)(lane < a.push.world ? lane : 0), 0, 0);
+    if (a.s.mode == kSignalNone) return s;
+    s.tile = plan_tile(row0, col0);
+    if (a.s.mode == kSignalGroup) s.group = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(window((int64_t)(uintptr_t)a.s.group_table), 4u * (uint32_t)s.tile, 0, 0);
+    // Tiles of this plan tile: those of its rows and columns that lie inside the segment and N.
+    const int pr = row0 / a.block_m * a.block_m, pc = col0 / a.block_n * a.block_n;
+    const int seg0 = a.segs > 1 ? row0 / a.seg_rows * a.seg_rows : 0;
+    const int rows = (pr + a.block_m < seg0 + a.seg_rows ? pr + a.block_m : seg0 + a.seg_rows) - pr;
+    const int cols = (pc + a.block_n < a.N ? pc + a.block_n : a.N) - pc;
+    s.tiles = (uint32_t)(((rows + kBM - 1) / kBM) * ((cols + kBN - 1) / kBN));
+    return s;
+  }
+  static TCCL_D int64_t base_of(const Signal& s, int p) {
+    const uint32_t lo = __builtin_amdgcn_readlane(s.base[0], p), hi = __builtin_amdgcn_readlane(s.base[1], p);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+  }
+
+  TCCL_D void publish(const Signal& signal) const {
     if (a.s.mode == kSignalNone) return;
     wait_vmem();  // this wavefront's write-through stores have landed
     __syncthreads();
     if (threadIdx.x != 0) return;
-    const int tile = plan_tile(row0, col0);
-    // Tiles of this plan tile: those of its rows and columns that lie inside the segment and N.
-    const int pr = row0 / a.block_m * a.block_m, pc = col0 / a.block_n * a.block_n;
-    const int seg0 = row0 / a.seg_rows * a.seg_rows;
-    const int rows = (pr + a.block_m < seg0 + a.seg_rows ? pr + a.block_m : seg0 + a.seg_rows) - pr;
-    const int cols = (pc + a.block_n < a.N ? pc + a.block_n : a.N) - pc;
-    const uint32_t n = (uint32_t)(((rows + kBM - 1) / kBM) * ((cols + kBN - 1) / kBN));
+    const uint32_t n = signal.tiles;
     // Counts to n - 1 and starts over by itself, so the word is zero again when the launch has ended.
-    const uint32_t before = n > 1 ? atomicInc(&a.arrivals[tile], n - 1) : 0u;
+    const uint32_t before = n > 1 ? atomicInc(&a.arrivals[kArrivalStride * signal.tile], n - 1) : 0u;
     if (before != n - 1) return;
     if (a.s.mode == kSignalTile)
-      tile_publish(a.s.locks, tile, a.s.epoch);
+      tile_publish(a.s.locks, signal.tile, a.s.epoch);
     else
-      tile_signal_add<true>(a.s.counter, a.s.group_table[tile], 1);
+      tile_signal_add<true>(a.s.counter, signal.group, 1);
   }
 };
 #endif  // __HIP_DEVICE_COMPILE__
@@ -462,8 +615,7 @@ struct StreamShape {
 constexpr StreamShape kStreamShapes[] = {{1, 1, 16}, {1, 2, 16}, {2, 2, 16}, {2, 4, 8}, {4, 4, 4}};
 constexpr int kStreamShapeCount = (int)(sizeof(kStreamShapes) / sizeof(kStreamShapes[0]));
 
-// Defined in tccl_stream.hip.  Fills in the tile counts and launches; `comm` non-NULL: `comm_wgs` workgroups
-// after the tiles' run the communication role with it (the pulls of an all-gather).  0 or a hipError_t.
-int launch_stream(int in_dtype, bool b_kmajor, int shape, StreamArgs& a, const CommArgs* comm, int comm_wgs, hipStream_t stream);
+// Defined in tccl_stream.hip.  Fills in the tile counts and launches.  0 or a hipError_t.
+int launch_stream(int in_dtype, bool b_kmajor, int shape, StreamArgs& a, hipStream_t stream);
 
 }  // namespace tccl

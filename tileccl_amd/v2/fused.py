@@ -110,6 +110,7 @@ class _FusedBase:
             host_plan=self.plan,
             spin_limit_ns=self.spin_limit_ns,
         )
+        self.words.tile_arrivals()
         if self.trace:
             self.words.trace_comm_counter = self.signals.trace_comm_counter
             self.words.trace_start_clock = self.signals.trace_start_clock
