@@ -210,6 +210,11 @@ int tccl_tile_coords(int32_t tile_id, int32_t tile_rows, int32_t tile_cols, int3
 /* Pure host helper: launch slot -> swizzled tile id after the XCD-aware remap (each XCD
  * takes `span` consecutive ids out of every block of xcds*span). */
 int tccl_tile_for_slot(int32_t slot, int32_t total_tiles, int32_t xcds, int32_t span, int32_t* tile_id);
+/* Pure host helper: how a launch of `tiles` small tiles is made up (launches with TCCL_GEMM_ARRIVALS).  Workgroups
+ * [0, *first_pull) hold a tile and never wait for another rank; [*first_pull, *workgroups) carry its pulls, if it has any
+ * (`pulls`), and are the only ones that wait. */
+int tccl_stream_grid(int32_t tiles, int32_t pulls, int32_t compute_units, int32_t world_size, int32_t* first_pull,
+                     int32_t* workgroups);
 
 /* ---- symmetric heap: one hipMalloc arena cut into world_size slices -------------------
  * Replaces one torch.empty per rank + IPC/peer mapping (tileccl_v2/heap.py:137,225-264;

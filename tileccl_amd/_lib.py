@@ -155,6 +155,7 @@ SIGNATURES = {
     "tccl_device_query": (C.c_int, [C.c_int, _P(DeviceInfo)]),
     "tccl_tile_coords": (C.c_int, [_i32, _i32, _i32, _i32, _P(_i32), _P(_i32)]),
     "tccl_tile_for_slot": (C.c_int, [_i32, _i32, _i32, _i32, _P(_i32)]),
+    "tccl_stream_grid": (C.c_int, [_i32, _i32, _i32, _i32, _P(_i32), _P(_i32)]),
     "tccl_heap_create": (C.c_int, [C.c_size_t, C.c_int, _P(_vp), _P(_i64)]),
     "tccl_heap_destroy": (C.c_int, [_vp]),
     "tccl_fill_i32": (C.c_int, [_vp, _i64, _i32, _vp]),

@@ -1339,6 +1339,15 @@ int tccl_tile_for_slot(int32_t slot, int32_t total_tiles, int32_t xcds, int32_t 
   return 0;
 }
 
+int tccl_stream_grid(int32_t tiles, int32_t pulls, int32_t compute_units, int32_t world_size, int32_t* first_pull, int32_t* workgroups) {
+  if (tiles <= 0 || compute_units <= 0 || world_size < 1 || world_size > TCCL_MAX_WORLD || !first_pull || !workgroups)
+    return fail(TCCL_ERR_INVALID, "stream_grid: bad arguments");
+  const tccl::StreamGrid g = tccl::stream_grid(tiles, pulls != 0, compute_units, world_size);
+  *first_pull = g.first;
+  *workgroups = g.wgs;
+  return 0;
+}
+
 int tccl_heap_create(size_t slice_bytes, int world_size, void** arena_out, int64_t* bases_out) {
   if (!arena_out || !bases_out) return fail(TCCL_ERR_INVALID, "heap_create: NULL output");
   if (slice_bytes == 0) return fail(TCCL_ERR_INVALID, "heap_create: slice size must be positive");

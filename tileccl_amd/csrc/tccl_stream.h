@@ -24,15 +24,12 @@ namespace tccl {
 // words of a line or two cost it 2.2 us (512 x 512 x 256, two ranks: 8.3 -> 6.0 us; 16 x 2048 x 4096 9.2 -> 8.5).
 constexpr int kArrivalStride = 32;
 
-// The pull half of an all-gather: this rank's copy of every peer's row block.  Where the tiles leave CUs idle, workgroups
-// behind theirs (`first` on) share it out and run beside them.  Otherwise (a tile's LDS fills most of a CU: such
-// workgroups would start when the tiles end) every workgroup takes a share: it looks at the words that the share depends
-// on when it starts; if the peers are ready the share is requested with its tile's stores, ahead of the wait that
-// those need anyway, and if not it waits (bounded) behind its own signal.
+// The pull half of an all-gather: this rank's copy of every peer's row block.  Workgroups behind those of the tiles share it
+// out and wait (bounded) for the peers; a workgroup with a tile never waits (stream_grid()).
 struct StreamPull {
   int active;
   int cus;              // of the device
-  int first;            // the first workgroup that pulls
+  int first;            // the first workgroup that pulls: all tiles are below it
   int rows;             // of a block
   uint32_t upr, pitch;  // 16-byte units and bytes per row
   int64_t block_bytes;  // from one block to the next
@@ -280,13 +277,10 @@ struct StreamGemm {
   }
 
   TCCL_D void run(int slot) {
-    if (!a.pull.active) {
-      tile(slot, nullptr);
-      return;
-    }
-    const bool pulls = slot >= a.pull.first, at_start = a.pull.first == 0 && pull_ready(slot, false);
-    if (tile(slot, a.pull.first == 0 ? &at_start : nullptr)) return;  // its share has gone out with the tile
-    if (pulls && pull_ready(slot, true)) pull_share(slot);
+    if (!a.pull.active || slot < a.pull.first)
+      tile(slot);
+    else if (pull_ready(slot))
+      pull_share(slot);
   }
 
   // The units of a block that workgroup `slot` pulls.
@@ -296,9 +290,9 @@ struct StreamGemm {
     lo = lo < units ? lo : units;
     hi = units - lo < per ? units : lo + per;
   }
-  // What the share depends on, for every peer: the TileGroups, or plan tiles, that cover its rows.  `wait`: spin until they
-  // are complete (false: a deadline passed); otherwise this thread's words alone, looked at once.
-  TCCL_D bool pull_ready(int slot, bool wait) const {
+  // What the share depends on, for every peer: the TileGroups, or plan tiles, that cover its rows.  Spins until they are
+  // complete; false: a deadline passed.
+  TCCL_D bool pull_ready(int slot) const {
     uint32_t lo, hi;
     share(slot, lo, hi);
     if (lo >= hi) return true;
@@ -306,7 +300,7 @@ struct StreamGemm {
     const int t0 = r0 / a.block_m, tiles = (r1 / a.block_m - t0 + 1) * a.plan_cols;
     const int per_peer = a.s.mode == kSignalTile ? tiles : a.pull.n_groups;
     bool ok = true;
-    const int64_t deadline = wait ? now_ticks() + a.pull.spin_ticks : 0;
+    const int64_t deadline = now_ticks() + a.pull.spin_ticks;
     for (int i = (int)threadIdx.x; i < per_peer * (a.world - 1); i += kWaves * 64) {
       const int q = i / per_peer, k = i - q * per_peer, p = q < a.rank ? q : q + 1;
       const int32_t* words = a.pull.word_stride ? (const int32_t*)((const char*)a.pull.words + (int64_t)(p - a.rank) * a.pull.word_stride)
@@ -319,13 +313,8 @@ struct StreamGemm {
         if (a.pull.row_starts[k] > r1 || a.pull.row_ends[k] <= r0) continue;
         need = (int32_t)((uint32_t)a.s.epoch * (uint32_t)a.pull.tile_counts[k]);
       }
-      if (wait) {
-        ok = ok && tile_wait_ge<true>(words, index, need, deadline);
-      } else {
-        ok = ok && word_reached(__hip_atomic_load(&words[index], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), need);
-      }
+      ok = ok && tile_wait_ge<true>(words, index, need, deadline);
     }
-    if (!wait) return ok;
     if (!ok && a.pull.fault) *a.pull.fault = 1;
     return __syncthreads_and(ok);
   }
@@ -334,7 +323,7 @@ struct StreamGemm {
     share(slot, lo, hi);
     const int64_t mine = a.heap_bases[a.rank];
     // Several peers' units are requested before any is stored: a wait for a load is also one for every store before it.
-    constexpr int kPeers = 4, kBatch = 2;
+    constexpr int kPeers = 4, kBatch = 4;
     for (int q0 = 0; q0 < a.world - 1; q0 += kPeers) {
       for (uint32_t u0 = lo + threadIdx.x; u0 < hi; u0 += kBatch * kWaves * 64) {
         u32x4 v[kPeers][kBatch];
@@ -366,16 +355,14 @@ struct StreamGemm {
     }
   }
 
-  // One tile.  `ready`: the launch pulls, and this thread's words were complete at the start; true if the share
-  // has been pulled here.
-  TCCL_D bool tile(int slot, const bool* ready) {
+  TCCL_D void tile(int slot) {
     // Every segment is spread over all XCDs (an XCD's link to memory would otherwise carry one owner's reductions alone).
     // Within an XCD's part row tiles run fastest: those that share a column slab of B.
     const int per_seg = a.tiles_m * a.tiles_n, slots_per_seg = a.per_xcd << a.xcd_shift;
     int seg = a.segs > 1 ? slot / slots_per_seg : 0;
     const int at = slot - seg * slots_per_seg;
     const int in = (at & ((1 << a.xcd_shift) - 1)) * a.per_xcd + (at >> a.xcd_shift);
-    if (in >= per_seg || at >= slots_per_seg) return false;
+    if (in >= per_seg || at >= slots_per_seg) return;
     const int tn = a.tiles_m > 1 ? (int)__umulhi((uint32_t)in, a.tiles_m_magic) : in, tm = in - tn * a.tiles_m;
     seg += a.first_seg;
     if (seg >= a.segs) seg -= a.segs;
@@ -462,10 +449,7 @@ struct StreamGemm {
       }
       finish(f, signal, owner, row_in, row0, col0, row, col, coherent, ok);
     }
-    const bool pulled = ready && __syncthreads_and(*ready);
-    if (pulled) pull_share(slot);
     publish(signal);
-    return pulled;
   }
 
   TCCL_D static void put(__amdgpu_buffer_rsrc_t w, uint32_t off, const float (&f)[8], int dtype, bool coherent) {
@@ -614,6 +598,30 @@ struct StreamShape {
 };
 constexpr StreamShape kStreamShapes[] = {{1, 1, 16}, {1, 2, 16}, {2, 2, 16}, {2, 4, 8}, {4, 4, 4}};
 constexpr int kStreamShapeCount = (int)(sizeof(kStreamShapes) / sizeof(kStreamShapes[0]));
+
+// The workgroups of a launch: `first` for tiles, the rest pull.  Two rules keep every wait finite:
+// - In an all-gather only pulling workgroups wait for another rank, and they are numbered, hence started, behind every tile:
+//   what a peer waits for never needs a place that one of them holds, however many tiles there are (e4m3: more than are
+//   resident).  (In a reduce-scatter the tiles of the own rows wait, the last ones: run_variant().)
+// - They are few enough that ranks which share a device find CUs for their tiles, the others' waiting workgroups
+//   notwithstanding (a workgroup takes 64 to 128 KiB of LDS, i.e. a CU): a 1/world of the CUs, or a quarter from four
+//   ranks on, since no more of one process's launches run at a time (HIP's four hardware queues).
+// Where an eighth of the CUs has no tile, they run beside the tiles and are no more than those CUs.
+// Measured against shares that every tile's workgroup pulled, and waited for, behind its own tile (peers complete): fp16, two ranks,
+// 176 x 1440 x 336 6.9 us both ways, 1000 x 1000 x 512 11.9 -> 9.8, 1024 x 1024 x 1024 13.3 -> 11.3 (eight ranks 19.8 -> 17.8),
+// e4m3 1536 x 2048 x 1024 24.6 -> 19.5; slower where 256 tiles of 32 x 32 leave the pulls for a second wave of workgroups:
+// 512 x 512 x 256 8.2 -> 8.4, four ranks 8.9 -> 9.5, eight 10.6 -> 11.9.
+constexpr int kLiveRanks = 4;
+struct StreamGrid {
+  int first, wgs;
+};
+inline StreamGrid stream_grid(int tiles, bool pulls, int cus, int world) {
+  if (!pulls) return {tiles, tiles};
+  const int ranks = world < kLiveRanks ? world : kLiveRanks;
+  int pullers = cus / ranks > 0 ? cus / ranks : 1;
+  if (cus - tiles >= cus / 8 && cus - tiles < pullers) pullers = cus - tiles;
+  return {tiles, tiles + pullers};
+}
 
 // Defined in tccl_stream.hip.  Fills in the tile counts and launches.  0 or a hipError_t.
 int launch_stream(int in_dtype, bool b_kmajor, int shape, StreamArgs& a, hipStream_t stream);

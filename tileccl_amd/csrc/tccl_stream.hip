@@ -26,15 +26,9 @@ int launch_t(StreamArgs& a, hipStream_t stream) {
   a.tiles_m_magic = 0xffffffffu / (uint32_t)a.tiles_m + 1u;
   const int xcds = 1 << a.xcd_shift;
   a.per_xcd = (a.tiles_m * a.tiles_n + xcds - 1) / xcds;
-  int wgs = a.segs * xcds * a.per_xcd;
-  // An eighth of the CUs idle: they pull beside the tiles.  176 x 1440 x 336, four ranks, 144 tiles: 7.8 us, 10.4 us with the pulls in
-  // every workgroup (13.0 in communication workgroups); 143 x 1336 x 352, 216 tiles: 7.9 and 9.4 (15.0).
-  a.pull.first = 0;
-  if (a.pull.active && a.pull.cus - wgs >= a.pull.cus / 8) {
-    a.pull.first = wgs;
-    wgs = a.pull.cus;
-  }
-  hipLaunchKernelGGL((stream_kernel<InT, s.mb, s.nb, s.waves, kBKMajor>), dim3(wgs), dim3(s.waves * 64), 0, stream, a);
+  const StreamGrid grid = stream_grid(a.segs * xcds * a.per_xcd, a.pull.active != 0, a.pull.cus, a.world);
+  a.pull.first = grid.first;
+  hipLaunchKernelGGL((stream_kernel<InT, s.mb, s.nb, s.waves, kBKMajor>), dim3(grid.wgs), dim3(s.waves * 64), 0, stream, a);
   return (int)hipGetLastError();
 }
 
