@@ -130,3 +130,49 @@ def test_descriptors_and_launch_numbers(table, variant, attr):
     setattr(words, attr, 3)
     capturing.append(1)
     assert numbers() == 40 and words.asked == 2
+
+
+@pytest.mark.parametrize("kind", ["sparse", "nested", "jagged", "vmap", "grad", "meta"])
+def test_tensors_without_an_address_find_no_call(table, kind):
+    """They throw when asked for one; that is "no call", and an ordinary error where a call is built for them."""
+    table, _ = table
+    a = torch.zeros(8, 8)
+    seen, keep = bound(table, ("op",), (a, a), heap=Heap(a, 256))
+
+    def asks(t):
+        assert table.launch(("op",), None, a, t) is None
+        assert table.launch(("op",), None, t, a) is None
+        if kind != "meta":  # (whose address is zero)
+            with pytest.raises(RuntimeError):
+                bound(table, ("op",), (t, a))
+        return t.sum() if kind in ("vmap", "grad") else None
+
+    if kind == "sparse":
+        asks(a.to_sparse())
+    elif kind == "nested":
+        asks(torch.nested.nested_tensor([a, a[:3]], layout=torch.strided))
+    elif kind == "jagged":
+        assert table.launch(("op",), None, a, torch.nested.nested_tensor([a, a[:3]], layout=torch.jagged)) is None
+    elif kind == "vmap":
+        torch.vmap(asks)(torch.zeros(3, 8, 8))
+    elif kind == "grad":
+        torch.func.grad(asks)(a)
+    else:
+        asks(torch.empty(8, 8, device="meta"))
+    assert seen == [] and table.launch(("op",), None, a, a) is True
+
+
+def test_operands_packed_into_something_without_an_address(table):
+    table, _ = table
+    a = torch.zeros(8, 8)
+    host = _lib.host()
+
+    @ENTRY
+    def entry(*_):
+        raise AssertionError("not reached")
+
+    for packed in (a.to_sparse(), None):
+        t = host.Table()
+        t.add(host.Call(C.cast(entry, C.c_void_p).value, "entry", ((0, 0), 1, (1, 0)), (a, a), ("op",), prepare=lambda *_: (packed, a)))
+        with pytest.raises((RuntimeError, TypeError)):
+            t.launch(("op",), None, a, a)

@@ -18,6 +18,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <vector>
 
 #include "../../include/tileccl_hip.h"
@@ -102,6 +103,26 @@ void call_dealloc(Call* self) {
   Py_TYPE(self)->tp_free((PyObject*)self);
 }
 
+// Tensors without memory of their own (sparse, nested, inside torch.vmap or torch.func.grad) throw when asked for an
+// address or strides, and the interpreter's frames above an entry of this module are no place for a C++ exception: every
+// entry that looks at tensors or allocates goes through here.
+template <typename Result, typename Body>
+Result guarded(Result failed, Body body) {
+  try {
+    return body();
+  } catch (const std::exception& e) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (...) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "unknown C++ exception");
+  }
+  return failed;
+}
+
+struct Reference {  // given up at the end of its scope
+  PyObject* object = nullptr;
+  ~Reference() { Py_XDECREF(object); }
+};
+
 PyObject* own(PyObject* o) {
   if (o == Py_None) return nullptr;
   Py_XINCREF(o);
@@ -109,7 +130,7 @@ PyObject* own(PyObject* o) {
 }
 
 // Call(entry, what, args, tensors, key, *, tag, gemm, c, sync, words, variant, on_heap, heap, bases, prepare, keep)
-int call_init(Call* self, PyObject* pos, PyObject* kw) {
+int call_init_checked(Call* self, PyObject* pos, PyObject* kw) {
   static const char* names[] = {"entry", "what", "args", "tensors", "key", "tag", "gemm", "c", "sync", "words", "variant",
                                 "on_heap", "heap", "bases", "prepare", "keep", nullptr};
   unsigned long long entry = 0, gemm = 0, sync = 0;
@@ -215,6 +236,10 @@ int call_init(Call* self, PyObject* pos, PyObject* kw) {
   return 0;
 }
 
+int call_init(Call* self, PyObject* pos, PyObject* kw) {
+  return guarded(-1, [&] { return call_init_checked(self, pos, kw); });
+}
+
 PyTypeObject CallType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // Same object, or the same plain value.  Anything else (a context, signal words, a contract) counts by identity.
@@ -273,25 +298,22 @@ bool next_number(const Call* c, int32_t& number) {
   return rc == 0;
 }
 
-// Issue the call on these tensors (of the layouts it was built for).  Returns the tag, or null with an exception set.
-PyObject* launch(Call* c, PyObject* const* tensors, PyObject* alpha) {
-  const size_t n = c->layouts->size();
-  int64_t at[kMaxTensors];
-  for (size_t i = 0; i < n; ++i) at[i] = (int64_t)(uintptr_t)THPVariable_Unpack(tensors[i]).data_ptr();
+// Issue the call on these tensors (of the layouts it was built for, at the addresses `at`).  Returns the tag, or null with an
+// exception set.
+PyObject* launch(Call* c, PyObject* const* tensors, int64_t* at, PyObject* alpha) {
   tccl_gemm_desc gemm;
   tccl_sync_desc_arrivals sync;
-  PyObject* prepared = nullptr;  // operands that had to be packed live until the launch is issued
+  Reference prepared;  // operands that had to be packed live until the launch is issued
   if (c->prepare) {
     PyObject* operands[2] = {tensors[0], tensors[1]};
-    prepared = PyObject_Vectorcall(c->prepare, operands, 2, nullptr);
-    if (!prepared) return nullptr;
-    if (!PyTuple_Check(prepared) || PyTuple_GET_SIZE(prepared) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(prepared, 0)) ||
-        !THPVariable_Check(PyTuple_GET_ITEM(prepared, 1))) {
-      Py_DECREF(prepared);
+    PyObject* pair = prepared.object = PyObject_Vectorcall(c->prepare, operands, 2, nullptr);
+    if (!pair) return nullptr;
+    if (!PyTuple_Check(pair) || PyTuple_GET_SIZE(pair) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(pair, 0)) ||
+        !THPVariable_Check(PyTuple_GET_ITEM(pair, 1))) {
       PyErr_SetString(PyExc_TypeError, "prepare must return the two operands");
       return nullptr;
     }
-    for (int i = 0; i < 2; ++i) at[i] = (int64_t)(uintptr_t)THPVariable_Unpack(PyTuple_GET_ITEM(prepared, i)).data_ptr();
+    for (int i = 0; i < 2; ++i) at[i] = (int64_t)(uintptr_t)THPVariable_Unpack(PyTuple_GET_ITEM(pair, i)).data_ptr();
   }
   bool ok = true;
   if (c->has_gemm) {
@@ -323,10 +345,7 @@ PyObject* launch(Call* c, PyObject* const* tensors, PyObject* alpha) {
     Py_XDECREF(s);
     ok = ok && !PyErr_Occurred();
   }
-  if (!ok) {
-    Py_XDECREF(prepared);
-    return nullptr;
-  }
+  if (!ok) return nullptr;
   for (size_t i = 0; i < c->args->size(); ++i) {
     const Arg& a = (*c->args)[i];
     v[i] = a.kind == Arg::kGemmCopy ? (int64_t)(uintptr_t)&gemm : a.kind == Arg::kSyncCopy ? (int64_t)(uintptr_t)&sync
@@ -339,7 +358,6 @@ PyObject* launch(Call* c, PyObject* const* tensors, PyObject* alpha) {
   rc = (int32_t)((int64_t(*)(int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t))c->entry)(
       v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11]);
   Py_END_ALLOW_THREADS;
-  Py_XDECREF(prepared);
   if (rc != 0) {
     PyObject* r = PyObject_CallFunction(report, "iO", (int)rc, c->what ? c->what : Py_None);
     Py_XDECREF(r);
@@ -351,19 +369,32 @@ PyObject* launch(Call* c, PyObject* const* tensors, PyObject* alpha) {
   return tag;
 }
 
-bool fits(const Call* c, PyObject* const* tensors, Py_ssize_t n) {
+// The tensors' addresses; false if one has none, which no call is for.
+bool addresses(PyObject* const* tensors, Py_ssize_t n, int64_t* at) {
+  try {
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      const at::Tensor& t = THPVariable_Unpack(tensors[i]);
+      if (t.layout() != c10::kStrided || t.unsafeGetTensorImpl()->is_nested()) return false;
+      at[i] = (int64_t)(uintptr_t)t.data_ptr();
+    }
+  } catch (...) {
+    return false;
+  }
+  return true;
+}
+
+bool fits(const Call* c, PyObject* const* tensors, const int64_t* at, Py_ssize_t n) {
   if ((Py_ssize_t)c->layouts->size() != n) return false;
   int64_t offset = 0;
   for (Py_ssize_t i = 0; i < n; ++i) {
     const at::Tensor& t = THPVariable_Unpack(tensors[i]);
-    const uintptr_t at = (uintptr_t)t.data_ptr();
-    if (!(*c->layouts)[i].matches(t, at)) return false;
+    if (!(*c->layouts)[i].matches(t, (uintptr_t)at[i])) return false;
     if (c->heap_size && ((c->on_heap >> i) & 1u)) {
-      const int64_t into = (int64_t)at - c->heap_lo;
+      const int64_t into = at[i] - c->heap_lo;
       if (!(into >= 0 && into < c->heap_size) && t.numel() != 0) return false;
     }
     if (!c->bases->empty()) {
-      const int64_t from_base = (int64_t)at - (*c->bases)[i];
+      const int64_t from_base = at[i] - (*c->bases)[i];
       if (i == 0) offset = from_base;
       if (from_base != offset) return false;
     }
@@ -377,9 +408,11 @@ struct Table {
 };
 
 PyObject* table_new(PyTypeObject* type, PyObject*, PyObject*) {
-  Table* t = (Table*)type->tp_alloc(type, 0);
-  if (t) t->calls = new std::vector<Call*>();
-  return (PyObject*)t;
+  return guarded((PyObject*)nullptr, [&] {
+    Table* t = (Table*)type->tp_alloc(type, 0);
+    if (t) t->calls = new std::vector<Call*>();
+    return (PyObject*)t;
+  });
 }
 int table_traverse(Table* self, visitproc visit, void* arg) {
   for (Call* c : *self->calls) Py_VISIT((PyObject*)c);
@@ -403,8 +436,12 @@ PyObject* table_add(Table* self, PyObject* call) {
     PyErr_SetString(PyExc_TypeError, "Table.add expects a Call");
     return nullptr;
   }
+  if (!guarded(false, [&] {
+        self->calls->push_back((Call*)call);
+        return true;
+      }))
+    return nullptr;
   Py_INCREF(call);
-  self->calls->push_back((Call*)call);
   if (self->calls->size() > kMaxCalls) {
     Call* oldest = self->calls->front();
     self->calls->erase(self->calls->begin());
@@ -421,15 +458,18 @@ PyObject* table_launch(Table* self, PyObject* const* args, Py_ssize_t nargs) {
   }
   for (Py_ssize_t i = 2; i < nargs; ++i)
     if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
-  for (size_t i = self->calls->size(); i-- > 0;) {
-    Call* c = (*self->calls)[i];
-    if (!fits(c, args + 2, nargs - 2) || !same_key(c->key, args[0])) continue;
-    Py_INCREF(c);  // another thread may drop it from the table meanwhile
-    PyObject* r = launch(c, args + 2, args[1]);
-    Py_DECREF(c);
-    return r;
-  }
-  Py_RETURN_NONE;
+  int64_t at[kMaxTensors];
+  if (!addresses(args + 2, nargs - 2, at)) Py_RETURN_NONE;
+  return guarded((PyObject*)nullptr, [&]() -> PyObject* {
+    for (size_t i = self->calls->size(); i-- > 0;) {
+      Call* c = (*self->calls)[i];
+      if (!fits(c, args + 2, at, nargs - 2) || !same_key(c->key, args[0])) continue;
+      Reference held{(PyObject*)c};  // another thread may drop it from the table meanwhile
+      Py_INCREF(c);
+      return launch(c, args + 2, at, args[1]);
+    }
+    Py_RETURN_NONE;
+  });
 }
 
 Py_ssize_t table_len(Table* self) { return (Py_ssize_t)self->calls->size(); }
