@@ -156,9 +156,11 @@ typedef struct tccl_sync_desc {
 } tccl_sync_desc;
 
 /* What `sync` points at in a launch whose gemm->flags has TCCL_GEMM_ARRIVALS (pass &x.sync).
- *   arrivals   uint32[TCCL_ARRIVAL_STRIDE * total_tiles] (a counter at the start of each tile's words, which
- *              no other tile's counting then holds up), device memory (in the heap or not), zeroed once by the host and zero
- *              again after every launch.
+ *   arrivals   uint32[TCCL_ARRIVAL_STRIDE * total_tiles] (each tile's words are a cache line of their own, which no
+ *              other tile's counting holds up), device memory (in the heap or not), all zeroed once by the host and zero
+ *              again after every launch.  A launch counts in the word of its `epoch` modulo TCCL_ARRIVAL_STRIDE / 2 (S1: of
+ *              the second half), so launches on the same words may overlap (two streams) if those differ; launches of one
+ *              epoch, such as those recorded into a graph, must run one after the other.
  * With them small problems are computed in tiles smaller than a plan tile (up to 5 times as fast at
  * 16 x 2048 x 4096): the last of a plan tile's tiles, found by counting here, publishes it. */
 #define TCCL_ARRIVAL_STRIDE 32

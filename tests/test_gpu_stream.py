@@ -151,3 +151,55 @@ def test_reduce_scatter_columns_of_any_row_count(lib, world, M, N, K, layout):
     finally:
         for c in ctxs:
             c.heap.cleanup()
+
+
+@pytest.mark.parametrize("variant", ["s1", "s2"])
+def test_counts_of_overlapping_launches_stay_apart(lib, variant):
+    """Launches that overlap share the arrival words.  What stands in those that other launches count in (here beyond what any
+    plan tile has: counted into, they would never publish) neither disturbs a launch nor is touched by it."""
+    from tileccl_amd import _lib
+    from tileccl_amd.v2 import FusedGemmAllGather, SymmetricHeap
+
+    M, N, K = 200, 600, 256
+    with SymmetricHeap.create_all(64 << 20, 1)[0] as heap:
+        op = FusedGemmAllGather(heap, M, N, torch.float16, directions="push", tau_min_bytes=1)
+        A, B = into_heap(heap, seeded((M, K), 1)), into_heap(heap, seeded((K, N), 2, scale=K**-0.5))
+        half = _lib.ARRIVAL_STRIDE // 2
+        for launch in range(1, 2 * half + 2):
+            words = op.words.arrivals.view(-1, _lib.ARRIVAL_STRIDE)
+            words.fill_(1 << 30)
+            words[:, launch % half + (half if variant == "s1" else 0)] = 0
+            before = words.clone()
+            op(A, B, variant)
+            op.check_faults()
+            assert torch.equal(words, before)
+            if variant == "s2":
+                assert op.signals.counter.tolist() == [launch * t for t in op.plan.tile_counts()]
+            else:
+                assert op.locks.tolist() == [launch] * op.locks.numel()
+
+
+def test_launches_of_different_tiles_on_two_streams_leave_no_counts(lib):
+    """One context's tile-by-tile calls share their words by the number of plan tiles: 16 here, of 16 tiles each in one
+    call and of 8 in the other."""
+    import tileccl_amd as tileccl
+
+    ctx = tileccl.init_local(world_size=1, heap_size=64 << 20)[0]
+    try:
+        K = 1024
+        calls = []
+        for M, N, stream in ((512, 512, torch.cuda.Stream()), (1, 2048, torch.cuda.Stream())):
+            A, B = seeded((M, K), M), seeded((K, N), N, scale=K**-0.5)
+            calls.append((into_heap(ctx.heap, A), into_heap(ctx.heap, B), ctx.zeros(M, N, dtype=torch.float16), A.float() @ B.float(), stream))
+        torch.cuda.synchronize()
+        for _ in range(30):
+            for A, B, C_out, _, stream in calls:
+                with torch.cuda.stream(stream):
+                    tileccl.ops.gemm_allscatter(A, B, C_out, ctx=ctx, pattern="wg_specialized")
+        torch.cuda.synchronize()
+        for _, _, C_out, want, _ in calls:
+            assert_gemm_close(C_out, want, tight=0.004)
+        words = [w for k, w in ctx._workspace_cache.items() if "locks" in k]
+        assert len(words) == 1 and words[0].lock_epoch == 60 and not words[0].arrivals.any()
+    finally:
+        ctx.heap.cleanup()

@@ -356,7 +356,11 @@ class SyncWords:
     its epoch cannot advance.  A TileGroup launch issued while the stream is capturing is
     therefore preceded by fill kernels that clear the counters (recorded with it; never a
     memset node) and runs as epoch 1; from then on every launch of these words does the
-    same, captured or not, so replays and eager launches can alternate freely.
+    same, captured or not, so replays and eager launches can alternate freely (one after the
+    other: what clears the words for one launch takes them from another that is still running).
+
+    Launches that overlap on two streams count their tiles in arrival words of their own
+    (``ARRIVAL_STRIDE / 2`` launch numbers in turn).
     """
 
     locks: torch.Tensor | None = None
@@ -373,7 +377,7 @@ class SyncWords:
     lock_epoch: int = 0
     spin_limit_ns: int = DEFAULT_SPIN_LIMIT_NS
     max_tasks_per_tile: int = 1 << 16
-    arrivals: torch.Tensor | None = None  # a counter per plan tile, zero between launches (tccl_sync_desc_arrivals)
+    arrivals: torch.Tensor | None = None  # counters, zero between launches (tccl_sync_desc_arrivals)
     arrivals_from_capture: bool = False  # zeroed by a recorded fill only: every launch has to clear them itself
     clear_every_launch: bool = False  # set by the first launch recorded into a graph
 

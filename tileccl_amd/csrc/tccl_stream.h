@@ -23,6 +23,13 @@ namespace tccl {
 // Counters of neighbouring plan tiles in one cache line take each other's time: 256 tiles of one launch counting into 16
 // words of a line or two cost it 2.2 us (512 x 512 x 256, two ranks: 8.3 -> 6.0 us; 16 x 2048 x 4096 9.2 -> 8.5).
 constexpr int kArrivalStride = 32;
+// Of a plan tile's words a launch counts in one that no launch near it in number uses, and neither does the other kind of
+// launch, which is numbered separately: launches of the same words that overlap (two streams), whatever their tile shapes, do not
+// add to each other's counts, so each of them leaves zero behind and publishes a plan tile exactly when it is complete.
+TCCL_HD int arrival_word(int plan_tile, int32_t epoch, bool by_tile) {
+  constexpr int kHalf = kArrivalStride / 2;
+  return kArrivalStride * plan_tile + (int)((uint32_t)epoch % kHalf) + (by_tile ? kHalf : 0);
+}
 
 // The pull half of an all-gather: this rank's copy of every peer's row block.  Workgroups behind those of the tiles share it
 // out and wait (bounded) for the peers; a workgroup with a tile never waits (stream_grid()).
@@ -62,7 +69,7 @@ struct StreamArgs {
   int xcd_shift, per_xcd;          // of 2^xcd_shift XCDs, XCD x works on tiles [x per_xcd, (x + 1) per_xcd) of a segment: neighbours share a slab of B in its L2
   // Signals: a plan tile is published when the last of its tiles has been stored.
   SignalArgs s;
-  uint32_t* arrivals;              // one per plan tile, kArrivalStride words apart, zero between launches
+  uint32_t* arrivals;              // kArrivalStride words per plan tile (arrival_word()), zero between launches
   int block_m, block_n, group_m, plan_rows, plan_cols;
   const int64_t* heap_bases;
   int rank, world;
@@ -582,7 +589,7 @@ struct StreamGemm {
     if (threadIdx.x != 0) return;
     const uint32_t n = signal.tiles;
     // Counts to n - 1 and starts over by itself, so the word is zero again when the launch has ended.
-    const uint32_t before = n > 1 ? atomicInc(&a.arrivals[kArrivalStride * signal.tile], n - 1) : 0u;
+    const uint32_t before = n > 1 ? atomicInc(&a.arrivals[arrival_word(signal.tile, a.s.epoch, a.s.mode == kSignalTile)], n - 1) : 0u;
     if (before != n - 1) return;
     if (a.s.mode == kSignalTile)
       tile_publish(a.s.locks, signal.tile, a.s.epoch);
