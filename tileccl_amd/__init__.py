@@ -130,6 +130,10 @@ class TileCCLContext:
             t.zero_()
         return t
 
+    def kept_workspace(self, name: str, *size: int, dtype: "torch.dtype") -> "torch.Tensor | None":
+        """What ``workspace`` has allocated for these arguments, if it has."""
+        return self._workspace_cache.get((name, _normalize_shape(size), str(dtype)))
+
     # -- pattern choice and support report (reference __init__.py:180-206) ---------------
     def auto_select_pattern(self, op: str, M: int, N: int, K: int, *, hw_info: object | None = None):
         """The pattern ``auto_select`` picks for this problem, bound to this context."""

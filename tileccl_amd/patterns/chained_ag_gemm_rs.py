@@ -29,6 +29,7 @@ import torch
 from tileccl_amd import _launch, _lib
 from tileccl_amd.patterns.hip_patterns import BulkSyncPattern, TileGroupPattern, WGSpecializedPattern
 
+_GATHERED = "chained_ag_gemm_rs.gathered_input"
 _SCHEDULES = {"bulk_sync": BulkSyncPattern, "wg_specialized": WGSpecializedPattern, "tile_group": TileGroupPattern}
 
 
@@ -72,27 +73,25 @@ class ChainedAGGemmRSPattern:
         gathered_workspace: torch.Tensor | None = None,
     ) -> torch.Tensor:
         heap = self.ctx.require_heap()
-        if gathered_workspace is None:
-            gathered_workspace = self.ctx.workspace(
-                "chained_ag_gemm_rs.gathered_input", input_shard.shape[0], W.shape[0], dtype=input_shard.dtype
-            )
+        own = gathered_workspace is None
+        if own and input_shard.ndim == W.ndim == 2:
+            gathered_workspace = self.ctx.kept_workspace(_GATHERED, input_shard.shape[0], W.shape[0], dtype=input_shard.dtype)
         key = (heap.local_base,)
-        ran = self._calls.launch(key, None, gathered_workspace, W, output, input_shard)
+        ran = None
+        if gathered_workspace is not None:
+            ran = self._calls.launch(key, None, gathered_workspace, W, output, input_shard)
         if ran is None:
-            if self.ctx.world_size > 1:
-                for name, t in (("input_shard", input_shard), ("output", output)):
-                    if not heap.owns_tensor(t):
-                        raise ValueError(
-                            f"{name} must live in the symmetric heap when world_size > 1: peers address it "
-                            "at the same offset in their slices"
-                        )
+            # Before anything is allocated for the call (the heap gives nothing back): the ranks' heaps stay in step.
+            self._check(input_shard, W, output, gathered_workspace, heap)
+            if own:
+                gathered_workspace = self.ctx.workspace(_GATHERED, input_shard.shape[0], W.shape[0], dtype=input_shard.dtype)
             self._bind(key, input_shard, W, output, gathered_workspace, heap)
             ran = _launch.issue(self._calls, key, None, gathered_workspace, W, output, input_shard)
         self._last_sync = None if ran is True else ran
         return output
 
-    def _bind(self, key, input_shard, W, output, gathered_workspace, heap) -> None:
-        """Check the shapes and build the descriptors of a call on tensors of these layouts."""
+    def _check(self, input_shard, W, output, gathered_workspace, heap) -> None:
+        """The contract of a call; ``gathered_workspace``: ``None`` if it has yet to be allocated."""
         M, K_shard = input_shard.shape
         K, N = W.shape
         world_size = self.ctx.world_size
@@ -102,8 +101,23 @@ class ChainedAGGemmRSPattern:
             )
         if tuple(output.shape) != (M, N):
             raise ValueError(f"output shape {tuple(output.shape)} must be (M, N) = ({M}, {N})")
-        if tuple(gathered_workspace.shape) != (M, K) or gathered_workspace.dtype != input_shard.dtype:
+        if input_shard.dtype != W.dtype:
+            raise ValueError(f"input_shard and W must share a dtype, got {input_shard.dtype} and {W.dtype}")
+        if world_size > 1:
+            for name, t in (("input_shard", input_shard), ("output", output)):
+                if not heap.owns_tensor(t):
+                    raise ValueError(
+                        f"{name} must live in the symmetric heap when world_size > 1: peers address it "
+                        "at the same offset in their slices"
+                    )
+        if gathered_workspace is not None and (tuple(gathered_workspace.shape) != (M, K) or gathered_workspace.dtype != input_shard.dtype):
             raise ValueError(f"gathered_workspace must be ({M}, {K}) of {input_shard.dtype}")
+
+    def _bind(self, key, input_shard, W, output, gathered_workspace, heap) -> None:
+        """Build the descriptors of a call on tensors of these layouts."""
+        M, K_shard = input_shard.shape
+        N = W.shape[1]
+        world_size = self.ctx.world_size
         compute_wgs, comm_wgs = self._stage._wg_split()
         gemm, plan = _launch._gemm_desc(
             gathered_workspace, W, output, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self._stage.GROUP_M,
