@@ -176,3 +176,35 @@ def test_operands_packed_into_something_without_an_address(table):
         t.add(host.Call(C.cast(entry, C.c_void_p).value, "entry", ((0, 0), 1, (1, 0)), (a, a), ("op",), prepare=lambda *_: (packed, a)))
         with pytest.raises((RuntimeError, TypeError)):
             t.launch(("op",), None, a, a)
+
+
+def test_changed_signal_words_are_seen(table):
+    """A bound call copies the words' descriptor; after a change of what that holds the call is built again, not launched."""
+    table, _ = table
+    fault = torch.zeros(1, dtype=torch.int64)
+    words = _launch.SyncWords(locks=torch.zeros(4, dtype=torch.int32), arrivals=torch.zeros(4), fault=fault)
+    seen = []
+
+    @C.CFUNCTYPE(C.c_int, C.POINTER(_lib.SyncDescArrivals), C.c_void_p)
+    def entry(sync, stream):
+        seen.append((sync[0].locks, sync[0].trace_done_clock, sync[0].epoch))
+        return 0
+
+    a = torch.zeros(8)
+
+    def call():
+        if table.launch(("w",), None, a) is None:
+            _launch.bind(table, ("w",), (a,), entry, (_launch.SYNC,), "w", words=words, variant="s1")
+            return _launch.issue(table, ("w",), None, a) and "bound"
+        return "known"
+
+    assert [call(), call()] == ["bound", "known"] and len(table) == 1
+    words.spin_limit_ns = 5  # read at every launch, like the launch number
+    assert call() == "known" and seen[-1] == (words.locks.data_ptr(), None, 3)
+    words.trace_done_clock = torch.zeros(4, dtype=torch.int64)
+    assert [call(), call()] == ["bound", "known"] and len(table) == 1
+    assert seen[-1] == (words.locks.data_ptr(), words.trace_done_clock.data_ptr(), 5)
+    words.locks = torch.zeros(4, dtype=torch.int32)
+    assert call() == "bound" and seen[-1] == (words.locks.data_ptr(), words.trace_done_clock.data_ptr(), 6)
+    with pytest.raises(AttributeError):  # a plan's vectors are only changed with the plan
+        _launch.DevicePlan(1, a, a, a, a).tile_counts = a

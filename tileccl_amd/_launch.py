@@ -315,7 +315,7 @@ def transport_desc(directions: int, copy_elems: int, reduce_elems: int | None, n
     return t
 
 
-@dataclass
+@dataclass(frozen=True)
 class DevicePlan:
     """Device-resident copy of a ``TileGroupPlan``'s vectors (uploaded once per plan)."""
 
@@ -380,6 +380,15 @@ class SyncWords:
     arrivals: torch.Tensor | None = None  # counters, zero between launches (tccl_sync_desc_arrivals)
     arrivals_from_capture: bool = False  # zeroed by a recorded fill only: every launch has to clear them itself
     clear_every_launch: bool = False  # set by the first launch recorded into a graph
+    revision: int = 0  # grows with every change of what the descriptor holds: calls bound with an earlier one are built again
+
+    _DESCRIBED = frozenset(("locks", "counter", "barrier", "plan", "fault", "arrivals", "trace_comm_counter", "trace_start_clock",
+                            "trace_ready_clock", "trace_done_clock"))
+
+    def __setattr__(self, name: str, value) -> None:
+        object.__setattr__(self, name, value)
+        if name in SyncWords._DESCRIBED:
+            object.__setattr__(self, "revision", self.__dict__.get("revision", 0) + 1)
 
     def reset(self) -> None:
         for t in (self.locks, self.counter, self.barrier, self.arrivals, self.trace_comm_counter, self.trace_start_clock,

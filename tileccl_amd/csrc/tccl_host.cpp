@@ -30,7 +30,7 @@ constexpr int kMaxTensors = 9;   // an operation's operands and output; one tens
 constexpr size_t kMaxCalls = 64;
 
 PyObject *kGemm, *kSync;                                       // stand for the descriptor copies in an argument list
-PyObject *sEpoch, *sLockEpoch, *sClear, *sMaxTasks, *sSpin, *sNext;  // attributes of the signal words
+PyObject *sEpoch, *sLockEpoch, *sClear, *sMaxTasks, *sSpin, *sNext, *sRevision;  // attributes of the signal words
 PyObject *current_stream, *is_capturing, *report, *device0;
 
 // Everything about a tensor that a descriptor depends on, except where it lies.
@@ -71,6 +71,7 @@ struct Call {
   uint32_t on_heap;
   std::vector<int64_t>* bases;  // per tensor: all must lie at one offset from these
   int counted;           // 0: the launch is not numbered, 1: by `epoch`, 2: by `lock_epoch`
+  long long revision;    // of the signal words when their descriptor was copied (< 0: they have none)
   PyObject *key, *tag, *what, *words, *prepare, *keep, *variant;
 };
 
@@ -127,6 +128,14 @@ PyObject* own(PyObject* o) {
   if (o == Py_None) return nullptr;
   Py_XINCREF(o);
   return o;
+}
+
+bool int_attr(PyObject* o, PyObject* name, long long& out) {
+  PyObject* v = PyObject_GetAttr(o, name);
+  if (!v) return false;
+  out = PyLong_AsLongLong(v);
+  Py_DECREF(v);
+  return !(out == -1 && PyErr_Occurred());
 }
 
 // Call(entry, what, args, tensors, key, *, tag, gemm, c, sync, words, variant, on_heap, heap, bases, prepare, keep)
@@ -225,6 +234,8 @@ int call_init_checked(Call* self, PyObject* pos, PyObject* kw) {
     if (!v) return -1;
     self->counted = !strcmp(v, "s2") ? 1 : !strcmp(v, "s1") ? 2 : 0;
   }
+  self->revision = -1;
+  if (sync && words != Py_None && PyObject_HasAttr(words, sRevision) && !int_attr(words, sRevision, self->revision)) return -1;
   Py_INCREF(key);
   self->key = key;
   self->tag = own(tag);
@@ -262,14 +273,6 @@ bool same_key(PyObject* a, PyObject* b) {
   return true;
 }
 
-bool int_attr(PyObject* o, PyObject* name, long long& out) {
-  PyObject* v = PyObject_GetAttr(o, name);
-  if (!v) return false;
-  out = PyLong_AsLongLong(v);
-  Py_DECREF(v);
-  return !(out == -1 && PyErr_Occurred());
-}
-
 // The launch's number: what SyncWords.next_epoch() gives.  The ordinary case (nothing to clear, no wrap-around near)
 // is one increment; the others are left to that method.
 bool next_number(const Call* c, int32_t& number) {
@@ -293,7 +296,7 @@ bool next_number(const Call* c, int32_t& number) {
   number = (int32_t)((by_lock ? lock_epoch : epoch) + 1);
   PyObject* n = PyLong_FromLong(number);
   if (!n) return false;
-  const int rc = PyObject_SetAttr(c->words, by_lock ? sLockEpoch : sEpoch, n);
+  const int rc = PyObject_GenericSetAttr(c->words, by_lock ? sLockEpoch : sEpoch, n);  // (no part of the words' descriptor)
   Py_DECREF(n);
   return rc == 0;
 }
@@ -450,6 +453,15 @@ PyObject* table_add(Table* self, PyObject* call) {
   Py_RETURN_NONE;
 }
 
+void drop(Table* self, Call* call) {
+  for (size_t i = 0; i < self->calls->size(); ++i) {
+    if ((*self->calls)[i] != call) continue;
+    self->calls->erase(self->calls->begin() + i);
+    Py_DECREF(call);
+    return;
+  }
+}
+
 // launch(key, alpha, *tensors): the tag of the call that was issued, or None if there is none for these tensors.
 PyObject* table_launch(Table* self, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs < 3 || nargs > 2 + kMaxTensors || !PyTuple_Check(args[0])) {
@@ -466,6 +478,14 @@ PyObject* table_launch(Table* self, PyObject* const* args, Py_ssize_t nargs) {
       if (!fits(c, args + 2, at, nargs - 2) || !same_key(c->key, args[0])) continue;
       Reference held{(PyObject*)c};  // another thread may drop it from the table meanwhile
       Py_INCREF(c);
+      if (c->revision >= 0) {
+        long long now = 0;
+        if (!int_attr(c->words, sRevision, now)) return nullptr;
+        if (now != c->revision) {  // what the copied descriptor points at may be gone: the call is built again
+          drop(self, c);
+          Py_RETURN_NONE;
+        }
+      }
       return launch(c, args + 2, at, args[1]);
     }
     Py_RETURN_NONE;
@@ -525,6 +545,7 @@ PyMODINIT_FUNC PyInit__host() {
   sMaxTasks = PyUnicode_InternFromString("max_tasks_per_tile");
   sSpin = PyUnicode_InternFromString("spin_limit_ns");
   sNext = PyUnicode_InternFromString("next_epoch");
+  sRevision = PyUnicode_InternFromString("revision");
   device0 = PyLong_FromLong(0);  // every rank lives on device 0
   PyObject* m = PyModule_Create(&module_def);
   if (!m) return nullptr;

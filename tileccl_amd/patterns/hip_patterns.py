@@ -56,6 +56,10 @@ class _HipAllScatterPattern(Pattern):
         """(GEMM workgroups or 0 for the library default, communication workgroups or 0)."""
         return self.NUM_SMS, 0
 
+    def _settings(self) -> tuple:
+        """What can be set on a pattern and changes its launches: part of the key of its bound calls."""
+        return (self.BLOCK_M, self.BLOCK_N, self.GROUP_M, self.NUM_SMS, self.COMPUTE_SMS, self.COMM_SMS)
+
     # -- execution ---------------------------------------------------------------------
     def execute(self, A, B, C_out, **kwargs: Any) -> None:
         spec = self.resolve_execution(
@@ -74,7 +78,7 @@ class _HipAllScatterPattern(Pattern):
                 "C must live in the symmetric heap when world_size > 1: the scatter writes it at the "
                 "same offset in every peer's slice"
             )
-        key = (heap.local_base, spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
+        key = (heap.local_base, *self._settings(), spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
         ran = self._calls.launch(key, None, A, B, C_out)
         if ran is None:
             self._bind(self._calls, key, (A, B, C_out), (2, 0), spec, heap)
@@ -185,6 +189,9 @@ class TileGroupPattern(_HipAllScatterPattern):
         self.tau_min_bytes = tau_min_bytes
         self.max_groups = max_groups
         self.last_plan: TileGroupPlan | None = None
+
+    def _settings(self) -> tuple:
+        return (*super()._settings(), self.target_group_tiles, self.copy_elems, self.tau_min_bytes, self.max_groups)
 
     def _copy_elems(self) -> int:
         return self.copy_elems

@@ -29,6 +29,7 @@ from tileccl_amd.v2.signal import TileGroupSignalState, allocate_tile_group_sign
 from tileccl_amd.v2.tile_group import TileGroupPlan, build_tile_group_plan
 from tileccl_amd.v2.transport import CommMode, P2PTransportPlan, build_p2p_transport_plan
 
+_OUT = (3, 0)  # `out` among a bound call's arguments: the address of its fourth tensor
 PEER_READY = 1 << 30  # word value that marks a resident peer's tiles / groups as complete for every launch
 
 
@@ -139,28 +140,31 @@ class _FusedBase:
             self.heap.peer_view(self.signals.counter, peer).fill_(PEER_READY)
             self.heap.peer_view(self.locks, peer).fill_(PEER_READY)
 
-    def _launch_known(self, A: torch.Tensor, B: torch.Tensor, variant: str, alpha: float, *settings: object) -> None:
-        """Issue the bound call for operands of these layouts and this operation's present settings, made if need be."""
-        key = (variant, self.directions, self.macro_tile, self.num_gemm_wgs, self.num_comm_wgs, self.words, self.transport,
-               self.heap.local_base, *settings)
-        if self._calls.launch(key, alpha, A, B) is None:
+    def _launch_known(self, A: torch.Tensor, B: torch.Tensor, product: torch.Tensor, variant: str, alpha: float, *settings: object) -> None:
+        """Issue the bound call for tensors of these layouts and this operation's present settings, made if need be.
+        Everything that can be set from outside is looked at: what a descriptor depends on is in the key, and the
+        tensors (operands, the GEMM's product, ``out``) are passed to the call."""
+        key = (variant, self.directions, self.macro_tile, self.num_gemm_wgs, self.num_comm_wgs, self.block_m, self.block_n, self.group_m,
+               self.words, self.transport, self.heap.local_base, *settings)
+        if self._calls.launch(key, alpha, A, B, product, self.out) is None:
             self.heap.get_heap_bases()  # raises once the heap has been cleaned up
             self._bind(key, A, B, variant)
-            _launch.issue(self._calls, key, alpha, A, B)
+            _launch.issue(self._calls, key, alpha, A, B, product, self.out)
 
-    def _bound(self, key: tuple, A: torch.Tensor, B: torch.Tensor, out: torch.Tensor, variant: str, flags: int, fn, what: str, args) -> None:
-        """Keep the call ``fn(gemm, *args(view, transport), variant)`` for operands of these layouts."""
+    def _bound(self, key: tuple, A: torch.Tensor, B: torch.Tensor, product: torch.Tensor, variant: str, flags: int, fn, what: str, args) -> None:
+        """Keep the call ``fn(gemm, *args(view, transport), variant)`` for tensors of these layouts; in ``args``, ``_OUT`` is the
+        address of ``out``."""
         if variant not in _launch.VARIANTS:
             raise ValueError(f"unknown variant {variant!r}; expected one of {sorted(_launch.VARIANTS)}")
         gemm, plan = _launch._gemm_desc(
-            A, B, out, block_m=self.block_m, block_n=self.block_n, group_m=self.group_m,
+            A, B, product, block_m=self.block_m, block_n=self.block_n, group_m=self.group_m,
             num_wgs=self.num_gemm_wgs, macro_tile=self.macro_tile, flags=flags | _lib.GEMM_ARRIVALS,
         )
         transport = _launch.transport_desc(
             self.directions, self.transport.copy_elems, self.transport.reduce_elems, self.num_comm_wgs
         )
-        _launch.bind(self._calls, key, (A, B), fn, (gemm, *args(_launch.view_of(self.heap), transport), _launch.VARIANTS[variant]),
-                     f"{what}[{variant}]", gemm=gemm, plan=plan, words=self.words, variant=variant)
+        _launch.bind(self._calls, key, (A, B, product, self.out), fn, (gemm, *args(_launch.view_of(self.heap), transport), _launch.VARIANTS[variant]),
+                     f"{what}[{variant}]", gemm=gemm, plan=plan, words=self.words, variant=variant, c=(2, 0))
 
     def check_faults(self) -> None:
         if self.words is not None:
@@ -192,12 +196,12 @@ class FusedGemmAllGather(_FusedBase):
     def __call__(self, A: torch.Tensor, B: torch.Tensor, variant: str = "s2", alpha: float = 1.0,
                  scale_a: float = 1.0, scale_b: float = 1.0) -> torch.Tensor:
         # per-tensor dequantisation scales of fp8 inputs
-        self._launch_known(A, B, variant, float(alpha) * float(scale_a) * float(scale_b))
+        self._launch_known(A, B, self.local_block, variant, float(alpha) * float(scale_a) * float(scale_b))
         return self.out
 
     def _bind(self, key: tuple, A: torch.Tensor, B: torch.Tensor, variant: str) -> None:
         self._bound(key, A, B, self.local_block, variant, 0, _lib.load().tccl_gemm_allgather, "tccl_gemm_allgather",
-                    lambda view, transport: (_launch.ptr(self.out), int(self.out.stride(0)), view, _launch.SYNC, transport))
+                    lambda view, transport: (_OUT, int(self.out.stride(0)), view, _launch.SYNC, transport))
 
 
 class FusedGemmReduceScatter(_FusedBase):
@@ -241,11 +245,12 @@ class FusedGemmReduceScatter(_FusedBase):
     def __call__(self, A: torch.Tensor, B: torch.Tensor, variant: str = "s2", alpha: float = 1.0,
                  scale_a: float = 1.0, scale_b: float = 1.0) -> torch.Tensor:
         # per-tensor dequantisation scales of fp8 inputs
-        self._launch_known(A, B, variant, float(alpha) * float(scale_a) * float(scale_b), self.emulate_peer, self.own_rows_in_registers)
+        self._launch_known(A, B, self.partial, variant, float(alpha) * float(scale_a) * float(scale_b), self.emulate_peer,
+                           self.own_rows_in_registers)
         return self.out
 
     def _bind(self, key: tuple, A: torch.Tensor, B: torch.Tensor, variant: str) -> None:
         self._bound(key, A, B, self.partial, variant, _lib.GEMM_OWN_ROWS_IN_REGISTERS if self.own_rows_in_registers else 0,
                     _lib.load().tccl_gemm_reducescatter, "tccl_gemm_reducescatter",
-                    lambda view, transport: (_launch.ptr(self.out), _launch.dtype_code(self.out.dtype), int(self.out.stride(0)), view,
+                    lambda view, transport: (_OUT, _launch.dtype_code(self.out.dtype), int(self.out.stride(0)), view,
                                              _launch.SYNC, transport, int(self.emulate_peer)))
