@@ -44,6 +44,7 @@ def test_gather_output_block_sizes_and_words(lib):
         op(A, B)
         torch.cuda.synchronize()
         assert int(fault.item()) == 1
+        fault.zero_()
         op.local_block = other[M:]  # not this rank's rows of `out`
         with pytest.raises(ValueError, match="rank"):
             op(A, B)
@@ -53,6 +54,10 @@ def test_gather_output_block_sizes_and_words(lib):
             with pytest.raises(ValueError, match="plan tile"):
                 op(A, B)
             setattr(op, name, 128)
+        # Refused launches were none: the counters, which a traced launch waits for itself, are still in step.
+        op.directions, op.words.spin_limit_ns, op.words.trace_ready_clock = 1, 2_000_000_000, op.signals.trace_ready_clock
+        op(A, B)
+        op.check_faults()
     finally:
         for h in heaps:
             h.cleanup()

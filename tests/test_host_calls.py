@@ -208,3 +208,26 @@ def test_changed_signal_words_are_seen(table):
     assert call() == "bound" and seen[-1] == (words.locks.data_ptr(), words.trace_done_clock.data_ptr(), 6)
     with pytest.raises(AttributeError):  # a plan's vectors are only changed with the plan
         _launch.DevicePlan(1, a, a, a, a).tile_counts = a
+
+
+@pytest.mark.parametrize("variant,attr", [("s2", "epoch"), ("s1", "lock_epoch")])
+def test_a_refused_launch_takes_no_number(table, variant, attr):
+    table, _ = table
+    words = _launch.SyncWords(locks=torch.zeros(4, dtype=torch.int32), arrivals=torch.zeros(4), fault=torch.zeros(1, dtype=torch.int64))
+    numbers, answers = [], [0, _lib.ERR_UNSUPPORTED, _lib.ERR_INVALID, 0, 700, 0]
+
+    @C.CFUNCTYPE(C.c_int, C.POINTER(_lib.SyncDescArrivals), C.c_void_p)
+    def entry(sync, stream):
+        numbers.append(sync[0].epoch)
+        return answers[len(numbers) - 1]
+
+    a = torch.zeros(8)
+    _launch.bind(table, ("n",), (a,), entry, (_launch.SYNC,), "n", words=words, variant=variant)
+    for rc in answers:
+        if rc:
+            with pytest.raises(ValueError if rc < 0 else RuntimeError):
+                table.launch(("n",), None, a)
+        else:
+            assert table.launch(("n",), None, a) is True
+    assert numbers == [1, 2, 2, 2, 3, 4]  # a HIP error may come after the launch: its number is gone
+    assert getattr(words, attr) == 4 and words.epoch + words.lock_epoch == 4

@@ -301,6 +301,20 @@ bool next_number(const Call* c, int32_t& number) {
   return rc == 0;
 }
 
+// A launch that the entry point refused has signalled nothing: its number goes to the next one, or the words would be
+// behind the numbers (and this rank's behind its peers') from here on.
+bool number_back(const Call* c, int32_t number) {
+  PyObject* name = c->counted == 2 ? sLockEpoch : sEpoch;
+  long long now = 0;
+  if (!int_attr(c->words, name, now)) return false;
+  if (now != number) return true;  // another thread has numbered a launch since
+  PyObject* n = PyLong_FromLong(number - 1);
+  if (!n) return false;
+  const int rc = PyObject_GenericSetAttr(c->words, name, n);
+  Py_DECREF(n);
+  return rc == 0;
+}
+
 // Issue the call on these tensors (of the layouts it was built for, at the addresses `at`).  Returns the tag, or null with an
 // exception set.
 PyObject* launch(Call* c, PyObject* const* tensors, int64_t* at, PyObject* alpha) {
@@ -362,6 +376,7 @@ PyObject* launch(Call* c, PyObject* const* tensors, int64_t* at, PyObject* alpha
       v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11]);
   Py_END_ALLOW_THREADS;
   if (rc != 0) {
+    if (rc < 0 && c->has_sync && c->words && c->counted && !number_back(c, sync.sync.epoch)) return nullptr;
     PyObject* r = PyObject_CallFunction(report, "iO", (int)rc, c->what ? c->what : Py_None);
     Py_XDECREF(r);
     if (!PyErr_Occurred()) PyErr_Format(PyExc_RuntimeError, "error code %d", (int)rc);
