@@ -165,7 +165,10 @@ struct StreamGemm {
     return kNB == 2 ? (k >> 3) & 1 : 0;
   }
   static TCCL_D int row_at(int k) { return kNB == 1 && kEsz == 2 ? k ^ (4 * ((k >> 3) & 1)) : k; }
+  // The hardware keeps the order of a wavefront's LDS accesses, the fences on both sides the compiler's: these writes come
+  // after the reads of the block before and ahead of the reads that other lanes make of them.
   TCCL_D void stage(const Block& v) const {
+    asm volatile("" ::: "memory");
     char* at = lds + wave * kWaveBytes;
 #pragma unroll
     for (int h = 0; h < 2 * kMB; ++h) {
@@ -183,6 +186,7 @@ struct StreamGemm {
         *(u32x4*)(at + row_at(k) * kRowBytes + ((c ^ (kEsz * swizzle(k))) << 4)) = v.b[h];
       }
     }
+    asm volatile("" ::: "memory");
   }
   // 16-byte chunk 4 h + l / 16 of row l % 16 of 16-row block `block` (A, k-major B): the 16-bit operand of 32-k half h (k
   // 8 (l / 16) .. + 7 of it); the e4m3 operand of a whole block is both (k 16 (l / 16) .. + 15 and 64 + that).
