@@ -231,3 +231,42 @@ def test_a_refused_launch_takes_no_number(table, variant, attr):
             assert table.launch(("n",), None, a) is True
     assert numbers == [1, 2, 2, 2, 3, 4]  # a HIP error may come after the launch: its number is gone
     assert getattr(words, attr) == 4 and words.epoch + words.lock_epoch == 4
+
+
+def test_the_call_unused_for_longest_goes_first(table):
+    host = _lib.host()
+    table, keep = host.Table(3), []
+    a = torch.zeros(8)
+
+    def found(n):
+        return table.launch(("op", n), None, a) is True
+
+    with pytest.raises(ValueError):
+        host.Table(0)
+    for n in range(3):
+        keep.append(bound_to(table, n, a))
+    assert found(0)
+    keep.append(bound_to(table, 3, a))
+    assert [found(n) for n in range(4)] == [True, False, True, True]
+
+
+def bound_to(table, n, t):
+    @ENTRY
+    def entry(*_):
+        return 0
+
+    _launch.bind(table, ("op", n), (t,), entry, ((0, 0), 1, 2), "entry")
+    return entry
+
+
+def test_a_program_that_goes_round_many_layouts_finds_its_calls(table):
+    """Gradient buckets of 500 sizes, several times round: bound once each."""
+    made = _launch.call_table({})
+    buf = torch.zeros(1 << 12)
+    keep = []
+    for turn in range(3):
+        for n in range(1, 501):
+            t = buf[:n]
+            if made.launch(("op", 0), None, t) is None:
+                keep.append(bound_to(made, 0, t))
+    assert len(keep) == len(made) == 500

@@ -238,10 +238,11 @@ SYNC = object()  # stands for the sync descriptor in the arguments of a bound ca
 
 
 def call_table(owner: dict):
-    """The bound calls kept with ``owner`` (a heap's or an operation's ``__dict__``, a context's workspaces): at most 64."""
+    """The bound calls kept with ``owner`` (a heap's or an operation's ``__dict__``, a context's workspaces): at most 1024, some
+    2 KiB each.  A program that goes round more layouts than that (of row counts, of gradient buckets) binds every call anew."""
     table = owner.get("tileccl_amd.calls")
     if table is None:
-        table = owner["tileccl_amd.calls"] = _lib.host().Table()
+        table = owner["tileccl_amd.calls"] = _lib.host().Table(1024)
     return table
 
 

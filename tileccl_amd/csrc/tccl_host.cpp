@@ -7,9 +7,10 @@
 // Python that took 3 to 5 us (a key of shapes, strides and types per tensor alone takes 1 us), beside the 2.5 us of
 // the launch itself; here it takes 0.3 us.
 //
-// `Table` holds the calls of one owner (a context, a heap, an operation), bounded, oldest dropped first.  Everything
-// runs under the interpreter lock except the C entry point; a Call does not change once it is built, and each launch
-// works on copies of its descriptors, so threads may share both.
+// `Table` holds the calls of one owner (a context, a heap, an operation), found by a hash of the key and the layouts, bounded, the
+// one that has not been used for longest dropped first.  Everything runs under the interpreter lock except the C entry
+// point; a Call does not change once it is built, and each launch works on copies of its descriptors, so threads may
+// share both.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -19,6 +20,8 @@
 #include <cstdint>
 #include <cstring>
 #include <exception>
+#include <list>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/tileccl_hip.h"
@@ -27,11 +30,13 @@ namespace {
 
 constexpr int kMaxArgs = 12;     // arguments of an entry point, the stream included
 constexpr int kMaxTensors = 9;   // an operation's operands and output; one tensor per rank
-constexpr size_t kMaxCalls = 64;
+constexpr unsigned long kCalls = 64;  // a table's bound unless it is given one
 
 PyObject *kGemm, *kSync;                                       // stand for the descriptor copies in an argument list
 PyObject *sEpoch, *sLockEpoch, *sClear, *sMaxTasks, *sSpin, *sNext, *sRevision;  // attributes of the signal words
 PyObject *current_stream, *is_capturing, *report, *device0;
+
+size_t mixed(size_t h, size_t v) { return (h ^ v) * 0x9e3779b97f4a7c15ull + (h >> 29); }
 
 // Everything about a tensor that a descriptor depends on, except where it lies.
 struct Layout {
@@ -43,6 +48,12 @@ struct Layout {
   explicit Layout(const at::Tensor& t)
       : type(t.scalar_type()), device(t.device()), misaligned((int)((uintptr_t)t.data_ptr() & 15)),
         sizes(t.sizes().begin(), t.sizes().end()), strides(t.strides().begin(), t.strides().end()) {}
+  static size_t hash(size_t h, const at::Tensor& t, uintptr_t at) {
+    h = mixed(h, (size_t)t.scalar_type() * 16 + (at & 15));
+    for (const int64_t n : t.sizes()) h = mixed(h, (size_t)n);
+    for (const int64_t n : t.strides()) h = mixed(h, (size_t)n);
+    return h;
+  }
   bool matches(const at::Tensor& t, uintptr_t at) const {
     return type == t.scalar_type() && misaligned == (int)(at & 15) && device == t.device() && t.sizes().equals(sizes) &&
            t.strides().equals(strides);
@@ -72,6 +83,7 @@ struct Call {
   std::vector<int64_t>* bases;  // per tensor: all must lie at one offset from these
   int counted;           // 0: the launch is not numbered, 1: by `epoch`, 2: by `lock_epoch`
   long long revision;    // of the signal words when their descriptor was copied (< 0: they have none)
+  size_t hash;           // of the key and the layouts
   PyObject *key, *tag, *what, *words, *prepare, *keep, *variant;
 };
 
@@ -138,6 +150,34 @@ bool int_attr(PyObject* o, PyObject* name, long long& out) {
   return !(out == -1 && PyErr_Occurred());
 }
 
+// Plain values of a key count by value, anything else (a context, signal words, a contract) by identity.
+bool plain(PyObject* o) { return PyLong_CheckExact(o) || PyUnicode_CheckExact(o) || PyFloat_CheckExact(o) || PyBool_Check(o); }
+bool same(PyObject* a, PyObject* b) {
+  if (a == b) return true;
+  if (Py_TYPE(a) != Py_TYPE(b) || !plain(a)) return false;
+  const int r = PyObject_RichCompareBool(a, b, Py_EQ);
+  if (r < 0) PyErr_Clear();
+  return r == 1;
+}
+bool same_key(PyObject* a, PyObject* b) {
+  if (a == b) return true;
+  const Py_ssize_t n = PyTuple_GET_SIZE(a);
+  if (n != PyTuple_GET_SIZE(b)) return false;
+  for (Py_ssize_t i = 0; i < n; ++i)
+    if (!same(PyTuple_GET_ITEM(a, i), PyTuple_GET_ITEM(b, i))) return false;
+  return true;
+}
+size_t key_hash(PyObject* key) {
+  size_t h = (size_t)PyTuple_GET_SIZE(key);
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(key); ++i) {
+    PyObject* o = PyTuple_GET_ITEM(key, i);
+    Py_hash_t v = (Py_hash_t)((uintptr_t)o >> 4);
+    if (plain(o) && (v = PyObject_Hash(o)) == -1) PyErr_Clear();
+    h = mixed(h, (size_t)v);
+  }
+  return h;
+}
+
 // Call(entry, what, args, tensors, key, *, tag, gemm, c, sync, words, variant, on_heap, heap, bases, prepare, keep)
 int call_init_checked(Call* self, PyObject* pos, PyObject* kw) {
   static const char* names[] = {"entry", "what", "args", "tensors", "key", "tag", "gemm", "c", "sync", "words", "variant",
@@ -162,12 +202,15 @@ int call_init_checked(Call* self, PyObject* pos, PyObject* kw) {
     PyErr_SetString(PyExc_ValueError, "a Call takes an entry point, 1 to 9 tensors and at most 11 arguments");
     return -1;
   }
+  self->hash = key_hash(key);
   for (Py_ssize_t i = 0; i < n; ++i) {
     if (!THPVariable_Check(PyTuple_GET_ITEM(tensors, i))) {
       PyErr_SetString(PyExc_TypeError, "a Call is built for tensors");
       return -1;
     }
-    self->layouts->emplace_back(THPVariable_Unpack(PyTuple_GET_ITEM(tensors, i)));
+    const at::Tensor& t = THPVariable_Unpack(PyTuple_GET_ITEM(tensors, i));
+    self->layouts->emplace_back(t);
+    self->hash = Layout::hash(self->hash, t, (uintptr_t)t.data_ptr());
   }
   if (gemm) {
     self->has_gemm = true;
@@ -252,26 +295,6 @@ int call_init(Call* self, PyObject* pos, PyObject* kw) {
 }
 
 PyTypeObject CallType = {PyVarObject_HEAD_INIT(nullptr, 0)};
-
-// Same object, or the same plain value.  Anything else (a context, signal words, a contract) counts by identity.
-bool same(PyObject* a, PyObject* b) {
-  if (a == b) return true;
-  if (Py_TYPE(a) != Py_TYPE(b)) return false;
-  if (PyLong_Check(a) || PyUnicode_Check(a) || PyFloat_Check(a)) {
-    const int r = PyObject_RichCompareBool(a, b, Py_EQ);
-    if (r < 0) PyErr_Clear();
-    return r == 1;
-  }
-  return false;
-}
-bool same_key(PyObject* a, PyObject* b) {
-  if (a == b) return true;
-  const Py_ssize_t n = PyTuple_GET_SIZE(a);
-  if (n != PyTuple_GET_SIZE(b)) return false;
-  for (Py_ssize_t i = 0; i < n; ++i)
-    if (!same(PyTuple_GET_ITEM(a, i), PyTuple_GET_ITEM(b, i))) return false;
-  return true;
-}
 
 // The launch's number: what SyncWords.next_epoch() gives.  The ordinary case (nothing to clear, no wrap-around near)
 // is one increment; the others are left to that method.
@@ -387,13 +410,14 @@ PyObject* launch(Call* c, PyObject* const* tensors, int64_t* at, PyObject* alpha
   return tag;
 }
 
-// The tensors' addresses; false if one has none, which no call is for.
-bool addresses(PyObject* const* tensors, Py_ssize_t n, int64_t* at) {
+// The tensors' addresses, and their layouts added to the hash; false if one has no address, which no call is for.
+bool addresses(PyObject* const* tensors, Py_ssize_t n, int64_t* at, size_t& hash) {
   try {
     for (Py_ssize_t i = 0; i < n; ++i) {
       const at::Tensor& t = THPVariable_Unpack(tensors[i]);
       if (t.layout() != c10::kStrided || t.unsafeGetTensorImpl()->is_nested()) return false;
       at[i] = (int64_t)(uintptr_t)t.data_ptr();
+      hash = Layout::hash(hash, t, (uintptr_t)at[i]);
     }
   } catch (...) {
     return false;
@@ -422,59 +446,82 @@ bool fits(const Call* c, PyObject* const* tensors, const int64_t* at, Py_ssize_t
 
 struct Table {
   PyObject_HEAD
-  std::vector<Call*>* calls;  // newest last
+  std::list<Call*>* order;  // used last first
+  std::unordered_multimap<size_t, std::list<Call*>::iterator>* by_hash;
+  size_t limit;
 };
 
-PyObject* table_new(PyTypeObject* type, PyObject*, PyObject*) {
+// Table(limit=64)
+PyObject* table_new(PyTypeObject* type, PyObject* args, PyObject* kw) {
+  static const char* names[] = {"limit", nullptr};
+  unsigned long limit = kCalls;
+  if (!PyArg_ParseTupleAndKeywords(args, kw, "|k", (char**)names, &limit)) return nullptr;
+  if (limit < 1) {
+    PyErr_SetString(PyExc_ValueError, "a Table holds at least one Call");
+    return nullptr;
+  }
   return guarded((PyObject*)nullptr, [&] {
     Table* t = (Table*)type->tp_alloc(type, 0);
-    if (t) t->calls = new std::vector<Call*>();
+    if (!t) return (PyObject*)nullptr;
+    Reference held{(PyObject*)t};
+    t->limit = limit;
+    t->order = new std::list<Call*>();
+    t->by_hash = new std::unordered_multimap<size_t, std::list<Call*>::iterator>();
+    held.object = nullptr;
     return (PyObject*)t;
   });
 }
 int table_traverse(Table* self, visitproc visit, void* arg) {
-  for (Call* c : *self->calls) Py_VISIT((PyObject*)c);
+  if (self->order)
+    for (Call* c : *self->order) Py_VISIT((PyObject*)c);
   return 0;
 }
 int table_clear(Table* self) {
-  std::vector<Call*> calls;
-  calls.swap(*self->calls);
+  if (self->by_hash) self->by_hash->clear();
+  std::list<Call*> calls;
+  if (self->order) calls.swap(*self->order);
   for (Call* c : calls) Py_DECREF(c);
   return 0;
 }
 void table_dealloc(Table* self) {
   PyObject_GC_UnTrack(self);
   table_clear(self);
-  delete self->calls;
+  delete self->order;
+  delete self->by_hash;
   Py_TYPE(self)->tp_free((PyObject*)self);
 }
 
-PyObject* table_add(Table* self, PyObject* call) {
-  if (!PyObject_TypeCheck(call, &CallType) || !((Call*)call)->layouts || !((Call*)call)->key) {
+void drop(Table* self, Call* call) {
+  const auto range = self->by_hash->equal_range(call->hash);
+  for (auto i = range.first; i != range.second; ++i) {
+    if (*i->second != call) continue;
+    self->order->erase(i->second);
+    self->by_hash->erase(i);
+    Py_DECREF(call);  // (may run other code: the table is in order by now)
+    return;
+  }
+}
+
+PyObject* table_add(Table* self, PyObject* object) {
+  if (!PyObject_TypeCheck(object, &CallType) || !((Call*)object)->layouts || !((Call*)object)->key) {
     PyErr_SetString(PyExc_TypeError, "Table.add expects a Call");
     return nullptr;
   }
-  if (!guarded(false, [&] {
-        self->calls->push_back((Call*)call);
-        return true;
-      }))
-    return nullptr;
+  Call* call = (Call*)object;
+  const bool added = guarded(false, [&] {
+    self->order->push_front(call);
+    try {
+      self->by_hash->emplace(call->hash, self->order->begin());
+    } catch (...) {
+      self->order->pop_front();
+      throw;
+    }
+    return true;
+  });
+  if (!added) return nullptr;
   Py_INCREF(call);
-  if (self->calls->size() > kMaxCalls) {
-    Call* oldest = self->calls->front();
-    self->calls->erase(self->calls->begin());
-    Py_DECREF(oldest);
-  }
+  if (self->order->size() > self->limit) drop(self, self->order->back());
   Py_RETURN_NONE;
-}
-
-void drop(Table* self, Call* call) {
-  for (size_t i = 0; i < self->calls->size(); ++i) {
-    if ((*self->calls)[i] != call) continue;
-    self->calls->erase(self->calls->begin() + i);
-    Py_DECREF(call);
-    return;
-  }
 }
 
 // launch(key, alpha, *tensors): the tag of the call that was issued, or None if there is none for these tensors.
@@ -485,14 +532,18 @@ PyObject* table_launch(Table* self, PyObject* const* args, Py_ssize_t nargs) {
   }
   for (Py_ssize_t i = 2; i < nargs; ++i)
     if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+  if (self->order->empty()) Py_RETURN_NONE;
   int64_t at[kMaxTensors];
-  if (!addresses(args + 2, nargs - 2, at)) Py_RETURN_NONE;
+  size_t hash = key_hash(args[0]);
+  if (!addresses(args + 2, nargs - 2, at, hash)) Py_RETURN_NONE;
   return guarded((PyObject*)nullptr, [&]() -> PyObject* {
-    for (size_t i = self->calls->size(); i-- > 0;) {
-      Call* c = (*self->calls)[i];
+    const auto range = self->by_hash->equal_range(hash);
+    for (auto i = range.first; i != range.second; ++i) {
+      Call* c = *i->second;
       if (!fits(c, args + 2, at, nargs - 2) || !same_key(c->key, args[0])) continue;
       Reference held{(PyObject*)c};  // another thread may drop it from the table meanwhile
       Py_INCREF(c);
+      self->order->splice(self->order->begin(), *self->order, i->second);
       if (c->revision >= 0) {
         long long now = 0;
         if (!int_attr(c->words, sRevision, now)) return nullptr;
@@ -507,9 +558,9 @@ PyObject* table_launch(Table* self, PyObject* const* args, Py_ssize_t nargs) {
   });
 }
 
-Py_ssize_t table_len(Table* self) { return (Py_ssize_t)self->calls->size(); }
+Py_ssize_t table_len(Table* self) { return (Py_ssize_t)self->order->size(); }
 
-PyMethodDef table_methods[] = {{"add", (PyCFunction)table_add, METH_O, "Keep a Call; past 64 the oldest one goes."},
+PyMethodDef table_methods[] = {{"add", (PyCFunction)table_add, METH_O, "Keep a Call; past the limit the one unused for longest goes."},
                                {"launch", (PyCFunction)(void (*)())table_launch, METH_FASTCALL,
                                 "launch(key, alpha, *tensors) -> the tag of the Call that was issued, or None."},
                                {nullptr, nullptr, 0, nullptr}};
