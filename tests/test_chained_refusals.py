@@ -11,7 +11,7 @@ from tileccl_amd.patterns.chained_ag_gemm_rs import ChainedAGGemmRSPattern
 
 
 class Heap:
-    local_base, size, rank, world_size = 4096, 1 << 20, 0, 2
+    local_base, live_id, size, rank, world_size = 4096, 1, 1 << 20, 0, 2
 
     def __init__(self, inside):
         self.inside, self.taken = inside, []

@@ -16,6 +16,7 @@ What differs by design: all ranks are slices of one device allocation (``Arena``
 
 from __future__ import annotations
 
+import itertools
 import logging
 import math
 
@@ -29,6 +30,9 @@ logger = logging.getLogger(__name__)
 
 def _element_size(dtype: torch.dtype) -> int:
     return torch.empty((), dtype=dtype).element_size()
+
+
+_live_ids = itertools.count(1)
 
 
 class SymmetricHeap:
@@ -74,6 +78,7 @@ class SymmetricHeap:
         self._buffer: torch.Tensor | None = self._arena.slice(rank)
         self._local_ptr = self._arena.bases[rank]
         self._bump = BumpAllocator(self._size, policy=self._BUMP_POLICY)
+        self._live_id = next(_live_ids)
         self._mode = "single_process"
         self._transport_strategy = "local_only" if world_size == 1 else "peer_access"
         self._cleaned_up = False
@@ -117,6 +122,12 @@ class SymmetricHeap:
     @property
     def local_base(self) -> int:
         return self._local_ptr
+
+    @property
+    def live_id(self) -> int:
+        """A number that no other heap of this process has had, 0 once this one has been cleaned up.  (A later heap may
+        lie at the same address.)"""
+        return self._live_id
 
     @property
     def size(self) -> int:
@@ -235,7 +246,7 @@ class SymmetricHeap:
             return
         self._cleaned_up = True
         self._buffer = None
-        self._local_ptr = 0
+        self._local_ptr = self._live_id = 0
         self._bump.reset()
         arena, self._arena = self._arena, None
         arena.release()

@@ -419,7 +419,7 @@ def _scatter(A: Any, B: Any, C: Any, ctx, pattern: PatternLike, hw_info, **how) 
     named = hw_info is None and (pattern is None or isinstance(pattern, str)) and ctx.heap is not None
     if named:
         calls = _launch.call_table(ctx._workspace_cache)
-        key = ("allscatter", ctx.heap.local_base, pattern, *how.values())
+        key = ("allscatter", ctx.heap.live_id, pattern, *how.values())
         if calls.launch(key, None, A, B, C) is not None:
             return C
     plan = _plan_for_call(A, B, C, ctx=ctx, pattern=pattern, hw_info=hw_info, **how)

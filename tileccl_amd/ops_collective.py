@@ -165,7 +165,7 @@ def run_gather(ctx, A: Any, B_shard: Any, Cx: Any, storage_kind: str, variant: s
     """``gemm_allgather``; ``expected``: a plan's contract, which the tensors' must equal (``ValueError`` otherwise)."""
     heap = ctx.require_heap()
     calls = _launch.call_table(ctx._workspace_cache)
-    key = ("gather", heap.local_base, variant, storage_kind, expected)
+    key = ("gather", heap.live_id, variant, storage_kind, expected)
     ran = calls.launch(key, None, A, B_shard, Cx)
     if ran is None:
         k = resolve_gemm_allgather_contract(A, B_shard, Cx, ctx=ctx, storage_kind=storage_kind)
@@ -203,12 +203,12 @@ def _gather_bind(ctx, k: GemmAllGatherContract, A: Any, B_shard: Any, Cx: Any, v
 
 def _reduce_scatter_words(ctx, world: int, M: int, cols: int):
     """Signal words and TileGroup plan of the fused column-shard reduce-scatter, kept per shape
-    on the context.  Every rank allocates them in the same order, so a peer's words sit at the
-    same offset of its slice."""
+    with the context's workspaces (they lie in its heap).  Every rank allocates them in the same order, so a
+    peer's words sit at the same offset of its slice."""
     from tileccl_amd.v2.tile_group import build_tile_group_plan
 
-    cache = ctx.__dict__.setdefault("_reduce_scatter_words", {})
-    key = (world, M, cols)
+    cache = ctx._workspace_cache
+    key = ("tileccl_amd.sync", "reduce_scatter", world, M, cols)
     if key not in cache:
         plan = build_tile_group_plan(world * M, cols, 128 * 128 * 4, row_split_boundaries=[M * q for q in range(1, world)])
         heap = ctx.require_heap()
@@ -267,7 +267,7 @@ def run_reduce(ctx, A: Any, B: Any, Cx: Any, storage_kind: str, variant: str, em
     """``gemm_reducescatter``; ``expected``: a plan's contract, which the tensors' must equal (``ValueError`` otherwise)."""
     heap = ctx.require_heap()
     calls = _launch.call_table(ctx._workspace_cache)
-    key = ("reduce", heap.local_base, variant, storage_kind, emulate_peer, own_rows_in_registers, peers_resident, expected)
+    key = ("reduce", heap.live_id, variant, storage_kind, emulate_peer, own_rows_in_registers, peers_resident, expected)
     ran = calls.launch(key, None, A, B, Cx)
     if ran is None:
         k = resolve_gemm_reducescatter_contract(A, B, Cx, ctx=ctx, storage_kind=storage_kind)

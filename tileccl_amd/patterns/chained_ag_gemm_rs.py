@@ -76,7 +76,7 @@ class ChainedAGGemmRSPattern:
         own = gathered_workspace is None
         if own and input_shard.ndim == W.ndim == 2:
             gathered_workspace = self.ctx.kept_workspace(_GATHERED, input_shard.shape[0], W.shape[0], dtype=input_shard.dtype)
-        key = (heap.local_base, self.BLOCK_M, self.BLOCK_N, *self._stage._settings())
+        key = (heap.live_id, self.BLOCK_M, self.BLOCK_N, *self._stage._settings())
         ran = None
         if gathered_workspace is not None:
             ran = self._calls.launch(key, None, gathered_workspace, W, output, input_shard)

@@ -78,7 +78,7 @@ class _HipAllScatterPattern(Pattern):
                 "C must live in the symmetric heap when world_size > 1: the scatter writes it at the "
                 "same offset in every peer's slice"
             )
-        key = (heap.local_base, *self._settings(), spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
+        key = (heap.live_id, *self._settings(), spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
         ran = self._calls.launch(key, None, A, B, C_out)
         if ran is None:
             self._bind(self._calls, key, (A, B, C_out), (2, 0), spec, heap)

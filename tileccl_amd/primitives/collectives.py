@@ -101,7 +101,7 @@ def allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> None:
         return
     nbytes = _check_allgather(tensor, output, heap)
     if nbytes:
-        table, key = _launch.call_table(heap.__dict__), ("allgather", heap.local_base)
+        table, key = _launch.call_table(heap.__dict__), ("allgather", heap.live_id)
         _launch.bind(
             table, key, (tensor, output), _lib.load().tccl_copy_block,
             ((1, heap.rank * nbytes), (1 << heap.world_size) - 1, (0, 0), heap.rank, 1, nbytes, nbytes, nbytes, _launch.view_of(heap)),
@@ -111,7 +111,7 @@ def allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> None:
 
 
 def run_known_allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> bool:
-    return _launch.call_table(heap.__dict__).launch(("allgather", heap.local_base), None, tensor, output) is not None
+    return _launch.call_table(heap.__dict__).launch(("allgather", heap.live_id), None, tensor, output) is not None
 
 
 def _check_allgather(tensor: torch.Tensor, output: torch.Tensor, heap) -> int:
@@ -180,7 +180,7 @@ def reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap, op: str = "
         return
     block, in_code, out_code = _check_reduce_scatter(tensor, output, heap)
     if block:
-        table, key = _launch.call_table(heap.__dict__), ("reduce_scatter", heap.local_base)
+        table, key = _launch.call_table(heap.__dict__), ("reduce_scatter", heap.live_id)
         _launch.bind(
             table, key, (tensor, output), _lib.load().tccl_reduce_rows,
             ((0, 0), in_code, block, (1, 0), out_code, block, heap.world_size, block, _launch.view_of(heap), None, 0),
@@ -190,7 +190,7 @@ def reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap, op: str = "
 
 
 def run_known_reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap) -> bool:
-    return _launch.call_table(heap.__dict__).launch(("reduce_scatter", heap.local_base), None, tensor, output) is not None
+    return _launch.call_table(heap.__dict__).launch(("reduce_scatter", heap.live_id), None, tensor, output) is not None
 
 
 def _check_reduce_scatter(tensor: torch.Tensor, output: torch.Tensor, heap) -> tuple[int, int, int]:
@@ -221,7 +221,7 @@ def allreduce(tensor: torch.Tensor, heap, op: str = "sum") -> None:
         return
     numel, code = _check_allreduce(tensor, heap)
     if numel:
-        table, key = _launch.call_table(heap.__dict__), ("allreduce", heap.local_base)
+        table, key = _launch.call_table(heap.__dict__), ("allreduce", heap.live_id)
         _launch.bind(
             table, key, (tensor,), _lib.load().tccl_allreduce_chunk,
             ((0, 0), code, numel, _launch.view_of(heap)), "tccl_allreduce_chunk", heap=heap,
@@ -230,7 +230,7 @@ def allreduce(tensor: torch.Tensor, heap, op: str = "sum") -> None:
 
 
 def run_known_allreduce(tensor: torch.Tensor, heap) -> bool:
-    return _launch.call_table(heap.__dict__).launch(("allreduce", heap.local_base), None, tensor) is not None
+    return _launch.call_table(heap.__dict__).launch(("allreduce", heap.live_id), None, tensor) is not None
 
 
 def _check_allreduce(tensor: torch.Tensor, heap) -> tuple[int, int]:

@@ -145,7 +145,7 @@ class _FusedBase:
         Everything that can be set from outside is looked at: what a descriptor depends on is in the key, and the
         tensors (operands, the GEMM's product, ``out``) are passed to the call."""
         key = (variant, self.directions, self.macro_tile, self.num_gemm_wgs, self.num_comm_wgs, self.block_m, self.block_n, self.group_m,
-               self.words, self.transport, self.heap.local_base, *settings)
+               self.words, self.transport, self.heap.live_id, *settings)
         if self._calls.launch(key, alpha, A, B, product, self.out) is None:
             self.heap.get_heap_bases()  # raises once the heap has been cleaned up
             self._bind(key, A, B, variant)
