@@ -174,3 +174,16 @@ def test_static_entry_launch_numbers(lib):
                         assert not reached(old_epoch, epoch)
     for bad in ((0, 1), (1, -1), (1, 16385)):
         assert lib.tccl_static_call_words(bad[0], bad[1], None, None, None) != 0
+
+
+def test_one_rank_of_ragged_rows_is_refused(lib):
+    """column_shards = 1 is a plain GEMM: its rows must be whole plan tiles (as rows of 0 x world they were divided by zero)."""
+    from tileccl_amd import _lib
+
+    d = _lib.GemmDesc(A=0x1000, B=0x1000, C=0x1000, M=100, N=128, K=64, lda=64, ldb=128, ldc=128, in_dtype=_lib.F16, out_dtype=_lib.F32,
+                      alpha=1.0, block_m=128, block_n=128, group_m=8)
+    h = _lib.HeapView(0x1000, 0, 1)
+    for shards in (0, 1):
+        d.column_shards = shards
+        rc = lib.tccl_gemm_reducescatter(C.byref(d), 0x1000, _lib.F16, 128, C.byref(h), None, None, _lib.RS_PEERS_RESIDENT, _lib.S0_BULK, None)
+        assert rc == _lib.ERR_INVALID and b"whole 128-row plan tiles" in lib.tccl_last_error_string()

@@ -2046,7 +2046,7 @@ int tccl_gemm_reducescatter(const tccl_gemm_desc* d, void* out, int32_t out_dtyp
   if (!out || ld_out < d->N) return fail(TCCL_ERR_INVALID, "reducescatter: bad output");
   const int esize = (int)dtype_size(d->out_dtype);
   const int shard = d->M / heap->world_size;
-  const bool ragged = d->column_shards == heap->world_size && d->M % heap->world_size == 0 && shard % d->block_m;
+  const bool ragged = d->column_shards > 1 && d->column_shards == heap->world_size && d->M % heap->world_size == 0 && shard % d->block_m;
   if (!ragged && (rc = check_sync(sync, variant))) return rc;
   if (ragged)
     return reduce_ragged_shards(d, out, out_dtype, ld_out, heap, sync, tr, emulate_peer, (hipStream_t)stream);
