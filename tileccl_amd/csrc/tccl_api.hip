@@ -545,8 +545,9 @@ struct TileChoice {
   double us;
 };
 
-// The quickest kernel for `segs` row blocks of `seg_rows` rows in a launch that carries nothing but pushes.  Measured, bf16,
-// on 40 shapes of 100 .. 2200 tiles of 128 x 128: the choice is the quickest kernel or within 12 % of it.
+// The kernel for `segs` row blocks of `seg_rows` rows in a launch that carries nothing but pushes.  Measured, bf16, on 40
+// seeded shapes of 100 .. 2200 tiles of 128 x 128, row-major and k-major B: the choice is the quickest kernel or within
+// 10 % of it for 74 of the 80, within 17 % for all, 2 % off on average; the 128-tile kernel alone would be 21 % off.
 // What keeps to the old rule: tiles named by the caller, plan tiles other than 128 x 128, workgroup counts.
 TileChoice choose_tiles(const tccl_gemm_desc* d, int64_t seg_rows, int64_t segs, bool allow256, bool pushes, const tccl_device_info& dev) {
   if (d->in_dtype == TCCL_F8E4M3) return {kTiles256, 0};
@@ -884,11 +885,13 @@ bool gather_in_place(const tccl_gemm_desc* d, const tccl_device_info& dev, int k
 }
 
 // ---- streaming path (tccl_stream.h) -------------------------------------------------------------
-// Estimated time of a launch, in us.  A tile's operands pass its CU's vector memory path once, at the rate measured
-// for its shape (KB/us, between that of a k-major and that of a row-major B: 73 and 33, 85 and 45, 85 and 58, 87 and
-// 72, 57 and 50); a tile's sums take the last term.  Measured on 16 .. 256 x
-// 2048 x 4096, 1024 x 1024 x 2048, 1000 x 2064 x 1000, 300 x 768 x 1024 and 512 x 512 x 256, bf16.  Neither the layout
-// of B nor the variant enters, so that all of them add the products up in the same order: the same bits.
+// Estimated time of a launch, in us.  A tile's operands pass its CU's vector memory path once, at a rate (KB/us) that
+// depends on its shape; a tile's sums take the last term.  The rates measured with 256 tiles, k-major and row-major B, are 72
+// and 33, 98 and 74, 97 and 79, 99 and 89, 73 and 49; the constants are those of the kernel's first form and lower, and as only
+// their ratios matter among the shapes, they choose the quickest shape or kernel, or one within 10 %, for 39 of 40 forms
+// measured (20 shapes of 1 .. 1024 rows, both layouts of B; 32 x 2048 x 4096 row-major: 17 % off) and 17 of 20 of e4m3 (row-major
+// B with 64 x 64 tiles, 12 % off, and 64 x 4096 x 4096, 21 %).  Neither the layout of B nor the variant enters, so that all
+// of them add the products up in the same order: the same bits.
 struct StreamCost {
   double rate, sums;
 };
@@ -2018,7 +2021,7 @@ static int reduce_ragged_shards(const tccl_gemm_desc* d, void* out, int32_t out_
   one.column_shards = 0;
   const TileChoice together = choose_tiles(d, g.wrap_rows, d->column_shards, false, false, dev);
   const double apart = d->column_shards * (kLaunchUs + choose_tiles(&one, one.M, 1, plan_tile_fits_macro(&one), false, dev).us);
-  if (d->in_dtype != TCCL_F8E4M3 && d->block_m == 128 && d->block_n == 128 && d->macro_tile != 256 && together.us < apart) {
+  if (d->block_m == 128 && d->block_n == 128 && d->macro_tile != 256 && together.us < apart) {
     g.ragged = 1;
     g.tile_rows = (g.wrap_rows + 127) / 128 * d->column_shards;
     tccl::SignalArgs s;

@@ -6,8 +6,8 @@
 // fp16 in both directions takes 20 us).  Small ones: the launch and one trip to memory, so the work is cut
 // finely enough to give every CU a share (launch_bulk_copy, launch_bulk_reduce) and every rank's value of a unit
 // is requested before the first is added.  The reduction of eight ranks' 2 MiB fp32 chunks took 45 us as 32
-// tasks of 16384 elements; eight such reductions and eight 2 MiB gathers, one call after the other: 462 us
-// before, 171 us now, most of it the host's calls.  S0 of the reduce-scatter with bf16 partials
+// tasks of 16384 elements, 6.0 us now; eight such reductions and eight 2 MiB gathers, one call after the other: 462 us
+// before, 108 us now, 7.2 us of device time a gather.  S0 of the reduce-scatter with bf16 partials
 // (16384 x 4096): 184 us before, 171 us now.
 #pragma once
 

@@ -240,7 +240,7 @@ struct GemmRole {
   char* st0;
   char* st1;
   char* st2;
-  char* st3;  // (five-stage form only)
+  char* st3;  // (forms of four and five stages)
   char* st4;
   const int tid, lane, wave, wm, wn;
 

@@ -2,17 +2,17 @@
 // most of the device idle (decoding rows, short prompts, ragged and narrow problems).
 //
 // One workgroup produces one output tile of (16 kMB) x (16 kNB); its kWaves wavefronts each take every
-// kWaves-th K block of 64 for the WHOLE tile, straight from memory into the operand registers of
-// v_mfma_f32_16x16x32 (no LDS and no barrier in the K loop), and add their accumulators up through LDS at the
-// end.  So a tile of 16 rows of a 4096-deep product is sixteen chains of four K blocks, all requested at once,
-// instead of one chain of 128 K steps.  Measured, bf16, 16 x 2048 x 4096: 7.3 us with a k-major B and 11.5 us row-major
-// against 29 us on the 128 x 128-tile kernel, whose 16 tiles keep 16 CUs busy (40 us in its fused form);
-// 1024 x 1024 x 2048: 12.4 against 20.8 us; an empty launch takes 3.7 us of that.
+// kWaves-th K block of 64 (e4m3: 128) for the WHOLE tile and add their accumulators up through LDS at the end.  A
+// wavefront loads its K blocks in whole lines and turns each to the operand order of v_mfma_f32_16x16x32 through LDS of
+// its own, so there is no barrier in the K loop.  A tile of 16 rows of a 4096-deep product is then sixteen chains of four
+// K blocks, all requested at once, instead of one chain of 128 K steps.  Measured, bf16, 16 x 2048 x 4096: 6.0 us with a
+// k-major B and 7.6 us row-major against 29 us on the 128 x 128-tile kernel, whose 16 tiles keep 16 CUs busy;
+// 1024 x 1024 x 2048: 11.9 and 15.4 against 19 us; an empty launch takes 3.7 us of that.
 //
-// What bounds it: the vector memory path of a CU delivers about 85 KB/us of operands here, and each operand
+// What bounds it: the vector memory path of a CU delivers 70 to 110 KB/us of operands here, and each operand
 // byte of a tile passes it once, (kMB + kNB) * 2 KiB per 64 k; tiles are as large as the output allows while
 // every CU still gets one (stream_shape() in tccl_api.hip).  A row-major B is slower because a narrow tile reads
-// 32 to 128 bytes of each k row.
+// 32 to 128 bytes of each k row.  The matrix pipes are busy 3 % (16 rows) to 15 % of the time.
 #pragma once
 
 #include "tccl_comm.h"
@@ -160,7 +160,6 @@ struct StreamGemm {
   //   32 lanes of a transposing read (ds_read_b64_tr_b16, _tr_b8) touch at a time lie in different banks.
   static TCCL_D int swizzle(int k) {
     if constexpr (kEsz == 1) return kNB == 4 ? ((k >> 2) & 1) | (((k >> 4) & 1) << 1) : (kNB == 2 ? (k >> 4) & 1 : 0);
-    if constexpr (kNB >= 8) return (2 * (k & 3)) ^ ((k >> 3) & 1);
     if constexpr (kNB == 4) return (k & 2) ^ ((k >> 3) & 1);
     return kNB == 2 ? (k >> 3) & 1 : 0;
   }
