@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import ctypes as C
 import sys
-from dataclasses import dataclass, field
+from dataclasses import dataclass
 from functools import partial
 
 import torch
@@ -340,7 +340,7 @@ class DevicePlan:
         )
 
 
-@dataclass
+@dataclass(init=False)
 class SyncWords:
     """Signal words of one fused operation plus the launch epoch.
 
@@ -373,7 +373,7 @@ class SyncWords:
     trace_start_clock: torch.Tensor | None = None
     trace_ready_clock: torch.Tensor | None = None
     trace_done_clock: torch.Tensor | None = None
-    fault: torch.Tensor = field(default_factory=lambda: torch.zeros(1, dtype=torch.int64, device="cuda:0"))
+    fault: torch.Tensor | None = None  # made by the constructor unless it is given one
     epoch: int = 0
     lock_epoch: int = 0
     spin_limit_ns: int = DEFAULT_SPIN_LIMIT_NS
@@ -386,10 +386,20 @@ class SyncWords:
     _DESCRIBED = frozenset(("locks", "counter", "barrier", "plan", "fault", "arrivals", "trace_comm_counter", "trace_start_clock",
                             "trace_ready_clock", "trace_done_clock"))
 
+    def __init__(self, **given) -> None:
+        unknown = given.keys() - self.__dataclass_fields__.keys()
+        if unknown:
+            raise TypeError(f"SyncWords has no {', '.join(sorted(unknown))}")
+        if given.get("fault") is None:
+            given["fault"] = torch.zeros(1, dtype=torch.int64, device="cuda:0")
+        mine = self.__dict__  # (field by field, counting changes, it took 8 us)
+        mine.update(epoch=0, lock_epoch=0, spin_limit_ns=DEFAULT_SPIN_LIMIT_NS, max_tasks_per_tile=1 << 16, clear_every_launch=False, revision=0)
+        mine.update(given)
+
     def __setattr__(self, name: str, value) -> None:
-        object.__setattr__(self, name, value)
+        self.__dict__[name] = value
         if name in SyncWords._DESCRIBED:
-            object.__setattr__(self, "revision", self.__dict__.get("revision", 0) + 1)
+            self.__dict__["revision"] = self.revision + 1
 
     def reset(self) -> None:
         for t in (self.locks, self.counter, self.barrier, self.arrivals, self.trace_comm_counter, self.trace_start_clock,

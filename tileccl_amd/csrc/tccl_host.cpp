@@ -143,6 +143,13 @@ PyObject* own(PyObject* o) {
 }
 
 bool int_attr(PyObject* o, PyObject* name, long long& out) {
+  PyObject** dict = _PyObject_GetDictPtr(o);  // signal words keep theirs there
+  PyObject* kept = dict && *dict ? PyDict_GetItemWithError(*dict, name) : nullptr;
+  if (kept) {
+    out = PyLong_AsLongLong(kept);
+    return !(out == -1 && PyErr_Occurred());
+  }
+  if (PyErr_Occurred()) return false;
   PyObject* v = PyObject_GetAttr(o, name);
   if (!v) return false;
   out = PyLong_AsLongLong(v);
@@ -410,14 +417,14 @@ PyObject* launch(Call* c, PyObject* const* tensors, int64_t* at, PyObject* alpha
   return tag;
 }
 
-// The tensors' addresses, and their layouts added to the hash; false if one has no address, which no call is for.
-bool addresses(PyObject* const* tensors, Py_ssize_t n, int64_t* at, size_t& hash) {
+// The tensors' addresses; false if one has none, or no sizes and strides, which no call is for.
+bool addresses(PyObject* const* tensors, Py_ssize_t n, int64_t* at) {
   try {
     for (Py_ssize_t i = 0; i < n; ++i) {
       const at::Tensor& t = THPVariable_Unpack(tensors[i]);
       if (t.layout() != c10::kStrided || t.unsafeGetTensorImpl()->is_nested()) return false;
       at[i] = (int64_t)(uintptr_t)t.data_ptr();
-      hash = Layout::hash(hash, t, (uintptr_t)at[i]);
+      t.strides();
     }
   } catch (...) {
     return false;
@@ -524,6 +531,22 @@ PyObject* table_add(Table* self, PyObject* object) {
   Py_RETURN_NONE;
 }
 
+// The call for these tensors, moved to the front; null if there is none.  A program that repeats one call finds it there.
+Call* find(Table* self, PyObject* key, PyObject* const* tensors, const int64_t* at, Py_ssize_t n) {
+  Call* first = self->order->front();
+  if (fits(first, tensors, at, n) && same_key(first->key, key)) return first;
+  size_t hash = key_hash(key);
+  for (Py_ssize_t i = 0; i < n; ++i) hash = Layout::hash(hash, THPVariable_Unpack(tensors[i]), (uintptr_t)at[i]);
+  const auto range = self->by_hash->equal_range(hash);
+  for (auto i = range.first; i != range.second; ++i) {
+    Call* c = *i->second;
+    if (!fits(c, tensors, at, n) || !same_key(c->key, key)) continue;
+    self->order->splice(self->order->begin(), *self->order, i->second);
+    return c;
+  }
+  return nullptr;
+}
+
 // launch(key, alpha, *tensors): the tag of the call that was issued, or None if there is none for these tensors.
 PyObject* table_launch(Table* self, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs < 3 || nargs > 2 + kMaxTensors || !PyTuple_Check(args[0])) {
@@ -534,27 +557,21 @@ PyObject* table_launch(Table* self, PyObject* const* args, Py_ssize_t nargs) {
     if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
   if (self->order->empty()) Py_RETURN_NONE;
   int64_t at[kMaxTensors];
-  size_t hash = key_hash(args[0]);
-  if (!addresses(args + 2, nargs - 2, at, hash)) Py_RETURN_NONE;
+  if (!addresses(args + 2, nargs - 2, at)) Py_RETURN_NONE;
   return guarded((PyObject*)nullptr, [&]() -> PyObject* {
-    const auto range = self->by_hash->equal_range(hash);
-    for (auto i = range.first; i != range.second; ++i) {
-      Call* c = *i->second;
-      if (!fits(c, args + 2, at, nargs - 2) || !same_key(c->key, args[0])) continue;
-      Reference held{(PyObject*)c};  // another thread may drop it from the table meanwhile
-      Py_INCREF(c);
-      self->order->splice(self->order->begin(), *self->order, i->second);
-      if (c->revision >= 0) {
-        long long now = 0;
-        if (!int_attr(c->words, sRevision, now)) return nullptr;
-        if (now != c->revision) {  // what the copied descriptor points at may be gone: the call is built again
-          drop(self, c);
-          Py_RETURN_NONE;
-        }
+    Call* c = find(self, args[0], args + 2, at, nargs - 2);
+    if (!c) Py_RETURN_NONE;
+    Reference held{(PyObject*)c};  // another thread may drop it from the table meanwhile
+    Py_INCREF(c);
+    if (c->revision >= 0) {
+      long long now = 0;
+      if (!int_attr(c->words, sRevision, now)) return nullptr;
+      if (now != c->revision) {  // what the copied descriptor points at may be gone: the call is built again
+        drop(self, c);
+        Py_RETURN_NONE;
       }
-      return launch(c, args + 2, at, args[1]);
     }
-    Py_RETURN_NONE;
+    return launch(c, args + 2, at, args[1]);
   });
 }
 

@@ -102,6 +102,7 @@ struct StreamGemm {
   // instructions with nothing to overlap them (176 x 1440 x 336, pushed to three peers: 8.5 -> 7.6 us).
   struct Signal {
     int tile;        // the plan tile under this tile
+    int word;        // and where its tiles are counted
     uint32_t tiles;  // tiles of it
     int32_t group;   // its TileGroup (group mode)
     u32x2 base;      // lane p: rank p's heap base
@@ -564,13 +565,14 @@ struct StreamGemm {
 
   TCCL_D Signal look_up(int row0, int col0) const {
     Signal s;
-    s.tile = 0;
+    s.tile = s.word = 0;
     s.tiles = 1;
     s.group = 0;
     s.base = u32x2{0, 0};
     if (a.push.world > 0) s.base = __builtin_amdgcn_raw_buffer_load_b64(window((int64_t)(uintptr_t)a.heap_bases), 8u * (uint32_t)(lane < a.push.world ? lane : 0), 0, 0);
     if (a.s.mode == kSignalNone) return s;
     s.tile = plan_tile(row0, col0);
+    s.word = arrival_word(s.tile, a.s.epoch, a.s.mode == kSignalTile);
     if (a.s.mode == kSignalGroup) s.group = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(window((int64_t)(uintptr_t)a.s.group_table), 4u * (uint32_t)s.tile, 0, 0);
     // Tiles of this plan tile: those of its rows and columns that lie inside the segment and N.
     const int pr = row0 / a.block_m * a.block_m, pc = col0 / a.block_n * a.block_n;
@@ -592,7 +594,7 @@ struct StreamGemm {
     if (threadIdx.x != 0) return;
     const uint32_t n = signal.tiles;
     // Counts to n - 1 and starts over by itself, so the word is zero again when the launch has ended.
-    const uint32_t before = n > 1 ? atomicInc(&a.arrivals[arrival_word(signal.tile, a.s.epoch, a.s.mode == kSignalTile)], n - 1) : 0u;
+    const uint32_t before = n > 1 ? atomicInc(&a.arrivals[signal.word], n - 1) : 0u;
     if (before != n - 1) return;
     if (a.s.mode == kSignalTile)
       tile_publish(a.s.locks, signal.tile, a.s.epoch);
