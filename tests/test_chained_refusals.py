@@ -51,4 +51,4 @@ def test_a_refused_call_allocates_nothing(lib, refused, match, schedule):
     for _ in range(2):
         with pytest.raises(ValueError, match=match):
             pattern.execute(shard, W, out, workspace)
-    assert heap.taken == [] and ctx._workspace_cache == {}
+    assert heap.taken == [] and not any(isinstance(v, torch.Tensor) for v in ctx._workspace_cache.values())

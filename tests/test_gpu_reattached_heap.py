@@ -70,3 +70,39 @@ def test_calls_and_words_go_with_the_heap(lib, kind):
         for h in old:
             h.cleanup()
         assert all(h.live_id == 0 for h in old)
+
+
+@pytest.mark.parametrize("kind", ["bulk_sync", "wg_specialized", "tile_group", "chained"])
+def test_the_old_heap_is_given_back(lib, kind):
+    """A pattern that has gone on to another heap holds nothing of the one before: its device memory is freed."""
+    import gc
+    import weakref
+
+    import tileccl_amd as tileccl
+    from tileccl_amd.memory.symmetric_heap import SymmetricHeap
+    from tileccl_amd.patterns import BulkSyncPattern, TileGroupPattern, WGSpecializedPattern
+    from tileccl_amd.patterns.chained_ag_gemm_rs import ChainedAGGemmRSPattern
+
+    made = {"bulk_sync": BulkSyncPattern, "wg_specialized": WGSpecializedPattern, "tile_group": TileGroupPattern,
+            "chained": ChainedAGGemmRSPattern}
+    (ctx,) = tileccl.init_local(world_size=1, heap_size=32 << 20)
+    pattern = made[kind](ctx)
+
+    def run():
+        A, B = put(ctx.heap, seeded((M, K), 1)), put(ctx.heap, seeded((K, N), 2, scale=K**-0.5))
+        out = ctx.heap.allocate_tensor((M, N), torch.float16)
+        for _ in range(2):
+            pattern.execute(A, B, out)
+        torch.cuda.synchronize()
+
+    run()
+    old = ctx.heap
+    arena = weakref.ref(old._arena)
+    new = SymmetricHeap(32 << 20, 0, 1)
+    ctx.attach_heap(new)
+    old.cleanup()
+    del old
+    run()
+    gc.collect()
+    assert arena() is None
+    new.cleanup()

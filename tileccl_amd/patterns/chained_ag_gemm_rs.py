@@ -63,7 +63,6 @@ class ChainedAGGemmRSPattern:
         # The GEMM + scatter stages reuse the all-scatter pattern's plan and signal words.
         self._stage = _SCHEDULES[schedule](ctx, BLOCK_M=BLOCK_M, BLOCK_N=BLOCK_N, BLOCK_K=BLOCK_K)
         self._last_sync: _launch.SyncWords | None = None
-        self._calls = _launch.call_table({})
 
     def execute(
         self,
@@ -76,17 +75,18 @@ class ChainedAGGemmRSPattern:
         own = gathered_workspace is None
         if own and input_shard.ndim == W.ndim == 2:
             gathered_workspace = self.ctx.kept_workspace(_GATHERED, input_shard.shape[0], W.shape[0], dtype=input_shard.dtype)
-        key = (heap.live_id, self.BLOCK_M, self.BLOCK_N, *self._stage._settings())
+        calls = _launch.call_table(self._stage._sync)
+        key = ("chained", self.schedule, heap.live_id, self.BLOCK_M, self.BLOCK_N, *self._stage._settings())
         ran = None
         if gathered_workspace is not None:
-            ran = self._calls.launch(key, None, gathered_workspace, W, output, input_shard)
+            ran = calls.launch(key, None, gathered_workspace, W, output, input_shard)
         if ran is None:
             # Before anything is allocated for the call (the heap gives nothing back): the ranks' heaps stay in step.
             self._check(input_shard, W, output, gathered_workspace, heap)
             if own:
                 gathered_workspace = self.ctx.workspace(_GATHERED, input_shard.shape[0], W.shape[0], dtype=input_shard.dtype)
-            self._bind(key, input_shard, W, output, gathered_workspace, heap)
-            ran = _launch.issue(self._calls, key, None, gathered_workspace, W, output, input_shard)
+            self._bind(calls, key, input_shard, W, output, gathered_workspace, heap)
+            ran = _launch.issue(calls, key, None, gathered_workspace, W, output, input_shard)
         self._last_sync = None if ran is True else ran
         return output
 
@@ -113,7 +113,7 @@ class ChainedAGGemmRSPattern:
         if gathered_workspace is not None and (tuple(gathered_workspace.shape) != (M, K) or gathered_workspace.dtype != input_shard.dtype):
             raise ValueError(f"gathered_workspace must be ({M}, {K}) of {input_shard.dtype}")
 
-    def _bind(self, key, input_shard, W, output, gathered_workspace, heap) -> None:
+    def _bind(self, calls, key, input_shard, W, output, gathered_workspace, heap) -> None:
         """Build the descriptors of a call on tensors of these layouts."""
         M, K_shard = input_shard.shape
         N = W.shape[1]
@@ -127,7 +127,7 @@ class ChainedAGGemmRSPattern:
         words = self._stage._sync_words(M, N, output)
         variant = {_lib.S0_BULK: "s0", _lib.S1_TILE: "s1", _lib.S2_TILEGROUP: "s2"}[self._stage.variant]
         _launch.bind(
-            self._calls, key, (gathered_workspace, W, output, input_shard), _lib.load().tccl_chained_ag_gemm_rs,
+            calls, key, (gathered_workspace, W, output, input_shard), _lib.load().tccl_chained_ag_gemm_rs,
             (gemm, (3, 0), _launch._row_major(input_shard, "input_shard"), K_shard, _launch.view_of(heap), _launch.SYNC, transport,
              self._stage.variant),
             f"tccl_chained_ag_gemm_rs[{self.schedule}]", gemm=gemm, plan=plan, words=words, variant=variant, tag=words, c=(2, 0),

@@ -43,10 +43,10 @@ class _HipAllScatterPattern(Pattern):
         # Signal words are cut from the heap, which never gives memory back, and a pattern named
         # by a string is instantiated anew on every call (ops._resolve_pattern_impl, as in the
         # reference, ops.py:1289-1296): they are therefore kept with the context, next to its
-        # workspaces, and shared by every pattern instance of the same kind and tiling.
+        # workspaces, and shared by every pattern instance of the same kind and tiling.  So are the bound
+        # calls, which hold on to those words: both go when another heap is attached.
         cache = getattr(ctx, "_workspace_cache", None)
         self._sync: dict[tuple, _launch.SyncWords] = cache if isinstance(cache, dict) else {}
-        self._calls = _launch.call_table({})
 
     # -- hooks -------------------------------------------------------------------------
     def _sync_words(self, M: int, N: int, C_out: torch.Tensor) -> _launch.SyncWords | None:
@@ -78,11 +78,13 @@ class _HipAllScatterPattern(Pattern):
                 "C must live in the symmetric heap when world_size > 1: the scatter writes it at the "
                 "same offset in every peer's slice"
             )
-        key = (heap.live_id, *self._settings(), spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset)
-        ran = self._calls.launch(key, None, A, B, C_out)
+        calls = _launch.call_table(self._sync)
+        key = (type(self), heap.live_id, *self._settings(), spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim,
+               spec.scatter_dst_col_offset)
+        ran = calls.launch(key, None, A, B, C_out)
         if ran is None:
-            self._bind(self._calls, key, (A, B, C_out), (2, 0), spec, heap)
-            ran = _launch.issue(self._calls, key, None, A, B, C_out)
+            self._bind(calls, key, (A, B, C_out), (2, 0), spec, heap)
+            ran = _launch.issue(calls, key, None, A, B, C_out)
         self._ran(ran)
 
     def _ran(self, words: "_launch.SyncWords | bool") -> None:
