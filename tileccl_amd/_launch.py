@@ -94,7 +94,11 @@ _PACKED_LIMIT = 8
 
 def _pack_buffer(t: torch.Tensor, rows: int, cols: int, role: str, stream: int) -> torch.Tensor:
     """A dense ``rows x cols`` buffer, kept per (role, shape, dtype, stream) and reused by the next call with that key, which
-    the stream orders behind this one's GEMM, unless a descriptor that has not been dropped yet still points at it."""
+    the stream orders behind this one's GEMM, unless a descriptor that has not been dropped yet still points at it.  A call that
+    is being recorded into a graph takes one from the graph's memory: a kept one might be dropped, and its memory be someone
+    else's, while the graph goes on writing it."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty((rows, cols), dtype=t.dtype, device=t.device)
     key = (role, rows, cols, t.dtype, t.device, stream)
     out = _PACKED.pop(key, None)
     if out is not None and sys.getrefcount(out) > 2:  # this name and the call's argument
