@@ -98,7 +98,8 @@ typedef struct tccl_gemm_desc {
   int32_t column_shards;
 } tccl_gemm_desc;
 
-/* tccl_gemm_reducescatter, variants S1 / S2 on the 256 x 256 tile with shards of whole tiles:
+/* tccl_gemm_reducescatter, variants S1 / S2 where the sums are made in the GEMM's epilogue (shards of whole 256 x 256
+ * tiles; small outputs with TCCL_GEMM_ARRIVALS; 128 x 128 tiles that wait for their peers, at most one per CU):
  * the partial of the rows this rank owns stays in the accumulators, takes the peers' partials
  * in the GEMM epilogue and is never stored to gemm->C (those rows of C keep their old
  * contents); the output is bit-identical to storing and reducing.  Ignored elsewhere.

@@ -60,8 +60,9 @@ def test_gemm_alone_e4m3(lib, M, N, K, layout):
 @pytest.mark.parametrize("world,layout", [(2, "kn"), (3, "nk")])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_all_gather_pushes_pulls_and_publishes(lib, M, N, K, world, layout, variant):
-    """Three launches in a row: the arrival counters start over by themselves, the published words reach every
-    launch's number, and a peer that waits for them (the second rank, pulling) is let through."""
+    """Three launches in a row: the arrival counters start over by themselves and the published words reach every launch's
+    number.  The peers are resident: their words are preset and they launch nothing.  (Waits for words that another launch
+    writes: ``test_gpu_stream_live.py``.)"""
     from tileccl_amd.v2 import FusedGemmAllGather, SymmetricHeap
 
     heaps = SymmetricHeap.create_all(128 << 20, world)

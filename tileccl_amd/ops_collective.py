@@ -229,11 +229,12 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     shape ``(world, M, N/world)``, fp32, at the same offset of every rank's slice; block
     ``q`` is ``A @ B[:, q's columns]`` (the reference's rank-major column-shard layout,
     ops.py:315,646).  Stacked, the blocks are the row shards of a ``(world*M, N/world)``
-    matrix, so the operation is one launch of the fused GEMM -> ReduceScatter kernel: the
-    GEMM produces row block ``q`` from ``B``'s column block ``q``, block ``rank`` is reduced
-    with the peers' partials as its tiles finish, and (``own_rows_in_registers``, the default)
-    that block never leaves the accumulators as a partial, so its part of the workspace is not
-    written.  ``variant`` picks the schedule (``"s0"`` bulk, ``"s1"`` tile by tile, ``"s2"``
+    matrix, so the operation is a GEMM -> ReduceScatter: the
+    GEMM produces row block ``q`` from ``B``'s column block ``q``, block ``rank`` is summed
+    with the peers' partials.  On 256 x 256 tiles and in the streaming kernel that is one launch, which
+    sums each tile as it finishes, and (``own_rows_in_registers``, the default)
+    block ``rank`` never leaves the accumulators as a partial: its part of the workspace is not
+    written.  On 128 x 128 tiles with the peers' partials resident the sums are a second launch.  ``variant`` picks the schedule (``"s0"`` bulk, ``"s1"`` tile by tile, ``"s2"``
     TileGroup).  ``emulate_peer`` (single-GPU emulation) also writes the other ranks' outputs
     into their slices.
 
@@ -250,8 +251,8 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     have made the same number of calls.
     ``implementation`` is accepted for signature parity; there is one implementation here.
     When ``M`` is not a multiple of the 128-row plan tile there are no signals: the peers' partials
-    are taken to be there, in one launch where the streaming kernel is the quicker one and
-    otherwise with one GEMM per column block and the bulk reduction.
+    are taken to be there.  The streaming kernel sums in its epilogue; otherwise one GEMM launch for all column
+    blocks, or one per block where each fills the device by itself, and the bulk reduction.
     """
     if implementation not in ("auto", "device", "hip"):
         raise ValueError(f"unsupported gemm_reducescatter implementation {implementation!r}")

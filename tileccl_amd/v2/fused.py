@@ -213,8 +213,8 @@ class FusedGemmReduceScatter(_FusedBase):
     fp32.  With ``emulate_peer`` the launch also performs the other owners' reductions into
     their slices, i.e. the whole two-rank operation on one GPU.
 
-    ``own_rows_in_registers``: in the one-launch variants on the 256 x 256 tile (shards of
-    whole tiles) the rows this rank owns never leave the accumulators as a partial: the peers'
+    ``own_rows_in_registers``: where a one-launch variant sums in the GEMM's epilogue (shards of
+    whole 256 x 256 tiles; small outputs) the rows this rank owns never leave the accumulators as a partial: the peers'
     partials are added in the GEMM epilogue.  ``out`` is bit-identical; those rows of
     ``partial`` keep whatever they held.  Ignored where it does not apply.
     """
