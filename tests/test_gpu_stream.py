@@ -204,3 +204,43 @@ def test_launches_of_different_tiles_on_two_streams_leave_no_counts(lib):
         assert len(words) == 1 and words[0].lock_epoch == 60 and not words[0].arrivals.any()
     finally:
         ctx.heap.cleanup()
+
+
+@pytest.mark.parametrize("pattern", ["wg_specialized", "tile_group"])
+def test_words_made_on_a_busy_stream_are_clear_for_another(lib, pattern):
+    """The first call of a shape makes its words, on a stream that is still at work; the next call comes on another one.  The
+    memory that the words are made in is not clear by itself."""
+    import tileccl_amd as tileccl
+    from tileccl_amd import _lib
+
+    ctx = tileccl.init_local(world_size=1, heap_size=64 << 20)[0]
+    try:
+        M, N, K = 300, 520, 264
+        A, B = seeded((M, K), 1), seeded((K, N), 2, scale=K**-0.5)
+        a, b, outs = into_heap(ctx.heap, A), into_heap(ctx.heap, B), [ctx.zeros(M, N, dtype=torch.float16) for _ in range(2)]
+        ctx.heap.get_peer_buffer(0)[ctx.heap.bytes_allocated:].fill_(5)
+        busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+        big = torch.randn(4096, 4096, device="cuda", dtype=torch.float16)
+        torch.cuda.synchronize()
+        tiles = 3 * 5
+        with torch.cuda.stream(busy):
+            dirty = [torch.full((tiles * _lib.ARRIVAL_STRIDE,), 5, dtype=torch.int32, device="cuda") for _ in range(4)]
+            del dirty
+            for _ in range(200):  # some 20 ms
+                big @ big
+            tileccl.ops.gemm_allscatter(a, b, outs[0], ctx=ctx, pattern=pattern)
+        with torch.cuda.stream(other):
+            tileccl.ops.gemm_allscatter(a, b, outs[1], ctx=ctx, pattern=pattern)
+            (words,) = [w for k, w in ctx._workspace_cache.items() if isinstance(k, tuple) and k[0] == "tileccl_amd.sync"]
+            assert not words.arrivals.any()
+            other.synchronize()
+            assert_gemm_close(outs[1], A.float() @ B.float(), tight=0.004)
+        torch.cuda.synchronize()
+        assert_gemm_close(outs[0], A.float() @ B.float(), tight=0.004)
+        assert not words.arrivals.any()
+        if pattern == "wg_specialized":
+            assert set(words.locks.tolist()) <= {1, 2}
+        else:
+            assert words.counter.tolist() == [2 * t for t in words.host_plan.tile_counts()]
+    finally:
+        ctx.heap.cleanup()

@@ -431,10 +431,23 @@ class SyncWords:
         self.epoch += 1
         return self.epoch
 
+    @classmethod
+    def made(cls, host_plan=None, **words) -> "SyncWords":
+        """Words cleared on the current stream (``words``), with what goes with them.  Another stream's launch may use them
+        next: they are clear for every stream when this returns (but for words made while a stream is capturing)."""
+        made = cls(host_plan=host_plan, **words)
+        made.tile_arrivals()
+        if host_plan is not None:
+            made.plan = DevicePlan.upload(host_plan)  # copies from host memory, which wait for the stream
+        elif not torch.cuda.is_current_stream_capturing():
+            torch.cuda.current_stream().synchronize()
+        return made
+
     def tile_arrivals(self) -> torch.Tensor:
         """The arrival counters, made on first use for every plan tile these words have signals for."""
         if self.arrivals is None:
-            tiles = max(int(t.numel()) for t in (self.locks, self.plan.group_table if self.plan is not None else None) if t is not None)
+            plan = self.plan or self.host_plan
+            tiles = max(int(t.numel()) for t in (self.locks, plan.group_table if plan is not None else None) if t is not None)
             self.arrivals_from_capture = torch.cuda.is_current_stream_capturing()
             self.arrivals = torch.zeros(tiles * _lib.ARRIVAL_STRIDE, dtype=torch.int32, device="cuda:0")
         return self.arrivals

@@ -216,7 +216,7 @@ def _reduce_scatter_words(ctx, world: int, M: int, cols: int):
                  (("counter", plan.n_groups), ("barrier", plan.n_groups), ("locks", int(plan.group_table.numel())))}
         for t in words.values():
             t.zero_()
-        cache[key] = _launch.SyncWords(plan=_launch.DevicePlan.upload(plan), host_plan=plan, **words)
+        cache[key] = _launch.SyncWords.made(host_plan=plan, **words)
     return cache[key]
 
 

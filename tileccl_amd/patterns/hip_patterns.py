@@ -161,7 +161,7 @@ class WGSpecializedPattern(_HipAllScatterPattern):
             heap = self.ctx.require_heap()
             locks = heap.allocate_tensor((tiles,), torch.int32)
             locks.zero_()
-            words = self._sync[key] = _launch.SyncWords(locks=locks)
+            words = self._sync[key] = _launch.SyncWords.made(locks=locks)
         return words
 
 
@@ -225,9 +225,6 @@ class TileGroupPattern(_HipAllScatterPattern):
             barrier = heap.allocate_tensor((plan.n_groups,), torch.int32)
             counter.zero_()
             barrier.zero_()
-            words = self._sync[key] = _launch.SyncWords(
-                counter=counter, barrier=barrier, plan=_launch.DevicePlan.upload(plan)
-            )
-            words.host_plan = plan
+            words = self._sync[key] = _launch.SyncWords.made(host_plan=plan, counter=counter, barrier=barrier)
         self.last_plan = words.host_plan
         return words

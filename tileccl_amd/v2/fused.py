@@ -103,15 +103,13 @@ class _FusedBase:
         self.signals.reset()
         tiles = int(self.plan.group_table.numel())
         self.locks = self.heap.allocate_signal_buffer(tiles)
-        self.words = _launch.SyncWords(
+        self.words = _launch.SyncWords.made(
             locks=self.locks,
             counter=self.signals.counter,
             barrier=self.signals.barrier,
-            plan=_launch.DevicePlan.upload(self.plan),
             host_plan=self.plan,
             spin_limit_ns=self.spin_limit_ns,
         )
-        self.words.tile_arrivals()
         if self.trace:
             self.words.trace_comm_counter = self.signals.trace_comm_counter
             self.words.trace_start_clock = self.signals.trace_start_clock
