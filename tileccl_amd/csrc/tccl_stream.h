@@ -287,11 +287,9 @@ struct StreamGemm {
     }
   }
 
-  TCCL_D void run(int slot) {
-    if (!a.pull.active || slot < a.pull.first)
-      tile(slot);
-    else if (pull_ready(slot))
-      pull_share(slot);
+  // Workgroups behind the tiles (launches that pull).
+  TCCL_D void pull(int slot) const {
+    if (pull_ready(slot)) pull_share(slot);
   }
 
   // The units of a block that workgroup `slot` pulls.
