@@ -547,7 +547,7 @@ struct TileChoice {
 
 // The kernel for `segs` row blocks of `seg_rows` rows in a launch that carries nothing but pushes.  Measured, bf16, on 40
 // seeded shapes of 100 .. 2200 tiles of 128 x 128, row-major and k-major B: the choice is the quickest kernel or within
-// 10 % of it for 74 of the 80, within 17 % for all, 2 % off on average; the 128-tile kernel alone would be 21 % off.
+// 10 % of it for 76 of the 80, within 18 % for all, 2 % off on average; the 128-tile kernel alone would be 22 % off.
 // What keeps to the old rule: tiles named by the caller, plan tiles other than 128 x 128, workgroup counts.
 TileChoice choose_tiles(const tccl_gemm_desc* d, int64_t seg_rows, int64_t segs, bool allow256, bool pushes, const tccl_device_info& dev) {
   if (d->in_dtype == TCCL_F8E4M3) return {kTiles256, 0};
@@ -887,10 +887,10 @@ bool gather_in_place(const tccl_gemm_desc* d, const tccl_device_info& dev, int k
 // ---- streaming path (tccl_stream.h) -------------------------------------------------------------
 // Estimated time of a launch, in us.  A tile's operands pass its CU's vector memory path once, at a rate (KB/us) that
 // depends on its shape; a tile's sums take the last term.  The rates measured with 256 tiles, k-major and row-major B, are 72
-// and 33, 98 and 74, 97 and 79, 99 and 89, 73 and 49; the constants are those of the kernel's first form and lower, and as only
+// and 33, 97 and 73, 97 and 78, 99 and 89, 73 and 50; the constants are those of the kernel's first form and lower, and as only
 // their ratios matter among the shapes, they choose the quickest shape or kernel, or one within 10 %, for 39 of 40 forms
-// measured (20 shapes of 1 .. 1024 rows, both layouts of B; 32 x 2048 x 4096 row-major: 17 % off) and 17 of 20 of e4m3 (row-major
-// B with 64 x 64 tiles, 12 % off, and 64 x 4096 x 4096, 21 %).  Neither the layout of B nor the variant enters, so that all
+// measured (20 shapes of 1 .. 1024 rows, both layouts of B; 32 x 2048 x 4096 row-major: 18 % off) and 19 of 20 of e4m3
+// (64 x 4096 x 4096 row-major: 14 % off).  Neither the layout of B nor the variant enters, so that all
 // of them add the products up in the same order: the same bits.
 struct StreamCost {
   double rate, sums;
