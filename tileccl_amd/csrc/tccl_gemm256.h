@@ -37,12 +37,25 @@
 // faster.  fp8 inputs use v_mfma_scale_f32_16x16x128_f8f6f4 for the same reason (3.5 against 4.0 PFLOP/s
 // sustained on N(0,1) e4m3 values; the fp8 GEMM, further from that bound, gained 2 %).
 //
-// Pipeline: LDS holds two stages.  The loads of step kt+1 are issued, woven between the
-// first MFMAs of step kt, into the stage step kt-1 has left.  The step's one barrier
-// (`s_waitcnt vmcnt(0) lgkmcnt(0)` + `s_barrier`) sits two items before the step's end: the
-// stage being read is finished with, the next one has landed, and the last items already fetch
-// the next step's first operands (see k_step16 / k_step8).
+// Pipeline.  LDS holds two stages, each of which is filled and left in quarters (the half of A of the waves' upper
+// 64 rows, that of their lower 64 rows, two halves of B).  A K step is four phases; in each a wavefront first moves
+// data (two global -> LDS loads, the phase's LDS reads) and then multiplies (256 clocks of MFMAs), with a
+// barrier behind either, and the wavefronts 4..7 run one such slot behind the wavefronts 0..3: of a SIMD's two
+// wavefronts one multiplies while the other moves data.  A quarter of a stage is refilled as soon as both sides have
+// read it, with the operands of two steps ahead, so a load has three quarters of a step to a step and a quarter to land and
+// the waits on it are counted, never vmcnt(0) (k_step).  What it is for: with all eight wavefronts in step the issue of
+// the loads (a wavefront is held while the address unit takes in a load, 16 clocks per KiB) and the MFMAs took
+// turns; at 8192 x 4096 x 4096 the loop without its loads ran a quarter faster.  Measured, bf16, k-major B, in turn with
+// the loop of one barrier per step that this one replaced: 8192 x 4096 x 4096 210 -> 190 us, with a push to one peer
+// 219 -> 197; 8192 x 4096 x 2048 with the push 121 -> 109; 4096 x 4096 x 1024 with the push 33.8 -> 33.5.  What bounds it
+// now is power: the matrix pipes are busy 69 % of the clocks (62 % before) at 1.82 GHz (1.89).
 //
+// Launches with a background transfer (a pull) keep a loop of one barrier per step (step_pulling): eight items, all eight
+// wavefronts in step, the next step's loads in the first four items, `s_waitcnt vmcnt(0)` + barrier before the last.  There the
+// transfer's bookkeeping, loads and stores fall into the slack of the older wavefronts; between the phases' barriers every
+// clock of it holds up both sides (4096 x 4096 x 1024, pushing and pulling: 41.9 us at best with the phases, four splits of the
+// transfer over them tried, 40.4 with the items; 4096 x 4096 x 2048 with its inputs gathered: 64.4 and 62.6).
+
 // The swapped-operand MFMA and the slab-wise epilogue are those of tccl_gemm.h.
 //
 // A macro tile covers (256/block_m) x (256/block_n) plan tiles; when it is stored, each of
@@ -61,7 +74,7 @@ constexpr int kARow256 = 128;                              // A: bytes per row o
 constexpr int kAStage256 = kMacro * kARow256;              // 32 768 B
 constexpr int kBStage256 = 32768;                          // B: (128 / element size) k rows of 256 columns
 constexpr int kStage256 = kAStage256 + kBStage256;         // A then B
-constexpr int kLds256 = 2 * kStage256;                     // two stages: 131 072 B (two arrays)
+constexpr int kLds256 = 2 * kStage256;                     // two stages: 131 072 B
 
 struct Macro {
   int rows, cols;        // macro tile grid
@@ -104,9 +117,8 @@ struct ReduceArgs {
 // A peer's block is cut into pieces of kPieceUnits units of 16 bytes; pulling wavefront w of
 // the launch (the kPullWaves older wavefronts of every workgroup, see below) owns pieces w,
 // w + W, w + 2W, ... (W = pulling wavefronts in the grid), so at any moment the grid sweeps a
-// contiguous stretch.  In every K step, behind the step's operand loads, such a wavefront
-// requests its next piece into registers; the step's barrier waits for this wave's loads
-// anyway, and mid-way through the following step the piece is stored.  A
+// contiguous stretch.  Once per K step such a wavefront stores the piece it requested a step before and
+// requests its next one, global -> LDS like the operands, into landing bytes of its own.  A
 // piece is fetched only once
 // the TileGroups covering its rows are complete on the peer (counter[g] >= epoch *
 // tile_counts[g], the readiness rule of tileccl_v2/signal.py:43-66); that is found out by
@@ -162,16 +174,13 @@ struct GatherArgs {
   int64_t ld_shard;    // elements
   int k_shard;         // columns per shard
 };
-constexpr int kBgWordBytes = 8 * 256;                   // a fetched counter word per wavefront (64 lanes x 4 B)
-// Of a SIMD's two wavefronts the older one (wavefronts 0..3 of the workgroup) wins the matrix
-// pipe and reaches each K step's barrier early, while the younger one runs alone for the rest of
-// the step; scalar work of the younger one therefore delays the step, that of the older one is
-// covered by the younger one's MFMAs.  The background pull is carried by the older wavefronts
-// alone, two 16-byte units per lane and step, so that its bookkeeping runs once per 2 KiB and
-// only where it is covered.
+// Of a SIMD's two wavefronts the older one (wavefronts 0..3 of the workgroup) wins the matrix pipe and reaches each K step's
+// barrier early, while the younger one runs alone for the rest of the step; what the older one does besides is covered by the
+// younger one's MFMAs.  The pull is carried by the older wavefronts alone, two 16-byte units per lane and step.
 constexpr int kPullWaves = 4;                           // wavefronts of a workgroup that pull
 constexpr int kPullLoads = 2;                           // 16-byte units per lane and piece
 constexpr int kPieceUnits = 64 * kPullLoads;            // units per piece
+constexpr int kBgLandingBytes = kPullWaves * (16 * kPieceUnits + 256);  // per pulling wavefront: a piece, a counter word per lane
 
 TCCL_HD TileCoord macro_coords(int id, const Macro& m) {
   const int per_band = m.rows_per_band * m.cols;
@@ -209,7 +218,8 @@ TCCL_D T late_kernarg(int offset) {
 // an (N, K) weight is: the reference's kernels take any strides, kernels/gemm.py:139-151).  The B
 // stage then has the A stage's layout (256 n rows of 128 bytes, same swizzle) and is read with
 // ds_read_b128 like A: no transposing reads.
-template <typename InT, typename OutT, bool kWithReduce = false, bool kGatherA = false, bool kBKMajor = false>
+// kPull: the launch may carry a background transfer; it runs the K loop of one barrier per step (step_pulling).
+template <typename InT, typename OutT, bool kWithReduce = false, bool kGatherA = false, bool kBKMajor = false, bool kPull = false>
 struct Gemm256 {
   typedef typename Mfma<InT>::Vec Vec;
   static constexpr int kEszIn = sizeof(InT);
@@ -228,11 +238,9 @@ struct Gemm256 {
   const int push_offset;    // byte offset of a PushArgs in the kernel arguments; < 0: no push
   const int reduce_offset;  // byte offset of a ReduceArgs in the kernel arguments; < 0: none
   const int gather_offset;  // byte offset of a GatherArgs in the kernel arguments (kGatherA only)
-  // The two pipeline stages are two separate __shared__ arrays: loads that write LDS directly
-  // are tracked per LDS variable, so a read of one stage need not wait for a load into the other.
-  char* lds;   // stage 0 (also the epilogue's staging area)
+  char* lds;   // stage 0 (also the epilogue's staging area), stage 1 behind it
   char* lds1;  // stage 1
-  char* bgw;   // landing words of the background transfer's counter fetches
+  char* bgw;   // landing bytes of the background transfer's pieces and counter fetches
   const int tid, lane, wave, wm, wn;
   // A per-lane value the optimiser must treat as new at this point (blocks hoisting of what is derived from it).
   static TCCL_D int fresh(int v) {
@@ -266,25 +274,55 @@ struct Gemm256 {
   typedef short s16x8 __attribute__((ext_vector_type(8)));
   typedef __attribute__((address_space(3))) s16x4 LdsQuad;
 
-  // Where this lane's four A pieces and four B pieces of a K step come from (byte offsets
-  // into the buffer resources at K step 0).  Piece i of wave w fills
-  //   A rows 8*(4w+i) .. +7      (lane l: row + l/8, slot l%8)
-  //   B k rows 2*(4w+i), +1      (lane l: k row + l/32, slot l%32)            16-bit inputs
-  //   B k rows 4*(4w+i) .. +3    (lane l: k row + l/16, slot l%16)            fp8 inputs
+  // Where a wavefront's pieces (1 KiB, one load) of a K step come from.  Operand halves are loaded one at a time, two pieces
+  // per wavefront:
+  //   A half h: rows 128 g + 64 h .. + 63, g = 0, 1 (what the wavefronts wm = g read in two of the four phases)
+  //   B half h: the first or second half of the step's k rows; k-major: columns 64 g + 32 h .. + 31, g = 0 .. 3.
+  // a_row() and b_row() give a piece's first row; lane l fetches row + l / 8, slot l % 8 of it (row-major B, 16-bit: k row +
+  // l / 32, slot l % 32; fp8: k row + l / 16, slot l % 16).
+  typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
   struct Source {
-    __amdgpu_buffer_rsrc_t a, b;
-    // Pieces 0 and 1 per lane; pieces 2 and 3 lie a fixed distance behind them (pair_a, pair_b), which is
-    // added where a load is issued: half the registers through the K loop.
-    uint32_t off_a[2], off_b[2];
-    uint32_t pair_a, pair_b;
+    Words4 a, b;                  // buffer descriptors
+    uint32_t off_a[2], off_b[2];  // this lane's byte offsets in the two pieces of half 0, K step 0
+    uint32_t half_a, half_b;      // distance of half 1
     uint32_t step_a, step_b;
     // kGatherA: `a` is the window onto the shard that holds K steps [kt_base, kt_switch)
     int kt_base, kt_switch, row0;
   };
+  static TCCL_D Words4 descriptor(const void* p, uint32_t bytes) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    Words4 d;
+    d[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    d[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
+    d[2] = __builtin_amdgcn_readfirstlane(bytes);
+    d[3] = 0x00020000u;
+    return d;
+  }
+  // 16 bytes per lane, global -> LDS, lane l's to `to` + 16 l.  Written out because the compiler makes every later read of
+  // an LDS array wait for all loads into it, whichever part they go to; the waits are k_step's own.  Bytes past the
+  // descriptor's end (scalar offset included) read as zero.  A load that reads M0 wants an instruction between it and
+  // the write of M0.  Every global -> LDS load of this kernel sets M0 itself.
+  static TCCL_D void dma16(char* to, Words4 from, uint32_t lane_off, uint32_t off) {
+    const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(lane_off), "s"(from), "s"(off) : "memory");
+  }
+  // The same past the caches (what a peer has written), 16 and 4 bytes per lane.
+  static TCCL_D void dma16_coherent(char* to, Words4 from, uint32_t lane_off) {
+    const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
+  }
+  static TCCL_D void dma4_coherent(char* to, Words4 from, uint32_t lane_off) {
+    const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
+  }
+  template <int kLeft>
+  static TCCL_D void wait_loads() {  // until at most kLeft of this wavefront's vector memory operations are under way
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLeft) : "memory");
+  }
   typedef const __attribute__((address_space(4))) GatherArgs* GatherPtr;
 
   // Point `s.a` at the shard that holds K step kt (kGatherA).  Steps past K stay on the last
-  // shard: their chunks are redirected past the end of the window by issue_a and read as zero.
+  // shard: their chunks are redirected past the end of the window by mask() and read as zero.
   TCCL_D void select_shard(Source& s, int kt) const {
     const GatherPtr ga = late_kernarg_ptr<GatherArgs>(gather_offset);
     const int per_shard = ga->k_shard / kStepK;
@@ -292,8 +330,7 @@ struct Gemm256 {
     if (p >= ga->world) p = ga->world - 1;
     const int64_t base = (int64_t)(uintptr_t)ga->shard + (table(ga->heap_bases, p) - table(ga->heap_bases, ga->rank)) +
                          (int64_t)s.row0 * ga->ld_shard * kEszIn;
-    s.a = __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)base, 0,
-                                            clamp_u32(((int64_t)(g.M - 1 - s.row0) * ga->ld_shard + ga->k_shard) * kEszIn), 0x00020000);
+    s.a = descriptor((const void*)(uintptr_t)base, clamp_u32(((int64_t)(g.M - 1 - s.row0) * ga->ld_shard + ga->k_shard) * kEszIn));
     s.kt_base = p * per_shard;
     s.kt_switch = p + 1 < ga->world ? (p + 1) * per_shard : 0x7fffffff;
   }
@@ -303,7 +340,15 @@ struct Gemm256 {
       if (kt >= s.kt_switch) select_shard(s, kt);
   }
 
-  static TCCL_D uint32_t clamp_u32(int64_t v) { return v > 0xffffffffll ? 0xffffffffu : (v < 0 ? 0u : (uint32_t)v); }
+  // (Less than kDeadOffset: an offset of that size is past the end of every window.)
+  static constexpr uint32_t kDeadOffset = 0xfffffff0u;
+  static TCCL_D uint32_t clamp_u32(int64_t v) { return v > 0xffffff00ll ? 0xffffff00u : (v < 0 ? 0u : (uint32_t)v); }
+
+  TCCL_D int a_row(int h, int i) const { return (wave >> 2) * 128 + h * 64 + (wave & 3) * 16 + 8 * i; }
+  TCCL_D int b_row(int h, int i) const {
+    if constexpr (kBKMajor) return (wave >> 1) * 64 + h * 32 + (wave & 1) * 16 + 8 * i;
+    return h * (kStepK / 2) + (2 * wave + i) * kBRowsPerPiece;
+  }
 
   TCCL_D Source make_source(int row0, int col0) const {
     constexpr int kEsz = sizeof(InT);
@@ -316,39 +361,34 @@ struct Gemm256 {
     const OperandOrigin o = operand_origin(g, row0, col0);
     const InT* A = (const InT*)g.A + (int64_t)o.a_row * g.lda;
     const InT* B = (const InT*)g.B + (kBKMajor ? (int64_t)o.b_col * g.ldb : (int64_t)o.b_col);
-    s.a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(((int64_t)(o.a_rows - 1 - o.a_row) * g.lda + g.K) * kEsz), 0x00020000);
+    s.a = descriptor(A, clamp_u32(((int64_t)(o.a_rows - 1 - o.a_row) * g.lda + g.K) * kEsz));
     if constexpr (kBKMajor)
-      s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K) * kEsz), 0x00020000);
+      s.b = descriptor(B, clamp_u32(((int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K) * kEsz));
     else
-      s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(((int64_t)(g.K - 1 - g.b_short) * g.ldb + (o.b_cols - o.b_col)) * kEsz), 0x00020000);
+      s.b = descriptor(B, clamp_u32(((int64_t)(g.K - 1 - g.b_short) * g.ldb + (o.b_cols - o.b_col)) * kEsz));
+    int64_t lda = g.lda;
+    if constexpr (kGatherA) lda = late_kernarg_ptr<GatherArgs>(gather_offset)->ld_shard;
+    // Half 1 lies a whole number of the swizzles' periods further on (rows: (row >> 1) & 7; k rows: k & 3 and bit 3,
+    // fp8 k & 7 and bit 4, which the wavefront alone decides): one lane offset serves both.
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int row = 8 * (4 * wave + i) + (lane >> 3);
+      const int row = a_row(0, i) + (lane >> 3);
       const int kc = (lane & 7) ^ ((row >> 1) & 7);
-      int64_t lda = g.lda;
-      if constexpr (kGatherA) lda = late_kernarg_ptr<GatherArgs>(gather_offset)->ld_shard;
       s.off_a[i] = (uint32_t)(row * lda * kEsz + kc * 16);
       if constexpr (kBKMajor) {
-        s.off_b[i] = (uint32_t)(row * g.ldb * kEsz + kc * 16);
+        s.off_b[i] = (uint32_t)((b_row(0, i) + (lane >> 3)) * g.ldb * kEsz + kc * 16);
       } else if constexpr (kFp8) {
-        const int k = 4 * (4 * wave + i) + (lane >> 4);
+        const int k = b_row(0, i) + (lane >> 4);
         const int c = (lane & 15) ^ (2 * (k & 7)) ^ ((k >> 4) & 1);
         s.off_b[i] = (uint32_t)(k * g.ldb * kEsz + c * 16);
       } else {
-        const int k = 2 * (4 * wave + i) + (lane >> 5);
+        const int k = b_row(0, i) + (lane >> 5);
         const int c = (lane & 31) ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1));
         s.off_b[i] = (uint32_t)(k * g.ldb * kEsz + c * 16);
       }
     }
-    // Piece i + 2 covers rows (k rows) 16 (2 * kBRowsPerPiece) further on; the swizzle terms repeat with
-    // that period (rows: (row >> 1) & 7; k rows: k & 3 resp. k & 7), and bit 3 of k (16-bit B) only
-    // depends on the wave.
-    {
-      int64_t lda = g.lda;
-      if constexpr (kGatherA) lda = late_kernarg_ptr<GatherArgs>(gather_offset)->ld_shard;
-      s.pair_a = (uint32_t)(16 * lda * kEsz);
-      s.pair_b = kBKMajor ? (uint32_t)(16 * g.ldb * kEsz) : (uint32_t)(2 * kBRowsPerPiece * g.ldb * kEsz);
-    }
+    s.half_a = (uint32_t)(64 * lda * kEsz);
+    s.half_b = kBKMajor ? (uint32_t)(32 * g.ldb * kEsz) : (uint32_t)(kStepK / 2 * g.ldb * kEsz);
     s.step_a = kStepK * kEsz;
     s.step_b = kBKMajor ? (uint32_t)(kStepK * kEsz) : (uint32_t)(kStepK * g.ldb * kEsz);
     s.kt_base = 0;
@@ -358,28 +398,48 @@ struct Gemm256 {
     return s;
   }
 
-  // Piece i of K step kt, straight into `stage`.  A chunks at k >= K are redirected past the
-  // end of the buffer so that they read as zero (B rows >= K already lie past it).
-  TCCL_D void issue_a(char* stage, const Source& s, int kt, int i) const {
-    const int kc = (lane & 7) ^ ((4 * (i & 1) + (lane >> 4)) & 7);  // as in make_source
-    const bool dead = kt * kStepK + kc * kChunkK >= g.K;
-    const uint32_t oa = dead ? 0xfffffff0u : s.off_a[i & 1] + ((kGatherA ? kt - s.kt_base : kt) * s.step_a + (i >> 1) * s.pair_a);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.a, (LdsVoid*)(stage + 8 * (4 * wave + i) * kARow256), 16, oa, 0, 0, 0);
+  // Half h of an operand of K step kt into `stage`: two loads (only_i: one of them).
+  TCCL_D void issue_a(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
+    const uint32_t off = (uint32_t)(kGatherA ? kt - s.kt_base : kt) * s.step_a + h * s.half_a;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (only_i < 0 || only_i == i) dma16(stage + a_row(h, i) * kARow256, s.a, s.off_a[i], off);
   }
-  TCCL_D void issue_b(char* stage, const Source& s, int kt, int i) const {
-    if constexpr (kBKMajor) {
-      const int kc = (lane & 7) ^ ((4 * (i & 1) + (lane >> 4)) & 7);
-      const bool dead = kt * kStepK + kc * kChunkK >= g.K;
-      const uint32_t ob = dead ? 0xfffffff0u : s.off_b[i & 1] + whole(kt * s.step_b + (i >> 1) * s.pair_b);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(s.b, (LdsVoid*)(stage + kAStage256 + 8 * (4 * wave + i) * kARow256), 16, ob, 0, 0, 0);
-      return;
+  TCCL_D void issue_b(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
+    const uint32_t off = (uint32_t)kt * s.step_b + h * s.half_b;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (only_i < 0 || only_i == i) dma16(stage + kAStage256 + b_row(h, i) * (kBKMajor ? kARow256 : kBPitch), s.b, s.off_b[i], off);
+  }
+  // Ahead of the first load of K step kt (steps come in ascending order): from the step that reaches past K on, chunks at
+  // k >= K are redirected past the end of the buffer for good and read as zero (row-major B rows >= K lie past it already).
+  TCCL_D void mask(uint32_t (&off)[2], int kt) const {
+    if ((kt + 1) * kStepK > g.K) {
+      const int ln = lane_now();
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int kc = (ln & 7) ^ ((4 * i + (ln >> 4)) & 7);  // as in make_source
+        if (kt * kStepK + kc * kChunkK >= g.K) off[i] = kDeadOffset;
+      }
     }
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.b, (LdsVoid*)(stage + kAStage256 + (4 * wave + i) * 1024), 16,
-                                             s.off_b[i & 1] + whole(kt * s.step_b + (i >> 1) * s.pair_b), 0, 0, 0);
   }
-  TCCL_D void issue_piece(char* stage, const Source& s, int kt, int i) const {
-    issue_a(stage, s, kt, i);
-    issue_b(stage, s, kt, i);
+  TCCL_D void mask_a(Source& s, int kt) const { mask(s.off_a, kt); }
+  TCCL_D void mask_b(Source& s, int kt) const {
+    if constexpr (kBKMajor) mask(s.off_b, kt);
+  }
+  // What the loop expects to be under way when it starts, in the order in which the first steps need it.
+  TCCL_D void issue_first(Source& s) const {
+    mask_a(s, 0);
+    mask_b(s, 0);
+    issue_b(lds, s, 0, 0);
+    issue_b(lds, s, 0, 1);
+    issue_a(lds, s, 0, 0);
+    issue_a(lds, s, 0, 1);
+    if constexpr (!kPull) {
+      mask_b(s, 1);
+      issue_b(lds1, s, 1, 0);
+      if constexpr (kFp8) issue_b(lds1, s, 1, 1);
+    }
   }
 
   // Per-lane LDS read addresses that do not depend on the k-chunk.
@@ -504,14 +564,17 @@ struct Gemm256 {
     int32_t need;            // epoch * tile_counts[gidx]: what the counters of group gidx must reach
     uint32_t group_units;    // ready_units once group gidx is complete
     int backoff;             // K steps to let pass before the counters are fetched again
-    int pend_lp;             // piece of the selected block that was requested and is not yet stored (-1: none)
-    // The piece itself.  One set of registers: a piece is stored (pull_retire) before the next one is
-    // requested, in every path; a second set costs the fused kernels registers they do not have.
-    u32x4 piece[1][kPullLoads];
-    int probe_off;           // this wavefront's counter landing words
-    // The counter word, read out of the landing words right behind a K step's barrier: read
-    // there, it is older than every operand fetch that follows, so using it never waits for those.
-    int32_t probe_val;
+    // What every K step looks at.  `left` = pieces of this wavefront, one stride apart from `next_lp` on, that are whole, lie in
+    // the selected block and may be fetched; `pending` = a piece is on its way into the landing bytes (it is
+    // stored before the next one is requested); `over` = nothing left to learn.
+    int left;
+    bool pending, over, placed;
+    Words4 src;
+    // Where this lane's units of the next piece lie inside the block (byte offsets on either side, column), carried from piece
+    // to piece by additions; where the pending one goes.
+    uint32_t to[kPullLoads], from[kPullLoads], col[kPullLoads], pend_to[kPullLoads];
+    uint32_t step_to, step_from, step_col, wrap_to, wrap_from;
+    int landing;             // this wavefront's landing bytes: the piece, behind it the counter words
     // What the per-step code needs from PullArgs, kept in registers (reading a field through
     // the argument block is a scalar load plus a wait that also drains the operand fetches).
     bool active;
@@ -533,7 +596,7 @@ struct Gemm256 {
   TCCL_D PullState pull_begin(PullPtr a, int wg, int num_wgs) const {
     PullState st;
     const int w = uniform(wave);
-    st.probe_off = w * 256;
+    st.landing = w * (kBgLandingBytes / kPullWaves);
     st.stride = num_wgs * kPullWaves;
     st.next_slot = 0;
     st.next_lp = wg * kPullWaves + w;
@@ -546,10 +609,13 @@ struct Gemm256 {
     st.need = 0;
     st.group_units = 0;
     st.backoff = 0;
-    st.pend_lp = -1;
-    st.probe_val = 0;
+    st.left = 0;
+    st.pending = st.placed = false;
+    st.over = true;
+    st.src = Words4{0, 0, 0, 0};
+    st.step_to = st.step_from = st.step_col = st.wrap_to = st.wrap_from = 0;
 #pragma unroll
-    for (int j = 0; j < kPullLoads; ++j) st.piece[0][j] = u32x4{0, 0, 0, 0};
+    for (int j = 0; j < kPullLoads; ++j) st.to[j] = st.from[j] = st.col[j] = st.pend_to[j] = 0;
     st.active = pull_offset >= 0 && a->mode != kBgNone && w < kPullWaves;
     st.units = 0;
     st.pieces = st.slots = st.n_groups = 0;
@@ -565,16 +631,14 @@ struct Gemm256 {
       st.row_shift = a->row_shift;
       st.row_pitch = a->row_pitch;
       pull_normalise(st, a);
+      st.over = st.next_slot >= st.slots;
     }
     return st;
   }
 
   // Where this lane's unit j of piece lp lies inside a block: byte offsets on the destination and the source
   // side (kNoUnit / the block's first unit for lanes beyond the block's end: their stores fall outside the
-  // buffer window and are dropped, their loads touch a unit that exists).  A handful of vector instructions
-  // from three scalars, formed where a piece is requested and again where it is stored: whatever a pulling
-  // lane carries from K step to K step besides the piece itself costs registers that the fused kernels do
-  // not have (kept in LDS instead, its reads and their waits made the per-step code several times as long).
+  // buffer window and are dropped, their loads touch a unit that exists).
   static constexpr uint32_t kNoUnit = 0xffffffffu;
   TCCL_D void pull_where(const PullState& st, PullPtr a, int lp, int j, int ln, uint32_t& to, uint32_t& from) const {
     const uint32_t u = (uint32_t)lp * (uint32_t)kPieceUnits + (uint32_t)(64 * j + ln);
@@ -588,24 +652,45 @@ struct Gemm256 {
     if constexpr (kGatherA) from = row * a->src_row_pitch + col * 16u;
   }
 
+  // The next piece's places, from scratch (a block's first piece of this wavefront) and from the piece before.
+  TCCL_D void pull_place(PullState& st, PullPtr a) const {
+    const int ln = lane_now();
+#pragma unroll
+    for (int j = 0; j < kPullLoads; ++j) {
+      const uint32_t u = (uint32_t)st.next_lp * (uint32_t)kPieceUnits + (uint32_t)(64 * j + ln);
+      const uint32_t row = st.row_magic ? (__umulhi(u, st.row_magic) >> st.row_shift) : (u >> st.row_shift);
+      st.col[j] = u - row * st.row_units;
+      st.to[j] = row * st.row_pitch + st.col[j] * 16u;
+      if constexpr (kGatherA) st.from[j] = row * a->src_row_pitch + st.col[j] * 16u;
+    }
+  }
+  TCCL_D void pull_advance(PullState& st) const {
+#pragma unroll
+    for (int j = 0; j < kPullLoads; ++j) {
+      const uint32_t col = st.col[j] + st.step_col;
+      const bool wraps = col >= st.row_units;
+      st.col[j] = wraps ? col - st.row_units : col;
+      st.to[j] += st.step_to + (wraps ? st.wrap_to : 0u);
+      if constexpr (kGatherA) st.from[j] += st.step_from + (wraps ? st.wrap_from : 0u);
+    }
+  }
+
   // Fetch the first counters in the first tile's prologue, so that the first K step can
   // already fetch a piece.
-  TCCL_D void pull_prime(PullState& st, PullPtr a, char* landing) const {
-    if constexpr (kWithReduce) return;  // that instantiation never pulls: its launch clears PullArgs
+  TCCL_D void pull_prime(PullState& st, PullPtr a) const {
     if (!st.active || st.next_slot >= a->slots) return;
     pull_select(st, a, st.next_slot);
-    pull_probe(st, a, landing);
+    pull_probe(st, a);
   }
 
   // Every lane fetches the same word; it is read back from LDS one K step later.
-  TCCL_D void pull_probe(PullState& st, PullPtr a, char* landing) const {
-    if (st.gidx >= st.n_groups) return;
+  TCCL_D void pull_probe(PullState& st, PullPtr a) const {
+    if (st.gidx >= st.n_groups || st.probe_group >= 0) return;
     if (st.backoff > 0) {
       --st.backoff;
       return;
     }
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(window(st.counter_base), (LdsVoid*)(bgw + st.probe_off), 4, probe_offset(a, st.gidx), 0, 0,
-                                             kCoherent);
+    dma4_coherent(bgw + st.landing + 16 * kPieceUnits, descriptor((const void*)(uintptr_t)st.counter_base, 0xffffffffu), probe_offset(a, st.gidx));
     st.probe_group = st.gidx;
   }
 
@@ -633,6 +718,7 @@ struct Gemm256 {
       const GatherPtr ga = late_kernarg_ptr<GatherArgs>(gather_offset);
       st.src_base = (int64_t)(uintptr_t)ga->shard + (table(ga->heap_bases, slot) - table(ga->heap_bases, ga->rank));
       st.dst_base = (int64_t)(uintptr_t)g.A + (int64_t)slot * ga->k_shard * kEszIn;
+      st.src = descriptor((const void*)(uintptr_t)st.src_base, 0xffffffffu);
       st.ready_units = a->units;
       st.gidx = a->n_groups;
       return;
@@ -642,6 +728,7 @@ struct Gemm256 {
     const int64_t theirs = table(a->heap_bases, peer);
     const int64_t rel = ((int64_t)(uintptr_t)a->src0 - mine) + (int64_t)peer * a->block_bytes;
     st.src_base = theirs + rel;
+    st.src = descriptor((const void*)(uintptr_t)st.src_base, 0xffffffffu);
     st.dst_base = mine + rel;
     const int64_t stride = a->word_stride;
     st.counter_base = (int64_t)(uintptr_t)a->counter + (stride ? (int64_t)(peer - a->rank) * stride : theirs - mine);
@@ -672,21 +759,17 @@ struct Gemm256 {
     }
   }
 
-  // Store the piece that is pending, if any.  Returns whether a store was issued.  The piece belongs
-  // to the selected block: pull_issue() stores what is pending before it selects another one.
-  TCCL_D bool pull_retire(PullState& st, PullPtr a, const char* landing, int) const {
-    if constexpr (kWithReduce) return false;
-    if (st.pend_lp < 0) return false;
+  // Store the piece that is pending, if any: it has landed (the caller has waited for it).
+  TCCL_D void pull_retire(PullState& st) const {
+    if (!st.pending) return;
     const __amdgpu_buffer_rsrc_t dst = window(st.dst_base);
     const int ln = lane_now();
+    u32x4 piece[kPullLoads];
 #pragma unroll
-    for (int j = 0; j < kPullLoads; ++j) {
-      uint32_t to, from;
-      pull_where(st, a, st.pend_lp, j, ln, to, from);
-      st16<kStreaming>(dst, to, st.piece[0][j]);
-    }
-    st.pend_lp = -1;
-    return true;
+    for (int j = 0; j < kPullLoads; ++j) piece[j] = *(const u32x4*)(bgw + st.landing + 16 * (64 * j + ln));
+#pragma unroll
+    for (int j = 0; j < kPullLoads; ++j) st16<kStreaming>(dst, st.pend_to[j], piece[j]);
+    st.pending = false;
   }
 
   // The two facts about group gidx that the per-step code needs, fetched when gidx changes.
@@ -725,54 +808,71 @@ struct Gemm256 {
     pull_group_facts(st, a);
   }
 
-  // Right behind a K step's barrier (this wave's loads, the counter fetch among them, have
-  // landed): take the counter word out of the landing words.
-  TCCL_D void pull_collect(PullState& st, PullPtr a, const char* landing, int slot) const {
-    if constexpr (kWithReduce) return;
-    if (!st.active) return;
-    st.probe_val = *(const int32_t*)(bgw + st.probe_off + 4 * lane_now());  // lane l's word landed at 4 l
-  }
-  // Once per K step: learn about readiness, request the next piece into slot `slot` (its
-  // previous piece was stored during the step before).  All control flow here is
-  // wavefront-uniform.  Returns whether a piece was requested.
-  TCCL_D bool pull_issue(PullState& st, PullPtr a, char* landing, int) const {
-    if constexpr (kWithReduce) return false;
-    if (!st.active) return false;
-    if (st.probe_group >= 0) {
-      const int g = st.probe_group;
-      st.probe_group = -1;
-      if (g == st.gidx) {
-        if (all_reached(st.probe_val, st.need))
-          pull_group_done(st, a);
-        else
-          st.backoff = 3;  // not there yet: fetching the counters every step only costs issue slots
-      }
-    }
-    if (st.next_slot >= st.slots) return false;
-    if (st.next_slot != st.slot) {
-      pull_retire(st, a, landing, 0);  // a piece still pending belongs to the block being left
-      pull_select(st, a, st.next_slot);
-      pull_probe(st, a, landing);
-      return false;
-    }
-    pull_probe(st, a, landing);  // look ahead: the next group's counters (issued before the piece, which stays the youngest load)
-    const uint32_t first = (uint32_t)st.next_lp * (uint32_t)kPieceUnits;
-    const uint32_t last = first + (uint32_t)(kPieceUnits - 1);
-    if ((last < st.units ? last : st.units - 1u) < st.ready_units) {
-      const __amdgpu_buffer_rsrc_t src = window(st.src_base);
-      const int ln = lane_now();
+  // Once per K step, behind pull_retire(): request the next piece.
+  TCCL_D void pull_request(PullState& st, PullPtr a) const {
+    if (__builtin_expect(!st.over && st.left <= 1, 0)) pull_more(st, a);
+    if (st.left > 0) {
 #pragma unroll
       for (int j = 0; j < kPullLoads; ++j) {
-        uint32_t to, from;
-        pull_where(st, a, st.next_lp, j, ln, to, from);
-        st.piece[0][j] = ld16<kCoherent>(src, from);
+        st.pend_to[j] = st.to[j];
+        dma16_coherent(bgw + st.landing + 1024 * j, st.src, kGatherA ? st.from[j] : st.to[j]);
       }
-      st.pend_lp = st.next_lp;
+      st.pending = true;
+      --st.left;
       st.next_lp += st.stride;
-      if (st.next_lp >= st.pieces) pull_normalise(st, a);  // block finished: rare
-      return true;
+      pull_advance(st);
     }
-    return false;
+  }
+  // The rare part of it: take in the counter word fetched before (it landed ahead of a barrier since), move on to the next
+  // block, count what may be fetched, fetch the next word.
+  TCCL_D void pull_more(PullState& st, PullPtr a) const {
+    // What the pieces' places need is worked out here, not in the kernel's first microseconds, which have no slack
+    // (4096 x 4096 x 1024: 1 us per launch).
+    if (!st.placed) {
+      st.placed = true;
+      const uint32_t ahead = (uint32_t)st.stride * (uint32_t)kPieceUnits;  // units from piece to piece
+      const uint32_t rows = st.row_magic ? (__umulhi(ahead, st.row_magic) >> st.row_shift) : (ahead >> st.row_shift);
+      const uint32_t src_pitch = kGatherA ? a->src_row_pitch : st.row_pitch;
+      st.step_col = ahead - rows * st.row_units;
+      st.step_to = rows * st.row_pitch + st.step_col * 16u;
+      st.step_from = rows * src_pitch + st.step_col * 16u;
+      st.wrap_to = st.row_pitch - st.row_units * 16u;
+      st.wrap_from = src_pitch - st.row_units * 16u;
+      pull_place(st, a);
+    }
+    if (st.probe_group >= 0) {
+      const int32_t word = *(const int32_t*)(bgw + st.landing + 16 * kPieceUnits + 4 * lane_now());  // lane l's word landed at 4 l
+      st.probe_group = -1;
+      if (all_reached(word, st.need))
+        pull_group_done(st, a);
+      else
+        st.backoff = 3;  // not there yet: fetching the counters every step only costs issue slots
+    }
+    if (st.left == 0 && st.next_lp >= st.pieces) pull_normalise(st, a);  // block finished
+    if (st.next_slot >= st.slots) {
+      st.over = true;
+      return;
+    }
+    if (st.next_slot != st.slot) {
+      pull_select(st, a, st.next_slot);
+      pull_place(st, a);
+    }
+    const int whole = (int)(st.ready_units / (uint32_t)kPieceUnits);
+    while (st.next_lp + st.left * st.stride < whole) ++st.left;
+    // (A block's last piece may be short: its lanes past the end fetch the block's first unit and store nothing.)
+    const uint32_t first = (uint32_t)st.next_lp * (uint32_t)kPieceUnits;
+    if (st.left == 0 && !st.pending && st.next_lp < st.pieces && st.ready_units >= st.units) {
+#pragma unroll
+      for (int j = 0; j < kPullLoads; ++j) {
+        const bool valid = first + (uint32_t)(64 * j + lane_now()) < st.units;
+        st.pend_to[j] = valid ? st.to[j] : kNoUnit;
+        dma16_coherent(bgw + st.landing + 1024 * j, st.src, valid ? (kGatherA ? st.from[j] : st.to[j]) : 0u);
+      }
+      st.pending = true;
+      st.next_lp += st.stride;
+      return;
+    }
+    pull_probe(st, a);
   }
 
   // Wait (bounded) until units [0, last] of the selected block may be fetched.
@@ -794,11 +894,10 @@ struct Gemm256 {
   }
 
   // After the last tile: finish what is in flight, move the remaining pieces, report.
-  TCCL_D void pull_finish(PullState& st, PullPtr a, const char* landing, int num_wgs) const {
-    if constexpr (kWithReduce) return;
+  TCCL_D void pull_finish(PullState& st, PullPtr a, int num_wgs) const {
     if (pull_offset < 0 || a->mode == kBgNone) return;  // the same for every wavefront: a barrier follows
     bool ok = true;
-    if (st.active) ok = pull_drain(st, a, landing);
+    if (st.active) ok = pull_drain(st, a);
     if (!ok && lane == 0 && a->fault) *a->fault = 1;
     wait_vmem();
     __syncthreads();
@@ -819,9 +918,10 @@ struct Gemm256 {
   }
 
   // The pulling wavefronts' part of pull_finish; false if a bounded wait expired.
-  TCCL_D bool pull_drain(PullState& st, PullPtr a, const char* landing) const {
+  TCCL_D bool pull_drain(PullState& st, PullPtr a) const {
     wait_vmem();
-    pull_retire(st, a, landing, 0);
+    pull_retire(st);
+    pull_normalise(st, a);  // (nothing left: the loop below is not entered)
     st.probe_group = -1;
     const int64_t deadline = now_ticks() + a->spin_ticks;
     bool ok = true;
@@ -870,135 +970,172 @@ struct Gemm256 {
     return ok;
   }
 
-  // 16-bit operand registers; they live across K steps.
+  // Operand registers of a K step.
   struct Frags {
-    Vec ring[4], fb[4];
+    Vec a[kFp8 ? 2 : 4];        // a phase's A operands
+    Vec b[kFp8 ? 1 : 2][4];     // the four B operands of either k block (fp8: of the step)
   };
 
-  // fp8 operand registers; they live across K steps.
-  struct Frags8 {
-    Vec ring[2], fb[4];
-  };
-
-  // One K step of the fp8 path (v_mfma_scale_f32_16x16x128_f8f6f4, 128 k per step): eight items of four
-  // MFMAs, item d = the 16-row block d of the wave tile against its four 16-column blocks, read from
-  // `cur` while the next step's operands stream into `nxt` (one pair of loads per item, items 0..3).
-  // An fp8 operand is 8 registers: the A operand is fetched one item ahead (two register sets), the four
-  // B operands have one set and are reloaded in place during the last item, each as soon as its MFMA is
-  // issued.  As in the 16-bit path the step's one barrier sits inside the step, before item 7: the reads
-  // of `cur` are done, the loads into `nxt` have landed, and item 7 fetches the next step's first
-  // operands from `nxt` behind it.
-  TCCL_D void k_step8(const char* cur, char* nxt, const Source& src, const Reader& rd, int kt_load, f32x16 (&acc)[4][2],
-                      Frags8& f, PullState& pull, int parity) const {
+  // What ends the data slot of a phase and what follows it: the barrier, the phase's MFMAs (256 clocks), the barrier
+  // that ends the multiplying slot.  `rb0` = first 16-row block, kh = k block.  The LDS reads of the data slot are waited
+  // for behind the barrier (by the waits that the compiler puts ahead of the MFMAs): waited for ahead of it they kept the
+  // other side waiting as well (8192 x 4096 x 4096: 6 % slower).
+  // acc[rb / 2][cb / 2] holds a 32 x 32 patch as four 16 x 16 blocks: registers 4 * q .. 4 * q + 3 are
+  // block q = 2 * (rb % 2) + cb % 2 (acc_spot() is the lane's place in it).
+  TCCL_D void multiply(f32x16 (&acc)[4][2], const Frags& f, int rb0, int kh) const {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int d = 0; d < 8; ++d) {
-      if (d == 7) {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        pull_collect(pull, pa(), bgw, parity);
-      }
-      const char* from = d + 1 < 8 ? cur : nxt;
-      f.ring[(d + 1) & 1] = load_a8(from, rd, (d + 1) & 7);
-      if (d < 4) issue_piece(nxt, src, kt_load, d);
-      // The background transfer's one place in the step, as in the 16-bit path: behind the step's last
-      // operand loads, the piece of the step before stored first, the next one requested into its registers.
-      if constexpr (!kWithReduce) {
-        if (d == 3 && pull.active) {
-          pull_retire(pull, pa(), bgw, parity ^ 1);
-          pull_issue(pull, pa(), bgw, parity);
-        }
-      }
+    for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        f32x16& patch = acc[d >> 1][cb >> 1];
-        const int q = 2 * (d & 1) + (cb & 1);
+      for (int r = 0; r < (kFp8 ? 2 : 4); ++r) {
+        const int rb = rb0 + r;
+        f32x16& patch = acc[rb >> 1][cb >> 1];
+        const int q = 2 * (rb & 1) + (cb & 1);
         f32x4 blk = {patch[4 * q], patch[4 * q + 1], patch[4 * q + 2], patch[4 * q + 3]};
-        blk = Mfma<InT>::run16(f.fb[cb], f.ring[d & 1], blk);
+        blk = Mfma<InT>::run16(f.b[kh][cb], f.a[r], blk);
 #pragma unroll
         for (int e = 0; e < 4; ++e) patch[4 * q + e] = blk[e];
-        if (d == 7) {
-          __builtin_amdgcn_sched_barrier(0);
-          f.fb[cb] = load_b8(nxt, rd, cb);
-        }
       }
-      __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  }
+  // K step kt, computed from the stage `cur`; `nxt` is the other one.
+  //
+  // 16-bit: phase 0 = upper 64 rows of the wave tile, first 32 k; phase 1 = upper rows, second 32 k; phases 2 and 3 the
+  // lower rows.  B operands are read in phases 0 and 1 and kept, A operands phase by phase.  fp8 (one MFMA is 128 k deep):
+  // phase p = 32 rows of the wave tile, all B operands read in phase 0.
+  //
+  // Who may refill what: a wavefront's reads of phase p have returned when its MFMAs of phase p begin, and every other
+  // wavefront's data slot of phase p + 2 begins behind a barrier after that (the two sides are one slot apart).
+  //   16-bit                    last read    refilled with step    in phase
+  //   B, both halves            1            kt + 2                3, and 0 of the next step
+  //   A, upper rows             1            kt + 2                1 of the next step
+  //   A, lower rows             3            kt + 2                2 of the next step
+  // fp8: B is free from phase 2 on (read in phase 0) and is refilled in 2 and 3, A in 0 and 1 of the next step.
+  // What is needed when (both sides have passed their wait and a barrier lies between): B and the upper rows of
+  // step kt + 1 are waited for at the end of phase 3's data slot, behind them the lower rows of kt + 1 and one half of
+  // B (fp8: lower rows, both halves) have been requested; the lower rows of step kt in phase 1, behind them three halves
+  // (fp8: four).
+  TCCL_D void k_step(char* cur, char* nxt, Source& src, const Reader& rd, int kt, f32x16 (&acc)[4][2], Frags& f) const {
+    if constexpr (kFp8) {
+      mask_a(src, kt + 1);
+      issue_a(nxt, src, kt + 1, 0);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) f.b[0][cb] = load_b8(cur, rd, cb);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) f.a[r] = load_a8(cur, rd, r);
+      multiply(acc, f, 0, 0);
+      issue_a(nxt, src, kt + 1, 1);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) f.a[r] = load_a8(cur, rd, 2 + r);
+      wait_loads<8>();
+      multiply(acc, f, 2, 0);
+      mask_b(src, kt + 2);
+      issue_b(cur, src, kt + 2, 0);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) f.a[r] = load_a8(cur, rd, 4 + r);
+      multiply(acc, f, 4, 0);
+      issue_b(cur, src, kt + 2, 1);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) f.a[r] = load_a8(cur, rd, 6 + r);
+      wait_loads<6>();
+      multiply(acc, f, 6, 0);
+    } else {
+      issue_b(nxt, src, kt + 1, 1);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) f.b[0][cb] = load_b16(cur, rd, 0, cb);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f.a[r] = load_a16(cur, rd, 0, r);
+      multiply(acc, f, 0, 0);
+      mask_a(src, kt + 1);
+      follow_shards(src, kt + 1);
+      issue_a(nxt, src, kt + 1, 0);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) f.b[1][cb] = load_b16(cur, rd, 1, cb);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f.a[r] = load_a16(cur, rd, 1, r);
+      wait_loads<6>();
+      multiply(acc, f, 0, 1);
+      issue_a(nxt, src, kt + 1, 1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f.a[r] = load_a16(cur, rd, 0, 4 + r);
+      multiply(acc, f, 4, 0);
+      mask_b(src, kt + 2);
+      issue_b(cur, src, kt + 2, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f.a[r] = load_a16(cur, rd, 1, 4 + r);
+      wait_loads<4>();
+      multiply(acc, f, 4, 1);
     }
   }
 
-  // One K step of the 16-bit path (v_mfma_f32_16x16x32): eight items of eight MFMAs each, read from `cur`
-  // while the next step's operands stream into `nxt`.  Item d covers k block kh = d / 4 (32 k) and the
-  // 16-row blocks 2 * (d % 4), + 1 of the wave tile, against all four 16-column blocks.
-  //
-  // A operands (two per item) are fetched one item ahead through four register sets.  B operands
-  // (four per k block) have ONE register set: the last item of a k block runs column block by
-  // column block, and as soon as a column block's two MFMAs are issued its registers take the next k
-  // block's operand, which is first needed six MFMAs later (the first item of a k block runs in the
-  // same order).  A second set would cost 16 registers, which the fused kernels do not have.
-  // The scheduling barriers pin this order (left alone, the compiler hoists every read of the step and
-  // spills).
-  //
-  // The step's one barrier sits before the last item, not at the end.  There this wave has issued
-  // (and, after the lgkmcnt wait, finished) its last read of `cur`, and its loads into `nxt`,
-  // issued during items 0..3, have landed; behind the barrier the last item already fetches
-  // the next step's first operands from `nxt`, so the matrix pipe does not drain while the
-  // first LDS reads of a step are in flight.
-  //
-  // Issuing a global load holds the wave for as long as the address unit takes to accept it (about 16
-  // clocks per KiB instruction, four times that when the four SIMDs' waves issue in the same item),
-  // and nothing else of the wave issues meanwhile; they go out two per item over items 0..3.
-  TCCL_D void k_step16(const char* cur, char* nxt, const Source& src, const Reader& rd, int kt_load, f32x16 (&acc)[4][2],
-                       Frags& f, PullState& pull, int parity) const {
+  // K step kt of a launch with a background transfer: eight items, item d's A operands fetched one item ahead, computed from
+  // `cur` while the next step's operands stream into `nxt` (one piece of A and of B per item, items 0..3).  16-bit: eight MFMAs per
+  // item, k block d / 4, 16-row blocks 2 (d % 4) and + 1; fp8: four, 16-row block d.  The four B operands have one register
+  // set: the last item of a k block runs column block by column block and reloads each in place.  The step's one barrier sits
+  // before the last item: there the wavefront's reads of `cur` are done, its loads into `nxt` have landed, and the last item
+  // already fetches the next step's first operands.  The transfer has one place, behind the step's last operand loads
+  // (spread over three items the same work cost 4096 x 4096 x 1024 1.3 us more).
+  struct Running {
+    Vec ring[kFp8 ? 2 : 4], fb[4];
+  };
+  TCCL_D Vec load_a(const char* stage, const Reader& r, int kh, int rb) const {
+    if constexpr (kFp8)
+      return load_a8(stage, r, rb);
+    else
+      return load_a16(stage, r, kh, rb);
+  }
+  TCCL_D Vec load_b(const char* stage, const Reader& r, int kh, int cb) const {
+    if constexpr (kFp8)
+      return load_b8(stage, r, cb);
+    else
+      return load_b16(stage, r, kh, cb);
+  }
+  TCCL_D void step_pulling(char* cur, char* nxt, Source& src, const Reader& rd, int kt, f32x16 (&acc)[4][2], Running& f, PullState& pull) const {
+    constexpr int kRows = kFp8 ? 1 : 2;            // 16-row blocks per item
+    constexpr int kPerBlock = 8 / kRows;           // items per k block
+    mask_a(src, kt + 1);
+    mask_b(src, kt + 1);
+    follow_shards(src, kt + 1);
 #pragma unroll
     for (int d = 0; d < 8; ++d) {
-      const int rp = d & 3;
+      const int rp = d % kPerBlock;
       if (d == 7) {
-        // This wave's loads (and background fetch) have landed, its reads of `cur` are done.
-        // The barrier is the bare instruction: __syncthreads() carries a workgroup-scope
-        // release fence.  The empty asm keeps the compiler from moving LDS accesses across it.
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        pull_collect(pull, pa(), bgw, parity);
       }
       const int dn = (d + 1) & 7;
       const char* from = d + 1 < 8 ? cur : nxt;
-      f.ring[2 * (dn & 1)] = load_a16(from, rd, dn >> 2, 2 * (dn & 3));
-      f.ring[2 * (dn & 1) + 1] = load_a16(from, rd, dn >> 2, 2 * (dn & 3) + 1);
-      if (d < 4) {
-        issue_a(nxt, src, kt_load, d);
-        issue_b(nxt, src, kt_load, d);
+      if (d < 4) issue_a(nxt, src, kt + 1, d >> 1, d & 1);
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) f.ring[kRows * (dn & 1) + r] = load_a(from, rd, dn / kPerBlock, kRows * (dn % kPerBlock) + r);
+      if (d < 4) issue_b(nxt, src, kt + 1, d >> 1, d & 1);
+      if (d == 3) {
+        pull_retire(pull);
+        pull_request(pull, pa());
       }
-      // The background transfer has one place in the step, behind the step's last operand loads (loads
-      // complete in issue order: a request that goes out to the peer's memory ahead of them would hold
-      // all of them back): the piece requested during the step before (it arrived before that step's
-      // barrier) is stored, then the next one is requested into the same registers.  One place, under one
-      // test: every call site splits the step into basic blocks, and where they join the compiler waits
-      // for more than the code needs.  Spread over three items (state read an item ahead of its use) the
-      // same work cost a launch of 4096 x 4096 x 1024 1.3 us more.
-      if constexpr (!kWithReduce) {
-        if (d == 3 && pull.active) {
-          pull_retire(pull, pa(), bgw, parity ^ 1);
-          pull_issue(pull, pa(), bgw, parity);
-        }
-      }
-      // acc[rb / 2][cb / 2] holds a 32 x 32 patch as four 16 x 16 blocks: registers 4 * q .. 4 * q + 3 are
-      // block q = 2 * (rb % 2) + cb % 2 (acc_spot() is the lane's place in it).
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-          const int rb = 2 * rp + r;
+        for (int r = 0; r < kRows; ++r) {
+          const int rb = kRows * rp + r;
           f32x16& patch = acc[rb >> 1][cb >> 1];
           const int q = 2 * (rb & 1) + (cb & 1);
           f32x4 blk = {patch[4 * q], patch[4 * q + 1], patch[4 * q + 2], patch[4 * q + 3]};
-          blk = Mfma<InT>::run16(f.fb[cb], f.ring[2 * (d & 1) + r], blk);
+          blk = Mfma<InT>::run16(f.fb[cb], f.ring[kRows * (d & 1) + r], blk);
 #pragma unroll
           for (int e = 0; e < 4; ++e) patch[4 * q + e] = blk[e];
         }
-        if (rp == 3) {
+        if (rp == kPerBlock - 1) {
           __builtin_amdgcn_sched_barrier(0);
-          f.fb[cb] = load_b16(from, rd, dn >> 2, cb);
+          f.fb[cb] = load_b(from, rd, dn / kPerBlock, cb);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -1239,13 +1376,9 @@ struct Gemm256 {
     if (!ahead) {
       src = make_source(row0, col0);
       __syncthreads();  // the previous tile's epilogue has left LDS
-#pragma unroll
-      for (int i = 0; i < 4; ++i) issue_piece(lds, src, 0, i);
+      issue_first(src);
     }
-    // K steps are taken in pairs so that each call names its two stages statically and the
-    // accumulators flow through one straight loop body.  An odd step count is rounded up: the
-    // extra step (like the final look-ahead load) lies wholly past K and reads zeros.
-    const int ksteps = ((g.K + kStepK - 1) / kStepK + 1) & ~1;
+    const int ksteps = (g.K + kStepK - 1) / kStepK;  // (loads of steps past them read zeros that nobody uses)
     // The accumulators are cleared two registers per instruction (64-bit moves): 128 single moves per
     // wavefront, two wavefronts per SIMD, were half a microsecond of a tile's start.
     f32x16 acc[4][2];
@@ -1264,35 +1397,35 @@ struct Gemm256 {
         acc[i][j] = __builtin_bit_cast(f32x16, z);
       }
     const Reader rd = make_reader();
-    wait_vmem();  // the first operands are there, and so is everything the previous tile stored
+    // The first step's operands (in the loop of phases but for the lower rows of A) are there, and so is everything the
+    // previous tile stored.
+    wait_loads<kPull ? 0 : (kFp8 ? 6 : 4)>();
     __syncthreads();
     publish_owed(s, unpublished);
-    pull_collect(pull, pa(), bgw, 0);  // the counters fetched before this tile (no piece is pending here)
-    if constexpr (kFp8) {
-      Frags8 f;
+    // One loop body for both stages, their places exchanged from step to step: half the code of two named stages,
+    // and fewer registers (189 instead of 223 in the plain bf16 kernel).
+    uint32_t at = 0;
+    if constexpr (kPull) {
+      Running f;
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b8(lds, rd, cb);
-      f.ring[0] = load_a8(lds, rd, 0);
+      for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b(lds, rd, 0, cb);
+#pragma unroll
+      for (int r = 0; r < (kFp8 ? 1 : 2); ++r) f.ring[r] = load_a(lds, rd, 0, r);
       for (int kt = 0; kt < ksteps; kt += 2) {
-        follow_shards(src, kt + 1);
-        k_step8(lds, lds1, src, rd, kt + 1, acc, f, pull, 0);
-        follow_shards(src, kt + 2);
-        k_step8(lds1, lds, src, rd, kt + 2, acc, f, pull, 1);
+        step_pulling(lds, lds1, src, rd, kt, acc, f, pull);
+        step_pulling(lds1, lds, src, rd, kt + 1, acc, f, pull);
       }
     } else {
       Frags f;
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b16(lds, rd, 0, cb);
-      f.ring[0] = load_a16(lds, rd, 0, 0);
-      f.ring[1] = load_a16(lds, rd, 0, 1);
-      for (int kt = 0; kt < ksteps; kt += 2) {
-        follow_shards(src, kt + 1);
-        k_step16(lds, lds1, src, rd, kt + 1, acc, f, pull, 0);
-        follow_shards(src, kt + 2);
-        k_step16(lds1, lds, src, rd, kt + 2, acc, f, pull, 1);
+      if (wm) __builtin_amdgcn_s_barrier();  // wavefronts 4..7 stay one slot behind wavefronts 0..3
+      for (int kt = 0; kt < ksteps; ++kt) {
+        k_step(lds + at, lds + (at ^ (uint32_t)kStage256), src, rd, kt, acc, f);
+        at ^= (uint32_t)kStage256;
       }
-      pull_retire(pull, pa(), bgw, 1);  // the last step's piece: nothing is carried through the epilogue
+      if (!wm) __builtin_amdgcn_s_barrier();
     }
+    wait_vmem();  // the loads past the last step: the epilogue stages through their LDS
+    if constexpr (kPull) pull_retire(pull);  // nothing is carried through the epilogue
     if constexpr (kWithReduce) {
       // Rows this rank owns, partial kept in registers: the peers' partials are added in the
       // epilogue and the tile's partial is never stored (it is still published: the counters
@@ -1500,6 +1633,9 @@ struct Gemm256 {
       const int32_t prev = tile_signal_add<true>(s.counter, group, count);
       if (prev + count == s.epoch * s.tile_counts[group]) s.trace_ready_clock[group] = now_ticks();
     } else {
+      // (Kept apart from the add above: made one, it returns its old value here as well, and the compiler waits for that
+      // register with vmcnt(0) inside the K loop that follows: 8192 x 4096 x 2048 with its reductions 154 -> 170 us.)
+      asm volatile("");
       (void)tile_signal_add<true>(s.counter, group, count);
     }
   }
@@ -1549,11 +1685,13 @@ struct Gemm256 {
     // (A workgroup beyond the last tile requests some tile's operands and never uses them.)
     const TileCoord c0 = tile_of_slot(wg < total ? wg : total - 1, total, m);
     Source src = make_source(c0.m * kMacro, c0.n * kMacro);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) issue_piece(lds, src, 0, i);
+    issue_first(src);
     __builtin_amdgcn_sched_barrier(0);
-    PullState pull = pull_begin(pa(), wg, num_wgs);
-    pull_prime(pull, pa(), bgw);
+    PullState pull;
+    if constexpr (kPull) {
+      pull = pull_begin(pa(), wg, num_wgs);
+      pull_prime(pull, pa());
+    }
     Owed unpublished = nothing_owed();
     // A launch with at most one tile per workgroup does not enter the tile loop: what the compiler computes
     // once for all tiles of a loop it computes ahead of the loop, i.e. between a workgroup's first operand
@@ -1581,7 +1719,7 @@ struct Gemm256 {
       __syncthreads();
       publish_owed(s, unpublished);
     }
-    pull_finish(pull, pa(), bgw, num_wgs);
+    if constexpr (kPull) pull_finish(pull, pa(), num_wgs);
   }
 };
 #endif  // __HIP_DEVICE_COMPILE__

@@ -17,12 +17,11 @@ namespace tccl {
 template <typename InT, typename OutT, bool kBKMajor>
 __global__ __launch_bounds__(512, 2) void gemm256_kernel(GemmArgs g, Macro m) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __attribute__((aligned(16))) char stage0[kStage256];
-  __shared__ __attribute__((aligned(16))) char stage1[kStage256];
+  __shared__ __attribute__((aligned(16))) char stages[kLds256];
   warm_kernargs<(int)(sizeof(GemmArgs) + sizeof(Macro))>();
   SignalArgs s;
   s.mode = kSignalNone;
-  Gemm256<InT, OutT, false, false, kBKMajor>(g, -1, -1, -1, stage0, stage1, nullptr).run(s, m, (int)blockIdx.x, (int)gridDim.x);
+  Gemm256<InT, OutT, false, false, kBKMajor>(g, -1, -1, -1, stages, stages + kStage256, nullptr).run(s, m, (int)blockIdx.x, (int)gridDim.x);
 #endif
 }
 
@@ -52,18 +51,17 @@ struct Fused256Args {
 template <typename InT, typename OutT, bool kWithReduce, bool kGatherA, bool kBKMajor, bool kPull = true>
 __global__ __launch_bounds__(512, 2) void fused256_kernel(Fused256Args f) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __attribute__((aligned(16))) char stage0[kStage256];
-  __shared__ __attribute__((aligned(16))) char stage1[kStage256];
-  __shared__ __attribute__((aligned(16))) char landing_words[kBgWordBytes];
+  __shared__ __attribute__((aligned(16))) char stages[kLds256];
+  __shared__ __attribute__((aligned(16))) char landing[kPull ? kBgLandingBytes : 16];
   warm_kernargs<(int)sizeof(Fused256Args)>();
   if (f.trace_start && blockIdx.x == 0 && threadIdx.x == 0) *f.trace_start = now_ticks();
-  Gemm256<InT, OutT, kWithReduce, kGatherA, kBKMajor>(f.g, kPull ? (int)offsetof(Fused256Args, pull) : -1, (int)offsetof(Fused256Args, push),
-                                                      (int)offsetof(Fused256Args, reduce), stage0, stage1, landing_words,
+  Gemm256<InT, OutT, kWithReduce, kGatherA, kBKMajor, kPull>(f.g, kPull ? (int)offsetof(Fused256Args, pull) : -1, (int)offsetof(Fused256Args, push),
+                                                      (int)offsetof(Fused256Args, reduce), stages, stages + kStage256, landing,
                                                       (int)offsetof(Fused256Args, gather))
       .run(f.s, f.m, (int)blockIdx.x, (int)gridDim.x);
   __syncthreads();
   const CommArgs c = late_kernarg<CommArgs>((int)offsetof(Fused256Args, comm));
-  comm_role<kThreads256>(c, (int)blockIdx.x, (int)gridDim.x, (int*)stage1);
+  comm_role<kThreads256>(c, (int)blockIdx.x, (int)gridDim.x, (int*)(stages + kStage256));
 #endif
 }
 
@@ -88,7 +86,7 @@ int launch_fused256_t(const Fused256Args& f, int wgs, hipStream_t stream) {
     else
       return kGatherTypes;
   } else if (f.reduce.active)
-    hipLaunchKernelGGL((fused256_kernel<InT, OutT, true, false, kBKMajor>), dim3(wgs), dim3(kThreads256), 0, stream, f);
+    hipLaunchKernelGGL((fused256_kernel<InT, OutT, true, false, kBKMajor, false>), dim3(wgs), dim3(kThreads256), 0, stream, f);
   else if (f.pull.mode == kBgNone)
     hipLaunchKernelGGL((fused256_kernel<InT, OutT, false, false, kBKMajor, false>), dim3(wgs), dim3(kThreads256), 0, stream, f);
   else
