@@ -1411,9 +1411,16 @@ struct Gemm256 {
       for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b(lds, rd, 0, cb);
 #pragma unroll
       for (int r = 0; r < (kFp8 ? 1 : 2); ++r) f.ring[r] = load_a(lds, rd, 0, r);
-      for (int kt = 0; kt < ksteps; kt += 2) {
-        step_pulling(lds, lds1, src, rd, kt, acc, f, pull);
-        step_pulling(lds1, lds, src, rd, kt + 1, acc, f, pull);
+      if constexpr (kBKMajor) {
+        for (int kt = 0; kt < ksteps; ++kt) {
+          step_pulling(lds + at, lds + (at ^ (uint32_t)kStage256), src, rd, kt, acc, f, pull);
+          at ^= (uint32_t)kStage256;
+        }
+      } else {  // two named stages: 1.5 % at 4096 x 4096 x 2048 with gathered inputs (a k-major B spills with them)
+        for (int kt = 0; kt < ksteps; kt += 2) {
+          step_pulling(lds, lds1, src, rd, kt, acc, f, pull);
+          step_pulling(lds1, lds, src, rd, kt + 1, acc, f, pull);
+        }
       }
     } else {
       Frags f;
