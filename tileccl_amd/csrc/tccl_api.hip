@@ -170,6 +170,17 @@ __global__ __launch_bounds__(256) void reduce_kernel(tccl::BulkReduceArgs a) {
   tccl::bulk_reduce<PT, OT, kRanks, tccl::kThreadsComm>(a, a.first_owner + (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x);
 }
 
+// The same behind a wait for the peers' words.  Loads pass the caches: the peers may still be writing when the launch starts.
+constexpr int kThreadsReady = 512;
+template <typename PT, typename OT, int kRanks>
+__global__ __launch_bounds__(kThreadsReady) void ready_reduce_kernel(tccl::BulkReduceArgs a, tccl::CommArgs c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int owner = a.first_owner + (int)blockIdx.y;
+  if (tccl::rows_published<kThreadsReady>(c, owner))
+    tccl::bulk_reduce<PT, OT, kRanks, kThreadsReady, tccl::kCoherent>(a, owner, (int)blockIdx.x, (int)gridDim.x);
+#endif
+}
+
 // Staged collectives: workgroup w carries slot w % slots of the (w / slots)-th rank named in a.ranks.
 __global__ __launch_bounds__(256) void staged_kernel(tccl::StagedArgs a) {
   __shared__ int word;
@@ -656,14 +667,16 @@ bool build_background(const tccl::CommArgs& c, tccl::PullArgs* p) {
   return true;
 }
 
-// A reduce-scatter whose reduction the large-tile kernel can perform tile by tile.
+// Can the large-tile kernel perform the reduction tile by tile?  A tile must not straddle two owners.
+bool reduces_in_tiles(const tccl::CommArgs& c) {
+  return c.op == tccl::kOpReduceScatter && c.world > 1 && c.M % c.world == 0 && c.M / c.world % tccl::kMacro == 0 &&
+         (c.out_dtype == tccl::kF16 || c.out_dtype == tccl::kBF16) && c.ld_rs_out_bytes % 8 == 0;
+}
+
 bool build_reduce(const tccl::CommArgs& c, const tccl_sync_desc* sync, int flags, tccl::ReduceArgs* r, tccl::Macro* m) {
   memset(r, 0, sizeof *r);
-  if (c.op != tccl::kOpReduceScatter || c.world <= 1 || c.M % c.world) return false;
+  if (!reduces_in_tiles(c)) return false;
   const int shard = c.M / c.world;
-  if (shard % tccl::kMacro) return false;  // a tile must not straddle two owners
-  if (c.out_dtype != tccl::kF16 && c.out_dtype != tccl::kBF16) return false;
-  if (c.ld_rs_out_bytes % 8) return false;
   r->active = 1;
   r->rank = c.rank;
   r->world = c.world;
@@ -756,7 +769,17 @@ int launch_bulk_copy(tccl::BulkCopyArgs& a, int transfers, int64_t rows, const t
 }
 
 template <typename PT, typename OT>
-void launch_reduce_t(const tccl::BulkReduceArgs& a, dim3 grid, int ranks, hipStream_t stream) {
+void launch_reduce_t(const tccl::BulkReduceArgs& a, dim3 grid, int ranks, hipStream_t stream, const tccl::CommArgs* waits) {
+  if (waits) {
+    const dim3 block(kThreadsReady);
+    if (ranks == 2)
+      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 2>), grid, block, 0, stream, a, *waits);
+    else if (ranks == 4)
+      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 4>), grid, block, 0, stream, a, *waits);
+    else
+      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 8>), grid, block, 0, stream, a, *waits);
+    return;
+  }
   const dim3 block(tccl::kThreadsComm);
   if (ranks == 2)
     hipLaunchKernelGGL((reduce_kernel<PT, OT, 2>), grid, block, 0, stream, a);
@@ -767,24 +790,24 @@ void launch_reduce_t(const tccl::BulkReduceArgs& a, dim3 grid, int ranks, hipStr
 }
 
 int launch_bulk_reduce(tccl::BulkReduceArgs& a, int owners, int64_t rows, int partial_dtype, int out_dtype, const tccl_device_info& dev,
-                       hipStream_t stream) {
+                       hipStream_t stream, const tccl::CommArgs* waits = nullptr, int most_waiting = 0) {
   a.units = (int)(rows * a.upr);
   if (a.units <= 0 || owners <= 0) return 0;
   const int ranks = a.world <= 2 ? 2 : (a.world <= 4 ? 4 : 8);
-  const int64_t per_wg = (int64_t)tccl::kThreadsComm * (8 / ranks);
+  const int64_t per_wg = (int64_t)(waits ? kThreadsReady : tccl::kThreadsComm) * (8 / ranks);
   int64_t x = (a.units + per_wg - 1) / per_wg;
-  const int64_t most = (int64_t)dev.compute_units * TCCL_BULK_REDUCE_WGS / owners;
-  if (x > most) x = most;
+  const int64_t most = (waits ? (int64_t)most_waiting : (int64_t)dev.compute_units * TCCL_BULK_REDUCE_WGS) / owners;
+  if (x > most) x = most > 0 ? most : 1;
   const dim3 grid((unsigned)x, (unsigned)owners);
   const int key = partial_dtype * 4 + out_dtype;
   switch (key) {
-    case TCCL_F32 * 4 + TCCL_F32: launch_reduce_t<float, float>(a, grid, ranks, stream); break;
-    case TCCL_F32 * 4 + TCCL_F16: launch_reduce_t<float, _Float16>(a, grid, ranks, stream); break;
-    case TCCL_F32 * 4 + TCCL_BF16: launch_reduce_t<float, __bf16>(a, grid, ranks, stream); break;
-    case TCCL_F16 * 4 + TCCL_F16: launch_reduce_t<_Float16, _Float16>(a, grid, ranks, stream); break;
-    case TCCL_F16 * 4 + TCCL_BF16: launch_reduce_t<_Float16, __bf16>(a, grid, ranks, stream); break;
-    case TCCL_BF16 * 4 + TCCL_BF16: launch_reduce_t<__bf16, __bf16>(a, grid, ranks, stream); break;
-    case TCCL_BF16 * 4 + TCCL_F16: launch_reduce_t<__bf16, _Float16>(a, grid, ranks, stream); break;
+    case TCCL_F32 * 4 + TCCL_F32: launch_reduce_t<float, float>(a, grid, ranks, stream, waits); break;
+    case TCCL_F32 * 4 + TCCL_F16: launch_reduce_t<float, _Float16>(a, grid, ranks, stream, waits); break;
+    case TCCL_F32 * 4 + TCCL_BF16: launch_reduce_t<float, __bf16>(a, grid, ranks, stream, waits); break;
+    case TCCL_F16 * 4 + TCCL_F16: launch_reduce_t<_Float16, _Float16>(a, grid, ranks, stream, waits); break;
+    case TCCL_F16 * 4 + TCCL_BF16: launch_reduce_t<_Float16, __bf16>(a, grid, ranks, stream, waits); break;
+    case TCCL_BF16 * 4 + TCCL_BF16: launch_reduce_t<__bf16, __bf16>(a, grid, ranks, stream, waits); break;
+    case TCCL_BF16 * 4 + TCCL_F16: launch_reduce_t<__bf16, _Float16>(a, grid, ranks, stream, waits); break;
     default: return fail(TCCL_ERR_UNSUPPORTED, "reduce: no kernel for partial dtype %d, output dtype %d", partial_dtype, out_dtype);
   }
   TCCL_HIP(hipGetLastError());
@@ -792,7 +815,8 @@ int launch_bulk_reduce(tccl::BulkReduceArgs& a, int owners, int64_t rows, int pa
 }
 
 // The transfer of a GEMM + collective operation as a launch of its own (the second kernel of S0).
-int launch_bulk(const tccl::CommArgs& c, const tccl_device_info& dev, hipStream_t stream) {
+// waits: the reductions wait for the peers' words, with at most this many workgroups.
+int launch_bulk(const tccl::CommArgs& c, const tccl_device_info& dev, hipStream_t stream, int waits = 0) {
   const int span = check_comm_span(c);
   if (span) return span;
   if (c.op == tccl::kOpReduceScatter) {
@@ -809,7 +833,7 @@ int launch_bulk(const tccl::CommArgs& c, const tccl_device_info& dev, hipStream_
     a.dst_pitch = (uint32_t)c.ld_rs_out_bytes;
     a.upr = c.N / 8;
     a.first_owner = c.emulate_peer ? 0 : c.rank;
-    return launch_bulk_reduce(a, c.emulate_peer ? c.world : 1, shard, c.partial_dtype, c.out_dtype, dev, stream);
+    return launch_bulk_reduce(a, c.emulate_peer ? c.world : 1, shard, c.partial_dtype, c.out_dtype, dev, stream, waits > 0 ? &c : nullptr, waits);
   }
   tccl::BulkCopyArgs a;
   memset(&a, 0, sizeof a);
@@ -1076,6 +1100,18 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
                 const GatherSpec* gather = nullptr, const tccl_heap_view* heap = nullptr) {
   const int span = c.op != tccl::kOpNone ? check_comm_span(c) : 0;
   if (span) return span;
+  const bool traced = sync && (sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock || sync->trace_comm_counter);
+  // Reduce-scatter: may the sums be a launch of their own, behind a GEMM that stores and publishes partials?  They are wherever
+  // tiles cannot sum themselves (own rows in whole 256-row tiles, or one streaming tile per CU): communication workgroups
+  // beside a three-stage GEMM and a large-tile kernel's workgroups turning to the reductions after their tiles, which this
+  // launch replaced, took longer.  bf16 1792 x 3408 x 2144 on two ranks 85 -> 48 us, e4m3 13824 x 736 x 2496 on four 86 -> 50,
+  // e4m3 512 x 7056 x 1888 on four 75 -> 35.
+  const bool apart = c.op == tccl::kOpReduceScatter && variant != TCCL_S0_BULK && c.world > 1 && !traced && !(tr && tr->num_comm_wgs > 0);
+  // Workgroups that wait for a peer leave half of the CUs to the peer's own launches, unless this rank carries out the peer's
+  // half itself (nobody else is waited for then; the sums of 1024 x 3248 fp32 on two ranks take 11.0 us on half of the CUs, 8.3 on all).
+  const int most = c.emulate_peer ? 2 * dev.compute_units : dev.compute_units / 2;
+  const int waiters = d->num_wgs > 0 && d->num_wgs < most ? d->num_wgs : most;
+  const auto sums_apart = [&] { return launch_bulk(c, dev, stream, c.peers_resident ? 0 : waiters); };
   if (!gather) {
     // Tiles of a reduce-scatter must not straddle two owners' rows.
     const int64_t seg = g.wrap_rows > 0 ? g.wrap_rows : (c.op == tccl::kOpReduceScatter ? d->M / c.world : d->M);
@@ -1084,21 +1120,26 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     const bool waits = c.op == tccl::kOpReduceScatter && variant != TCCL_S0_BULK && !c.peers_resident && c.world > 1;
     if (shape >= 0 && !(waits && stream_tiles(shape, seg, 1, d->N) > dev.compute_units))
       return run_stream(d, c, sync, variant, shape, seg, dev, g, stream);
+    if (shape >= 0 && apart) {
+      tccl::CommArgs none = c;
+      none.op = tccl::kOpNone;
+      const int rc = run_stream(d, none, sync, variant, shape, seg, dev, g, stream);
+      c.granularity = none.granularity;
+      return rc ? rc : sums_apart();
+    }
   }
-  const bool traced = sync && (sync->trace_start_clock || sync->trace_ready_clock || sync->trace_done_clock || sync->trace_comm_counter);
-  // Does the launch carry nothing but pushes (reductions over resident partials follow as a kernel of their own)?
-  const bool resident_sums = c.op == tccl::kOpReduceScatter && c.peers_resident && !c.emulate_peer;
+  // Does the launch carry nothing but pushes?
   const bool lone = !gather && (variant == TCCL_S0_BULK ||
                                 (!traced && !(tr && tr->num_comm_wgs > 0) &&
-                                 (c.op == tccl::kOpReduceScatter ? resident_sums && c.world > 1
+                                 (c.op == tccl::kOpReduceScatter ? apart
                                                                  : c.world <= 1 || c.op != tccl::kOpAllGather || !(c.directions & tccl::kDirPull))));
   // A reduce-scatter on large tiles sums in their epilogue: the rule for launches that carry more decides there.
-  const bool sums_inside = variant != TCCL_S0_BULK && c.op == tccl::kOpReduceScatter && use_macro(d, dev, true);
+  const bool sums_inside = variant != TCCL_S0_BULK && use_macro(d, dev, true) && reduces_in_tiles(c) &&
+                           !(apart && c.world > 2 && !(d->flags & TCCL_GEMM_OWN_ROWS_IN_REGISTERS));
   TileKernel kernel = use_macro(d, dev, variant != TCCL_S0_BULK) ? kTiles256 : kTiles128;
   if (lone && !sums_inside) {
     const int segs = d->column_shards > 1 ? d->column_shards : 1;
-    const bool allow256 = plan_tile_fits_macro(d) && !(variant != TCCL_S0_BULK && c.op == tccl::kOpReduceScatter);
-    kernel = choose_tiles(d, d->M / segs, segs, allow256, variant != TCCL_S0_BULK && c.op != tccl::kOpReduceScatter && c.world > 1, dev).kernel;
+    kernel = choose_tiles(d, d->M / segs, segs, plan_tile_fits_macro(d), variant != TCCL_S0_BULK && c.op != tccl::kOpReduceScatter && c.world > 1, dev).kernel;
   }
   const int total_tiles = g.tile_rows * g.tile_cols;
   const int compute = tile_wgs(kernel, d, dev, total_tiles);
@@ -1139,9 +1180,18 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     memset(&f.gather, 0, sizeof f.gather);
     if (gather) {
       build_gather_background(d, *gather, heap, c, &f.pull, &f.gather);
-    } else if (build_reduce(c, sync, d->flags, &f.reduce, &f.m)) {
-      c.op = tccl::kOpNone;
+    } else if (!(apart && !sums_inside) && build_reduce(c, sync, d->flags, &f.reduce, &f.m)) {
       memset(&f.pull, 0, sizeof f.pull);
+      c.op = tccl::kOpNone;
+    } else if (apart) {
+      const int rc = [&] {
+        tccl::CommArgs none = c;
+        none.op = tccl::kOpNone;
+        memset(&f.pull, 0, sizeof f.pull);
+        f.comm = none;
+        return launch_fused256(d->in_dtype, d->out_dtype, f, wgs, stream);
+      }();
+      return rc ? rc : sums_apart();
     } else if (build_background(c, &f.pull)) {
       c.directions &= ~tccl::kDirPull;
     }
@@ -1174,20 +1224,16 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // launch keeps the pushes in the communication role, whose tasks carry the per-group clock stamps.
   tccl::PushArgs push;
   memset(&push, 0, sizeof push);
-  if (c.op == tccl::kOpReduceScatter && !traced && c.world > 1 && !(tr && tr->num_comm_wgs > 0)) {
-    // With the peers' partials there the sums follow as a kernel of their own: one in `world` tiles would do all the
-    // reading otherwise, on as many CUs (1024 x 4096 x 2048, four ranks: 37 us; GEMM and reduction one after the other
-    // 30 us; communication workgroups beside a three-stage GEMM 48 us).
-    if (resident_sums) {
-      const int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, kernel, compute, 0, nullptr, stream);
-      return rc ? rc : launch_bulk(c, dev, stream);
-    }
-    // Otherwise they happen in the epilogue.  Workgroups that wait for a peer's partials must leave room for the peer's own
-    // launch: at most one per CU (two fit).
-    if (c.peers_resident || compute <= dev.compute_units) {
-      const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
-      return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);
-    }
+  // Two ranks, at most a tile per CU, few K steps: the second launch costs more than 128-row tiles lose that sum in their
+  // epilogue (bf16, us, in the epilogue and apart: 4352 x 752 x 336 19.0 / 23.2, 3328 x 800 x 640 20.9 / 21.9, 2560 x 1536 x
+  // 1024 25.5 / 26.4; 1792 x 1200 x 1520 30.9 / 28.6, 1280 x 3136 x 3968 54.6 / 48.8).
+  if (apart && !c.peers_resident && c.world == 2 && compute <= dev.compute_units && kernel != kTilesWide && d->K <= 1024) {
+    const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
+    return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);
+  }
+  if (apart) {
+    const int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, kernel, compute, 0, nullptr, stream);
+    return rc ? rc : sums_apart();
   }
   if (!traced && build_push(c, g, &push)) {
     c.directions &= ~tccl::kDirPush;

@@ -65,7 +65,7 @@ struct BulkReduceArgs {
 };
 
 // kRanks: the most ranks this instantiation holds in registers at once (2, 4 or 8; world <= kRanks).
-template <typename PT, typename OT, int kRanks, int kThreads>
+template <typename PT, typename OT, int kRanks, int kThreads, int kLoadPolicy = kBulkReducePolicy>
 TCCL_D void bulk_reduce(const BulkReduceArgs& a, int owner, int wg, int num_wgs) {
   constexpr uint32_t kSrcUnit = 8 * sizeof(PT), kDstUnit = 8 * sizeof(OT);
   // Units per thread and round: 256 bytes of requests in flight per thread for fp32, 128 for the 16-bit types.
@@ -107,7 +107,7 @@ TCCL_D void bulk_reduce(const BulkReduceArgs& a, int owner, int wg, int num_wgs)
 #pragma unroll
         for (int k = 0; k < kUnits; ++k)
 #pragma unroll
-          for (int h = 0; h < (int)sizeof(PT) / 2; ++h) raw[k][i][h] = ld16<kBulkReducePolicy>(from[i], soff[k] + 16u * h);
+          for (int h = 0; h < (int)sizeof(PT) / 2; ++h) raw[k][i][h] = ld16<kLoadPolicy>(from[i], soff[k] + 16u * h);
       }
     float acc[kUnits][8];
 #pragma unroll
@@ -128,6 +128,34 @@ TCCL_D void bulk_reduce(const BulkReduceArgs& a, int owner, int wg, int num_wgs)
         if (live[k]) store8<OT, kBulkReducePolicy>(to, doff[k], acc[k]);
     }
   }
+}
+
+// ---- reductions that wait ---------------------------------------------------------------------------
+// The second launch of a reduce-scatter whose tiles do not sum themselves (run_variant() in tccl_api.hip): this rank's
+// partials are in memory, the peers' are once their words say so.  Every workgroup looks at all words of its owner's
+// rows, a word per lane; false if a bounded wait expired (the fault word is raised).
+template <int kThreads>
+TCCL_D bool rows_published(const CommArgs& c, int owner) {
+  const int64_t deadline = now_ticks() + c.spin_ticks;
+  const int shard = c.M / c.world, lo = owner * shard, hi = lo + shard;
+  bool ok = true;
+  for (int p = 0; p < c.world; ++p) {
+    if (p == c.rank) continue;
+    if (c.granularity == kPerTile) {
+      const int32_t* words = peer_words(c, c.locks, p);
+      const int first = lo / c.block_m, n = ((hi - 1) / c.block_m - first + 1) * c.tile_cols;
+      for (int i = (int)threadIdx.x; i < n && ok; i += kThreads)
+        ok = tile_wait_ge<true>(words, tile_id_of(first + i / c.tile_cols, i % c.tile_cols, c.tile_rows, c.tile_cols, c.group_m), c.epoch, deadline);
+    } else {
+      const int32_t* words = peer_words(c, c.counter, p);
+      for (int g = (int)threadIdx.x; g < c.n_groups && ok; g += kThreads)
+        if (group_hi(c, g) > lo && group_lo(c, g) < hi)
+          ok = tile_wait_ge<true>(words, g, (int32_t)((uint32_t)c.epoch * (uint32_t)c.tile_counts[g]), deadline);
+    }
+  }
+  const bool all = __syncthreads_and(ok ? 1 : 0) != 0;
+  if (!all && threadIdx.x == 0 && c.fault) *c.fault = 1;
+  return all;
 }
 
 }  // namespace tccl
