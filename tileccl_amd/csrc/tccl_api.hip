@@ -543,8 +543,9 @@ constexpr TileCost kCostDeep = {0.42, 0.13, 0.12, 2.0, 0.0, 1.5};
 constexpr TileCost kCost128 = {0.50, 0.15, 0.12, 0.5, 0.0, 1.5};   // one workgroup per CU
 constexpr TileCost kCost128Two = {1.25, 0.0, 0.10, 1.5, 0.0, 1.5}; // two: as soon as some CU has two
 
-double rounds_us(const TileCost& c, int64_t tiles, int slots, int K, bool pushes) {
-  const double steps = (K + 63) / 64, step = c.idle + (K % 32 ? c.misaligned : 0.0), end = c.stores + (pushes ? c.pushes : 0.0);
+double rounds_us(const TileCost& c, int64_t tiles, int slots, const tccl_gemm_desc* d, bool pushes) {
+  const bool aligned = d->lda % 32 == 0 && (!(d->flags & TCCL_GEMM_B_KMAJOR) || d->ldb % 32 == 0);
+  const double steps = (d->K + 63) / 64, step = c.idle + (aligned ? 0.0 : c.misaligned), end = c.stores + (pushes ? c.pushes : 0.0);
   const double rest = (double)(tiles % slots) / slots;
   double us = (double)(tiles / slots) * (steps * (step + c.busy) + end + c.stores_busy);
   if (rest > 0) us += steps * (step + c.busy * rest) + end + c.stores_busy * rest;
@@ -566,14 +567,14 @@ TileChoice choose_tiles(const tccl_gemm_desc* d, int64_t seg_rows, int64_t segs,
     return {allow256 && use_macro(d, dev, false) ? kTiles256 : kTiles128, 0};
   const int cus = dev.compute_units;
   const int64_t rows = (seg_rows + 127) / 128 * segs, small = rows * ((d->N + 127) / 128), wide = rows * ((d->N + 255) / 256);
-  TileChoice best = {kTiles128, small <= cus ? rounds_us(kCost128, small, cus, d->K, pushes) : rounds_us(kCost128Two, small, 2 * cus, d->K, pushes)};
+  TileChoice best = {kTiles128, small <= cus ? rounds_us(kCost128, small, cus, d, pushes) : rounds_us(kCost128Two, small, 2 * cus, d, pushes)};
   const auto offer = [&](TileKernel kernel, double us) {
     if (us < best.us) best = {kernel, us};
   };
-  if (small <= cus) offer(kTiles128Deep, rounds_us(kCostDeep, small, cus, d->K, pushes));
-  if (small > cus) offer(kTilesWide, rounds_us(kCostWide, wide, cus, d->K, pushes));
+  if (small <= cus) offer(kTiles128Deep, rounds_us(kCostDeep, small, cus, d, pushes));
+  if (small > cus) offer(kTilesWide, rounds_us(kCostWide, wide, cus, d, pushes));
   if (allow256 && (segs == 1 || seg_rows % 256 == 0))
-    offer(kTiles256, rounds_us(kCost256, (seg_rows + 255) / 256 * segs * ((d->N + 255) / 256), cus, d->K, pushes));
+    offer(kTiles256, rounds_us(kCost256, (seg_rows + 255) / 256 * segs * ((d->N + 255) / 256), cus, d, pushes));
   return best;
 }
 
