@@ -1524,6 +1524,7 @@ struct Gemm256 {
   TCCL_D bool reduce_wait(ReducePtr ra, const SignalArgs& s, int mm, int mn) const {
     if (ra->peers_resident) return true;  // the same for every wavefront
     volatile int* verdict = (volatile int*)lds1;
+    __syncthreads();  // the other wavefronts' loads past the last step have landed in that stage
     if (tid == 0) {
       bool ok = true;
       const int64_t deadline = now_ticks() + ra->spin_ticks;
