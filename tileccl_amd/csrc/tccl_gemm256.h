@@ -1591,25 +1591,36 @@ struct Gemm256 {
         dst[k] = (uint32_t)((r * ld_out + c * kE) * 2);
         mine[k] = ld16<0>(r_mine, src[k]);  // written by this workgroup itself: a plain load sees it
       }
-      for (int step = 0; step < world; ++step) {
-        // owner first, then the other ranks in ascending order
-        const int p = step == 0 ? owner : (step - 1 < owner ? step - 1 : step);
-        u32x4 addend[kUnroll];
-        if (p == rank) {
+      // Owner first, then the other ranks in ascending order.  The addends of four ranks are requested before the first is
+      // added (rank by rank, each batch waited a trip to memory per rank: four ranks emulated, fp16 4096 x 4752 x 1472
+      // 171.6 -> 168.5 us, 8192 x 2352 x 976 153.9 -> 152.5).
+      constexpr int kPeers = 4;
+      for (int s0 = 0; s0 < world; s0 += kPeers) {
+        u32x4 addend[kPeers][kUnroll];
 #pragma unroll
-          for (int k = 0; k < kUnroll; ++k) addend[k] = mine[k];
-        } else {
-          const __amdgpu_buffer_rsrc_t r_peer = window((int64_t)(uintptr_t)g.C + (ra->heap_bases[p] - my_base) + tile_off);
+        for (int i = 0; i < kPeers; ++i) {
+          const int step = s0 + i, p = step == 0 ? owner : (step - 1 < owner ? step - 1 : step);
+          if (step >= world) break;
+          if (p == rank) {
 #pragma unroll
-          for (int k = 0; k < kUnroll; ++k) addend[k] = ld16<kCoherent>(r_peer, src[k]);
+            for (int k = 0; k < kUnroll; ++k) addend[i][k] = mine[k];
+          } else {
+            const __amdgpu_buffer_rsrc_t r_peer = window((int64_t)(uintptr_t)g.C + (ra->heap_bases[p] - my_base) + tile_off);
+#pragma unroll
+            for (int k = 0; k < kUnroll; ++k) addend[i][k] = ld16<kCoherent>(r_peer, src[k]);
+          }
         }
 #pragma unroll
-        for (int k = 0; k < kUnroll; ++k) {
-          float f[8];
-          int n;
-          unpack(addend[k], f, n);
+        for (int i = 0; i < kPeers; ++i) {
+          if (s0 + i >= world) break;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) sum[k][e] = step == 0 ? f[e] : sum[k][e] + f[e];
+          for (int k = 0; k < kUnroll; ++k) {
+            float f[8];
+            int n;
+            unpack(addend[i][k], f, n);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[k][e] = s0 + i == 0 ? f[e] : sum[k][e] + f[e];
+          }
         }
       }
 #pragma unroll
