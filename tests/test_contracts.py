@@ -313,3 +313,49 @@ def test_spill_check_tells_reduce_scatter_kernels_apart():
     assert is_reduce("_ZN4tccl15fused256_kernelINS_7fp8e4m3EDF16bLb1ELb0ELb1ELb1EEEvNS_12Fused256ArgsE")
     assert not is_reduce("_ZN4tccl15fused256_kernelIDF16_DF16_Lb0ELb1ELb0ELb1EEEvNS_12Fused256ArgsE")
     assert not is_reduce("_ZN4tccl14gemm256_kernelIDF16_fLb1EEEvNS_8GemmArgsENS_5MacroE")
+
+
+LISTING = """
+	v_readlane_b32 s9, v253, 60
+.LBB0_1:
+	s_mov_b32 m0, s1
+	s_nop {nop}
+	buffer_load_dwordx4 v217, s[48:51], s9 offen lds
+	s_cbranch_scc1 .LBB0_1
+	s_endpgm
+"""
+
+
+def test_listing_check_counts_wait_states_across_blocks():
+    """A scalar register written by a vector instruction is read by a vector memory instruction five wait states later at the
+    earliest, whichever way control came; s_nop n is n + 1 of them, a scalar write in between ends the wait."""
+    from tileccl_amd.csrc.check_spills import early_reads
+
+    assert early_reads(LISTING.format(nop=0).split("\n")) == [(5, 1)]
+    assert early_reads(LISTING.format(nop=2).split("\n")) == [(5, 1)]
+    assert early_reads(LISTING.format(nop=3).split("\n")) == []
+    assert early_reads(LISTING.replace("v_readlane_b32 s9", "v_readlane_b32 s8").format(nop=0).split("\n")) == []
+    assert early_reads(LISTING.replace("s_nop {nop}", "s_mov_b32 s9, 0").split("\n")) == []
+    # the loop's own branch is the only way to its first line here
+    looped = LISTING.format(nop=0).replace("\tv_readlane_b32 s9, v253, 60\n", "\ts_endpgm\n").replace("\ts_cbranch", "\tv_readfirstlane_b32 s50, v1\n\ts_cbranch")
+    assert early_reads(looped.split("\n")) == [(5, 6)]
+    assert early_reads(looped.replace("\ts_cbranch", "\ts_nop 1\n\ts_cbranch").split("\n")) == []
+
+
+def test_loads_written_as_assembly_wait_for_their_scalar_registers_themselves():
+    """The compiler does not look inside inline assembly: a block with a load spends the five wait states before it."""
+    import re
+    from pathlib import Path
+
+    import tileccl_amd
+    from tileccl_amd.csrc.check_spills import WAIT_STATES, decode, states
+
+    blocks = 0
+    for header in sorted((Path(tileccl_amd.__file__).parent / "csrc").glob("*.h")):
+        for asm in re.findall(r"asm volatile\(((?:\s*\"[^\"]*\")+)", header.read_text()):
+            lines = [decode(line) for line in "".join(re.findall(r'"([^"]*)"', asm)).replace("\\t", "").split("\\n")]
+            loads = [i for i, ins in enumerate(lines) if ins and ins[0].startswith("buffer_load")]
+            if loads:
+                blocks += 1
+                assert sum(states(*ins) for ins in lines[:loads[0]]) >= WAIT_STATES, (header.name, asm)
+    assert blocks

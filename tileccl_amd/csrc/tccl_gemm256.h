@@ -302,18 +302,29 @@ struct Gemm256 {
   // an LDS array wait for all loads into it, whichever part they go to; the waits are k_step's own.  Bytes past the
   // descriptor's end (scalar offset included) read as zero.  A load that reads M0 wants an instruction between it and
   // the write of M0.  Every global -> LDS load of this kernel sets M0 itself.
+  // A scalar register that a vector instruction has written (v_readlane of a spilled one, v_readfirstlane) may be read by a
+  // vector memory instruction five wait states later; the hardware does not wait and the compiler does not look in here, so
+  // each block spends five before its first load (check_spills.py looks at the listing, too).
   static TCCL_D void dma16(char* to, Words4 from, uint32_t lane_off, uint32_t off) {
     const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(lane_off), "s"(from), "s"(off) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(lane_off), "s"(from), "s"(off) : "memory");
+  }
+  // Two of them: the wait states once.
+  static TCCL_D void dma16_pair(char* to0, char* to1, Words4 from, const uint32_t (&lane_off)[2], uint32_t off) {
+    const uint32_t dst0 = (uint32_t)(uintptr_t)(LdsVoid*)to0, dst1 = (uint32_t)(uintptr_t)(LdsVoid*)to1;
+    asm volatile(
+        "s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
+        "s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, %5 offen lds" ::"s"(dst0), "s"(dst1), "v"(lane_off[0]), "v"(lane_off[1]), "s"(from), "s"(off)
+        : "memory");
   }
   // The same past the caches (what a peer has written), 16 and 4 bytes per lane.
   static TCCL_D void dma16_coherent(char* to, Words4 from, uint32_t lane_off) {
     const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
   }
   static TCCL_D void dma4_coherent(char* to, Words4 from, uint32_t lane_off) {
     const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
   }
   template <int kLeft>
   static TCCL_D void wait_loads() {  // until at most kLeft of this wavefront's vector memory operations are under way
@@ -401,15 +412,19 @@ struct Gemm256 {
   // Half h of an operand of K step kt into `stage`: two loads (only_i: one of them).
   TCCL_D void issue_a(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
     const uint32_t off = (uint32_t)(kGatherA ? kt - s.kt_base : kt) * s.step_a + h * s.half_a;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if (only_i < 0 || only_i == i) dma16(stage + a_row(h, i) * kARow256, s.a, s.off_a[i], off);
+    if (only_i < 0)
+      dma16_pair(stage + a_row(h, 0) * kARow256, stage + a_row(h, 1) * kARow256, s.a, s.off_a, off);
+    else
+      dma16(stage + a_row(h, only_i) * kARow256, s.a, s.off_a[only_i], off);
   }
   TCCL_D void issue_b(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
+    constexpr int kPitch = kBKMajor ? kARow256 : kBPitch;
     const uint32_t off = (uint32_t)kt * s.step_b + h * s.half_b;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if (only_i < 0 || only_i == i) dma16(stage + kAStage256 + b_row(h, i) * (kBKMajor ? kARow256 : kBPitch), s.b, s.off_b[i], off);
+    char* to = stage + kAStage256;
+    if (only_i < 0)
+      dma16_pair(to + b_row(h, 0) * kPitch, to + b_row(h, 1) * kPitch, s.b, s.off_b, off);
+    else
+      dma16(to + b_row(h, only_i) * kPitch, s.b, s.off_b[only_i], off);
   }
   // Ahead of the first load of K step kt (steps come in ascending order): from the step that reaches past K on, chunks at
   // k >= K are redirected past the end of the buffer for good and read as zero (row-major B rows >= K lie past it already).
