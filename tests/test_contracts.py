@@ -359,3 +359,19 @@ def test_loads_written_as_assembly_wait_for_their_scalar_registers_themselves():
                 blocks += 1
                 assert sum(states(*ins) for ins in lines[:loads[0]]) >= WAIT_STATES, (header.name, asm)
     assert blocks
+
+
+def test_assembly_that_writes_m0_says_so():
+    """M0 may hold something of the compiler's: a block that sets it names it among what it changes."""
+    import re
+    from pathlib import Path
+
+    import tileccl_amd
+
+    blocks = 0
+    for header in sorted((Path(tileccl_amd.__file__).parent / "csrc").glob("*.h")):
+        for asm in re.findall(r"asm volatile\(.*?\);", header.read_text(), flags=re.S):
+            if "s_mov_b32 m0" in asm:
+                blocks += 1
+                assert re.search(r':\s*"memory", "m0"\)', asm), (header.name, asm)
+    assert blocks

@@ -298,16 +298,18 @@ struct Gemm256 {
     d[3] = 0x00020000u;
     return d;
   }
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
   // 16 bytes per lane, global -> LDS, lane l's to `to` + 16 l.  Written out because the compiler makes every later read of
   // an LDS array wait for all loads into it, whichever part they go to; the waits are k_step's own.  Bytes past the
   // descriptor's end (scalar offset included) read as zero.  A load that reads M0 wants an instruction between it and
-  // the write of M0.  Every global -> LDS load of this kernel sets M0 itself.
+  // the write of M0, which each block says that it writes (the compiler reserves M0, hence the warnings switched off).
   // A scalar register that a vector instruction has written (v_readlane of a spilled one, v_readfirstlane) may be read by a
   // vector memory instruction five wait states later; the hardware does not wait and the compiler does not look in here, so
   // each block spends five before its first load (check_spills.py looks at the listing, too).
   static TCCL_D void dma16(char* to, Words4 from, uint32_t lane_off, uint32_t off) {
     const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(lane_off), "s"(from), "s"(off) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(lane_off), "s"(from), "s"(off) : "memory", "m0");
   }
   // Two of them: the wait states once.
   static TCCL_D void dma16_pair(char* to0, char* to1, Words4 from, const uint32_t (&lane_off)[2], uint32_t off) {
@@ -315,17 +317,18 @@ struct Gemm256 {
     asm volatile(
         "s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
         "s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, %5 offen lds" ::"s"(dst0), "s"(dst1), "v"(lane_off[0]), "v"(lane_off[1]), "s"(from), "s"(off)
-        : "memory");
+        : "memory", "m0");
   }
   // The same past the caches (what a peer has written), 16 and 4 bytes per lane.
   static TCCL_D void dma16_coherent(char* to, Words4 from, uint32_t lane_off) {
     const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory", "m0");
   }
   static TCCL_D void dma4_coherent(char* to, Words4 from, uint32_t lane_off) {
     const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory", "m0");
   }
+#pragma clang diagnostic pop
   template <int kLeft>
   static TCCL_D void wait_loads() {  // until at most kLeft of this wavefront's vector memory operations are under way
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLeft) : "memory");
