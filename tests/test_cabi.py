@@ -99,6 +99,22 @@ def test_bad_descriptors_are_rejected_on_the_host(lib):
     assert lib.tccl_fill_i32(None, 0, 0, None) == 0
 
 
+def test_operands_end_below_the_offsets_that_read_as_zero(lib):
+    """The kernels fetch what they must not read at offset 2^32 - 16: an operand that reaches it is refused, one that ends there is not."""
+    from tileccl_amd import _lib
+
+    d = _lib.GemmDesc()
+    d.A = d.B = d.C = 0x1000
+    d.in_dtype, d.out_dtype = _lib.F8E4M3, _lib.BF16
+    d.block_m, d.block_n, d.group_m = 128, 128, 8
+    d.M, d.K, d.lda, d.ldb = 16, 16, 16, 0xFFFFFF00 // 15
+    for n, refused in ((248, True), (240, False)):  # B's last row ends at 2^32 - 8, 2^32 - 16
+        d.N = d.ldc = n
+        assert (d.K - 1) * d.ldb + n == 2**32 - (8 if refused else 16)
+        assert lib.tccl_gemm(C.byref(d), None) != 0
+        assert (b"spans more than 4 GiB" in lib.tccl_last_error_string()) == refused, lib.tccl_last_error_string()
+
+
 @pytest.mark.parametrize("tile_rows,tile_cols,group_m", [(32, 32, 8), (12, 2, 8), (7, 5, 3), (1, 9, 8), (64, 32, 8), (5, 1, 1)])
 def test_device_tile_order_equals_the_reference_swizzle(lib, tile_rows, tile_cols, group_m):
     tm, tn = C.c_int32(), C.c_int32()

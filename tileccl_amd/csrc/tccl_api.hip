@@ -301,11 +301,13 @@ int check_gemm(const tccl_gemm_desc* d, bool ragged_shards = false) {
     return fail(TCCL_ERR_UNSUPPORTED, "gemm: A, B, C rows must start on 16-byte boundaries");
   // The kernels address an operand with 32-bit byte offsets from a per-tile base: B from its
   // first row down to row K-1 (k-major B: over the 256 columns of a tile), A and C over the 256 rows of a tile.
-  const int64_t limit = 0xffffffffll;
+  // Offsets from 0xfffffff0 on mean "reads as zero" there; A, a k-major B and 16-bit ones are whole 16-byte vectors and never
+  // that long unless they are longer.
+  const int64_t limit = 0xffffffffll, operand_limit = 0xfffffff0ll;
   const int64_t b_span = (b_kmajor ? 255 * d->ldb + d->K : (int64_t)(d->K - 1) * d->ldb + (int64_t)d->N * shards) * (int64_t)isz;
   const int64_t a_span = (255 * d->lda + d->K) * (int64_t)isz;
   const int64_t c_span = (255 * d->ldc + d->N) * (int64_t)osz;
-  if (b_span > limit || a_span > limit || c_span > limit)
+  if (b_span > operand_limit || a_span > operand_limit || c_span > limit)
     return fail(TCCL_ERR_UNSUPPORTED, "gemm: an operand spans more than 4 GiB from a tile's base (B %lld, A %lld, C %lld bytes)",
                 (long long)b_span, (long long)a_span, (long long)c_span);
   return 0;

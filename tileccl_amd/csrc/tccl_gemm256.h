@@ -301,8 +301,8 @@ struct Gemm256 {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
   // 16 bytes per lane, global -> LDS, lane l's to `to` + 16 l.  Written out because the compiler makes every later read of
-  // an LDS array wait for all loads into it, whichever part they go to; the waits are k_step's own.  Bytes past the
-  // descriptor's end (scalar offset included) read as zero.  A load that reads M0 wants an instruction between it and
+  // an LDS array wait for all loads into it, whichever part they go to; the waits are k_step's own.  A lane reads zero
+  // where its offset is not below the descriptor's size less the scalar offset, which must not exceed the size: within().  A load that reads M0 wants an instruction between it and
   // the write of M0, which each block says that it writes (the compiler reserves M0, hence the warnings switched off).
   // A scalar register that a vector instruction has written (v_readlane of a spilled one, v_readfirstlane) may be read by a
   // vector memory instruction five wait states later; the hardware does not wait and the compiler does not look in here, so
@@ -354,9 +354,14 @@ struct Gemm256 {
       if (kt >= s.kt_switch) select_shard(s, kt);
   }
 
-  // (Less than kDeadOffset: an offset of that size is past the end of every window.)
+  // An offset that is past the end of every window, and the largest window (check_gemm).
   static constexpr uint32_t kDeadOffset = 0xfffffff0u;
-  static TCCL_D uint32_t clamp_u32(int64_t v) { return v > 0xffffff00ll ? 0xffffff00u : (v < 0 ? 0u : (uint32_t)v); }
+  static TCCL_D uint32_t clamp_u32(int64_t v) { return v > (int64_t)kDeadOffset ? kDeadOffset : (v < 0 ? 0u : (uint32_t)v); }
+
+  // A scalar offset no larger than the window: beyond that nothing says what the hardware's difference is.  At the window's size
+  // every lane reads zero.  It happens in steps that count: the second half of a last step whose rows of B are all past K,
+  // the lower rows of a last tile of few rows.
+  static TCCL_D uint32_t within(Words4 window, uint32_t off) { return off < window[2] ? off : window[2]; }
 
   TCCL_D int a_row(int h, int i) const { return (wave >> 2) * 128 + h * 64 + (wave & 3) * 16 + 8 * i; }
   TCCL_D int b_row(int h, int i) const {
@@ -414,7 +419,7 @@ struct Gemm256 {
 
   // Half h of an operand of K step kt into `stage`: two loads (only_i: one of them).
   TCCL_D void issue_a(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
-    const uint32_t off = (uint32_t)(kGatherA ? kt - s.kt_base : kt) * s.step_a + h * s.half_a;
+    const uint32_t off = within(s.a, (uint32_t)(kGatherA ? kt - s.kt_base : kt) * s.step_a + h * s.half_a);
     if (only_i < 0)
       dma16_pair(stage + a_row(h, 0) * kARow256, stage + a_row(h, 1) * kARow256, s.a, s.off_a, off);
     else
@@ -422,7 +427,7 @@ struct Gemm256 {
   }
   TCCL_D void issue_b(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
     constexpr int kPitch = kBKMajor ? kARow256 : kBPitch;
-    const uint32_t off = (uint32_t)kt * s.step_b + h * s.half_b;
+    const uint32_t off = within(s.b, (uint32_t)kt * s.step_b + h * s.half_b);
     char* to = stage + kAStage256;
     if (only_i < 0)
       dma16_pair(to + b_row(h, 0) * kPitch, to + b_row(h, 1) * kPitch, s.b, s.off_b, off);
