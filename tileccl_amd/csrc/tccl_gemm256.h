@@ -54,8 +54,9 @@
 // wavefronts in step, the next step's loads in the first four items, `s_waitcnt vmcnt(0)` + barrier before the last.  There the
 // transfer's bookkeeping, loads and stores fall into the slack of the older wavefronts; between the phases' barriers every
 // clock of it holds up both sides (4096 x 4096 x 1024, pushing and pulling: 41.9 us at best with the phases, four splits of the
-// transfer over them tried, 40.4 with the items; 4096 x 4096 x 2048 with its inputs gathered: 64.4 and 62.6).
-
+// transfer over them tried, 40.4 with the items; 4096 x 4096 x 2048 with its inputs gathered: 64.4 and 62.6).  Its operand loads are the
+// compiler's, into two LDS arrays (a read of one stage does not wait for a load into the other).
+//
 // The swapped-operand MFMA and the slab-wise epilogue are those of tccl_gemm.h.
 //
 // A macro tile covers (256/block_m) x (256/block_n) plan tiles; when it is stored, each of
@@ -117,8 +118,9 @@ struct ReduceArgs {
 // A peer's block is cut into pieces of kPieceUnits units of 16 bytes; pulling wavefront w of
 // the launch (the kPullWaves older wavefronts of every workgroup, see below) owns pieces w,
 // w + W, w + 2W, ... (W = pulling wavefronts in the grid), so at any moment the grid sweeps a
-// contiguous stretch.  Once per K step such a wavefront stores the piece it requested a step before and
-// requests its next one, global -> LDS like the operands, into landing bytes of its own.  A
+// contiguous stretch.  In every K step, behind the step's operand loads, such a wavefront
+// requests its next piece into registers; the step's barrier waits for this wave's loads
+// anyway, and mid-way through the following step the piece is stored.  A
 // piece is fetched only once
 // the TileGroups covering its rows are complete on the peer (counter[g] >= epoch *
 // tile_counts[g], the readiness rule of tileccl_v2/signal.py:43-66); that is found out by
@@ -177,10 +179,10 @@ struct GatherArgs {
 // Of a SIMD's two wavefronts the older one (wavefronts 0..3 of the workgroup) wins the matrix pipe and reaches each K step's
 // barrier early, while the younger one runs alone for the rest of the step; what the older one does besides is covered by the
 // younger one's MFMAs.  The pull is carried by the older wavefronts alone, two 16-byte units per lane and step.
+constexpr int kBgWordBytes = 8 * 256;                   // a fetched counter word per wavefront (64 lanes x 4 B)
 constexpr int kPullWaves = 4;                           // wavefronts of a workgroup that pull
 constexpr int kPullLoads = 2;                           // 16-byte units per lane and piece
 constexpr int kPieceUnits = 64 * kPullLoads;            // units per piece
-constexpr int kBgLandingBytes = kPullWaves * (16 * kPieceUnits + 256);  // per pulling wavefront: a piece, a counter word per lane
 
 TCCL_HD TileCoord macro_coords(int id, const Macro& m) {
   const int per_band = m.rows_per_band * m.cols;
@@ -238,26 +240,25 @@ struct Gemm256 {
   const int push_offset;    // byte offset of a PushArgs in the kernel arguments; < 0: no push
   const int reduce_offset;  // byte offset of a ReduceArgs in the kernel arguments; < 0: none
   const int gather_offset;  // byte offset of a GatherArgs in the kernel arguments (kGatherA only)
-  char* lds;   // stage 0 (also the epilogue's staging area), stage 1 behind it
+  char* lds;   // stage 0 (also the epilogue's staging area); without kPull, stage 1 lies behind it
   char* lds1;  // stage 1
-  char* bgw;   // landing bytes of the background transfer's pieces and counter fetches
+  char* bgw;   // landing words of the background transfer's counter fetches
   const int tid, lane, wave, wm, wn;
   // A per-lane value the optimiser must treat as new at this point (blocks hoisting of what is derived from it).
   static TCCL_D int fresh(int v) {
     asm volatile("" : "+v"(v));
     return v;
   }
-  // The lane's number, counted afresh (two instructions): what the per-step code of the background
-  // transfer derives from it is then formed where it is used instead of sitting in registers through
-  // the K loop.
   // A wavefront-uniform sum the optimiser must take as a whole: split up, its loop-invariant part is added
   // to the per-lane offsets ahead of the K loop, one register per combination.
   static TCCL_D uint32_t whole(uint32_t v) {
     asm("" : "+s"(v));
     return v;
   }
+  // The lane's number, counted afresh (two instructions): what the per-step code of the background
+  // transfer derives from it is then formed where it is used instead of sitting in registers through
+  // the K loop.
   static TCCL_D int lane_now() { return fresh((int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
-
 
   TCCL_D Gemm256(const GemmArgs& args, int pull_args_offset, int push_args_offset, int reduce_args_offset, char* stage0,
                  char* stage1, char* landing_words, int gather_args_offset = -1)
@@ -281,22 +282,35 @@ struct Gemm256 {
   // a_row() and b_row() give a piece's first row; lane l fetches row + l / 8, slot l % 8 of it (row-major B, 16-bit: k row +
   // l / 32, slot l % 32; fp8: k row + l / 16, slot l % 16).
   typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
+  template <bool kOne, typename One, typename Other>
+  struct Either {
+    typedef One Type;
+  };
+  template <typename One, typename Other>
+  struct Either<false, One, Other> {
+    typedef Other Type;
+  };
+  typedef typename Either<kPull, __amdgpu_buffer_rsrc_t, Words4>::Type Window;  // a buffer descriptor, as the loads take it
   struct Source {
-    Words4 a, b;                  // buffer descriptors
+    Window a, b;
     uint32_t off_a[2], off_b[2];  // this lane's byte offsets in the two pieces of half 0, K step 0
     uint32_t half_a, half_b;      // distance of half 1
     uint32_t step_a, step_b;
     // kGatherA: `a` is the window onto the shard that holds K steps [kt_base, kt_switch)
     int kt_base, kt_switch, row0;
   };
-  static TCCL_D Words4 descriptor(const void* p, uint32_t bytes) {
-    const uint64_t a = (uint64_t)(uintptr_t)p;
-    Words4 d;
-    d[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
-    d[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
-    d[2] = __builtin_amdgcn_readfirstlane(bytes);
-    d[3] = 0x00020000u;
-    return d;
+  static TCCL_D Window descriptor(const void* p, uint32_t bytes) {
+    if constexpr (kPull) {
+      return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00020000);
+    } else {
+      const uint64_t a = (uint64_t)(uintptr_t)p;
+      Words4 d;
+      d[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+      d[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
+      d[2] = __builtin_amdgcn_readfirstlane(bytes);
+      d[3] = 0x00020000u;
+      return d;
+    }
   }
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
@@ -307,26 +321,13 @@ struct Gemm256 {
   // A scalar register that a vector instruction has written (v_readlane of a spilled one, v_readfirstlane) may be read by a
   // vector memory instruction five wait states later; the hardware does not wait and the compiler does not look in here, so
   // each block spends five before its first load (check_spills.py looks at the listing, too).
-  static TCCL_D void dma16(char* to, Words4 from, uint32_t lane_off, uint32_t off) {
-    const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(lane_off), "s"(from), "s"(off) : "memory", "m0");
-  }
-  // Two of them: the wait states once.
+  // (Two loads to a block: the wait states once.)
   static TCCL_D void dma16_pair(char* to0, char* to1, Words4 from, const uint32_t (&lane_off)[2], uint32_t off) {
     const uint32_t dst0 = (uint32_t)(uintptr_t)(LdsVoid*)to0, dst1 = (uint32_t)(uintptr_t)(LdsVoid*)to1;
     asm volatile(
         "s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
         "s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, %5 offen lds" ::"s"(dst0), "s"(dst1), "v"(lane_off[0]), "v"(lane_off[1]), "s"(from), "s"(off)
         : "memory", "m0");
-  }
-  // The same past the caches (what a peer has written), 16 and 4 bytes per lane.
-  static TCCL_D void dma16_coherent(char* to, Words4 from, uint32_t lane_off) {
-    const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory", "m0");
-  }
-  static TCCL_D void dma4_coherent(char* to, Words4 from, uint32_t lane_off) {
-    const uint32_t dst = (uint32_t)(uintptr_t)(LdsVoid*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen sc0 sc1 lds" ::"s"(dst), "v"(lane_off), "s"(from) : "memory", "m0");
   }
 #pragma clang diagnostic pop
   template <int kLeft>
@@ -336,7 +337,7 @@ struct Gemm256 {
   typedef const __attribute__((address_space(4))) GatherArgs* GatherPtr;
 
   // Point `s.a` at the shard that holds K step kt (kGatherA).  Steps past K stay on the last
-  // shard: their chunks are redirected past the end of the window by mask() and read as zero.
+  // shard: their chunks are redirected past the end of the window by issue_piece() and read as zero.
   TCCL_D void select_shard(Source& s, int kt) const {
     const GatherPtr ga = late_kernarg_ptr<GatherArgs>(gather_offset);
     const int per_shard = ga->k_shard / kStepK;
@@ -417,22 +418,28 @@ struct Gemm256 {
     return s;
   }
 
-  // Half h of an operand of K step kt into `stage`: two loads (only_i: one of them).
-  TCCL_D void issue_a(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
-    const uint32_t off = within(s.a, (uint32_t)(kGatherA ? kt - s.kt_base : kt) * s.step_a + h * s.half_a);
-    if (only_i < 0)
-      dma16_pair(stage + a_row(h, 0) * kARow256, stage + a_row(h, 1) * kARow256, s.a, s.off_a, off);
-    else
-      dma16(stage + a_row(h, only_i) * kARow256, s.a, s.off_a[only_i], off);
+  // Half h of an operand of K step kt into `stage`: two loads.
+  TCCL_D void issue_a(char* stage, const Source& s, int kt, int h) const {
+    const uint32_t off = within(s.a, (uint32_t)kt * s.step_a + h * s.half_a);
+    dma16_pair(stage + a_row(h, 0) * kARow256, stage + a_row(h, 1) * kARow256, s.a, s.off_a, off);
   }
-  TCCL_D void issue_b(char* stage, const Source& s, int kt, int h, int only_i = -1) const {
+  TCCL_D void issue_b(char* stage, const Source& s, int kt, int h) const {
     constexpr int kPitch = kBKMajor ? kARow256 : kBPitch;
     const uint32_t off = within(s.b, (uint32_t)kt * s.step_b + h * s.half_b);
     char* to = stage + kAStage256;
-    if (only_i < 0)
-      dma16_pair(to + b_row(h, 0) * kPitch, to + b_row(h, 1) * kPitch, s.b, s.off_b, off);
-    else
-      dma16(to + b_row(h, only_i) * kPitch, s.b, s.off_b[only_i], off);
+    dma16_pair(to + b_row(h, 0) * kPitch, to + b_row(h, 1) * kPitch, s.b, s.off_b, off);
+  }
+  // The same loads one by one in a launch with a pull: piece i (half i / 2) of K step kt.  Chunks at k >= K are redirected past
+  // the end of the buffer so that they read as zero (row-major B rows >= K already lie past it).
+  TCCL_D void issue_piece(char* stage, const Source& s, int kt, int i) const {
+    const int h = i >> 1, j = i & 1;
+    const int kc = (lane & 7) ^ ((4 * j + (lane >> 4)) & 7);  // as in make_source
+    const bool dead = kt * kStepK + kc * kChunkK >= g.K;
+    const uint32_t oa = dead ? kDeadOffset : s.off_a[j] + ((kGatherA ? kt - s.kt_base : kt) * s.step_a + h * s.half_a);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.a, (LdsVoid*)(stage + a_row(h, j) * kARow256), 16, oa, 0, 0, 0);
+    uint32_t ob = s.off_b[j] + whole(kt * s.step_b + h * s.half_b);
+    if constexpr (kBKMajor) ob = dead ? kDeadOffset : ob;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.b, (LdsVoid*)(stage + kAStage256 + b_row(h, j) * (kBKMajor ? kARow256 : kBPitch)), 16, ob, 0, 0, 0);
   }
   // Ahead of the first load of K step kt (steps come in ascending order): from the step that reaches past K on, chunks at
   // k >= K are redirected past the end of the buffer for good and read as zero (row-major B rows >= K lie past it already).
@@ -452,13 +459,16 @@ struct Gemm256 {
   }
   // What the loop expects to be under way when it starts, in the order in which the first steps need it.
   TCCL_D void issue_first(Source& s) const {
-    mask_a(s, 0);
-    mask_b(s, 0);
-    issue_b(lds, s, 0, 0);
-    issue_b(lds, s, 0, 1);
-    issue_a(lds, s, 0, 0);
-    issue_a(lds, s, 0, 1);
-    if constexpr (!kPull) {
+    if constexpr (kPull) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) issue_piece(lds, s, 0, i);
+    } else {
+      mask_a(s, 0);
+      mask_b(s, 0);
+      issue_b(lds, s, 0, 0);
+      issue_b(lds, s, 0, 1);
+      issue_a(lds, s, 0, 0);
+      issue_a(lds, s, 0, 1);
       mask_b(s, 1);
       issue_b(lds1, s, 1, 0);
       if constexpr (kFp8) issue_b(lds1, s, 1, 1);
@@ -587,17 +597,14 @@ struct Gemm256 {
     int32_t need;            // epoch * tile_counts[gidx]: what the counters of group gidx must reach
     uint32_t group_units;    // ready_units once group gidx is complete
     int backoff;             // K steps to let pass before the counters are fetched again
-    // What every K step looks at.  `left` = pieces of this wavefront, one stride apart from `next_lp` on, that are whole, lie in
-    // the selected block and may be fetched; `pending` = a piece is on its way into the landing bytes (it is
-    // stored before the next one is requested); `over` = nothing left to learn.
-    int left;
-    bool pending, over, placed;
-    Words4 src;
-    // Where this lane's units of the next piece lie inside the block (byte offsets on either side, column), carried from piece
-    // to piece by additions; where the pending one goes.
-    uint32_t to[kPullLoads], from[kPullLoads], col[kPullLoads], pend_to[kPullLoads];
-    uint32_t step_to, step_from, step_col, wrap_to, wrap_from;
-    int landing;             // this wavefront's landing bytes: the piece, behind it the counter words
+    int pend_lp;             // piece of the selected block that was requested and is not yet stored (-1: none)
+    // The piece itself.  One set of registers: a piece is stored (pull_retire) before the next one is
+    // requested, in every path; a second set costs the fused kernels registers they do not have.
+    u32x4 piece[kPullLoads];
+    int probe_off;           // this wavefront's counter landing words
+    // The counter word, read out of the landing words right behind a K step's barrier: read
+    // there, it is older than every operand fetch that follows, so using it never waits for those.
+    int32_t probe_val;
     // What the per-step code needs from PullArgs, kept in registers (reading a field through
     // the argument block is a scalar load plus a wait that also drains the operand fetches).
     bool active;
@@ -619,7 +626,7 @@ struct Gemm256 {
   TCCL_D PullState pull_begin(PullPtr a, int wg, int num_wgs) const {
     PullState st;
     const int w = uniform(wave);
-    st.landing = w * (kBgLandingBytes / kPullWaves);
+    st.probe_off = w * 256;
     st.stride = num_wgs * kPullWaves;
     st.next_slot = 0;
     st.next_lp = wg * kPullWaves + w;
@@ -632,13 +639,10 @@ struct Gemm256 {
     st.need = 0;
     st.group_units = 0;
     st.backoff = 0;
-    st.left = 0;
-    st.pending = st.placed = false;
-    st.over = true;
-    st.src = Words4{0, 0, 0, 0};
-    st.step_to = st.step_from = st.step_col = st.wrap_to = st.wrap_from = 0;
+    st.pend_lp = -1;
+    st.probe_val = 0;
 #pragma unroll
-    for (int j = 0; j < kPullLoads; ++j) st.to[j] = st.from[j] = st.col[j] = st.pend_to[j] = 0;
+    for (int j = 0; j < kPullLoads; ++j) st.piece[j] = u32x4{0, 0, 0, 0};
     st.active = pull_offset >= 0 && a->mode != kBgNone && w < kPullWaves;
     st.units = 0;
     st.pieces = st.slots = st.n_groups = 0;
@@ -654,14 +658,16 @@ struct Gemm256 {
       st.row_shift = a->row_shift;
       st.row_pitch = a->row_pitch;
       pull_normalise(st, a);
-      st.over = st.next_slot >= st.slots;
     }
     return st;
   }
 
   // Where this lane's unit j of piece lp lies inside a block: byte offsets on the destination and the source
   // side (kNoUnit / the block's first unit for lanes beyond the block's end: their stores fall outside the
-  // buffer window and are dropped, their loads touch a unit that exists).
+  // buffer window and are dropped, their loads touch a unit that exists).  A handful of vector instructions
+  // from three scalars, formed where a piece is requested and again where it is stored: whatever a pulling
+  // lane carries from K step to K step besides the piece itself costs registers that the fused kernels do
+  // not have (kept in LDS instead, its reads and their waits made the per-step code several times as long).
   static constexpr uint32_t kNoUnit = 0xffffffffu;
   TCCL_D void pull_where(const PullState& st, PullPtr a, int lp, int j, int ln, uint32_t& to, uint32_t& from) const {
     const uint32_t u = (uint32_t)lp * (uint32_t)kPieceUnits + (uint32_t)(64 * j + ln);
@@ -675,29 +681,6 @@ struct Gemm256 {
     if constexpr (kGatherA) from = row * a->src_row_pitch + col * 16u;
   }
 
-  // The next piece's places, from scratch (a block's first piece of this wavefront) and from the piece before.
-  TCCL_D void pull_place(PullState& st, PullPtr a) const {
-    const int ln = lane_now();
-#pragma unroll
-    for (int j = 0; j < kPullLoads; ++j) {
-      const uint32_t u = (uint32_t)st.next_lp * (uint32_t)kPieceUnits + (uint32_t)(64 * j + ln);
-      const uint32_t row = st.row_magic ? (__umulhi(u, st.row_magic) >> st.row_shift) : (u >> st.row_shift);
-      st.col[j] = u - row * st.row_units;
-      st.to[j] = row * st.row_pitch + st.col[j] * 16u;
-      if constexpr (kGatherA) st.from[j] = row * a->src_row_pitch + st.col[j] * 16u;
-    }
-  }
-  TCCL_D void pull_advance(PullState& st) const {
-#pragma unroll
-    for (int j = 0; j < kPullLoads; ++j) {
-      const uint32_t col = st.col[j] + st.step_col;
-      const bool wraps = col >= st.row_units;
-      st.col[j] = wraps ? col - st.row_units : col;
-      st.to[j] += st.step_to + (wraps ? st.wrap_to : 0u);
-      if constexpr (kGatherA) st.from[j] += st.step_from + (wraps ? st.wrap_from : 0u);
-    }
-  }
-
   // Fetch the first counters in the first tile's prologue, so that the first K step can
   // already fetch a piece.
   TCCL_D void pull_prime(PullState& st, PullPtr a) const {
@@ -708,12 +691,13 @@ struct Gemm256 {
 
   // Every lane fetches the same word; it is read back from LDS one K step later.
   TCCL_D void pull_probe(PullState& st, PullPtr a) const {
-    if (st.gidx >= st.n_groups || st.probe_group >= 0) return;
+    if (st.gidx >= st.n_groups) return;
     if (st.backoff > 0) {
       --st.backoff;
       return;
     }
-    dma4_coherent(bgw + st.landing + 16 * kPieceUnits, descriptor((const void*)(uintptr_t)st.counter_base, 0xffffffffu), probe_offset(a, st.gidx));
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(window(st.counter_base), (LdsVoid*)(bgw + st.probe_off), 4, probe_offset(a, st.gidx), 0, 0,
+                                             kCoherent);
     st.probe_group = st.gidx;
   }
 
@@ -741,7 +725,6 @@ struct Gemm256 {
       const GatherPtr ga = late_kernarg_ptr<GatherArgs>(gather_offset);
       st.src_base = (int64_t)(uintptr_t)ga->shard + (table(ga->heap_bases, slot) - table(ga->heap_bases, ga->rank));
       st.dst_base = (int64_t)(uintptr_t)g.A + (int64_t)slot * ga->k_shard * kEszIn;
-      st.src = descriptor((const void*)(uintptr_t)st.src_base, 0xffffffffu);
       st.ready_units = a->units;
       st.gidx = a->n_groups;
       return;
@@ -751,7 +734,6 @@ struct Gemm256 {
     const int64_t theirs = table(a->heap_bases, peer);
     const int64_t rel = ((int64_t)(uintptr_t)a->src0 - mine) + (int64_t)peer * a->block_bytes;
     st.src_base = theirs + rel;
-    st.src = descriptor((const void*)(uintptr_t)st.src_base, 0xffffffffu);
     st.dst_base = mine + rel;
     const int64_t stride = a->word_stride;
     st.counter_base = (int64_t)(uintptr_t)a->counter + (stride ? (int64_t)(peer - a->rank) * stride : theirs - mine);
@@ -782,17 +764,19 @@ struct Gemm256 {
     }
   }
 
-  // Store the piece that is pending, if any: it has landed (the caller has waited for it).
-  TCCL_D void pull_retire(PullState& st) const {
-    if (!st.pending) return;
+  // Store the piece that is pending, if any.  It belongs
+  // to the selected block: pull_issue() stores what is pending before it selects another one.
+  TCCL_D void pull_retire(PullState& st, PullPtr a) const {
+    if (st.pend_lp < 0) return;
     const __amdgpu_buffer_rsrc_t dst = window(st.dst_base);
     const int ln = lane_now();
-    u32x4 piece[kPullLoads];
 #pragma unroll
-    for (int j = 0; j < kPullLoads; ++j) piece[j] = *(const u32x4*)(bgw + st.landing + 16 * (64 * j + ln));
-#pragma unroll
-    for (int j = 0; j < kPullLoads; ++j) st16<kStreaming>(dst, st.pend_to[j], piece[j]);
-    st.pending = false;
+    for (int j = 0; j < kPullLoads; ++j) {
+      uint32_t to, from;
+      pull_where(st, a, st.pend_lp, j, ln, to, from);
+      st16<kStreaming>(dst, to, st.piece[j]);
+    }
+    st.pend_lp = -1;
   }
 
   // The two facts about group gidx that the per-step code needs, fetched when gidx changes.
@@ -831,71 +815,48 @@ struct Gemm256 {
     pull_group_facts(st, a);
   }
 
-  // Once per K step, behind pull_retire(): request the next piece.
-  TCCL_D void pull_request(PullState& st, PullPtr a) const {
-    if (__builtin_expect(!st.over && st.left <= 1, 0)) pull_more(st, a);
-    if (st.left > 0) {
-#pragma unroll
-      for (int j = 0; j < kPullLoads; ++j) {
-        st.pend_to[j] = st.to[j];
-        dma16_coherent(bgw + st.landing + 1024 * j, st.src, kGatherA ? st.from[j] : st.to[j]);
-      }
-      st.pending = true;
-      --st.left;
-      st.next_lp += st.stride;
-      pull_advance(st);
-    }
+  // Right behind a K step's barrier (this wave's loads, the counter fetch among them, have
+  // landed): take the counter word out of the landing words.
+  TCCL_D void pull_collect(PullState& st) const {
+    if (!st.active) return;
+    st.probe_val = *(const int32_t*)(bgw + st.probe_off + 4 * lane_now());  // lane l's word landed at 4 l
   }
-  // The rare part of it: take in the counter word fetched before (it landed ahead of a barrier since), move on to the next
-  // block, count what may be fetched, fetch the next word.
-  TCCL_D void pull_more(PullState& st, PullPtr a) const {
-    // What the pieces' places need is worked out here, not in the kernel's first microseconds, which have no slack
-    // (4096 x 4096 x 1024: 1 us per launch).
-    if (!st.placed) {
-      st.placed = true;
-      const uint32_t ahead = (uint32_t)st.stride * (uint32_t)kPieceUnits;  // units from piece to piece
-      const uint32_t rows = st.row_magic ? (__umulhi(ahead, st.row_magic) >> st.row_shift) : (ahead >> st.row_shift);
-      const uint32_t src_pitch = kGatherA ? a->src_row_pitch : st.row_pitch;
-      st.step_col = ahead - rows * st.row_units;
-      st.step_to = rows * st.row_pitch + st.step_col * 16u;
-      st.step_from = rows * src_pitch + st.step_col * 16u;
-      st.wrap_to = st.row_pitch - st.row_units * 16u;
-      st.wrap_from = src_pitch - st.row_units * 16u;
-      pull_place(st, a);
-    }
+  // Once per K step: learn about readiness, request the next piece (the previous
+  // one has been stored).  All control flow here is wavefront-uniform.
+  TCCL_D void pull_issue(PullState& st, PullPtr a) const {
     if (st.probe_group >= 0) {
-      const int32_t word = *(const int32_t*)(bgw + st.landing + 16 * kPieceUnits + 4 * lane_now());  // lane l's word landed at 4 l
+      const int g = st.probe_group;
       st.probe_group = -1;
-      if (all_reached(word, st.need))
-        pull_group_done(st, a);
-      else
-        st.backoff = 3;  // not there yet: fetching the counters every step only costs issue slots
+      if (g == st.gidx) {
+        if (all_reached(st.probe_val, st.need))
+          pull_group_done(st, a);
+        else
+          st.backoff = 3;  // not there yet: fetching the counters every step only costs issue slots
+      }
     }
-    if (st.left == 0 && st.next_lp >= st.pieces) pull_normalise(st, a);  // block finished
-    if (st.next_slot >= st.slots) {
-      st.over = true;
+    if (st.next_slot >= st.slots) return;
+    if (st.next_slot != st.slot) {
+      pull_retire(st, a);  // a piece still pending belongs to the block being left
+      pull_select(st, a, st.next_slot);
+      pull_probe(st, a);
       return;
     }
-    if (st.next_slot != st.slot) {
-      pull_select(st, a, st.next_slot);
-      pull_place(st, a);
-    }
-    const int whole = (int)(st.ready_units / (uint32_t)kPieceUnits);
-    while (st.next_lp + st.left * st.stride < whole) ++st.left;
-    // (A block's last piece may be short: its lanes past the end fetch the block's first unit and store nothing.)
+    pull_probe(st, a);  // look ahead: the next group's counters (issued before the piece, which stays the youngest load)
     const uint32_t first = (uint32_t)st.next_lp * (uint32_t)kPieceUnits;
-    if (st.left == 0 && !st.pending && st.next_lp < st.pieces && st.ready_units >= st.units) {
+    const uint32_t last = first + (uint32_t)(kPieceUnits - 1);
+    if ((last < st.units ? last : st.units - 1u) < st.ready_units) {
+      const __amdgpu_buffer_rsrc_t src = window(st.src_base);
+      const int ln = lane_now();
 #pragma unroll
       for (int j = 0; j < kPullLoads; ++j) {
-        const bool valid = first + (uint32_t)(64 * j + lane_now()) < st.units;
-        st.pend_to[j] = valid ? st.to[j] : kNoUnit;
-        dma16_coherent(bgw + st.landing + 1024 * j, st.src, valid ? (kGatherA ? st.from[j] : st.to[j]) : 0u);
+        uint32_t to, from;
+        pull_where(st, a, st.next_lp, j, ln, to, from);
+        st.piece[j] = ld16<kCoherent>(src, from);
       }
-      st.pending = true;
+      st.pend_lp = st.next_lp;
       st.next_lp += st.stride;
-      return;
+      if (st.next_lp >= st.pieces) pull_normalise(st, a);  // block finished: rare
     }
-    pull_probe(st, a);
   }
 
   // Wait (bounded) until units [0, last] of the selected block may be fetched.
@@ -943,8 +904,7 @@ struct Gemm256 {
   // The pulling wavefronts' part of pull_finish; false if a bounded wait expired.
   TCCL_D bool pull_drain(PullState& st, PullPtr a) const {
     wait_vmem();
-    pull_retire(st);
-    pull_normalise(st, a);  // (nothing left: the loop below is not entered)
+    pull_retire(st, a);
     st.probe_group = -1;
     const int64_t deadline = now_ticks() + a->spin_ticks;
     bool ok = true;
@@ -1077,7 +1037,6 @@ struct Gemm256 {
       for (int r = 0; r < 4; ++r) f.a[r] = load_a16(cur, rd, 0, r);
       multiply(acc, f, 0, 0);
       mask_a(src, kt + 1);
-      follow_shards(src, kt + 1);
       issue_a(nxt, src, kt + 1, 0);
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) f.b[1][cb] = load_b16(cur, rd, 1, cb);
@@ -1099,12 +1058,23 @@ struct Gemm256 {
   }
 
   // K step kt of a launch with a background transfer: eight items, item d's A operands fetched one item ahead, computed from
-  // `cur` while the next step's operands stream into `nxt` (one piece of A and of B per item, items 0..3).  16-bit: eight MFMAs per
-  // item, k block d / 4, 16-row blocks 2 (d % 4) and + 1; fp8: four, 16-row block d.  The four B operands have one register
-  // set: the last item of a k block runs column block by column block and reloads each in place.  The step's one barrier sits
+  // `cur` while the next step's operands stream into `nxt` (one piece of A and of B per item, items 0..3: issuing a load holds the
+  // wavefront while the address unit takes it in).  16-bit: eight MFMAs per item, k block d / 4, 16-row blocks 2 (d % 4) and + 1; fp8:
+  // four, 16-row block d.  The four B operands have one register set: the last item of a k block runs column block by column block and
+  // reloads each in place (a second set would cost 16 registers, which these kernels do not have).  The step's one barrier sits
   // before the last item: there the wavefront's reads of `cur` are done, its loads into `nxt` have landed, and the last item
-  // already fetches the next step's first operands.  The transfer has one place, behind the step's last operand loads
-  // (spread over three items the same work cost 4096 x 4096 x 1024 1.3 us more).
+  // already fetches the next step's first operands.  The scheduling barriers pin this order (left alone, the compiler hoists
+  // every read of the step and spills).
+  //
+  // The transfer has one place, behind the step's last operand loads (loads complete in issue order: a request to the peer's memory
+  // ahead of them would hold all of them back): the piece requested a step before (it arrived before that step's barrier) is stored,
+  // the next one requested into the same registers.  One place, under one test: every call site splits the step into basic blocks, and
+  // where they join the compiler waits for more than the code needs (spread over three items the same work cost 4096 x 4096 x 1024
+  // 1.3 us more).  The counter word is taken out of its landing words right behind the barrier: older than every operand load that
+  // follows, it never waits for those.
+  //
+  // (Pieces landing in LDS, with their places carried from step to step, and hand-written operand loads were tried in place of this:
+  // 4096 x 4096 x 1024 +1.4 %, with gathered inputs +1.6 %.)
   struct Running {
     Vec ring[kFp8 ? 2 : 4], fb[4];
   };
@@ -1120,12 +1090,9 @@ struct Gemm256 {
     else
       return load_b16(stage, r, kh, cb);
   }
-  TCCL_D void step_pulling(char* cur, char* nxt, Source& src, const Reader& rd, int kt, f32x16 (&acc)[4][2], Running& f, PullState& pull) const {
+  TCCL_D void step_pulling(const char* cur, char* nxt, const Source& src, const Reader& rd, int kt, f32x16 (&acc)[4][2], Running& f, PullState& pull) const {
     constexpr int kRows = kFp8 ? 1 : 2;            // 16-row blocks per item
     constexpr int kPerBlock = 8 / kRows;           // items per k block
-    mask_a(src, kt + 1);
-    mask_b(src, kt + 1);
-    follow_shards(src, kt + 1);
 #pragma unroll
     for (int d = 0; d < 8; ++d) {
       const int rp = d % kPerBlock;
@@ -1133,16 +1100,16 @@ struct Gemm256 {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+        pull_collect(pull);
       }
       const int dn = (d + 1) & 7;
       const char* from = d + 1 < 8 ? cur : nxt;
-      if (d < 4) issue_a(nxt, src, kt + 1, d >> 1, d & 1);
 #pragma unroll
       for (int r = 0; r < kRows; ++r) f.ring[kRows * (dn & 1) + r] = load_a(from, rd, dn / kPerBlock, kRows * (dn % kPerBlock) + r);
-      if (d < 4) issue_b(nxt, src, kt + 1, d >> 1, d & 1);
-      if (d == 3) {
-        pull_retire(pull);
-        pull_request(pull, pa());
+      if (d < 4) issue_piece(nxt, src, kt + 1, d);
+      if (d == 3 && pull.active) {
+        pull_retire(pull, pa());
+        pull_issue(pull, pa());
       }
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
@@ -1425,37 +1392,35 @@ struct Gemm256 {
     wait_loads<kPull ? 0 : (kFp8 ? 6 : 4)>();
     __syncthreads();
     publish_owed(s, unpublished);
-    // One loop body for both stages, their places exchanged from step to step: half the code of two named stages,
-    // and fewer registers (189 instead of 223 in the plain bf16 kernel).
-    uint32_t at = 0;
     if constexpr (kPull) {
+      pull_collect(pull);  // the counters fetched before this tile
       Running f;
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b(lds, rd, 0, cb);
 #pragma unroll
       for (int r = 0; r < (kFp8 ? 1 : 2); ++r) f.ring[r] = load_a(lds, rd, 0, r);
-      if constexpr (kBKMajor) {
-        for (int kt = 0; kt < ksteps; ++kt) {
-          step_pulling(lds + at, lds + (at ^ (uint32_t)kStage256), src, rd, kt, acc, f, pull);
-          at ^= (uint32_t)kStage256;
-        }
-      } else {  // two named stages: 1.5 % at 4096 x 4096 x 2048 with gathered inputs (a k-major B spills with them)
-        for (int kt = 0; kt < ksteps; kt += 2) {
-          step_pulling(lds, lds1, src, rd, kt, acc, f, pull);
-          step_pulling(lds1, lds, src, rd, kt + 1, acc, f, pull);
-        }
+      // Steps are taken in pairs so that each call names its two stages statically.  An odd count is rounded up: the
+      // extra step (like the final look-ahead loads) lies wholly past K and reads zeros.
+      for (int kt = 0; kt < ksteps; kt += 2) {
+        follow_shards(src, kt + 1);
+        step_pulling(lds, lds1, src, rd, kt, acc, f, pull);
+        follow_shards(src, kt + 2);
+        step_pulling(lds1, lds, src, rd, kt + 1, acc, f, pull);
       }
+      pull_retire(pull, pa());  // the last step's piece: nothing is carried through the epilogue
     } else {
+      // One loop body for both stages, their places exchanged from step to step: half the code of two named stages,
+      // and fewer registers (189 instead of 223 in the plain bf16 kernel).
       Frags f;
+      uint32_t at = 0;
       if (wm) __builtin_amdgcn_s_barrier();  // wavefronts 4..7 stay one slot behind wavefronts 0..3
       for (int kt = 0; kt < ksteps; ++kt) {
         k_step(lds + at, lds + (at ^ (uint32_t)kStage256), src, rd, kt, acc, f);
         at ^= (uint32_t)kStage256;
       }
       if (!wm) __builtin_amdgcn_s_barrier();
+      wait_vmem();  // the loads past the last step: the epilogue stages through their LDS
     }
-    wait_vmem();  // the loads past the last step: the epilogue stages through their LDS
-    if constexpr (kPull) pull_retire(pull);  // nothing is carried through the epilogue
     if constexpr (kWithReduce) {
       // Rows this rank owns, partial kept in registers: the peers' partials are added in the
       // epilogue and the tile's partial is never stored (it is still published: the counters

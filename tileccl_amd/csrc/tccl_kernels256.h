@@ -51,17 +51,20 @@ struct Fused256Args {
 template <typename InT, typename OutT, bool kWithReduce, bool kGatherA, bool kBKMajor, bool kPull = true>
 __global__ __launch_bounds__(512, 2) void fused256_kernel(Fused256Args f) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __attribute__((aligned(16))) char stages[kLds256];
-  __shared__ __attribute__((aligned(16))) char landing[kPull ? kBgLandingBytes : 16];
+  // Two arrays with kPull (the compiler tracks the loads that write LDS by array), else one.
+  __shared__ __attribute__((aligned(16))) char stages[kPull ? kStage256 : kLds256];
+  __shared__ __attribute__((aligned(16))) char second[kPull ? kStage256 : 16];
+  __shared__ __attribute__((aligned(16))) char landing_words[kPull ? kBgWordBytes : 16];
+  char* const stage1 = kPull ? second : stages + kStage256;
   warm_kernargs<(int)sizeof(Fused256Args)>();
   if (f.trace_start && blockIdx.x == 0 && threadIdx.x == 0) *f.trace_start = now_ticks();
   Gemm256<InT, OutT, kWithReduce, kGatherA, kBKMajor, kPull>(f.g, kPull ? (int)offsetof(Fused256Args, pull) : -1, (int)offsetof(Fused256Args, push),
-                                                      (int)offsetof(Fused256Args, reduce), stages, stages + kStage256, landing,
+                                                      (int)offsetof(Fused256Args, reduce), stages, stage1, landing_words,
                                                       (int)offsetof(Fused256Args, gather))
       .run(f.s, f.m, (int)blockIdx.x, (int)gridDim.x);
   __syncthreads();
   const CommArgs c = late_kernarg<CommArgs>((int)offsetof(Fused256Args, comm));
-  comm_role<kThreads256>(c, (int)blockIdx.x, (int)gridDim.x, (int*)(stages + kStage256));
+  comm_role<kThreads256>(c, (int)blockIdx.x, (int)gridDim.x, (int*)stage1);
 #endif
 }
 
