@@ -51,7 +51,8 @@ def run(world, M, N, K, macro, in_dtype, partial, out, variant, emulate, mark=Tr
     (3, 384, 264, 72, 128, torch.bfloat16, torch.float32, torch.bfloat16),   # three ranks, one tile row each
     (4, 512, 520, 136, 256, torch.float16, torch.float32, torch.float16),    # 256-row tiles across two owners
     (2, 256, 272, 144, 256, F8, torch.bfloat16, torch.bfloat16),             # one tile, two owners
-    (2, 768, 2064, 272, 0, F8, torch.bfloat16, torch.bfloat16),              # streaming tiles, more than one per CU
+    (2, 768, 2064, 272, 0, F8, torch.bfloat16, torch.bfloat16),              # streaming tiles that sum themselves, most CUs at work
+    (2, 1536, 2048, 1024, 0, F8, torch.bfloat16, torch.bfloat16),            # streaming tiles, those of the own rows beyond one per CU
     (2, 1280, 3400, 1040, 0, torch.bfloat16, torch.bfloat16, torch.bfloat16),  # the kernel chosen by cost
 ])
 def test_sums_behind_the_gemm_are_the_oracles(lib, variant, emulate, world, M, N, K, macro, in_dtype, partial, out):
@@ -67,4 +68,11 @@ def test_sums_behind_the_gemm_are_the_oracles(lib, variant, emulate, world, M, N
 def test_a_peer_that_has_not_published_is_waited_for_and_reported(lib, variant):
     """Nobody marks the peers' words: the bounded wait expires, nothing is summed, the fault is raised on the host."""
     _, outs = run(2, 768, 264, 1048, 128, torch.float16, torch.float32, torch.float16, variant, True, mark=False, spin_limit_ns=200_000)
+    assert all(torch.all(o == 0) for o in outs)
+
+
+@pytest.mark.parametrize("variant", ["s1", "s2"])
+def test_sums_behind_a_wait_of_their_own_do_not_run_where_it_expired(lib, variant):
+    """Three ranks: one workgroup per owner waits in a launch ahead of the sums."""
+    _, outs = run(3, 384, 264, 72, 128, torch.bfloat16, torch.float32, torch.bfloat16, variant, True, mark=False, spin_limit_ns=200_000)
     assert all(torch.all(o == 0) for o in outs)

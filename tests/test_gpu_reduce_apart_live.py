@@ -11,12 +11,12 @@ import torch
 from oracle import collectives as oracle
 from tests.gpu_util import bits
 from tests.test_gpu_concurrent_ranks import SPIN_NS, both_at_once, streams  # noqa: F401
-from tests.test_gpu_stream_live import E4M3, Rank, operands, out_type
+from tests.test_gpu_stream_live import E4M3, Rank, operands, out_type, small_tiles_ran
 from tests.test_gpu_two_rank_readiness import SHORT_NS, expect_timeout
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(768, 264, 1048, 128, torch.float16), (768, 264, 1048, 256, torch.float16), (768, 2064, 272, 0, E4M3), (4352, 2056, 1040, 0, torch.bfloat16)]
+SHAPES = [(768, 264, 1048, 128, torch.float16), (768, 264, 1048, 256, torch.float16), (1536, 2048, 1024, 0, E4M3), (4352, 2056, 1040, 0, torch.bfloat16)]
 
 
 def reducers(heaps, M, N, macro, dtype, **kw):
@@ -48,6 +48,7 @@ def test_two_live_ranks(lib, streams, M, N, K, macro, dtype, emulate, variant): 
             for r, op in enumerate(ops):
                 assert torch.equal(bits(op.out).cpu(), bits(sums(*ops, r, dtype))), (launch, r)
                 assert torch.allclose(op.partial.float().cpu(), each[r][2], rtol=1e-2, atol=1e-1)
+        assert dtype is not E4M3 or small_tiles_ran(ops[0], *each[0][:2], variant, each[0][3])
     finally:
         for h in heaps:
             h.cleanup()

@@ -170,13 +170,21 @@ __global__ __launch_bounds__(256) void reduce_kernel(tccl::BulkReduceArgs a) {
   tccl::bulk_reduce<PT, OT, kRanks, tccl::kThreadsComm>(a, a.first_owner + (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x);
 }
 
-// The same behind a wait for the peers' words.  Loads pass the caches: the peers may still be writing when the launch starts.
+// Sums of partials that peers may still be writing.  A waiting workgroup holds what a peer's launch on the same device may need, so
+// either at most half of the CUs wait and then add up (two ranks: the other one finds the other half), or one workgroup
+// per owner waits in a launch of its own and the launch behind it, which fills the device, only looks at the words and leaves where
+// the wait has expired (a fault is raised, nothing is summed): `patience` ticks of waiting, 0 to look.  Loads pass the caches.
 constexpr int kThreadsReady = 512;
+__global__ __launch_bounds__(kThreadsReady) void rows_wait_kernel(tccl::CommArgs c, int first_owner) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  tccl::rows_published<kThreadsReady>(c, first_owner + (int)blockIdx.x, tccl::now_ticks() + c.spin_ticks);
+#endif
+}
 template <typename PT, typename OT, int kRanks>
-__global__ __launch_bounds__(kThreadsReady) void ready_reduce_kernel(tccl::BulkReduceArgs a, tccl::CommArgs c) {
+__global__ __launch_bounds__(kThreadsReady) void ready_reduce_kernel(tccl::BulkReduceArgs a, tccl::CommArgs c, int64_t patience) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const int owner = a.first_owner + (int)blockIdx.y;
-  if (tccl::rows_published<kThreadsReady>(c, owner))
+  if (tccl::rows_published<kThreadsReady>(c, owner, tccl::now_ticks() + patience))
     tccl::bulk_reduce<PT, OT, kRanks, kThreadsReady, tccl::kCoherent>(a, owner, (int)blockIdx.x, (int)gridDim.x);
 #endif
 }
@@ -750,6 +758,11 @@ int check_comm_span(const tccl::CommArgs& c) {
 #ifndef TCCL_BULK_REDUCE_WGS
 #define TCCL_BULK_REDUCE_WGS 8
 #endif
+constexpr int kReadyReduceWgs = 2;  // of the reductions behind a wait, 512 threads each
+// Up to this many bytes read and written half of the CUs are quicker than a launch more (two ranks, whole operation, us, on half of
+// the CUs / behind a wait of their own: 1792 x 1200 x 1520 30.7 / 32.0, 1792 x 3408 x 2144 (58 MiB) 49.6 / 51.6, 9472 x 736 x 1120
+// (66 MiB) 45.6 / 43.7, 12544 x 3072 x 1024 215.7 / 175.8; with all CUs waiting, which leaves a peer none, 28.5, 47.8, 40.0, 171.7).
+constexpr int64_t kWaitInsideBytes = 64ll << 20;
 // Units a copying workgroup takes at a time: one 16-byte access per thread while that does not fill the
 // device, then more, up to 32 KiB (tasks of 128 KiB took 21.7 us instead of 19.7 on that exchange).
 constexpr int kBulkTaskUnits = 2048;
@@ -772,15 +785,15 @@ int launch_bulk_copy(tccl::BulkCopyArgs& a, int transfers, int64_t rows, const t
 }
 
 template <typename PT, typename OT>
-void launch_reduce_t(const tccl::BulkReduceArgs& a, dim3 grid, int ranks, hipStream_t stream, const tccl::CommArgs* waits) {
+void launch_reduce_t(const tccl::BulkReduceArgs& a, dim3 grid, int ranks, hipStream_t stream, const tccl::CommArgs* waits, int64_t patience) {
   if (waits) {
     const dim3 block(kThreadsReady);
     if (ranks == 2)
-      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 2>), grid, block, 0, stream, a, *waits);
+      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 2>), grid, block, 0, stream, a, *waits, patience);
     else if (ranks == 4)
-      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 4>), grid, block, 0, stream, a, *waits);
+      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 4>), grid, block, 0, stream, a, *waits, patience);
     else
-      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 8>), grid, block, 0, stream, a, *waits);
+      hipLaunchKernelGGL((ready_reduce_kernel<PT, OT, 8>), grid, block, 0, stream, a, *waits, patience);
     return;
   }
   const dim3 block(tccl::kThreadsComm);
@@ -793,24 +806,31 @@ void launch_reduce_t(const tccl::BulkReduceArgs& a, dim3 grid, int ranks, hipStr
 }
 
 int launch_bulk_reduce(tccl::BulkReduceArgs& a, int owners, int64_t rows, int partial_dtype, int out_dtype, const tccl_device_info& dev,
-                       hipStream_t stream, const tccl::CommArgs* waits = nullptr, int most_waiting = 0) {
+                       hipStream_t stream, const tccl::CommArgs* waits = nullptr, int most_wgs = 0) {
   a.units = (int)(rows * a.upr);
   if (a.units <= 0 || owners <= 0) return 0;
   const int ranks = a.world <= 2 ? 2 : (a.world <= 4 ? 4 : 8);
   const int64_t per_wg = (int64_t)(waits ? kThreadsReady : tccl::kThreadsComm) * (8 / ranks);
   int64_t x = (a.units + per_wg - 1) / per_wg;
-  const int64_t most = (waits ? (int64_t)most_waiting : (int64_t)dev.compute_units * TCCL_BULK_REDUCE_WGS) / owners;
+  // Two ranks and little to add: half of the CUs wait themselves.
+  const int64_t bytes = (int64_t)a.units * 8 * owners * (a.world * (int64_t)dtype_size(partial_dtype) + (int64_t)dtype_size(out_dtype));
+  const bool wait_inside = waits && a.world == 2 && bytes <= kWaitInsideBytes;
+  int64_t most = !waits ? (int64_t)dev.compute_units * TCCL_BULK_REDUCE_WGS : wait_inside ? dev.compute_units / 2 : (int64_t)dev.compute_units * kReadyReduceWgs;
+  if (most_wgs > 0 && most_wgs < most) most = most_wgs;
+  most /= owners;
   if (x > most) x = most > 0 ? most : 1;
+  const int64_t patience = wait_inside ? waits->spin_ticks : 0;
+  if (waits && !wait_inside) hipLaunchKernelGGL(rows_wait_kernel, dim3((unsigned)owners), dim3(kThreadsReady), 0, stream, *waits, a.first_owner);
   const dim3 grid((unsigned)x, (unsigned)owners);
   const int key = partial_dtype * 4 + out_dtype;
   switch (key) {
-    case TCCL_F32 * 4 + TCCL_F32: launch_reduce_t<float, float>(a, grid, ranks, stream, waits); break;
-    case TCCL_F32 * 4 + TCCL_F16: launch_reduce_t<float, _Float16>(a, grid, ranks, stream, waits); break;
-    case TCCL_F32 * 4 + TCCL_BF16: launch_reduce_t<float, __bf16>(a, grid, ranks, stream, waits); break;
-    case TCCL_F16 * 4 + TCCL_F16: launch_reduce_t<_Float16, _Float16>(a, grid, ranks, stream, waits); break;
-    case TCCL_F16 * 4 + TCCL_BF16: launch_reduce_t<_Float16, __bf16>(a, grid, ranks, stream, waits); break;
-    case TCCL_BF16 * 4 + TCCL_BF16: launch_reduce_t<__bf16, __bf16>(a, grid, ranks, stream, waits); break;
-    case TCCL_BF16 * 4 + TCCL_F16: launch_reduce_t<__bf16, _Float16>(a, grid, ranks, stream, waits); break;
+    case TCCL_F32 * 4 + TCCL_F32: launch_reduce_t<float, float>(a, grid, ranks, stream, waits, patience); break;
+    case TCCL_F32 * 4 + TCCL_F16: launch_reduce_t<float, _Float16>(a, grid, ranks, stream, waits, patience); break;
+    case TCCL_F32 * 4 + TCCL_BF16: launch_reduce_t<float, __bf16>(a, grid, ranks, stream, waits, patience); break;
+    case TCCL_F16 * 4 + TCCL_F16: launch_reduce_t<_Float16, _Float16>(a, grid, ranks, stream, waits, patience); break;
+    case TCCL_F16 * 4 + TCCL_BF16: launch_reduce_t<_Float16, __bf16>(a, grid, ranks, stream, waits, patience); break;
+    case TCCL_BF16 * 4 + TCCL_BF16: launch_reduce_t<__bf16, __bf16>(a, grid, ranks, stream, waits, patience); break;
+    case TCCL_BF16 * 4 + TCCL_F16: launch_reduce_t<__bf16, _Float16>(a, grid, ranks, stream, waits, patience); break;
     default: return fail(TCCL_ERR_UNSUPPORTED, "reduce: no kernel for partial dtype %d, output dtype %d", partial_dtype, out_dtype);
   }
   TCCL_HIP(hipGetLastError());
@@ -818,8 +838,8 @@ int launch_bulk_reduce(tccl::BulkReduceArgs& a, int owners, int64_t rows, int pa
 }
 
 // The transfer of a GEMM + collective operation as a launch of its own (the second kernel of S0).
-// waits: the reductions wait for the peers' words, with at most this many workgroups.
-int launch_bulk(const tccl::CommArgs& c, const tccl_device_info& dev, hipStream_t stream, int waits = 0) {
+// waits: the reductions wait for the peers' words.  most_wgs > 0: with at most that many workgroups.
+int launch_bulk(const tccl::CommArgs& c, const tccl_device_info& dev, hipStream_t stream, bool waits = false, int most_wgs = 0) {
   const int span = check_comm_span(c);
   if (span) return span;
   if (c.op == tccl::kOpReduceScatter) {
@@ -836,7 +856,7 @@ int launch_bulk(const tccl::CommArgs& c, const tccl_device_info& dev, hipStream_
     a.dst_pitch = (uint32_t)c.ld_rs_out_bytes;
     a.upr = c.N / 8;
     a.first_owner = c.emulate_peer ? 0 : c.rank;
-    return launch_bulk_reduce(a, c.emulate_peer ? c.world : 1, shard, c.partial_dtype, c.out_dtype, dev, stream, waits > 0 ? &c : nullptr, waits);
+    return launch_bulk_reduce(a, c.emulate_peer ? c.world : 1, shard, c.partial_dtype, c.out_dtype, dev, stream, waits ? &c : nullptr, waits ? most_wgs : 0);
   }
   tccl::BulkCopyArgs a;
   memset(&a, 0, sizeof a);
@@ -1110,11 +1130,7 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // launch replaced, took longer.  bf16 1792 x 3408 x 2144 on two ranks 85 -> 48 us, e4m3 13824 x 736 x 2496 on four 86 -> 50,
   // e4m3 512 x 7056 x 1888 on four 75 -> 35.
   const bool apart = c.op == tccl::kOpReduceScatter && variant != TCCL_S0_BULK && c.world > 1 && !traced && !(tr && tr->num_comm_wgs > 0);
-  // Workgroups that wait for a peer leave half of the CUs to the peer's own launches, unless this rank carries out the peer's
-  // half itself (nobody else is waited for then; the sums of 1024 x 3248 fp32 on two ranks take 11.0 us on half of the CUs, 8.3 on all).
-  const int most = c.emulate_peer ? 2 * dev.compute_units : dev.compute_units / 2;
-  const int waiters = d->num_wgs > 0 && d->num_wgs < most ? d->num_wgs : most;
-  const auto sums_apart = [&] { return launch_bulk(c, dev, stream, c.peers_resident ? 0 : waiters); };
+  const auto sums_apart = [&] { return launch_bulk(c, dev, stream, !c.peers_resident, d->num_wgs); };
   if (!gather) {
     // Tiles of a reduce-scatter must not straddle two owners' rows.
     const int64_t seg = g.wrap_rows > 0 ? g.wrap_rows : (c.op == tccl::kOpReduceScatter ? d->M / c.world : d->M);

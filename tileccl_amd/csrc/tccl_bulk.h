@@ -1,6 +1,6 @@
 // Stand-alone transfers and reductions between the slices of the symmetric heap: the second kernel of S0,
 // the copies and reductions of the stand-alone collectives, and the collectives whose every role is carried
-// by one launch.  Nothing here waits: the launch's inputs are complete when it starts (stream order).
+// by one launch.  The inputs of all but the last part (sums behind a wait) are complete when the launch starts (stream order).
 //
 // What bounds them.  Large ones: HBM (a copy reads and writes each byte once; 128 MiB of traffic at 4096 x 4096
 // fp16 in both directions takes 20 us).  Small ones: the launch and one trip to memory, so the work is cut
@@ -130,28 +130,24 @@ TCCL_D void bulk_reduce(const BulkReduceArgs& a, int owner, int wg, int num_wgs)
   }
 }
 
-// ---- reductions that wait ---------------------------------------------------------------------------
-// The second launch of a reduce-scatter whose tiles do not sum themselves (run_variant() in tccl_api.hip): this rank's
-// partials are in memory, the peers' are once their words say so.  Every workgroup looks at all words of its owner's
-// rows, a word per lane; false if a bounded wait expired (the fault word is raised).
+// ---- reductions behind a wait ---------------------------------------------------------------------
+// The sums of a reduce-scatter whose tiles do not sum themselves (run_variant() in tccl_api.hip): this rank's partials are in
+// memory, the peers' are once their words say so.  One workgroup looks at all words of an owner's rows, a word per
+// lane, until `deadline`; false if some word has not come by then (the fault word is raised).
 template <int kThreads>
-TCCL_D bool rows_published(const CommArgs& c, int owner) {
-  const int64_t deadline = now_ticks() + c.spin_ticks;
-  const int shard = c.M / c.world, lo = owner * shard, hi = lo + shard;
+TCCL_D bool rows_published(const CommArgs& c, int owner, int64_t deadline) {
+  const int shard = c.M / c.world, lo = owner * shard, hi = lo + shard, peers = c.world - 1;
+  const bool by_tile = c.granularity == kPerTile;
+  const int first = lo / c.block_m;
+  const int n = by_tile ? ((hi - 1) / c.block_m - first + 1) * c.tile_cols : c.n_groups;  // words per peer
   bool ok = true;
-  for (int p = 0; p < c.world; ++p) {
-    if (p == c.rank) continue;
-    if (c.granularity == kPerTile) {
-      const int32_t* words = peer_words(c, c.locks, p);
-      const int first = lo / c.block_m, n = ((hi - 1) / c.block_m - first + 1) * c.tile_cols;
-      for (int i = (int)threadIdx.x; i < n && ok; i += kThreads)
-        ok = tile_wait_ge<true>(words, tile_id_of(first + i / c.tile_cols, i % c.tile_cols, c.tile_rows, c.tile_cols, c.group_m), c.epoch, deadline);
-    } else {
-      const int32_t* words = peer_words(c, c.counter, p);
-      for (int g = (int)threadIdx.x; g < c.n_groups && ok; g += kThreads)
-        if (group_hi(c, g) > lo && group_lo(c, g) < hi)
-          ok = tile_wait_ge<true>(words, g, (int32_t)((uint32_t)c.epoch * (uint32_t)c.tile_counts[g]), deadline);
-    }
+  for (int i = (int)threadIdx.x; i < n * peers && ok; i += kThreads) {
+    const int p = i / n, word = i - p * n, peer = p < c.rank ? p : p + 1;
+    if (by_tile)
+      ok = tile_wait_ge<true>(peer_words(c, c.locks, peer), tile_id_of(first + word / c.tile_cols, word % c.tile_cols, c.tile_rows, c.tile_cols, c.group_m),
+                              c.epoch, deadline);
+    else if (group_hi(c, word) > lo && group_lo(c, word) < hi)
+      ok = tile_wait_ge<true>(peer_words(c, c.counter, peer), word, (int32_t)((uint32_t)c.epoch * (uint32_t)c.tile_counts[word]), deadline);
   }
   const bool all = __syncthreads_and(ok ? 1 : 0) != 0;
   if (!all && threadIdx.x == 0 && c.fault) *c.fault = 1;
