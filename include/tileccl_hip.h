@@ -99,8 +99,8 @@ typedef struct tccl_gemm_desc {
 } tccl_gemm_desc;
 
 /* tccl_gemm_reducescatter, variants S1 / S2 where the sums are made in the GEMM's epilogue (shards of whole 256 x 256
- * tiles; small outputs with TCCL_GEMM_ARRIVALS; two ranks' 128 x 128 tiles that wait for the peer, at most one per CU and
- * K <= 1024; elsewhere the sums are a launch of their own and every partial is stored):
+ * tiles; small outputs with TCCL_GEMM_ARRIVALS; 128 x 128 tiles that wait for their peers, at most one per CU; elsewhere the
+ * sums are a launch of their own and every partial is stored):
  * the partial of the rows this rank owns stays in the accumulators, takes the peers' partials
  * in the GEMM epilogue and is never stored to gemm->C (those rows of C keep their old
  * contents); the output is bit-identical to storing and reducing.  Ignored elsewhere.

@@ -76,3 +76,37 @@ def test_sums_behind_a_wait_of_their_own_do_not_run_where_it_expired(lib, varian
     """Three ranks: one workgroup per owner waits in a launch ahead of the sums."""
     _, outs = run(3, 384, 264, 72, 128, torch.bfloat16, torch.float32, torch.bfloat16, variant, True, mark=False, spin_limit_ns=200_000)
     assert all(torch.all(o == 0) for o in outs)
+
+
+@pytest.mark.parametrize("variant", ["s1", "s2"])
+@pytest.mark.parametrize("world,M,N,K,macro", [(2, 768, 264, 1048, 128), (3, 768, 264, 136, 128), (2, 1792, 1200, 1520, 0)])
+def test_own_rows_kept_in_registers_are_never_stored(lib, variant, world, M, N, K, macro):
+    """128-row tiles that wait, at most one per CU: asked to keep its own rows in registers, the launch sums in its tiles, and
+    those rows of the partial keep what they held."""
+    from tileccl_amd.v2 import FusedGemmReduceScatter, SymmetricHeap
+
+    peers = [seeded((M, N), 10 + p, torch.float32) * (1000.0 if world > 2 else 1.0) for p in range(1, world)]
+    A_cpu, B_cpu = seeded((M, K), 0, torch.bfloat16), seeded((K, N), 1, torch.bfloat16, scale=K**-0.5)
+    got = []
+    for own in (False, True):
+        heaps = SymmetricHeap.create_all(128 << 20, world)
+        try:
+            ops = [FusedGemmReduceScatter(h, M, N, out_dtype=torch.bfloat16, macro_tile=macro, own_rows_in_registers=own) for h in heaps]
+            A, B = into_heap(heaps[0], A_cpu), into_heap(heaps[0], B_cpu)
+            for op, peer in zip(ops[1:], peers):
+                op.partial.copy_(peer)
+            ops[0].partial.fill_(-3.0)
+            ops[0].mark_peers_ready()
+            ops[0](A, B, variant)
+            ops[0].check_faults()
+            got.append((ops[0].partial.cpu(), [op.out.cpu() for op in ops]))
+        finally:
+            for h in heaps:
+                h.cleanup()
+    (stored, outs), (kept, kept_outs) = got
+    shard = M // world
+    for owner in range(world):
+        assert torch.equal(bits(outs[owner]), bits(oracle.reduce_rows([stored, *peers], owner, torch.bfloat16))), owner
+        assert torch.equal(bits(kept_outs[owner]), bits(outs[owner])), owner
+    assert torch.all(kept[:shard] == -3.0) and not torch.any(stored[:shard] == -3.0)
+    assert torch.equal(bits(kept[shard:]), bits(stored[shard:]))

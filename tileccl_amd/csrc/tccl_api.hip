@@ -1130,6 +1130,11 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // launch replaced, took longer.  bf16 1792 x 3408 x 2144 on two ranks 85 -> 48 us, e4m3 13824 x 736 x 2496 on four 86 -> 50,
   // e4m3 512 x 7056 x 1888 on four 75 -> 35.
   const bool apart = c.op == tccl::kOpReduceScatter && variant != TCCL_S0_BULK && c.world > 1 && !traced && !(tr && tr->num_comm_wgs > 0);
+  // Own rows that the caller keeps out of memory (a promise of the header) stay in the epilogue of 128-row tiles that wait for their
+  // peers, at most one per CU (bf16 on two ranks, us, there and with the sums apart: 1792 x 1200 x 1520 31.2 / 30.7, 1280 x 3136 x 3968
+  // 50.5 / 47.8).
+  const bool keeps_own = apart && !c.peers_resident && (d->flags & TCCL_GEMM_OWN_ROWS_IN_REGISTERS) && !use_macro(d, dev, true) &&
+                         default_gemm_wgs(d, dev, g.tile_rows * g.tile_cols) <= dev.compute_units;
   const auto sums_apart = [&] { return launch_bulk(c, dev, stream, !c.peers_resident, d->num_wgs); };
   if (!gather) {
     // Tiles of a reduce-scatter must not straddle two owners' rows.
@@ -1139,7 +1144,7 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     const bool waits = c.op == tccl::kOpReduceScatter && variant != TCCL_S0_BULK && !c.peers_resident && c.world > 1;
     if (shape >= 0 && !(waits && stream_tiles(shape, seg, 1, d->N) > dev.compute_units))
       return run_stream(d, c, sync, variant, shape, seg, dev, g, stream);
-    if (shape >= 0 && apart) {
+    if (shape >= 0 && apart) {  // (e4m3: 16-bit inputs take no more streaming tiles than one per CU)
       tccl::CommArgs none = c;
       none.op = tccl::kOpNone;
       const int rc = run_stream(d, none, sync, variant, shape, seg, dev, g, stream);
@@ -1156,7 +1161,7 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   const bool sums_inside = variant != TCCL_S0_BULK && use_macro(d, dev, true) && reduces_in_tiles(c) &&
                            !(apart && c.world > 2 && !(d->flags & TCCL_GEMM_OWN_ROWS_IN_REGISTERS));
   TileKernel kernel = use_macro(d, dev, variant != TCCL_S0_BULK) ? kTiles256 : kTiles128;
-  if (lone && !sums_inside) {
+  if (lone && !sums_inside && !keeps_own) {
     const int segs = d->column_shards > 1 ? d->column_shards : 1;
     kernel = choose_tiles(d, d->M / segs, segs, plan_tile_fits_macro(d), variant != TCCL_S0_BULK && c.op != tccl::kOpReduceScatter && c.world > 1, dev).kernel;
   }
@@ -1246,7 +1251,7 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // Two ranks, at most a tile per CU, few K steps: the second launch costs more than 128-row tiles lose that sum in their
   // epilogue (bf16, us, in the epilogue and apart: 4352 x 752 x 336 19.0 / 23.2, 3328 x 800 x 640 20.9 / 21.9, 2560 x 1536 x
   // 1024 25.5 / 26.4; 1792 x 1200 x 1520 30.9 / 28.6, 1280 x 3136 x 3968 54.6 / 48.8).
-  if (apart && !c.peers_resident && c.world == 2 && compute <= dev.compute_units && kernel != kTilesWide && d->K <= 1024) {
+  if (keeps_own || (apart && !c.peers_resident && c.world == 2 && compute <= dev.compute_units && kernel != kTilesWide && d->K <= 1024)) {
     const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
     return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);
   }
