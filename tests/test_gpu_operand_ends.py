@@ -20,7 +20,7 @@ LENGTHS = [(torch.float16, 72), (torch.float16, 104), (torch.bfloat16, 136), (to
 
 def front_of(heap, cpu, rows, cols, behind):
     """`cpu` as the front of a (rows, cols) tensor of the heap whose other elements are `behind`."""
-    whole = heap.allocate_tensor((rows, cols), cpu.dtype)
+    whole = heap.allocate_tensor((rows, -(-cols // 16) * 16), cpu.dtype)  # rows on 16-byte boundaries
     if cpu.dtype == F8:
         whole.view(torch.uint8).fill_(0x7F if behind != 0 else 0)  # e4m3: NaN
     else:
@@ -30,7 +30,7 @@ def front_of(heap, cpu, rows, cols, behind):
     return view
 
 
-def operands(heap, dtype, K, kmajor, behind):
+def operands(heap, dtype, K, kmajor, behind, M=M, N=N):
     half = torch.float16 if dtype == F8 else dtype
     A_cpu, B_cpu = seeded((M, K), 0, half).to(dtype), seeded((K, N), 1, half, scale=K**-0.5).to(dtype)
     A = front_of(heap, A_cpu, M + 256, K + 512, behind)
@@ -59,6 +59,29 @@ def test_all_gather(lib, dtype, K, directions, kmajor):
                 assert_gemm_close(ops[0].local_block, want)
                 got.append(bits(ops[0].local_block).cpu().clone())
         assert all(torch.equal(g, got[0]) for g in got)
+    finally:
+        for h in heaps:
+            h.cleanup()
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("rows,cols", [(256 + 64, 256 + 32), (256 + 72, 256 + 40), (8, 8)])  # last tiles without and with a second half
+@pytest.mark.parametrize("dtype,K", [LENGTHS[0], LENGTHS[3], LENGTHS[7]])
+def test_last_tiles(lib, dtype, K, rows, cols, kmajor):
+    from tileccl_amd.v2 import FusedGemmAllGather, SymmetricHeap
+
+    heaps = SymmetricHeap.create_all(64 << 20, 2)
+    try:
+        out = torch.bfloat16 if dtype == F8 else dtype
+        ops = [FusedGemmAllGather(h, rows, cols, out, directions="push", macro_tile=256) for h in heaps]
+        got = []
+        for behind in (0.0, float("nan")):
+            A, B, want = operands(heaps[0], dtype, K, kmajor, behind, rows, cols)
+            ops[0](A, B, "s2")
+            ops[0].check_faults()
+            assert_gemm_close(ops[0].local_block, want)
+            got.append(bits(ops[0].local_block).cpu().clone())
+        assert torch.equal(got[0], got[1])
     finally:
         for h in heaps:
             h.cleanup()

@@ -547,7 +547,7 @@ struct TileCost {
   double stores, stores_busy; // end of a tile
   double pushes;              // and for each tile that goes to peers as well
 };
-constexpr TileCost kCost256 = {1.05, 0.28, 0.08, 3.0, 4.0, 3.5};
+constexpr TileCost kCost256 = {1.05, 0.28, 0.08, 3.0, 4.0, 3.5};   // fitted to its loop of one barrier per step; full launches are up to 12 % quicker now
 constexpr TileCost kCostWide = {0.60, 0.25, 0.12, 2.5, 1.5, 3.0};
 constexpr TileCost kCostDeep = {0.42, 0.13, 0.12, 2.0, 0.0, 1.5};
 constexpr TileCost kCost128 = {0.50, 0.15, 0.12, 0.5, 0.0, 1.5};   // one workgroup per CU
@@ -569,7 +569,7 @@ struct TileChoice {
 
 // The kernel for `segs` row blocks of `seg_rows` rows in a launch that carries nothing but pushes.  Measured, bf16, on 40
 // seeded shapes of 100 .. 2200 tiles of 128 x 128, row-major and k-major B: the choice is the quickest kernel or within
-// 10 % of it for 76 of the 80, within 18 % for all, 2 % off on average; the 128-tile kernel alone would be 22 % off.
+// 10 % of it for 73 of the 80, within 25 % for all, 2.6 % off on average; the 128-tile kernel alone would be 25 % off.
 // What keeps to the old rule: tiles named by the caller, plan tiles other than 128 x 128, workgroup counts.
 TileChoice choose_tiles(const tccl_gemm_desc* d, int64_t seg_rows, int64_t segs, bool allow256, bool pushes, const tccl_device_info& dev) {
   if (d->in_dtype == TCCL_F8E4M3) return {kTiles256, 0};
@@ -1128,11 +1128,12 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // tiles cannot sum themselves (own rows in whole 256-row tiles, or one streaming tile per CU): communication workgroups
   // beside a three-stage GEMM and a large-tile kernel's workgroups turning to the reductions after their tiles, which this
   // launch replaced, took longer.  bf16 1792 x 3408 x 2144 on two ranks 85 -> 48 us, e4m3 13824 x 736 x 2496 on four 86 -> 50,
-  // e4m3 512 x 7056 x 1888 on four 75 -> 35.
+  // e4m3 512 x 7056 x 1888 on four 75 -> 35 (before the wait made room for a peer on the same device: launch_bulk_reduce()).
+  // Measured with all partials in one memory: where a peer's come over a link this gives up the overlap with the GEMM, and the
+  // rule has to be measured again.
   const bool apart = c.op == tccl::kOpReduceScatter && variant != TCCL_S0_BULK && c.world > 1 && !traced && !(tr && tr->num_comm_wgs > 0);
   // Own rows that the caller keeps out of memory (a promise of the header) stay in the epilogue of 128-row tiles that wait for their
-  // peers, at most one per CU (bf16 on two ranks, us, there and with the sums apart: 1792 x 1200 x 1520 31.2 / 30.7, 1280 x 3136 x 3968
-  // 50.5 / 47.8).
+  // peers, at most one per CU.  (Calls without that flag take the quicker of the two: below.)
   const bool keeps_own = apart && !c.peers_resident && (d->flags & TCCL_GEMM_OWN_ROWS_IN_REGISTERS) && !use_macro(d, dev, true) &&
                          default_gemm_wgs(d, dev, g.tile_rows * g.tile_cols) <= dev.compute_units;
   const auto sums_apart = [&] { return launch_bulk(c, dev, stream, !c.peers_resident, d->num_wgs); };
@@ -1249,8 +1250,8 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   tccl::PushArgs push;
   memset(&push, 0, sizeof push);
   // Two ranks, at most a tile per CU, few K steps: the second launch costs more than 128-row tiles lose that sum in their
-  // epilogue (bf16, us, in the epilogue and apart: 4352 x 752 x 336 19.0 / 23.2, 3328 x 800 x 640 20.9 / 21.9, 2560 x 1536 x
-  // 1024 25.5 / 26.4; 1792 x 1200 x 1520 30.9 / 28.6, 1280 x 3136 x 3968 54.6 / 48.8).
+  // epilogue (bf16, us, in the epilogue and apart: 4352 x 752 x 336 21.3 / 22.9, 3328 x 800 x 640 22.9 / 24.6, 2560 x 1536 x
+  // 1024 27.0 / 28.3; 2048 x 1408 x 1280 29.0 / 28.1, 1792 x 1200 x 1520 31.4 / 30.5, 1280 x 3136 x 3968 51.7 / 49.4).
   if (keeps_own || (apart && !c.peers_resident && c.world == 2 && compute <= dev.compute_units && kernel != kTilesWide && d->K <= 1024)) {
     const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
     return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);

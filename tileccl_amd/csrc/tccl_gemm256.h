@@ -360,8 +360,8 @@ struct Gemm256 {
   static TCCL_D uint32_t clamp_u32(int64_t v) { return v > (int64_t)kDeadOffset ? kDeadOffset : (v < 0 ? 0u : (uint32_t)v); }
 
   // A scalar offset no larger than the window: beyond that nothing says what the hardware's difference is.  At the window's size
-  // every lane reads zero.  It happens in steps that count: the second half of a last step whose rows of B are all past K,
-  // the lower rows of a last tile of few rows.
+  // every lane reads zero.  A row-major B needs it in the last step, where all rows of the second half can be past K.  (For A and a
+  // k-major B make_source() sees to it, which costs the K loop nothing: 8192 x 8192 x 4096, k-major, was 0.6 % slower with it.)
   static TCCL_D uint32_t within(Words4 window, uint32_t off) { return off < window[2] ? off : window[2]; }
 
   TCCL_D int a_row(int h, int i) const { return (wave >> 2) * 128 + h * 64 + (wave & 3) * 16 + 8 * i; }
@@ -409,6 +409,13 @@ struct Gemm256 {
     }
     s.half_a = (uint32_t)(64 * lda * kEsz);
     s.half_b = kBKMajor ? (uint32_t)(32 * g.ldb * kEsz) : (uint32_t)(kStepK / 2 * g.ldb * kEsz);
+    if constexpr (!kPull) {
+      // A last tile that has nothing in half 1 fetches half 0 twice (those rows and columns of the product are not stored): with more than
+      // 64 rows (32 columns) the window reaches past K of the first one in half 1, so no step that counts exceeds it; the
+      // steps behind those have no lane with k < K.
+      if (o.a_rows - o.a_row <= 64) s.half_a = 0;
+      if (kBKMajor && o.b_cols - o.b_col <= 32) s.half_b = 0;
+    }
     s.step_a = kStepK * kEsz;
     s.step_b = kBKMajor ? (uint32_t)(kStepK * kEsz) : (uint32_t)(kStepK * g.ldb * kEsz);
     s.kt_base = 0;
@@ -420,12 +427,12 @@ struct Gemm256 {
 
   // Half h of an operand of K step kt into `stage`: two loads.
   TCCL_D void issue_a(char* stage, const Source& s, int kt, int h) const {
-    const uint32_t off = within(s.a, (uint32_t)kt * s.step_a + h * s.half_a);
-    dma16_pair(stage + a_row(h, 0) * kARow256, stage + a_row(h, 1) * kARow256, s.a, s.off_a, off);
+    dma16_pair(stage + a_row(h, 0) * kARow256, stage + a_row(h, 1) * kARow256, s.a, s.off_a, (uint32_t)kt * s.step_a + h * s.half_a);
   }
   TCCL_D void issue_b(char* stage, const Source& s, int kt, int h) const {
     constexpr int kPitch = kBKMajor ? kARow256 : kBPitch;
-    const uint32_t off = within(s.b, (uint32_t)kt * s.step_b + h * s.half_b);
+    uint32_t off = (uint32_t)kt * s.step_b + h * s.half_b;
+    if constexpr (!kBKMajor) off = within(s.b, off);
     char* to = stage + kAStage256;
     dma16_pair(to + b_row(h, 0) * kPitch, to + b_row(h, 1) * kPitch, s.b, s.off_b, off);
   }
