@@ -314,14 +314,14 @@ struct Gemm256 {
   }
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-  // 16 bytes per lane, global -> LDS, lane l's to `to` + 16 l.  Written out because the compiler makes every later read of
-  // an LDS array wait for all loads into it, whichever part they go to; the waits are k_step's own.  A lane reads zero
-  // where its offset is not below the descriptor's size less the scalar offset, which must not exceed the size: within().  A load that reads M0 wants an instruction between it and
-  // the write of M0, which each block says that it writes (the compiler reserves M0, hence the warnings switched off).
-  // A scalar register that a vector instruction has written (v_readlane of a spilled one, v_readfirstlane) may be read by a
-  // vector memory instruction five wait states later; the hardware does not wait and the compiler does not look in here, so
-  // each block spends five before its first load (check_spills.py looks at the listing, too).
-  // (Two loads to a block: the wait states once.)
+  // Two loads of 16 bytes per lane, global -> LDS, lane l's to `to` + 16 l.  Written out because the compiler makes every later
+  // read of an LDS array wait for all loads into it, whichever part they go to; the waits are k_step's own.  A lane reads zero where its
+  // offset is not below the descriptor's size less the scalar offset, which must not exceed the size (within()).  A load that
+  // reads M0 wants an instruction between it and the write of M0, which the block says that it writes (the compiler reserves M0,
+  // hence the warnings switched off).  A scalar register that a vector instruction has written (v_readlane of a spilled one,
+  // v_readfirstlane) may be read by a vector memory instruction five wait states later; the hardware does not wait and the compiler
+  // does not look in here, so the block spends five before its first load (check_spills.py looks at the listing, too;
+  // 8192 x 8192 x 4096 gather 405.5 -> 409.2 us).
   static TCCL_D void dma16_pair(char* to0, char* to1, Words4 from, const uint32_t (&lane_off)[2], uint32_t off) {
     const uint32_t dst0 = (uint32_t)(uintptr_t)(LdsVoid*)to0, dst1 = (uint32_t)(uintptr_t)(LdsVoid*)to1;
     asm volatile(
