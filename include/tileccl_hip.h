@@ -116,6 +116,12 @@ typedef struct tccl_gemm_desc {
 /* Row-major B has n (0 .. 15, less than a 16-byte vector) rows fewer than K: they are taken as zero.  For a K that is
  * no whole number of vectors: A is then a zero-filled copy, B may stay where it is.  flags |= n << this. */
 #define TCCL_GEMM_B_SHORT_SHIFT 8
+/* A is given by columns: element (m, k) is at A[k * lda + m], i.e. A is the `.t()` view of a (K, M) tensor (the input of
+ * a weight gradient); lda >= M is then the pitch between columns.  16-bit inputs, M a multiple of 8, row-major B, no column
+ * shards, 128 x 128 tiles; tccl_gemm, _allscatter and _allgather.  tccl_gemm_reads_columns() says whether a call is better off so.  The last n
+ * (0 .. 7) of the K columns may be missing, they are taken as zero: flags |= n << TCCL_GEMM_A_SHORT_SHIFT. */
+#define TCCL_GEMM_A_COLUMNS 16
+#define TCCL_GEMM_A_SHORT_SHIFT 12
 /* The launch's sync descriptor is the head of a tccl_sync_desc_arrivals. */
 #define TCCL_GEMM_ARRIVALS 4
 
@@ -256,6 +262,8 @@ int tccl_prim_wait_ge(int32_t* words, int32_t index, int32_t threshold, int64_t 
 
 /* ---- GEMM alone ------------------------------------------------------------------------ */
 int tccl_gemm(const tccl_gemm_desc* gemm, void* stream);
+/* Pure host helper: 1 if this problem, its A given by columns (TCCL_GEMM_A_COLUMNS), is quicker so than with a copy of A in rows. */
+int tccl_gemm_reads_columns(const tccl_gemm_desc* gemm);
 
 /* ---- communication phases alone (the second kernel of S0) ------------------------------
  * tccl_scatter_cols: BulkSyncPattern._scatter_kernel (patterns/bulk_sync.py:242-299).

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import ctypes as C
 import sys
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from functools import partial
 
 import torch
@@ -200,8 +200,10 @@ def _gemm_desc(
     macro_tile: int = 0,
     flags: int = 0,
     column_shards: int = 0,
+    a_columns: bool = False,
 ) -> tuple[_lib.GemmDesc, OperandPlan]:
-    """The descriptor without its operands' addresses, and how those are to be read."""
+    """The descriptor without its operands' addresses, and how those are to be read.  ``a_columns``: the operation takes an A
+    that is given by columns (a transposed view) where it lies; the kernels that would run decide."""
     if not (A.is_cuda and B.is_cuda and C_out.is_cuda):
         raise ValueError("GEMM operands must be device tensors")
     if A.dtype != B.dtype:
@@ -228,6 +230,18 @@ def _gemm_desc(
     d.macro_tile = int(macro_tile)
     d.flags = int(flags) | plan.b_flags
     d.column_shards = int(column_shards)
+    if a_columns and plan.pack_a and not plan.pack_b and M > 1 and A.stride(0) == 1:
+        pitch = int(A.stride(1)) if K > 1 else int(M)
+        if pitch >= M and _rows_vectorised(A, pitch):
+            kept = d.lda, d.flags, d.A, d.B
+            d.lda, d.flags = pitch, d.flags | _lib.GEMM_A_COLUMNS | (plan.K - K) << _lib.GEMM_A_SHORT_SHIFT
+            d.A, d.B = A.data_ptr(), B.data_ptr()
+            taken = _lib.load().tccl_gemm_reads_columns(C.byref(d))
+            d.A, d.B = kept[2:]
+            if taken:
+                plan = replace(plan, pack_a=False, lda=pitch)
+            else:
+                d.lda, d.flags = kept[:2]
     return d, plan
 
 

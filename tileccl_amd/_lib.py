@@ -66,6 +66,8 @@ GEMM_B_KMAJOR = 2  # TCCL_GEMM_B_KMAJOR
 GEMM_ARRIVALS = 4  # TCCL_GEMM_ARRIVALS
 ARRIVAL_STRIDE = 32  # words per plan tile of tccl_sync_desc_arrivals.arrivals
 GEMM_B_SHORT_SHIFT = 8  # TCCL_GEMM_B_SHORT_SHIFT
+GEMM_A_COLUMNS = 16  # TCCL_GEMM_A_COLUMNS
+GEMM_A_SHORT_SHIFT = 12  # TCCL_GEMM_A_SHORT_SHIFT
 STAGED_ALLREDUCE, STAGED_ALLGATHER, STAGED_REDUCE_SCATTER, STAGED_BROADCAST, STAGED_SCATTER = range(5)  # TCCL_STAGED_*
 
 
@@ -166,6 +168,7 @@ SIGNATURES = {
     "tccl_prim_try_wait": (C.c_int, [_vp, _i32, _i32, _i32, _vp, _vp]),
     "tccl_prim_wait_ge": (C.c_int, [_vp, _i32, _i32, _i64, _vp, _vp]),
     "tccl_gemm": (C.c_int, [_P(GemmDesc), _vp]),
+    "tccl_gemm_reads_columns": (C.c_int, [_P(GemmDesc)]),
     "tccl_scatter_cols": (C.c_int, [_vp, _i32, _i64, _i32, _P(ScatterDesc), _P(HeapView), _vp]),
     "tccl_exchange_rows": (C.c_int, [_vp, _i32, _i32, _i64, _i32, _P(HeapView), _P(TransportDesc), _vp]),
     "tccl_reduce_rows": (

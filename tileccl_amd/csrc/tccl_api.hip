@@ -303,7 +303,13 @@ int check_gemm(const tccl_gemm_desc* d, bool ragged_shards = false) {
   const int b_short = (d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15;
   if (b_short >= in_vec || b_short >= d->K || (b_short && b_kmajor))
     return fail(TCCL_ERR_INVALID, "gemm: B can lack fewer than %d rows of K, and only row-major (%d)", in_vec, b_short);
-  if (d->lda < d->K || d->ldb < (b_kmajor ? (int64_t)d->K : (int64_t)d->N * shards) || d->ldc < d->N)
+  const bool a_columns = (d->flags & TCCL_GEMM_A_COLUMNS) != 0;
+  const int a_short = (d->flags >> TCCL_GEMM_A_SHORT_SHIFT) & 15;
+  if (a_columns && (a_short >= in_vec || a_short >= d->K))
+    return fail(TCCL_ERR_INVALID, "gemm: A can lack fewer than %d columns of K where it is given by columns (%d)", in_vec, a_short);
+  if (a_columns && (isz != 2 || b_kmajor || shards > 1 || d->macro_tile == 256 || d->M % in_vec))
+    return fail(TCCL_ERR_UNSUPPORTED, "gemm: A by columns takes 16-bit inputs, M=%d in whole vectors, a row-major B, no column shards and 128x128 tiles", d->M);
+  if (d->lda < (a_columns ? d->M : d->K) || d->ldb < (b_kmajor ? (int64_t)d->K : (int64_t)d->N * shards) || d->ldc < d->N)
     return fail(TCCL_ERR_INVALID, "gemm: leading dimension smaller than the row length");
   if (d->lda % in_vec || d->ldb % in_vec || d->ldc % out_vec || !aligned16(d->A) || !aligned16(d->B) || !aligned16(d->C))
     return fail(TCCL_ERR_UNSUPPORTED, "gemm: A, B, C rows must start on 16-byte boundaries");
@@ -313,7 +319,7 @@ int check_gemm(const tccl_gemm_desc* d, bool ragged_shards = false) {
   // that long unless they are longer.
   const int64_t limit = 0xffffffffll, operand_limit = 0xfffffff0ll;
   const int64_t b_span = (b_kmajor ? 255 * d->ldb + d->K : (int64_t)(d->K - 1) * d->ldb + (int64_t)d->N * shards) * (int64_t)isz;
-  const int64_t a_span = (255 * d->lda + d->K) * (int64_t)isz;
+  const int64_t a_span = (a_columns ? (int64_t)(d->K - 1) * d->lda + d->M : 255 * d->lda + d->K) * (int64_t)isz;
   const int64_t c_span = (255 * d->ldc + d->N) * (int64_t)osz;
   if (b_span > operand_limit || a_span > operand_limit || c_span > limit)
     return fail(TCCL_ERR_UNSUPPORTED, "gemm: an operand spans more than 4 GiB from a tile's base (B %lld, A %lld, C %lld bytes)",
@@ -359,6 +365,8 @@ int build_gemm_args(const tccl_gemm_desc* d, const tccl_device_info& dev, tccl::
   g->ragged = 0;
   g->b_kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) ? 1 : 0;
   g->b_short = (d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15;
+  g->a_columns = (d->flags & TCCL_GEMM_A_COLUMNS) ? 1 : 0;
+  g->a_short = (d->flags >> TCCL_GEMM_A_SHORT_SHIFT) & 15;
   return 0;
 }
 
@@ -502,7 +510,7 @@ int launch_fused(int in_dtype, int out_dtype, const tccl::GemmArgs& gemm, const 
 // against 58.5 us); the fused launches keep the large tiles there (their transfers ride on the K loops).
 bool use_macro(const tccl_gemm_desc* d, const tccl_device_info& dev, bool fused = true) {
   if (d->in_dtype == TCCL_F8E4M3) return true;  // fp8 exists only as the large-tile kernel (check_gemm vets the plan tile)
-  if (!plan_tile_fits_macro(d)) return false;
+  if (!plan_tile_fits_macro(d) || (d->flags & TCCL_GEMM_A_COLUMNS)) return false;
   if (d->column_shards > 1 && (d->M / d->column_shards) % 256) return false;  // a tile must not straddle two row blocks
   if (d->macro_tile == 128) return false;
   if (d->macro_tile == 256) return true;
@@ -583,7 +591,7 @@ TileChoice choose_tiles(const tccl_gemm_desc* d, int64_t seg_rows, int64_t segs,
   };
   if (small <= cus) offer(kTiles128Deep, rounds_us(kCostDeep, small, cus, d, pushes));
   if (small > cus) offer(kTilesWide, rounds_us(kCostWide, wide, cus, d, pushes));
-  if (allow256 && (segs == 1 || seg_rows % 256 == 0))
+  if (allow256 && !(d->flags & TCCL_GEMM_A_COLUMNS) && (segs == 1 || seg_rows % 256 == 0))
     offer(kTiles256, rounds_us(kCost256, (seg_rows + 255) / 256 * segs * ((d->N + 255) / 256), cus, d, pushes));
   return best;
 }
@@ -987,6 +995,7 @@ int stream_shape(const tccl_gemm_desc* d, const tccl_sync_desc* sync, const tccl
                  const tccl_device_info& dev) {
   const bool f8 = d->in_dtype == TCCL_F8E4M3;
   if (!f8 && d->out_dtype != TCCL_F32 && d->out_dtype != d->in_dtype) return -1;
+  if (d->flags & TCCL_GEMM_A_COLUMNS) return -1;
   if (d->macro_tile != 0 || d->num_wgs > 0 || (tr && tr->num_comm_wgs > 0)) return -1;
   const bool fused = variant != TCCL_S0_BULK;
   if (fused) {
@@ -1550,6 +1559,18 @@ int tccl_gemm(const tccl_gemm_desc* d, void* stream) {
                       (hipStream_t)stream);
 }
 
+// The 128 x 128-tile kernels read an A given by columns in place; the streaming and the large-tile kernel do not, and where they would run a
+// launch that turns A into rows comes first (as it does for what check_gemm() refuses).  1000 x 2064 x 1003 bf16 pushed to one peer: 15.5 us in place,
+// 21.6 with that launch.
+int tccl_gemm_reads_columns(const tccl_gemm_desc* d) {
+  if (!d || !(d->flags & TCCL_GEMM_A_COLUMNS) || d->macro_tile != 0 || d->block_m != 128 || d->block_n != 128 || check_gemm(d)) return 0;
+  tccl_device_info dev;
+  if (query_device(-1, &dev)) return 0;
+  tccl_gemm_desc rows = *d;
+  rows.flags &= ~TCCL_GEMM_A_COLUMNS;
+  return !use_macro(&rows, dev, true) && stream_shape(&rows, nullptr, nullptr, TCCL_S0_BULK, d->M, dev) < 0;
+}
+
 static int check_scatter(const tccl_scatter_desc* sc, int M, int N, int esize, int64_t ldc, const void* C) {
   if (!sc) return fail(TCCL_ERR_INVALID, "scatter descriptor is NULL");
   if (sc->cols <= 0 || sc->src_col_offset < 0 || sc->dst_col_offset < 0 || sc->dst_ld <= 0)
@@ -1926,6 +1947,7 @@ int tccl_chained_ag_gemm_rs(const tccl_gemm_desc* d, const void* shard, int64_t 
   int rc = check_gemm(d);
   if (rc) return rc;
   if ((rc = check_heap(heap))) return rc;
+  if (d->flags & TCCL_GEMM_A_COLUMNS) return fail(TCCL_ERR_UNSUPPORTED, "chained: the gathered workspace has rows");
   if (k_shard <= 0 || (int64_t)k_shard * heap->world_size != d->K)
     return fail(TCCL_ERR_INVALID, "chained: input_shard columns (%d) * world_size (%d) != W rows (%d)", k_shard,
                 heap->world_size, d->K);
@@ -2121,6 +2143,7 @@ int tccl_gemm_reducescatter(const tccl_gemm_desc* d, void* out, int32_t out_dtyp
   const int esize = (int)dtype_size(d->out_dtype);
   const int shard = d->M / heap->world_size;
   const bool ragged = d->column_shards > 1 && d->column_shards == heap->world_size && d->M % heap->world_size == 0 && shard % d->block_m;
+  if (d->flags & TCCL_GEMM_A_COLUMNS) return fail(TCCL_ERR_UNSUPPORTED, "reducescatter: A given by columns");
   if (!ragged && (rc = check_sync(sync, variant))) return rc;
   if (ragged)
     return reduce_ragged_shards(d, out, out_dtype, ld_out, heap, sync, tr, emulate_peer, (hipStream_t)stream);

@@ -22,6 +22,9 @@
 //   side, by the choice of the chunk a lane fetches.  Rows >= M, columns >= N and k >= K read as
 //   zero through the buffer bounds (A chunks at k >= K are redirected past the buffer's end).
 //   A k-major B (GemmArgs::b_kmajor: element (k, n) at B[n * ldb + k]) takes A's route and layout.
+//   A given by columns (GemmArgs::a_columns: element (m, k) at A[k * lda + m]; the input of a weight gradient) takes a
+//   row-major B's, 128 rows wide: its operands come out through the transposing reads as well.  1000 x 2064 x 1003 pushed to one
+//   peer: 15.5 us, and 21.6 where a launch of its own turns A into rows first.
 //
 // Pipeline (S stages: 3 in the fused launches, 5 in the GEMM-only kernel): step t computes from stage
 // t % S and issues the loads of K step t + S - 1 into stage (t - 1) % S, which every wavefront finished
@@ -82,6 +85,8 @@ struct GemmArgs {
   int b_kmajor;
   // Row-major B lacks its last b_short of the K rows: they read as zero (A is zero there as well).
   int b_short;
+  // A is given by columns: element (m, k) at A[k * lda + m]; of the K columns it lacks the last a_short, which read as zero.
+  int a_columns, a_short;
 };
 
 // Where a tile whose first output row is row0 and first output column col0 reads its operands.
@@ -224,6 +229,7 @@ struct GemmRole {
   static constexpr int kBPitch = kCols * 2;                     // bytes of a k row of B in a stage
   static constexpr int kStage = kAStage + kStepK * kBPitch;
   static constexpr int kBLanes = kBPitch / 16;                  // lanes that fetch a k row of B
+  static constexpr int kAPitch = kTile * 2, kALanes = kAPitch / 16;  // of a k row of an A given by columns
   static constexpr int kALoads = kAStage / 1024 / kWaves;           // 1 KiB pieces per wavefront and step
   static constexpr int kBLoads = kStepK * kBPitch / 1024 / kWaves;
   static constexpr int kLoads = kALoads + kBLoads;
@@ -271,21 +277,29 @@ struct GemmRole {
   // Swizzle of an A row (of a k-major B row) in a stage: 16-byte chunk c in slot c ^ swizzle(row).
   static TCCL_D int swizzle(int row) { return (row >> 1) & (kRowLanes - 1); }
 
-  template <bool kBKMajor>
+  template <bool kBKMajor, bool kAColumns>
   TCCL_D Source make_source(int row0, int col0) const {
     Source s;
     const int ln = fresh(lane);
     const OperandOrigin o = operand_origin(g, row0, col0);
-    const InT* A = (const InT*)g.A + (int64_t)o.a_row * g.lda;
+    const InT* A = (const InT*)g.A + (kAColumns ? (int64_t)o.a_row : (int64_t)o.a_row * g.lda);
     const InT* B = (const InT*)g.B + (kBKMajor ? (int64_t)o.b_col * g.ldb : (int64_t)o.b_col);
-    s.a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(((int64_t)(o.a_rows - 1 - o.a_row) * g.lda + g.K) * 2), 0x00020000);
+    const int64_t a_elems = kAColumns ? (int64_t)(g.K - 1 - g.a_short) * g.lda + (o.a_rows - o.a_row) : (int64_t)(o.a_rows - 1 - o.a_row) * g.lda + g.K;
+    s.a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(a_elems * 2), 0x00020000);
     const int64_t b_elems = kBKMajor ? (int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K : (int64_t)(g.K - 1 - g.b_short) * g.ldb + (o.b_cols - o.b_col);
     s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(b_elems * 2), 0x00020000);
     constexpr int kRows = 64 / kRowLanes;  // rows of a piece
 #pragma unroll
     for (int i = 0; i < 2; ++i) s.k_lane[i] = ((ln % kRowLanes) ^ swizzle(kRows * i + ln / kRowLanes)) * 8;
 #pragma unroll
-    for (int i = 0; i < kALoads; ++i) s.off_a[i] = (uint32_t)((kRows * (kALoads * wave + i) + ln / kRowLanes) * g.lda * 2 + s.k_lane[i & 1] * 2);
+    for (int i = 0; i < kALoads; ++i) {
+      if constexpr (kAColumns) {
+        const int k = 64 / kALanes * (kALoads * wave + i) + ln / kALanes;
+        s.off_a[i] = (uint32_t)(k * g.lda * 2 + ((ln % kALanes) ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1))) * 16);
+      } else {
+        s.off_a[i] = (uint32_t)((kRows * (kALoads * wave + i) + ln / kRowLanes) * g.lda * 2 + s.k_lane[i & 1] * 2);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < kBLoads; ++j) {
       if constexpr (kBKMajor) {
@@ -297,14 +311,15 @@ struct GemmRole {
         s.off_b[j] = (uint32_t)(k * g.ldb * 2 + c * 16);
       }
     }
-    s.step_a = kStepK * 2;
+    s.step_a = kAColumns ? (uint32_t)(kStepK * g.lda * 2) : (uint32_t)(kStepK * 2);
     s.step_b = kBKMajor ? (uint32_t)(kStepK * 2) : (uint32_t)(kStepK * g.ldb * 2);
     return s;
   }
 
   // Piece i of K step kt, straight into `stage`.
+  template <bool kAColumns>
   TCCL_D void issue_a(char* stage, const Source& s, int kt, int i) const {
-    const bool dead = kt * kStepK + s.k_lane[i & 1] >= g.K;
+    const bool dead = !kAColumns && kt * kStepK + s.k_lane[i & 1] >= g.K;  // (by columns: those >= K lie past the end of the buffer)
     const uint32_t oa = dead ? 0xfffffff0u : s.off_a[i] + kt * s.step_a;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(s.a, (LdsVoid*)(stage + (kALoads * wave + i) * 1024), 16, oa, 0, 0, 0);
   }
@@ -315,17 +330,17 @@ struct GemmRole {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(s.b, (LdsVoid*)(stage + kAStage + (kBLoads * wave + i) * 1024), 16, ob, 0, 0, 0);
   }
   // Load number n of a K step: A 0, B 0, A 1, B 1, then the rest of B.
-  template <bool kBKMajor>
+  template <bool kBKMajor, bool kAColumns>
   TCCL_D void issue(char* stage, const Source& s, int kt, int n) const {
     if (n < 2 * kALoads && !(n & 1))
-      issue_a(stage, s, kt, n >> 1);
+      issue_a<kAColumns>(stage, s, kt, n >> 1);
     else
       issue_b<kBKMajor>(stage, s, kt, n < 2 * kALoads ? n >> 1 : n - kALoads);
   }
-  template <bool kBKMajor>
+  template <bool kBKMajor, bool kAColumns>
   TCCL_D void issue_step(char* stage, const Source& s, int kt) const {
 #pragma unroll
-    for (int n = 0; n < kLoads; ++n) issue<kBKMajor>(stage, s, kt, n);
+    for (int n = 0; n < kLoads; ++n) issue<kBKMajor, kAColumns>(stage, s, kt, n);
   }
 
   // ---- LDS -> MFMA operands -------------------------------------------------------------------
@@ -335,11 +350,16 @@ struct GemmRole {
     uint32_t a_base;   // this lane's row of A row block 0, slot applied
     uint32_t b_base0;  // this lane's address for column block 0
   };
-  template <bool kBKMajor>
+  template <bool kBKMajor, bool kAColumns>
   TCCL_D Reader make_reader() const {
     const int i16 = lane & 15, kg = lane >> 4;
     Reader r;
-    r.a_base = (uint32_t)((wm * 64 + i16) * kRowB + ((kg ^ swizzle(i16)) << 4));
+    if constexpr (kAColumns) {
+      const int t = i16 >> 2, cq = i16 & 3;
+      r.a_base = (uint32_t)((8 * kg + t) * kAPitch + ((wm * 8 + (cq >> 1)) ^ (4 * t) ^ (2 * (kg & 1))) * 16 + (cq & 1) * 8);
+    } else {
+      r.a_base = (uint32_t)((wm * 64 + i16) * kRowB + ((kg ^ swizzle(i16)) << 4));
+    }
     if constexpr (kBKMajor) {
       r.b_base0 = (uint32_t)(kAStage + (wn * 64 + i16) * kRowB + ((kg ^ swizzle(i16)) << 4));
     } else {
@@ -350,18 +370,22 @@ struct GemmRole {
     }
     return r;
   }
+  // Two transposing reads, at `p` and four k rows of `pitch` bytes further on.
+  static TCCL_D Vec turned(const char* p, int pitch) {
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)p);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)(p + 4 * pitch));
+    return __builtin_bit_cast(Vec, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+  template <bool kAColumns>
   TCCL_D Vec load_a(const char* stage, const Reader& r, int h, int rb) const {
+    if constexpr (kAColumns) return turned(stage + (r.a_base ^ (uint32_t)(32 * rb)) + 32 * h * kAPitch, kAPitch);
     return *(const Vec*)(stage + (r.a_base ^ (uint32_t)(64 * h)) + rb * 16 * kRowB);
   }
   template <bool kBKMajor>
   TCCL_D Vec load_b(const char* stage, const Reader& r, int h, int cb) const {
     if constexpr (kBKMajor) return *(const Vec*)(stage + (r.b_base0 ^ (uint32_t)(64 * h)) + cb * 16 * kRowB);
     // column block cb: two chunks further on (the XOR commutes with the swizzle terms)
-    const char* pb = stage + (r.b_base0 ^ (uint32_t)(32 * cb)) + 32 * h * kBPitch;
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)pb);
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsQuad*)(pb + 4 * kBPitch));
-    const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(Vec, both);
+    return turned(stage + (r.b_base0 ^ (uint32_t)(32 * cb)) + 32 * h * kBPitch, kBPitch);
   }
 
   struct Frags {
@@ -377,7 +401,7 @@ struct GemmRole {
   // (four-wavefront form: less the fourth one, which goes out behind the barrier).
   static constexpr int kItems = 4 * kHalves;
   static constexpr int kInFlight = kLoads * (kStages - 2) - (kLoads >= kItems ? kLoads - kItems + 1 : 0);
-  template <bool kBKMajor>
+  template <bool kBKMajor, bool kAColumns>
   TCCL_D void k_step(const char* cur, const char* nxt, char* far, const Source& src, const Reader& rd, int kt_load,
                      f32x4 (&acc)[4][4], Frags& f) const {
 #pragma unroll
@@ -395,12 +419,12 @@ struct GemmRole {
         asm volatile("" ::: "memory");
       }
       if (rb == 3) {
-        f.fa[0] = load_a(from, rd, hn, 0);
-        f.fa[1] = load_a(from, rd, hn, 1);
+        f.fa[0] = load_a<kAColumns>(from, rd, hn, 0);
+        f.fa[1] = load_a<kAColumns>(from, rd, hn, 1);
       } else if (rb < 2) {
-        f.fa[rb + 2] = load_a(cur, rd, h, rb + 2);
+        f.fa[rb + 2] = load_a<kAColumns>(cur, rd, h, rb + 2);
       }
-      if (it < kLoads) issue<kBKMajor>(far, src, kt_load, it);
+      if (it < kLoads) issue<kBKMajor, kAColumns>(far, src, kt_load, it);
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
         acc[rb][cb] = Mfma<InT>::run16(f.fb[cb], f.fa[rb], acc[rb][cb]);
@@ -557,7 +581,7 @@ struct GemmRole {
   }
 
   // ---- one 128 x kCols sub-tile -------------------------------------------------------------------
-  template <int kPolicy, bool kBKMajor, bool kReduce>
+  template <int kPolicy, bool kBKMajor, bool kReduce, bool kAColumns = false>
   TCCL_D void subtile(int row0, int row_end, int col0, int tile_id, const SignalArgs& s) const {
     f32x4 acc[4][4];  // cleared two registers per instruction
 #pragma unroll
@@ -575,21 +599,21 @@ struct GemmRole {
         acc[i][j] = __builtin_bit_cast(f32x4, z);
       }
 
-    const Source src = make_source<kBKMajor>(row0, col0);
-    const Reader rd = make_reader<kBKMajor>();
+    const Source src = make_source<kBKMajor, kAColumns>(row0, col0);
+    const Reader rd = make_reader<kBKMajor, kAColumns>();
     const int ksteps = (g.K + kStepK - 1) / kStepK;
     __syncthreads();  // the previous sub-tile's epilogue has left LDS
     // K steps 0 .. kStages - 2 go out up front (past K: zeros, never consumed).
-    issue_step<kBKMajor>(st0, src, 0);
-    issue_step<kBKMajor>(st1, src, 1);
-    if constexpr (kStages >= 4) issue_step<kBKMajor>(st2, src, 2);
-    if constexpr (kStages == 5) issue_step<kBKMajor>(st3, src, 3);
+    issue_step<kBKMajor, kAColumns>(st0, src, 0);
+    issue_step<kBKMajor, kAColumns>(st1, src, 1);
+    if constexpr (kStages >= 4) issue_step<kBKMajor, kAColumns>(st2, src, 2);
+    if constexpr (kStages == 5) issue_step<kBKMajor, kAColumns>(st3, src, 3);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads * (kStages - 2)) : "memory");  // stage 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     Frags f;
-    f.fa[0] = load_a(st0, rd, 0, 0);
-    f.fa[1] = load_a(st0, rd, 0, 1);
+    f.fa[0] = load_a<kAColumns>(st0, rd, 0, 0);
+    f.fa[1] = load_a<kAColumns>(st0, rd, 0, 1);
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) f.fb[cb] = load_b<kBKMajor>(st0, rd, 0, cb);
     // Step t computes from stage t % kStages, fetches its last operands from the next one and loads K step
@@ -597,35 +621,35 @@ struct GemmRole {
     // per array), so the loop comes in rounds of kStages steps with an exit after every step.
     if constexpr (kStages == 3) {
       for (int kt = 0;; kt += 3) {
-        k_step<kBKMajor>(st0, st1, st2, src, rd, kt + 2, acc, f);
+        k_step<kBKMajor, kAColumns>(st0, st1, st2, src, rd, kt + 2, acc, f);
         if (kt + 1 >= ksteps) break;
-        k_step<kBKMajor>(st1, st2, st0, src, rd, kt + 3, acc, f);
+        k_step<kBKMajor, kAColumns>(st1, st2, st0, src, rd, kt + 3, acc, f);
         if (kt + 2 >= ksteps) break;
-        k_step<kBKMajor>(st2, st0, st1, src, rd, kt + 4, acc, f);
+        k_step<kBKMajor, kAColumns>(st2, st0, st1, src, rd, kt + 4, acc, f);
         if (kt + 3 >= ksteps) break;
       }
     } else if constexpr (kStages == 4) {
       for (int kt = 0;; kt += 4) {
-        k_step<kBKMajor>(st0, st1, st3, src, rd, kt + 3, acc, f);
+        k_step<kBKMajor, kAColumns>(st0, st1, st3, src, rd, kt + 3, acc, f);
         if (kt + 1 >= ksteps) break;
-        k_step<kBKMajor>(st1, st2, st0, src, rd, kt + 4, acc, f);
+        k_step<kBKMajor, kAColumns>(st1, st2, st0, src, rd, kt + 4, acc, f);
         if (kt + 2 >= ksteps) break;
-        k_step<kBKMajor>(st2, st3, st1, src, rd, kt + 5, acc, f);
+        k_step<kBKMajor, kAColumns>(st2, st3, st1, src, rd, kt + 5, acc, f);
         if (kt + 3 >= ksteps) break;
-        k_step<kBKMajor>(st3, st0, st2, src, rd, kt + 6, acc, f);
+        k_step<kBKMajor, kAColumns>(st3, st0, st2, src, rd, kt + 6, acc, f);
         if (kt + 4 >= ksteps) break;
       }
     } else {
       for (int kt = 0;; kt += 5) {
-        k_step<kBKMajor>(st0, st1, st4, src, rd, kt + 4, acc, f);
+        k_step<kBKMajor, kAColumns>(st0, st1, st4, src, rd, kt + 4, acc, f);
         if (kt + 1 >= ksteps) break;
-        k_step<kBKMajor>(st1, st2, st0, src, rd, kt + 5, acc, f);
+        k_step<kBKMajor, kAColumns>(st1, st2, st0, src, rd, kt + 5, acc, f);
         if (kt + 2 >= ksteps) break;
-        k_step<kBKMajor>(st2, st3, st1, src, rd, kt + 6, acc, f);
+        k_step<kBKMajor, kAColumns>(st2, st3, st1, src, rd, kt + 6, acc, f);
         if (kt + 3 >= ksteps) break;
-        k_step<kBKMajor>(st3, st4, st2, src, rd, kt + 7, acc, f);
+        k_step<kBKMajor, kAColumns>(st3, st4, st2, src, rd, kt + 7, acc, f);
         if (kt + 4 >= ksteps) break;
-        k_step<kBKMajor>(st4, st0, st3, src, rd, kt + 8, acc, f);
+        k_step<kBKMajor, kAColumns>(st4, st0, st3, src, rd, kt + 8, acc, f);
         if (kt + 5 >= ksteps) break;
       }
     }
@@ -689,7 +713,12 @@ struct GemmRole {
         for (int sn = 0; sn < per * g.block_n; sn += kCols) {
           const int row0 = first_row + sm, col0 = tc.n * g.block_n + sn;
           if (row0 >= row_end || col0 >= g.N) continue;
-          if (s.mode == kSignalNone) {
+          if (!kReduce && g.a_columns) {  // (with a row-major B: check_gemm)
+            if (s.mode == kSignalNone)
+              subtile<0, false, false, !kReduce>(row0, row_end, col0, tile_id, s);
+            else
+              subtile<kCoherent, false, false, !kReduce>(row0, row_end, col0, tile_id, s);
+          } else if (s.mode == kSignalNone) {
             if (g.b_kmajor)
               subtile<0, true, kReduce>(row0, row_end, col0, tile_id, s);
             else
