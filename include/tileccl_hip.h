@@ -99,7 +99,8 @@ typedef struct tccl_gemm_desc {
 } tccl_gemm_desc;
 
 /* tccl_gemm_reducescatter, variants S1 / S2 where the sums are made in the GEMM's epilogue (shards of whole 256 x 256
- * tiles; small outputs with TCCL_GEMM_ARRIVALS; 128 x 128 tiles that wait for their peers, at most one per CU; elsewhere the
+ * tiles; small outputs with TCCL_GEMM_ARRIVALS; 128 x 128 tiles that wait for their peers, at most one per CU;
+ * fp32 partials of column shards with TCCL_RS_PEERS_RESIDENT (and TCCL_GEMM_ARRIVALS), at most a tile per CU; elsewhere the
  * sums are a launch of their own and every partial is stored):
  * the partial of the rows this rank owns stays in the accumulators, takes the peers' partials
  * in the GEMM epilogue and is never stored to gemm->C (those rows of C keep their old

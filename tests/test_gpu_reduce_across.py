@@ -1,0 +1,101 @@
+"""Reduce-scatters of column shards whose sub-tiles run across the owners: every workgroup has a part of this rank's columns
+and sums it behind its own product.
+
+The sums are made in fp32 from the partials, owner first, the others ascending, and rounded once: bit for bit what the oracle
+makes of the partials, this rank's as the launch with stored partials leaves it."""
+
+import pytest
+import torch
+
+import tileccl_amd as tileccl
+from oracle import collectives as oracle
+from tests.gpu_util import assert_gemm_close, bits, seeded
+
+pytestmark = pytest.mark.gpu
+
+
+def reduce(world, rank, M, N, K, dtype, kmajor, variant, own, launches=1):
+    """(out, this rank's partial as (world, M, N / world), A @ B, the peers' partials) after `launches` launches."""
+    ctxs = tileccl.init_local(world_size=world, heap_size=128 << 20)
+    try:
+        A_cpu, B_cpu = seeded((M, K), 0, dtype), seeded((K, N), 1, dtype, scale=K**-0.5)
+        # (every rank allocates the same things in the same order: the workspaces sit at the same offset)
+        operands = [(c.zeros(M, K, dtype=dtype), c.zeros(N, K, dtype=dtype).t() if kmajor else c.zeros(K, N, dtype=dtype),
+                     c.zeros(M, N // world, dtype=dtype)) for c in ctxs]
+        ctx, (A, B, out) = ctxs[rank], operands[rank]
+        A.copy_(A_cpu)
+        B.copy_(B_cpu)
+        peers = {}
+        for p, c in enumerate(ctxs):  # the order of the sums matters
+            part = c.workspace("gemm_reducescatter.partial", world, M, N // world, dtype=torch.float32)
+            part.fill_(-7.0)
+            if p != rank:
+                peers[p] = seeded((world, M, N // world), 10 + p, torch.float32) * 1000.0
+                part.copy_(peers[p])
+        got = []
+        for _ in range(launches):
+            out.zero_()
+            tileccl.ops.gemm_reducescatter(A, B, out, ctx=ctx, variant=variant, own_rows_in_registers=own)
+            torch.cuda.synchronize()
+            got.append(out.cpu().clone())
+        assert all(torch.equal(bits(o), bits(got[0])) for o in got)
+        partial = ctx.workspace("gemm_reducescatter.partial", world, M, N // world, dtype=torch.float32).cpu().clone()
+        return got[0], partial, A_cpu.float() @ B_cpu.float(), peers
+    finally:
+        for c in ctxs:
+            c.heap.cleanup()
+
+
+# Last columns in the first and in a later run of a tile, runs of a tile that do not exist, a last tile of few rows.
+SHAPES = [
+    (2, 0, 1024, 2 * 776, 1160, torch.float16),
+    (2, 1, 1000, 2 * 904, 1032, torch.bfloat16),
+    (4, 0, 768, 4 * 648, 1160, torch.bfloat16),
+    (4, 2, 640, 4 * 848, 1480, torch.float16),
+    (4, 3, 700, 4 * 712, 1032, torch.float16),
+    (4, 1, 513, 4 * 1024, 2048, torch.bfloat16),
+    (8, 1, 256, 8 * 776, 1096, torch.float16),
+    (8, 6, 330, 8 * 776, 1032, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("variant", ["s1", "s2"])
+@pytest.mark.parametrize("world,rank,M,N,K,dtype", SHAPES)
+def test_sums_are_the_oracles(lib, world, rank, M, N, K, dtype, kmajor, variant):
+    out, partial, want, peers = reduce(world, rank, M, N, K, dtype, kmajor, variant, own=False, launches=2)
+    cols = N // world
+    assert_gemm_close(torch.cat(list(partial), 1), want)
+    partials = [partial if p == rank else peers[p] for p in range(world)]
+    tall = [p.reshape(world * M, cols) for p in partials]
+    assert torch.equal(bits(out), bits(oracle.reduce_rows(tall, rank, dtype)))
+    kept, registers, _, _ = reduce(world, rank, M, N, K, dtype, kmajor, variant, own=True)
+    assert torch.equal(bits(kept), bits(out))
+    others = [q for q in range(world) if q != rank]
+    assert torch.equal(registers[others], partial[others])
+    if kmajor or world < 8:  # (a row-major B on eight ranks keeps the reduction of its own, which reads a stored partial)
+        assert torch.all(registers[rank] == -7.0)
+
+
+def test_every_plan_tile_is_published_once(lib):
+    """The words that the peers of the next launch look at: locks hold the launch's number, counters all tiles of every launch,
+    and the arrival words are zero again."""
+    from tileccl_amd import ops_collective
+
+    M, cols, K, world = 384, 904, 1032, 4
+    ctxs = tileccl.init_local(world_size=world, heap_size=128 << 20)
+    try:
+        A, B = ctxs[0].zeros(M, K, dtype=torch.float16), ctxs[0].zeros(world * cols, K, dtype=torch.float16).t()
+        out = ctxs[0].zeros(M, cols, dtype=torch.float16)
+        words = ops_collective._reduce_scatter_words(ctxs[0], world, M, cols)
+        counts = words.host_plan.tile_counts()
+        for launch in (1, 2, 3):
+            for variant in ("s1", "s2"):
+                tileccl.ops.gemm_reducescatter(A, B, out, ctx=ctxs[0], variant=variant)
+            torch.cuda.synchronize()
+            assert torch.all(words.locks == launch)
+            assert words.counter.tolist() == [launch * int(c) for c in counts]
+            assert torch.all(words.arrivals == 0)
+    finally:
+        for c in ctxs:
+            c.heap.cleanup()

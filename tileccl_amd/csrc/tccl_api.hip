@@ -145,6 +145,28 @@ __global__ __launch_bounds__(256, 1) void gemm128_deep_kernel(tccl::GemmArgs g, 
 #endif
 }
 
+// A reduce-scatter of column shards whose peers' partials are there, at most one tile per CU.  A tile of one owner's columns
+// leaves all of this rank's sums to the CUs that happen to have its tiles (a quarter of them on four ranks: 196 KiB of
+// addends each, 36 us where a reduction of its own behind the GEMM takes 29), and that reduction waits for the whole GEMM, a
+// launch and the memory's first answer.  So a sub-tile takes a run of every owner's columns: each CU has 1 / world of its sums
+// to make, asks for their addends three K steps before its product is done, and publishes its part of `world` plan tiles.
+// bf16, GEMM and reduction before, this after: k-major B 1024 x 4096 x 2048 on 2 / 4 / 8 ranks 30.9 / 30.2 / 30.1 -> 25.1 / 25.1
+// / 26.7 us, 512 x 8192 x 1024 22.3 / 22.0 / 22.1 -> 16.7 / 17.7 / 19.3; row-major 1024 x 4096 x 2048 on 2 / 4 31.6 / 30.2 ->
+// 26.7 / 27.5, 512 x 8192 x 1024 22.5 / 22.2 -> 17.6 / 19.3.  What bounds it is the operands' way from L2, as in the deep form.
+template <typename InT, int kWorld, bool kBKMajor>
+__global__ __launch_bounds__(256, 1) void gemm_across_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::EpilogueReduce reduce) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef tccl::GemmRole<InT, float, 4, 4, 2, kWorld, tccl::across_cols(kWorld, kBKMajor) / 64> Role;
+  __shared__ __attribute__((aligned(1024))) char stage0[Role::kStage];
+  __shared__ __attribute__((aligned(1024))) char stage1[Role::kStage];
+  __shared__ __attribute__((aligned(1024))) char stage2[Role::kStage];
+  __shared__ __attribute__((aligned(1024))) char stage3[Role::kStage];
+  tccl::PushArgs none;
+  none.world = 0;
+  Role(g, none, reduce, stage0, stage1, stage2, stage3).template run_across<kBKMajor>(s, (int)blockIdx.x, (int)gridDim.x);
+#endif
+}
+
 // 128 x 256 tiles, eight wavefronts, K steps of 64 in three stages of 48 KiB: a quarter less operand traffic per FLOP
 // than two 128 x 128 workgroups on a CU, and half as many tiles to share out.  bf16, row-major / k-major B, against
 // those two: 6854 x 520 x 2248 51.2 / 61.0 -> 32.1 / 37.7 us, 534 x 7088 x 2960 60.0 / 72.8 -> 38.8 / 45.7, 1956 x
@@ -1068,6 +1090,60 @@ tccl::EpilogueReduce build_epilogue_reduce(const tccl::CommArgs& c, const tccl_g
   return r;
 }
 
+// May a reduce-scatter of column shards run on sub-tiles across the owners?  Where the 128 x 128-tile kernel of one tile per CU
+// would precede a reduction of its own, the peers' partials are there and only this rank's columns are summed.
+bool sums_across(const tccl_gemm_desc* d, const tccl::CommArgs& c, TileKernel kernel, int tiles, int cus) {
+  if (kernel != kTiles128Deep || d->out_dtype != TCCL_F32 || !c.peers_resident || c.emulate_peer || d->column_shards != c.world) return false;
+  if (c.out_dtype != tccl::kF16 && c.out_dtype != tccl::kBF16) return false;
+  if (c.ld_rs_out_bytes % 16 || ((uintptr_t)c.rs_out & 15)) return false;
+  if (d->K <= 3 * 64) return false;  // the last three K steps are apart, and one goes before them
+  const bool kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) != 0;
+  // A k-major B costs the same in runs.  A row-major one on two ranks costs a tenth more per K step; on four (64 x 256) a third
+  // more, which the reduction's time pays for up to here, bf16: 1024 x 4096 x 2048 31.2 -> 28.1 us, 2048 x 2048 x 2560 33.1 ->
+  // 32.2, 1024 x 4096 x 3072 36.1 -> 36.2, 1500 x 2208 x 2600 38.4 -> 41.5; a device less than half full: 512 x 2048 x 2048 16.9
+  // -> 17.2.  On eight it never does: 1024 x 4096 x 2048 30.4 -> 43.7.
+  const bool pays = kmajor ? (c.world == 2 || c.world == 4 || c.world == 8)
+                           : c.world == 2 || (c.world == 4 && d->K <= 2048 && 2 * tiles >= cus);
+  if (!pays) return false;
+  // 32-bit offsets that now run over all shards.
+  const int64_t limit = 0xfffffff0ll;
+  return (kmajor ? (int64_t)c.world * d->N : (int64_t)d->K) * d->ldb * 2 <= limit && (int64_t)d->M * d->ldc * 4 <= limit;
+}
+
+template <typename InT>
+void launch_across_t(const tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::EpilogueReduce& r, int wgs, hipStream_t stream) {
+  const dim3 grid(wgs), block(tccl::kThreads);
+  if (r.world == 2 && !g.b_kmajor)
+    hipLaunchKernelGGL((gemm_across_kernel<InT, 2, false>), grid, block, 0, stream, g, s, r);
+  else if (r.world == 2)
+    hipLaunchKernelGGL((gemm_across_kernel<InT, 2, true>), grid, block, 0, stream, g, s, r);
+  else if (r.world == 4 && !g.b_kmajor)
+    hipLaunchKernelGGL((gemm_across_kernel<InT, 4, false>), grid, block, 0, stream, g, s, r);
+  else if (r.world == 4)
+    hipLaunchKernelGGL((gemm_across_kernel<InT, 4, true>), grid, block, 0, stream, g, s, r);
+  else
+    hipLaunchKernelGGL((gemm_across_kernel<InT, 8, true>), grid, block, 0, stream, g, s, r);
+}
+
+int launch_across(const tccl_gemm_desc* d, const tccl::GemmArgs& gemm, const tccl::SignalArgs& s, const tccl::CommArgs& c, uint32_t* arrivals,
+                  hipStream_t stream) {
+  tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
+  r.arrivals = arrivals;
+  tccl::GemmArgs g = gemm;
+  const int cols = tccl::across_cols(r.world, g.b_kmajor), rows = 128 * 128 / cols;  // of a sub-tile
+  const int total = (g.wrap_rows + rows - 1) / rows * g.tile_cols * (128 * r.world / cols);
+  // A patch as high in rows as the other kernels': the XCD that has fewer columns of B fetches less of what costs more (64 x 256,
+  // 1024 x 4096 x 2048: bands of 2 / 4 / 8 / 16 sub-tiles 33.6 / 30.2 / 28.9 / 27.5 us).
+  r.band = cols == 256 ? 2 * g.group_m : g.group_m;
+  g.span = gemm_span(total, r.band, g.xcds);
+  if (d->in_dtype == TCCL_F16)
+    launch_across_t<_Float16>(g, s, r, total, stream);
+  else
+    launch_across_t<__bf16>(g, s, r, total, stream);
+  TCCL_HIP(hipGetLastError());
+  return 0;
+}
+
 void add_stream_reduce(const tccl::CommArgs& c, const tccl_gemm_desc* d, tccl::StreamArgs* a) {
   a->heap_bases = c.heap_bases;
   a->rank = c.rank;
@@ -1265,6 +1341,8 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
     const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
     return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);
   }
+  if (apart && arrival_words(d, sync) && sums_across(d, c, kernel, total_tiles, dev.compute_units))
+    return launch_across(d, g, s, c, arrival_words(d, sync), stream);
   if (apart) {
     const int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, kernel, compute, 0, nullptr, stream);
     return rc ? rc : sums_apart();
@@ -2119,6 +2197,7 @@ static int reduce_ragged_shards(const tccl_gemm_desc* d, void* out, int32_t out_
     g.tile_rows = (g.wrap_rows + 127) / 128 * d->column_shards;
     tccl::SignalArgs s;
     memset(&s, 0, sizeof s);
+    if (sums_across(d, c, together.kernel, g.tile_rows * g.tile_cols, dev.compute_units)) return launch_across(d, g, s, c, nullptr, stream);
     rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, together.kernel, tile_wgs(together.kernel, d, dev, g.tile_rows * g.tile_cols), 0,
                       nullptr, stream);
     return rc ? rc : launch_bulk(c, dev, stream);

@@ -141,6 +141,17 @@ struct PushArgs {
   const int64_t* heap_bases;  // C's address inside target q is C + heap_bases[q] - heap_bases[rank]
 };
 
+// Counters of neighbouring plan tiles in one cache line take each other's time: 256 tiles of one launch counting into 16
+// words of a line or two cost it 2.2 us (512 x 512 x 256, two ranks: 8.3 -> 6.0 us; 16 x 2048 x 4096 9.2 -> 8.5).
+constexpr int kArrivalStride = 32;
+// Of a plan tile's words a launch counts in one that no launch near it in number uses, and neither does the other kind of
+// launch, which is numbered separately: launches of the same words that overlap (two streams), whatever their tile shapes, do not
+// add to each other's counts, so each of them leaves zero behind and publishes a plan tile exactly when it is complete.
+TCCL_HD int arrival_word(int plan_tile, int32_t epoch, bool by_tile) {
+  constexpr int kHalf = kArrivalStride / 2;
+  return kArrivalStride * plan_tile + (int)((uint32_t)epoch % kHalf) + (by_tile ? kHalf : 0);
+}
+
 // Reduce-scatter carried out in the epilogue of the GEMM: the tiles of rows this rank owns take the peers' partials
 // and leave as output; under single-GPU emulation the other owners' rows are reduced as well.
 struct EpilogueReduce {
@@ -157,7 +168,14 @@ struct EpilogueReduce {
   const int32_t* tile_counts;
   int64_t* fault;
   int64_t spin_ticks;
+  int band;              // sub-tiles across the owners: rows of sub-tiles in a band (tile_coords())
+  uint32_t* arrivals;    // kArrivalStride words per plan tile (arrival_word()), zero between launches
 };
+
+// Columns of a sub-tile across the owners (its rows: 16384 over that).  A row-major B is read in runs of an owner's columns:
+// those of four ranks get 64, whole 128-byte lines, in a sub-tile of 64 x 256.  With runs of 32 they take as long per K step,
+// with a quarter less to read; the eight ranks' runs of 16 take half as long again (sums_across()).
+TCCL_HD constexpr int across_cols(int world, bool b_kmajor) { return world == 4 && !b_kmajor ? 256 : 128; }
 
 template <typename T>
 struct Mfma;
@@ -219,17 +237,21 @@ TCCL_D void warm_kernargs() {
   asm volatile("" ::"s"(any));
 }
 
-template <typename InT, typename OutT, int kStages = 3, int kWaves = 4, int kHalves = 1>
+// kWorld: sub-tiles across the owners of a reduce-scatter of so many column shards (run_across()).
+template <typename InT, typename OutT, int kStages = 3, int kWaves = 4, int kHalves = 1, int kWorld = 0, int kWn = kWaves / 2>
 struct GemmRole {
-  static constexpr int kWn = kWaves / 2, kCols = 64 * kWn;      // wavefronts across, columns of a sub-tile
+  static constexpr int kCols = 64 * kWn, kRows = 64 * (kWaves / kWn);  // of a sub-tile (kWn: wavefronts across)
+  // Column block cb of wavefront wn: columns 64 wn + 16 cb .. + 15, or, spread, 64 cb + 16 wn .. + 15: every wavefront has a
+  // part of each owner's run of 64.
+  static constexpr bool kSpread = kWorld == 4 && kWn == 4;
   static constexpr int kStepK = 32 * kHalves;
   static constexpr int kRowB = 2 * kStepK;                      // bytes of an A row in a stage
   static constexpr int kRowLanes = kRowB / 16;                  // lanes that fetch one
-  static constexpr int kAStage = kTile * kRowB;
+  static constexpr int kAStage = kRows * kRowB;
   static constexpr int kBPitch = kCols * 2;                     // bytes of a k row of B in a stage
   static constexpr int kStage = kAStage + kStepK * kBPitch;
   static constexpr int kBLanes = kBPitch / 16;                  // lanes that fetch a k row of B
-  static constexpr int kAPitch = kTile * 2, kALanes = kAPitch / 16;  // of a k row of an A given by columns
+  static constexpr int kAPitch = kRows * 2, kALanes = kAPitch / 16;  // of a k row of an A given by columns
   static constexpr int kALoads = kAStage / 1024 / kWaves;           // 1 KiB pieces per wavefront and step
   static constexpr int kBLoads = kStepK * kBPitch / 1024 / kWaves;
   static constexpr int kLoads = kALoads + kBLoads;
@@ -277,38 +299,45 @@ struct GemmRole {
   // Swizzle of an A row (of a k-major B row) in a stage: 16-byte chunk c in slot c ^ swizzle(row).
   static TCCL_D int swizzle(int row) { return (row >> 1) & (kRowLanes - 1); }
 
+  // Column `c` of a sub-tile, as one of B's counted from the sub-tile's first: across the owners, equal runs of every shard.
+  TCCL_D int64_t across(int c) const {
+    if constexpr (kWorld == 0) return c;
+    return (int64_t)(c / kRun) * g.N + c % kRun;
+  }
+
   template <bool kBKMajor, bool kAColumns>
   TCCL_D Source make_source(int row0, int col0) const {
     Source s;
     const int ln = fresh(lane);
-    const OperandOrigin o = operand_origin(g, row0, col0);
+    OperandOrigin o = operand_origin(g, kWorld ? 0 : row0, col0);
+    if constexpr (kWorld != 0) o.a_row = row0;
     const InT* A = (const InT*)g.A + (kAColumns ? (int64_t)o.a_row : (int64_t)o.a_row * g.lda);
     const InT* B = (const InT*)g.B + (kBKMajor ? (int64_t)o.b_col * g.ldb : (int64_t)o.b_col);
     const int64_t a_elems = kAColumns ? (int64_t)(g.K - 1 - g.a_short) * g.lda + (o.a_rows - o.a_row) : (int64_t)(o.a_rows - 1 - o.a_row) * g.lda + g.K;
     s.a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, clamp_u32(a_elems * 2), 0x00020000);
     const int64_t b_elems = kBKMajor ? (int64_t)(o.b_cols - 1 - o.b_col) * g.ldb + g.K : (int64_t)(g.K - 1 - g.b_short) * g.ldb + (o.b_cols - o.b_col);
     s.b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, clamp_u32(b_elems * 2), 0x00020000);
-    constexpr int kRows = 64 / kRowLanes;  // rows of a piece
+    constexpr int kPiece = 64 / kRowLanes;  // rows of a piece
 #pragma unroll
-    for (int i = 0; i < 2; ++i) s.k_lane[i] = ((ln % kRowLanes) ^ swizzle(kRows * i + ln / kRowLanes)) * 8;
+    for (int i = 0; i < 2; ++i) s.k_lane[i] = ((ln % kRowLanes) ^ swizzle(kPiece * i + ln / kRowLanes)) * 8;
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) {
       if constexpr (kAColumns) {
         const int k = 64 / kALanes * (kALoads * wave + i) + ln / kALanes;
         s.off_a[i] = (uint32_t)(k * g.lda * 2 + ((ln % kALanes) ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1))) * 16);
       } else {
-        s.off_a[i] = (uint32_t)((kRows * (kALoads * wave + i) + ln / kRowLanes) * g.lda * 2 + s.k_lane[i & 1] * 2);
+        s.off_a[i] = (uint32_t)((kPiece * (kALoads * wave + i) + ln / kRowLanes) * g.lda * 2 + s.k_lane[i & 1] * 2);
       }
     }
 #pragma unroll
     for (int j = 0; j < kBLoads; ++j) {
       if constexpr (kBKMajor) {
-        const int row = kRows * (kBLoads * wave + j) + ln / kRowLanes;
-        s.off_b[j] = (uint32_t)(row * g.ldb * 2 + s.k_lane[j & 1] * 2);
+        const int row = kPiece * (kBLoads * wave + j) + ln / kRowLanes;
+        s.off_b[j] = (uint32_t)(across(row) * g.ldb * 2 + s.k_lane[j & 1] * 2);
       } else {
         const int k = 64 / kBLanes * (kBLoads * wave + j) + ln / kBLanes;
         const int c = (ln % kBLanes) ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1));
-        s.off_b[j] = (uint32_t)(k * g.ldb * 2 + c * 16);
+        s.off_b[j] = (uint32_t)(k * g.ldb * 2 + across(c * 8) * 2);
       }
     }
     s.step_a = kAColumns ? (uint32_t)(kStepK * g.lda * 2) : (uint32_t)(kStepK * 2);
@@ -365,7 +394,7 @@ struct GemmRole {
     } else {
       // Lane group kg covers k rows 8 kg .. + 7 in two transposing reads (k + 0, k + 4).
       const int t = i16 >> 2, cq = i16 & 3;
-      const int chunk = (wn * 8 + (cq >> 1)) ^ (4 * t) ^ (2 * (kg & 1));
+      const int chunk = (wn * (kSpread ? 2 : 8) + (cq >> 1)) ^ (4 * t) ^ (2 * (kg & 1));
       r.b_base0 = (uint32_t)(kAStage + (8 * kg + t) * kBPitch + chunk * 16 + (cq & 1) * 8);
     }
     return r;
@@ -384,8 +413,8 @@ struct GemmRole {
   template <bool kBKMajor>
   TCCL_D Vec load_b(const char* stage, const Reader& r, int h, int cb) const {
     if constexpr (kBKMajor) return *(const Vec*)(stage + (r.b_base0 ^ (uint32_t)(64 * h)) + cb * 16 * kRowB);
-    // column block cb: two chunks further on (the XOR commutes with the swizzle terms)
-    return turned(stage + (r.b_base0 ^ (uint32_t)(32 * cb)) + 32 * h * kBPitch, kBPitch);
+    // column block cb: two chunks further on, spread eight (the XOR commutes with the swizzle terms)
+    return turned(stage + (r.b_base0 ^ (uint32_t)((kSpread ? 128 : 32) * cb)) + 32 * h * kBPitch, kBPitch);
   }
 
   struct Frags {
@@ -400,8 +429,10 @@ struct GemmRole {
   // together.  At the barrier the loads that may still be in flight are those of the kStages - 2 steps before
   // (four-wavefront form: less the fourth one, which goes out behind the barrier).
   static constexpr int kItems = 4 * kHalves;
-  static constexpr int kInFlight = kLoads * (kStages - 2) - (kLoads >= kItems ? kLoads - kItems + 1 : 0);
-  template <bool kBKMajor, bool kAColumns>
+  static constexpr int kInFlight = kLoads * (kStages - 2) - (kLoads >= kItems ? 1 : 0);
+  // kLeft > 0: one of the last steps of a sub-tile across the owners, behind request_sums(): no loads go out any more and
+  // `kLeft - 1` steps follow; what has been requested stays in flight.
+  template <bool kBKMajor, bool kAColumns, int kLeft = 0>
   TCCL_D void k_step(const char* cur, const char* nxt, char* far, const Source& src, const Reader& rd, int kt_load,
                      f32x4 (&acc)[4][4], Frags& f) const {
 #pragma unroll
@@ -410,7 +441,17 @@ struct GemmRole {
       const bool last = it == kItems - 1;
       const char* from = last ? nxt : cur;  // of the next half's operands
       const int hn = last ? 0 : h + 1;
-      if (last) {
+      if (last && kLeft > 0) {
+        if (kLeft == 1) {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        } else if (sums_here()) {
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kLeft == 3 ? kLoads : 0) + kAddends) : "memory");
+        } else {
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kLeft == 3 ? kLoads : 0) : "memory");
+        }
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      } else if (last) {
         // The loads of K step t + 1 (into `nxt`) have landed; this wavefront's reads of `cur` are done.
         // The barrier is the bare instruction (__syncthreads() carries a release fence); the empty asm
         // keeps LDS accesses from moving across it.
@@ -418,19 +459,21 @@ struct GemmRole {
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
       }
-      if (rb == 3) {
+      if (rb == 3 && last && kLeft == 1) {
+      } else if (rb == 3) {
         f.fa[0] = load_a<kAColumns>(from, rd, hn, 0);
         f.fa[1] = load_a<kAColumns>(from, rd, hn, 1);
       } else if (rb < 2) {
         f.fa[rb + 2] = load_a<kAColumns>(cur, rd, h, rb + 2);
       }
-      if (it < kLoads) issue<kBKMajor, kAColumns>(far, src, kt_load, it);
+      if (kLeft == 0 && it < kLoads) issue<kBKMajor, kAColumns>(far, src, kt_load, it);
+      if (kLeft == 0 && it + kItems < kLoads) issue<kBKMajor, kAColumns>(far, src, kt_load, it + kItems);
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
         acc[rb][cb] = Mfma<InT>::run16(f.fb[cb], f.fa[rb], acc[rb][cb]);
         if (rb == 3) {
           __builtin_amdgcn_sched_barrier(0);
-          f.fb[cb] = load_b<kBKMajor>(from, rd, hn, cb);
+          if (!(last && kLeft == 1)) f.fb[cb] = load_b<kBKMajor>(from, rd, hn, cb);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -580,6 +623,99 @@ struct GemmRole {
     }
   }
 
+  // ---- sub-tiles across the owners: the sums -------------------------------------------------------------
+  // Each owner has kRun of the columns.  The wavefronts that hold this rank's sum them; their addends are requested three K
+  // steps before the last one ends.
+  static constexpr int kRun = kWorld ? kCols / (kWorld ? kWorld : 1) : 16;
+  static constexpr int kOwnCols = kSpread ? 16 : kRun, kOwners = 64 / kOwnCols;  // of an owner in a wavefront; owners there
+  static constexpr int kOwnChunks = kOwnCols / 4, kOwnRounds = 32 * kOwnChunks / 64;  // 16 bytes of fp32; per 32-row slab
+  static constexpr int kAddends = 2 * kOwnRounds * (kWorld - 1);                  // per lane
+  struct Addends {
+    f32x4 v[2][kOwnRounds][kWorld > 1 ? kWorld - 1 : 1];
+  };
+  TCCL_D bool sums_here() const { return kSpread || wn == reduce.rank / kOwners; }
+  // This lane's chunk of round r: row of the slab, column of the run.
+  static TCCL_D int own_row(int ln, int r) { return (ln + 64 * r) / kOwnChunks; }
+  TCCL_D int own_col(int ln) const { return (kSpread ? wn * kOwnCols : 0) + ln % kOwnChunks * 4; }  // (64 is a multiple of kOwnChunks)
+  TCCL_D void request_sums(int row0, int col0, Addends& w) const {
+    if (!sums_here()) return;
+    const int ln = (int)((uint32_t)fresh(lane) & 63u), rows = g.wrap_rows - row0, col = own_col(ln);
+    const bool live = col < g.N - col0;
+    const int64_t first = (int64_t)(uintptr_t)((const float*)g.C + ((int64_t)reduce.rank * g.wrap_rows + row0) * g.ldc + col0);
+    const uint32_t pitch = (uint32_t)(g.ldc * 4);
+#pragma unroll
+    for (int n = 0; n < kWorld - 1; ++n) {
+      const int p = n + (n >= reduce.rank);
+      const __amdgpu_buffer_rsrc_t from = window(first + (reduce.heap_bases[p] - reduce.heap_bases[reduce.rank]));
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+        for (int r = 0; r < kOwnRounds; ++r) {  // (a chunk that does not exist: the first one instead)
+          const uint32_t row = wm * 64 + bi * 32 + own_row(ln, r);
+          w.v[bi][r][n] = __builtin_bit_cast(f32x4, ld16<kCoherent>(from, live && (int)row < rows ? row * pitch + col * 4 : 0u));
+        }
+    }
+  }
+  template <bool kBKMajor>
+  TCCL_D void last_steps(const char* s0, const char* s1, const char* s2, const char* s3, const Source& src, const Reader& rd,
+                         f32x4 (&acc)[4][4], Frags& f) const {
+    k_step<kBKMajor, false, 3>(s0, s1, nullptr, src, rd, 0, acc, f);
+    k_step<kBKMajor, false, 2>(s1, s2, nullptr, src, rd, 0, acc, f);
+    k_step<kBKMajor, false, 1>(s2, s3, nullptr, src, rd, 0, acc, f);
+  }
+  template <int kPolicy>
+  TCCL_D void epilogue_across(int row0, int col0, const f32x4 (&acc)[4][4], const Addends& w) const {
+    static_assert(sizeof(OutT) == 4 || kWorld == 0, "fp32 partials");
+    static_assert(kStage >= 32768 || kWorld == 0, "a staging window per wavefront");
+    constexpr int kRowBytes = 256, kChunks = 16, kRounds = 32 * kChunks / 64;
+    char* win = st0 + wave * 8192;
+    const int ln = (int)((uint32_t)fresh(lane) & 63u), i16 = ln & 15, kg = ln >> 4;
+    const int rows = g.wrap_rows - row0, cols = g.N - col0;
+    const bool mine = sums_here();
+    const int first = reduce.rank % kOwners * kOwnChunks;  // this rank's first chunk in a row of the wavefront
+    const __amdgpu_buffer_rsrc_t rc = window((int64_t)(uintptr_t)((float*)g.C + (int64_t)row0 * g.ldc + col0));
+    const __amdgpu_buffer_rsrc_t to = window((int64_t)(uintptr_t)reduce.out + (int64_t)row0 * reduce.ld_out_bytes + (int64_t)col0 * 2);
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi) {
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+          const int row = 16 * r + i16;
+          *(f32x4*)(win + row * kRowBytes + ((4 * cb + kg) ^ (row & 7)) * 16) = acc[2 * bi + r][cb] * g.alpha;
+        }
+      asm volatile("" ::: "memory");  // staged by this wavefront itself: LDS keeps the order
+#pragma unroll
+      for (int r = 0; r < kRounds; ++r) {
+        const int row = (ln + 64 * r) / kChunks, chunk = ln % kChunks, lrow = wm * 64 + bi * 32 + row;
+        const int q = (kSpread ? 0 : wn * kOwners) + chunk / kOwnChunks, col = own_col(chunk);
+        const u32x4 v = *(const u32x4*)(win + row * kRowBytes + ((chunk ^ (row & 7)) * 16));
+        if (lrow < rows && col < cols && !(q == reduce.rank && reduce.own_in_registers))
+          __builtin_amdgcn_raw_buffer_store_b128(v, rc, (uint32_t)((((int64_t)q * g.wrap_rows + lrow) * g.ldc + col) * 4), 0, kPolicy);
+      }
+      if (mine) {
+        const int col = own_col(ln), chunk = first + ln % kOwnChunks;
+#pragma unroll
+        for (int r = 0; r < kOwnRounds; ++r) {
+          const int row = own_row(ln, r), lrow = wm * 64 + bi * 32 + row;
+          f32x4 sum = *(const f32x4*)(win + row * kRowBytes + ((chunk ^ (row & 7)) * 16));  // the owner's first
+#pragma unroll
+          for (int n = 0; n < kWorld - 1; ++n) sum += w.v[bi][r][n];
+          uint16_t h[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            h[j] = reduce.out_dtype == kBF16 ? __builtin_bit_cast(uint16_t, (__bf16)sum[j]) : __builtin_bit_cast(uint16_t, (_Float16)sum[j]);
+          typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+          u32x2 o;
+          __builtin_memcpy(&o, h, 8);
+          if (lrow < rows && col < cols)
+            __builtin_amdgcn_raw_buffer_store_b64(o, to, (uint32_t)(lrow * reduce.ld_out_bytes + col * 2), 0, kStreaming);
+        }
+      }
+      asm volatile("" ::: "memory");
+    }
+  }
+
   // ---- one 128 x kCols sub-tile -------------------------------------------------------------------
   template <int kPolicy, bool kBKMajor, bool kReduce, bool kAColumns = false>
   TCCL_D void subtile(int row0, int row_end, int col0, int tile_id, const SignalArgs& s) const {
@@ -619,7 +755,35 @@ struct GemmRole {
     // Step t computes from stage t % kStages, fetches its last operands from the next one and loads K step
     // t + kStages - 1 into the one before.  Stages are named statically (the compiler tracks loads into LDS
     // per array), so the loop comes in rounds of kStages steps with an exit after every step.
-    if constexpr (kStages == 3) {
+    if constexpr (kWorld != 0) {
+      Addends w;
+      int left = 0;  // stage of the first of the last three steps
+      for (int kt = 0, n = ksteps - 3;; kt += 4) {
+        k_step<kBKMajor, kAColumns>(st0, st1, st3, src, rd, kt + 3, acc, f);
+        left = 1;
+        if (kt + 1 >= n) break;
+        k_step<kBKMajor, kAColumns>(st1, st2, st0, src, rd, kt + 4, acc, f);
+        left = 2;
+        if (kt + 2 >= n) break;
+        k_step<kBKMajor, kAColumns>(st2, st3, st1, src, rd, kt + 5, acc, f);
+        left = 3;
+        if (kt + 3 >= n) break;
+        k_step<kBKMajor, kAColumns>(st3, st0, st2, src, rd, kt + 6, acc, f);
+        left = 0;
+        if (kt + 4 >= n) break;
+      }
+      request_sums(row0, col0, w);
+      if (left == 0)
+        last_steps<kBKMajor>(st0, st1, st2, st3, src, rd, acc, f);
+      else if (left == 1)
+        last_steps<kBKMajor>(st1, st2, st3, st0, src, rd, acc, f);
+      else if (left == 2)
+        last_steps<kBKMajor>(st2, st3, st0, st1, src, rd, acc, f);
+      else
+        last_steps<kBKMajor>(st3, st0, st1, st2, src, rd, acc, f);
+      epilogue_across<kPolicy>(row0, col0, acc, w);
+      return;
+    } else if constexpr (kStages == 3) {
       for (int kt = 0;; kt += 3) {
         k_step<kBKMajor, kAColumns>(st0, st1, st2, src, rd, kt + 2, acc, f);
         if (kt + 1 >= ksteps) break;
@@ -685,6 +849,39 @@ struct GemmRole {
     }
     __syncthreads();
     return *verdict != 0;
+  }
+
+  // ---- sub-tiles across the owners ----------------------------------------------------------------------
+  // A sub-tile has kRows rows of A and kRun columns of every owner's shard; plan tiles of 128 x 128.
+  template <bool kBKMajor>
+  TCCL_D void run_across(const SignalArgs& s, int wg, int num_wgs) const {
+    constexpr int kParts = 128 / kRun;  // runs of a plan tile
+    const int tiles = (g.wrap_rows + kRows - 1) / kRows, cols = g.tile_cols * kParts, total = tiles * cols;
+    for (int slot = wg; slot < total; slot += num_wgs) {
+      const TileCoord tc = tile_coords(tile_for_slot(slot, total, g.xcds, g.span), tiles, cols, reduce.band);
+      const int n = tc.n / kParts, col0 = n * 128 + tc.n % kParts * kRun;
+      if (col0 >= g.N) continue;
+      if (s.mode == kSignalNone) {
+        subtile<0, kBKMajor, true>(tc.m * kRows, 0, col0, 0, s);
+        continue;
+      }
+      subtile<kCoherent, kBKMajor, true>(tc.m * kRows, 0, col0, 0, s);
+      wait_vmem();  // the write-through stores have landed
+      __syncthreads();
+      if (tid < kWorld) {  // one plan tile of each shard; the last sub-tile to cover a part of it publishes
+        const int id = tile_id_of(tid * (g.tile_rows / kWorld) + tc.m * kRows / 128, n, g.tile_rows, g.tile_cols, g.group_m);
+        const int left = (g.N - n * 128 + kRun - 1) / kRun;
+        const uint32_t parts = (uint32_t)(128 / kRows * (left < kParts ? left : kParts));  // (with signals: whole plan tiles of rows)
+        // Counts to parts - 1 and starts over by itself, so the word is zero again when the launch has ended.
+        const uint32_t before = parts > 1 ? atomicInc(&reduce.arrivals[arrival_word(id, s.epoch, s.mode == kSignalTile)], parts - 1) : 0u;
+        if (before == parts - 1) {
+          if (s.mode == kSignalTile)
+            tile_publish(s.locks, id, s.epoch);
+          else
+            tile_signal_add<true>(s.counter, s.group_table[id], 1);
+        }
+      }
+    }
   }
 
   // ---- persistent loop over plan tiles ----------------------------------------------------------

@@ -20,17 +20,6 @@
 
 namespace tccl {
 
-// Counters of neighbouring plan tiles in one cache line take each other's time: 256 tiles of one launch counting into 16
-// words of a line or two cost it 2.2 us (512 x 512 x 256, two ranks: 8.3 -> 6.0 us; 16 x 2048 x 4096 9.2 -> 8.5).
-constexpr int kArrivalStride = 32;
-// Of a plan tile's words a launch counts in one that no launch near it in number uses, and neither does the other kind of
-// launch, which is numbered separately: launches of the same words that overlap (two streams), whatever their tile shapes, do not
-// add to each other's counts, so each of them leaves zero behind and publishes a plan tile exactly when it is complete.
-TCCL_HD int arrival_word(int plan_tile, int32_t epoch, bool by_tile) {
-  constexpr int kHalf = kArrivalStride / 2;
-  return kArrivalStride * plan_tile + (int)((uint32_t)epoch % kHalf) + (by_tile ? kHalf : 0);
-}
-
 // The pull half of an all-gather: this rank's copy of every peer's row block.  Workgroups behind those of the tiles share it
 // out and wait (bounded) for the peers; a workgroup with a tile never waits (stream_grid()).
 struct StreamPull {

@@ -234,7 +234,9 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     with the peers' partials.  On 256 x 256 tiles and in the streaming kernel that is one launch, which
     sums each tile as it finishes, and (``own_rows_in_registers``, the default)
     block ``rank`` never leaves the accumulators as a partial: its part of the workspace is not
-    written.  On 128 x 128 tiles with the peers' partials resident the sums are a second launch.  ``variant`` picks the schedule (``"s0"`` bulk, ``"s1"`` tile by tile, ``"s2"``
+    written.  So is one with at most a 128 x 128 tile per CU and the peers' partials resident, on 2, 4 or 8 ranks
+    (a row-major ``B`` on four ranks up to ``K`` = 2048, not on eight); elsewhere on 128 x 128 tiles with resident partials
+    the sums are a second launch.  ``variant`` picks the schedule (``"s0"`` bulk, ``"s1"`` tile by tile, ``"s2"``
     TileGroup).  ``emulate_peer`` (single-GPU emulation) also writes the other ranks' outputs
     into their slices.
 
@@ -251,8 +253,8 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     have made the same number of calls.
     ``implementation`` is accepted for signature parity; there is one implementation here.
     When ``M`` is not a multiple of the 128-row plan tile there are no signals: the peers' partials
-    are taken to be there.  The streaming kernel sums in its epilogue; otherwise one GEMM launch for all column
-    blocks, or one per block where each fills the device by itself, and the bulk reduction.
+    are taken to be there.  The streaming kernel and the one-launch form sum in their epilogue; otherwise one GEMM launch
+    for all column blocks, or one per block where each fills the device by itself, and the bulk reduction.
     """
     if implementation not in ("auto", "device", "hip"):
         raise ValueError(f"unsupported gemm_reducescatter implementation {implementation!r}")
