@@ -56,6 +56,10 @@ SHAPES = [
     (4, 1, 513, 4 * 1024, 2048, torch.bfloat16),
     (8, 1, 256, 8 * 776, 1096, torch.float16),
     (8, 6, 330, 8 * 776, 1032, torch.bfloat16),
+    # (few K steps: the costs name the five-stage kernel)
+    (2, 1, 1920, 2 * 752, 264, torch.bfloat16),
+    (4, 3, 512, 4 * 1568, 200, torch.float16),
+    (8, 5, 1000, 8 * 504, 360, torch.bfloat16),
 ]
 
 

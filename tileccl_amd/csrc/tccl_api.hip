@@ -1092,8 +1092,14 @@ tccl::EpilogueReduce build_epilogue_reduce(const tccl::CommArgs& c, const tccl_g
 
 // May a reduce-scatter of column shards run on sub-tiles across the owners?  Where the 128 x 128-tile kernel of one tile per CU
 // would precede a reduction of its own, the peers' partials are there and only this rank's columns are summed.
+// Either kernel of one tile per CU: where the costs name the five-stage one, the two are within a tenth of each other, and the
+// launch that goes is a fifth to a third of the time.  bf16, K = 200 / 360 / 744, before -> after: row-major 1024 x 4096 on two
+// ranks 17.1 / 19.5 / 22.2 -> 12.2 / 13.0 / 16.2 us, on four 16.2 / 17.4 / 21.2 -> 11.8 / 13.0 / 16.2; k-major 1920 x 1504 on two
+// 14.7 / 17.1 / 20.7 -> 11.5 / 12.3 / 17.0, 1920 x 1472 on eight 14.8 / 16.8 / 23.0 -> 13.6 / 15.2 / 19.4.
 bool sums_across(const tccl_gemm_desc* d, const tccl::CommArgs& c, TileKernel kernel, int tiles, int cus) {
-  if (kernel != kTiles128Deep || d->out_dtype != TCCL_F32 || !c.peers_resident || c.emulate_peer || d->column_shards != c.world) return false;
+  const bool named = d->macro_tile != 0 || d->num_wgs > 0 || d->block_m != 128 || d->block_n != 128;  // by the caller
+  if (kernel != kTiles128Deep && (kernel != kTiles128 || tiles > cus || named)) return false;
+  if (d->out_dtype != TCCL_F32 || !c.peers_resident || c.emulate_peer || d->column_shards != c.world) return false;
   if (c.out_dtype != tccl::kF16 && c.out_dtype != tccl::kBF16) return false;
   if (c.ld_rs_out_bytes % 16 || ((uintptr_t)c.rs_out & 15)) return false;
   if (d->K <= 3 * 64) return false;  // the last three K steps are apart, and one goes before them
