@@ -115,6 +115,26 @@ def test_operands_end_below_the_offsets_that_read_as_zero(lib):
         assert (b"spans more than 4 GiB" in lib.tccl_last_error_string()) == refused, lib.tccl_last_error_string()
 
 
+@pytest.mark.parametrize("K,pitch,refused", [(2040, 1052840, True), (2040, 1049088, True), (2040, 1049080, False), (2048, 1049080, False),
+                                             (1, 34100000, True), (1, 1000, False)])
+def test_the_last_step_of_an_a_by_columns_is_within_reach(lib, K, pitch, refused):
+    """The K step that holds the last column ends at a multiple of 64; what it fetches past column K must lie behind the operand, not
+    at its start again (offsets have 32 bits).  (No heap is given: nothing is launched.)"""
+    from tileccl_amd import _lib
+
+    d = _lib.GemmDesc()
+    d.A = d.B = d.C = 0x1000
+    d.in_dtype = d.out_dtype = _lib.BF16
+    d.block_m, d.block_n, d.group_m = 128, 128, 8
+    d.M, d.N, d.K, d.lda, d.ldb, d.ldc = 1000, 2064, -(-K // 8) * 8, pitch, 2064, 2064
+    d.flags = _lib.GEMM_A_COLUMNS | (d.K - K) << _lib.GEMM_A_SHORT_SHIFT | (d.K - K) << _lib.GEMM_B_SHORT_SHIFT
+    assert ((K - 1) * pitch + 1000) * 2 < 2**32 - 16 and refused == ((-(-K // 64) * 64 - 1) * pitch * 2 + 2000 > 2**32 - 16)
+    assert lib.tccl_gemm_allgather(C.byref(d), 0x1000, 2064, None, None, None, _lib.S0_BULK, None) != 0
+    assert (b"spans more than 4 GiB" if refused else b"heap") in lib.tccl_last_error_string(), lib.tccl_last_error_string()
+    if refused:  # and the caller is told to give A by rows
+        assert lib.tccl_gemm_reads_columns(C.byref(d)) == 0
+
+
 @pytest.mark.parametrize("tile_rows,tile_cols,group_m", [(32, 32, 8), (12, 2, 8), (7, 5, 3), (1, 9, 8), (64, 32, 8), (5, 1, 1)])
 def test_device_tile_order_equals_the_reference_swizzle(lib, tile_rows, tile_cols, group_m):
     tm, tn = C.c_int32(), C.c_int32()

@@ -338,10 +338,11 @@ int check_gemm(const tccl_gemm_desc* d, bool ragged_shards = false) {
   // The kernels address an operand with 32-bit byte offsets from a per-tile base: B from its
   // first row down to row K-1 (k-major B: over the 256 columns of a tile), A and C over the 256 rows of a tile.
   // Offsets from 0xfffffff0 on mean "reads as zero" there; A, a k-major B and 16-bit ones are whole 16-byte vectors and never
-  // that long unless they are longer.
+  // that long unless they are longer.  An A by columns has nothing but its end to make the columns of the last K step (of 64) zero,
+  // so these have to be within reach as well: an offset that goes past 2^32 is one of the first columns'.
   const int64_t limit = 0xffffffffll, operand_limit = 0xfffffff0ll;
   const int64_t b_span = (b_kmajor ? 255 * d->ldb + d->K : (int64_t)(d->K - 1) * d->ldb + (int64_t)d->N * shards) * (int64_t)isz;
-  const int64_t a_span = (a_columns ? (int64_t)(d->K - 1) * d->lda + d->M : 255 * d->lda + d->K) * (int64_t)isz;
+  const int64_t a_span = (a_columns ? (((int64_t)d->K + 63) / 64 * 64 - 1) * d->lda + d->M : 255 * d->lda + d->K) * (int64_t)isz;
   const int64_t c_span = (255 * d->ldc + d->N) * (int64_t)osz;
   if (b_span > operand_limit || a_span > operand_limit || c_span > limit)
     return fail(TCCL_ERR_UNSUPPORTED, "gemm: an operand spans more than 4 GiB from a tile's base (B %lld, A %lld, C %lld bytes)",
