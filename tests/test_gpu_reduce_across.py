@@ -81,6 +81,38 @@ def test_sums_are_the_oracles(lib, world, rank, M, N, K, dtype, kmajor, variant)
         assert torch.all(registers[rank] == -7.0)
 
 
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("where", ["A", "B", "behind A"])
+@pytest.mark.parametrize("world,M,K", [(2, 1024, 776), (4, 700, 648)])
+def test_output_in_an_operands_memory(lib, world, M, K, where, kmajor):
+    """A square layer in place: nothing is stored to memory that the product still reads.  The GEMM and the reduction behind it store
+    this rank's partial, the sums in the GEMM's epilogue do not."""
+    dtype, cols = torch.bfloat16, K
+    ctxs = tileccl.init_local(world_size=world, heap_size=128 << 20)
+    try:
+        ctx = ctxs[0]
+        A_cpu, B_cpu = seeded((M, K), 0, dtype), seeded((K, world * cols), 1, dtype, scale=K**-0.5)
+        room = ctx.zeros(2 * M, K, dtype=dtype)
+        A, apart = room[:M], ctx.zeros(M, cols, dtype=dtype)
+        B = ctx.zeros(world * cols, K, dtype=dtype).t() if kmajor else ctx.zeros(K, world * cols, dtype=dtype)
+        part = ctx.workspace("gemm_reducescatter.partial", world, M, cols, dtype=torch.float32)
+        stored = B.t() if kmajor else B
+        out = {"A": A, "B": stored.reshape(-1)[: M * cols].view(M, cols), "behind A": room[M:]}[where]
+        got = []
+        for o in (apart, out):
+            A.copy_(A_cpu)
+            B.copy_(B_cpu)
+            part.fill_(-7.0)
+            tileccl.ops.gemm_reducescatter(A, B, o, ctx=ctx)
+            torch.cuda.synchronize()
+            got.append((bits(o).cpu().clone(), bool(torch.all(part[0] == -7.0))))
+        assert torch.equal(got[0][0], got[1][0])
+        assert got[0][1] and got[1][1] == (where == "behind A")
+    finally:
+        for c in ctxs:
+            c.heap.cleanup()
+
+
 def test_every_plan_tile_is_published_once(lib):
     """The words that the peers of the next launch look at: locks hold the launch's number, counters all tiles of every launch,
     and the arrival words are zero again."""

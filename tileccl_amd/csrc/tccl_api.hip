@@ -1091,6 +1091,11 @@ tccl::EpilogueReduce build_epilogue_reduce(const tccl::CommArgs& c, const tccl_g
   return r;
 }
 
+bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return x < y + (uint64_t)b_bytes && y < x + (uint64_t)a_bytes;
+}
+
 // May a reduce-scatter of column shards run on sub-tiles across the owners?  Where the 128 x 128-tile kernel of one tile per CU
 // would precede a reduction of its own, the peers' partials are there and only this rank's columns are summed.
 // Either kernel of one tile per CU: where the costs name the five-stage one, the two are within a tenth of each other, and the
@@ -1112,6 +1117,12 @@ bool sums_across(const tccl_gemm_desc* d, const tccl::CommArgs& c, TileKernel ke
   const bool pays = kmajor ? (c.world == 2 || c.world == 4 || c.world == 8)
                            : c.world == 2 || (c.world == 4 && d->K <= 2048 && 2 * tiles >= cus);
   if (!pays) return false;
+  // The first sums are stored while other workgroups still read A and B: an output that shares memory with them (a square layer in
+  // place) is written by a launch behind the GEMM.
+  const int64_t rows = d->M / c.world, cols = (int64_t)c.world * d->N, k_rows = d->K - ((d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15);
+  const int64_t out_bytes = (rows - 1) * c.ld_rs_out_bytes + (int64_t)d->N * 2;
+  if (overlap(c.rs_out, out_bytes, d->A, ((rows - 1) * d->lda + d->K) * 2)) return false;
+  if (overlap(c.rs_out, out_bytes, d->B, (kmajor ? (cols - 1) * d->ldb + d->K : (k_rows - 1) * d->ldb + cols) * 2)) return false;
   // 32-bit offsets that now run over all shards.
   const int64_t limit = 0xfffffff0ll;
   return (kmajor ? (int64_t)c.world * d->N : (int64_t)d->K) * d->ldb * 2 <= limit && (int64_t)d->M * d->ldc * 4 <= limit;
