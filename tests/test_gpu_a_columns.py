@@ -76,6 +76,35 @@ def test_all_scatter(lib, M, N, K, schedule):
             c.heap.cleanup()
 
 
+@pytest.mark.parametrize("in_place_first", [False, True])
+def test_all_scatter_into_its_own_input(lib, in_place_first):
+    """``C.t() @ B`` into ``C``, beside the same call on tensors that lie apart: A is read before anything is stored."""
+    import tileccl_amd
+    from tileccl_amd import _launch, ops
+
+    n, dtype = 1040, torch.bfloat16
+    ctxs = tileccl_amd.init_local(world_size=2, heap_size=128 << 20)
+    try:
+        A_cpu, B_cpu = seeded((n, n), 0, dtype), seeded((n, n), 1, dtype, scale=n**-0.5)
+        outs, spare = [c.zeros(n, n, dtype=dtype) for c in ctxs], [c.zeros(n, n, dtype=dtype) for c in ctxs]
+        B = ctxs[0].zeros(n, n, dtype=dtype)
+        B.copy_(B_cpu)
+        assert [_launch._gemm_desc(t.t(), B, outs[0], a_columns=True)[1].pack_a for t in (spare[0], outs[0])] == [False, True]
+        got = []
+        for in_place in (in_place_first, not in_place_first, in_place_first):
+            held = outs[0] if in_place else spare[0]
+            held.copy_(A_cpu.t())
+            ops.gemm_allscatter(held.t(), B, outs[0], ctx=ctxs[0])
+            torch.cuda.synchronize()
+            got.append([bits(o[:, : n // 2]).cpu().clone() for o in outs])
+        for x in got[1:]:
+            assert all(torch.equal(a, b) for a, b in zip(x, got[0]))
+        assert_gemm_close(outs[0], A_cpu.float() @ B_cpu.float())
+    finally:
+        for c in ctxs:
+            c.heap.cleanup()
+
+
 def test_refusals(lib):
     from tileccl_amd import _launch, _lib
 

@@ -132,6 +132,34 @@ def test_descriptors_and_launch_numbers(table, variant, attr):
     assert numbers() == 40 and words.asked == 2
 
 
+def test_an_a_by_columns_lies_apart_from_c(table):
+    """The launch reads it while it stores C: tensors that share memory find no such call (and one that packs A is built for them)."""
+    table, _ = table
+    buf = torch.zeros(4096, dtype=torch.float16)
+    M, N, K, pitch = 8, 16, 24, 32
+    base = buf.data_ptr() + (-buf.data_ptr()) % 16 - buf.data_ptr()
+    at = lambda first, rows, cols, ld: buf.as_strided((rows, cols), (ld, 1), base // 2 + first)
+    a = at(0, K, M, pitch).t()  # 23 * 32 + 8 elements
+    b, c = at(2048, K, N, N), at(1024, M, N, N)
+    gemm = _lib.GemmDesc(M=M, N=N, K=K, lda=pitch, ldb=N, ldc=N, in_dtype=_lib.F16, out_dtype=_lib.F16, flags=_lib.GEMM_A_COLUMNS)
+    seen = []
+
+    @C.CFUNCTYPE(C.c_int, C.POINTER(_lib.GemmDesc), C.c_void_p)
+    def entry(g, stream):
+        seen.append((g[0].A, g[0].C))
+        return 0
+
+    _launch.bind(table, ("columns",), (a, b, c), entry, (gemm,), "columns", gemm=gemm, c=(2, 0))
+    for first, fits in ((1024, True), (0, False), (736, False), (744, True)):
+        out = at(first, M, N, N)
+        assert table.launch(("columns",), None, a, b, out) == (True if fits else None), first
+        assert _launch._apart(a, out) == fits, first
+    moved = at(128, K, M, pitch).t()  # C right before A, and one vector into it
+    assert table.launch(("columns",), None, moved, b, at(0, M, N, N)) is True and _launch._apart(moved, at(0, M, N, N))
+    assert table.launch(("columns",), None, moved, b, at(8, M, N, N)) is None and not _launch._apart(moved, at(8, M, N, N))
+    assert len(seen) == 3
+
+
 @pytest.mark.parametrize("kind", ["sparse", "nested", "jagged", "vmap", "grad", "meta"])
 def test_tensors_without_an_address_find_no_call(table, kind):
     """They throw when asked for one; that is "no call", and an ordinary error where a call is built for them."""

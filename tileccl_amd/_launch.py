@@ -187,6 +187,14 @@ def gemm_operands(A: torch.Tensor, B: torch.Tensor) -> tuple[torch.Tensor, torch
     return A, B, plan.K, plan.lda, plan.ldb, plan.b_flags
 
 
+def _apart(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """No byte from the first to the last element of ``a`` lies among those of ``b``."""
+    (a_first, a_end), (b_first, b_end) = (
+        (t.data_ptr(), t.data_ptr() + (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride()))) * t.element_size()) for t in (a, b)
+    )
+    return a_end <= b_first or b_end <= a_first
+
+
 def _gemm_desc(
     A: torch.Tensor,
     B: torch.Tensor,
@@ -203,7 +211,8 @@ def _gemm_desc(
     a_columns: bool = False,
 ) -> tuple[_lib.GemmDesc, OperandPlan]:
     """The descriptor without its operands' addresses, and how those are to be read.  ``a_columns``: the operation takes an A
-    that is given by columns (a transposed view) where it lies; the kernels that would run decide."""
+    that is given by columns (a transposed view) where it lies, if C lies elsewhere (``C.t() @ B`` into ``C`` takes a copy of A
+    before it stores anything); the kernels that would run decide."""
     if not (A.is_cuda and B.is_cuda and C_out.is_cuda):
         raise ValueError("GEMM operands must be device tensors")
     if A.dtype != B.dtype:
@@ -230,7 +239,7 @@ def _gemm_desc(
     d.macro_tile = int(macro_tile)
     d.flags = int(flags) | plan.b_flags
     d.column_shards = int(column_shards)
-    if a_columns and plan.pack_a and not plan.pack_b and M > 1 and A.stride(0) == 1:
+    if a_columns and plan.pack_a and not plan.pack_b and M > 1 and A.stride(0) == 1 and _apart(A, C_out):
         pitch = int(A.stride(1)) if K > 1 else int(M)
         if pitch >= M and _rows_vectorised(A, pitch):
             kept = d.lda, d.flags, d.A, d.B

@@ -78,6 +78,7 @@ struct Call {
   bool has_gemm, has_sync;
   int c_tensor;          // tensor whose address plus c_offset is the GEMM's C (< 0: C is fixed)
   int64_t c_offset;
+  int64_t a_bytes, c_bytes;  // of an A that the GEMM reads by columns (0: it does not) and of its C: they must lie apart
   int64_t heap_lo, heap_size;  // the tensors in `on_heap` (a bit mask) must start in this range
   uint32_t on_heap;
   std::vector<int64_t>* bases;  // per tensor: all must lie at one offset from these
@@ -259,6 +260,11 @@ int call_init_checked(Call* self, PyObject* pos, PyObject* kw) {
   if ((gemm && n < 2) || (c != Py_None && !tensor_index(self->c_tensor))) {
     PyErr_SetString(PyExc_ValueError, "a GEMM's operands are the first two tensors of the Call");
     return -1;
+  }
+  if (gemm && (self->gemm.flags & TCCL_GEMM_A_COLUMNS)) {
+    const tccl_gemm_desc& d = self->gemm;
+    self->a_bytes = ((int64_t)(d.K - 1 - ((d.flags >> TCCL_GEMM_A_SHORT_SHIFT) & 15)) * d.lda + d.M) * 2;
+    self->c_bytes = ((int64_t)(d.M - 1) * d.ldc + d.N) * (d.out_dtype == TCCL_F32 ? 4 : 2);
   }
   if (heap != Py_None) {
     long long lo = 0, size = 0;
@@ -447,6 +453,10 @@ bool fits(const Call* c, PyObject* const* tensors, const int64_t* at, Py_ssize_t
       if (i == 0) offset = from_base;
       if (from_base != offset) return false;
     }
+  }
+  if (c->a_bytes) {
+    const int64_t out = c->c_tensor >= 0 ? at[c->c_tensor] + c->c_offset : (int64_t)(uintptr_t)c->gemm.C;
+    if (at[0] < out + c->c_bytes && out < at[0] + c->a_bytes) return false;
   }
   return true;
 }
