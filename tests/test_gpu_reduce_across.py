@@ -81,6 +81,22 @@ def test_sums_are_the_oracles(lib, world, rank, M, N, K, dtype, kmajor, variant)
         assert torch.all(registers[rank] == -7.0)
 
 
+@pytest.mark.parametrize("world,rank,M,N,K,kmajor", [(2, 1, 1000, 2 * 904, 1032, False), (4, 3, 700, 4 * 712, 1032, True), (2, 0, 1024, 2 * 776, 1160, False),
+                                                     (2, 1, 24, 2 * 512, 512, True)])
+def test_the_bulk_schedule_stores_every_partial(lib, world, rank, M, N, K, kmajor):
+    """Whatever the shards' rows and kernel: the flag that keeps this rank's block in registers is one of the fused schedules."""
+    got = {}
+    for variant, own in (("s0", False), ("s0", True), ("s1", True), ("s2", True)):
+        got[variant, own] = reduce(world, rank, M, N, K, torch.bfloat16, kmajor, variant, own)[:2]
+    out, partial = got["s0", False]
+    for kept, registers in got.values():
+        assert torch.equal(bits(kept), bits(out))
+    assert torch.equal(got["s0", True][1], partial)
+    others = [q for q in range(world) if q != rank]
+    for variant in ("s1", "s2"):
+        assert torch.equal(got[variant, True][1][others], partial[others]) and torch.all(got[variant, True][1][rank] == -7.0)
+
+
 @pytest.mark.parametrize("kmajor", [False, True])
 @pytest.mark.parametrize("where", ["A", "B", "behind A"])
 @pytest.mark.parametrize("world,M,K", [(2, 1024, 776), (4, 700, 648)])

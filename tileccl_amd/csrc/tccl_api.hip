@@ -2242,8 +2242,11 @@ int tccl_gemm_reducescatter(const tccl_gemm_desc* d, void* out, int32_t out_dtyp
   const bool ragged = d->column_shards > 1 && d->column_shards == heap->world_size && d->M % heap->world_size == 0 && shard % d->block_m;
   if (d->flags & TCCL_GEMM_A_COLUMNS) return fail(TCCL_ERR_UNSUPPORTED, "reducescatter: A given by columns");
   if (!ragged && (rc = check_sync(sync, variant))) return rc;
-  if (ragged)
-    return reduce_ragged_shards(d, out, out_dtype, ld_out, heap, sync, tr, emulate_peer, (hipStream_t)stream);
+  if (ragged) {
+    tccl_gemm_desc own = *d;
+    if (variant == TCCL_S0_BULK) own.flags &= ~TCCL_GEMM_OWN_ROWS_IN_REGISTERS;  // S0 stores every partial
+    return reduce_ragged_shards(&own, out, out_dtype, ld_out, heap, sync, tr, emulate_peer, (hipStream_t)stream);
+  }
   if (d->M % heap->world_size || shard % d->block_m)
     return fail(TCCL_ERR_INVALID, "reducescatter: M=%d must split into world_size=%d shards of whole %d-row plan tiles", d->M, heap->world_size, d->block_m);
   tccl_device_info dev;
