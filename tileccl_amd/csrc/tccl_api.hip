@@ -94,7 +94,9 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // One launch holds both roles: workgroups [0, num_compute) run the GEMM, the rest move
 // data.  Three waves per SIMD (two GEMM workgroups plus one communication workgroup per
 // CU) bounds the register budget.
-template <typename InT, typename OutT>
+// kAColumns, here and below: A is given by columns.  Kernels of their own: the loop for it beside the others takes registers from
+// them (10 here, 24 in the deep form; wide form, 1500 x 2240 x 1000 for eight ranks: 28.3 us with it, 28.0 without).
+template <typename InT, typename OutT, bool kAColumns>
 __global__ __launch_bounds__(256, 3) void fused_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::CommArgs c, tccl::PushArgs push,
                                                        int num_compute, int64_t* trace_start) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(256, 3) void fused_kernel(tccl::GemmArgs g, tccl::S
     if (trace_start && blockIdx.x == 0 && threadIdx.x == 0) *trace_start = tccl::now_ticks();
     tccl::EpilogueReduce none;
     none.active = 0;
-    tccl::GemmRole<InT, OutT>(g, push, none, stage0, stage1, stage2).run(s, (int)blockIdx.x, num_compute);
+    tccl::GemmRole<InT, OutT>(g, push, none, stage0, stage1, stage2).template run<false, kAColumns>(s, (int)blockIdx.x, num_compute);
   } else {
     tccl::comm_role(c, (int)blockIdx.x - num_compute, (int)gridDim.x - num_compute, (int*)stage0);
   }
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(256, 3) void fused_kernel(tccl::GemmArgs g, tccl::S
 // (kReduce).  Nothing has to fit beside two of them on a CU, so they take five stages (80 KiB): a load then has three
 // steps and a half to arrive instead of one and a half.  1000 x 2064 x 1008 with its push: 18.3 us with three stages,
 // 16.4 with five (traced).
-template <typename InT, typename OutT, bool kReduce>
+template <typename InT, typename OutT, bool kReduce, bool kAColumns>
 __global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::PushArgs push, tccl::EpilogueReduce reduce) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) char stage0[tccl::kStage128];
@@ -124,7 +126,8 @@ __global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g, tccl:
   __shared__ __attribute__((aligned(1024))) char stage2[tccl::kStage128];
   __shared__ __attribute__((aligned(1024))) char stage3[tccl::kStage128];
   __shared__ __attribute__((aligned(1024))) char stage4[tccl::kStage128];
-  tccl::GemmRole<InT, OutT, 5>(g, push, reduce, stage0, stage1, stage2, stage3, stage4).template run<kReduce>(s, (int)blockIdx.x, (int)gridDim.x);
+  tccl::GemmRole<InT, OutT, 5> role(g, push, reduce, stage0, stage1, stage2, stage3, stage4);
+  role.template run<kReduce, kAColumns>(s, (int)blockIdx.x, (int)gridDim.x);
 #endif
 }
 
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(256, 2) void gemm128_kernel(tccl::GemmArgs g, tccl:
 // half the barriers, and 128-byte pieces of the rows of A (of a k-major B), which cost less where rows start off a
 // 64-byte boundary.  bf16, row-major / k-major B: 2573 x 968 x 3520 41.7 / 42.0 -> 34.3 / 31.8 us, 370 x 5280 x 1656
 // 23.0 / 27.6 -> 21.1 / 22.7, 512 x 7168 x 2944 33.7 / 34.2 -> 29.0 / 28.2.
-template <typename InT, typename OutT>
+template <typename InT, typename OutT, bool kAColumns>
 __global__ __launch_bounds__(256, 1) void gemm128_deep_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::PushArgs push) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) char stage0[tccl::kStageDeep];
@@ -141,7 +144,8 @@ __global__ __launch_bounds__(256, 1) void gemm128_deep_kernel(tccl::GemmArgs g, 
   __shared__ __attribute__((aligned(1024))) char stage3[tccl::kStageDeep];
   tccl::EpilogueReduce none;
   none.active = 0;
-  tccl::GemmRole<InT, OutT, 4, 4, 2>(g, push, none, stage0, stage1, stage2, stage3).run(s, (int)blockIdx.x, (int)gridDim.x);
+  tccl::GemmRole<InT, OutT, 4, 4, 2> role(g, push, none, stage0, stage1, stage2, stage3);
+  role.template run<false, kAColumns>(s, (int)blockIdx.x, (int)gridDim.x);
 #endif
 }
 
@@ -171,7 +175,7 @@ __global__ __launch_bounds__(256, 1) void gemm_across_kernel(tccl::GemmArgs g, t
 // than two 128 x 128 workgroups on a CU, and half as many tiles to share out.  bf16, row-major / k-major B, against
 // those two: 6854 x 520 x 2248 51.2 / 61.0 -> 32.1 / 37.7 us, 534 x 7088 x 2960 60.0 / 72.8 -> 38.8 / 45.7, 1956 x
 // 2784 x 2096 43.2 / 51.9 -> 31.2 / 35.7, 1061 x 4432 x 1088 24.5 / 24.0 -> 19.1 / 18.1.
-template <typename InT, typename OutT>
+template <typename InT, typename OutT, bool kAColumns>
 __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::PushArgs push) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) char stage0[tccl::kStageWide];
@@ -179,7 +183,8 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(tccl::GemmArgs g, tcc
   __shared__ __attribute__((aligned(1024))) char stage2[tccl::kStageWide];
   tccl::EpilogueReduce none;
   none.active = 0;
-  tccl::GemmRole<InT, OutT, 3, 8, 2>(g, push, none, stage0, stage1, stage2).run(s, (int)blockIdx.x, (int)gridDim.x);
+  tccl::GemmRole<InT, OutT, 3, 8, 2> role(g, push, none, stage0, stage1, stage2);
+  role.template run<false, kAColumns>(s, (int)blockIdx.x, (int)gridDim.x);
 #endif
 }
 
@@ -388,8 +393,6 @@ int build_gemm_args(const tccl_gemm_desc* d, const tccl_device_info& dev, tccl::
   g->ragged = 0;
   g->b_kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) ? 1 : 0;
   g->b_short = (d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15;
-  g->a_columns = (d->flags & TCCL_GEMM_A_COLUMNS) ? 1 : 0;
-  g->a_short = (d->flags >> TCCL_GEMM_A_SHORT_SHIFT) & 15;
   return 0;
 }
 
@@ -483,26 +486,35 @@ int check_sync(const tccl_sync_desc* s, int variant) {
 // same bits.
 enum TileKernel { kTiles128, kTiles128Deep, kTilesWide, kTiles256 };
 
-template <typename InT, typename OutT>
-int launch_fused_t(tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::CommArgs& c, const tccl::PushArgs& push,
-                   const tccl::EpilogueReduce& reduce, TileKernel kernel, int compute, int comm, int64_t* trace_start, hipStream_t stream) {
+template <typename InT, typename OutT, bool kAColumns>
+void launch_tiles(const tccl::GemmArgs& g, const tccl::SignalArgs& s, const tccl::CommArgs& c, const tccl::PushArgs& push,
+                  const tccl::EpilogueReduce& reduce, TileKernel kernel, int compute, int comm, int64_t* trace_start, hipStream_t stream) {
   const dim3 block(tccl::kThreads);
-  if (reduce.active)
-    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, true>), dim3(compute), block, 0, stream, g, s, push, reduce);
-  else if (comm > 0 || trace_start)
-    hipLaunchKernelGGL((fused_kernel<InT, OutT>), dim3(compute + comm), block, 0, stream, g, s, c, push, compute, trace_start);
+  if (comm > 0 || trace_start)
+    hipLaunchKernelGGL((fused_kernel<InT, OutT, kAColumns>), dim3(compute + comm), block, 0, stream, g, s, c, push, compute, trace_start);
   else if (kernel == kTilesWide)
-    hipLaunchKernelGGL((gemm_wide_kernel<InT, OutT>), dim3(compute), dim3(tccl::kThreadsWide), 0, stream, g, s, push);
+    hipLaunchKernelGGL((gemm_wide_kernel<InT, OutT, kAColumns>), dim3(compute), dim3(tccl::kThreadsWide), 0, stream, g, s, push);
   else if (kernel == kTiles128Deep)
-    hipLaunchKernelGGL((gemm128_deep_kernel<InT, OutT>), dim3(compute), block, 0, stream, g, s, push);
+    hipLaunchKernelGGL((gemm128_deep_kernel<InT, OutT, kAColumns>), dim3(compute), block, 0, stream, g, s, push);
   else
-    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, false>), dim3(compute), block, 0, stream, g, s, push, reduce);
+    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, false, kAColumns>), dim3(compute), block, 0, stream, g, s, push, reduce);
+}
+
+template <typename InT, typename OutT>
+int launch_fused_t(const tccl::GemmArgs& g, bool a_columns, const tccl::SignalArgs& s, const tccl::CommArgs& c, const tccl::PushArgs& push,
+                   const tccl::EpilogueReduce& reduce, TileKernel kernel, int compute, int comm, int64_t* trace_start, hipStream_t stream) {
+  if (reduce.active)  // (A by rows: tccl_gemm_reducescatter)
+    hipLaunchKernelGGL((gemm128_kernel<InT, OutT, true, false>), dim3(compute), dim3(tccl::kThreads), 0, stream, g, s, push, reduce);
+  else if (a_columns)
+    launch_tiles<InT, OutT, true>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  else
+    launch_tiles<InT, OutT, false>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
   TCCL_HIP(hipGetLastError());
   return 0;
 }
 
 // `compute` workgroups for the tiles of 128 x 128; the other kernels take what is left of them.
-int launch_fused(int in_dtype, int out_dtype, const tccl::GemmArgs& gemm, const tccl::SignalArgs& s, const tccl::CommArgs& c,
+int launch_fused(const tccl_gemm_desc* d, const tccl::GemmArgs& gemm, const tccl::SignalArgs& s, const tccl::CommArgs& c,
                  TileKernel kernel, int compute, int comm, int64_t* trace_start, hipStream_t stream, const tccl::PushArgs* push_args = nullptr,
                  const tccl::EpilogueReduce* reduce_args = nullptr) {
   tccl::PushArgs push;
@@ -517,10 +529,13 @@ int launch_fused(int in_dtype, int out_dtype, const tccl::GemmArgs& gemm, const 
     if (compute > total) compute = total;
     g.span = gemm_span(compute, g.group_m, g.xcds);
   }
-  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F16) return launch_fused_t<_Float16, _Float16>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F32) return launch_fused_t<_Float16, float>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_BF16) return launch_fused_t<__bf16, __bf16>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
-  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_F32) return launch_fused_t<__bf16, float>(g, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  const bool a_columns = (d->flags & TCCL_GEMM_A_COLUMNS) != 0;
+  if (a_columns) g.a_short = (d->flags >> TCCL_GEMM_A_SHORT_SHIFT) & 15;
+  const int in_dtype = d->in_dtype, out_dtype = d->out_dtype;
+  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F16) return launch_fused_t<_Float16, _Float16>(g, a_columns, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_F16 && out_dtype == TCCL_F32) return launch_fused_t<_Float16, float>(g, a_columns, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_BF16) return launch_fused_t<__bf16, __bf16>(g, a_columns, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
+  if (in_dtype == TCCL_BF16 && out_dtype == TCCL_F32) return launch_fused_t<__bf16, float>(g, a_columns, s, c, push, reduce, kernel, compute, comm, trace_start, stream);
   return fail(TCCL_ERR_UNSUPPORTED, "gemm: no kernel for in_dtype=%d, out_dtype=%d", in_dtype, out_dtype);
 }
 
@@ -1330,7 +1345,7 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   if (variant == TCCL_S0_BULK) {
     tccl::CommArgs none;
     memset(&none, 0, sizeof none);
-    int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, none, kernel, compute, 0, trace_start, stream);
+    int rc = launch_fused(d, g, s, none, kernel, compute, 0, trace_start, stream);
     if (rc) return rc;
     if (c.world <= 1 && c.op != tccl::kOpReduceScatter) return 0;
     return launch_bulk(c, dev, stream);
@@ -1357,19 +1372,19 @@ int run_variant(const tccl_gemm_desc* d, tccl::CommArgs& c, const tccl_sync_desc
   // 1024 27.0 / 28.3; 2048 x 1408 x 1280 29.0 / 28.1, 1792 x 1200 x 1520 31.4 / 30.5, 1280 x 3136 x 3968 51.7 / 49.4).
   if (keeps_own || (apart && !c.peers_resident && c.world == 2 && compute <= dev.compute_units && kernel != kTilesWide && d->K <= 1024)) {
     const tccl::EpilogueReduce r = build_epilogue_reduce(c, d);
-    return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);
+    return launch_fused(d, g, s, c, kTiles128, compute, 0, nullptr, stream, nullptr, &r);
   }
   if (apart && arrival_words(d, sync) && sums_across(d, c, kernel, total_tiles, dev.compute_units))
     return launch_across(d, g, s, c, arrival_words(d, sync), stream);
   if (apart) {
-    const int rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, kernel, compute, 0, nullptr, stream);
+    const int rc = launch_fused(d, g, s, c, kernel, compute, 0, nullptr, stream);
     return rc ? rc : sums_apart();
   }
   if (!traced && build_push(c, g, &push)) {
     c.directions &= ~tccl::kDirPush;
     if (c.op != tccl::kOpReduceScatter && !(c.directions & tccl::kDirPull)) comm = 0;
   }
-  return launch_fused(d->in_dtype, d->out_dtype, g, s, c, kernel, compute, comm, trace_start, stream, &push);
+  return launch_fused(d, g, s, c, kernel, compute, comm, trace_start, stream, &push);
 }
 
 
@@ -1651,7 +1666,7 @@ int tccl_gemm(const tccl_gemm_desc* d, void* stream) {
   }
   tccl::CommArgs none;
   memset(&none, 0, sizeof none);
-  return launch_fused(d->in_dtype, d->out_dtype, g, s, none, kernel, tile_wgs(kernel, d, dev, g.tile_rows * g.tile_cols), 0, nullptr,
+  return launch_fused(d, g, s, none, kernel, tile_wgs(kernel, d, dev, g.tile_rows * g.tile_cols), 0, nullptr,
                       (hipStream_t)stream);
 }
 
@@ -2216,7 +2231,7 @@ static int reduce_ragged_shards(const tccl_gemm_desc* d, void* out, int32_t out_
     tccl::SignalArgs s;
     memset(&s, 0, sizeof s);
     if (sums_across(d, c, together.kernel, g.tile_rows * g.tile_cols, dev.compute_units)) return launch_across(d, g, s, c, nullptr, stream);
-    rc = launch_fused(d->in_dtype, d->out_dtype, g, s, c, together.kernel, tile_wgs(together.kernel, d, dev, g.tile_rows * g.tile_cols), 0,
+    rc = launch_fused(d, g, s, c, together.kernel, tile_wgs(together.kernel, d, dev, g.tile_rows * g.tile_cols), 0,
                       nullptr, stream);
     return rc ? rc : launch_bulk(c, dev, stream);
   }

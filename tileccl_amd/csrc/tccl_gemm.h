@@ -22,7 +22,7 @@
 //   side, by the choice of the chunk a lane fetches.  Rows >= M, columns >= N and k >= K read as
 //   zero through the buffer bounds (A chunks at k >= K are redirected past the buffer's end).
 //   A k-major B (GemmArgs::b_kmajor: element (k, n) at B[n * ldb + k]) takes A's route and layout.
-//   A given by columns (GemmArgs::a_columns: element (m, k) at A[k * lda + m]; the input of a weight gradient) takes a
+//   A given by columns (kAColumns: element (m, k) at A[k * lda + m]; the input of a weight gradient) takes a
 //   row-major B's, 128 rows wide: its operands come out through the transposing reads as well.  1000 x 2064 x 1003 pushed to one
 //   peer: 15.5 us, and 21.6 where a launch of its own turns A into rows first.
 //
@@ -81,12 +81,16 @@ struct GemmArgs {
   int wrap_rows;
   // The row blocks are no whole tiles: each starts a tile row of its own (tile_rows counts them all).
   int ragged;
-  // B is k-major: element (k, n) at B[n * ldb + k] (the `.t()` view of an (N, K) tensor).
-  int b_kmajor;
+  union {
+    // B is k-major: element (k, n) at B[n * ldb + k] (the `.t()` view of an (N, K) tensor).
+    int b_kmajor;
+    // Kernels for an A given by columns (element (m, k) at A[k * lda + m]; B is row-major): of the K columns it lacks the last
+    // a_short, which read as zero.  (No word of its own: with more fields here the compiler laid out the large-tile
+    // kernels, which read none of them, another way; 4096 x 4096 x 1024 gathered by rows 45.7 -> 46.4 us.)
+    int a_short;
+  };
   // Row-major B lacks its last b_short of the K rows: they read as zero (A is zero there as well).
   int b_short;
-  // A is given by columns: element (m, k) at A[k * lda + m]; of the K columns it lacks the last a_short, which read as zero.
-  int a_columns, a_short;
 };
 
 // Where a tile whose first output row is row0 and first output column col0 reads its operands.
@@ -887,7 +891,7 @@ struct GemmRole {
   // ---- persistent loop over plan tiles ----------------------------------------------------------
   // A workgroup takes a plan tile at a time, as sub-tiles; in the wide form, where one is narrower than a sub-tile, the
   // one on its right with it.
-  template <bool kReduce = false>
+  template <bool kReduce = false, bool kAColumns = false>
   TCCL_D void run(const SignalArgs& s, int wg, int num_wgs) const {
     const int per = kWn == 4 ? kCols / g.block_n : 1;  // plan tiles across
     const int cols = kWn == 4 ? (g.tile_cols + per - 1) / per : g.tile_cols;
@@ -910,11 +914,12 @@ struct GemmRole {
         for (int sn = 0; sn < per * g.block_n; sn += kCols) {
           const int row0 = first_row + sm, col0 = tc.n * g.block_n + sn;
           if (row0 >= row_end || col0 >= g.N) continue;
-          if (!kReduce && g.a_columns) {  // (with a row-major B: check_gemm)
+          if constexpr (kAColumns) {  // (with a row-major B: check_gemm)
+            static_assert(!kReduce, "an A given by columns is not reduced");
             if (s.mode == kSignalNone)
-              subtile<0, false, false, !kReduce>(row0, row_end, col0, tile_id, s);
+              subtile<0, false, false, true>(row0, row_end, col0, tile_id, s);
             else
-              subtile<kCoherent, false, false, !kReduce>(row0, row_end, col0, tile_id, s);
+              subtile<kCoherent, false, false, true>(row0, row_end, col0, tile_id, s);
           } else if (s.mode == kSignalNone) {
             if (g.b_kmajor)
               subtile<0, true, kReduce>(row0, row_end, col0, tile_id, s);
