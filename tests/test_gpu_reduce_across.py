@@ -14,7 +14,7 @@ from tests.gpu_util import assert_gemm_close, bits, seeded
 pytestmark = pytest.mark.gpu
 
 
-def reduce(world, rank, M, N, K, dtype, kmajor, variant, own, launches=1):
+def reduce(world, rank, M, N, K, dtype, kmajor, variant, own, launches=1, spoil=None):
     """(out, this rank's partial as (world, M, N / world), A @ B, the peers' partials) after `launches` launches."""
     ctxs = tileccl.init_local(world_size=world, heap_size=128 << 20)
     try:
@@ -31,6 +31,8 @@ def reduce(world, rank, M, N, K, dtype, kmajor, variant, own, launches=1):
             part.fill_(-7.0)
             if p != rank:
                 peers[p] = seeded((world, M, N // world), 10 + p, torch.float32) * 1000.0
+                if spoil is not None:
+                    spoil(p, peers[p])
                 part.copy_(peers[p])
         got = []
         for _ in range(launches):
@@ -79,6 +81,27 @@ def test_sums_are_the_oracles(lib, world, rank, M, N, K, dtype, kmajor, variant)
     assert torch.equal(registers[others], partial[others])
     if kmajor or world < 8:  # (a row-major B on eight ranks keeps the reduction of its own, which reads a stored partial)
         assert torch.all(registers[rank] == -7.0)
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("world,rank,M,N,K,dtype", [SHAPES[1], SHAPES[2], SHAPES[4], SHAPES[6], SHAPES[7]])
+def test_only_this_ranks_block_is_added(lib, world, rank, M, N, K, dtype, kmajor):
+    """Infinities and NaN in this rank's block of the peers' partials come out as the oracle's sums; those of the other blocks,
+    right before and behind it, are never read."""
+
+    def spoil(p, partial):
+        partial[[q for q in range(world) if q != rank]] = float("nan")
+        partial[rank, p % M, ::3] = float("inf")
+        partial[rank, (7 * p + 64) % M, 1::3] = float("-inf")
+        partial[rank, -1, p::9] = float("nan")
+        partial[rank, -1, -1 - p] = float("-inf")
+
+    out, partial, _, peers = reduce(world, rank, M, N, K, dtype, kmajor, "s2", own=False, spoil=spoil)
+    want = oracle.reduce_rows([(partial if p == rank else peers[p]).reshape(world * M, N // world) for p in range(world)], rank, dtype)
+    assert torch.equal(out.isnan(), want.isnan()) and 0 < int(out.isnan().sum()) < out.numel() // 8
+    assert torch.equal(bits(out)[~out.isnan()], bits(want)[~want.isnan()])
+    kept, _, _, _ = reduce(world, rank, M, N, K, dtype, kmajor, "s1", own=True, spoil=spoil)
+    assert torch.equal(kept.isnan(), want.isnan()) and torch.equal(bits(kept)[~kept.isnan()], bits(want)[~want.isnan()])
 
 
 @pytest.mark.parametrize("world,rank,M,N,K,kmajor", [(2, 1, 1000, 2 * 904, 1032, False), (4, 3, 700, 4 * 712, 1032, True), (2, 0, 1024, 2 * 776, 1160, False),

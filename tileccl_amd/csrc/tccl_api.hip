@@ -154,9 +154,9 @@ __global__ __launch_bounds__(256, 1) void gemm128_deep_kernel(tccl::GemmArgs g, 
 // addends each, 36 us where a reduction of its own behind the GEMM takes 29), and that reduction waits for the whole GEMM, a
 // launch and the memory's first answer.  So a sub-tile takes a run of every owner's columns: each CU has 1 / world of its sums
 // to make, asks for their addends three K steps before its product is done, and publishes its part of `world` plan tiles.
-// bf16, GEMM and reduction before, this after: k-major B 1024 x 4096 x 2048 on 2 / 4 / 8 ranks 30.9 / 30.2 / 30.1 -> 25.1 / 25.1
-// / 26.7 us, 512 x 8192 x 1024 22.3 / 22.0 / 22.1 -> 16.7 / 17.7 / 19.3; row-major 1024 x 4096 x 2048 on 2 / 4 31.6 / 30.2 ->
-// 26.7 / 27.5, 512 x 8192 x 1024 22.5 / 22.2 -> 17.6 / 19.3.  What bounds it is the operands' way from L2, as in the deep form.
+// bf16, GEMM and reduction before, this after: k-major B 1024 x 4096 x 2048 on 2 / 4 / 8 ranks 31.3 / 30.5 / 30.7 -> 25.6 / 24.7
+// / 26.5 us, 512 x 8192 x 1024 23.1 / 22.6 / 22.3 -> 16.8 / 17.1 / 18.8; row-major 1024 x 4096 x 2048 on 2 / 4 31.7 / 30.7 ->
+// 26.1 / 27.8, 512 x 8192 x 1024 22.8 / 22.5 -> 17.3 / 19.2.  What bounds it is the operands' way from L2, as in the deep form.
 template <typename InT, int kWorld, bool kBKMajor>
 __global__ __launch_bounds__(256, 1) void gemm_across_kernel(tccl::GemmArgs g, tccl::SignalArgs s, tccl::EpilogueReduce reduce) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1115,8 +1115,8 @@ bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
 // would precede a reduction of its own, the peers' partials are there and only this rank's columns are summed.
 // Either kernel of one tile per CU: where the costs name the five-stage one, the two are within a tenth of each other, and the
 // launch that goes is a fifth to a third of the time.  bf16, K = 200 / 360 / 744, before -> after: row-major 1024 x 4096 on two
-// ranks 17.1 / 19.5 / 22.2 -> 12.2 / 13.0 / 16.2 us, on four 16.2 / 17.4 / 21.2 -> 11.8 / 13.0 / 16.2; k-major 1920 x 1504 on two
-// 14.7 / 17.1 / 20.7 -> 11.5 / 12.3 / 17.0, 1920 x 1472 on eight 14.8 / 16.8 / 23.0 -> 13.6 / 15.2 / 19.4.
+// ranks 17.0 / 19.4 / 22.0 -> 11.7 / 12.9 / 15.8 us, on four 16.1 / 17.0 / 20.1 -> 11.5 / 12.5 / 15.8; k-major 1920 x 1504 on two
+// 15.1 / 17.4 / 20.7 -> 11.1 / 12.1 / 16.7, 1920 x 1472 on eight 14.7 / 16.6 / 22.6 -> 12.5 / 13.8 / 18.4.
 bool sums_across(const tccl_gemm_desc* d, const tccl::CommArgs& c, TileKernel kernel, int tiles, int cus) {
   const bool named = d->macro_tile != 0 || d->num_wgs > 0 || d->block_m != 128 || d->block_n != 128;  // by the caller
   if (kernel != kTiles128Deep && (kernel != kTiles128 || tiles > cus || named)) return false;

@@ -47,6 +47,8 @@
 // written (gemm.py:163-167); the K tail is zero-filled (gemm.py:153-160).
 #pragma once
 
+#include <type_traits>
+
 #include "tccl_comm.h"
 #include "tccl_device.h"
 
@@ -448,10 +450,8 @@ struct GemmRole {
       if (last && kLeft > 0) {
         if (kLeft == 1) {
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        } else if (sums_here()) {
-          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kLeft == 3 ? kLoads : 0) + kAddends) : "memory");
         } else {
-          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kLeft == 3 ? kLoads : 0) : "memory");
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kLeft == 3 ? kLoads : 0) + kAddends) : "memory");
         }
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -641,22 +641,34 @@ struct GemmRole {
   // This lane's chunk of round r: row of the slab, column of the run.
   static TCCL_D int own_row(int ln, int r) { return (ln + 64 * r) / kOwnChunks; }
   TCCL_D int own_col(int ln) const { return (kSpread ? wn * kOwnCols : 0) + ln % kOwnChunks * 4; }  // (64 is a multiple of kOwnChunks)
+  // Every wavefront issues the same loads, so that the waits behind them count the same everywhere; where there is nothing to sum they
+  // fetch nothing.  (Under a branch the compiler waits for all of them before the next step's first operand.)  The peers' bases
+  // come through scalar loads: a vector load's answer is waited for together with the operands under way, and each addend's
+  // descriptor has to be made uniform first.  bf16 1000 x 4032 x 256 / 1024 x 4096 x 1000 k-major on eight ranks 13.7 / 21.4 -> 12.5 / 20.2
+  // us, 512 x 4096 x 1000 on four 16.0 -> 15.1, 1500 x 2208 x 2048 on two 23.8 -> 23.0.
+  // Where every wavefront sums (row-major, four ranks) the branch is none and the vector loads stay: without them the compiler moves
+  // operands between register files in the K loop (1920 x 2048 x 904 20.6, 20.9 us with scalar ones).
   TCCL_D void request_sums(int row0, int col0, Addends& w) const {
-    if (!sums_here()) return;
     const int ln = (int)((uint32_t)fresh(lane) & 63u), rows = g.wrap_rows - row0, col = own_col(ln);
-    const bool live = col < g.N - col0;
+    const bool live = sums_here() && col < g.N - col0;
     const int64_t first = (int64_t)(uintptr_t)((const float*)g.C + ((int64_t)reduce.rank * g.wrap_rows + row0) * g.ldc + col0);
     const uint32_t pitch = (uint32_t)(g.ldc * 4);
+    // A window ends with this rank's block (below 0xfffffff0: sums_across()), so that the offset of what does not exist is past it.
+    const uint32_t end = kSpread ? 0xffffffffu : (uint32_t)(rows - 1) * pitch + (uint32_t)(g.N - col0) * 4u;
+    const uint32_t nowhere = kSpread ? 0u : 0xfffffff0u;  // (kSpread: the first chunk instead, inside every window)
+    typedef typename std::conditional<kSpread, const int64_t*, const __attribute__((address_space(4))) int64_t*>::type Bases;
+    const Bases bases = (Bases)reduce.heap_bases;
 #pragma unroll
     for (int n = 0; n < kWorld - 1; ++n) {
       const int p = n + (n >= reduce.rank);
-      const __amdgpu_buffer_rsrc_t from = window(first + (reduce.heap_bases[p] - reduce.heap_bases[reduce.rank]));
+      const __amdgpu_buffer_rsrc_t from =
+          __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(first + (bases[p] - bases[reduce.rank])), 0, end, 0x00020000);
 #pragma unroll
       for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
-        for (int r = 0; r < kOwnRounds; ++r) {  // (a chunk that does not exist: the first one instead)
+        for (int r = 0; r < kOwnRounds; ++r) {
           const uint32_t row = wm * 64 + bi * 32 + own_row(ln, r);
-          w.v[bi][r][n] = __builtin_bit_cast(f32x4, ld16<kCoherent>(from, live && (int)row < rows ? row * pitch + col * 4 : 0u));
+          w.v[bi][r][n] = __builtin_bit_cast(f32x4, ld16<kCoherent>(from, live && (int)row < rows ? row * pitch + col * 4 : nowhere));
         }
     }
   }
