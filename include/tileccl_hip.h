@@ -101,7 +101,7 @@ typedef struct tccl_gemm_desc {
 /* tccl_gemm_reducescatter, variants S1 / S2 where the sums are made in the GEMM's epilogue: shards of whole 256 x 256
  * tiles; small outputs with TCCL_GEMM_ARRIVALS or of ragged column shards; 128 x 128 tiles that wait for their peers, at most
  * one per CU; and 16-bit inputs as column shards with TCCL_RS_PEERS_RESIDENT (TCCL_GEMM_ARRIVALS too where the shards are whole plan tiles),
- * fp32 partials and a 16-bit `out` that has 16-byte rows and shares no memory with A or B, on 2, 4 or 8 ranks, K > 192, where 128 x 128
+ * fp32 partials and a 16-bit `out` that has 16-byte rows and shares no memory with A, B or C, on 2, 4 or 8 ranks, K > 192, where 128 x 128
  * tiles named by nobody are at most one per CU (a row-major B: two ranks, or four up to K = 2048 with half the CUs at
  * work).  Elsewhere the sums are a launch of their own and every partial is stored; a caller who reads these rows of C leaves the flag out.
  * the partial of the rows this rank owns stays in the accumulators, takes the peers' partials

@@ -121,11 +121,11 @@ def test_the_bulk_schedule_stores_every_partial(lib, world, rank, M, N, K, kmajo
 
 
 @pytest.mark.parametrize("kmajor", [False, True])
-@pytest.mark.parametrize("where", ["A", "B", "behind A"])
+@pytest.mark.parametrize("where", ["A", "B", "behind A", "C"])
 @pytest.mark.parametrize("world,M,K", [(2, 1024, 776), (4, 700, 648)])
 def test_output_in_an_operands_memory(lib, world, M, K, where, kmajor):
-    """A square layer in place: nothing is stored to memory that the product still reads.  The GEMM and the reduction behind it store
-    this rank's partial, the sums in the GEMM's epilogue do not."""
+    """A square layer in place: nothing is stored to memory that the product still reads, nor to that of another owner's partial, which it
+    still writes.  The GEMM and the reduction behind it store this rank's partial, the sums in the GEMM's epilogue do not."""
     dtype, cols = torch.bfloat16, K
     ctxs = tileccl.init_local(world_size=world, heap_size=128 << 20)
     try:
@@ -136,7 +136,7 @@ def test_output_in_an_operands_memory(lib, world, M, K, where, kmajor):
         B = ctx.zeros(world * cols, K, dtype=dtype).t() if kmajor else ctx.zeros(K, world * cols, dtype=dtype)
         part = ctx.workspace("gemm_reducescatter.partial", world, M, cols, dtype=torch.float32)
         stored = B.t() if kmajor else B
-        out = {"A": A, "B": stored.reshape(-1)[: M * cols].view(M, cols), "behind A": room[M:]}[where]
+        out = {"A": A, "B": stored.reshape(-1)[: M * cols].view(M, cols), "behind A": room[M:], "C": part[1].view(dtype).reshape(-1)[: M * cols].view(M, cols)}[where]
         got = []
         for o in (apart, out):
             A.copy_(A_cpu)

@@ -1132,10 +1132,11 @@ bool sums_across(const tccl_gemm_desc* d, const tccl::CommArgs& c, TileKernel ke
   const bool pays = kmajor ? (c.world == 2 || c.world == 4 || c.world == 8)
                            : c.world == 2 || (c.world == 4 && d->K <= 2048 && 2 * tiles >= cus);
   if (!pays) return false;
-  // The first sums are stored while other workgroups still read A and B: an output that shares memory with them (a square layer in
-  // place) is written by a launch behind the GEMM.
+  // The first sums are stored while other workgroups still read A and B and store partials: an output that shares memory with them (a
+  // square layer in place) is written by a launch behind the GEMM.
   const int64_t rows = d->M / c.world, cols = (int64_t)c.world * d->N, k_rows = d->K - ((d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15);
   const int64_t out_bytes = (rows - 1) * c.ld_rs_out_bytes + (int64_t)d->N * 2;
+  if (overlap(c.rs_out, out_bytes, d->C, ((int64_t)(d->M - 1) * d->ldc + d->N) * 4)) return false;
   if (overlap(c.rs_out, out_bytes, d->A, ((rows - 1) * d->lda + d->K) * 2)) return false;
   if (overlap(c.rs_out, out_bytes, d->B, (kmajor ? (cols - 1) * d->ldb + d->K : (k_rows - 1) * d->ldb + cols) * 2)) return false;
   // 32-bit offsets that now run over all shards.
