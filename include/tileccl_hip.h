@@ -102,8 +102,9 @@ typedef struct tccl_gemm_desc {
  * tiles; small outputs with TCCL_GEMM_ARRIVALS or of ragged column shards; 128 x 128 tiles that wait for their peers, at most
  * one per CU; and 16-bit inputs as column shards with TCCL_RS_PEERS_RESIDENT (TCCL_GEMM_ARRIVALS too where the shards are whole plan tiles),
  * fp32 partials and a 16-bit `out` that has 16-byte rows and shares no memory with A, B or C, on 2, 4 or 8 ranks, K > 192, where 128 x 128
- * tiles named by nobody are at most one per CU (a row-major B: two ranks, or four up to K = 2048 with half the CUs at
- * work).  Elsewhere the sums are a launch of their own and every partial is stored; a caller who reads these rows of C leaves the flag out.
+ * tiles named by nobody are at most one per CU (a row-major B: two ranks, K up to 6144 where a shard's rows start off 64-byte
+ * boundaries, or four with half the CUs at work, K up to 1280 off such boundaries (1536 if A's rows lie off them too), 1792 on them
+ * and 2048 on 128-byte ones).  Elsewhere the sums are a launch of their own and every partial is stored; a caller who reads these rows of C leaves the flag out.
  * the partial of the rows this rank owns stays in the accumulators, takes the peers' partials
  * in the GEMM epilogue and is never stored to gemm->C (those rows of C keep their old
  * contents); the output is bit-identical to storing and reducing.  Ignored elsewhere and in S0.

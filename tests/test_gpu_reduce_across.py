@@ -120,6 +120,23 @@ def test_the_bulk_schedule_stores_every_partial(lib, world, rank, M, N, K, kmajo
         assert torch.equal(got[variant, True][1][others], partial[others]) and torch.all(got[variant, True][1][rank] == -7.0)
 
 
+@pytest.mark.parametrize("world,rank,M,cols,K,kmajor,across", [
+    (4, 1, 1024, 704, 2048, False, True), (4, 1, 1024, 704, 2056, False, False), (4, 2, 700, 736, 1792, False, True),
+    (4, 2, 700, 736, 1800, False, False), (4, 3, 1000, 648, 1280, False, True), (4, 3, 1000, 648, 1312, False, False),
+    (4, 0, 1000, 648, 1528, False, True), (4, 0, 1000, 648, 1544, False, False), (4, 0, 1000, 648, 2048, True, True),
+    (2, 1, 1000, 904, 6144, False, True), (2, 1, 1000, 904, 6152, False, False), (2, 1, 1000, 928, 6152, False, True)])
+def test_longest_k_of_a_row_major_b(lib, world, rank, M, cols, K, kmajor, across):
+    """Beyond it the runs of B cost more than the second launch, which reads a stored partial: the sums are the same."""
+    for own in (False, True):
+        out, partial, want, peers = reduce(world, rank, M, world * cols, K, torch.bfloat16, kmajor, "s2", own)
+        assert torch.all(partial[rank] == -7.0) == (across and own)
+        if not own:
+            tall = [(partial if p == rank else peers[p]).reshape(world * M, cols) for p in range(world)]
+            sums = oracle.reduce_rows(tall, rank, torch.bfloat16)
+            assert_gemm_close(torch.cat(list(partial), 1), want)
+        assert torch.equal(bits(out), bits(sums))
+
+
 @pytest.mark.parametrize("kmajor", [False, True])
 @pytest.mark.parametrize("where", ["A", "B", "behind A", "C"])
 @pytest.mark.parametrize("world,M,K", [(2, 1024, 776), (4, 700, 648)])

@@ -1125,13 +1125,25 @@ bool sums_across(const tccl_gemm_desc* d, const tccl::CommArgs& c, TileKernel ke
   if (c.ld_rs_out_bytes % 16 || ((uintptr_t)c.rs_out & 15)) return false;
   if (d->K <= 3 * 64) return false;  // the last three K steps are apart, and one goes before them
   const bool kmajor = (d->flags & TCCL_GEMM_B_KMAJOR) != 0;
-  // A k-major B costs the same in runs.  A row-major one on two ranks costs a tenth more per K step; on four (64 x 256) a third
-  // more, which the reduction's time pays for up to here, bf16: 1024 x 4096 x 2048 31.2 -> 28.1 us, 2048 x 2048 x 2560 33.1 ->
-  // 32.2, 1024 x 4096 x 3072 36.1 -> 36.2, 1500 x 2208 x 2600 38.4 -> 41.5; a device less than half full: 512 x 2048 x 2048 16.9
-  // -> 17.2.  On eight it never does: 1024 x 4096 x 2048 30.4 -> 43.7.
-  const bool pays = kmajor ? (c.world == 2 || c.world == 4 || c.world == 8)
-                           : c.world == 2 || (c.world == 4 && d->K <= 2048 && 2 * tiles >= cus);
-  if (!pays) return false;
+  // A k-major B costs the same in runs.  A row-major one costs more per K step, on two ranks a tenth, on four (64 x 256) a third, and
+  // twice that where its runs of 64 columns start off 64-byte boundaries and take a line more each (less of it where the tiles beside
+  // them lose as much by A's rows): up to here the reduction's time pays for it (at the line itself some shapes gain and others lose 3 %).  bf16, GEMM and
+  // reduction -> this:
+  //   four ranks, whole lines: 1024 x 4096 x 2048 30.5 -> 27.7 us, 2048 x 2048 x 2560 33.1 -> 32.2, 1024 x 4096 x 3072 36.1 -> 36.2
+  //   64-byte boundaries: 1920 x 1920 x 1600 27.2 -> 25.7, x 1800 30.5 -> 29.9, x 2048 30.2 -> 30.2; 768 x 2944 x 1600 / 2048 24.0 / 26.9 -> 23.8 / 27.8
+  //   off them: 1500 x 2208 x 1024 / 1280 / 1600 22.3 / 24.7 / 26.9 -> 21.4 / 24.3 / 28.0, 1000 x 2592 20.8 / 22.9 / 25.0 -> 20.6 / 23.3 / 26.7
+  //   and A's rows too: 1500 x 2208 x 1304 / 1528 / 1800 26.8 / 28.3 / 31.3 -> 25.7 / 28.2 / 31.8, 1000 x 2592 24.8 / 26.4 / 29.0 -> 24.6 / 27.4 / 30.5
+  //   two ranks off them: 1500 x 2208 x 4096 / 6144 / 8192 / 16384 44.3 / 60.2 / 75.4 / 136 -> 42.3 / 59.3 / 75.6 / 143; on them x 16384 no loss
+  //   four ranks, a device less than half full: 512 x 2048 x 2048 16.9 -> 17.2; eight: 1024 x 4096 x 2048 30.4 -> 43.7
+  const bool on64 = ((uintptr_t)d->B & 63) == 0 && d->ldb % 32 == 0 && d->N % 32 == 0;
+  int longest = 0;  // K
+  if (kmajor ? c.world == 2 || c.world == 4 || c.world == 8 : c.world == 2 && on64)
+    longest = INT32_MAX;
+  else if (c.world == 2)
+    longest = 6144;
+  else if (c.world == 4 && 2 * tiles >= cus)
+    longest = on64 ? (d->N % 64 == 0 ? 2048 : 1792) : (d->lda % 32 ? 1536 : 1280);
+  if (d->K > longest) return false;
   // The first sums are stored while other workgroups still read A and B and store partials: an output that shares memory with them (a
   // square layer in place) is written by a launch behind the GEMM.
   const int64_t rows = d->M / c.world, cols = (int64_t)c.world * d->N, k_rows = d->K - ((d->flags >> TCCL_GEMM_B_SHORT_SHIFT) & 15);

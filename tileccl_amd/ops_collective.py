@@ -235,7 +235,7 @@ def gemm_reducescatter(A: Any, B: Any, Cx: Any, *, ctx=None, implementation: str
     sums each tile as it finishes, and (``own_rows_in_registers``, the default)
     block ``rank`` never leaves the accumulators as a partial: its part of the workspace is not
     written (``"s0"`` stores every block).  So is one with at most a 128 x 128 tile per CU and the peers' partials resident, on 2, 4 or 8 ranks
-    (a row-major ``B`` on four ranks up to ``K`` = 2048, not on eight); elsewhere on 128 x 128 tiles with resident partials
+    (a row-major ``B`` on four ranks up to ``K`` = 2048, 1280 where its shards are no whole 64-byte pieces, not on eight); elsewhere on 128 x 128 tiles with resident partials
     the sums are a second launch.  ``variant`` picks the schedule (``"s0"`` bulk, ``"s1"`` tile by tile, ``"s2"``
     TileGroup).  ``emulate_peer`` (single-GPU emulation) also writes the other ranks' outputs
     into their slices.
