@@ -105,6 +105,42 @@ def test_all_scatter_into_its_own_input(lib, in_place_first):
             c.heap.cleanup()
 
 
+@pytest.mark.parametrize("variant", ["s0", "s1", "s2"])
+@pytest.mark.parametrize("world,directions,how", [(2, "pull", {}), (2, "both", {}), (2, "push", {"trace": True}), (2, "both", {"trace": True}),
+                                                  (3, "push", {"num_gemm_wgs": 40}), (4, "push", {})])
+@pytest.mark.parametrize("M,N,K", [(1032, 2056, 203), (1000, 2064, 1003)])
+def test_all_gather(lib, monkeypatch, world, directions, how, variant, M, N, K):
+    """Pulls beside the GEMM, transfers kept apart by clock stamps, pushes to several peers, workgroups counted by the caller."""
+    from functools import partial
+
+    from tileccl_amd import _launch, _lib
+    from tileccl_amd.v2 import FusedGemmAllGather, SymmetricHeap
+
+    heaps = SymmetricHeap.create_all(96 << 20, world)
+    try:
+        ops = [FusedGemmAllGather(h, M, N, torch.bfloat16, directions=directions, **how) for h in heaps]
+        A_cpu, B_cpu = seeded((M, K), 0, torch.bfloat16), seeded((K, N), 1, torch.bfloat16, scale=K**-0.5)
+        B = B_cpu.cuda()
+        given, got = _launch._gemm_desc, []
+        assert given(columns(A_cpu, 1040, 0.0), B, ops[0].local_block, a_columns=True)[0].flags & _lib.GEMM_A_COLUMNS
+        for A, in_place in ((A_cpu.cuda(), False), (columns(A_cpu, 1040, float("nan")), True)):
+            monkeypatch.setattr(_launch, "_gemm_desc", partial(given, a_columns=in_place))
+            for r, op in enumerate(ops):
+                op.out.zero_()
+                op.local_block.copy_(seeded((M, N), 5 + r, torch.bfloat16))
+            ops[0].mark_peers_ready()
+            ops[0](A, B, variant)
+            ops[0].check_faults()
+            torch.cuda.synchronize()
+            got.append([bits(op.out).cpu().clone() for op in ops])
+        for x, y in zip(*got):
+            assert torch.equal(x, y)
+        assert_gemm_close(ops[0].local_block, A_cpu.float() @ B_cpu.float())
+    finally:
+        for h in heaps:
+            h.cleanup()
+
+
 def test_refusals(lib):
     from tileccl_amd import _launch, _lib
 

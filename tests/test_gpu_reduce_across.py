@@ -191,3 +191,56 @@ def test_every_plan_tile_is_published_once(lib):
     finally:
         for c in ctxs:
             c.heap.cleanup()
+
+
+@pytest.mark.parametrize("variant", ["s1", "s2"])
+@pytest.mark.parametrize("world,kmajor", [(4, False), (8, True)])
+def test_two_streams_and_a_recorded_graph(lib, world, kmajor, variant):
+    """Launches that overlap count in the same lines of arrival words; a recorded launch counts in the word it was recorded with,
+    between eager ones.  All leave the words zero, every plan tile published once by each, and the sums of one launch alone."""
+    from tileccl_amd import ops_collective
+
+    M, cols, K = 384, 904, 1032
+    ctxs = tileccl.init_local(world_size=world, heap_size=128 << 20)
+    try:
+        ctx = ctxs[0]
+        A = ctx.zeros(M, K, dtype=torch.float16)
+        B = ctx.zeros(world * cols, K, dtype=torch.float16).t() if kmajor else ctx.zeros(K, world * cols, dtype=torch.float16)
+        A.copy_(seeded((M, K), 0))
+        B.copy_(seeded((K, world * cols), 1, scale=K**-0.5))
+        outs = [ctx.zeros(M, cols, dtype=torch.float16) for _ in range(3)]
+        for p, c in enumerate(ctxs):
+            c.workspace("gemm_reducescatter.partial", world, M, cols, dtype=torch.float32).copy_(seeded((world, M, cols), 10 + p, torch.float32))
+        call = lambda out: tileccl.ops.gemm_reducescatter(A, B, out, ctx=ctx, variant=variant)
+        call(outs[2])
+        torch.cuda.synchronize()
+        alone = outs[2].clone()
+        words = ops_collective._reduce_scatter_words(ctx, world, M, cols)
+
+        def check(launches, which):
+            torch.cuda.synchronize()
+            assert all(torch.equal(bits(outs[i]), bits(alone)) for i in which)
+            assert not words.arrivals.any()
+            if variant == "s2":
+                assert words.counter.tolist() == [launches * int(c) for c in words.host_plan.tile_counts()]
+            for o in outs:
+                o.zero_()
+            torch.cuda.synchronize()
+
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        for _ in range(20):
+            for out, stream in zip(outs, streams):
+                with torch.cuda.stream(stream):
+                    call(out)
+        check(41, (0, 1))
+        graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+            call(outs[0])
+        for _ in range(4):  # (from here on every launch starts from cleared counters: SyncWords)
+            graph.replay()
+            call(outs[1])
+            check(1, (0, 1))
+            assert (torch.randn(256, 256, device="cuda") @ torch.randn(256, 256, device="cuda")).isfinite().all()
+    finally:
+        for c in ctxs:
+            c.heap.cleanup()
