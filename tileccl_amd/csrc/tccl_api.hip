@@ -600,6 +600,7 @@ constexpr TileCost kCost128 = {0.50, 0.15, 0.12, 0.5, 0.0, 1.5};   // one workgr
 constexpr TileCost kCost128Two = {1.25, 0.0, 0.10, 1.5, 0.0, 1.5}; // two: as soon as some CU has two
 
 double rounds_us(const TileCost& c, int64_t tiles, int slots, const tccl_gemm_desc* d, bool pushes) {
+  // (An A given by columns is judged by its pitch as well: the costs were fitted on rows.)
   const bool aligned = d->lda % 32 == 0 && (!(d->flags & TCCL_GEMM_B_KMAJOR) || d->ldb % 32 == 0);
   const double steps = (d->K + 63) / 64, step = c.idle + (aligned ? 0.0 : c.misaligned), end = c.stores + (pushes ? c.pushes : 0.0);
   const double rest = (double)(tiles % slots) / slots;
@@ -1683,9 +1684,11 @@ int tccl_gemm(const tccl_gemm_desc* d, void* stream) {
                       (hipStream_t)stream);
 }
 
-// The 128 x 128-tile kernels read an A given by columns in place; the streaming and the large-tile kernel do not, and where they would run a
-// launch that turns A into rows comes first (as it does for what check_gemm() refuses).  1000 x 2064 x 1003 bf16 pushed to one peer: 15.5 us in place,
-// 21.6 with that launch.
+// The 128-row tile kernels read an A given by columns in place; the streaming and the large-tile kernel do not, and where they would run a
+// launch that turns A into rows comes first (as it does for what check_gemm() refuses).  From CUs / 2 large tiles on it always does, also where
+// choose_tiles() would name a 128-row kernel for a launch of pushes.  bf16 pushed to one peer, with that launch -> in place: 1000 x 2064 x 1003
+// 21.6 -> 15.3 us, 256 x 6144 x 72 11.7 -> 7.2, 2048 x 2048 x 2048 33.3 -> 24.7, 1544 x 4112 x 8192 119 -> 113 (60 shapes, K = 72 to 8192: 1.05 to 1.79
+// times as fast).
 int tccl_gemm_reads_columns(const tccl_gemm_desc* d) {
   if (!d || !(d->flags & TCCL_GEMM_A_COLUMNS) || d->macro_tile != 0 || d->block_m != 128 || d->block_n != 128 || check_gemm(d)) return 0;
   tccl_device_info dev;

@@ -179,7 +179,7 @@ struct EpilogueReduce {
 };
 
 // Columns of a sub-tile across the owners (its rows: 16384 over that).  A row-major B is read in runs of an owner's columns:
-// those of four ranks get 64, whole 128-byte lines, in a sub-tile of 64 x 256.  With runs of 32 they take as long per K step,
+// those of four ranks get 64, whole lines where a shard's rows start on them, in a sub-tile of 64 x 256.  With runs of 32 they take as long per K step,
 // with a quarter less to read; the eight ranks' runs of 16 take half as long again (sums_across()).
 TCCL_HD constexpr int across_cols(int world, bool b_kmajor) { return world == 4 && !b_kmajor ? 256 : 128; }
 
