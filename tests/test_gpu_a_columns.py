@@ -105,6 +105,33 @@ def test_all_scatter_into_its_own_input(lib, in_place_first):
             c.heap.cleanup()
 
 
+def test_all_scatter_from_a_peers_copy_of_its_output(lib):
+    """``C.t() @ B`` into ``C`` with the input taken from the other rank's copy, which the launch stores to."""
+    import tileccl_amd
+    from tileccl_amd import ops
+
+    n, dtype = 1040, torch.bfloat16
+    ctxs = tileccl_amd.init_local(world_size=2, heap_size=128 << 20)
+    try:
+        A_cpu, B_cpu = seeded((n, n), 0, dtype), seeded((n, n), 1, dtype, scale=n**-0.5)
+        outs, spare = [c.zeros(n, n, dtype=dtype) for c in ctxs], [c.zeros(n, n, dtype=dtype) for c in ctxs]
+        B = ctxs[0].zeros(n, n, dtype=dtype)
+        B.copy_(B_cpu)
+        assert [ctxs[0].heap.lies_with_a_peer(t) for t in (*outs, B_cpu.cuda())] == [False, True, False]
+        got = []
+        for held in (spare[0], outs[1], spare[0], outs[1]):
+            held.copy_(A_cpu.t())
+            ops.gemm_allscatter(held.t(), B, outs[0], ctx=ctxs[0])
+            torch.cuda.synchronize()
+            got.append([bits(o[:, : n // 2]).cpu().clone() for o in outs])
+        for x in got[1:]:
+            assert all(torch.equal(a, b) for a, b in zip(x, got[0]))
+        assert_gemm_close(outs[0], A_cpu.float() @ B_cpu.float())
+    finally:
+        for c in ctxs:
+            c.heap.cleanup()
+
+
 @pytest.mark.parametrize("variant", ["s0", "s1", "s2"])
 @pytest.mark.parametrize("world,directions,how", [(2, "pull", {}), (2, "both", {}), (2, "push", {"trace": True}), (2, "both", {"trace": True}),
                                                   (3, "push", {"num_gemm_wgs": 40}), (4, "push", {})])

@@ -158,6 +158,14 @@ def test_an_a_by_columns_lies_apart_from_c(table):
     assert table.launch(("columns",), None, moved, b, at(0, M, N, N)) is True and _launch._apart(moved, at(0, M, N, N))
     assert table.launch(("columns",), None, moved, b, at(8, M, N, N)) is None and not _launch._apart(moved, at(8, M, N, N))
     assert len(seen) == 3
+    # Three ranks' heaps, this one's in the middle: an A that starts in another's may be what the launch stores to that rank.
+    heap = Heap(at(1024, 1, 1, 1), 2048)
+    heap.all_ranks = (heap.local_base - 2048, 3 * 2048)
+    _launch.bind(table, ("peers",), (at(1024, K, M, pitch).t(), b, c), entry, (gemm,), "columns", gemm=gemm, c=(2, 0), heap=heap, on_heap=0)
+    behind = torch.zeros(8192, dtype=torch.float16)
+    for first, fits in ((1024, True), (1016, None), (0, None), (2048, None), (3064, None), (3072, True)):
+        out = behind.as_strided((M, N), (N, 1), -(behind.data_ptr() // 2) % 8)
+        assert table.launch(("peers",), None, at(first, K, M, pitch).t(), b, out) == fits, first
 
 
 @pytest.mark.parametrize("kind", ["sparse", "nested", "jagged", "vmap", "grad", "meta"])

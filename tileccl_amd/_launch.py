@@ -286,7 +286,8 @@ def bind(table, key: tuple, tensors: tuple, fn, args: tuple, what: str, *, gemm:
     first where ``plan`` says so) and, with ``c=(i, offset)``, tensor ``i``'s as C; ``SYNC`` for ``words``' descriptor with
     the launch's number; ``(i, offset)`` for the address of tensor ``i``; other descriptors are passed as they are.
     The tensors of the bit mask ``on_heap`` (default: all) must start inside ``heap``; with ``bases`` all tensors must lie at
-    one distance from their base.  Tensors for which that does not hold find no call."""
+    one distance from their base.  An A that is read by columns lies apart from C and, with ``heap``, in no other rank's.
+    Tensors for which that does not hold find no call."""
     host = _lib.host()
     entry = _ENTRIES.get(what)
     if entry is None or entry[0] is not fn:
@@ -304,10 +305,11 @@ def bind(table, key: tuple, tensors: tuple, fn, args: tuple, what: str, *, gemm:
         passed.append(a)
     sync = None if words is None else words.desc(variant)
     packs = plan is not None and (plan.pack_a or plan.pack_b)
+    by_columns = gemm is not None and gemm.flags & _lib.GEMM_A_COLUMNS
     table.add(host.Call(
         entry[1], what, tuple(passed), tensors, key, tag=tag, gemm=0 if gemm is None else C.addressof(gemm), c=c,
         sync=0 if sync is None else C.addressof(sync), words=words, variant=variant, on_heap=on_heap,
-        heap=None if heap is None else (heap.local_base, heap.size), bases=bases,
+        heap=None if heap is None else (heap.local_base, heap.size, *(heap.all_ranks if by_columns else ())), bases=bases,
         prepare=partial(planned_operands, plan) if packs else None, keep=keep,
     ))
 

@@ -80,6 +80,7 @@ struct Call {
   int64_t c_offset;
   int64_t a_bytes, c_bytes;  // of an A that the GEMM reads by columns (0: it does not) and of its C: they must lie apart
   int64_t heap_lo, heap_size;  // the tensors in `on_heap` (a bit mask) must start in this range
+  int64_t ranks_lo, ranks_size;  // all ranks' heaps: an A by columns lies in none but this rank's, where launches store to the peers'
   uint32_t on_heap;
   std::vector<int64_t>* bases;  // per tensor: all must lie at one offset from these
   int counted;           // 0: the launch is not numbered, 1: by `epoch`, 2: by `lock_epoch`
@@ -267,10 +268,12 @@ int call_init_checked(Call* self, PyObject* pos, PyObject* kw) {
     self->c_bytes = ((int64_t)(d.M - 1) * d.ldc + d.N) * (d.out_dtype == TCCL_F32 ? 4 : 2);
   }
   if (heap != Py_None) {
-    long long lo = 0, size = 0;
-    if (!PyArg_ParseTuple(heap, "LL", &lo, &size)) return -1;
+    long long lo = 0, size = 0, all_lo = 0, all_size = 0;
+    if (!PyArg_ParseTuple(heap, "LL|LL", &lo, &size, &all_lo, &all_size)) return -1;
     self->heap_lo = lo;
     self->heap_size = size;
+    self->ranks_lo = all_lo;
+    self->ranks_size = all_size;
     self->on_heap = on_heap == Py_None ? ~0u : (uint32_t)PyLong_AsUnsignedLongMask(on_heap);
     if (PyErr_Occurred()) return -1;
   }
@@ -457,6 +460,8 @@ bool fits(const Call* c, PyObject* const* tensors, const int64_t* at, Py_ssize_t
   if (c->a_bytes) {
     const int64_t out = c->c_tensor >= 0 ? at[c->c_tensor] + c->c_offset : (int64_t)(uintptr_t)c->gemm.C;
     if (at[0] < out + c->c_bytes && out < at[0] + c->a_bytes) return false;
+    auto starts_in = [at](int64_t lo, int64_t size) { return at[0] - lo >= 0 && at[0] - lo < size; };
+    if (starts_in(c->ranks_lo, c->ranks_size) && !starts_in(c->heap_lo, c->heap_size)) return false;
   }
   return true;
 }

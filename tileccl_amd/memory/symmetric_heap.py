@@ -124,6 +124,12 @@ class SymmetricHeap:
         return self._local_ptr
 
     @property
+    def all_ranks(self) -> tuple[int, int]:
+        """(first byte, bytes) of the memory that holds every rank's heap."""
+        bases = self._arena.bases
+        return bases[0], bases[-1] + self._size - bases[0]
+
+    @property
     def live_id(self) -> int:
         """A number that no other heap of this process has had, 0 once this one has been cleaned up.  (A later heap may
         lie at the same address.)"""
@@ -181,6 +187,11 @@ class SymmetricHeap:
         return 0 <= tensor.data_ptr() - self._local_ptr < self._size or tensor.numel() == 0
 
     is_symmetric = owns_tensor
+
+    def lies_with_a_peer(self, tensor: torch.Tensor) -> bool:
+        """The tensor starts in another rank's heap."""
+        first, size = self.all_ranks
+        return 0 <= tensor.data_ptr() - first < size and not self.owns_tensor(tensor)
 
     def import_external_tensor(self, tensor: torch.Tensor) -> torch.Tensor:
         """Copy a contiguous device tensor into the heap."""

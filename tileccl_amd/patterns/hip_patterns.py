@@ -99,7 +99,7 @@ class _HipAllScatterPattern(Pattern):
         C_out = C_out if C_out is not None else tensors[2]
         gemm, plan = _launch._gemm_desc(
             tensors[0], tensors[1], C_out, block_m=self.BLOCK_M, block_n=self.BLOCK_N, group_m=self.GROUP_M, num_wgs=compute_wgs,
-            flags=_lib.GEMM_ARRIVALS, a_columns=True,
+            flags=_lib.GEMM_ARRIVALS, a_columns=spec.world_size == 1 or not heap.lies_with_a_peer(tensors[0]),
         )
         scatter = _lib.ScatterDesc(
             spec.scatter_src_col_offset, spec.scatter_cols, spec.scatter_dst_leading_dim, spec.scatter_dst_col_offset
