@@ -122,7 +122,7 @@ typedef struct tccl_gemm_desc {
 #define TCCL_GEMM_B_SHORT_SHIFT 8
 /* A is given by columns: element (m, k) is at A[k * lda + m], i.e. A is the `.t()` view of a (K, M) tensor (the input of
  * a weight gradient); lda >= M is then the pitch between columns.  16-bit inputs, M a multiple of 8, row-major B, no column
- * shards, 128 x 128 tiles, no memory shared with C; tccl_gemm, _allscatter and _allgather.  tccl_gemm_reads_columns() says whether a call is better off so.  The last n
+ * shards, 128 x 128 tiles, no memory shared with C or its copies; tccl_gemm, _allscatter and _allgather.  tccl_gemm_reads_columns() says whether a call is better off so.  The last n
  * (0 .. 7) of the K columns may be missing, they are taken as zero: flags |= n << TCCL_GEMM_A_SHORT_SHIFT. */
 #define TCCL_GEMM_A_COLUMNS 16
 #define TCCL_GEMM_A_SHORT_SHIFT 12
